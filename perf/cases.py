@@ -93,7 +93,7 @@ def _sequences(case):
 
 def _config(case):
     longest = max(c + t for c, t in _sequences(case))
-    return get_config(case["model"], num_layers=LAYERS[case["model"]], max_position=max(8192, longest + 64))
+    return get_config(case["model"], num_layers=LAYERS[case["model"]], max_position=max(8192, 1 << (longest + 15).bit_length()))
 
 
 def _keys(case):
@@ -183,10 +183,10 @@ def prepare(case, seed):
             else:
                 L["gate_up"].copy_(ops.interleave_gate_up(w["gate"], w["up"]))
                 L["down"].copy_(w["down"])
-    longest = max(c + t for c, t in seqs)
+    longest = max(c + t for c, t in seqs) + 16
     pages = sum(-(-(c + t) // BLOCK_SIZE) for c, t in seqs) + 8
     rows = 256 if len(seqs) <= 256 else 1024
-    eng = Engine(model, EngineConfig(max_num_seqs=rows, max_num_batched_tokens=STEP, max_model_len=longest + 16,
+    eng = Engine(model, EngineConfig(max_num_seqs=rows, max_num_batched_tokens=STEP, max_model_len=max(4096, 1 << (longest - 1).bit_length()),
                                      num_kv_blocks=pages, enable_prefix_caching=False))
     eng.kv.wait_ready()
     eng.alloc.grow(eng.kv.ready_blocks())
