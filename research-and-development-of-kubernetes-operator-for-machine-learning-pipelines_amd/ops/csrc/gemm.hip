@@ -1335,6 +1335,30 @@ static bool sk_halves_ok(long T, int nk) {
   return b && T * 2 <= b->cus && sk_choose_d((int)T, nk, b->cus, sk_min_half()) >= 2;
 }
 
+// Variant 7, the weight stream of gemm_mid.hip, for up to 384 rows: where its tasks take at least three
+// quarters of the CUs, in one K range with 256 or 128 columns, or (65 rows and more) with K in up to 8 ranges of
+// at least 12 K-steps.  Below that, and for split K at 64 rows and fewer, the small tiles are as fast or faster
+// (o 4096 x 4096 at 100 rows 17.5 us against 18.6 in six ranges; down 4096 x 14336 at 16 / 64 rows 24.2 / 29.2
+// against 26.6 / 29.5); from 512 rows on the four-wave kernel is (gate_up 93 us against 115).
+static bool mid_plan(int M, int N, int K, Plan& p) {
+  constexpr int max_m = 384, fill = 192;
+  if (M > max_m || K % kBK || N % 8) return false;
+  const int m_tiles = M <= 256 ? 1 : 2, rows = (M + m_tiles - 1) / m_tiles;
+  const int bm = rows <= 64 ? 64 : rows <= 192 ? (rows + 31) / 32 * 32 : 256;
+  const int t256 = (N + 255) / 256 * m_tiles, t128 = (N + 127) / 128 * m_tiles, nk = K / kBK;
+  int s = 1;
+  if (t256 < fill && t128 < fill) {
+    s = std::min({kMaxSplits, 256 / t128, nk / 12});
+    if (M <= 64 || t128 * s < fill) return false;
+  }
+  p.variant = 7;
+  p.BM = bm;
+  p.BN = t256 >= fill ? 256 : 128;
+  p.k_chunk = (nk + s - 1) / s * kBK;
+  p.splits = (K + p.k_chunk - 1) / p.k_chunk;
+  return true;
+}
+
 static Plan plan(int M, int N, int K, bool grouped, int n_groups, int rows_per_group) {
   Plan p{};
   p.variant = 0;
@@ -1346,7 +1370,8 @@ static Plan plan(int M, int N, int K, bool grouped, int n_groups, int rows_per_g
   // 474 -> 370 / 266 -> 200 us, 1024 rows 692 -> 389 / 375 -> 208 us; 48 rows per expert equal
   // (scripts/bench_moe_decode.py, profiles/r05_moe_decode.md)
   constexpr int pp_group_min_rows = 56;
-  if (grouped && mrows >= pp_group_min_rows && K % kBK == 0 && N % 256 == 0) {
+  if (!grouped && g_dp[0] < 0 && mid_plan(M, N, K, p)) {
+  } else if (grouped && mrows >= pp_group_min_rows && K % kBK == 0 && N % 256 == 0) {
     p.BM = 256; p.BN = 256; p.variant = 3;  // grouped ping-pong
   } else if (mrows <= 64 && !grouped && g_small_tile == 1) {
     // per shape (scripts/run137.sh, cold us at M = 16): wide N (gate_up) 64 columns with a
@@ -1482,6 +1507,7 @@ static Plan plan(int M, int N, int K, bool grouped, int n_groups, int rows_per_g
   const int n_tiles = (N + p.BN - 1) / p.BN;
   const int real_m_tiles = (M + p.BM - 1) / p.BM;
   p.m_tiles = grouped ? real_m_tiles + n_groups : real_m_tiles;
+  if (p.variant == 7) return p;
   p.splits = 1;
   p.k_chunk = K;
   const long tiles = (long)n_tiles * real_m_tiles;
@@ -1523,7 +1549,9 @@ static void launch_plan(const Plan& p, const uint16_t* A, int lda, const uint16_
     // weight-streaming tiles (M <= 128): a deeper LDS-DMA ring keeps more weight bytes in
     // flight per CU (3 stages x 16 KB per workgroup streamed gate_up at 4.7 TB/s at M = 64)
     const int sst = p.stages ? p.stages : g_small_stages;
-    if (!GROUPED && p.variant == 6 && p.splits == 1 && gemm_w4_ok(M, N, K, lda, ldb, ldc))
+    if (!GROUPED && p.variant == 7)
+      launch_mid(EPI, p.BM, p.BN, A, lda, B, ldb, C, ldc, ws, M, N, K, p.splits, p.k_chunk, st, re);
+    else if (!GROUPED && p.variant == 6 && p.splits == 1 && gemm_w4_ok(M, N, K, lda, ldb, ldc))
       run_w4(EPI, A, lda, B, ldb, C, ldc, M, N, K, st, re, 128);
     else if (!GROUPED && p.variant == 6) run_pp<EPI>(A, lda, B, ldb, C, ldc, M, N, K, st, re);
     else if (p.BM == 16 && p.BN == 32 && sst >= 8) MLOP_GEMM(16, 32, 1, 2, 8, false);
@@ -1571,7 +1599,7 @@ int gemm_sk_workgroups(int M, int N, int K) {
 // fused into the RoPE + cache kernel (one launch instead of reduce + rope_cache).
 static bool rope_slabs_ok(const Plan& p, int M, int N) {
   const SkBuf* b = sk_buf();
-  return p.splits > 1 && p.variant != 3 && p.variant < 5 && b != nullptr &&
+  return p.splits > 1 && (p.variant == 7 || (p.variant != 3 && p.variant < 5)) && b != nullptr &&
          (size_t)p.splits * M * N <= (size_t)2 * kSkMaxWg * 256 * 256;
 }
 
@@ -1596,11 +1624,14 @@ static Plan rope_plan(int M, int N, int K) {
   return p;
 }
 
+// plans whose kernel has the RoPE epilogue (whole heads per tile)
+static bool rope_tiles(const Plan& p) { return p.variant != 7 && (p.BM == 256 || p.variant == 6) && p.BN >= 128; }
+
 bool gemm_rope_supported(int M, int N, int K) {
   if (M <= 0 || N % 128 || K % kBK) return false;
   if (gemv_takes(M, N, K, EPI_ROPE)) return true;  // decode M <= 8: gemv.hip
   const Plan p = rope_plan(M, N, K);
-  return ((p.BM == 256 || p.variant == 6) && p.BN >= 128) || rope_slabs_ok(p, M, N);
+  return rope_tiles(p) || rope_slabs_ok(p, M, N);
 }
 
 bool launch_gemm_rope(const void* A, int lda, const void* B, int M, int N, int K, const RopeEpi& re,
@@ -1616,7 +1647,7 @@ bool launch_gemm_rope(const void* A, int lda, const void* B, int M, int N, int K
     return true;
   }
   Plan p = rope_plan(M, N, K);
-  if (!((p.BM == 256 || p.variant == 6) && p.BN >= 128)) {  // small M: split-K slabs + fused reduce / RoPE / cache
+  if (!rope_tiles(p)) {  // small M: split-K slabs + fused reduce / RoPE / cache
     float* ws = sk_buf()->ws;
     launch_plan<EPI_NONE, false>(p, (const uint16_t*)A, lda, (const uint16_t*)B, K, nullptr, N, ws,
                                  M, N, K, nullptr, 0, st);
@@ -1681,9 +1712,10 @@ bool mid_chain_ok(int M, int N, int K, int epi) {
   if (epi == EPI_ROPE) {
     if (ws_prefer(M, N, K, EPI_ROPE)) return K % 512 == 0;
     const Plan p = rope_plan(M, N, K);
-    return !((p.BM == 256 || p.variant == 6) && p.BN >= 128) && rope_slabs_ok(p, M, N);
+    return !rope_tiles(p) && rope_slabs_ok(p, M, N);
   }
   const Plan p = plan(M, N, K, false, 0, 0);
+  if (epi == EPI_SILU_MUL && p.variant == 7) return p.splits == 1;
   if (p.variant != 0 || p.BM > 64 || N % p.BN) return false;
   if (epi == EPI_SILU_MUL) return p.splits == 1;
   if (epi != EPI_NONE || p.splits < 2) return false;

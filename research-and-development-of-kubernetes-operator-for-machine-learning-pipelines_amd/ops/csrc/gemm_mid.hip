@@ -1,0 +1,293 @@
+// K1 / K2 at 5-384 rows: a weight stream that feeds the matrix cores.
+//
+//   C[M, N] = A[M, K] . B[N, K]^T      (A activations, B weights [out, in], both bf16)
+//
+// What bounds it: reading B once (every weight byte from HBM, ~6.5 TB/s at best); A is small and comes
+// from L2, once per workgroup.  The LDS-ring tiles of gemm.hip keep one ring for both operands: at 128
+// rows two thirds of what is in flight is A, and the loop waits out the HBM latency of the rest.  Here
+//   * the operands have rings of their own: half of the waves load A two or three K-steps ahead (L2), the
+//     other half load B as many steps ahead as the 160 KB of LDS hold.  vmcnt retires in order, so one
+//     wave cannot run two depths;
+//   * column tile bx starts its walk of K at step bx % nk and wraps around.  Weight rows are a multiple of
+//     4 KB apart: tiles that walk K in step ask for the same offset of every row, that is for the same
+//     few memory channels (B alone, gate_up of Llama-3-8B: 43.8 -> 36.8 us);
+//   * the second half of a K-step's fragments is read while the first half multiplies, and the next
+//     step's first half while the second does: LDS reads (three quarters of a step's time) and MFMAs
+//     overlap inside a wave;
+//   * a workgroup walks its tiles without draining the rings: the next tile's first K-steps load under
+//     this one's last (lm_head: four tiles per workgroup).
+// Tiles are 256 columns where such tiles fill the chip (A is read half as often), else 128; rows are the
+// batch in steps of 32, two row tiles above 256 rows (side by side on one XCD, so that the second reads
+// the weights from L2); K is split over workgroups where the columns alone are too few.  C^T accumulators
+// (the weights are the MFMA's first operand): a lane holds four neighbouring columns, gate and up of an
+// output sit in one lane, and nothing is staged for the epilogue.
+// Measured (cold weights, us, the LDS-ring tiles -> this kernel): gate_up 28672 x 4096 at 16 / 64 / 100 /
+// 150 / 300 rows 42 -> 37, 49 -> 39, 59 -> 45, 68 -> 51, 134 -> 82; lm_head 128256 x 4096 at 64 / 100 /
+// 150 / 256 / 300 rows 211 -> 168, 247 -> 175, 280 -> 181, 297 -> 251, 548 -> 339; down 4096 x 14336 with
+// its reduce at 100 / 150 / 300 rows 37 -> 34, 46 -> 39, 68 -> 56.
+#include "common.h"
+#include "launch.h"
+
+#include <stdexcept>
+#include <type_traits>
+
+namespace mlop {
+
+namespace {
+
+__device__ __forceinline__ int mid_swz(int r) { return (r >> 1) & 7; }
+
+// s_waitcnt vmcnt(min(n, MAX) * PER) for a wave-uniform n
+template <int MAX, int PER>
+__device__ __forceinline__ void wait_stages(int n) {
+  if constexpr (MAX <= 0) {
+    wait_vmcnt<0>();
+  } else {
+    if (n >= MAX) wait_vmcnt<MAX * PER>();
+    else wait_stages<MAX - 1, PER>(n);
+  }
+}
+
+// Tasks (column tile, row tile, K range), row tile fastest; a workgroup takes lid, lid + G, ...  SA / SB: ring
+// depths in K-steps of 64.  EPI 0: plain (with an activation, RopeEpi::act), 1: gate / up; several K ranges leave
+// fp32 slabs [range][M][N] in ws instead.
+template <int BM, int BN, int WM, int WN, int SA, int SB, int EPI>
+__global__ void __launch_bounds__(WM * WN * 64) gemm_mid_kernel(
+    const uint16_t* __restrict__ A, int lda, const uint16_t* __restrict__ B, int ldb, uint16_t* __restrict__ C, int ldc,
+    float* __restrict__ ws, int M, int N, int K, int k_chunk, int m_tiles, int n_splits, int n_tasks, RopeEpi re) {
+  constexpr int NW = WM * WN, HW = NW / 2;   // half of the waves issue A, half B
+  constexpr int WTM = BM / WM, WTN = BN / WN, TM = WTM / 16, TN = WTN / 16;
+  constexpr int PA = BM / 8 / HW, PB = BN / 8 / HW;  // 1-KiB pieces per issuing wave and K-step
+  static_assert(BM % (8 * HW) == 0 && BN % (8 * HW) == 0 && WTM % 16 == 0 && WTN % 16 == 0, "tile");
+  static_assert((SA - 1) * PA < 64 && (SB - 1) * PB < 64, "vmcnt");
+  extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
+  uint16_t* const ringA = smem;
+  uint16_t* const ringB = smem + SA * BM * 64;
+  const int lane = threadIdx.x & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wid / WN, wn = wid % WN;
+  const int G = gridDim.x, L = blockIdx.x;
+  const int q = G >> 3, rr = G & 7, xcd = L & 7, slot = L >> 3;
+  const int lid = (xcd < rr ? xcd * (q + 1) : rr * (q + 1) + (xcd - rr) * q) + slot;
+  const int gx = (N + BN - 1) / BN;
+  const int nk_all = K / 64, nk_c = k_chunk / 64;
+  auto place = [&](int t, int& bx, int& by, int& bz, int& nk) {
+    by = t % m_tiles;
+    bx = (t / m_tiles) % gx;
+    bz = t / (m_tiles * gx);
+    nk = min(nk_c, nk_all - bz * nk_c);
+  };
+  const bool is_b = wid >= HW;
+  const int iw = is_b ? wid - HW : wid;
+  const bool nt = re.b_nt != 0;
+
+  // load side: K-step i_kt of task i_task is the next to load
+  constexpr int PMAX = PA > PB ? PA : PB;
+  const uint16_t* src[PMAX];
+  int i_task = lid, i_kt = 0, i_nk = 0, i_rot = 0, i_buf = 0;
+  auto set_src = [&]() {
+    int bx, by, bz;
+    place(i_task, bx, by, bz, i_nk);
+    i_rot = bx % i_nk;
+#pragma unroll
+    for (int i = 0; i < PMAX; ++i) {
+      const int r = (iw + HW * i) * 8 + (lane >> 3);
+      const int ch = (lane & 7) ^ mid_swz(r);
+      src[i] = (is_b ? B + (size_t)min(bx * BN + r, N - 1) * ldb : A + (size_t)min(by * BM + r, M - 1) * lda) +
+               bz * k_chunk + ch * 8;
+    }
+  };
+  int total = 0;
+  for (int t = lid; t < n_tasks; t += G) {
+    int bx, by, bz, nk;
+    place(t, bx, by, bz, nk);
+    total += nk;
+  }
+  int issued = 0;
+  auto issue = [&]() {
+    if (issued >= total) return;
+    if (i_kt == i_nk) {
+      i_task += G;
+      i_kt = 0;
+      set_src();
+    }
+    int k = i_kt + i_rot;
+    k = (k >= i_nk ? k - i_nk : k) * 64;
+    if (is_b) {
+      uint16_t* base = ringB + i_buf * (BN * 64);
+      i_buf = i_buf == SB - 1 ? 0 : i_buf + 1;
+#pragma unroll
+      for (int i = 0; i < PB; ++i) {
+        if (nt) __builtin_amdgcn_global_load_lds((const void*)(src[i] + k), (lds_void_t*)(base + (iw + HW * i) * 512), 16, 0, 2);
+        else __builtin_amdgcn_global_load_lds((const void*)(src[i] + k), (lds_void_t*)(base + (iw + HW * i) * 512), 16, 0, 0);
+      }
+    } else {
+      uint16_t* base = ringA + i_buf * (BM * 64);
+      i_buf = i_buf == SA - 1 ? 0 : i_buf + 1;
+#pragma unroll
+      for (int i = 0; i < PA; ++i)
+        __builtin_amdgcn_global_load_lds((const void*)(src[i] + k), (lds_void_t*)(base + (iw + HW * i) * 512), 16, 0, 0);
+    }
+    ++i_kt;
+    ++issued;
+  };
+  set_src();
+  const int depth = is_b ? SB : SA;
+  for (int s = 0; s < depth; ++s) issue();
+
+  f32x4 acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  const int arow = (wm * WTM + (lane & 15)) * 64, brow = (wn * WTN + (lane & 15)) * 64;
+  const int sw = mid_swz(lane & 15), g4 = lane >> 4;
+  const int off0 = (g4 ^ sw) << 3, off1 = ((4 + g4) ^ sw) << 3;
+  bf16x8 fa[2][TM], fb[2][TN];  // fragments of the K-step's two halves
+  int rbufA = 0, rbufB = 0;
+  auto read = [&](auto kk_) {
+    constexpr int kk = decltype(kk_)::value;
+    const uint16_t* sA = ringA + rbufA * (BM * 64) + arow + (kk ? off1 : off0);
+    const uint16_t* sB = ringB + rbufB * (BN * 64) + brow + (kk ? off1 : off0);
+#pragma unroll
+    for (int j = 0; j < TN; ++j) fb[kk][j] = *reinterpret_cast<const bf16x8*>(sB + j * 1024);
+#pragma unroll
+    for (int i = 0; i < TM; ++i) fa[kk][i] = *reinterpret_cast<const bf16x8*>(sA + i * 1024);
+  };
+  auto multiply = [&](auto kk_) {
+    constexpr int kk = decltype(kk_)::value;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) acc[i][j] = mfma16(fb[kk][j], fa[kk][i], acc[i][j]);
+  };
+  using H0 = std::integral_constant<int, 0>;
+  using H1 = std::integral_constant<int, 1>;
+  int c_task = lid, c_kt = 0, c_bx, c_by, c_bz, c_nk;
+  place(c_task, c_bx, c_by, c_bz, c_nk);
+
+  auto epilogue = [&]() {
+    // C^T accumulators: lane holds row i * 16 + (lane & 15), columns j * 16 + 4 g4 + 0..3
+    const int mr = c_by * BM + wm * WTM + (lane & 15), nc = c_bx * BN + wn * WTN + 4 * g4;
+    if (n_splits > 1) {
+      float* P = ws + (size_t)c_bz * M * N;
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        const int m = mr + i * 16;
+        if (m < M) {
+#pragma unroll
+          for (int j = 0; j < TN; ++j) {
+            const int n = nc + j * 16;
+            if (n < N) __builtin_nontemporal_store(acc[i][j], reinterpret_cast<f32x4*>(P + (size_t)m * N + n));
+          }
+        }
+      }
+      return;
+    }
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      const int m = mr + i * 16;
+      if (m >= M) continue;
+      if constexpr (EPI == 0) {
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          const int n = nc + j * 16;
+          if (n >= N) continue;
+          float v[4] = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
+          act_outs(re, v, n);
+          *reinterpret_cast<u32x2*>(C + (size_t)m * ldc + n) = u32x2{pack2(v[0], v[1]), pack2(v[2], v[3])};
+        }
+      } else {
+        static_assert(EPI == 0 || TN % 2 == 0, "gate / up pairs");
+        // (launch_mid_rs: the row's RMSNorm factor first)
+        const float f = re.ss_in != nullptr ? rsqrtf(re.ss_in[m] * re.ss_inv_k + re.ss_eps) : 1.f;
+#pragma unroll
+        for (int j = 0; j < TN; j += 2) {
+          const int n = nc + j * 16;
+          if (n >= N) continue;
+          const f32x4 g = acc[i][j] * f, u = acc[i][j + 1] * f;
+          const int o = (c_bx * BN + wn * WTN + j * 16) / 2 + 4 * g4;
+          *reinterpret_cast<u32x2*>(C + (size_t)m * ldc + o) =
+              u32x2{pack2(glu_out(re, g[0], u[0]), glu_out(re, g[1], u[1])),
+                    pack2(glu_out(re, g[2], u[2]), glu_out(re, g[3], u[3]))};
+        }
+      }
+    }
+  };
+
+  if (is_b) wait_stages<SB - 1, PB>(total - 1);
+  else wait_stages<SA - 1, PA>(total - 1);
+  raw_barrier();
+  read(H0{});
+  for (int s = 0; s < total; ++s) {
+    read(H1{});
+    multiply(H0{});
+    if (s + 1 < total) {
+      if (is_b) wait_stages<SB - 2, PB>(total - 2 - s);
+      else wait_stages<SA - 2, PA>(total - 2 - s);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this wave has step s in registers
+      raw_barrier();                                      // step s + 1 landed; step s's buffers are free
+      issue();
+      rbufA = rbufA == SA - 1 ? 0 : rbufA + 1;
+      rbufB = rbufB == SB - 1 ? 0 : rbufB + 1;
+      read(H0{});
+    }
+    multiply(H1{});
+    if (++c_kt == c_nk) {
+      epilogue();
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      c_kt = 0;
+      c_task += G;
+      if (c_task < n_tasks) place(c_task, c_bx, c_by, c_bz, c_nk);
+    }
+  }
+}
+
+template <int BM, int BN, int WM, int WN, int SA, int SB, int EPI>
+static void run_mid(const uint16_t* A, int lda, const uint16_t* B, int ldb, uint16_t* C, int ldc, float* ws, int M, int N,
+                    int K, int splits, int k_chunk, hipStream_t st, const RopeEpi& re) {
+  constexpr size_t lds = (size_t)(SA * BM + SB * BN) * 128;
+  static_assert(lds <= 163840, "LDS budget");
+  auto kern = gemm_mid_kernel<BM, BN, WM, WN, SA, SB, EPI>;
+  static const bool attr =
+      hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess;
+  (void)attr;
+  const int m_tiles = (M + BM - 1) / BM, gx = (N + BN - 1) / BN;
+  const int tasks = gx * m_tiles * splits;
+  constexpr int per_cu = (int)(163840 / lds) >= 2 ? 2 : 1;
+  RopeEpi r = re;
+  r.b_nt = m_tiles == 1;
+  kern<<<std::min(tasks, 256 * per_cu), WM * WN * 64, lds, st>>>(A, lda, B, ldb, C, ldc, ws, M, N, K, k_chunk, m_tiles,
+                                                                 splits, tasks, r);
+}
+}  // namespace
+
+void launch_mid(int epi, int bm, int bn, const uint16_t* A, int lda, const uint16_t* B, int ldb, uint16_t* C, int ldc,
+                float* ws, int M, int N, int K, int splits, int k_chunk, hipStream_t st, const RopeEpi& re) {
+#define MLOP_MID(m, n, wm, wn, sa, sb)                                                                                  \
+  if (bm == m && bn == n) {                                                                                             \
+    if (epi == 0) return run_mid<m, n, wm, wn, sa, sb, 0>(A, lda, B, ldb, C, ldc, ws, M, N, K, splits, k_chunk, st, re); \
+    return run_mid<m, n, wm, wn, sa, sb, 1>(A, lda, B, ldb, C, ldc, ws, M, N, K, splits, k_chunk, st, re);               \
+  }
+  // ring depths: what fits 160 KB, B before A (64 x 128: half of it, two workgroups per CU)
+  MLOP_MID(64, 128, 2, 4, 2, 4)
+  MLOP_MID(96, 128, 2, 4, 3, 7)
+  MLOP_MID(128, 128, 2, 4, 3, 7)
+  MLOP_MID(160, 128, 2, 4, 3, 6)
+  MLOP_MID(192, 128, 2, 4, 3, 5)
+  MLOP_MID(256, 128, 4, 2, 2, 6)
+  MLOP_MID(64, 256, 2, 4, 3, 4)
+  MLOP_MID(96, 256, 2, 4, 2, 4)
+  MLOP_MID(128, 256, 2, 4, 3, 3)
+  MLOP_MID(160, 256, 2, 4, 3, 3)
+  MLOP_MID(192, 256, 2, 4, 2, 3)
+  MLOP_MID(256, 256, 2, 4, 2, 3)
+#undef MLOP_MID
+  throw std::runtime_error("gemm_mid: no such tile");
+}
+
+}  // namespace mlop

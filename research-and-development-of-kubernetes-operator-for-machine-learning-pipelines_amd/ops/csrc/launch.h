@@ -142,6 +142,9 @@ bool run_w4(int epi, const uint16_t* A, int lda, const uint16_t* B, int ldb, uin
 bool w4_chain_ok(int M, int N, int K);
 bool launch_w4_chain(int epi, const void* A, int lda, const void* B, void* C, int ldc, int M, int N, int K,
                      const RopeEpi& re, hipStream_t st);
+// 5-384 rows, weights in a ring of their own (gemm_mid.hip): tile bm x bn as gemm.hip's mid_plan gives it
+void launch_mid(int epi, int bm, int bn, const uint16_t* A, int lda, const uint16_t* B, int ldb, uint16_t* C, int ldc,
+                float* ws, int M, int N, int K, int splits, int k_chunk, hipStream_t st, const RopeEpi& re);
 int gemm_small_stages(int set);  // LDS-DMA ring depth of the M <= 128 tiles (3, or 5/6)
 int gemm_small_tile(int set);    // M <= 64 tiles: 0 = 64 x 64, 32 / 64 = row-fitted BM x BN
 // non-temporal weight loads of the one-m-tile gemm_kernel launches: bit 0 dense, bit 1 grouped,

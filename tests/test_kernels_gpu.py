@@ -441,6 +441,46 @@ def test_gemm(gpu, M, N, K):
 
 
 @pytest.mark.parametrize("M,N,K,epi", [
+    # 256-column tiles: every row tile, both row counts of each edge, one and two K-steps, a ragged last column tile
+    (1, 49160, 64, 0), (5, 49152, 192, 1), (64, 49160, 128, 0), (65, 49152, 64, 1), (96, 49160, 320, 0), (97, 65600, 64, 0),
+    (128, 49152, 576, 1), (129, 49160, 64, 6), (160, 49160, 320, 8), (161, 49152, 192, 1), (193, 49160, 128, 0), (256, 49152, 192, 1),
+    # two row tiles
+    (257, 24584, 64, 0), (320, 24576, 320, 1), (321, 24584, 192, 0), (384, 24576, 128, 1),
+    # 128-column tiles in one K range
+    (9, 24584, 64, 0), (64, 24576, 1088, 1), (90, 24584, 320, 7), (150, 24576, 640, 1), (192, 24584, 64, 0), (255, 24576, 192, 1), (300, 12296, 320, 0),
+    # K in several ranges, the last one shorter; gate / up and an activation in the reduce
+    (66, 4096, 14336, 0), (100, 6152, 3904, 0), (140, 8200, 2048, 6), (200, 6144, 4096, 1), (256, 4096, 6464, 0), (300, 4128, 4096, 1), (384, 6152, 3200, 0),
+])
+def test_gemm_weight_stream(gpu, M, N, K, epi):
+    """Up to 384 rows on gemm_mid.hip against fp32: one bf16 rounding (two in the gate / up unit: the gate's and the
+    unit's) and fp32 sums in another order; x rows with a stride, three launches alike."""
+    torch.manual_seed(M + N + K)
+    x = torch.randn(M, K + 8, device=gpu, dtype=bf)[:, :K]
+    w = (0.05 * torch.randn(N, K, device=gpu)).to(bf)
+    kw = {"xielu": (0.8, 0.3)} if epi == ops.EPI_XIELU else {}
+    if epi > 1:
+        kw["act_from"] = 128
+    outs = [ops.gemm(x, w, epi=epi, **kw) for _ in range(3)]
+    y = x.float() @ w.float().t()
+    if epi == 1:
+        g, u = ops.deinterleave_cols(y).chunk(2, -1)
+        exp = g * g.sigmoid() * u
+        slack = 4 * 2.0 ** -8 * (g.abs() * u.abs())  # roundings of gate, up and silu(gate), then of the product
+    else:
+        act = {0: lambda v: v, 6: ref.relu2, 7: lambda v: ref.xielu(v, 0.8, 0.3), 8: ref.gelu_tanh}[epi]
+        exp = torch.cat([y[:, :128], act(y[:, 128:])], -1)
+        slack = 2.0 ** -8 * exp.abs()
+    sums = 2.0 ** -20 * (x.float().abs() @ w.float().abs().t())  # fp32 sums: far below K ulp of the terms' magnitudes
+    if epi == 1:
+        sg, su = ops.deinterleave_cols(sums).chunk(2, -1)
+        sums = sg * u.abs() + su * g.abs()
+    elif epi:
+        sums = sums * (1 + 2 * y.abs())
+    assert ((outs[0].float() - exp).abs() <= slack + sums + 1e-6).all()
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+
+
+@pytest.mark.parametrize("M,N,K,epi", [
     (2040, 28672, 4096, 1),   # 896 tiles: 768 data-parallel + 128 tail tiles in 2 halves (gate_up, SiLU)
     (4352, 4096, 14336, 0),   # 272 tiles: 16 tail tiles x 224 K-tiles in 8 ranges (re-read sum path)
     (3072, 6144, 4096, 0),    # 288 tiles: 32 tail tiles in 4 ranges of 16 K-tiles
