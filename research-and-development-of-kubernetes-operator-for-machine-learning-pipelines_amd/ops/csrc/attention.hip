@@ -68,23 +68,84 @@ __device__ __forceinline__ uint32_t vt_base(int lane) {
   const int row = 8 * g4 + q, sw = vswz(row & 15);
   return 256u * row + 16u * ((p >> 1) ^ (sw & 1)) + 8u * (p & 1) + 32u * (sw >> 1);
 }
-__device__ __forceinline__ bf16x8 vt_frag(uint32_t b, int d) {
-  const uint32_t a0 = b ^ (32u * d), a1 = (a0 ^ 16u) + 1024u;
-  const v4s16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s16*)(uintptr_t)a0);
-  const v4s16 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s16*)(uintptr_t)a1);
-  bf16x8 f;
+// the fragments of four dim blocks d..d+3 (b = vt_base ^ 32 d), read and waited for in one statement: the compiler
+// orders LDS reads that it knows of behind every vector memory operation in flight, not only behind the image's DMA
+__device__ __forceinline__ void vt_frag4(uint32_t b, bf16x8 (&f)[4]) {
+  v4s16 r[8];
+  const uint32_t a0 = b, a1 = b ^ 32u, a2 = b ^ 64u, a3 = b ^ 96u;
+  asm volatile(
+      "ds_read_b64_tr_b16 %0, %8\n"
+      "ds_read_b64_tr_b16 %1, %9 offset:1024\n"
+      "ds_read_b64_tr_b16 %2, %10\n"
+      "ds_read_b64_tr_b16 %3, %11 offset:1024\n"
+      "ds_read_b64_tr_b16 %4, %12\n"
+      "ds_read_b64_tr_b16 %5, %13 offset:1024\n"
+      "ds_read_b64_tr_b16 %6, %14\n"
+      "ds_read_b64_tr_b16 %7, %15 offset:1024\n"
+      "s_waitcnt lgkmcnt(0)"
+      : "=&v"(r[0]), "=&v"(r[1]), "=&v"(r[2]), "=&v"(r[3]), "=&v"(r[4]), "=&v"(r[5]), "=&v"(r[6]), "=&v"(r[7])
+      : "v"(a0), "v"(a0 ^ 16u), "v"(a1), "v"(a1 ^ 16u), "v"(a2), "v"(a2 ^ 16u), "v"(a3), "v"(a3 ^ 16u)
+      : "memory");
 #pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    f[e] = lo[e];
-    f[4 + e] = hi[e];
-  }
-  return f;
+  for (int d = 0; d < 4; ++d)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      f[d][e] = r[2 * d][e];
+      f[d][4 + e] = r[2 * d + 1][e];
+    }
 }
 
 __device__ __forceinline__ int wid_of(unsigned t) { return __builtin_amdgcn_readfirstlane((int)(t >> 6)); }
 
+// Keys per partition of one sequence: the launch's nparts shares of its own keys, in page pairs.  A captured decode
+// step plans nparts for the longest context the engine admits; a fixed length cut for that one leaves shorter
+// sequences on a few workgroups (13 sequences of 2500 keys under a limit of 4096: 5 of 8 partitions).
+__device__ __forceinline__ int seq_part(int kv_end, int part_tokens, int nparts) {
+  constexpr int min_part = 128;  // attn_meta.MIN_PART
+  const int even = ((kv_end + nparts - 1) / nparts + 31) & ~31;
+  return nparts > 1 ? min(part_tokens, max(min_part, even)) : part_tokens;
+}
+
+// Row rr, dims c..c+7 of a (tile, kv head)'s combined output from its partitions' slabs.  Four partitions' loads
+// are in flight together: one at a time, 32 partitions were 64 round trips behind each other.
+__device__ __forceinline__ void combine_parts(const float* part_o, const float* part_ml, size_t base, int nvalid, int rr,
+                                              int c, u32x4& ov) {
+  constexpr int U = 4;
+  float M = kNegBig, L = 0.f, a[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  for (int p0 = 0; p0 < nvalid; p0 += U) {
+    float2 ml[U];
+    float4 x[U], y[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {  // past the end: the last partition again, weighted 0
+      const size_t pb = (base + min(p0 + u, nvalid - 1)) * 16 + rr;
+      ml[u] = *reinterpret_cast<const float2*>(part_ml + pb * 2);
+      const float4* po = reinterpret_cast<const float4*>(part_o + pb * kD + c);
+      x[u] = po[0];
+      y[u] = po[1];
+    }
+    float mn = M;
+#pragma unroll
+    for (int u = 0; u < U; ++u) mn = fmaxf(mn, ml[u].x);
+    const float alpha = exp2f(M - mn);
+    M = mn;
+    L *= alpha;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) a[j] *= alpha;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const float f = p0 + u < nvalid ? exp2f(ml[u].x - mn) : 0.f;
+      L += f * ml[u].y;
+      a[0] += f * x[u].x; a[1] += f * x[u].y; a[2] += f * x[u].z; a[3] += f * x[u].w;
+      a[4] += f * y[u].x; a[5] += f * y[u].y; a[6] += f * y[u].z; a[7] += f * y[u].w;
+    }
+  }
+  const float inv = L > 0.f ? 1.f / L : 0.f;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) ov[j] = pack2(a[2 * j] * inv, a[2 * j + 1] * inv);
+}
+
 template <int G, int NT>  // NT bit 0: K / V loads non-temporal, bit 1: the output stores
-__global__ void __launch_bounds__(256) paged_attn_kernel(
+__global__ void __launch_bounds__(256, 3) paged_attn_kernel(
     uint16_t* __restrict__ out, float* __restrict__ part_o, float* __restrict__ part_ml,
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ kc,
     const uint16_t* __restrict__ vc, const int* __restrict__ block_tables, int bt_stride,
@@ -93,8 +154,7 @@ __global__ void __launch_bounds__(256) paged_attn_kernel(
     const int* __restrict__ ctx_len, int Hq, int Hkv, float scale_log2, int part_tokens,
     int nparts, int num_blocks, int* __restrict__ sem) {
   constexpr int QT = 16 / G;
-  // (3 waves per SIMD at 134 VGPRs; forcing 4 (127 VGPRs, amdgpu_waves_per_eu) measured the
-  // same on every decode shape and the headline, scripts/history/r4_occ.sh)
+  // (3 waves per SIMD: 154 VGPRs; asked for two fewer the compiler keeps O in AGPRs and copies it for every rescale)
   // wave w stages its page pair's V image (2 x 16 token rows x 256 B = 8 KB) inside sm_o[w]
   // (8448 B, 256-B aligned: vt_frag), which it alone writes after its loop.  (A second image per
   // wave, prefetching the next pair, measured 1-4 % SLOWER on every decode shape: r04 profile.)
@@ -106,21 +166,17 @@ __global__ void __launch_bounds__(256) paged_attn_kernel(
   const int tile = blockIdx.x, kvh = blockIdx.y, part = blockIdx.z;
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   const int s = tile_seq[tile], q0 = tile_q0[tile];
-  const int p_begin = part * part_tokens;
-  // The wave's first page pair, read as soon as the sequence id is known (clamped into the
-  // row, used only if the pair exists): in the same round trip as ctx_len / q_len instead of
-  // behind them, so the chain to the first K load is tile_seq -> block table -> K.
   const int* bt = block_tables + (size_t)s * bt_stride;
-  const int bt0 = 2 * ((p_begin >> 5) + wid_of(threadIdx.x));
-  const int rawA = bt[min(bt0, bt_stride - 1)], rawB = bt[min(bt0 + 1, bt_stride - 1)];
   const int ql = q_len[s], ctx = ctx_len[s], qs = q_start[s];
   const int last_q = min(q0 + QT, ql) - 1;           // last valid query of the tile
   const int kv_end = last_q >= 0 ? ctx - ql + last_q + 1 : 0;
+  part_tokens = seq_part(kv_end, part_tokens, nparts);
+  const int p_begin = part * part_tokens;
   const int p_end = min(kv_end, p_begin + part_tokens);
-  if (p_begin >= p_end && nparts > 1) {              // reducer skips empty partitions
+  if (p_begin >= p_end) {                            // reducer skips empty partitions
     // kv_end == 0 (graph-bucket padding rows, ctx 0): no partition draws the last ticket of
     // the in-launch combine, so partition 0 writes the zero row attn_reduce_kernel would
-    if (sem != nullptr && part == 0 && kv_end <= 0) {
+    if ((sem != nullptr || nparts == 1) && part == 0 && kv_end <= 0) {
       const int rr = threadIdx.x >> 4, c = (threadIdx.x & 15) * 8;
       const int qi2 = q0 + rr / G;
       if (qi2 < ql)
@@ -160,8 +216,7 @@ __global__ void __launch_bounds__(256) paged_attn_kernel(
   // (a generic pointer's low 32 bits are the LDS offset)
   const uint32_t vimg = (uint32_t)(uintptr_t)&sm_o[0][0][0] + wid * 8448u;
   // clamp: a corrupt block table must not become an out-of-bounds fault
-  auto page_a = [&](int pp) { return min(max(bt[2 * pp], 0), num_blocks - 1); };
-  auto page_b = [&](int pp, int pa) { return (2 * pp + 1 < n_pages) ? min(max(bt[2 * pp + 1], 0), num_blocks - 1) : pa; };
+  auto page_of = [&](int raw) { return min(max(raw, 0), num_blocks - 1); };
   // the pair's 32 token rows of this kv head by LDS-DMA into this wave's V image
   auto issue_v = [&](int pa, int pb) {
     const uint16_t* vA = vc + pa * page_stride + (size_t)kvh * kBS * kD;
@@ -175,19 +230,11 @@ __global__ void __launch_bounds__(256) paged_attn_kernel(
                                        (NT & 1) ? 2 /* nt */ : 0);
     }
   };
-  // page ids one pair ahead: the block-table loads of pair pp + 4 run under pair pp
-  int pgA = 0, pgB = 0;
-  if (pp_begin + wid < pp_end) {
-    pgA = min(max(rawA, 0), num_blocks - 1);
-    pgB = (bt0 + 1 < n_pages) ? min(max(rawB, 0), num_blocks - 1) : pgA;
-  }
-  for (int pp = pp_begin + wid; pp < pp_end; pp += 4) {
-    const uint16_t* kA = kc + pgA * page_stride + (size_t)kvh * kBS * kD;
-    const uint16_t* kB = kc + pgB * page_stride + (size_t)kvh * kBS * kD;
-
-    // K rows of MFMA row r: pair tokens 8*(r>>2) + (r&3) (first S MFMA) and +4 (second)
-    const uint16_t* kR = (r >> 3 ? kB : kA) + (8 * ((r >> 2) & 1) + (r & 3)) * kD;
-    bf16x8 ka[4], kb[4];
+  // K rows of MFMA row r: pair tokens 8*(r>>2) + (r&3) (first S MFMA) and +4 (second)
+  bf16x8 ka[4], kb[4];
+  auto load_k = [&](int pa, int pb) {
+    const uint16_t* kP = kc + (r >> 3 ? pb : pa) * page_stride + (size_t)kvh * kBS * kD;
+    const uint16_t* kR = kP + (8 * ((r >> 2) & 1) + (r & 3)) * kD;
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk) {
       if constexpr ((NT & 1) != 0) {
@@ -198,21 +245,48 @@ __global__ void __launch_bounds__(256) paged_attn_kernel(
         kb[kk] = *reinterpret_cast<const bf16x8*>(kR + 4 * kD + kk * 32 + g4 * 8);
       }
     }
-    // this pair's V image, issued behind the K loads (the S MFMAs wait for those only; the
-    // previous pair's transposed reads are complete: their MFMAs consumed them)
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  };
+  // A pair's K loads (registers) and V image (LDS) are issued a pair ahead: K(p + 4) as soon as the S MFMAs have
+  // taken K(p), V(p + 4) as soon as the transposed reads have taken V(p).  The workgroups of a launch run in step, and
+  // memory stood still while they all multiplied (100 sequences of 1000 keys 96.7 -> 90.2 us, 64 of 4000 217 -> 196).
+  int pgA = 0, pgB = 0, rawA = 0, rawB = 0;  // page ids of the pair whose K is loading; the next pair's as read
+  auto load_pages = [&](int pp) {  // (past the end: entries of the row, never used)
+    rawA = bt[min(2 * pp, bt_stride - 1)];
+    rawB = bt[min(2 * pp + 1, bt_stride - 1)];
+  };
+  auto take_pages = [&](int pp) {
+    pgA = page_of(rawA);
+    pgB = 2 * pp + 1 < n_pages ? page_of(rawB) : pgA;
+  };
+  int pp = pp_begin + wid_of(threadIdx.x);
+  {
+    // (a wave without a pair loads the last one and waits for it: a branch here would make every wait in the loop
+    // one for everything)
+    const int first = min(pp, pp_end - 1);
+    load_pages(first);
+    take_pages(first);
+    load_k(pgA, pgB);
+    asm volatile("" ::: "memory");
+    load_pages(pp + 4);
+    asm volatile("" ::: "memory");
     issue_v(pgA, pgB);
-    if (pp + 4 < pp_end) {
-      pgA = page_a(pp + 4);
-      pgB = page_b(pp + 4, pgA);
-    }
-    bf16x8 vf8[8];
+  }
+  auto pair = [&](auto more_) {
+    constexpr bool more = decltype(more_)::value;
     // S^T[token][row]: lane holds row r, tokens 4*g4 + i of each page
     f32x4 sa = {0.f, 0.f, 0.f, 0.f}, sb = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk) {
       sa = mfma16(ka[kk], qf[kk], sa);
       sb = mfma16(kb[kk], qf[kk], sb);
+    }
+    asm volatile("" : "+v"(sa), "+v"(sb)::"memory");  // the next K loads stay behind the MFMAs that read this pair's
+    if constexpr (more) {
+      take_pages(pp + 4);
+      load_k(pgA, pgB);
+      asm volatile("" ::: "memory");
+      load_pages(pp + 8);
+      asm volatile("" ::: "memory");
     }
     const int tokA = pp * 32 + g4 * 8, tokB = tokA + 4;
     float pa[4], pb[4];
@@ -242,19 +316,27 @@ __global__ void __launch_bounds__(256) paged_attn_kernel(
       pf[i] = (short)f2bf(pa[i]);
       pf[4 + i] = (short)f2bf(pb[i]);
     }
-    {
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's V image has landed
-      uint32_t b0 = vimg + vt_base(lane);
-      asm volatile("" : "+v"(b0));  // no hoisting of the 16 read addresses out of the loop
+    // this wave's V image has landed: at least the eight K loads are younger
+    if constexpr (more) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    const uint32_t b0 = vimg + vt_base(lane);
 #pragma unroll
-      for (int d = 0; d < 8; ++d) vf8[d] = vt_frag(b0, d);
-    }
+    for (int h = 0; h < 2; ++h) {
+      bf16x8 vf[4];
+      vt_frag4(b0 ^ (128u * h), vf);
+      if constexpr (more) {
+        if (h == 1) issue_v(pgA, pgB);  // the image is in registers
+      }
 #pragma unroll
-    for (int d = 0; d < 8; ++d) {
-      o[d] *= alpha;
-      o[d] = mfma16(vf8[d], pf, o[d]);
+      for (int d = 0; d < 4; ++d) {
+        o[4 * h + d] *= alpha;
+        o[4 * h + d] = mfma16(vf[d], pf, o[4 * h + d]);
+      }
     }
-  }
+  };
+  for (; pp + 4 < pp_end; pp += 4) pair(std::true_type{});
+  if (pp < pp_end) pair(std::false_type{});
+  else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
   l = sum_x16_x32(l);
   // O^T[d][row]: lane holds row r, dims 16*dblk + 4*g4 + i
@@ -340,22 +422,8 @@ __global__ void __launch_bounds__(256) paged_attn_kernel(
   __syncthreads();
   if (!row_valid) return;
   const size_t base = ((size_t)tile * Hkv + kvh) * nparts;
-  float MM = kNegBig;
-  for (int p = 0; p < nvalid; ++p) MM = fmaxf(MM, part_ml[((base + p) * 16 + rr) * 2]);
-  float LL = 0.f, a2[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  for (int p = 0; p < nvalid; ++p) {
-    const size_t pb = (base + p) * 16 + rr;
-    const float f = exp2f(part_ml[pb * 2] - MM);
-    LL += f * part_ml[pb * 2 + 1];
-    const float4* po = reinterpret_cast<const float4*>(part_o + pb * kD + c);
-    const float4 x0 = po[0], x1 = po[1];
-    a2[0] += f * x0.x; a2[1] += f * x0.y; a2[2] += f * x0.z; a2[3] += f * x0.w;
-    a2[4] += f * x1.x; a2[5] += f * x1.y; a2[6] += f * x1.z; a2[7] += f * x1.w;
-  }
-  const float inv = LL > 0.f ? 1.f / LL : 0.f;
   u32x4 ov;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) ov[j] = pack2(a2[2 * j] * inv, a2[2 * j + 1] * inv);
+  combine_parts(part_o, part_ml, base, nvalid, rr, c, ov);
   *reinterpret_cast<u32x4*>(out + ((size_t)(qs + qi2) * Hq + head2) * kD + c) = ov;
 }
 
@@ -372,27 +440,14 @@ __global__ void __launch_bounds__(256) attn_reduce_kernel(
   const int ql = q_len[s], ctx = ctx_len[s], qs = q_start[s];
   const int last_q = min(q0 + QT, ql) - 1;
   const int kv_end = last_q >= 0 ? ctx - ql + last_q + 1 : 0;
+  part_tokens = seq_part(kv_end, part_tokens, nparts);
   const int nvalid = min(nparts, (kv_end + part_tokens - 1) / part_tokens);
   const int rr = threadIdx.x >> 4, c = (threadIdx.x & 15) * 8;
   const int qi = q0 + rr / G;
   if (qi >= ql) return;
   const size_t base = ((size_t)tile * Hkv + kvh) * nparts;
-  float M = kNegBig;
-  for (int p = 0; p < nvalid; ++p) M = fmaxf(M, part_ml[((base + p) * 16 + rr) * 2]);
-  float L = 0.f, acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  for (int p = 0; p < nvalid; ++p) {
-    const size_t pb = (base + p) * 16 + rr;
-    const float f = exp2f(part_ml[pb * 2] - M);
-    L += f * part_ml[pb * 2 + 1];
-    const float4* po = reinterpret_cast<const float4*>(part_o + pb * kD + c);
-    float4 a = po[0], b = po[1];
-    acc[0] += f * a.x; acc[1] += f * a.y; acc[2] += f * a.z; acc[3] += f * a.w;
-    acc[4] += f * b.x; acc[5] += f * b.y; acc[6] += f * b.z; acc[7] += f * b.w;
-  }
-  const float inv = L > 0.f ? 1.f / L : 0.f;
   u32x4 ov;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) ov[j] = pack2(acc[2 * j] * inv, acc[2 * j + 1] * inv);
+  combine_parts(part_o, part_ml, base, nvalid, rr, c, ov);
   const int head = kvh * G + (rr % G);
   *reinterpret_cast<u32x4*>(out + ((size_t)(qs + qi) * Hq + head) * kD + c) = ov;
 }
@@ -406,12 +461,23 @@ int attn_kv_nt(int set) {
   return g_attn_kv_nt;
 }
 
+// Workgroups from which a launch takes no further partitions: one per CU.  A partition more costs its slab, a ticket
+// and its share of the combine; the metadata plans up to four per CU, with which 1 x 24000 keys took 47 us (27.6 with
+// 32 partitions), 3 x 24000 64 (58), 7 x 1000 14.1 (12.2), 13 x 2500 34.6 (35.1), 20 x 800 23.9 (22.4).
+constexpr int kAttnWgs = 256;
+
 template <int G>
 static void launch_g(void* out, float* part_o, float* part_ml, const void* q, const void* kc,
                      const void* vc, const int* bt, int bt_stride, const int* tile_seq,
                      const int* tile_q0, const int* q_start, const int* q_len, const int* ctx_len,
                      int num_tiles, int Hq, int Hkv, float scale_log2, int part_tokens, int nparts,
                      int num_blocks, int* sem, hipStream_t st) {
+  const int base = num_tiles * Hkv;
+  const int want = std::max(1, (kAttnWgs + base - 1) / base);
+  if (nparts > want) {
+    part_tokens = ((part_tokens * nparts + want - 1) / want + 31) / 32 * 32;
+    nparts = want;
+  }
   dim3 grid(num_tiles, Hkv, nparts);
   // K / V pages non-temporal (attn_kv_nt op): each is read once per step by one workgroup
   // (below 8 query tiles the default policy: batch 4 lost 0.7 % with it, batch 16 gained 1.8 %)

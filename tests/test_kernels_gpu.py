@@ -258,6 +258,27 @@ def test_paged_attention(gpu, Hq, Hkv, case, attn_fused_all):
     close(out, exp, atol=2e-2, rtol=2e-2)
 
 
+@pytest.mark.parametrize("Hq,Hkv,part_tokens,nparts", [(4, 1, 128, 64), (8, 1, 512, 9), (32, 8, 4096, 2), (32, 8, 1024, 32), (16, 16, 160, 40)])
+def test_paged_attention_partitions_of_a_longer_limit(gpu, Hq, Hkv, part_tokens, nparts, attn_fused_all):
+    """Partitions planned for a longer context than any sequence has (a captured decode step): every sequence cuts its
+    own keys.  Lengths around a page pair, a wave's share and a partition's minimum, beside padding rows."""
+    torch.manual_seed(0)
+    np.random.seed(0)
+    ctx_lens = [1, 31, 32, 33, 127, 128, 129, 257, 513, 1000, 1025, 0, 0]
+    NB = sum((c + 15) // 16 for c in ctx_lens) + 8
+    kc = torch.randn(NB, Hkv, 16, 128, device=gpu, dtype=bf)
+    vc = torch.randn(NB, Hkv, 16, 128, device=gpu, dtype=bf)
+    m, T = make_meta(gpu, [1] * len(ctx_lens), ctx_lens, Hkv, Hq // Hkv, NB, part_tokens=part_tokens, nparts=nparts)
+    m.part_sem = torch.zeros(m.tile_seq.numel() * Hkv, dtype=torch.int32, device=gpu)
+    q = torch.randn(T, Hq, 128, device=gpu, dtype=bf)
+    exp = ref.paged_attention(q, kc, vc, m)
+    for _ in range(3):
+        out = torch.full_like(q, float("nan"))
+        ops.paged_attention(q, kc, vc, m, out=out)
+        close(out, exp, atol=2e-2, rtol=2e-2)
+        assert (out[-2:] == 0).all() and int(m.part_sem.abs().sum()) == 0
+
+
 @pytest.mark.parametrize("fused", [False, True])
 def test_paged_attention_padded_bucket(gpu, fused, attn_fused_all):
     """Graph-bucket padding rows (q_len 1, ctx 0) under forced split-KV: both combine
