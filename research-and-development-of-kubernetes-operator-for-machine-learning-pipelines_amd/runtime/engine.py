@@ -712,6 +712,7 @@ class Engine:
         return outs
 
     def _prefill_step(self):
+        self._wait_meta()
         batch, chunks = self._collect_prefill(self.cfg.max_num_batched_tokens)
         if not batch:
             return None
@@ -742,6 +743,7 @@ class Engine:
         separate M=B pass; the ragged paged-attention kernel takes both kinds
         of tile.  Returns None (caller decodes alone) when nothing fits."""
         t0 = time.perf_counter()
+        self._wait_meta()
         rows, ctx_d = self._decode_rows()
         B = len(rows)
         budget = self.cfg.max_num_batched_tokens - B
@@ -1072,6 +1074,7 @@ class Engine:
 
     def _decode_step(self):
         t0 = time.perf_counter()
+        self._wait_meta()
         rows, ctx = self._decode_rows()
         B = len(rows)
         if B == 0:
@@ -1238,7 +1241,12 @@ class Engine:
         idx = [at[s.seq_id] + (j if len(toks) > 1 else 0) for s, toks, want in live for j in range(len(want))]
         if not idx:
             return None
-        return logits[torch.tensor(idx, device=logits.device)]
+        # the device is not waited for: a caller may feed the next step while this one runs
+        if self.model.ps.tp.size == 1 and idx == list(range(len(idx))):
+            rows = logits[:len(idx)]
+            return rows if portions or self.graphs.get(bucket) is None else rows.clone()  # (a graph's buffer is its own)
+        at_d = torch.tensor(idx, pin_memory=logits.is_cuda).to(logits.device, non_blocking=True)
+        return logits[at_d]
 
     # --------------------------------------------------------- execution --
     def _launch(self, kind: int, T: int, nt: int, nl: int, part: int, nparts: int, bucket: int,
@@ -1270,7 +1278,7 @@ class Engine:
             self.step_sync.send(self, kind, T, nt, nl, part, nparts, bucket, npt, int(greedy))
             self.stats["tp_sync_us"] += int(1e6 * (time.perf_counter() - t0))
             self.stats["tp_sync_calls"] += 1
-        if self._async and self.device.type == "cuda":
+        if self.device.type == "cuda":
             self._meta_ev = torch.cuda.Event()
             self._meta_ev.record()
         return self._execute(kind, T, nt, nl, part, nparts, bucket, npt, greedy)

@@ -147,3 +147,39 @@ def test_kernel_time_sampler_on_engine_steps(gpu, graphs, async_reduce):
     assert s.host_ms and s.warm_ms is not None
     assert abs(sum(sh.values()) - 1.0) < 1e-6
     assert sh.get("gemm", 0) > 0 and sh.get("attention", 0) > 0, sh
+
+
+@pytest.mark.parametrize("async_scheduling", [True, False])
+def test_feed_does_not_wait(gpu, async_scheduling):
+    """Steps fed one behind the other, without a look at the device between them (graph steps, prompts, both at once,
+    wanted rows out of order, none wanted), then a generation: every result as when each step is waited for."""
+    from mlopamd.models import build_model
+
+    cfg = get_config("tiny-llama")
+
+    def run(wait):
+        eng = Engine(build_model(cfg, device=gpu, seed=3),
+                     EngineConfig(max_num_seqs=8, max_num_batched_tokens=512, max_model_len=512, num_kv_blocks=200,
+                                  graph_buckets=(1, 4), enable_prefix_caching=False, async_scheduling=async_scheduling))
+        a, b, c = (eng.open_sequence() for _ in range(3))
+        steps = [[(a, list(range(20, 320)), [299])], [(b, list(range(40, 60)), [5, 19, 2]), (a, [7], [0])], [(a, [9], [0]), (b, [11], [0])],
+                 [(b, [3], []), (a, [5], [0])], [(c, list(range(90, 300)), [])], [(a, [8], [0]), (b, [9], [0]), (c, [10], [0])]]
+        outs = []
+        for s in steps:
+            outs.append(eng.feed(s))
+            if wait:
+                torch.cuda.synchronize()
+        for k in range(40):  # one graph step behind the other
+            outs.append(eng.feed([(a, [10 + k], [0]), (c, [30 + k], [0])]))
+            if wait:
+                torch.cuda.synchronize()
+        for s in (a, b, c):
+            eng.close_sequence(s)
+        toks = eng.generate([[5, 6, 7, 8] * 20, [9, 10, 11]], SamplingParams(max_tokens=6, ignore_eos=True))
+        torch.cuda.synchronize()
+        return outs, toks
+
+    (x, tx), (y, ty) = run(True), run(False)
+    assert [o is None for o in x] == [o is None for o in y] and tx == ty
+    for p, q in zip(x, y):
+        assert p is None or torch.equal(p, q)
