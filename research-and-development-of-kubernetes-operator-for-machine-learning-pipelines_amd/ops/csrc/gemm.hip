@@ -258,7 +258,11 @@ __global__ void __launch_bounds__(WM * WN * 64) gemm_kernel(
   }
   // weight pieces non-temporal when re.b_nt (wave-uniform: a piece is A or B by its index)
   const bool b_nt = re.b_nt != 0;
+  // experts: column tile bx walks K from step bx % nk on (the channels of tiles in step: gemm_mid.hip; down of eight
+  // experts at 20 rows 145 -> 140 us).  Dense split-K ranges are too short for it (qkv 17.5 -> 17.8)
+  const int rot = GROUPED ? bx % nk : 0;
   auto issue = [&](int buf, int kt) {
+    kt = kt + rot >= nk ? kt + rot - nk : kt + rot;
     uint16_t* base = smem + buf * STAGE;
 #pragma unroll
     for (int i = 0; i < PPW; ++i) {
