@@ -631,6 +631,8 @@ void gemm_dense_plan(int variant, int bm, int bn, int splits, int stages) {
     for (const auto& t : ok) found = found || (t[0] == bm && t[1] == bn);
     if (!found) throw std::runtime_error("gemm_dense_plan: no dense config for this tile");
   }
+  if (variant == 6 && bm > 0 && bm != 128 && bm != 160 && bm != 192)
+    throw std::runtime_error("gemm_dense_plan: four-wave tiles between are 128, 160 or 192 rows");
   g_dp[0] = variant, g_dp[1] = bm, g_dp[2] = bn, g_dp[3] = splits, g_dp[4] = stages > 0 ? stages : 0;
 }
 
@@ -1348,18 +1350,60 @@ static bool mid_plan(int M, int N, int K, Plan& p) {
   constexpr int max_m = 384, fill = 192;
   if (M > max_m || K % kBK || N % 8) return false;
   const int m_tiles = M <= 256 ? 1 : 2, rows = (M + m_tiles - 1) / m_tiles;
-  const int bm = rows <= 64 ? 64 : rows <= 192 ? (rows + 31) / 32 * 32 : 256;
+  const int bm = rows <= 64 ? 64 : (rows + 31) / 32 * 32;
   const int t256 = (N + 255) / 256 * m_tiles, t128 = (N + 127) / 128 * m_tiles, nk = K / kBK;
   int s = 1;
   if (t256 < fill && t128 < fill) {
     s = std::min({kMaxSplits, 256 / t128, nk / 12});
     if (M <= 64 || t128 * s < fill) return false;
+    // where the 64-column tiles need no K ranges, the slabs have to be small beside the weights (12544 x 2048 in two
+    // ranges at 100 / 200 rows: 22 / 31 us against 20 / 24; 10240 x 8192 in three: 42 against 65)
+    if ((N + 63) / 64 >= 160 && 4l * s * M > K * 3l / 10) return false;
   }
   p.variant = 7;
   p.BM = bm;
   p.BN = t256 >= fill ? 256 : 128;
   p.k_chunk = (nk + s - 1) / s * kBK;
   p.splits = (K + p.k_chunk - 1) / p.k_chunk;
+  return true;
+}
+
+// Above the weight stream's rows: the four-wave kernel's tile height, or the ping-pong kernel with its stream-K tail,
+// by estimated time in us.  A round of 256-row tiles takes 5.6 + 0.0212 K; lower tiles cost more per row (192 rows 0.80
+// of it, 160 0.725, 128 0.61: fewer MFMAs per fragment read), and an only round that fills a share f of the CUs runs
+// faster, the less the lower the tile.  A tail of at most half the CUs is cut into K-halves: half a round and the
+// hand-off of the partials (behind whole rounds the more the more of them there are).  The ping-pong kernel cuts every tile of a grid of up to half the CUs, runs a round as it
+// is above that, and spreads the remainder of several evenly at 1.08 of a round's rate.
+// Constants fitted to qkv, o, gate_up, down and lm_head of Llama-3-8B at 17 row counts from 400 to 4096, every variant
+// measured: the choice is within 5 % of the best of the five at all of them.  Against the earlier rule (heights 256 and
+// 128 only): gate_up at M = 400 / 700 / 1152 138 -> 92, 158 -> 147, 245 -> 219 us, o at 1152 / 2300 / 2600 55 -> 43,
+// 79 -> 62, 83 -> 68, down at 600 / 1500 / 2300 102 -> 88, 150 -> 135, 253 -> 213, qkv at 700 / 1500 / 2600 53 -> 43,
+// 79 -> 63, 132 -> 111, lm_head at 400 558 -> 394.
+static bool big_plan(int M, int N, int K, bool pp_ok, Plan& p) {
+  const SkBuf* b = sk_buf();
+  if (!b || !gemm_w4_ok(M, N, K, K, K)) return false;
+  struct Tile { int rows; float round, slope; };
+  constexpr Tile tiles[] = {{256, 1.f, .55f}, {192, .80f, .55f}, {160, .725f, .35f}, {128, .61f, .10f}};
+  const float full = 5.6f + 0.0212f * (float)K, C = (float)b->cus;
+  const float f = (float)((M + 255) / 256) * (float)(N / 256) / C;  // rounds of 256-row tiles
+  float best = !pp_ok ? 1e30f : f <= .5f ? .87f * full * f + 28.f + .06f * full : f <= 1.f ? 1.11f * full * (.5f + .5f * f) : 1.08f * full * f + 25.f;
+  p.variant = 3;
+  p.BM = p.BN = 256;
+  for (const Tile& t : tiles) {
+    if (t.rows < 256 && !g_half_tile) break;
+    const long T = (long)((M + t.rows - 1) / t.rows) * (N / 256), q = T / b->cus, r = T % b->cus;
+    const float one = full * t.round;
+    float us = (float)q * one;
+    const bool halves = r > 0 && gemm_w4_split_ok((int)T, K / kBK);
+    const float fill = (halves ? 2.f : 1.f) * (float)r / C, slope = q > 0 ? 0.f : t.slope;
+    if (r > 0) us += (halves ? .5f : 1.f) * one * (1.f - slope * (1.f - fill));
+    if (halves) us += q > 0 ? std::max(0.f, 28.f * fill - 5.f) : 9.f + .1f * (float)(t.rows - 128);
+    if (us < best) {
+      best = us;
+      p.variant = t.rows == 256 ? 5 : 6;
+      p.BM = t.rows;
+    }
+  }
   return true;
 }
 
@@ -1447,14 +1491,19 @@ static Plan plan(int M, int N, int K, bool grouped, int n_groups, int rows_per_g
     // 114.7 vs 129.5); from 72 tiles (qkv at M = 768, 70B qkv at 512) the large-M kernels win.
     constexpr int wide_min_m = 512;
     constexpr int mid_tiles = 72;
+    // Fewer than 64 half-height tiles leave most CUs idle whatever the tile: the split-K tiles (variant 0).  So does
+    // long K on a narrow N at up to 512 rows (down at M = 400 / 512 70.9 / 72.8 us, the best of big_plan's 72.5 / 80).
+    const bool by_time = !grouped && big == 5 && (long)((M + 127) / 128) * (N / 256) >= 64 &&
+                         !(K >= 8192 && M <= 512 && t256 < mid_tiles) && big_plan(M, N, K, pp_ok, p);
     const int big_from = t256 >= mid_tiles ? std::min(big_min_m, wide_min_m) : std::max(big_min_m, 2048);
-    if (big == 5 && !(mrows >= big_from && !grouped && w4_fills && gemm_w4_ok(M, N, K, K, K))) {
+    if (by_time) {
+    } else if (big == 5 && !(mrows >= big_from && !grouped && w4_fills && gemm_w4_ok(M, N, K, K, K))) {
       if (mrows >= big_from && !grouped && pp_ok) { p.BN = 256; p.variant = 3; }
     } else if (big && mrows >= big_from && !grouped && (big < 3 || pp_ok)) {
       p.BN = 256;
       p.variant = big;
     }
-    if (!grouped && big == 5) {
+    if (!grouped && big == 5 && !by_time) {
       // long-K narrow projections (down, K = 14336) at 40-71 tiles of 256 x 256 (M 640-1279):
       // the ping-pong kernel's stream-K tail spreads the few tiles' K over every CU (down at
       // M = 768: 105 -> 90 us, 1024: 118 -> 108; hipBLASLt 90 / 111)
@@ -1463,32 +1512,11 @@ static Plan plan(int M, int N, int K, bool grouped, int n_groups, int rows_per_g
         p.BN = 256;
         p.variant = 3;
       }
-      // four-wave vs ping-pong past one full round: the four-wave kernel runs whole rounds of
-      // 256 x 256 tiles (a tail of r <= CUs / 2 tiles in K-halves), the ping-pong kernel ~7 %
-      // slower per tile but with a stream-K tail that balances ANY remainder.  Estimated time in
-      // four-wave tile rounds: w4 = q + (r ? (2r <= C ? 0.55 : 1) : 0), pp = 1.08 T / C + 0.05.
-      // (M = 4608: o 147 -> 134 us, down 476 -> 403, qkv 181 -> 172; the headline's M ~ 4088 is
-      // whole rounds for every projection and stays on the four-wave kernel; bench_mid_m.py)
+      // the half-height four-wave tile with its own K-half tail (t128 <= CUs / 2); below ~80 tiles the 256 x 128
+      // split-K kernel wins (down at M = 512: 83.1 vs 67.6)
       const SkBuf* b = sk_buf();
-      if (p.variant == 5 && b && t256 > b->cus && pp_ok) {
-        const long C = b->cus, q = t256 / C, r = t256 % C;
-        const float w4_est = (float)q + (r == 0 ? 0.f : (2 * r <= C ? 0.55f : 1.f));
-        const float pp_est = 1.08f * (float)t256 / (float)C + 0.05f;
-        if (pp_est < w4_est - 0.03f) p.variant = 3;
-      }
-      // variant 6, the half-height (128 x 256) four-wave tile, where its grid is at most one
-      // round: up to twice the workgroups of the 256 x 256 grid (a lone tile of either height
-      // runs ~1.8x faster than one in a full round, so idle CUs cost more than the half tile's
-      // lower MFMA density).  bench_mid_m.py (profiles/r05_gemm_w4h.md), planner before -> after:
-      // o at M = 1024 / 1536 / 2048 46.2 -> 38.3 / 56.0 -> 47.6 / 65.6 -> 55.2 us, qkv at 384 /
-      // 512 / 1024 43.1 -> 33.1 / 44.4 -> 35.3 / 56.0 -> 47.5; past one round it loses to the
-      // full tile (qkv 1408: 75.9 vs 72.3).  Long K (down): only with its own K-half tail
-      // (t128 <= CUs / 2: 96 -> 256 items, M = 1024 110.8 -> 98.5); without it the full tile's
-      // K-halves win (M = 1152: 153.7 vs 131.1), and below ~80 tiles the 256 x 128 split-K kernel
-      // (M = 512: 83.1 vs 67.6).
       const long t128 = (long)((M + 127) / 128) * ((N + 255) / 256);
-      const bool long_k = K >= 8192;
-      if (g_half_tile && b && mrows >= 384 && (long_k ? t128 >= 80 && 2 * t128 <= b->cus : t128 >= 64 && t128 <= b->cus) &&
+      if (g_half_tile && b && mrows >= 384 && K >= 8192 && t128 >= 80 && 2 * t128 <= b->cus &&
           (p.variant == 0 || p.variant == 3 || p.variant == 5) && gemm_w4_ok(M, N, K, K, K)) {
         p.BM = 128;
         p.BN = 256;
@@ -1498,7 +1526,7 @@ static Plan plan(int M, int N, int K, bool grouped, int n_groups, int rows_per_g
   }
   if (!grouped && g_dp[0] >= 0) {  // bench override (gemm_dense_plan)
     p.variant = g_dp[0];
-    p.BM = p.variant == 0 ? g_dp[1] : p.variant == 6 ? 128 : 256;
+    p.BM = p.variant == 0 || (p.variant == 6 && g_dp[1] > 0) ? g_dp[1] : p.variant == 6 ? 128 : 256;
     p.BN = p.variant == 0 ? g_dp[2] : 256;
     p.stages = g_dp[4];
   }
@@ -1556,7 +1584,7 @@ static void launch_plan(const Plan& p, const uint16_t* A, int lda, const uint16_
     if (!GROUPED && p.variant == 7)
       launch_mid(EPI, p.BM, p.BN, A, lda, B, ldb, C, ldc, ws, M, N, K, p.splits, p.k_chunk, st, re);
     else if (!GROUPED && p.variant == 6 && p.splits == 1 && gemm_w4_ok(M, N, K, lda, ldb, ldc))
-      run_w4(EPI, A, lda, B, ldb, C, ldc, M, N, K, st, re, 128);
+      run_w4(EPI, A, lda, B, ldb, C, ldc, M, N, K, st, re, p.BM);
     else if (!GROUPED && p.variant == 6) run_pp<EPI>(A, lda, B, ldb, C, ldc, M, N, K, st, re);
     else if (p.BM == 16 && p.BN == 32 && sst >= 8) MLOP_GEMM(16, 32, 1, 2, 8, false);
     else if (p.BM == 16 && p.BN == 32 && sst >= 6) MLOP_GEMM(16, 32, 1, 2, 6, false);

@@ -279,12 +279,14 @@ void launch_mid(int epi, int bm, int bn, const uint16_t* A, int lda, const uint1
   MLOP_MID(128, 128, 2, 4, 3, 7)
   MLOP_MID(160, 128, 2, 4, 3, 6)
   MLOP_MID(192, 128, 2, 4, 3, 5)
+  MLOP_MID(224, 128, 2, 4, 2, 6)
   MLOP_MID(256, 128, 4, 2, 2, 6)
   MLOP_MID(64, 256, 2, 4, 3, 4)
   MLOP_MID(96, 256, 2, 4, 2, 4)
   MLOP_MID(128, 256, 2, 4, 3, 3)
   MLOP_MID(160, 256, 2, 4, 3, 3)
   MLOP_MID(192, 256, 2, 4, 2, 3)
+  MLOP_MID(224, 256, 2, 4, 2, 3)
   MLOP_MID(256, 256, 2, 4, 2, 3)
 #undef MLOP_MID
   throw std::runtime_error("gemm_mid: no such tile");

@@ -13,7 +13,9 @@
 // fragments of tile t in registers, so one buffer pair keeps a whole tile in flight.
 // BMT = 128 is the half-height tile (planner variant 6, grids of at most one round): 64 x 128
 // outputs per wave (a[0:127]), 12 DMA pieces per K-tile, its own generated loop
-// (MLOP_W4H_KLOOP_*, 64 MFMAs per K-tile), every epilogue shared with the full tile.
+// (MLOP_W4H_KLOOP_*, 64 MFMAs per K-tile), every epilogue shared with the full tile.  BMT = 160 and 192
+// (80 and 96 output rows per wave, loops MLOP_W4_160_* / _192_*) stand between them for grids that both fill
+// badly: whole rounds take 0.725 and 0.80 of the full tile's (gemm.hip big_plan has the choice and its figures).
 //
 // HIP handles the rest: tile placement (XCD-contiguous bands, as gemm_pp_kernel), per-lane
 // DMA source offsets (rows clamped to the last valid row, XOR swizzle in the source), the
@@ -87,7 +89,7 @@ __global__ void __launch_bounds__(256, 1) gemm_w4_kernel(
   // BMT = 256: 128 x 128 outputs per wave; BMT = 128 (the half-height tile, twice the tiles for
   // the mid-M and QKV grids): 64 x 128 per wave, 4 x 8 accumulators, 12 DMA pieces per K-tile
   constexpr int BM = BMT, BN = 256;
-  static_assert(BMT == 256 || BMT == 128, "tile heights of the generated K-loops");
+  static_assert(BMT == 256 || BMT == 192 || BMT == 160 || BMT == 128, "tile heights of the generated K-loops");
   constexpr int NI = BMT / 32;      // 16-row accumulator blocks per wave
   constexpr int NPC = NI + 8;       // DMA pieces per wave and K-tile (NI of A, 8 of B)
   // epilogue store instructions per wave and tile (the next tile's K-loop waits for its
@@ -245,6 +247,42 @@ __global__ void __launch_bounds__(256, 1) gemm_w4_kernel(
     [vn10] "v"(vn[10]), [vn11] "v"(vn[11]), [srdA] "s"(srdA), [srdB] "s"(srdB), [k128] "s"(k128),               \
     [first] "s"(s_first), [has_next] "s"(s_next)                                                                 \
   : "memory", "scc", MLOP_W4_AGPR_CLOBBERS
+// 160 rows: A fragments 0-4, DMA pieces 0-12
+#define MLOP_W4_160_OPERANDS                                                                                    \
+  : [fa0_0] "=&v"(fa0_0), [fa0_1] "=&v"(fa0_1), [fa0_2] "=&v"(fa0_2), [fa0_3] "=&v"(fa0_3),                     \
+    [fa0_4] "=&v"(fa0_4), [fb0_0] "=&v"(fb0_0), [fb0_1] "=&v"(fb0_1), [fb0_2] "=&v"(fb0_2),                     \
+    [fb0_3] "=&v"(fb0_3), [fb0_4] "=&v"(fb0_4), [fb0_5] "=&v"(fb0_5), [fb0_6] "=&v"(fb0_6),                     \
+    [fb0_7] "=&v"(fb0_7), [fa1_0] "=&v"(fa1_0), [fa1_1] "=&v"(fa1_1), [fa1_2] "=&v"(fa1_2),                     \
+    [fa1_3] "=&v"(fa1_3), [fa1_4] "=&v"(fa1_4), [fb1_0] "=&v"(fb1_0), [fb1_1] "=&v"(fb1_1),                     \
+    [fb1_2] "=&v"(fb1_2), [fb1_3] "=&v"(fb1_3), [fb1_4] "=&v"(fb1_4), [fb1_5] "=&v"(fb1_5),                     \
+    [fb1_6] "=&v"(fb1_6), [fb1_7] "=&v"(fb1_7), [rA0] "+v"(rA0), [rA1] "+v"(rA1), [rB0] "+v"(rB0),              \
+    [rB1] "+v"(rB1), [koff] "+s"(koff), [dbase] "+s"(dbase), [iter] "+s"(iter), [m0save] "=&s"(m0save)          \
+  : [vo0] "v"(vo[0]), [vo1] "v"(vo[1]), [vo2] "v"(vo[2]), [vo3] "v"(vo[3]), [vo4] "v"(vo[4]), [vo5] "v"(vo[5]), \
+    [vo6] "v"(vo[6]), [vo7] "v"(vo[7]), [vo8] "v"(vo[8]), [vo9] "v"(vo[9]), [vo10] "v"(vo[10]),                 \
+    [vo11] "v"(vo[11]), [vo12] "v"(vo[12]), [vn0] "v"(vn[0]), [vn1] "v"(vn[1]), [vn2] "v"(vn[2]),               \
+    [vn3] "v"(vn[3]), [vn4] "v"(vn[4]), [vn5] "v"(vn[5]), [vn6] "v"(vn[6]), [vn7] "v"(vn[7]), [vn8] "v"(vn[8]), \
+    [vn9] "v"(vn[9]), [vn10] "v"(vn[10]), [vn11] "v"(vn[11]), [vn12] "v"(vn[12]), [srdA] "s"(srdA),             \
+    [srdB] "s"(srdB), [k128] "s"(k128), [first] "s"(s_first), [has_next] "s"(s_next)                            \
+  : "memory", "scc", MLOP_W4_AGPR_CLOBBERS
+// 192 rows: A fragments 0-5, DMA pieces 0-13
+#define MLOP_W4_192_OPERANDS                                                                                    \
+  : [fa0_0] "=&v"(fa0_0), [fa0_1] "=&v"(fa0_1), [fa0_2] "=&v"(fa0_2), [fa0_3] "=&v"(fa0_3),                     \
+    [fa0_4] "=&v"(fa0_4), [fa0_5] "=&v"(fa0_5), [fb0_0] "=&v"(fb0_0), [fb0_1] "=&v"(fb0_1),                     \
+    [fb0_2] "=&v"(fb0_2), [fb0_3] "=&v"(fb0_3), [fb0_4] "=&v"(fb0_4), [fb0_5] "=&v"(fb0_5),                     \
+    [fb0_6] "=&v"(fb0_6), [fb0_7] "=&v"(fb0_7), [fa1_0] "=&v"(fa1_0), [fa1_1] "=&v"(fa1_1),                     \
+    [fa1_2] "=&v"(fa1_2), [fa1_3] "=&v"(fa1_3), [fa1_4] "=&v"(fa1_4), [fa1_5] "=&v"(fa1_5),                     \
+    [fb1_0] "=&v"(fb1_0), [fb1_1] "=&v"(fb1_1), [fb1_2] "=&v"(fb1_2), [fb1_3] "=&v"(fb1_3),                     \
+    [fb1_4] "=&v"(fb1_4), [fb1_5] "=&v"(fb1_5), [fb1_6] "=&v"(fb1_6), [fb1_7] "=&v"(fb1_7), [rA0] "+v"(rA0),    \
+    [rA1] "+v"(rA1), [rB0] "+v"(rB0), [rB1] "+v"(rB1), [koff] "+s"(koff), [dbase] "+s"(dbase),                  \
+    [iter] "+s"(iter), [m0save] "=&s"(m0save)                                                                   \
+  : [vo0] "v"(vo[0]), [vo1] "v"(vo[1]), [vo2] "v"(vo[2]), [vo3] "v"(vo[3]), [vo4] "v"(vo[4]), [vo5] "v"(vo[5]), \
+    [vo6] "v"(vo[6]), [vo7] "v"(vo[7]), [vo8] "v"(vo[8]), [vo9] "v"(vo[9]), [vo10] "v"(vo[10]),                 \
+    [vo11] "v"(vo[11]), [vo12] "v"(vo[12]), [vo13] "v"(vo[13]), [vn0] "v"(vn[0]), [vn1] "v"(vn[1]),             \
+    [vn2] "v"(vn[2]), [vn3] "v"(vn[3]), [vn4] "v"(vn[4]), [vn5] "v"(vn[5]), [vn6] "v"(vn[6]), [vn7] "v"(vn[7]), \
+    [vn8] "v"(vn[8]), [vn9] "v"(vn[9]), [vn10] "v"(vn[10]), [vn11] "v"(vn[11]), [vn12] "v"(vn[12]),             \
+    [vn13] "v"(vn[13]), [srdA] "s"(srdA), [srdB] "s"(srdB), [k128] "s"(k128), [first] "s"(s_first),             \
+    [has_next] "s"(s_next)                                                                                      \
+  : "memory", "scc", MLOP_W4_AGPR_CLOBBERS
     // one generated K-loop per count of VMEM ops between the prefetched K-tiles and the loop: the
     // previous epilogue's NS stores (+ the two row-sum DMAs of W4_RS, issued above)
     constexpr int NQ = NS + (RS ? 2 : 0);
@@ -254,6 +292,18 @@ __global__ void __launch_bounds__(256, 1) gemm_w4_kernel(
       else if constexpr (NQ == 16) asm volatile(MLOP_W4_KLOOP_S16_P0_ASM MLOP_W4_OPERANDS);
       else if constexpr (NQ == 34) asm volatile(MLOP_W4_KLOOP_S34_P0_ASM MLOP_W4_OPERANDS);
       else asm volatile(MLOP_W4_KLOOP_S18_P0_ASM MLOP_W4_OPERANDS);
+    } else if constexpr (BMT == 192) {
+      static_assert(NQ == 24 || NQ == 12 || NQ == 26 || NQ == 14, "one generated K-loop per VMEM count");
+      if constexpr (NQ == 24) asm volatile(MLOP_W4_192_KLOOP_S24_ASM MLOP_W4_192_OPERANDS);
+      else if constexpr (NQ == 12) asm volatile(MLOP_W4_192_KLOOP_S12_ASM MLOP_W4_192_OPERANDS);
+      else if constexpr (NQ == 26) asm volatile(MLOP_W4_192_KLOOP_S26_ASM MLOP_W4_192_OPERANDS);
+      else asm volatile(MLOP_W4_192_KLOOP_S14_ASM MLOP_W4_192_OPERANDS);
+    } else if constexpr (BMT == 160) {
+      static_assert(NQ == 20 || NQ == 10 || NQ == 22 || NQ == 12, "one generated K-loop per VMEM count");
+      if constexpr (NQ == 20) asm volatile(MLOP_W4_160_KLOOP_S20_ASM MLOP_W4_160_OPERANDS);
+      else if constexpr (NQ == 10) asm volatile(MLOP_W4_160_KLOOP_S10_ASM MLOP_W4_160_OPERANDS);
+      else if constexpr (NQ == 22) asm volatile(MLOP_W4_160_KLOOP_S22_ASM MLOP_W4_160_OPERANDS);
+      else asm volatile(MLOP_W4_160_KLOOP_S12_ASM MLOP_W4_160_OPERANDS);
     } else {
       static_assert(NQ == 16 || NQ == 8 || NQ == 18 || NQ == 10, "one generated K-loop per VMEM count");
       if constexpr (NQ == 16) asm volatile(MLOP_W4H_KLOOP_S16_ASM MLOP_W4H_OPERANDS);
@@ -263,6 +313,8 @@ __global__ void __launch_bounds__(256, 1) gemm_w4_kernel(
     }
 #undef MLOP_W4_OPERANDS
 #undef MLOP_W4H_OPERANDS
+#undef MLOP_W4_160_OPERANDS
+#undef MLOP_W4_192_OPERANDS
 
     // read-out: the K-loop accumulates C^T, so acc(i, j)[r] of lane l is
     //   C[m0 + wm*BMT/2 + 16i + (l & 15)][n0 + wn*128 + 16j + 4(l >> 4) + r]
@@ -680,6 +732,8 @@ static bool run_w4_h(int epi, const uint16_t* A, int lda, const uint16_t* B, int
 bool run_w4(int epi, const uint16_t* A, int lda, const uint16_t* B, int ldb, uint16_t* C, int ldc, int M, int N,
             int K, hipStream_t st, const RopeEpi& re, int bm) {
   if (bm == 128) return run_w4_h<128>(epi, A, lda, B, ldb, C, ldc, M, N, K, st, re);
+  if (bm == 160) return run_w4_h<160>(epi, A, lda, B, ldb, C, ldc, M, N, K, st, re);
+  if (bm == 192) return run_w4_h<192>(epi, A, lda, B, ldb, C, ldc, M, N, K, st, re);
   if (bm == 256) return run_w4_h<256>(epi, A, lda, B, ldb, C, ldc, M, N, K, st, re);
   return false;
 }

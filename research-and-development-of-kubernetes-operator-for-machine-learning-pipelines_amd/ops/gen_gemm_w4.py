@@ -86,6 +86,11 @@ SCHEDS = [Sched(rd1=[1 + 2 * k for k in range(16)], b1=38, dma=[40 + 4 * k for k
 # the half-height tile (BM = 128): 64 MFMAs, 12 fragment reads per k-half, 12 DMA pieces
 SCHED_H = Sched(rd1=[1 + k for k in range(12)], b1=20, dma=[21 + 2 * k for k in range(12)], b2=45,
                 rd0=[46 + k for k in range(12)], toggle1=19, bm=128)
+# the heights between: 80 / 96 MFMAs, 13 / 14 fragment reads per k-half and DMA pieces
+SCHED_160 = Sched(rd1=[1 + k for k in range(13)], b1=22, dma=[23 + round(2.5 * k) for k in range(13)], b2=57,
+                  rd0=[58 + round(k * 15 / 12) for k in range(13)], toggle1=21, bm=160)
+SCHED_192 = Sched(rd1=[1 + round(k * 16 / 13) for k in range(14)], b1=26, dma=[27 + 3 * k for k in range(14)], b2=70,
+                  rd0=[71 + round(k * 18 / 13) for k in range(14)], toggle1=22, bm=192)
 
 
 def frag(name, i):
@@ -287,6 +292,14 @@ def render() -> str:
             out.append(f'  "{ln}\\n" \\')
         out.append('  ""')
         out.append("")
+    # the heights between: 4 stores per 16-row block and wave (SiLU-mul 2), the same four counts
+    for sc in (SCHED_160, SCHED_192):
+        for ns in (4 * sc.nfa, 2 * sc.nfa, 4 * sc.nfa + 2, 2 * sc.nfa + 2):
+            out.append(f"#define MLOP_W4_{sc.bm}_KLOOP_S{ns}_ASM \\")
+            for ln in kloop(ns, sc):
+                out.append(f'  "{ln}\\n" \\')
+            out.append('  ""')
+            out.append("")
     for i in range(8):
         out.append(f"#define MLOP_W4_READ{i}_ASM \\")
         for ln in readout(i):
