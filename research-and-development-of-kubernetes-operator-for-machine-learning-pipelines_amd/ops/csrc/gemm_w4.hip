@@ -94,9 +94,11 @@ __global__ void __launch_bounds__(256, 1) gemm_w4_kernel(
   constexpr int NPC = NI + 8;       // DMA pieces per wave and K-tile (NI of A, 8 of B)
   // epilogue store instructions per wave and tile (the next tile's K-loop waits for its
   // prefetched K-tile 0 with vmcnt(16 + NS): the count must be exact, so every store is
-  // issued, rows >= M dropped by the buffer range check instead of a branch)
-  // (RoPE: every wave loads its rows' slots or positions first, and the compiler's wait for
-  // those loads retires the older prefetch DMAs anyway)
+  // issued, rows >= M dropped by the buffer range check instead of a branch -- and a store that
+  // is dropped whole may leave the count before the older DMAs, so a tile with rows >= M waits for
+  // them at its end)
+  // (RoPE: a wave with rows < M loads its rows' slots or positions first, and the compiler's wait
+  // for those loads retires the older prefetch DMAs anyway)
   // (ADD_SS: the 32 stores come after its residual loads, which retire the DMAs anyway; RS: the
   // ss loads likewise)
   constexpr int BASE = EPI & 3;
@@ -645,6 +647,11 @@ __global__ void __launch_bounds__(256, 1) gemm_w4_kernel(
         }
       }
     }
+    // rows past M (stores dropped or, RoPE, not issued), or a RoPE wave of padding columns: the counted wait at the next
+    // tile's start does not cover the prefetched DMAs (K = 192, M = 643: a few blocks of the next tile read its K-tile 0
+    // too early)
+    if (m0 + BM > M || (BASE == W4_ROPE && (n0 + wn * 128) / 128 >= re.Hq + 2 * re.Hkv))
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   }
 }
 

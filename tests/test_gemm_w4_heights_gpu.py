@@ -93,3 +93,23 @@ def test_norm_chain(gpu, height, M):
             else:
                 bound = 2.0 ** -8 * z.abs()
             assert ((got - z).abs() <= bound + 2e-3).all()
+
+
+# a tile with rows past M, then another on the same workgroup, at short K (the next tile's first K-tile is in flight)
+@pytest.mark.parametrize("variant,bm", [(6, 128), (6, 160), (6, 192), (5, 256)])
+@pytest.mark.parametrize("tiles,off", [(1, 1), (2, 17), (5, 3)])
+@pytest.mark.parametrize("K", [192, 448])
+def test_tile_after_a_partial_one(gpu, variant, bm, tiles, off, K):
+    M, N = tiles * bm + off, 32768
+    torch.manual_seed(M + K)
+    x = torch.randn(M, K, device=gpu, dtype=bf)
+    w = (0.05 * torch.randn(N, K, device=gpu)).to(bf)
+    y = x.float() @ w.float().t()
+    bound = 2.0 ** -8 * y.abs() + 2.0 ** -19 * (x.float().abs() @ w.float().abs().t()) + 1e-6
+    ops._sk_reserve(torch.device(gpu))
+    torch.ops.mlop.gemm_dense_plan(variant, bm, 256, -1)
+    try:
+        for _ in range(30):
+            assert ((ops.gemm(x, w).float() - y).abs() <= bound).all()
+    finally:
+        torch.ops.mlop.gemm_dense_plan(-1, -1, -1, -1)
