@@ -537,7 +537,8 @@ void grouped_gemm(Tensor out, Tensor a, Tensor w, Tensor offsets, int64_t max_ro
   mlop::launch_grouped_gemm(a.data_ptr(), w.data_ptr(), out.data_ptr(), offsets.data_ptr<int>(),
                             (int)G, (int)M, (int)N, (int)K, (int)max_rows, (int)epi, cur_stream(),
                             a_rows ? a_rows->data_ptr<int>() : nullptr, nullptr, nullptr,
-                            row_scale ? row_scale->data_ptr<float>() : nullptr, (float)p0, (float)p1);
+                            row_scale ? row_scale->data_ptr<float>() : nullptr, (float)p0, (float)p1,
+                            (int)std::min<int64_t>(a.size(0), INT_MAX));
 }
 
 void moe_route(Tensor topw, Tensor topi, Tensor logits) {

@@ -1604,6 +1604,8 @@ static void launch_plan(const Plan& p, const uint16_t* A, int lda, const uint16_
     else if (p.BM == 128) MLOP_GEMM(128, 64, 2, 2, 3, false);
     else if (p.BN == 64) MLOP_GEMM(256, 64, 4, 2, 3, false);
     else if (p.BN == 128) MLOP_GEMM(256, 128, 4, 2, 3, false);
+    else if (GROUPED && p.variant == 5)
+      run_w4_grouped(EPI, A, lda, B, ldb, C, ldc, M, N, K, st, re, offsets, n_groups);
     else if (GROUPED && p.variant == 3)
       run_pp<EPI, true>(A, lda, B, ldb, C, ldc, M, N, K, st, re, offsets, n_groups);
     else if (!GROUPED && p.variant == 5 && p.splits == 1 && gemm_w4_ok(M, N, K, lda, ldb, ldc))
@@ -1869,7 +1871,7 @@ bool launch_gemm_add_rmsnorm(const void* A, int lda, const void* B, void* out, v
 
 void launch_grouped_gemm(const void* A, const void* B, void* C, const int* offsets, int n_groups,
                          int M, int N, int K, int max_rows, int epi, hipStream_t st, const int* a_rows,
-                         float** defer_ws, int* defer_splits, const float* row_scale, float p0, float p1) {
+                         float** defer_ws, int* defer_splits, const float* row_scale, float p0, float p1, int a_n) {
   if (defer_splits) *defer_splits = 1;
   if (M == 0) return;
   if (a_rows == nullptr && row_scale == nullptr && defer_splits == nullptr && gemv_grouped_takes(M, N, K, epi)) {  // MoE decode: stream only the routed experts' weights
@@ -1877,13 +1879,22 @@ void launch_grouped_gemm(const void* A, const void* B, void* C, const int* offse
     return;
   }
   Plan p = plan(M, N, K, true, n_groups, max_rows);
-  // Mid-size MoE batches (a few dozen rows per expert): one m-tile per expert x N/64 tiles
-  // is too few workgroups to stream every expert's weights at full rate (down at batch 64:
-  // 512 workgroups of K = 14336, 4.7 TB/s).  Split K like the dense path, partials in the
-  // stream-K slab buffer (same stream, so never in use by another launch), then the reduce
-  // kernel applies the epilogue.  Routed tiles are estimated as one m-tile per expert.
+  // The four-wave kernel where the 256-row tiles make three rounds or more (gate_up): with fewer, stream-K's even split
+  // of the tail wins (down of 8 experts at 350 / 450 / 1024 rows each 320 / 355 / 791 us against 318 / 375 / 798).
+  // gate_up of 8 experts, ping-pong -> four-wave: 75 / 125 / 300 / 350 / 500 / 625 / 1024 rows each 374 -> 353, 376 ->
+  // 364, 630 -> 530, 654 -> 604, 828 -> 772, 1047 -> 978, 1606 -> 1479 us, and with the experts 0.6 - 1.4 of that 370
+  // -> 351, 375 -> 352, 636 -> 595, 666 -> 646, 877 -> 848, 1072 -> 954, 1620 -> 1481.  Not at 160 - 240 and 368 - 440
+  // rows, where an expert is most of one or two 256-row tiles but not the lower ones, and the ping-pong kernel skips a
+  // tile's empty 64-row quadrants (200 rows 397 us against 436, 375 677 against 737, 425 714 against 745).
+  const bool quadrants = (max_rows >= 160 && max_rows < 240) || (max_rows >= 368 && max_rows < 440);
+  if (p.variant == 3 && g_gp[0] <= 0 && !quadrants) {
+    const SkBuf* b = sk_buf();
+    if (b && (long)n_groups * std::max(1, (max_rows + 128) / 256) * (N / 256) >= 3l * b->cus &&
+        gemm_w4_grouped_ok(M, N, K, n_groups, a_n))
+      p.variant = 5;
+  }
   float* ws = nullptr;
-  if (p.variant != 3 && K >= 2048 && g_gp[3] != 1 && !(p.nosplit && g_gp[0] <= 0)) {
+  if (p.variant == 0 && K >= 2048 && g_gp[3] != 1 && !(p.nosplit && g_gp[0] <= 0)) {
     const SkBuf* b = sk_buf();
     const long t_est = (long)((N + p.BN - 1) / p.BN) * std::max(1, std::min(n_groups, (M + p.BM - 1) / p.BM + n_groups));
     constexpr int target = 1024;

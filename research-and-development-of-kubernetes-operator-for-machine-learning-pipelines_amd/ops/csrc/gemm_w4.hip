@@ -81,11 +81,15 @@ __device__ __forceinline__ void unroll(F&& f) {
 }
 }  // namespace
 
-template <int EPI, int BMT>
-__global__ void __launch_bounds__(256, 1) gemm_w4_kernel(
+// GROUPED (the experts' products): A rows sorted by expert, rows offsets[e] .. offsets[e + 1] - 1 against B + e N ldb;
+// A row r is re.a_rows[r] where given.  The routed tiles are counted here, from the offsets, as is their tail split.
+template <int EPI, int BMT, bool GROUPED>
+__device__ __forceinline__ void gemm_w4_tiles(
     const uint16_t* __restrict__ A, int lda, const uint16_t* __restrict__ B, int ldb,
     uint16_t* __restrict__ C, int ldc, int M, int N, int K, int n_tiles_x, int m_tiles, int group_m,
-    RopeEpi re, int n_dp, int n_items, float* __restrict__ ws, int* __restrict__ cnt) {
+    const RopeEpi& re, int n_dp, int n_items, float* __restrict__ ws, int* __restrict__ cnt,
+    const int* __restrict__ offsets, int n_groups) {
+  static_assert(!GROUPED || EPI == W4_NONE || EPI == W4_SILU_MUL, "grouped epilogues");
   // BMT = 256: 128 x 128 outputs per wave; BMT = 128 (the half-height tile, twice the tiles for
   // the mid-M and QKV grids): 64 x 128 per wave, 4 x 8 accumulators, 12 DMA pieces per K-tile
   constexpr int BM = BMT, BN = 256;
@@ -122,7 +126,46 @@ __global__ void __launch_bounds__(256, 1) gemm_w4_kernel(
   const int G = gridDim.x, Lb = blockIdx.x;
   const int q = G >> 3, rr = G & 7, xcd = Lb & 7, slot = Lb >> 3;
   const int lid = (xcd < rr ? xcd * (q + 1) : rr * (q + 1) + (xcd - rr) * q) + slot;
-  auto origin = [&](int t, int& m0, int& n0) {
+  // GROUPED tables past the K-tile buffers: [0, 65) the offsets, [65, 129) the row tiles up to and with each expert,
+  // then per wave three items' A rows
+  int* tab = reinterpret_cast<int*>(smem + 65536);
+  int* rows_lds = tab + 192 + wid * 192;
+  if constexpr (GROUPED) {
+    int o0 = 0, o1 = 0;
+    if (lane < n_groups) o0 = offsets[lane], o1 = offsets[lane + 1];
+    int c = (o1 - o0 + BM - 1) / BM;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int x = __shfl_up(c, d);
+      if (lane >= d) c += x;
+    }
+    const int T = __builtin_amdgcn_readfirstlane(__shfl(c, 63)) * n_tiles_x, r = T % G;
+    if (wid == 0) {
+      if (lane < n_groups) tab[lane] = o0;
+      if (lane == n_groups - 1) tab[n_groups] = o1;
+      tab[65 + lane] = lane < n_groups ? c : 0x7fffffff;
+    }
+    __syncthreads();
+    const bool halves = ws != nullptr && r > 0 && 2 * r <= G && nk % 2 == 0 && nk / 2 >= 3;  // gemm_w4_split_ok
+    n_dp = halves ? T - r : T;
+    n_items = halves ? T + r : T;
+  }
+  // (GROUPED: an expert's tiles are consecutive, its row tiles fastest: they share a B panel, and the next column
+  // tile reuses their A rows.  B offsets carry the expert, the rows end at m_end.)
+  auto origin = [&](int t, int& m0, int& n0, int& m_end, uint32_t& b0) {
+    m_end = M;
+    b0 = 0;
+    if constexpr (GROUPED) {
+      const int e = __popcll(__ballot(tab[65 + lane] <= t / n_tiles_x));  // the first expert whose tiles end past t
+      const int base = e > 0 ? __builtin_amdgcn_readfirstlane(tab[64 + e]) : 0;
+      const int c = __builtin_amdgcn_readfirstlane(tab[65 + e]) - base, ti = t - base * n_tiles_x;
+      const int r0 = __builtin_amdgcn_readfirstlane(tab[e]);
+      m_end = __builtin_amdgcn_readfirstlane(tab[e + 1]);
+      m0 = r0 + ti % c * BM;
+      n0 = ti / c * BN;
+      b0 = (uint32_t)e * (uint32_t)N * (uint32_t)(ldb * 2);
+      return;
+    }
     const int band = t / (group_m * n_tiles_x), in_band = t % (group_m * n_tiles_x);
     const int gm_here = min(group_m, m_tiles - band * group_m);
     m0 = (band * group_m + in_band % gm_here) * BM;
@@ -133,26 +176,43 @@ __global__ void __launch_bounds__(256, 1) gemm_w4_kernel(
   // DMA piece i (0..NPC-1) of this wave: p = wid + 4 i, 8 rows x 128 B at LDS byte 1024 p;
   // i < NI A rows 8p.., else B rows 8(p - 4 NI).. (B starts at LDS byte 128 BMT); lane -> row
   // 8p + lane / 8, LDS slot lane % 8 holds source chunk (lane % 8) ^ swz(row)
-  auto item = [&](int i, int& m0, int& n0, int& kb, int& nkl) {
+  auto item = [&](int i, int& m0, int& n0, int& m_end, uint32_t& b0, int& kb, int& nkl) {
     const bool tail = i >= n_dp;
-    origin(tail ? n_dp + ((i - n_dp) >> 1) : i, m0, n0);
+    origin(tail ? n_dp + ((i - n_dp) >> 1) : i, m0, n0, m_end, b0);
     kb = tail ? ((i - n_dp) & 1) * (nk >> 1) : 0;
     nkl = tail ? nk >> 1 : nk;
   };
-  auto dma_offsets = [&](int m0, int n0, int kb, uint32_t (&vo)[NPC]) {
+  auto dma_offsets = [&](int m0, int n0, int m_end, uint32_t b0, int kb, const int* rows, uint32_t (&vo)[NPC]) {
 #pragma unroll
     for (int i = 0; i < NPC; ++i) {
       const int p = wid + 4 * i;
       const int r = (i < NI ? p : p - 4 * NI) * 8 + (lane >> 3);
       const uint32_t ch = (uint32_t)(((lane & 7) ^ ((r >> 1) & 7)) << 4);
-      if (i < NI) vo[i] = (uint32_t)min(m0 + r, M - 1) * (uint32_t)(lda * 2) + ch + kb * 128;
-      else vo[i] = (uint32_t)min(n0 + r, N - 1) * (uint32_t)(ldb * 2) + ch + kb * 128;
+      if (i < NI) {
+        int row = min(m0 + r, m_end - 1);
+        if (GROUPED && re.a_rows != nullptr) row = rows[8 * i + (lane >> 3)];
+        vo[i] = (uint32_t)row * (uint32_t)(lda * 2) + ch + kb * 128;
+      } else {
+        vo[i] = b0 + (uint32_t)min(n0 + r, N - 1) * (uint32_t)(ldb * 2) + ch + kb * 128;
+      }
     }
   };
   const i32x4 srdA = make_srd(A), srdB = make_srd(B);
-  // C rows >= M fall outside num_records: their stores are dropped, never branched around
-  const auto srdC = __builtin_amdgcn_make_buffer_rsrc((void*)C, 0, (int)((uint32_t)M * (uint32_t)ldc * 2u), 0x00020000);
   const uint32_t lbase = (uint32_t)(uintptr_t)((lds_u16*)smem);
+  // GROUPED: lane l holds the row of piece l / 8's row l % 8 (l / 8 < NI)
+  auto row_of = [&](int l) { return (wid + 4 * (l >> 3)) * 8 + (l & 7); };
+  int slot_i = 0;
+  if constexpr (GROUPED) {
+    if (re.a_rows != nullptr && lid < n_items) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        int m, n, e, kb, nkl;
+        uint32_t b;
+        item(lid + j * G < n_items ? lid + j * G : lid, m, n, e, b, kb, nkl);
+        rows_lds[j * 64 + lane] = re.a_rows[min(m + row_of(lane), e - 1)];
+      }
+    }
+  }
   // fragment read addresses (buffer 0): row = wm*BMT/2 + (lane & 15) (+16 per fragment via the
   // offset field), chunk (k-half h) = (4h + lane / 16) ^ swz(row); swz depends on lane only
   const uint32_t sw = ((lane & 15) >> 1) & 7;
@@ -160,7 +220,6 @@ __global__ void __launch_bounds__(256, 1) gemm_w4_kernel(
   const uint32_t a_row = lbase + (uint32_t)(wm * (BMT / 2) + (lane & 15)) * 128;
   const uint32_t b_row = lbase + BMT * 128 + (uint32_t)(wn * 128 + (lane & 15)) * 128;
   const uint32_t dbase0 = __builtin_amdgcn_readfirstlane(lbase + wid * 1024);
-  const uint32_t k128 = 128;
   // W4_RS: per-wave row sums of squares after the two 64 KiB K-tile buffers; W4_ADD_SS: the
   // band ticket's flag after them (run_w4_t sizes the LDS)
   float* rinv_lds = reinterpret_cast<float*>(smem + 65536);
@@ -170,16 +229,52 @@ __global__ void __launch_bounds__(256, 1) gemm_w4_kernel(
     // offsets of this item (recomputed, not carried from the previous iteration: nothing but
     // the item index stays live across the epilogue) and of the next one (prefetched at the
     // end of the K-loop statement)
-    int m0, n0, kb, nkl;
-    item(it, m0, n0, kb, nkl);
+    int m0, n0, m_end, kb, nkl;
+    uint32_t b0;
+    item(it, m0, n0, m_end, b0, kb, nkl);
     uint32_t vo[NPC], vn[NPC];
-    dma_offsets(m0, n0, kb, vo);
+    dma_offsets(m0, n0, m_end, b0, kb, rows_lds + slot_i * 64, vo);
     const bool next = it + G < n_items;
+    // the K walk starts at another eighth per XCD (GROUPED): tiles in step would otherwise all read the columns of the
+    // same few memory channels
+    auto k_at = [&](int len, int j) {
+      const int k = (GROUPED ? xcd * len / 8 : 0) + j;
+      return (uint32_t)__builtin_amdgcn_readfirstlane((k >= len ? k - len : k) * 128);
+    };
+    const uint32_t k0 = k_at(nkl, 0), k1 = k_at(nkl, 1), kend = __builtin_amdgcn_readfirstlane(nkl * 128);
+    uint32_t kn0, kn1;
     {
-      int m1 = m0, n1 = n0, kb1 = kb, nkl1 = nkl;
-      if (next) item(it + G, m1, n1, kb1, nkl1);
-      dma_offsets(m1, n1, kb1, vn);
+      int m1 = m0, n1 = n0, e1 = m_end, kb1 = kb, nkl1 = nkl;
+      uint32_t b1 = b0;
+      if (next) item(it + G, m1, n1, e1, b1, kb1, nkl1);
+      dma_offsets(m1, n1, e1, b1, kb1, rows_lds + (slot_i == 2 ? 0 : slot_i + 1) * 64, vn);
+      kn0 = k_at(nkl1, 0), kn1 = k_at(nkl1, 1);
     }
+    if constexpr (GROUPED) {
+      // the A rows of the item after the next into the third slot, by LDS-DMA like W4_RS's below and for its reason
+      int m2 = m0, n2, e2 = m_end, kb2, nkl2;
+      uint32_t b2;
+      if (it + 2 * G < n_items) item(it + 2 * G, m2, n2, e2, b2, kb2, nkl2);
+      const auto rs_rows = __builtin_amdgcn_make_buffer_rsrc((void*)re.a_rows, 0, re.a_rows != nullptr ? (int)((uint32_t)M * 4u) : 0,
+                                                             0x00020000);
+      const uint32_t voff = (uint32_t)min(m2 + row_of(lane), e2 - 1) * 4u;
+      const uint32_t lds_dst =
+          __builtin_amdgcn_readfirstlane(lbase + 131072u + (uint32_t)(192 + wid * 192 + (slot_i == 0 ? 2 : slot_i - 1) * 64) * 4u);
+      uint32_t msave;
+      asm volatile(
+          "s_mov_b32 %[ms], m0\n"
+          "s_mov_b32 m0, %[dst]\n"
+          "s_nop 0\n"
+          "buffer_load_dword %[vo], %[srd], 0 offen lds\n"
+          "buffer_load_dword %[vo], %[srd], 0 offen lds\n"  // (twice: the built K-loops count two)
+          "s_mov_b32 m0, %[ms]\n"
+          : [ms] "=&s"(msave)
+          : [dst] "s"(lds_dst), [vo] "v"(voff), [srd] "s"(rs_rows)
+          : "memory", "scc");
+      slot_i = slot_i == 2 ? 0 : slot_i + 1;
+    }
+    // C rows >= m_end fall outside num_records: their stores are dropped, never branched around
+    const auto srdC = __builtin_amdgcn_make_buffer_rsrc((void*)C, 0, (int)((uint32_t)m_end * (uint32_t)ldc * 2u), 0x00020000);
     // W4_RS: the sums of squares of the wave's BMT / 2 rows (BMT = 128: the second load reads
     // rows past them, unused, so both tile heights count two VMEM ops) go to its LDS slot past the two K-tile
     // buffers by LDS-DMA, issued BEFORE the K-loop and invisible to the compiler: a load it
@@ -206,7 +301,7 @@ __global__ void __launch_bounds__(256, 1) gemm_w4_kernel(
           : "memory", "scc");
     }
     uint32_t rA0 = a_row + c0, rA1 = a_row + c1, rB0 = b_row + c0, rB1 = b_row + c1;
-    uint32_t dbase = dbase0, koff = 256, m0save;
+    uint32_t dbase = dbase0, koff = k_at(nkl, 2), m0save;
     uint32_t iter = __builtin_amdgcn_readfirstlane(nkl - 3);
     const uint32_t s_first = __builtin_amdgcn_readfirstlane(first), s_next = __builtin_amdgcn_readfirstlane((int)next);
     bf16x8 fa0_0, fa0_1, fa0_2, fa0_3, fa0_4, fa0_5, fa0_6, fa0_7;
@@ -230,7 +325,7 @@ __global__ void __launch_bounds__(256, 1) gemm_w4_kernel(
     [vn0] "v"(vn[0]), [vn1] "v"(vn[1]), [vn2] "v"(vn[2]), [vn3] "v"(vn[3]), [vn4] "v"(vn[4]), [vn5] "v"(vn[5]), \
     [vn6] "v"(vn[6]), [vn7] "v"(vn[7]), [vn8] "v"(vn[8]), [vn9] "v"(vn[9]), [vn10] "v"(vn[10]),                 \
     [vn11] "v"(vn[11]), [vn12] "v"(vn[12]), [vn13] "v"(vn[13]), [vn14] "v"(vn[14]), [vn15] "v"(vn[15]),         \
-    [srdA] "s"(srdA), [srdB] "s"(srdB), [k128] "s"(k128), [first] "s"(s_first), [has_next] "s"(s_next)          \
+    [srdA] "s"(srdA), [srdB] "s"(srdB), [k0] "s"(k0), [k1] "s"(k1), [n0] "s"(kn0), [n1] "s"(kn1), [kend] "s"(kend), [first] "s"(s_first), [has_next] "s"(s_next)          \
   : "memory", "scc", MLOP_W4_AGPR_CLOBBERS
 // the half-height loop: A fragments 0-3, DMA pieces 0-11 (accumulators a[0:127])
 #define MLOP_W4H_OPERANDS                                                                                        \
@@ -246,7 +341,7 @@ __global__ void __launch_bounds__(256, 1) gemm_w4_kernel(
     [vo6] "v"(vo[6]), [vo7] "v"(vo[7]), [vo8] "v"(vo[8]), [vo9] "v"(vo[9]), [vo10] "v"(vo[10]),                 \
     [vo11] "v"(vo[11]), [vn0] "v"(vn[0]), [vn1] "v"(vn[1]), [vn2] "v"(vn[2]), [vn3] "v"(vn[3]),                 \
     [vn4] "v"(vn[4]), [vn5] "v"(vn[5]), [vn6] "v"(vn[6]), [vn7] "v"(vn[7]), [vn8] "v"(vn[8]), [vn9] "v"(vn[9]), \
-    [vn10] "v"(vn[10]), [vn11] "v"(vn[11]), [srdA] "s"(srdA), [srdB] "s"(srdB), [k128] "s"(k128),               \
+    [vn10] "v"(vn[10]), [vn11] "v"(vn[11]), [srdA] "s"(srdA), [srdB] "s"(srdB), [k0] "s"(k0), [k1] "s"(k1), [n0] "s"(kn0), [n1] "s"(kn1), [kend] "s"(kend),               \
     [first] "s"(s_first), [has_next] "s"(s_next)                                                                 \
   : "memory", "scc", MLOP_W4_AGPR_CLOBBERS
 // 160 rows: A fragments 0-4, DMA pieces 0-12
@@ -264,7 +359,7 @@ __global__ void __launch_bounds__(256, 1) gemm_w4_kernel(
     [vo11] "v"(vo[11]), [vo12] "v"(vo[12]), [vn0] "v"(vn[0]), [vn1] "v"(vn[1]), [vn2] "v"(vn[2]),               \
     [vn3] "v"(vn[3]), [vn4] "v"(vn[4]), [vn5] "v"(vn[5]), [vn6] "v"(vn[6]), [vn7] "v"(vn[7]), [vn8] "v"(vn[8]), \
     [vn9] "v"(vn[9]), [vn10] "v"(vn[10]), [vn11] "v"(vn[11]), [vn12] "v"(vn[12]), [srdA] "s"(srdA),             \
-    [srdB] "s"(srdB), [k128] "s"(k128), [first] "s"(s_first), [has_next] "s"(s_next)                            \
+    [srdB] "s"(srdB), [k0] "s"(k0), [k1] "s"(k1), [n0] "s"(kn0), [n1] "s"(kn1), [kend] "s"(kend), [first] "s"(s_first), [has_next] "s"(s_next)                            \
   : "memory", "scc", MLOP_W4_AGPR_CLOBBERS
 // 192 rows: A fragments 0-5, DMA pieces 0-13
 #define MLOP_W4_192_OPERANDS                                                                                    \
@@ -282,12 +377,12 @@ __global__ void __launch_bounds__(256, 1) gemm_w4_kernel(
     [vo11] "v"(vo[11]), [vo12] "v"(vo[12]), [vo13] "v"(vo[13]), [vn0] "v"(vn[0]), [vn1] "v"(vn[1]),             \
     [vn2] "v"(vn[2]), [vn3] "v"(vn[3]), [vn4] "v"(vn[4]), [vn5] "v"(vn[5]), [vn6] "v"(vn[6]), [vn7] "v"(vn[7]), \
     [vn8] "v"(vn[8]), [vn9] "v"(vn[9]), [vn10] "v"(vn[10]), [vn11] "v"(vn[11]), [vn12] "v"(vn[12]),             \
-    [vn13] "v"(vn[13]), [srdA] "s"(srdA), [srdB] "s"(srdB), [k128] "s"(k128), [first] "s"(s_first),             \
+    [vn13] "v"(vn[13]), [srdA] "s"(srdA), [srdB] "s"(srdB), [k0] "s"(k0), [k1] "s"(k1), [n0] "s"(kn0), [n1] "s"(kn1), [kend] "s"(kend), [first] "s"(s_first),             \
     [has_next] "s"(s_next)                                                                                      \
   : "memory", "scc", MLOP_W4_AGPR_CLOBBERS
     // one generated K-loop per count of VMEM ops between the prefetched K-tiles and the loop: the
     // previous epilogue's NS stores (+ the two row-sum DMAs of W4_RS, issued above)
-    constexpr int NQ = NS + (RS ? 2 : 0);
+    constexpr int NQ = NS + (RS || GROUPED ? 2 : 0);
     if constexpr (BMT == 256) {
       static_assert(NQ == 32 || NQ == 16 || NQ == 34 || NQ == 18, "one generated K-loop per VMEM count");
       if constexpr (NQ == 32) asm volatile(MLOP_W4_KLOOP_S32_P0_ASM MLOP_W4_OPERANDS);
@@ -526,6 +621,13 @@ __global__ void __launch_bounds__(256, 1) gemm_w4_kernel(
         float v[32];
         fetch(I_, v);
         const uint32_t row_off = (uint32_t)(m0 + lr + I * 16) * (uint32_t)ldc * 2u;
+        if constexpr (GROUPED && BASE == W4_SILU_MUL) {
+          if (re.row_scale != nullptr) {
+            const float f = re.row_scale[min(m0 + lr + I * 16, m_end - 1)];
+#pragma unroll
+            for (int e = 0; e < 32; ++e) v[e] *= f;
+          }
+        }
         if constexpr (BASE == W4_SILU_MUL) {
           float o[16];
           if (BASE == W4_SILU_MUL && re.p0 > 0.f) {
@@ -650,9 +752,58 @@ __global__ void __launch_bounds__(256, 1) gemm_w4_kernel(
     // rows past M (stores dropped or, RoPE, not issued), or a RoPE wave of padding columns: the counted wait at the next
     // tile's start does not cover the prefetched DMAs (K = 192, M = 643: a few blocks of the next tile read its K-tile 0
     // too early)
-    if (m0 + BM > M || (BASE == W4_ROPE && (n0 + wn * 128) / 128 >= re.Hq + 2 * re.Hkv))
+    if (m0 + BM > m_end || (BASE == W4_ROPE && (n0 + wn * 128) / 128 >= re.Hq + 2 * re.Hkv))
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   }
+}
+
+template <int EPI, int BMT>
+__global__ void __launch_bounds__(256, 1) gemm_w4_kernel(
+    const uint16_t* __restrict__ A, int lda, const uint16_t* __restrict__ B, int ldb,
+    uint16_t* __restrict__ C, int ldc, int M, int N, int K, int n_tiles_x, int m_tiles, int group_m,
+    RopeEpi re, int n_dp, int n_items, float* __restrict__ ws, int* __restrict__ cnt) {
+  gemm_w4_tiles<EPI, BMT, false>(A, lda, B, ldb, C, ldc, M, N, K, n_tiles_x, m_tiles, group_m, re, n_dp, n_items, ws, cnt,
+                                 nullptr, 0);
+}
+
+// The experts' products of a prompt.  What the grid loses is rows of partial tiles and the last round, and both hang on
+// the routing, which only the device knows: the height is chosen here, by estimated time in rounds of 256-row tiles (a
+// round of the lower ones .79 / .69, K-halves .59; W: the weights' rounds at one tile per expert, which bound the lower
+// tiles).  gate_up of 8 experts, 256 / 192 / 160 rows: 300 rows each 738 / 619 / 532 us, 350 747 / 595 / 691, 500 779 /
+// 836 / 911, 550 1021 / 836 / 941, 1024 1497 / 1561 / 1598 (1.29 PFLOP/s); over 22 sizes, even and with the experts
+// 0.6 - 1.4 of the mean, the choice is within 1 % of the best of the three on average.  One XCD's workgroups share
+// panels and stay in step; each XCD's K walk starts at another eighth, and nothing is loaded between tiles that the
+// stores and the next tile's DMAs would be waited for with (offsets in LDS, gathered rows two tiles ahead): 1661 / 1577
+// / 1501 us before at 1024 rows, 800 before and 745 after at 450.
+template <int EPI>
+__global__ void __launch_bounds__(256, 1) gemm_w4_grouped_kernel(
+    const uint16_t* __restrict__ A, int lda, const uint16_t* __restrict__ B, int ldb, uint16_t* __restrict__ C, int ldc,
+    int M, int N, int K, int n_tiles_x, RopeEpi re, float* __restrict__ ws, int* __restrict__ cnt,
+    const int* __restrict__ offsets, int n_groups) {
+  const int lane = threadIdx.x & 63, G = gridDim.x, nk = K / 64;
+  const int rows = lane < n_groups ? offsets[lane + 1] - offsets[lane] : 0;
+  // (16 bits each: M K < 2^30 and K >= 192 keep every count below 2^16)
+  uint32_t a = (uint32_t)((rows + 255) / 256) | (uint32_t)((rows + 191) / 192) << 16, b = (uint32_t)((rows + 159) / 160);
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    a += __shfl_xor(a, d);
+    b += __shfl_xor(b, d);
+  }
+  a = __builtin_amdgcn_readfirstlane(a);
+  b = __builtin_amdgcn_readfirstlane(b);
+  auto rounds = [&](uint32_t t) {
+    const int T = (int)t * n_tiles_x, r = T % G;
+    return (float)(T / G) + (r == 0 ? 0.f : 2 * r <= G && nk % 2 == 0 && ws != nullptr ? .59f : 1.f);
+  };
+  const float W = (float)(__popcll(__ballot(rows > 0)) * n_tiles_x) / (float)G;
+  const float t256 = rounds(a & 0xffff), t192 = fmaxf(.79f * rounds(a >> 16), .88f * W), t160 = fmaxf(.69f * rounds(b), .81f * W);
+  const int h = __builtin_amdgcn_readfirstlane(t256 <= t192 && t256 <= t160 ? 256 : t192 <= t160 ? 192 : 160);
+#define MLOP_W4_GROUPED(h_)                                                                                           \
+  gemm_w4_tiles<EPI, h_, true>(A, lda, B, ldb, C, ldc, M, N, K, n_tiles_x, 0, 1, re, 0, 0, ws, cnt, offsets, n_groups)
+  if (h == 256) MLOP_W4_GROUPED(256);
+  else if (h == 192) MLOP_W4_GROUPED(192);
+  else MLOP_W4_GROUPED(160);
+#undef MLOP_W4_GROUPED
 }
 
 // the r = T % CUs tail tiles are cut into K-halves (one extra round of half-length items)
@@ -719,6 +870,36 @@ static bool run_w4_t(const uint16_t* A, int lda, const uint16_t* B, int ldb, uin
   }
   kern<<<grid, 256, lds, st>>>(A, lda, B, ldb, C, ldc, M, N, K, gx, gy, gm, re2, n_dp, n_items, ws, cnt);
   return true;
+}
+
+// (a_n: A's rows where a_rows picks them; the kernel's offsets are 32 bits and its tables hold 64 experts)
+bool gemm_w4_grouped_ok(int M, int N, int K, int n_groups, int a_n) {
+  return M > 0 && n_groups <= 64 && K % 64 == 0 && K >= 192 && N % 256 == 0 && (long)std::max(M, a_n) * K * 2 < (1l << 31) &&
+         (long)M * N * 2 < (1l << 31) && (long)n_groups * N * K * 2 < (1l << 31);
+}
+
+template <int EPI>
+static void run_w4_grouped_t(const uint16_t* A, int lda, const uint16_t* B, int ldb, uint16_t* C, int ldc, int M, int N,
+                             int K, hipStream_t st, const RopeEpi& re, const int* offsets, int n_groups) {
+  constexpr size_t lds = 2ull * 65536 + 4096;
+  auto kern = gemm_w4_grouped_kernel<EPI>;
+  static const bool attr =
+      hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess;
+  (void)attr;
+  float* ws = nullptr;
+  int *cnt = nullptr, cus = 256;
+  gemm_sk_scratch(&ws, &cnt, &cus);  // without it: no K-halves
+  const long most = (long)(N / 256) * ((M + 159) / 160 + n_groups);  // every expert's last tile partial
+  RopeEpi re2 = re;
+  re2.ws_nt = gemm_slab_nt(-1);
+  kern<<<(int)std::min<long>(most, cus), 256, lds, st>>>(A, lda, B, ldb, C, ldc, M, N, K, N / 256, re2, ws, cnt, offsets,
+                                                          n_groups);
+}
+
+void run_w4_grouped(int epi, const uint16_t* A, int lda, const uint16_t* B, int ldb, uint16_t* C, int ldc, int M, int N,
+                    int K, hipStream_t st, const RopeEpi& re, const int* offsets, int n_groups) {
+  if (epi == W4_NONE) run_w4_grouped_t<W4_NONE>(A, lda, B, ldb, C, ldc, M, N, K, st, re, offsets, n_groups);
+  else run_w4_grouped_t<W4_SILU_MUL>(A, lda, B, ldb, C, ldc, M, N, K, st, re, offsets, n_groups);
 }
 
 template <int BMT>

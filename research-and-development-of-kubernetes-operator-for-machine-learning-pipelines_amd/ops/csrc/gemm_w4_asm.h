@@ -9,100 +9,100 @@
   "s_cbranch_scc1 L_w4_pref_%=\n" \
   "s_mov_b32 m0, %[dbase]\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo0], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo0], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo1], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo1], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo2], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo2], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo6], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo6], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo7], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo7], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo8], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo8], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo9], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo9], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo10], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo10], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo12], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo12], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo13], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo13], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo14], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo14], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo15], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo15], %[srdB], %[k0] offen lds\n" \
   "s_xor_b32 m0, %[dbase], 0x10000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo0], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo0], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo1], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo1], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo2], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo2], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo6], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo6], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo7], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo7], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo8], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo8], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo9], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo9], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo10], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo10], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo12], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo12], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo13], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo13], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo14], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo14], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo15], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo15], %[srdB], %[k1] offen lds\n" \
   "s_waitcnt vmcnt(16)\n" \
   "s_branch L_w4_go_%=\n" \
   "L_w4_pref_%=:\n" \
@@ -283,6 +283,8 @@
   "buffer_load_dwordx4 %[vo15], %[srdB], %[koff] offen lds\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
+  "s_cmp_eq_u32 %[koff], %[kend]\n" \
+  "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
   "s_waitcnt vmcnt(16)\n" \
@@ -492,6 +494,8 @@
   "buffer_load_dwordx4 %[vo15], %[srdB], %[koff] offen lds\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
+  "s_cmp_eq_u32 %[koff], %[kend]\n" \
+  "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
   "s_waitcnt vmcnt(16)\n" \
@@ -887,100 +891,100 @@
   "s_cbranch_scc1 L_w4_end_%=\n" \
   "s_mov_b32 m0, %[dbase]\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn0], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn0], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn1], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn1], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn2], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn2], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn3], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn3], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn4], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn4], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn5], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn5], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn6], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn6], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn7], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn7], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn8], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn8], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn9], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn9], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn10], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn10], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn11], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn11], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn12], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn12], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn13], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn13], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn14], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn14], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn15], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn15], %[srdB], %[n0] offen lds\n" \
   "s_xor_b32 m0, %[dbase], 0x10000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn0], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn0], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn1], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn1], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn2], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn2], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn3], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn3], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn4], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn4], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn5], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn5], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn6], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn6], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn7], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn7], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn8], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn8], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn9], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn9], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn10], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn10], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn11], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn11], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn12], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn12], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn13], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn13], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn14], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn14], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn15], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn15], %[srdB], %[n1] offen lds\n" \
   "L_w4_end_%=:\n" \
   "s_nop 7\n" \
   "s_nop 7\n" \
@@ -995,100 +999,100 @@
   "s_cbranch_scc1 L_w4_pref_%=\n" \
   "s_mov_b32 m0, %[dbase]\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo0], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo0], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo1], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo1], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo2], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo2], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo6], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo6], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo7], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo7], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo8], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo8], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo9], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo9], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo10], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo10], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo12], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo12], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo13], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo13], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo14], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo14], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo15], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo15], %[srdB], %[k0] offen lds\n" \
   "s_xor_b32 m0, %[dbase], 0x10000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo0], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo0], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo1], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo1], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo2], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo2], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo6], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo6], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo7], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo7], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo8], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo8], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo9], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo9], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo10], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo10], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo12], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo12], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo13], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo13], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo14], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo14], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo15], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo15], %[srdB], %[k1] offen lds\n" \
   "s_waitcnt vmcnt(16)\n" \
   "s_branch L_w4_go_%=\n" \
   "L_w4_pref_%=:\n" \
@@ -1269,6 +1273,8 @@
   "buffer_load_dwordx4 %[vo15], %[srdB], %[koff] offen lds\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
+  "s_cmp_eq_u32 %[koff], %[kend]\n" \
+  "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
   "s_waitcnt vmcnt(16)\n" \
@@ -1478,6 +1484,8 @@
   "buffer_load_dwordx4 %[vo15], %[srdB], %[koff] offen lds\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
+  "s_cmp_eq_u32 %[koff], %[kend]\n" \
+  "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
   "s_waitcnt vmcnt(16)\n" \
@@ -1873,100 +1881,100 @@
   "s_cbranch_scc1 L_w4_end_%=\n" \
   "s_mov_b32 m0, %[dbase]\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn0], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn0], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn1], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn1], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn2], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn2], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn3], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn3], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn4], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn4], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn5], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn5], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn6], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn6], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn7], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn7], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn8], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn8], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn9], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn9], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn10], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn10], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn11], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn11], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn12], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn12], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn13], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn13], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn14], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn14], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn15], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn15], %[srdB], %[n0] offen lds\n" \
   "s_xor_b32 m0, %[dbase], 0x10000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn0], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn0], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn1], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn1], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn2], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn2], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn3], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn3], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn4], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn4], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn5], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn5], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn6], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn6], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn7], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn7], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn8], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn8], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn9], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn9], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn10], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn10], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn11], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn11], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn12], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn12], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn13], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn13], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn14], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn14], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn15], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn15], %[srdB], %[n1] offen lds\n" \
   "L_w4_end_%=:\n" \
   "s_nop 7\n" \
   "s_nop 7\n" \
@@ -1981,100 +1989,100 @@
   "s_cbranch_scc1 L_w4_pref_%=\n" \
   "s_mov_b32 m0, %[dbase]\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo0], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo0], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo1], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo1], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo2], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo2], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo6], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo6], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo7], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo7], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo8], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo8], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo9], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo9], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo10], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo10], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo12], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo12], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo13], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo13], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo14], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo14], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo15], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo15], %[srdB], %[k0] offen lds\n" \
   "s_xor_b32 m0, %[dbase], 0x10000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo0], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo0], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo1], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo1], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo2], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo2], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo6], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo6], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo7], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo7], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo8], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo8], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo9], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo9], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo10], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo10], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo12], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo12], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo13], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo13], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo14], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo14], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo15], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo15], %[srdB], %[k1] offen lds\n" \
   "s_waitcnt vmcnt(16)\n" \
   "s_branch L_w4_go_%=\n" \
   "L_w4_pref_%=:\n" \
@@ -2255,6 +2263,8 @@
   "buffer_load_dwordx4 %[vo15], %[srdB], %[koff] offen lds\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
+  "s_cmp_eq_u32 %[koff], %[kend]\n" \
+  "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
   "s_waitcnt vmcnt(16)\n" \
@@ -2464,6 +2474,8 @@
   "buffer_load_dwordx4 %[vo15], %[srdB], %[koff] offen lds\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
+  "s_cmp_eq_u32 %[koff], %[kend]\n" \
+  "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
   "s_waitcnt vmcnt(16)\n" \
@@ -2859,100 +2871,100 @@
   "s_cbranch_scc1 L_w4_end_%=\n" \
   "s_mov_b32 m0, %[dbase]\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn0], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn0], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn1], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn1], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn2], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn2], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn3], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn3], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn4], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn4], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn5], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn5], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn6], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn6], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn7], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn7], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn8], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn8], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn9], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn9], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn10], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn10], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn11], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn11], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn12], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn12], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn13], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn13], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn14], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn14], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn15], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn15], %[srdB], %[n0] offen lds\n" \
   "s_xor_b32 m0, %[dbase], 0x10000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn0], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn0], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn1], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn1], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn2], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn2], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn3], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn3], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn4], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn4], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn5], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn5], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn6], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn6], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn7], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn7], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn8], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn8], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn9], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn9], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn10], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn10], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn11], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn11], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn12], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn12], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn13], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn13], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn14], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn14], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn15], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn15], %[srdB], %[n1] offen lds\n" \
   "L_w4_end_%=:\n" \
   "s_nop 7\n" \
   "s_nop 7\n" \
@@ -2967,100 +2979,100 @@
   "s_cbranch_scc1 L_w4_pref_%=\n" \
   "s_mov_b32 m0, %[dbase]\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo0], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo0], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo1], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo1], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo2], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo2], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo6], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo6], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo7], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo7], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo8], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo8], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo9], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo9], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo10], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo10], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo12], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo12], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo13], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo13], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo14], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo14], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo15], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo15], %[srdB], %[k0] offen lds\n" \
   "s_xor_b32 m0, %[dbase], 0x10000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo0], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo0], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo1], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo1], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo2], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo2], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo6], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo6], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo7], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo7], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo8], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo8], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo9], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo9], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo10], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo10], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo12], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo12], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo13], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo13], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo14], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo14], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo15], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo15], %[srdB], %[k1] offen lds\n" \
   "s_waitcnt vmcnt(16)\n" \
   "s_branch L_w4_go_%=\n" \
   "L_w4_pref_%=:\n" \
@@ -3241,6 +3253,8 @@
   "buffer_load_dwordx4 %[vo15], %[srdB], %[koff] offen lds\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
+  "s_cmp_eq_u32 %[koff], %[kend]\n" \
+  "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
   "s_waitcnt vmcnt(16)\n" \
@@ -3450,6 +3464,8 @@
   "buffer_load_dwordx4 %[vo15], %[srdB], %[koff] offen lds\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
+  "s_cmp_eq_u32 %[koff], %[kend]\n" \
+  "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
   "s_waitcnt vmcnt(16)\n" \
@@ -3845,100 +3861,100 @@
   "s_cbranch_scc1 L_w4_end_%=\n" \
   "s_mov_b32 m0, %[dbase]\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn0], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn0], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn1], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn1], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn2], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn2], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn3], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn3], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn4], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn4], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn5], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn5], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn6], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn6], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn7], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn7], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn8], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn8], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn9], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn9], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn10], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn10], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn11], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn11], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn12], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn12], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn13], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn13], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn14], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn14], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn15], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn15], %[srdB], %[n0] offen lds\n" \
   "s_xor_b32 m0, %[dbase], 0x10000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn0], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn0], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn1], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn1], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn2], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn2], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn3], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn3], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn4], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn4], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn5], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn5], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn6], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn6], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn7], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn7], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn8], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn8], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn9], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn9], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn10], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn10], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn11], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn11], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn12], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn12], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn13], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn13], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn14], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn14], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn15], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn15], %[srdB], %[n1] offen lds\n" \
   "L_w4_end_%=:\n" \
   "s_nop 7\n" \
   "s_nop 7\n" \
@@ -3953,76 +3969,76 @@
   "s_cbranch_scc1 L_w4_pref_%=\n" \
   "s_mov_b32 m0, %[dbase]\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo0], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo0], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo1], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo1], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo2], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo2], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo6], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo6], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo7], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo7], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo8], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo8], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo9], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo9], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo10], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo10], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[k0] offen lds\n" \
   "s_xor_b32 m0, %[dbase], 0x10000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo0], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo0], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo1], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo1], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo2], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo2], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo6], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo6], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo7], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo7], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo8], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo8], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo9], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo9], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo10], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo10], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[k1] offen lds\n" \
   "s_waitcnt vmcnt(12)\n" \
   "s_branch L_w4_go_%=\n" \
   "L_w4_pref_%=:\n" \
@@ -4129,6 +4145,8 @@
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
+  "s_cmp_eq_u32 %[koff], %[kend]\n" \
+  "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "s_waitcnt vmcnt(12)\n" \
@@ -4257,6 +4275,8 @@
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
+  "s_cmp_eq_u32 %[koff], %[kend]\n" \
+  "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "s_waitcnt vmcnt(12)\n" \
@@ -4491,76 +4511,76 @@
   "s_cbranch_scc1 L_w4_end_%=\n" \
   "s_mov_b32 m0, %[dbase]\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn0], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn0], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn1], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn1], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn2], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn2], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn3], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn3], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn4], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn4], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn5], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn5], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn6], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn6], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn7], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn7], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn8], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn8], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn9], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn9], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn10], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn10], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn11], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn11], %[srdB], %[n0] offen lds\n" \
   "s_xor_b32 m0, %[dbase], 0x10000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn0], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn0], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn1], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn1], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn2], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn2], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn3], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn3], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn4], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn4], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn5], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn5], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn6], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn6], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn7], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn7], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn8], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn8], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn9], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn9], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn10], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn10], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn11], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn11], %[srdB], %[n1] offen lds\n" \
   "L_w4_end_%=:\n" \
   "s_nop 7\n" \
   "s_nop 7\n" \
@@ -4575,76 +4595,76 @@
   "s_cbranch_scc1 L_w4_pref_%=\n" \
   "s_mov_b32 m0, %[dbase]\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo0], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo0], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo1], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo1], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo2], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo2], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo6], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo6], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo7], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo7], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo8], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo8], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo9], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo9], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo10], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo10], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[k0] offen lds\n" \
   "s_xor_b32 m0, %[dbase], 0x10000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo0], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo0], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo1], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo1], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo2], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo2], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo6], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo6], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo7], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo7], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo8], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo8], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo9], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo9], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo10], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo10], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[k1] offen lds\n" \
   "s_waitcnt vmcnt(12)\n" \
   "s_branch L_w4_go_%=\n" \
   "L_w4_pref_%=:\n" \
@@ -4751,6 +4771,8 @@
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
+  "s_cmp_eq_u32 %[koff], %[kend]\n" \
+  "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "s_waitcnt vmcnt(12)\n" \
@@ -4879,6 +4901,8 @@
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
+  "s_cmp_eq_u32 %[koff], %[kend]\n" \
+  "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "s_waitcnt vmcnt(12)\n" \
@@ -5113,76 +5137,76 @@
   "s_cbranch_scc1 L_w4_end_%=\n" \
   "s_mov_b32 m0, %[dbase]\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn0], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn0], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn1], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn1], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn2], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn2], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn3], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn3], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn4], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn4], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn5], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn5], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn6], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn6], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn7], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn7], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn8], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn8], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn9], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn9], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn10], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn10], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn11], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn11], %[srdB], %[n0] offen lds\n" \
   "s_xor_b32 m0, %[dbase], 0x10000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn0], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn0], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn1], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn1], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn2], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn2], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn3], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn3], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn4], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn4], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn5], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn5], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn6], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn6], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn7], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn7], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn8], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn8], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn9], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn9], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn10], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn10], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn11], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn11], %[srdB], %[n1] offen lds\n" \
   "L_w4_end_%=:\n" \
   "s_nop 7\n" \
   "s_nop 7\n" \
@@ -5197,76 +5221,76 @@
   "s_cbranch_scc1 L_w4_pref_%=\n" \
   "s_mov_b32 m0, %[dbase]\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo0], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo0], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo1], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo1], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo2], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo2], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo6], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo6], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo7], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo7], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo8], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo8], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo9], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo9], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo10], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo10], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[k0] offen lds\n" \
   "s_xor_b32 m0, %[dbase], 0x10000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo0], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo0], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo1], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo1], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo2], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo2], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo6], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo6], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo7], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo7], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo8], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo8], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo9], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo9], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo10], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo10], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[k1] offen lds\n" \
   "s_waitcnt vmcnt(12)\n" \
   "s_branch L_w4_go_%=\n" \
   "L_w4_pref_%=:\n" \
@@ -5373,6 +5397,8 @@
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
+  "s_cmp_eq_u32 %[koff], %[kend]\n" \
+  "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "s_waitcnt vmcnt(12)\n" \
@@ -5501,6 +5527,8 @@
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
+  "s_cmp_eq_u32 %[koff], %[kend]\n" \
+  "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "s_waitcnt vmcnt(12)\n" \
@@ -5735,76 +5763,76 @@
   "s_cbranch_scc1 L_w4_end_%=\n" \
   "s_mov_b32 m0, %[dbase]\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn0], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn0], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn1], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn1], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn2], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn2], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn3], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn3], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn4], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn4], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn5], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn5], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn6], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn6], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn7], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn7], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn8], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn8], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn9], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn9], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn10], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn10], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn11], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn11], %[srdB], %[n0] offen lds\n" \
   "s_xor_b32 m0, %[dbase], 0x10000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn0], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn0], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn1], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn1], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn2], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn2], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn3], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn3], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn4], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn4], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn5], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn5], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn6], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn6], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn7], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn7], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn8], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn8], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn9], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn9], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn10], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn10], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn11], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn11], %[srdB], %[n1] offen lds\n" \
   "L_w4_end_%=:\n" \
   "s_nop 7\n" \
   "s_nop 7\n" \
@@ -5819,76 +5847,76 @@
   "s_cbranch_scc1 L_w4_pref_%=\n" \
   "s_mov_b32 m0, %[dbase]\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo0], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo0], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo1], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo1], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo2], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo2], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo6], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo6], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo7], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo7], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo8], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo8], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo9], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo9], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo10], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo10], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[k0] offen lds\n" \
   "s_xor_b32 m0, %[dbase], 0x10000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo0], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo0], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo1], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo1], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo2], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo2], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo6], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo6], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo7], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo7], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo8], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo8], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo9], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo9], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo10], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo10], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[k1] offen lds\n" \
   "s_waitcnt vmcnt(12)\n" \
   "s_branch L_w4_go_%=\n" \
   "L_w4_pref_%=:\n" \
@@ -5995,6 +6023,8 @@
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
+  "s_cmp_eq_u32 %[koff], %[kend]\n" \
+  "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "s_waitcnt vmcnt(12)\n" \
@@ -6123,6 +6153,8 @@
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
+  "s_cmp_eq_u32 %[koff], %[kend]\n" \
+  "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "s_waitcnt vmcnt(12)\n" \
@@ -6357,76 +6389,76 @@
   "s_cbranch_scc1 L_w4_end_%=\n" \
   "s_mov_b32 m0, %[dbase]\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn0], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn0], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn1], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn1], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn2], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn2], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn3], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn3], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn4], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn4], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn5], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn5], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn6], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn6], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn7], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn7], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn8], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn8], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn9], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn9], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn10], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn10], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn11], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn11], %[srdB], %[n0] offen lds\n" \
   "s_xor_b32 m0, %[dbase], 0x10000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn0], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn0], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn1], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn1], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn2], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn2], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn3], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn3], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn4], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn4], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn5], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn5], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn6], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn6], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn7], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn7], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn8], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn8], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn9], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn9], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn10], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn10], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn11], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn11], %[srdB], %[n1] offen lds\n" \
   "L_w4_end_%=:\n" \
   "s_nop 7\n" \
   "s_nop 7\n" \
@@ -6441,82 +6473,82 @@
   "s_cbranch_scc1 L_w4_pref_%=\n" \
   "s_mov_b32 m0, %[dbase]\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo0], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo0], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo1], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo1], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo2], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo2], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo6], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo6], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo7], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo7], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo8], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo8], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo9], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo9], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo10], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo10], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo12], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo12], %[srdB], %[k0] offen lds\n" \
   "s_xor_b32 m0, %[dbase], 0x10000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo0], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo0], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo1], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo1], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo2], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo2], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo6], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo6], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo7], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo7], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo8], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo8], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo9], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo9], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo10], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo10], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo12], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo12], %[srdB], %[k1] offen lds\n" \
   "s_waitcnt vmcnt(13)\n" \
   "s_branch L_w4_go_%=\n" \
   "L_w4_pref_%=:\n" \
@@ -6637,6 +6669,8 @@
   "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
+  "s_cmp_eq_u32 %[koff], %[kend]\n" \
+  "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
@@ -6785,6 +6819,8 @@
   "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
+  "s_cmp_eq_u32 %[koff], %[kend]\n" \
+  "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
@@ -7065,82 +7101,82 @@
   "s_cbranch_scc1 L_w4_end_%=\n" \
   "s_mov_b32 m0, %[dbase]\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn0], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn0], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn1], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn1], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn2], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn2], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn3], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn3], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn4], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn4], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn5], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn5], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn6], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn6], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn7], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn7], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn8], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn8], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn9], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn9], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn10], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn10], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn11], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn11], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn12], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn12], %[srdB], %[n0] offen lds\n" \
   "s_xor_b32 m0, %[dbase], 0x10000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn0], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn0], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn1], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn1], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn2], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn2], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn3], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn3], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn4], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn4], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn5], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn5], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn6], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn6], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn7], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn7], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn8], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn8], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn9], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn9], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn10], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn10], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn11], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn11], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn12], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn12], %[srdB], %[n1] offen lds\n" \
   "L_w4_end_%=:\n" \
   "s_nop 7\n" \
   "s_nop 7\n" \
@@ -7155,82 +7191,82 @@
   "s_cbranch_scc1 L_w4_pref_%=\n" \
   "s_mov_b32 m0, %[dbase]\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo0], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo0], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo1], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo1], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo2], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo2], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo6], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo6], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo7], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo7], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo8], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo8], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo9], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo9], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo10], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo10], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo12], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo12], %[srdB], %[k0] offen lds\n" \
   "s_xor_b32 m0, %[dbase], 0x10000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo0], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo0], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo1], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo1], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo2], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo2], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo6], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo6], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo7], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo7], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo8], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo8], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo9], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo9], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo10], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo10], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo12], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo12], %[srdB], %[k1] offen lds\n" \
   "s_waitcnt vmcnt(13)\n" \
   "s_branch L_w4_go_%=\n" \
   "L_w4_pref_%=:\n" \
@@ -7351,6 +7387,8 @@
   "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
+  "s_cmp_eq_u32 %[koff], %[kend]\n" \
+  "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
@@ -7499,6 +7537,8 @@
   "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
+  "s_cmp_eq_u32 %[koff], %[kend]\n" \
+  "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
@@ -7779,82 +7819,82 @@
   "s_cbranch_scc1 L_w4_end_%=\n" \
   "s_mov_b32 m0, %[dbase]\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn0], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn0], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn1], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn1], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn2], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn2], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn3], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn3], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn4], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn4], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn5], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn5], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn6], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn6], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn7], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn7], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn8], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn8], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn9], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn9], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn10], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn10], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn11], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn11], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn12], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn12], %[srdB], %[n0] offen lds\n" \
   "s_xor_b32 m0, %[dbase], 0x10000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn0], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn0], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn1], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn1], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn2], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn2], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn3], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn3], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn4], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn4], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn5], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn5], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn6], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn6], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn7], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn7], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn8], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn8], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn9], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn9], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn10], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn10], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn11], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn11], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn12], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn12], %[srdB], %[n1] offen lds\n" \
   "L_w4_end_%=:\n" \
   "s_nop 7\n" \
   "s_nop 7\n" \
@@ -7869,82 +7909,82 @@
   "s_cbranch_scc1 L_w4_pref_%=\n" \
   "s_mov_b32 m0, %[dbase]\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo0], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo0], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo1], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo1], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo2], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo2], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo6], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo6], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo7], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo7], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo8], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo8], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo9], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo9], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo10], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo10], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo12], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo12], %[srdB], %[k0] offen lds\n" \
   "s_xor_b32 m0, %[dbase], 0x10000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo0], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo0], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo1], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo1], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo2], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo2], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo6], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo6], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo7], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo7], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo8], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo8], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo9], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo9], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo10], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo10], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo12], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo12], %[srdB], %[k1] offen lds\n" \
   "s_waitcnt vmcnt(13)\n" \
   "s_branch L_w4_go_%=\n" \
   "L_w4_pref_%=:\n" \
@@ -8065,6 +8105,8 @@
   "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
+  "s_cmp_eq_u32 %[koff], %[kend]\n" \
+  "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
@@ -8213,6 +8255,8 @@
   "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
+  "s_cmp_eq_u32 %[koff], %[kend]\n" \
+  "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
@@ -8493,82 +8537,82 @@
   "s_cbranch_scc1 L_w4_end_%=\n" \
   "s_mov_b32 m0, %[dbase]\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn0], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn0], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn1], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn1], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn2], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn2], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn3], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn3], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn4], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn4], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn5], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn5], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn6], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn6], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn7], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn7], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn8], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn8], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn9], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn9], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn10], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn10], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn11], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn11], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn12], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn12], %[srdB], %[n0] offen lds\n" \
   "s_xor_b32 m0, %[dbase], 0x10000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn0], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn0], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn1], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn1], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn2], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn2], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn3], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn3], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn4], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn4], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn5], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn5], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn6], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn6], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn7], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn7], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn8], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn8], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn9], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn9], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn10], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn10], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn11], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn11], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn12], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn12], %[srdB], %[n1] offen lds\n" \
   "L_w4_end_%=:\n" \
   "s_nop 7\n" \
   "s_nop 7\n" \
@@ -8583,82 +8627,82 @@
   "s_cbranch_scc1 L_w4_pref_%=\n" \
   "s_mov_b32 m0, %[dbase]\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo0], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo0], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo1], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo1], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo2], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo2], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo6], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo6], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo7], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo7], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo8], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo8], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo9], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo9], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo10], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo10], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo12], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo12], %[srdB], %[k0] offen lds\n" \
   "s_xor_b32 m0, %[dbase], 0x10000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo0], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo0], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo1], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo1], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo2], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo2], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo6], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo6], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo7], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo7], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo8], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo8], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo9], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo9], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo10], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo10], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo12], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo12], %[srdB], %[k1] offen lds\n" \
   "s_waitcnt vmcnt(13)\n" \
   "s_branch L_w4_go_%=\n" \
   "L_w4_pref_%=:\n" \
@@ -8779,6 +8823,8 @@
   "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
+  "s_cmp_eq_u32 %[koff], %[kend]\n" \
+  "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
@@ -8927,6 +8973,8 @@
   "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
+  "s_cmp_eq_u32 %[koff], %[kend]\n" \
+  "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
@@ -9207,82 +9255,82 @@
   "s_cbranch_scc1 L_w4_end_%=\n" \
   "s_mov_b32 m0, %[dbase]\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn0], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn0], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn1], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn1], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn2], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn2], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn3], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn3], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn4], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn4], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn5], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn5], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn6], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn6], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn7], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn7], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn8], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn8], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn9], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn9], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn10], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn10], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn11], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn11], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn12], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn12], %[srdB], %[n0] offen lds\n" \
   "s_xor_b32 m0, %[dbase], 0x10000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn0], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn0], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn1], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn1], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn2], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn2], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn3], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn3], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn4], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn4], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn5], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn5], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn6], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn6], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn7], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn7], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn8], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn8], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn9], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn9], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn10], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn10], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn11], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn11], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn12], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn12], %[srdB], %[n1] offen lds\n" \
   "L_w4_end_%=:\n" \
   "s_nop 7\n" \
   "s_nop 7\n" \
@@ -9297,88 +9345,88 @@
   "s_cbranch_scc1 L_w4_pref_%=\n" \
   "s_mov_b32 m0, %[dbase]\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo0], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo0], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo1], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo1], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo2], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo2], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo6], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo6], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo7], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo7], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo8], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo8], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo9], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo9], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo10], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo10], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo12], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo12], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo13], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo13], %[srdB], %[k0] offen lds\n" \
   "s_xor_b32 m0, %[dbase], 0x10000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo0], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo0], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo1], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo1], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo2], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo2], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo6], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo6], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo7], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo7], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo8], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo8], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo9], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo9], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo10], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo10], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo12], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo12], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo13], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo13], %[srdB], %[k1] offen lds\n" \
   "s_waitcnt vmcnt(14)\n" \
   "s_branch L_w4_go_%=\n" \
   "L_w4_pref_%=:\n" \
@@ -9516,6 +9564,8 @@
   "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
+  "s_cmp_eq_u32 %[koff], %[kend]\n" \
+  "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
@@ -9684,6 +9734,8 @@
   "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
+  "s_cmp_eq_u32 %[koff], %[kend]\n" \
+  "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
@@ -10005,88 +10057,88 @@
   "s_cbranch_scc1 L_w4_end_%=\n" \
   "s_mov_b32 m0, %[dbase]\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn0], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn0], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn1], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn1], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn2], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn2], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn3], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn3], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn4], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn4], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn5], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn5], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn6], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn6], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn7], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn7], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn8], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn8], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn9], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn9], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn10], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn10], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn11], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn11], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn12], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn12], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn13], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn13], %[srdB], %[n0] offen lds\n" \
   "s_xor_b32 m0, %[dbase], 0x10000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn0], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn0], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn1], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn1], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn2], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn2], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn3], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn3], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn4], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn4], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn5], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn5], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn6], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn6], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn7], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn7], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn8], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn8], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn9], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn9], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn10], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn10], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn11], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn11], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn12], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn12], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn13], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn13], %[srdB], %[n1] offen lds\n" \
   "L_w4_end_%=:\n" \
   "s_nop 7\n" \
   "s_nop 7\n" \
@@ -10101,88 +10153,88 @@
   "s_cbranch_scc1 L_w4_pref_%=\n" \
   "s_mov_b32 m0, %[dbase]\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo0], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo0], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo1], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo1], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo2], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo2], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo6], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo6], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo7], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo7], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo8], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo8], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo9], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo9], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo10], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo10], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo12], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo12], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo13], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo13], %[srdB], %[k0] offen lds\n" \
   "s_xor_b32 m0, %[dbase], 0x10000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo0], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo0], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo1], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo1], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo2], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo2], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo6], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo6], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo7], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo7], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo8], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo8], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo9], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo9], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo10], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo10], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo12], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo12], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo13], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo13], %[srdB], %[k1] offen lds\n" \
   "s_waitcnt vmcnt(14)\n" \
   "s_branch L_w4_go_%=\n" \
   "L_w4_pref_%=:\n" \
@@ -10320,6 +10372,8 @@
   "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
+  "s_cmp_eq_u32 %[koff], %[kend]\n" \
+  "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
@@ -10488,6 +10542,8 @@
   "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
+  "s_cmp_eq_u32 %[koff], %[kend]\n" \
+  "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
@@ -10809,88 +10865,88 @@
   "s_cbranch_scc1 L_w4_end_%=\n" \
   "s_mov_b32 m0, %[dbase]\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn0], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn0], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn1], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn1], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn2], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn2], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn3], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn3], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn4], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn4], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn5], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn5], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn6], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn6], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn7], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn7], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn8], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn8], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn9], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn9], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn10], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn10], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn11], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn11], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn12], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn12], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn13], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn13], %[srdB], %[n0] offen lds\n" \
   "s_xor_b32 m0, %[dbase], 0x10000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn0], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn0], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn1], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn1], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn2], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn2], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn3], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn3], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn4], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn4], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn5], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn5], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn6], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn6], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn7], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn7], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn8], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn8], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn9], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn9], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn10], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn10], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn11], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn11], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn12], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn12], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn13], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn13], %[srdB], %[n1] offen lds\n" \
   "L_w4_end_%=:\n" \
   "s_nop 7\n" \
   "s_nop 7\n" \
@@ -10905,88 +10961,88 @@
   "s_cbranch_scc1 L_w4_pref_%=\n" \
   "s_mov_b32 m0, %[dbase]\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo0], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo0], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo1], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo1], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo2], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo2], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo6], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo6], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo7], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo7], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo8], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo8], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo9], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo9], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo10], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo10], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo12], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo12], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo13], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo13], %[srdB], %[k0] offen lds\n" \
   "s_xor_b32 m0, %[dbase], 0x10000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo0], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo0], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo1], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo1], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo2], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo2], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo6], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo6], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo7], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo7], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo8], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo8], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo9], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo9], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo10], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo10], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo12], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo12], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo13], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo13], %[srdB], %[k1] offen lds\n" \
   "s_waitcnt vmcnt(14)\n" \
   "s_branch L_w4_go_%=\n" \
   "L_w4_pref_%=:\n" \
@@ -11124,6 +11180,8 @@
   "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
+  "s_cmp_eq_u32 %[koff], %[kend]\n" \
+  "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
@@ -11292,6 +11350,8 @@
   "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
+  "s_cmp_eq_u32 %[koff], %[kend]\n" \
+  "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
@@ -11613,88 +11673,88 @@
   "s_cbranch_scc1 L_w4_end_%=\n" \
   "s_mov_b32 m0, %[dbase]\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn0], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn0], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn1], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn1], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn2], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn2], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn3], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn3], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn4], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn4], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn5], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn5], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn6], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn6], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn7], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn7], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn8], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn8], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn9], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn9], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn10], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn10], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn11], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn11], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn12], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn12], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn13], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn13], %[srdB], %[n0] offen lds\n" \
   "s_xor_b32 m0, %[dbase], 0x10000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn0], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn0], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn1], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn1], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn2], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn2], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn3], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn3], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn4], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn4], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn5], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn5], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn6], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn6], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn7], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn7], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn8], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn8], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn9], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn9], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn10], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn10], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn11], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn11], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn12], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn12], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn13], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn13], %[srdB], %[n1] offen lds\n" \
   "L_w4_end_%=:\n" \
   "s_nop 7\n" \
   "s_nop 7\n" \
@@ -11709,88 +11769,88 @@
   "s_cbranch_scc1 L_w4_pref_%=\n" \
   "s_mov_b32 m0, %[dbase]\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo0], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo0], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo1], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo1], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo2], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo2], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdA], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo6], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo6], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo7], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo7], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo8], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo8], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo9], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo9], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo10], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo10], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo12], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo12], %[srdB], %[k0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo13], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vo13], %[srdB], %[k0] offen lds\n" \
   "s_xor_b32 m0, %[dbase], 0x10000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo0], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo0], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo1], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo1], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo2], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo2], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdA], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo6], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo6], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo7], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo7], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo8], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo8], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo9], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo9], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo10], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo10], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo12], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo12], %[srdB], %[k1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vo13], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vo13], %[srdB], %[k1] offen lds\n" \
   "s_waitcnt vmcnt(14)\n" \
   "s_branch L_w4_go_%=\n" \
   "L_w4_pref_%=:\n" \
@@ -11928,6 +11988,8 @@
   "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
+  "s_cmp_eq_u32 %[koff], %[kend]\n" \
+  "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
@@ -12096,6 +12158,8 @@
   "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
+  "s_cmp_eq_u32 %[koff], %[kend]\n" \
+  "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
@@ -12417,88 +12481,88 @@
   "s_cbranch_scc1 L_w4_end_%=\n" \
   "s_mov_b32 m0, %[dbase]\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn0], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn0], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn1], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn1], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn2], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn2], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn3], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn3], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn4], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn4], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn5], %[srdA], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn5], %[srdA], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn6], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn6], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn7], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn7], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn8], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn8], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn9], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn9], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn10], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn10], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn11], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn11], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn12], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn12], %[srdB], %[n0] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn13], %[srdB], 0 offen lds\n" \
+  "buffer_load_dwordx4 %[vn13], %[srdB], %[n0] offen lds\n" \
   "s_xor_b32 m0, %[dbase], 0x10000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn0], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn0], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn1], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn1], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn2], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn2], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn3], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn3], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn4], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn4], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn5], %[srdA], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn5], %[srdA], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn6], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn6], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn7], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn7], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn8], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn8], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn9], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn9], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn10], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn10], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn11], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn11], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn12], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn12], %[srdB], %[n1] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "s_nop 0\n" \
-  "buffer_load_dwordx4 %[vn13], %[srdB], %[k128] offen lds\n" \
+  "buffer_load_dwordx4 %[vn13], %[srdB], %[n1] offen lds\n" \
   "L_w4_end_%=:\n" \
   "s_nop 7\n" \
   "s_nop 7\n" \

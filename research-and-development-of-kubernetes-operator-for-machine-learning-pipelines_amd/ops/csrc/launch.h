@@ -137,6 +137,10 @@ bool gemm_sk_scratch(float** ws, int** cnt, int* cus);
 bool gemm_sk_available(int* cus);
 bool run_w4(int epi, const uint16_t* A, int lda, const uint16_t* B, int ldb, uint16_t* C, int ldc, int M, int N,
             int K, hipStream_t st, const RopeEpi& re, int bm = 256);
+// the experts' products on it (offsets on the device; a_n: A's rows)
+bool gemm_w4_grouped_ok(int M, int N, int K, int n_groups, int a_n);
+void run_w4_grouped(int epi, const uint16_t* A, int lda, const uint16_t* B, int ldb, uint16_t* C, int ldc, int M, int N,
+                    int K, hipStream_t st, const RopeEpi& re, const int* offsets, int n_groups);
 // norm chain on the four-wave kernel (epi flags: 4 = C += A.B^T with ss partials, 8 = rows scaled
 // by re.ss_in; 4, 0|8, 1|8, 3|8 are built): true when every such GEMM of this shape runs there
 bool w4_chain_ok(int M, int N, int K);
@@ -217,7 +221,7 @@ bool launch_gemm_add_rmsnorm(const void* A, int lda, const void* B, void* out, v
 void launch_grouped_gemm(const void* A, const void* B, void* C, const int* offsets, int n_groups,
                          int M, int N, int K, int max_rows, int epi, hipStream_t st, const int* a_rows = nullptr,
                          float** defer_ws = nullptr, int* defer_splits = nullptr,
-                         const float* row_scale = nullptr, float p0 = 0.f, float p1 = 0.f);
+                         const float* row_scale = nullptr, float p0 = 0.f, float p1 = 0.f, int a_n = 0);
 bool launch_moe_down_combine_add_rmsnorm(void* out, void* residual, void* y, const void* a, const void* w2,
                                          const int* offsets, int n_groups, int R, int H, int I, int max_rows,
                                          const int* inv, const float* topw, const void* norm_w, float eps, int T,

@@ -163,6 +163,8 @@ def body(s: Stream, sc: Sched, kind: str, first: bool = False):
             if k < sc.npc - 1:
                 slots[m].append(("emit", "s_add_u32 m0, m0, 0x1000"))
         slots[sc.dma[-1] + 1].append(("emit", "s_add_u32 %[koff], %[koff], 0x80"))
+        slots[sc.dma[-1] + 1].append(("emit", "s_cmp_eq_u32 %[koff], %[kend]"))
+        slots[sc.dma[-1] + 1].append(("emit", "s_cselect_b32 %[koff], 0, %[koff]"))
         slots[sc.dma[-1] + 1].append(("emit", "s_xor_b32 %[dbase], %[dbase], 0x10000"))
     slots[sc.toggle1].append(("emit", "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]"))
     slots[sc.toggle1].append(("emit", "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]"))
@@ -204,13 +206,14 @@ def suffix(q, q0):
 
 
 def issue_two(s: Stream, vo: str, sc: Sched):
-    """LDS-DMA of a tile's K-tiles 0 and 1 into buffers 0 and 1 (per-lane offsets %[{vo}k])."""
+    """LDS-DMA of a tile's first two K-tiles (byte offsets %[k0] / %[k1], for the next tile %[n0] / %[n1]) into
+    buffers 0 and 1 (per-lane offsets %[{vo}k])."""
     for t in range(2):
         s.emit("s_mov_b32 m0, %[dbase]" if t == 0 else "s_xor_b32 m0, %[dbase], 0x10000")
         s.emit("s_nop 0")
         for k in range(sc.npc):
             srd = "srdA" if k < sc.na else "srdB"
-            soff = "0" if t == 0 else "%[k128]"
+            soff = f"%[{'k' if vo == 'vo' else 'n'}{t}]"
             s.emit(f"buffer_load_dwordx4 %[{vo}{k}], %[{srd}], {soff} offen{sc.pol[srd]} lds")
             if k < sc.npc - 1:
                 s.emit("s_add_u32 m0, m0, 0x1000")

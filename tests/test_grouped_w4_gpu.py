@@ -1,0 +1,64 @@
+"""The experts' products on four-wave tiles (gemm_w4_grouped_kernel, gate_up of prompts) against fp32: routings that
+lead to each tile height, empty and full experts, gathered rows, every epilogue, with and without the K-half tail."""
+import pytest
+import torch
+
+from mlopamd import ops
+
+pytestmark = pytest.mark.gpu
+bf = torch.bfloat16
+G, N = 8, 24576
+
+COUNTS = {
+    "even-150": [150] * G,  # one tile of 160 rows each
+    "one-row-over": [161, 193, 257, 160, 192, 256, 1, 0],
+    "one-expert": [0, 0, 0, 0, 0, 0, 0, 613],
+    "first-and-last": [257, 0, 0, 0, 0, 0, 0, 300],
+    "even-190": [190] * G,
+    "even-250": [250, 256, 249, 255, 251, 256, 240, 256],
+    "skewed": [1500, 3, 17, 0, 64, 5, 90, 700],
+    "single-row": [0, 0, 0, 1, 0, 0, 0, 0],
+}
+
+
+def glu(z, lim):
+    g, u = ops.deinterleave_cols(z).chunk(2, -1)
+    if lim is None:
+        return g, u, g * g.sigmoid() * u
+    gc, uc = g.clamp(max=lim[1]), u.clamp(-lim[1], lim[1])
+    return gc, uc + 1, gc * (lim[0] * gc).sigmoid() * (uc + 1)
+
+
+@pytest.mark.parametrize("counts", COUNTS.values(), ids=COUNTS.keys())
+@pytest.mark.parametrize("K", [192, 448, 1536])
+@pytest.mark.parametrize("kind", ["plain", "silu", "gathered", "scaled", "clamped"])
+def test_grouped(gpu, counts, K, kind):
+    torch.manual_seed(K + sum(counts))
+    off = torch.tensor([0] + counts, device=gpu).cumsum(0).int()
+    R = int(off[-1])
+    w = 0.05 * torch.randn(G, N, K, device=gpu, dtype=bf)
+    gather = kind not in ("plain", "silu")
+    toks = torch.randn(R // 2 + 1 if gather else R, K, device=gpu, dtype=bf)
+    rows = torch.randint(0, toks.shape[0], (R,), device=gpu, dtype=torch.int32) if gather else None
+    scale = 0.5 + torch.rand(R, device=gpu) if kind == "scaled" else None
+    lim = (1.702, 3.0) if kind == "clamped" else None
+    epi = 0 if kind == "plain" else 1
+    got = [ops.grouped_gemm(toks, w, off, epi=epi, avg_rows=64, a_rows=rows,
+                            row_scale=scale, glu=lim) for _ in range(8)]
+    assert all(torch.equal(got[0], g) for g in got[1:])
+    x = toks[rows.long()] if gather else toks
+    for e in range(G):
+        a, b = int(off[e]), int(off[e + 1])
+        if a == b:
+            continue
+        xe, we = x[a:b].float(), w[e].float()
+        y, sums = xe @ we.t(), 2.0 ** -20 * (xe.abs() @ we.abs().t())  # fp32 sums in another order
+        if scale is not None:
+            y, sums = y * scale[a:b, None], sums * scale[a:b, None]
+        if epi == 0:
+            exp, bound = y, 2.0 ** -8 * y.abs() + 2 * sums
+        else:  # roundings of gate, up, the gated half and the product; |d (g sigmoid) / dg| <= 1.1
+            g, u, exp = glu(y, lim)
+            sg, su = ops.deinterleave_cols(sums).chunk(2, -1)
+            bound = 4 * 2.0 ** -8 * g.abs() * (u.abs() + (lim is not None)) + 1.1 * sg * u.abs() + su * g.abs()
+        assert ((got[0][a:b].float() - exp).abs() <= bound + 1e-5).all(), e
