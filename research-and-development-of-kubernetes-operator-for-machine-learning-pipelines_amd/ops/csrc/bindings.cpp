@@ -107,6 +107,36 @@ void embedding(Tensor out, Tensor table, Tensor ids, int64_t vocab_start) {
                          cur_stream());
 }
 
+// runs: (offset, length) pairs in int32 words, then rows, columns, pitch, offset of a block; all but rows even
+void upload(Tensor dst, Tensor src, at::IntArrayRef runs) {
+  check_i32(dst, "dst");
+  TORCH_CHECK(src.is_cpu() && src.scalar_type() == at::kInt && src.is_contiguous(), "src: pinned int32");
+  const int64_t cap = std::min(dst.numel(), src.numel()), n = ((int64_t)runs.size() - 4) / 2;
+  TORCH_CHECK(runs.size() >= 4 && runs.size() % 2 == 0 && n <= mlop::UploadRuns::kMax && cap < (1l << 31), "upload runs");
+  mlop::UploadRuns r{};
+  int64_t total = 0;
+  for (size_t i = 0; i < runs.size(); ++i)
+    TORCH_CHECK(runs[i] >= 0 && runs[i] <= cap && (runs[i] % 2 == 0 || (int64_t)i == 2 * n), "upload runs");
+  for (r.n = 0; r.n < n; ++r.n) {
+    const int64_t off = runs[2 * r.n], len = runs[2 * r.n + 1];
+    TORCH_CHECK(off + len <= cap, "upload run past the end");
+    r.off[r.n] = (int)(off / 2), r.len[r.n] = (int)(len / 2);
+    total += len / 2;
+  }
+  const int64_t rows = runs[2 * n], cols = runs[2 * n + 1], pitch = runs[2 * n + 2], base = runs[2 * n + 3];
+  if (rows > 0 && cols > 0) {
+    TORCH_CHECK(cols <= pitch && base + (rows - 1) * pitch + cols <= cap, "upload block past the end");
+    r.rows = (int)rows, r.cols = (int)(cols / 2), r.pitch = (int)(pitch / 2), r.base = (int)(base / 2);
+    total += rows * (cols / 2);
+  }
+  TORCH_CHECK(total < (1l << 31), "upload runs");
+  c10::DeviceGuard g(dst.device());
+  void* dev = nullptr;  // the buffer as the device sees it; fails for memory that is not pinned
+  TORCH_CHECK(hipHostGetDevicePointer(&dev, src.data_ptr(), 0) == hipSuccess && dev != nullptr, "upload: src is not pinned");
+  TORCH_CHECK(((uintptr_t)dev | (uintptr_t)dst.data_ptr()) % 8 == 0, "upload: 8-byte alignment");
+  mlop::launch_upload(dst.data_ptr(), dev, r, (int)total, cur_stream());
+}
+
 void flash_prefill(Tensor out, Tensor q, Tensor k_cache, Tensor v_cache, Tensor block_tables,
                    Tensor ptile_seq, Tensor ptile_q0, Tensor q_start, Tensor q_len, Tensor ctx_len,
                    double scale) {
@@ -965,6 +995,7 @@ TORCH_LIBRARY(mlop, m) {
         "Tensor pos, Tensor cos_sin, Tensor slots) -> ()");
   m.def("silu_mul(Tensor(a!) out, Tensor x, int interleaved=0) -> ()");
   m.def("embedding(Tensor(a!) out, Tensor table, Tensor ids, int vocab_start) -> ()");
+  m.def("upload(Tensor(a!) dst, Tensor src, int[] runs) -> ()");
   m.def("gemm_ws(Tensor(a!) out, Tensor a, Tensor w, int epi, bool rs, float eps) -> bool");
   m.def("flash_prefill(Tensor(a!) out, Tensor q, Tensor k_cache, Tensor v_cache, Tensor block_tables, "
         "Tensor ptile_seq, Tensor ptile_q0, Tensor q_start, Tensor q_len, Tensor ctx_len, float scale) -> ()");
@@ -980,6 +1011,7 @@ TORCH_LIBRARY_IMPL(mlop, CUDA, m) {
   m.impl("rope_cache", &rope_cache);
   m.impl("silu_mul", &silu_mul);
   m.impl("embedding", &embedding);
+  m.impl("upload", &upload);
   m.impl("paged_attention", &paged_attention);
   m.impl("flash_prefill", &flash_prefill);
   m.impl("gemm", &gemm);

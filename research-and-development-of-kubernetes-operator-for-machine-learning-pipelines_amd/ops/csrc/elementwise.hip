@@ -1,4 +1,4 @@
-// Element-wise / gather kernels: SiLU-and-mul (K8) and embedding row gather (K9).
+// Element-wise / gather kernels: SiLU-and-mul (K8), embedding row gather (K9), the step's upload.
 // Memory-bound: 16-byte vectors per lane, grid-stride (cdna_hip_programming.md Guideline 11/13).
 #include "common.h"
 #include "launch.h"
@@ -63,6 +63,26 @@ void launch_embedding(void* out, const void* table, const long* ids, int T, int 
   if (T == 0) return;
   embedding_kernel<<<T, 256, 0, st>>>((uint16_t*)out, (const uint16_t*)table, ids, H, vocab_start,
                                       vocab_end);
+}
+
+// A step's host arrays to the device: runs of 8-byte words of one pinned buffer to the same places of a device buffer,
+// then `rows` rows of `cols` words, `pitch` apart.  Bound by a trip over the bus: every lane moves one word, and only
+// what the step wrote, where the copy engine moved one range, the whole capacity of every array (a step of 1 / 700 /
+// 7900 tokens 15 / 28 / 15 -> 3.8 / 8.3 / 8.8 us).  System-scope loads: the host rewrites the buffer between steps, no
+// cache may serve it.
+__global__ void __launch_bounds__(256) upload_kernel(unsigned long long* __restrict__ dst, const unsigned long long* __restrict__ src,
+                                                     UploadRuns r, int total) {
+  for (int i = blockIdx.x * 256 + threadIdx.x; i < total; i += gridDim.x * 256) {
+    int at = i, k = 0;
+    while (k < r.n && at >= r.len[k]) at -= r.len[k++];
+    const long w = k < r.n ? r.off[k] + at : r.base + (long)(at / r.cols) * r.pitch + at % r.cols;
+    dst[w] = __hip_atomic_load(src + w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+
+void launch_upload(void* dst, const void* src, const UploadRuns& r, int total, hipStream_t st) {
+  if (total <= 0) return;
+  upload_kernel<<<std::min((total + 255) / 256, 1024), 256, 0, st>>>((unsigned long long*)dst, (const unsigned long long*)src, r, total);
 }
 
 // Fault injection only (MLOP_INJECT_STEP_DEVICE_US, runtime/engine.py): one wave that waits until

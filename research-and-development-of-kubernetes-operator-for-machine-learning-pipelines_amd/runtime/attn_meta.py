@@ -179,7 +179,7 @@ class MetaBuffers:
         # metadata views keep their old names; offsets in self.off are into the whole buffer
         self.h, self.d = self.hbuf, self.dbuf
         self.hn = self.hbuf.numpy()
-        self._meta_hi = meta_hi
+        self._meta_hi, self._ids_lo, self._lidx_lo = meta_hi, ids_lo, lidx_lo
         self.ids_h = self.hbuf[ids_lo:ids_lo + 2 * max_tokens].view(torch.int64)
         self.ids_hn = self.ids_h.numpy()
         self.ids_d = self.dbuf[ids_lo:ids_lo + 2 * max_tokens].view(torch.int64)
@@ -215,9 +215,24 @@ class MetaBuffers:
 
     def upload(self, n_ids: int = 0, n_logits: int = 0, rows_hi: int | None = None):
         """ONE async H2D of header + metadata + ids + logits index (+ the block-table rows in
-        use) on the current stream."""
+        use) on the current stream: of the per-token arrays the first ``n_ids`` entries (a step's tokens,
+        tiles and flash tiles are no more), of the logits index ``n_logits``, of a block-table row the pages
+        up to the longest context."""
         n = self.extent(rows_hi)
-        self.dbuf[:n].copy_(self.hbuf[:n], non_blocking=True)
+        if self.device.type != "cuda" or not n_ids or rows_hi is None or self.mb % 2:
+            self.dbuf[:n].copy_(self.hbuf[:n], non_blocking=True)
+            return
+        t = n_ids + n_ids % 2  # (every array is padded to 64 words)
+        rows = min(max(0, rows_hi), self.max_seqs)
+        cols = 0
+        if rows:
+            pages = -(-int(self.view_h("ctx_len")[:rows].max()) // BLOCK_SIZE)
+            cols = min(self.mb, (pages + 3) // 4 * 4)
+        off = self.off
+        torch.ops.mlop.upload(self.dbuf, self.hbuf, [
+            0, self.HDR + t, off["slots"][0], t, off["tile_seq"][0], t, off["tile_q0"][0], t,
+            off["ptile_seq"][0], t, off["ptile_q0"][0], t, off["q_start"][0], self._meta_hi - off["q_start"][0],
+            self._ids_lo, 2 * t, self._lidx_lo, 2 * n_logits, rows, cols, self.mb, off["block_tables"][0]])
 
     def set_header(self, vals) -> None:
         self.hdr_hn[:len(vals)] = vals
