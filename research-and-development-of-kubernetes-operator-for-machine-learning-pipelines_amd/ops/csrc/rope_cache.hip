@@ -19,23 +19,40 @@ namespace mlop {
 // to bf16 (splitk_reduce_kernel's order and rounding), so one launch replaces reduce + RoPE.
 // f: the row's RMSNorm factor of the mid norm chain (1 otherwise), applied to the summed
 // accumulators before the bf16 rounding (W4_RS's order)
-template <bool SLABS>
-__device__ __forceinline__ u32x4 load8(const uint16_t* row, const float* ws, int t, int T, int stride,
-                                       int splits, int col, float f = 1.f) {
+// NV vectors' slabs are loaded together, four slabs at a time: a loop over the slabs waited for each in turn, 1 + 2
+// splits trips to memory per rotated pair (100 / 150 rows, 4 slabs: 8.4 and 9.3 us a call, now 6.2 and 6.9).
+template <bool SLABS, int NV>
+__device__ __forceinline__ void load8(const uint16_t* row, const float* ws, int t, int T, int stride, int splits,
+                                      const int (&col)[NV], float f, u32x4 (&o)[NV]) {
   if constexpr (!SLABS) {
-    return *reinterpret_cast<const u32x4*>(row + col);
-  } else {
-    float a[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    for (int s = 0; s < splits; ++s) {
-      const float4* p = reinterpret_cast<const float4*>(ws + ((size_t)s * T + t) * stride + col);
-      const float4 x = p[0], y = p[1];
-      a[0] += x.x; a[1] += x.y; a[2] += x.z; a[3] += x.w;
-      a[4] += y.x; a[5] += y.y; a[6] += y.z; a[7] += y.w;
-    }
-    u32x4 o;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) o[j] = pack2(a[2 * j] * f, a[2 * j + 1] * f);
-    return o;
+    for (int v = 0; v < NV; ++v) o[v] = *reinterpret_cast<const u32x4*>(row + col[v]);
+  } else {
+    float a[NV][8] = {};
+    for (int s0 = 0; s0 < splits; s0 += 4) {
+      float4 x[NV][4], y[NV][4];
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+        if (s0 + s < splits)
+#pragma unroll
+          for (int v = 0; v < NV; ++v) {
+            const float4* p = reinterpret_cast<const float4*>(ws + ((size_t)(s0 + s) * T + t) * stride + col[v]);
+            x[v][s] = p[0];
+            y[v][s] = p[1];
+          }
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+        if (s0 + s < splits)
+#pragma unroll
+          for (int v = 0; v < NV; ++v) {
+            a[v][0] += x[v][s].x; a[v][1] += x[v][s].y; a[v][2] += x[v][s].z; a[v][3] += x[v][s].w;
+            a[v][4] += y[v][s].x; a[v][5] += y[v][s].y; a[v][6] += y[v][s].z; a[v][7] += y[v][s].w;
+          }
+    }
+#pragma unroll
+    for (int v = 0; v < NV; ++v)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) o[v][j] = pack2(a[v][2 * j] * f, a[v][2 * j + 1] * f);
   }
 }
 
@@ -64,11 +81,12 @@ __global__ void __launch_bounds__(256) rope_cache_kernel(
     if (it < n_rope) {
       const int h = it / vph, c = (it % vph) * 8;
       // q heads then k heads are contiguous
-      u32x4 a = load8<SLABS>(row, ws, t, T, qkv_stride, splits, h * D + c, f);
-      u32x4 b = load8<SLABS>(row, ws, t, T, qkv_stride, splits, h * D + half + c, f);
       const float4* cp = reinterpret_cast<const float4*>(cs + c);
       const float4* sp = reinterpret_cast<const float4*>(cs + half + c);
       float4 c0 = cp[0], c1 = cp[1], s0 = sp[0], s1 = sp[1];
+      u32x4 ab[2];
+      load8<SLABS, 2>(row, ws, t, T, qkv_stride, splits, {h * D + c, h * D + half + c}, f, ab);
+      const u32x4 a = ab[0], b = ab[1];
       float cc[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
       float ss[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
       u32x4 oa, ob;
@@ -92,8 +110,9 @@ __global__ void __launch_bounds__(256) rope_cache_kernel(
     } else if (slot >= 0) {
       const int iv = it - n_rope;
       const int kh = iv / (D >> 3), c = (iv % (D >> 3)) * 8;
-      u32x4 a = load8<SLABS>(row, ws, t, T, qkv_stride, splits, (Hq + Hkv + kh) * D + c, f);
-      *reinterpret_cast<u32x4*>(v_cache + (((size_t)blk * Hkv + kh) * BS + off) * D + c) = a;
+      u32x4 a[1];
+      load8<SLABS, 1>(row, ws, t, T, qkv_stride, splits, {(Hq + Hkv + kh) * D + c}, f, a);
+      *reinterpret_cast<u32x4*>(v_cache + (((size_t)blk * Hkv + kh) * BS + off) * D + c) = a[0];
     }
   }
 }
