@@ -1372,8 +1372,10 @@ static bool mid_plan(int M, int N, int K, Plan& p) {
 // by estimated time in us.  A round of 256-row tiles takes 5.6 + 0.0212 K; lower tiles cost more per row (192 rows 0.80
 // of it, 160 0.725, 128 0.61: fewer MFMAs per fragment read), and an only round that fills a share f of the CUs runs
 // faster, the less the lower the tile.  A tail of at most half the CUs is cut into K-halves: half a round and the
-// hand-off of the partials (behind whole rounds the more the more of them there are).  The ping-pong kernel cuts every tile of a grid of up to half the CUs, runs a round as it
-// is above that, and spreads the remainder of several evenly at 1.08 of a round's rate.
+// hand-off of the partials (behind whole rounds the more the more of them there are).  The ping-pong kernel cuts every
+// tile of a grid of up to half the CUs and skips empty 64-row quadrants there (down at 520 / 560 rows 86 / 87 us, the
+// best four-wave height 94 / 98), runs a round as it is above that, and spreads the remainder of several evenly at 1.08
+// of a round's rate.
 // Constants fitted to qkv, o, gate_up, down and lm_head of Llama-3-8B at 17 row counts from 400 to 4096, every variant
 // measured: the choice is within 5 % of the best of the five at all of them.  Against the earlier rule (heights 256 and
 // 128 only): gate_up at M = 400 / 700 / 1152 138 -> 92, 158 -> 147, 245 -> 219 us, o at 1152 / 2300 / 2600 55 -> 43,
@@ -1386,7 +1388,9 @@ static bool big_plan(int M, int N, int K, bool pp_ok, Plan& p) {
   constexpr Tile tiles[] = {{256, 1.f, .55f}, {192, .80f, .55f}, {160, .725f, .35f}, {128, .61f, .10f}};
   const float full = 5.6f + 0.0212f * (float)K, C = (float)b->cus;
   const float f = (float)((M + 255) / 256) * (float)(N / 256) / C;  // rounds of 256-row tiles
-  float best = !pp_ok ? 1e30f : f <= .5f ? .87f * full * f + 28.f + .06f * full : f <= 1.f ? 1.11f * full * (.5f + .5f * f) : 1.08f * full * f + 25.f;
+  // (to 3/8 of the CUs without a tile's empty 64-row quadrants; nearer to half they no longer show)
+  const float fq = f > .375f ? f : (float)((M + 63) / 64) * (float)(N / 256) / (4.f * C);
+  float best = !pp_ok ? 1e30f : f <= .5f ? .87f * full * fq + 28.f + .06f * full : f <= 1.f ? 1.11f * full * (.5f + .5f * f) : 1.08f * full * f + 25.f;
   p.variant = 3;
   p.BM = p.BN = 256;
   for (const Tile& t : tiles) {
