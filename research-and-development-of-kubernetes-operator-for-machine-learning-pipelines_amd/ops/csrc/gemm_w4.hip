@@ -264,7 +264,7 @@ __device__ __forceinline__ void gemm_w4_tiles(
       asm volatile(
           "s_mov_b32 %[ms], m0\n"
           "s_mov_b32 m0, %[dst]\n"
-          "s_nop 0\n"
+          "s_nop 4\n"  // (the descriptor may come straight from v_readfirstlane / v_readlane)
           "buffer_load_dword %[vo], %[srd], 0 offen lds\n"
           "buffer_load_dword %[vo], %[srd], 0 offen lds\n"  // (twice: the built K-loops count two)
           "s_mov_b32 m0, %[ms]\n"
@@ -290,7 +290,7 @@ __device__ __forceinline__ void gemm_w4_tiles(
       asm volatile(
           "s_mov_b32 %[ms], m0\n"
           "s_mov_b32 m0, %[dst]\n"
-          "s_nop 0\n"
+          "s_nop 4\n"  // (the descriptor may come straight from v_readfirstlane / v_readlane)
           "buffer_load_dword %[vo], %[srd], 0 offen lds\n"
           "s_add_u32 m0, m0, 0x100\n"
           "s_nop 0\n"
