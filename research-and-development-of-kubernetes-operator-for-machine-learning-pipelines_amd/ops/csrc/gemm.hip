@@ -260,7 +260,7 @@ __global__ void __launch_bounds__(WM * WN * 64) gemm_kernel(
   const bool b_nt = re.b_nt != 0;
   // experts: column tile bx walks K from step bx % nk on (the channels of tiles in step: gemm_mid.hip; down of eight
   // experts at 20 rows 145 -> 140 us).  Dense split-K ranges are too short for it (qkv 17.5 -> 17.8)
-  const int rot = GROUPED ? bx % nk : 0;
+  const int rot = GROUPED && nk > 0 ? bx % nk : 0;
   auto issue = [&](int buf, int kt) {
     kt = kt + rot >= nk ? kt + rot - nk : kt + rot;
     uint16_t* base = smem + buf * STAGE;
@@ -1348,7 +1348,7 @@ static bool sk_halves_ok(long T, int nk) {
 // against 26.6 / 29.5); from 512 rows on the four-wave kernel is (gate_up 93 us against 115).
 static bool mid_plan(int M, int N, int K, Plan& p) {
   constexpr int max_m = 384, fill = 192;
-  if (M > max_m || K % kBK || N % 8) return false;
+  if (M > max_m || K < kBK || K % kBK || N % 8) return false;  // (no K-step: gemm_kernel writes the empty sums)
   const int m_tiles = M <= 256 ? 1 : 2, rows = (M + m_tiles - 1) / m_tiles;
   const int bm = rows <= 64 ? 64 : (rows + 31) / 32 * 32;
   const int t256 = (N + 255) / 256 * m_tiles, t128 = (N + 127) / 128 * m_tiles, nk = K / kBK;

@@ -501,6 +501,18 @@ def test_gemm_weight_stream(gpu, M, N, K, epi):
     assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
 
 
+@pytest.mark.parametrize("M", [16, 64, 100, 200, 300, 384])
+@pytest.mark.parametrize("N", [4096, 24576, 49152])
+@pytest.mark.parametrize("epi", [0, 1, 6])
+def test_gemm_without_terms(gpu, M, N, epi):
+    """K = 0: every sum is empty, so every output is zero (and the units of zero are)."""
+    x = torch.randn(M, 64, device=gpu, dtype=bf)[:, :0]
+    w = torch.empty(N, 0, device=gpu, dtype=bf)
+    out = torch.full((M, N // 2 if epi == 1 else N), float("nan"), device=gpu, dtype=bf)
+    torch.ops.mlop.gemm(out, x, w, torch.empty(0, device=gpu), epi)
+    assert (out == 0).all()
+
+
 @pytest.mark.parametrize("M,N,K,epi", [
     (2040, 28672, 4096, 1),   # 896 tiles: 768 data-parallel + 128 tail tiles in 2 halves (gate_up, SiLU)
     (4352, 4096, 14336, 0),   # 272 tiles: 16 tail tiles x 224 K-tiles in 8 ranges (re-read sum path)
