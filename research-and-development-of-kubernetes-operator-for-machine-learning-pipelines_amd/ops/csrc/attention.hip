@@ -97,13 +97,45 @@ __device__ __forceinline__ void vt_frag4(uint32_t b, bf16x8 (&f)[4]) {
 
 __device__ __forceinline__ int wid_of(unsigned t) { return __builtin_amdgcn_readfirstlane((int)(t >> 6)); }
 
-// Keys per partition of one sequence: the launch's nparts shares of its own keys, in page pairs.  A captured decode
-// step plans nparts for the longest context the engine admits; a fixed length cut for that one leaves shorter
-// sequences on a few workgroups (13 sequences of 2500 keys under a limit of 4096: 5 of 8 partitions).
-__device__ __forceinline__ int seq_part(int kv_end, int part_tokens, int nparts) {
+constexpr int kEnoughParts = 8;
+// Keys per partition of one sequence: `even` shares of its own keys where a launch's lengths are alike.  (A captured
+// decode step plans for the longest context the engine admits; a fixed length cut for that one leaves shorter
+// sequences on a few workgroups: 13 sequences of 2500 keys under a limit of 4096 on 5 of 8 partitions.)
+// A sequence of more than 1.6 times the launch's mean is what the launch would end on: it gets up to the nparts that
+// were planned, of a 512th of the launch's keys or 512 keys each (8 kv heads, whole or in two -> so: 1 x 4000 keys beside
+// 40 x 200 67 -> 28 us, 1 x 24000 beside 20 x 500 195 -> 102, 10 x 4000 beside 10 x 100 70 -> 43).  From kEnoughParts shares
+// on, further slabs cost what shorter walks save (2 x 16000 beside 2 x 200 in 8 shares 38.7 us, in 31 45.5).  Every
+// workgroup of the launch and the reduction sum the same integers.
+__device__ __forceinline__ int seq_part(int kv_end, int part_tokens, int nparts, int even, const int* tile_seq,
+                                        const int* ctx_len, int tiles, int Hkv) {
   constexpr int min_part = 128;  // attn_meta.MIN_PART
-  const int even = ((kv_end + nparts - 1) / nparts + 31) & ~31;
-  return nparts > 1 ? min(part_tokens, max(min_part, even)) : part_tokens;
+  constexpr int long_part = 512;
+  if (nparts == 1) return part_tokens;
+  int n = even;
+  if (even < nparts && kv_end > long_part * 3 / 2 * even) {  // (two long shares or more)
+    float sum = 0.f;  // (below 2^24 exact, above the same everywhere)
+    int live = 0;
+    for (int i = 0; i < tiles; i += 256) {
+      const int l = i + (threadIdx.x & 63);
+      int c[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) c[u] = tile_seq[min(l + 64 * u, tiles - 1)];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) c[u] = ctx_len[c[u]];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const bool in = l + 64 * u < tiles && c[u] > 0;
+        sum += in ? (float)c[u] : 0.f;
+        live += __popcll(__ballot(in));
+      }
+    }
+    const int keys = __builtin_amdgcn_readfirstlane((int)wave_sum(sum));  // (uniform: page numbers hang on it)
+    if (10l * kv_end * live > 16l * keys) {
+      const int share = max(long_part, (int)((long)keys * Hkv / 512));
+      n = max(even, min(nparts, (kv_end + share / 2) / share));
+    }
+  }
+  return max(min_part, ((kv_end + n - 1) / n + 31) & ~31);
 }
 
 // Row rr, dims c..c+7 of a (tile, kv head)'s combined output from its partitions' slabs.  Four partitions' loads
@@ -152,7 +184,7 @@ __global__ void __launch_bounds__(256, 3) paged_attn_kernel(
     const int* __restrict__ tile_seq, const int* __restrict__ tile_q0,
     const int* __restrict__ q_start, const int* __restrict__ q_len,
     const int* __restrict__ ctx_len, int Hq, int Hkv, float scale_log2, int part_tokens,
-    int nparts, int num_blocks, int* __restrict__ sem) {
+    int nparts, int even, int num_blocks, int* __restrict__ sem) {
   constexpr int QT = 16 / G;
   // (3 waves per SIMD: 154 VGPRs; asked for two fewer the compiler keeps O in AGPRs and copies it for every rescale)
   // wave w stages its page pair's V image (2 x 16 token rows x 256 B = 8 KB) inside sm_o[w]
@@ -170,7 +202,7 @@ __global__ void __launch_bounds__(256, 3) paged_attn_kernel(
   const int ql = q_len[s], ctx = ctx_len[s], qs = q_start[s];
   const int last_q = min(q0 + QT, ql) - 1;           // last valid query of the tile
   const int kv_end = last_q >= 0 ? ctx - ql + last_q + 1 : 0;
-  part_tokens = seq_part(kv_end, part_tokens, nparts);
+  part_tokens = seq_part(kv_end, part_tokens, nparts, even, tile_seq, ctx_len, gridDim.x, Hkv);
   const int p_begin = part * part_tokens;
   const int p_end = min(kv_end, p_begin + part_tokens);
   if (p_begin >= p_end) {                            // reducer skips empty partitions
@@ -249,6 +281,8 @@ __global__ void __launch_bounds__(256, 3) paged_attn_kernel(
   // A pair's K loads (registers) and V image (LDS) are issued a pair ahead: K(p + 4) as soon as the S MFMAs have
   // taken K(p), V(p + 4) as soon as the transposed reads have taken V(p).  The workgroups of a launch run in step, and
   // memory stood still while they all multiplied (100 sequences of 1000 keys 96.7 -> 90.2 us, 64 of 4000 217 -> 196).
+  // K is in flight under the softmax and P.V; V only from its issue to the loop's top, where the compiler waits for
+  // everything (vmcnt(0) before the first S MFMA: it does not count loads into registers apart from the LDS-DMA).
   int pgA = 0, pgB = 0, rawA = 0, rawB = 0;  // page ids of the pair whose K is loading; the next pair's as read
   auto load_pages = [&](int pp) {  // (past the end: entries of the row, never used)
     rawA = bt[min(2 * pp, bt_stride - 1)];
@@ -260,8 +294,7 @@ __global__ void __launch_bounds__(256, 3) paged_attn_kernel(
   };
   int pp = pp_begin + wid_of(threadIdx.x);
   {
-    // (a wave without a pair loads the last one and waits for it: a branch here would make every wait in the loop
-    // one for everything)
+    // (a wave without a pair loads the last one and waits for it)
     const int first = min(pp, pp_end - 1);
     load_pages(first);
     take_pages(first);
@@ -316,7 +349,8 @@ __global__ void __launch_bounds__(256, 3) paged_attn_kernel(
       pf[i] = (short)f2bf(pa[i]);
       pf[4 + i] = (short)f2bf(pb[i]);
     }
-    // this wave's V image has landed: at least the eight K loads are younger
+    // this wave's V image has landed: at least the eight K loads are younger (the wait at the loop's top covers it
+    // as long as the compiler puts one there)
     if constexpr (more) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     const uint32_t b0 = vimg + vt_base(lane);
@@ -365,7 +399,8 @@ __global__ void __launch_bounds__(256, 3) paged_attn_kernel(
   const int qi2 = q0 + rr / G;
   const bool row_valid = qi2 < ql;
   const int head2 = kvh * G + (rr % G);
-  if (nparts == 1) {
+  const int nvalid = min(nparts, (kv_end + part_tokens - 1) / part_tokens);
+  if (nvalid == 1) {  // nothing to combine
     if (!row_valid) return;
     const float inv = L > 0.f ? 1.f / L : 0.f;
     u32x4 ov;
@@ -404,7 +439,6 @@ __global__ void __launch_bounds__(256, 3) paged_attn_kernel(
   // nvalid-1 keeps the agent acquire (this kernel runs two workgroups per CU, outside the
   // guide's fence-free table row) and reduces every slab, then re-arms the counter for
   // the next launch (the buffer is zero-initialised once).
-  const int nvalid = min(nparts, (kv_end + part_tokens - 1) / part_tokens);
   int* cnt = sem + (size_t)tile * Hkv + kvh;
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
@@ -433,18 +467,18 @@ __global__ void __launch_bounds__(256) attn_reduce_kernel(
     const float* __restrict__ part_ml, const int* __restrict__ tile_seq,
     const int* __restrict__ tile_q0, const int* __restrict__ q_start,
     const int* __restrict__ q_len, const int* __restrict__ ctx_len, int Hq, int Hkv,
-    int part_tokens, int nparts) {
+    int part_tokens, int nparts, int even) {
   constexpr int QT = 16 / G;
   const int tile = blockIdx.x, kvh = blockIdx.y;
   const int s = tile_seq[tile], q0 = tile_q0[tile];
   const int ql = q_len[s], ctx = ctx_len[s], qs = q_start[s];
   const int last_q = min(q0 + QT, ql) - 1;
   const int kv_end = last_q >= 0 ? ctx - ql + last_q + 1 : 0;
-  part_tokens = seq_part(kv_end, part_tokens, nparts);
+  part_tokens = seq_part(kv_end, part_tokens, nparts, even, tile_seq, ctx_len, gridDim.x, Hkv);
   const int nvalid = min(nparts, (kv_end + part_tokens - 1) / part_tokens);
   const int rr = threadIdx.x >> 4, c = (threadIdx.x & 15) * 8;
   const int qi = q0 + rr / G;
-  if (qi >= ql) return;
+  if (qi >= ql || nvalid == 1) return;  // (one partition: written by the kernel before)
   const size_t base = ((size_t)tile * Hkv + kvh) * nparts;
   u32x4 ov;
   combine_parts(part_o, part_ml, base, nvalid, rr, c, ov);
@@ -461,10 +495,16 @@ int attn_kv_nt(int set) {
   return g_attn_kv_nt;
 }
 
-// Workgroups from which a launch takes no further partitions: one per CU.  A partition more costs its slab, a ticket
-// and its share of the combine; the metadata plans up to four per CU, with which 1 x 24000 keys took 47 us (27.6 with
-// 32 partitions), 3 x 24000 64 (58), 7 x 1000 14.1 (12.2), 13 x 2500 34.6 (35.1), 20 x 800 23.9 (22.4).
-constexpr int kAttnWgs = 256;
+// Partitions of a sequence in a launch of `base` (tile, kv head) pairs of like lengths: the CUs filled once.  A partition
+// more costs its slab, a ticket and its share of the combine; the metadata plans up to four workgroups per CU, with
+// which 1 x 24000 keys took 47 us (27.6 with 32 partitions), 3 x 24000 64 (58), 7 x 1000 14.1 (12.2), 13 x 2500 34.6
+// (35.1), 20 x 800 23.9 (22.4).  Counts a little above one per CU run as long as two (not powers of two, as steps beside
+// prompts have: 104 pairs in 3 shares 36.9 us, in 2 33; 136 pairs in 2 41, in 3 33; 288 pairs whole 77, in 2 66).
+static int even_parts(int base) {
+  constexpr int wgs = 256, two = 384;
+  if (base <= wgs / 2) return wgs / base;
+  return base == wgs || base >= two ? 1 : (two + base - 1) / base;
+}
 
 template <int G>
 static void launch_g(void* out, float* part_o, float* part_ml, const void* q, const void* kc,
@@ -472,12 +512,8 @@ static void launch_g(void* out, float* part_o, float* part_ml, const void* q, co
                      const int* tile_q0, const int* q_start, const int* q_len, const int* ctx_len,
                      int num_tiles, int Hq, int Hkv, float scale_log2, int part_tokens, int nparts,
                      int num_blocks, int* sem, hipStream_t st) {
-  const int base = num_tiles * Hkv;
-  const int want = std::max(1, (kAttnWgs + base - 1) / base);
-  if (nparts > want) {
-    part_tokens = ((part_tokens * nparts + want - 1) / want + 31) / 32 * 32;
-    nparts = want;
-  }
+  const int even = std::min(nparts, even_parts(num_tiles * Hkv));
+  if (num_tiles == 1 || even >= kEnoughParts) nparts = even;  // (seq_part: none needs more)
   dim3 grid(num_tiles, Hkv, nparts);
   // K / V pages non-temporal (attn_kv_nt op): each is read once per step by one workgroup
   // (below 8 query tiles the default policy: batch 4 lost 0.7 % with it, batch 16 gained 1.8 %)
@@ -485,11 +521,11 @@ static void launch_g(void* out, float* part_o, float* part_ml, const void* q, co
   auto kern = nt == 3 ? paged_attn_kernel<G, 3> : nt ? paged_attn_kernel<G, 1> : paged_attn_kernel<G, 0>;
   kern<<<grid, 256, 0, st>>>((uint16_t*)out, part_o, part_ml, (const uint16_t*)q, (const uint16_t*)kc,
                              (const uint16_t*)vc, bt, bt_stride, tile_seq, tile_q0, q_start, q_len, ctx_len,
-                             Hq, Hkv, scale_log2, part_tokens, nparts, num_blocks, sem);
+                             Hq, Hkv, scale_log2, part_tokens, nparts, even, num_blocks, sem);
   if (nparts > 1 && sem == nullptr) {
     attn_reduce_kernel<G><<<dim3(num_tiles, Hkv), 256, 0, st>>>(
         (uint16_t*)out, part_o, part_ml, tile_seq, tile_q0, q_start, q_len, ctx_len, Hq, Hkv,
-        part_tokens, nparts);
+        part_tokens, nparts, even);
   }
 }
 

@@ -280,6 +280,48 @@ def test_paged_attention_partitions_of_a_longer_limit(gpu, Hq, Hkv, part_tokens,
 
 
 @pytest.mark.parametrize("fused", [False, True])
+@pytest.mark.parametrize("Hq,Hkv,long,short,padding", [
+    (32, 8, [4000], [100] * 20, 0),            # all of the 7 shares that are planned
+    (32, 8, [3000], [97 + 3 * i for i in range(30)], 3),
+    (8, 1, [6000, 5000], [60] * 30, 32),       # one kv head, a padded step
+    (16, 16, [513, 4097], [33] * 9, 0),
+    (32, 4, [3200] * 10, [100] * 10, 0),       # half of the launch
+])
+def test_paged_attention_long_among_short(gpu, Hq, Hkv, long, short, padding, fused, attn_fused_all):
+    """A sequence far longer than its launch's mean is cut into the shares that were planned for it (counted in its
+    slabs), the short ones beside it are not; values as ever, by both combines."""
+    from mlopamd.runtime.attn_meta import plan_partitions
+
+    torch.manual_seed(0)
+    np.random.seed(0)
+    lens = short[:3] + long + short[3:] + [0] * padding
+    NB = sum((c + 15) // 16 for c in lens) + 8
+    kc = torch.randn(NB, Hkv, 16, 128, device=gpu, dtype=bf)
+    vc = torch.randn(NB, Hkv, 16, 128, device=gpu, dtype=bf)
+    part, nparts = plan_partitions(len(lens), Hkv, max(lens))
+    m, T = make_meta(gpu, [1] * len(lens), lens, Hkv, Hq // Hkv, NB, part_tokens=part, nparts=nparts)
+    if fused:
+        m.part_sem = torch.zeros(m.tile_seq.numel() * Hkv, dtype=torch.int32, device=gpu)
+    q = torch.randn(T, Hq, 128, device=gpu, dtype=bf)
+    m.part_ml.fill_(float("nan"))
+    for _ in range(2):
+        out = torch.full_like(q, float("nan"))
+        ops.paged_attention(q, kc, vc, m, out=out)
+        close(out, ref.paged_attention(q, kc, vc, m), atol=2e-2, rtol=2e-2)
+        assert not fused or int(m.part_sem.abs().sum()) == 0
+    n = len(lens) * Hkv * nparts
+    slabs = torch.isfinite(m.part_ml.view(-1, 16, 2)[:n, 0, 0]).view(len(lens), Hkv, nparts).sum(-1).cpu()
+    keys, live = sum(lens), len(long) + len(short)
+    for i, c in enumerate(lens):
+        if c * live > 1.6 * keys and c > 1024:
+            share = max(512, keys * Hkv // 512)
+            assert (slabs[i] >= min(nparts, c // (share + 64))).all(), (c, slabs[i])
+            assert (slabs[i] >= 2).all()
+        elif c <= 128:
+            assert (slabs[i] == 0).all(), (c, slabs[i])
+
+
+@pytest.mark.parametrize("fused", [False, True])
 def test_paged_attention_padded_bucket(gpu, fused, attn_fused_all):
     """Graph-bucket padding rows (q_len 1, ctx 0) under forced split-KV: both combine
     paths (second-launch reduce and in-launch last-ticket combine) must write a zero
