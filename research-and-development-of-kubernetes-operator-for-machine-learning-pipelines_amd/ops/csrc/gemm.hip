@@ -708,6 +708,11 @@ struct SkArgs {
 //   1                        a second pipeline fill + ticket
 // 0: keep the data-parallel grid.  Host (plain launches) and device (grouped launches, whose
 // tile count depends on the routing) evaluate the same function.
+__host__ __device__ inline float sk_tail_cost(int r, int nk, int d) {
+  const float w = 0.04f * r * d;
+  return nk / d + (w > 2.f ? w : 2.f) + 2.f * (d >= 3 ? d : d - 1) + 1.f;
+}
+
 __host__ __device__ inline int sk_choose_d(int T, int nk, int cus, int min_half) {
   const int r = T % cus;
   if (r == 0) return 0;
@@ -716,8 +721,7 @@ __host__ __device__ inline int sk_choose_d(int T, int nk, int cus, int min_half)
   const int dmax = cus / r < 32 ? cus / r : 32;
   for (int d = 2; d <= dmax; ++d) {
     if (nk % d || nk / d < min_half) continue;
-    const float w = 0.04f * r * d;
-    const float cost = nk / d + (w > 2.f ? w : 2.f) + 2.f * (d >= 3 ? d : d - 1) + 1.f;
+    const float cost = sk_tail_cost(r, nk, d);
     if (cost < best) {
       best = cost;
       best_d = d;
@@ -1369,39 +1373,43 @@ static bool mid_plan(int M, int N, int K, Plan& p) {
 }
 
 // Above the weight stream's rows: the four-wave kernel's tile height, or the ping-pong kernel with its stream-K tail,
-// by estimated time in us.  A round of 256-row tiles takes 5.6 + 0.0212 K; lower tiles cost more per row (192 rows 0.80
-// of it, 160 0.725, 128 0.61: fewer MFMAs per fragment read), and an only round that fills a share f of the CUs runs
-// faster, the less the lower the tile.  A tail of at most half the CUs is cut into K-halves: half a round and the
-// hand-off of the partials (behind whole rounds the more the more of them there are).  The ping-pong kernel cuts every
-// tile of a grid of up to half the CUs and skips empty 64-row quadrants there (down at 520 / 560 rows 86 / 87 us, the
-// best four-wave height 94 / 98), runs a round as it is above that, and spreads the remainder of several evenly at 1.08
-// of a round's rate.
-// Constants fitted to qkv, o, gate_up, down and lm_head of Llama-3-8B at 17 row counts from 400 to 4096, every variant
-// measured: the choice is within 5 % of the best of the five at all of them.  Against the earlier rule (heights 256 and
-// 128 only): gate_up at M = 400 / 700 / 1152 138 -> 92, 158 -> 147, 245 -> 219 us, o at 1152 / 2300 / 2600 55 -> 43,
-// 79 -> 62, 83 -> 68, down at 600 / 1500 / 2300 102 -> 88, 150 -> 135, 253 -> 213, qkv at 700 / 1500 / 2600 53 -> 43,
-// 79 -> 63, 132 -> 111, lm_head at 400 558 -> 394.
+// by estimated time in us.  A round of 256-row tiles takes 4.5 + 0.021 K; lower tiles cost more per row (192 rows 0.80
+// of it, 160 0.685, 128 0.645: fewer MFMAs per fragment read), and an only round that fills a share f of the CUs runs
+// faster.  A tail of at most half the CUs is cut into K-halves: half a round and the hand-off of the partials, behind
+// whole rounds the more the more of them there are.  A round of the ping-pong kernel takes 14 + 0.0208 K, its tail what
+// sk_tail_cost says.
+// Constants fitted to 30 weight shapes (the projections of Llama-3-8B and 70B, whole and in 2 - 8 shards, Mixtral's,
+// and shapes of no model here: N 2048 - 128256, K 1024 - 28672) at 38 row counts from 385 to 8000, every variant measured
+// in one process, twice: the choice is 0.2 % slower than the best of the five on average, more than 5 % at 4 of 1147
+// points, 12 % at worst; fitted to half of the shapes, 0.3 % on the others.  (Constants fitted to Llama-3-8B's matrices
+// alone: 1.4 %, 110 points and 38 %, and at 46 slower than the rule by tile counts that was here before: 70B qkv at 640
+// rows 113 us against 102, o at 1000 116 against 107, down at 2300 839 against 785; all three are 3 % from it now.)  That
+// rule, heights 256 and 128 only, was 8.4 % slower than the best (gate_up of Llama-3-8B at 400 / 700 / 1152 rows 138 ->
+// 92, 158 -> 147, 245 -> 219 us, o at 1152 / 2300 / 2600 55 -> 43, 79 -> 62, 83 -> 68).
 static bool big_plan(int M, int N, int K, bool pp_ok, Plan& p) {
   const SkBuf* b = sk_buf();
   if (!b || !gemm_w4_ok(M, N, K, K, K)) return false;
   struct Tile { int rows; float round, slope; };
-  constexpr Tile tiles[] = {{256, 1.f, .55f}, {192, .80f, .55f}, {160, .725f, .35f}, {128, .61f, .10f}};
-  const float full = 5.6f + 0.0212f * (float)K, C = (float)b->cus;
-  const float f = (float)((M + 255) / 256) * (float)(N / 256) / C;  // rounds of 256-row tiles
-  // (to 3/8 of the CUs without a tile's empty 64-row quadrants; nearer to half they no longer show)
-  const float fq = f > .375f ? f : (float)((M + 63) / 64) * (float)(N / 256) / (4.f * C);
-  float best = !pp_ok ? 1e30f : f <= .5f ? .87f * full * fq + 28.f + .06f * full : f <= 1.f ? 1.11f * full * (.5f + .5f * f) : 1.08f * full * f + 25.f;
+  constexpr Tile tiles[] = {{256, 1.f, .2f}, {192, .80f, .2f}, {160, .685f, .05f}, {128, .645f, .15f}};
+  const float full = 4.5f + 0.021f * (float)K, C = (float)b->cus;
+  const int nk = K / kBK;
+  float best = 1e30f;
   p.variant = 3;
   p.BM = p.BN = 256;
+  if (pp_ok) {
+    const int T = (M + 255) / 256 * (N / 256), q = T / b->cus, r = T % b->cus, d = sk_choose_d(T, nk, b->cus, sk_min_half());
+    const float tail = d ? sk_tail_cost(r, nk, d) / (float)nk : r > 0 ? 1.f : 0.f;
+    best = (14.f + 0.0208f * (float)K) * ((float)q + tail);
+  }
   for (const Tile& t : tiles) {
     if (t.rows < 256 && !g_half_tile) break;
     const long T = (long)((M + t.rows - 1) / t.rows) * (N / 256), q = T / b->cus, r = T % b->cus;
     const float one = full * t.round;
     float us = (float)q * one;
-    const bool halves = r > 0 && gemm_w4_split_ok((int)T, K / kBK);
+    const bool halves = r > 0 && gemm_w4_split_ok((int)T, nk);
     const float fill = (halves ? 2.f : 1.f) * (float)r / C, slope = q > 0 ? 0.f : t.slope;
     if (r > 0) us += (halves ? .5f : 1.f) * one * (1.f - slope * (1.f - fill));
-    if (halves) us += q > 0 ? std::max(0.f, 28.f * fill - 5.f) : 9.f + .1f * (float)(t.rows - 128);
+    if (halves) us += q > 0 ? 15.f * fill : 14.f;
     if (us < best) {
       best = us;
       p.variant = t.rows == 256 ? 5 : 6;
@@ -1496,9 +1504,10 @@ static Plan plan(int M, int N, int K, bool grouped, int n_groups, int rows_per_g
     constexpr int wide_min_m = 512;
     constexpr int mid_tiles = 72;
     // Fewer than 64 half-height tiles leave most CUs idle whatever the tile: the split-K tiles (variant 0).  So does
-    // long K on a narrow N at up to 512 rows (down at M = 400 / 512 70.9 / 72.8 us, the best of big_plan's 72.5 / 80).
-    const bool by_time = !grouped && big == 5 && (long)((M + 127) / 128) * (N / 256) >= 64 &&
-                         !(K >= 8192 && M <= 512 && t256 < mid_tiles) && big_plan(M, N, K, pp_ok, p);
+    // long K on a narrow N: fewer than 40 tiles of 256 rows (2048 x 8192 at M = 960 / 1000 47.3 us, the best of
+    // big_plan's 59.3), and at up to 512 rows fewer than 72 (down at M = 400 / 512 70.9 / 72.8, the best 72.5 / 80).
+    const bool narrow = K >= 8192 && (t256 < 40 || (M <= 512 && t256 < mid_tiles));
+    const bool by_time = !grouped && big == 5 && (long)((M + 127) / 128) * (N / 256) >= 64 && !narrow && big_plan(M, N, K, pp_ok, p);
     const int big_from = t256 >= mid_tiles ? std::min(big_min_m, wide_min_m) : std::max(big_min_m, 2048);
     if (by_time) {
     } else if (big == 5 && !(mrows >= big_from && !grouped && w4_fills && gemm_w4_ok(M, N, K, K, K))) {
