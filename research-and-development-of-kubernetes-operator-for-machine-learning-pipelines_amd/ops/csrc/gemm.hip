@@ -1419,7 +1419,7 @@ static bool big_plan(int M, int N, int K, bool pp_ok, Plan& p) {
   return true;
 }
 
-static Plan plan(int M, int N, int K, bool grouped, int n_groups, int rows_per_group) {
+static Plan plan(int M, int N, int K, bool grouped, int n_groups, int rows_per_group, bool stream = true) {
   Plan p{};
   p.variant = 0;
   const int mrows = grouped ? rows_per_group : M;
@@ -1430,7 +1430,7 @@ static Plan plan(int M, int N, int K, bool grouped, int n_groups, int rows_per_g
   // 474 -> 370 / 266 -> 200 us, 1024 rows 692 -> 389 / 375 -> 208 us; 48 rows per expert equal
   // (scripts/bench_moe_decode.py, profiles/r05_moe_decode.md)
   constexpr int pp_group_min_rows = 56;
-  if (!grouped && g_dp[0] < 0 && mid_plan(M, N, K, p)) {
+  if (!grouped && stream && g_dp[0] < 0 && mid_plan(M, N, K, p)) {
   } else if (grouped && mrows >= pp_group_min_rows && K % kBK == 0 && N % 256 == 0) {
     p.BM = 256; p.BN = 256; p.variant = 3;  // grouped ping-pong
   } else if (mrows <= 64 && !grouped && g_small_tile == 1) {
@@ -1663,6 +1663,7 @@ int gemm_rope_split(int set) {
 
 static Plan rope_plan(int M, int N, int K) {
   Plan p = plan(M, N, K, false, 0, 0);
+  if (p.variant == 7 && p.splits == 1) p = plan(M, N, K, false, 0, 0, false);  // no slabs, and no RoPE epilogue
   if (g_rope_split_k > 1 && p.splits == 1 && p.variant == 0 && p.BM <= 64 && K >= 2048) {
     const int kc = ((K / g_rope_split_k + kBK - 1) / kBK) * kBK;
     p.splits = (K + kc - 1) / kc;

@@ -607,6 +607,32 @@ def test_gemv(gpu, M, N, K):
     close(y, exp, atol=2e-2 * exp.abs().max().item() / 10 + 1e-2, rtol=2e-2)
 
 
+@pytest.mark.parametrize("M,Hq,Hkv", [(257, 32, 32), (300, 32, 32), (384, 32, 32), (130, 128, 32), (200, 128, 32), (256, 160, 16), (16, 128, 32), (48, 128, 32)])
+def test_qkv_rope_cache_fused_wide(gpu, M, Hq, Hkv):
+    """Wide QKV projections, as without grouped heads: one launch (or slabs and one launch), not product and rotation."""
+    from mlopamd.models.layers import rope_table
+
+    D, K, BS = 128, 2048, 16
+    N, NB = (Hq + 2 * Hkv) * D, M // BS + 8
+    ops._sk_reserve(torch.device(gpu))
+    torch.manual_seed(M)
+    cs = rope_table(D, 8192, 5e5, device=gpu)
+    x = torch.randn(M, K, device=gpu, dtype=bf)
+    w = (0.03 * torch.randn(N, K, device=gpu)).to(bf)
+    pos = torch.randint(0, 8000, (M,), device=gpu, dtype=torch.int32)
+    slots = torch.randperm(NB * BS, device=gpu)[:M].to(torch.int32)
+    slots[5] = slots[M - 1] = -1
+    kc = torch.zeros(NB, Hkv, BS, D, device=gpu, dtype=bf)
+    vc = torch.zeros_like(kc)
+    q = torch.empty(M, Hq, D, device=gpu, dtype=bf)
+    assert torch.ops.mlop.gemm_rope_supported(M, N, K)
+    assert torch.ops.mlop.gemm_rope_cache(q, kc, vc, x, w, pos, cs, slots)
+    kr, vr = torch.zeros_like(kc).cpu(), torch.zeros_like(vc).cpu()
+    qr = ref.rope_cache((x.float() @ w.float().t()).to(bf).cpu(), pos.cpu(), cs.cpu(), slots.cpu(), kr, vr, Hq)
+    for got, want in ((q, qr), (kc, kr), (vc, vr)):  # the product's rounding may fall the other way: one ulp, rotated
+        torch.testing.assert_close(got.float().cpu(), want.float(), atol=2e-2, rtol=2e-2)
+
+
 @pytest.mark.parametrize("M", [5, 13, 16, 24, 32, 48, 64])
 @pytest.mark.parametrize("tile", [1, 32, 64])
 @pytest.mark.parametrize("N,K,epi", [(6144, 4096, 0), (4096, 14336, 0), (7168, 4096, 1), (1280, 8192, 0),
