@@ -1349,7 +1349,7 @@ static bool sk_halves_ok(long T, int nk) {
 // quarters of the CUs, in one K range with 256 or 128 columns, or (65 rows and more) with K in up to 8 ranges of
 // at least 12 K-steps.  Below that, and for split K at 64 rows and fewer, the small tiles are as fast or faster
 // (o 4096 x 4096 at 100 rows 17.5 us against 18.6 in six ranges; down 4096 x 14336 at 16 / 64 rows 24.2 / 29.2
-// against 26.6 / 29.5); from 512 rows on the four-wave kernel is (gate_up 93 us against 115).
+// against 26.6 / 29.5).
 static bool mid_plan(int M, int N, int K, Plan& p) {
   constexpr int max_m = 384, fill = 192;
   if (M > max_m || K < kBK || K % kBK || N % 8) return false;  // (no K-step: gemm_kernel writes the empty sums)
@@ -1360,10 +1360,20 @@ static bool mid_plan(int M, int N, int K, Plan& p) {
   if (t256 < fill && t128 < fill) {
     s = std::min({kMaxSplits, 256 / t128, nk / 12});
     if (M <= 64 || t128 * s < fill) return false;
+    const int t64 = (N + 63) / 64;
     // where the 64-column tiles need no K ranges, the slabs have to be small beside the weights (12544 x 2048 in two
-    // ranges at 100 / 200 rows: 22 / 31 us against 20 / 24; 10240 x 8192 in three: 42 against 65)
-    if ((N + 63) / 64 >= 160 && 4l * s * M > K * 3l / 10) return false;
+    // ranges at 100 / 200 rows: 22 / 31 us against 20 / 24; 10240 x 8192 in three: 42 against 65); less so where those
+    // tiles fill the CUs with K in a few ranges (8192 x 3584 in four at 80 / 112 / 128 rows 23 / 26.0 / 26.5 us against 24 /
+    // 24.2 / 24.5, at 160 / 192 / 256 rows 28.5 / 31.6 / 36.4 against 29.6 / 30.2 / 32.2)
+    if (t64 >= 160 && 4l * s * M > K * 3l / 10) return false;
+    if (m_tiles == 1 && t64 < 160 && t64 * std::max(1, 256 / t64) >= 250 && 400l * s * M > K * (M <= 128 ? 43l : 80l)) return false;
   }
+  // Two row tiles read the weights twice (the second from L2).  Where the four-wave kernel's lower tiles have a grid, they
+  // are faster without K ranges, and with them above 320 rows (257 / 384 rows of gate_up 28672 x 4096 80 / 92 us ->
+  // 71 / 73, lm_head 128256 x 4096 340 / 432 -> 272 / 332, 12288 x 4096 53 / 62 -> 43 / 49; down of Llama-3-70B at 350 rows
+  // 255 -> 229, its quarter 8192 x 7168 at 384 66 -> 61)
+  if (m_tiles == 2 && (s == 1 || M > 320) && (M + 127) / 128 * (N / 256) >= 64 && sk_buf() != nullptr && gemm_w4_ok(M, N, K, K, K))
+    return false;
   p.variant = 7;
   p.BM = bm;
   p.BN = t256 >= fill ? 256 : 128;
@@ -1804,6 +1814,15 @@ bool launch_mid_rs(const void* A, int lda, const void* B, void* out, int ldo, in
   launch_plan<EPI_SILU_MUL, false>(p, (const uint16_t*)A, lda, (const uint16_t*)B, K, (uint16_t*)out, ldo, nullptr,
                                    M, N, K, nullptr, 0, st, re);
   return true;
+}
+
+void gemm_plan(int M, int N, int K, int out[4]) {
+  if (gemv_takes(M, N, K, EPI_NONE)) {
+    out[0] = -1, out[1] = out[2] = 0, out[3] = 1;
+    return;
+  }
+  const Plan p = plan(M, N, K, false, 0, 0);
+  out[0] = p.variant, out[1] = p.BM, out[2] = p.BN, out[3] = p.splits;
 }
 
 long gemm_workspace_floats(int M, int N, int K, int epi) {

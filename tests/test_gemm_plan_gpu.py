@@ -1,5 +1,5 @@
-"""The dense planner's choice held against what it chose from, measured here: large row counts (four-wave heights and the
-ping-pong kernel)."""
+"""The dense planner's choice: held against what it chose from, measured here, for large row counts (four-wave heights and
+the ping-pong kernel), and the weight stream's limits."""
 import pytest
 import torch
 
@@ -33,19 +33,33 @@ def test_large_rows(gpu, M, N, K):
     """The choice is at most 15 % slower than the best variant (noise of two runs: 5 %; the model's own worst: 11 %)."""
     ops._sk_reserve(torch.device(gpu))
     x = torch.randn(M, K, device=gpu, dtype=bf)
-    w = [(0.02 * torch.randn(N, K, device=gpu)).to(bf) for _ in range(2)]
+    n = int(6e8 / (2 * N * K)) + 2  # more than the caches hold: a layer's weights are read once per step
+    w = [(0.02 * torch.randn(N, K, device=gpu)).to(bf) for _ in range(n)]
     out = torch.empty(M, N, device=gpu, dtype=bf)
+    no_ws = torch.empty(0, device=gpu)
     plan = torch.ops.mlop.gemm_dense_plan
 
     def run(variant):
         def go():
             plan(*variant)
             try:
-                for i in range(6):
-                    torch.ops.mlop.gemm(out, x, w[i % 2], torch.empty(0, device=gpu), 0)
+                for a in w:
+                    torch.ops.mlop.gemm(out, x, a, no_ws, 0)
             finally:
                 plan(-1, -1, -1, -1)
         return go
 
-    t = best_times({"choice": run((-1, -1, -1, -1)), **{n: run((v, bm, 256, -1)) for n, (v, bm) in VARIANTS.items()}})
-    assert t["choice"] <= 1.15 * min(t[n] for n in VARIANTS), {n: round(v / 6, 1) for n, v in t.items()}
+    t = best_times({"choice": run((-1, -1, -1, -1)), **{name: run((v, bm, 256, -1)) for name, (v, bm) in VARIANTS.items()}})
+    assert t["choice"] <= 1.15 * min(t[v] for v in VARIANTS), {k: round(v / n, 1) for k, v in t.items()}
+
+
+@pytest.mark.parametrize("M,N,K,stream", [
+    # two row tiles: not in one K range where the four-wave kernel has a grid (columns in 256s, K >= 192), nor above 320 rows
+    (256, 28672, 4096, True), (257, 28672, 4096, False), (384, 12288, 4096, False), (300, 12296, 4096, True), (300, 28672, 128, True),
+    (320, 8192, 7168, True), (321, 8192, 7168, False), (384, 4096, 14336, True), (385, 4096, 14336, False),
+    # slabs beside the weights
+    (96, 8192, 3584, True), (97, 8192, 3584, False), (160, 8192, 3584, True), (192, 8192, 3584, False), (256, 5120, 5120, True),
+    (64, 8192, 28672, False), (65, 8192, 28672, True)])
+def test_weight_stream_limits(gpu, M, N, K, stream):
+    ops._sk_reserve(torch.device(gpu))
+    assert (torch.ops.mlop.gemm_plan(M, N, K)[0] == 7) == stream
