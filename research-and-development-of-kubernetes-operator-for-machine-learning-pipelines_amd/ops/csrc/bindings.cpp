@@ -294,9 +294,9 @@ int64_t gemm_workspace(int64_t M, int64_t N, int64_t K, int64_t epi) {
 }
 
 std::vector<int64_t> gemm_plan(int64_t M, int64_t N, int64_t K) {
-  int p[4];
+  int p[5];
   mlop::gemm_plan((int)M, (int)N, (int)K, p);
-  return {p[0], p[1], p[2], p[3]};
+  return {p[0], p[1], p[2], p[3], p[4]};
 }
 
 // out[M, N or N/2] = epi(a[M, K] . w[N, K]^T)

@@ -556,6 +556,11 @@ int gemm_slab_nt(int set) {
   if (set >= 0) g_slab_nt = set;
   return g_slab_nt;
 }
+// of the dense weight-streaming launches (gemm_kernel, gemm_mid.hip): 1 weights non-temporal, where one workgroup
+// streams each of them, 2 slabs non-temporal
+int gemm_stream_policy(int m_tiles) {
+  return ((g_small_nt_flags & 1) != 0 && m_tiles == 1 ? 1 : 0) | ((g_slab_nt & 1) != 0 ? 2 : 0);
+}
 
 template <int BM, int BN, int WM, int WN, int EPI, bool GROUPED, int STAGES, bool SETPRIO>
 static void run_cfg(const uint16_t* A, int lda, const uint16_t* B, int ldb, uint16_t* C, int ldc,
@@ -575,7 +580,7 @@ static void run_cfg(const uint16_t* A, int lda, const uint16_t* B, int ldb, uint
   // non-temporal weights where each weight byte is streamed by ONE workgroup: one m-tile
   // (dense), or the grouped decode tiles (an expert's few routed rows)
   RopeEpi r = re;
-  r.b_nt = GROUPED ? (g_small_nt_flags & 2) != 0 && BM <= 64 : (g_small_nt_flags & 1) != 0 && m_tiles == 1;
+  r.b_nt = GROUPED ? (g_small_nt_flags & 2) != 0 && BM <= 64 : (gemm_stream_policy(m_tiles) & 1) != 0;
   r.ws_nt = g_slab_nt;
   kern<<<blocks, T, lds, st>>>(A, lda, B, ldb, C, ldc, ws, M, N, K, k_chunk, offsets, n_groups, gx,
                                m_tiles, splits, r);
@@ -1353,6 +1358,7 @@ static bool sk_halves_ok(long T, int nk) {
 static bool mid_plan(int M, int N, int K, Plan& p) {
   constexpr int max_m = 384, fill = 192;
   if (M > max_m || K < kBK || K % kBK || N % 8) return false;  // (no K-step: gemm_kernel writes the empty sums)
+  if (M <= 64 && g_small_tile != 1) return false;              // one of gemm_kernel's tiles is asked for
   const int m_tiles = M <= 256 ? 1 : 2, rows = (M + m_tiles - 1) / m_tiles;
   const int bm = rows <= 64 ? 64 : (rows + 31) / 32 * 32;
   const int t256 = (N + 255) / 256 * m_tiles, t128 = (N + 127) / 128 * m_tiles, nk = K / kBK;
@@ -1816,13 +1822,14 @@ bool launch_mid_rs(const void* A, int lda, const void* B, void* out, int ldo, in
   return true;
 }
 
-void gemm_plan(int M, int N, int K, int out[4]) {
+void gemm_plan(int M, int N, int K, int out[5]) {
   if (gemv_takes(M, N, K, EPI_NONE)) {
-    out[0] = -1, out[1] = out[2] = 0, out[3] = 1;
+    out[0] = -1, out[1] = out[2] = out[4] = 0, out[3] = 1;
     return;
   }
   const Plan p = plan(M, N, K, false, 0, 0);
   out[0] = p.variant, out[1] = p.BM, out[2] = p.BN, out[3] = p.splits;
+  out[4] = p.variant == 0 || p.variant == 7 ? gemm_stream_policy((M + p.BM - 1) / p.BM) : 0;
 }
 
 long gemm_workspace_floats(int M, int N, int K, int epi) {

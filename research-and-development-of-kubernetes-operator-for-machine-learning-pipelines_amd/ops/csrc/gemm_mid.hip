@@ -172,17 +172,24 @@ __global__ void __launch_bounds__(WM * WN * 64) gemm_mid_kernel(
     const int mr = c_by * BM + wm * WTM + (lane & 15), nc = c_bx * BN + wn * WTN + 4 * g4;
     if (n_splits > 1) {
       float* P = ws + (size_t)c_bz * M * N;
+      auto slab = [&](auto nt_) {
 #pragma unroll
-      for (int i = 0; i < TM; ++i) {
-        const int m = mr + i * 16;
-        if (m < M) {
+        for (int i = 0; i < TM; ++i) {
+          const int m = mr + i * 16;
+          if (m < M) {
 #pragma unroll
-          for (int j = 0; j < TN; ++j) {
-            const int n = nc + j * 16;
-            if (n < N) __builtin_nontemporal_store(acc[i][j], reinterpret_cast<f32x4*>(P + (size_t)m * N + n));
+            for (int j = 0; j < TN; ++j) {
+              const int n = nc + j * 16;
+              f32x4* dst = reinterpret_cast<f32x4*>(P + (size_t)m * N + n);
+              if (n >= N) continue;
+              if constexpr (decltype(nt_)::value) __builtin_nontemporal_store(acc[i][j], dst);
+              else *dst = acc[i][j];
+            }
           }
         }
-      }
+      };
+      if (re.ws_nt) slab(std::true_type{});
+      else slab(std::false_type{});
       return;
     }
 #pragma unroll
@@ -260,7 +267,9 @@ static void run_mid(const uint16_t* A, int lda, const uint16_t* B, int ldb, uint
   const int tasks = gx * m_tiles * splits;
   constexpr int per_cu = (int)(163840 / lds) >= 2 ? 2 : 1;
   RopeEpi r = re;
-  r.b_nt = m_tiles == 1;
+  const int policy = gemm_stream_policy(m_tiles);
+  r.b_nt = policy & 1;
+  r.ws_nt = policy >> 1;
   kern<<<std::min(tasks, 256 * per_cu), WM * WN * 64, lds, st>>>(A, lda, B, ldb, C, ldc, ws, M, N, K, k_chunk, m_tiles,
                                                                  splits, tasks, r);
 }

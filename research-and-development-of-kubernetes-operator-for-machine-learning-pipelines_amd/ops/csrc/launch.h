@@ -127,8 +127,10 @@ constexpr int epi_act(int epi) {
 // split-K reduce fused in: small-M launch_gemm_rope)
 void launch_rope_cache_slabs(const RopeEpi& re, const float* ws, int splits, int T, int N, hipStream_t st);
 long gemm_workspace_floats(int M, int N, int K, int epi);
-// what a plain product of this shape takes: kernel variant (gemm.hip plan; -1 the GEMV), tile rows, columns, K ranges
-void gemm_plan(int M, int N, int K, int out[4]);
+// what a plain product of this shape takes: kernel variant (gemm.hip plan; -1 the GEMV), tile rows, columns, K ranges,
+// cache policy of the weight-streaming tiles
+void gemm_plan(int M, int N, int K, int out[5]);
+int gemm_stream_policy(int m_tiles);
 // large-M kernel variant of the GEMM planner (gemm.hip plan(): 0 256x128, 1/2 256x256
 // 8-wave, 3 ping-pong, 5 four-wave asm K-loop); set >= 0 overrides (in-process A/B), returns the current value
 int gemm_big_variant(int set);

@@ -1,5 +1,5 @@
 """The dense planner's choice: held against what it chose from, measured here, for large row counts (four-wave heights and
-the ping-pong kernel), and the weight stream's limits."""
+the ping-pong kernel), the weight stream's limits, and the switches that it follows."""
 import pytest
 import torch
 
@@ -63,3 +63,33 @@ def test_large_rows(gpu, M, N, K):
 def test_weight_stream_limits(gpu, M, N, K, stream):
     ops._sk_reserve(torch.device(gpu))
     assert (torch.ops.mlop.gemm_plan(M, N, K)[0] == 7) == stream
+
+
+@pytest.mark.parametrize("M,N,K", [(16, 6144, 4096), (16, 28672, 4096), (64, 28672, 4096), (100, 6144, 4096), (200, 28672, 4096), (200, 4096, 14336)])
+def test_cache_policy_switches(gpu, M, N, K):
+    """Weights and slabs of the weight-streaming tiles go by gemm_small_nt and gemm_slab_nt, whichever kernel has them."""
+    ops._sk_reserve(torch.device(gpu))
+    o = torch.ops.mlop
+    prev = o.gemm_small_nt(-1), o.gemm_slab_nt(-1)
+    try:
+        for small in (0, 1, 6, 7):
+            for slab in (0, 1, 14, 15):
+                o.gemm_small_nt(small), o.gemm_slab_nt(slab)
+                assert o.gemm_plan(M, N, K)[4] == (small & 1) + 2 * (slab & 1)
+    finally:
+        o.gemm_small_nt(prev[0]), o.gemm_slab_nt(prev[1])
+
+
+@pytest.mark.parametrize("M", [5, 16, 32, 64, 65])
+@pytest.mark.parametrize("N", [6144, 28672, 49152])
+def test_small_tile_switch(gpu, M, N):
+    """gemm_small_tile's tiles are what runs at up to 64 rows, on wide weights too."""
+    prev = torch.ops.mlop.gemm_small_tile()
+    try:
+        for tile, bn in ((0, 64), (32, 32), (64, 64)):
+            torch.ops.mlop.gemm_small_tile(tile)
+            v, bm, n = torch.ops.mlop.gemm_plan(M, N, 4096)[:3]
+            if M <= 64:
+                assert (v, n, bm) == (0, bn, 64 if tile == 0 else 16 if M <= 16 else 32 if M <= 32 else 64)
+    finally:
+        torch.ops.mlop.gemm_small_tile(prev)
