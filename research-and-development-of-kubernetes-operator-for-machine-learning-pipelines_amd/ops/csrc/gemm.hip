@@ -624,8 +624,8 @@ void gemm_grouped_plan(int bm, int bn, int stages, int splits) {
 
 // dense-plan override (scripts/bench_mid_m.py sweeps the mid-M projection tilings in one
 // process): variant (0 = gemm_kernel BM x BN, 1 = 256x256 two-stage, 3 = ping-pong, 5 =
-// four-wave, 6 = four-wave half height), BM, BN, K splits (plain gemm_kernel only), LDS ring
-// depth of the small tiles (0 = the default); -1 = the planner's own choice
+// four-wave, 6 = four-wave of BM 160 or 192 rows, else half height), BM, BN, K splits (plain gemm_kernel only), LDS
+// ring depth of the small tiles (0 = the default); -1 = the planner's own choice
 static int g_dp[5] = {-1, -1, -1, -1, 0};
 void gemm_dense_plan(int variant, int bm, int bn, int splits, int stages) {
   if (variant >= 0 && variant != 0 && variant != 1 && variant != 3 && variant != 5 && variant != 6)
@@ -636,8 +636,6 @@ void gemm_dense_plan(int variant, int bm, int bn, int splits, int stages) {
     for (const auto& t : ok) found = found || (t[0] == bm && t[1] == bn);
     if (!found) throw std::runtime_error("gemm_dense_plan: no dense config for this tile");
   }
-  if (variant == 6 && bm > 0 && bm != 128 && bm != 160 && bm != 192)
-    throw std::runtime_error("gemm_dense_plan: four-wave tiles between are 128, 160 or 192 rows");
   g_dp[0] = variant, g_dp[1] = bm, g_dp[2] = bn, g_dp[3] = splits, g_dp[4] = stages > 0 ? stages : 0;
 }
 
@@ -1555,7 +1553,7 @@ static Plan plan(int M, int N, int K, bool grouped, int n_groups, int rows_per_g
   }
   if (!grouped && g_dp[0] >= 0) {  // bench override (gemm_dense_plan)
     p.variant = g_dp[0];
-    p.BM = p.variant == 0 || (p.variant == 6 && g_dp[1] > 0) ? g_dp[1] : p.variant == 6 ? 128 : 256;
+    p.BM = p.variant == 0 || (p.variant == 6 && (g_dp[1] == 160 || g_dp[1] == 192)) ? g_dp[1] : p.variant == 6 ? 128 : 256;
     p.BN = p.variant == 0 ? g_dp[2] : 256;
     p.stages = g_dp[4];
   }

@@ -1,5 +1,5 @@
 """The dense planner's choice: held against what it chose from, measured here, for large row counts (four-wave heights and
-the ping-pong kernel), the weight stream's limits, and the switches that it follows."""
+the ping-pong kernel), the weight stream's limits, and the switches and overrides."""
 import pytest
 import torch
 
@@ -93,3 +93,19 @@ def test_small_tile_switch(gpu, M, N):
                 assert (v, n, bm) == (0, bn, 64 if tile == 0 else 16 if M <= 16 else 32 if M <= 32 else 64)
     finally:
         torch.ops.mlop.gemm_small_tile(prev)
+
+
+@pytest.mark.parametrize("bm,rows", [(-1, 128), (0, 128), (64, 128), (128, 128), (160, 160), (192, 192), (256, 128)])
+def test_four_wave_override(gpu, bm, rows):
+    """Variant 6 takes any tile height, as ever: the two between as they are, the half height for all others."""
+    ops._sk_reserve(torch.device(gpu))
+    x = torch.randn(300, 256, device=gpu, dtype=bf)
+    w = (0.05 * torch.randn(512, 256, device=gpu)).to(bf)
+    try:
+        torch.ops.mlop.gemm_dense_plan(6, bm, 256, -1)
+        assert torch.ops.mlop.gemm_plan(300, 512, 256)[:3] == [6, rows, 256]
+        y = ops.gemm(x, w)
+    finally:
+        torch.ops.mlop.gemm_dense_plan(-1, -1, -1, -1)
+    z = x.float() @ w.float().t()
+    assert ((y.float() - z).abs() <= 2.0 ** -8 * z.abs() + 2.0 ** -19 * (x.float().abs() @ w.float().abs().t()) + 1e-6).all()
