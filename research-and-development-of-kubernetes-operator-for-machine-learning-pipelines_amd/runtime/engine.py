@@ -585,7 +585,7 @@ class Engine:
         any_work, eager, t_max, bucket = self.ep_sync.agree(0, 0, 0, 0, int(self.has_work()))
         if not any_work:
             return
-        self._wait_meta()  # async: the previous step's metadata H2D must have read the host buffer
+        self._wait_meta()  # the previous step's metadata H2D must have read the host buffer
         empty = np.zeros(0, dtype=np.int32)
         if eager or bucket not in self.graphs:
             self.meta.fill_decode(empty, empty, np.zeros(0, dtype=np.int64), pad_to=1)
@@ -596,7 +596,7 @@ class Engine:
             self.meta.fill_decode(empty, empty, np.zeros(0, dtype=np.int64), pad_to=bucket)
             self.meta.upload(bucket, bucket, self.rows_hi)
             self.graphs[bucket][0].replay()
-        if self._async and self.device.type == "cuda":
+        if self.device.type == "cuda":
             self._meta_ev = torch.cuda.Event()
             self._meta_ev.record()
         self.stats["ep_idle_steps"] += 1

@@ -183,3 +183,26 @@ def test_feed_does_not_wait(gpu, async_scheduling):
     assert [o is None for o in x] == [o is None for o in y] and tx == ty
     for p, q in zip(x, y):
         assert p is None or torch.equal(p, q)
+
+
+@pytest.mark.parametrize("eager", [True, False])
+@pytest.mark.parametrize("async_scheduling", [True, False])
+def test_idle_lock_step_guards_the_step_buffer(gpu, async_scheduling, eager):
+    """A rank with nothing to schedule joins its group's step with padding: the host buffer that the device still reads
+    is waited for before the next step writes it, with either kind of scheduling."""
+    from mlopamd.models import build_model
+
+    class Group:
+        last_busy = 0
+
+        def agree(self, *a):
+            return 1, int(eager), 1, 4
+
+    eng = Engine(build_model(get_config("tiny-llama"), device=gpu, seed=3),
+                 EngineConfig(max_num_seqs=8, max_num_batched_tokens=512, max_model_len=512, num_kv_blocks=64,
+                              graph_buckets=(1, 4), async_scheduling=async_scheduling))
+    eng.ep_sync = Group()
+    eng._ep_idle()
+    assert eng._meta_ev is not None and eng.stats["ep_idle_steps"] == 1
+    eng._wait_meta()
+    assert eng._meta_ev is None
