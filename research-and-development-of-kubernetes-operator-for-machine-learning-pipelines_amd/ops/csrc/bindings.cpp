@@ -299,6 +299,10 @@ std::vector<int64_t> gemm_plan(int64_t M, int64_t N, int64_t K) {
   return {p[0], p[1], p[2], p[3], p[4]};
 }
 
+int64_t gemm_grouped_variant(int64_t M, int64_t N, int64_t K, int64_t groups, int64_t rows, int64_t a_n) {
+  return mlop::gemm_grouped_variant((int)M, (int)N, (int)K, (int)groups, (int)rows, (int)a_n);
+}
+
 // out[M, N or N/2] = epi(a[M, K] . w[N, K]^T)
 void gemm(Tensor out, Tensor a, Tensor w, Tensor ws, int64_t epi, double p0, double p1, int64_t act_from) {
   TORCH_CHECK(a.is_cuda() && a.scalar_type() == at::kBFloat16 && a.dim() == 2 && a.stride(1) == 1,
@@ -930,6 +934,7 @@ TORCH_LIBRARY(mlop, m) {
   m.def("ep_destroy(int h) -> ()", &ep_destroy);
   m.def("gemm_workspace(int M, int N, int K, int epi) -> int", &gemm_workspace);
   m.def("gemm_plan(int M, int N, int K) -> int[]", &gemm_plan);
+  m.def("gemm_grouped_variant(int M, int N, int K, int groups, int rows, int a_n) -> int", &gemm_grouped_variant);
   m.def("gemm_big_variant(int set=-1) -> int", &gemm_big_variant);
   m.def("gemm_half_tile(int set=-1) -> int", &gemm_half_tile);
   m.def("gemm_small_nt(int set=-1) -> int", &gemm_small_nt);

@@ -1340,7 +1340,9 @@ struct Plan {
 //   large M: variant 0 = 256x128 (3-stage ring), 1 = 256x256 (2-stage, 128x64 per
 //   wave: half the LDS + L2 bytes per FLOP), 2 = 256x256 + setprio around MFMAs,
 //   3 = 256x256 two-group ping-pong (gemm_pp_kernel), 5 (default) = the four-wave kernel with
-//   the hand-scheduled asm K-loop (gemm_w4.hip) where its grid fills the chip, else 3.  (A four-wave 128x128-per-wave
+//   the hand-scheduled asm K-loop (gemm_w4.hip), 256 rows, 6 = its tiles of 128, 160 and 192 rows (big_plan
+//   chooses between 3, 5 and 6; without its scratch 5 where the grid fills the chip, else 3), 7 = the weight
+//   stream of gemm_mid.hip (mid_plan, up to 384 rows, before all others).  (A four-wave 128x128-per-wave
 //   variant was measured 10-20% slower: profiles/r02_gemm_fourwave_rejected.md.)
 // true when the stream-K tail is available here and splits ALL T (<= C / 2) tiles
 static bool sk_halves_ok(long T, int nk) {
@@ -1907,6 +1909,36 @@ bool launch_gemm_add_rmsnorm(const void* A, int lda, const void* B, void* out, v
   return true;
 }
 
+// The experts' products: gemm_kernel's tiles, the ping-pong kernel (variant 3) or the four-wave kernel (5).  The latter
+// where the 256-row tiles make three rounds or more (gate_up): with fewer, stream-K's even split of the tail wins (down
+// of 8 experts at 350 / 450 / 1024 rows each 320 / 355 / 791 us against 318 / 375 / 798).
+// gate_up of 8 experts, ping-pong -> four-wave: 75 / 125 / 300 / 350 / 500 / 625 / 1024 rows each 374 -> 353, 376 ->
+// 364, 630 -> 530, 654 -> 604, 828 -> 772, 1047 -> 978, 1606 -> 1479 us, and with the experts 0.6 - 1.4 of that 370
+// -> 351, 375 -> 352, 636 -> 595, 666 -> 646, 877 -> 848, 1072 -> 954, 1620 -> 1481.  Not at 160 - 240 and 368 - 440
+// rows on average, where experts of exactly that size are most of one or two 256-row tiles but not of lower ones, and the
+// ping-pong kernel skips a tile's empty 64-row quadrants (200 rows 397 us against 436, 425 714 against 745).
+// The bands are those of this one shape and of equal experts.  Measured in one process on others (8 experts of half the
+// width, 4 of the same, 16 x 12800 x 4096, 32 x 8192 x 2048, 64 x 2816 x 2048; 43 row counts; equal experts, random
+// tokens, experts 0.6 - 1.4 of the mean, one expert of two fifths of the tokens): outside the bands the choice is at
+// most 6 % slower than ping-pong (at 240 - 256 equal rows) and 13 % faster on average; inside them the four-wave kernel
+// would be 4 - 16 % faster on 4 - 16 experts, by routing, and 10 - 37 % on 32 and 64, at single sizes up to 9 % slower: a
+// choice on the host, from the mean alone, cannot tell.
+static Plan grouped_plan(int M, int N, int K, int n_groups, int max_rows, int a_n) {
+  Plan p = plan(M, N, K, true, n_groups, max_rows);
+  const bool quadrants = (max_rows >= 160 && max_rows < 240) || (max_rows >= 368 && max_rows < 440);
+  if (p.variant == 3 && g_gp[0] <= 0 && !quadrants) {
+    const SkBuf* b = sk_buf();
+    if (b && (long)n_groups * std::max(1, (max_rows + 128) / 256) * (N / 256) >= 3l * b->cus &&
+        gemm_w4_grouped_ok(M, N, K, n_groups, a_n))
+      p.variant = 5;
+  }
+  return p;
+}
+
+int gemm_grouped_variant(int M, int N, int K, int n_groups, int max_rows, int a_n) {
+  return grouped_plan(M, N, K, n_groups, max_rows, a_n).variant;
+}
+
 void launch_grouped_gemm(const void* A, const void* B, void* C, const int* offsets, int n_groups,
                          int M, int N, int K, int max_rows, int epi, hipStream_t st, const int* a_rows,
                          float** defer_ws, int* defer_splits, const float* row_scale, float p0, float p1, int a_n) {
@@ -1916,21 +1948,7 @@ void launch_grouped_gemm(const void* A, const void* B, void* C, const int* offse
     launch_gemv_grouped(A, B, C, offsets, n_groups, M, N, K, epi, st, p0, p1);
     return;
   }
-  Plan p = plan(M, N, K, true, n_groups, max_rows);
-  // The four-wave kernel where the 256-row tiles make three rounds or more (gate_up): with fewer, stream-K's even split
-  // of the tail wins (down of 8 experts at 350 / 450 / 1024 rows each 320 / 355 / 791 us against 318 / 375 / 798).
-  // gate_up of 8 experts, ping-pong -> four-wave: 75 / 125 / 300 / 350 / 500 / 625 / 1024 rows each 374 -> 353, 376 ->
-  // 364, 630 -> 530, 654 -> 604, 828 -> 772, 1047 -> 978, 1606 -> 1479 us, and with the experts 0.6 - 1.4 of that 370
-  // -> 351, 375 -> 352, 636 -> 595, 666 -> 646, 877 -> 848, 1072 -> 954, 1620 -> 1481.  Not at 160 - 240 and 368 - 440
-  // rows, where an expert is most of one or two 256-row tiles but not the lower ones, and the ping-pong kernel skips a
-  // tile's empty 64-row quadrants (200 rows 397 us against 436, 375 677 against 737, 425 714 against 745).
-  const bool quadrants = (max_rows >= 160 && max_rows < 240) || (max_rows >= 368 && max_rows < 440);
-  if (p.variant == 3 && g_gp[0] <= 0 && !quadrants) {
-    const SkBuf* b = sk_buf();
-    if (b && (long)n_groups * std::max(1, (max_rows + 128) / 256) * (N / 256) >= 3l * b->cus &&
-        gemm_w4_grouped_ok(M, N, K, n_groups, a_n))
-      p.variant = 5;
-  }
+  Plan p = grouped_plan(M, N, K, n_groups, max_rows, a_n);
   float* ws = nullptr;
   if (p.variant == 0 && K >= 2048 && g_gp[3] != 1 && !(p.nosplit && g_gp[0] <= 0)) {
     const SkBuf* b = sk_buf();

@@ -11,9 +11,10 @@
 //   * column tile bx starts its walk of K at step bx % nk and wraps around.  Weight rows are a multiple of
 //     4 KB apart: tiles that walk K in step ask for the same offset of every row, that is for the same
 //     few memory channels (B alone, gate_up of Llama-3-8B: 43.8 -> 36.8 us);
-//   * the second half of a K-step's fragments is read while the first half multiplies, and the next
-//     step's first half while the second does: LDS reads (three quarters of a step's time) and MFMAs
-//     overlap inside a wave;
+//   * the next K-step's first half of fragments is read while this one's second half multiplies.  The
+//     second half's reads stand before the first half's MFMAs as well, but the compiler waits for all LDS
+//     reads in between (lgkmcnt(0): the epilogue's scalar loads share the counter), so half of the LDS
+//     reads (three quarters of a step's time) overlap MFMAs inside a wave, the other half only across waves;
 //   * a workgroup walks its tiles without draining the rings: the next tile's first K-steps load under
 //     this one's last (lm_head: four tiles per workgroup).
 // Tiles are 256 columns where such tiles fill the chip (A is read half as often), else 128; rows are the

@@ -11,18 +11,18 @@
 // re-orders a HIP-source version of it (profiles/r03_gemm_fourwave.md: 126-137 us at 4096^3).
 // The DMA for K-tile t+2 goes into the buffer of tile t as soon as every wave has its
 // fragments of tile t in registers, so one buffer pair keeps a whole tile in flight.
-// BMT = 128 is the half-height tile (planner variant 6, grids of at most one round): 64 x 128
+// BMT = 128 is the half-height tile (planner variant 6): 64 x 128
 // outputs per wave (a[0:127]), 12 DMA pieces per K-tile, its own generated loop
 // (MLOP_W4H_KLOOP_*, 64 MFMAs per K-tile), every epilogue shared with the full tile.  BMT = 160 and 192
 // (80 and 96 output rows per wave, loops MLOP_W4_160_* / _192_*) stand between them for grids that both fill
-// badly: whole rounds take 0.725 and 0.80 of the full tile's (gemm.hip big_plan has the choice and its figures).
+// badly: whole rounds take 0.685 and 0.80 of the full tile's (gemm.hip big_plan has the choice and its figures).
 //
 // HIP handles the rest: tile placement (XCD-contiguous bands, as gemm_pp_kernel), per-lane
 // DMA source offsets (rows clamped to the last valid row, XOR swizzle in the source), the
 // accumulator read-out (v_accvgpr_read statements) and the epilogues, all straight from the
 // accumulators (the loop computes C^T, so each lane owns 4 consecutive columns): plain store,
 // SiLU-mul (gate / up interleaved in groups of 16 columns), RoPE + paged K / V (both pages
-// token-major; a wave's 128 columns are one head; rotate-half partners sit in the same lane).  Requirements: K % 64 == 0, K >= 128, lda / ldb % 8 == 0.
+// token-major; a wave's 128 columns are one head; rotate-half partners sit in the same lane).  Requirements: K % 64 == 0, K >= 192, lda / ldb % 8 == 0.
 #include "common.h"
 #include "launch.h"
 #include "gemm_w4_asm.h"

@@ -27,6 +27,9 @@ Schedule of iteration t (MFMA slot m = 0..127; H0 = k-half 0 of tile t, H1 = k-h
   m 40..100  16 LDS-DMA pieces of tile t+2 into buffer t&1 (one per 4 MFMAs)
   m  102     vmcnt(16) + s_barrier (B2): tile t+1 (issued one iteration ago) has landed
   m 103..127 ds_read k-half-0 fragments of tile t+1 (FB0, FA0) from buffer (t+1)&1
+Lower tiles (128, 160, 192 rows: 64, 80, 96 MFMAs per K-tile, 12 - 14 pieces and 12 - 14 reads per half) have the same
+phases at their own slots (SCHED_H, SCHED_160, SCHED_192).  The K offset of the DMA runs through an operand: it starts
+where the caller says and wraps to 0 at %[kend], so that tiles may walk K from different steps.
 MFMA order: H0 = (i, j) row-major over FA0[i] x FB0[j]; H1 = the same over FA1 x FB1.
 lgkmcnt waits are derived here from the in-order LDS return queue (each MFMA waits only
 for the fragments it reads).  The last two iterations are peeled: t = nk-2 issues no DMA

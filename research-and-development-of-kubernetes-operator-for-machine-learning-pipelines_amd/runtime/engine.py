@@ -1181,7 +1181,8 @@ class Engine:
         whose logits are wanted).  All entries run as one batch, from the pages and states earlier
         steps left: one-token entries as decode rows (the captured graph when there is nothing
         else), longer ones as prompt portions beside them.  Returns the wanted logits [n, V] in the
-        order of the entries and offsets, or None."""
+        order of the entries and offsets, or None.  They are ordered on the current stream: the step may still run when
+        this returns, the next may be fed meanwhile, and the device's errors and time show where it is next waited for."""
         self._wait_meta()
         entries = [(s, list(toks), list(want)) for s, toks, want in entries]
         V = self.model.cfg.vocab_size

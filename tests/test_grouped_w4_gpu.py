@@ -43,6 +43,8 @@ def test_grouped(gpu, counts, K, kind):
     scale = 0.5 + torch.rand(R, device=gpu) if kind == "scaled" else None
     lim = (1.702, 3.0) if kind == "clamped" else None
     epi = 0 if kind == "plain" else 1
+    ops._sk_reserve(torch.device(gpu))
+    assert torch.ops.mlop.gemm_grouped_variant(R, N, K, G, 64, toks.shape[0]) == 5
     got = [ops.grouped_gemm(toks, w, off, epi=epi, avg_rows=64, a_rows=rows,
                             row_scale=scale, glu=lim) for _ in range(8)]
     assert all(torch.equal(got[0], g) for g in got[1:])
