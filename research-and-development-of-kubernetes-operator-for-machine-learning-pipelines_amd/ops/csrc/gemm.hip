@@ -542,7 +542,7 @@ int gemm_small_nt(int set) {
 }
 
 // non-temporal stores of GEMM outputs the next launch reads (gemm_slab_nt op; not left dirty in
-// L2 for the kernel boundary's write-back, MI355X_MICROARCH.md "boundary"): bit 0 the split-K
+// L2 for the kernel boundary's write-back, MI355X_MICROARCH.md "boundary"): bit 0 gemm_kernel's split-K
 // slabs (batch 256 +0.6 %, batch 64 neutral), bit 1 the four-wave kernel's C (headline +1.2 %),
 // bit 2 the ping-pong kernel's C (Mixtral batch 256 / 1024 and Llama batch 512 +0.3-0.4 %),
 // bit 3 the four-wave RoPE epilogue's q / K / V (with attn_kv_nt 3: headline +0.5 % over 5 pairs)
@@ -556,11 +556,9 @@ int gemm_slab_nt(int set) {
   if (set >= 0) g_slab_nt = set;
   return g_slab_nt;
 }
-// of the dense weight-streaming launches (gemm_kernel, gemm_mid.hip): 1 weights non-temporal, where one workgroup
-// streams each of them, 2 slabs non-temporal
-int gemm_stream_policy(int m_tiles) {
-  return ((g_small_nt_flags & 1) != 0 && m_tiles == 1 ? 1 : 0) | ((g_slab_nt & 1) != 0 ? 2 : 0);
-}
+// weights of the dense weight-streaming launches (gemm_kernel, gemm_mid.hip) non-temporal: where one workgroup streams
+// each of them
+bool gemm_weights_nt(int m_tiles) { return (g_small_nt_flags & 1) != 0 && m_tiles == 1; }
 
 template <int BM, int BN, int WM, int WN, int EPI, bool GROUPED, int STAGES, bool SETPRIO>
 static void run_cfg(const uint16_t* A, int lda, const uint16_t* B, int ldb, uint16_t* C, int ldc,
@@ -580,7 +578,7 @@ static void run_cfg(const uint16_t* A, int lda, const uint16_t* B, int ldb, uint
   // non-temporal weights where each weight byte is streamed by ONE workgroup: one m-tile
   // (dense), or the grouped decode tiles (an expert's few routed rows)
   RopeEpi r = re;
-  r.b_nt = GROUPED ? (g_small_nt_flags & 2) != 0 && BM <= 64 : (gemm_stream_policy(m_tiles) & 1) != 0;
+  r.b_nt = GROUPED ? (g_small_nt_flags & 2) != 0 && BM <= 64 : gemm_weights_nt(m_tiles);
   r.ws_nt = g_slab_nt;
   kern<<<blocks, T, lds, st>>>(A, lda, B, ldb, C, ldc, ws, M, N, K, k_chunk, offsets, n_groups, gx,
                                m_tiles, splits, r);
@@ -1829,7 +1827,7 @@ void gemm_plan(int M, int N, int K, int out[5]) {
   }
   const Plan p = plan(M, N, K, false, 0, 0);
   out[0] = p.variant, out[1] = p.BM, out[2] = p.BN, out[3] = p.splits;
-  out[4] = p.variant == 0 || p.variant == 7 ? gemm_stream_policy((M + p.BM - 1) / p.BM) : 0;
+  out[4] = (p.variant == 0 || p.variant == 7) && gemm_weights_nt((M + p.BM - 1) / p.BM);
 }
 
 long gemm_workspace_floats(int M, int N, int K, int epi) {

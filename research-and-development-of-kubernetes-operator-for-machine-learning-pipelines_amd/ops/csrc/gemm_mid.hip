@@ -51,7 +51,7 @@ __device__ __forceinline__ void wait_stages(int n) {
 
 // Tasks (column tile, row tile, K range), row tile fastest; a workgroup takes lid, lid + G, ...  SA / SB: ring
 // depths in K-steps of 64.  EPI 0: plain (with an activation, RopeEpi::act), 1: gate / up; several K ranges leave
-// fp32 slabs [range][M][N] in ws instead.
+// fp32 slabs [range][M][N] in ws instead, non-temporal always (a second form of the stores cost 3 % at 200 rows).
 template <int BM, int BN, int WM, int WN, int SA, int SB, int EPI>
 __global__ void __launch_bounds__(WM * WN * 64) gemm_mid_kernel(
     const uint16_t* __restrict__ A, int lda, const uint16_t* __restrict__ B, int ldb, uint16_t* __restrict__ C, int ldc,
@@ -173,24 +173,17 @@ __global__ void __launch_bounds__(WM * WN * 64) gemm_mid_kernel(
     const int mr = c_by * BM + wm * WTM + (lane & 15), nc = c_bx * BN + wn * WTN + 4 * g4;
     if (n_splits > 1) {
       float* P = ws + (size_t)c_bz * M * N;
-      auto slab = [&](auto nt_) {
 #pragma unroll
-        for (int i = 0; i < TM; ++i) {
-          const int m = mr + i * 16;
-          if (m < M) {
+      for (int i = 0; i < TM; ++i) {
+        const int m = mr + i * 16;
+        if (m < M) {
 #pragma unroll
-            for (int j = 0; j < TN; ++j) {
-              const int n = nc + j * 16;
-              f32x4* dst = reinterpret_cast<f32x4*>(P + (size_t)m * N + n);
-              if (n >= N) continue;
-              if constexpr (decltype(nt_)::value) __builtin_nontemporal_store(acc[i][j], dst);
-              else *dst = acc[i][j];
-            }
+          for (int j = 0; j < TN; ++j) {
+            const int n = nc + j * 16;
+            if (n < N) __builtin_nontemporal_store(acc[i][j], reinterpret_cast<f32x4*>(P + (size_t)m * N + n));
           }
         }
-      };
-      if (re.ws_nt) slab(std::true_type{});
-      else slab(std::false_type{});
+      }
       return;
     }
 #pragma unroll
@@ -268,9 +261,7 @@ static void run_mid(const uint16_t* A, int lda, const uint16_t* B, int ldb, uint
   const int tasks = gx * m_tiles * splits;
   constexpr int per_cu = (int)(163840 / lds) >= 2 ? 2 : 1;
   RopeEpi r = re;
-  const int policy = gemm_stream_policy(m_tiles);
-  r.b_nt = policy & 1;
-  r.ws_nt = policy >> 1;
+  r.b_nt = gemm_weights_nt(m_tiles);
   kern<<<std::min(tasks, 256 * per_cu), WM * WN * 64, lds, st>>>(A, lda, B, ldb, C, ldc, ws, M, N, K, k_chunk, m_tiles,
                                                                  splits, tasks, r);
 }

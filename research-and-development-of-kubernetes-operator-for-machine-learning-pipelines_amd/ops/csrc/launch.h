@@ -128,9 +128,9 @@ constexpr int epi_act(int epi) {
 void launch_rope_cache_slabs(const RopeEpi& re, const float* ws, int splits, int T, int N, hipStream_t st);
 long gemm_workspace_floats(int M, int N, int K, int epi);
 // what a plain product of this shape takes: kernel variant (gemm.hip plan; -1 the GEMV), tile rows, columns, K ranges,
-// cache policy of the weight-streaming tiles
+// weights loaded non-temporal (weight-streaming tiles)
 void gemm_plan(int M, int N, int K, int out[5]);
-int gemm_stream_policy(int m_tiles);
+bool gemm_weights_nt(int m_tiles);
 // the experts' product of M routed rows, max_rows of them per expert on average, from a_n rows: gemm.hip grouped_plan
 int gemm_grouped_variant(int M, int N, int K, int n_groups, int max_rows, int a_n);
 // large-M kernel variant of the GEMM planner (gemm.hip plan(): 0 256x128, 1/2 256x256

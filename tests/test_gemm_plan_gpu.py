@@ -67,17 +67,16 @@ def test_weight_stream_limits(gpu, M, N, K, stream):
 
 @pytest.mark.parametrize("M,N,K", [(16, 6144, 4096), (16, 28672, 4096), (64, 28672, 4096), (100, 6144, 4096), (200, 28672, 4096), (200, 4096, 14336)])
 def test_cache_policy_switches(gpu, M, N, K):
-    """Weights and slabs of the weight-streaming tiles go by gemm_small_nt and gemm_slab_nt, whichever kernel has them."""
+    """The weights of the weight-streaming tiles go by gemm_small_nt, whichever kernel has them."""
     ops._sk_reserve(torch.device(gpu))
     o = torch.ops.mlop
-    prev = o.gemm_small_nt(-1), o.gemm_slab_nt(-1)
+    prev = o.gemm_small_nt(-1)
     try:
-        for small in (0, 1, 6, 7):
-            for slab in (0, 1, 14, 15):
-                o.gemm_small_nt(small), o.gemm_slab_nt(slab)
-                assert o.gemm_plan(M, N, K)[4] == (small & 1) + 2 * (slab & 1)
+        for nt in (0, 1, 6, 7):
+            o.gemm_small_nt(nt)
+            assert o.gemm_plan(M, N, K)[4] == (nt & 1)
     finally:
-        o.gemm_small_nt(prev[0]), o.gemm_slab_nt(prev[1])
+        o.gemm_small_nt(prev)
 
 
 @pytest.mark.parametrize("M", [5, 16, 32, 64, 65])
