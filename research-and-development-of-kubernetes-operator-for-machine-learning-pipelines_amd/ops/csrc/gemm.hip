@@ -1390,11 +1390,12 @@ static bool mid_plan(int M, int N, int K, Plan& p) {
 // by estimated time in us.  A round of 256-row tiles takes 4.5 + 0.021 K; lower tiles cost more per row (192 rows 0.80
 // of it, 160 0.685, 128 0.645: fewer MFMAs per fragment read), and an only round that fills a share f of the CUs runs
 // faster.  A tail of at most half the CUs is cut into K-halves: half a round and the hand-off of the partials, behind
-// whole rounds the more the more of them there are.  A round of the ping-pong kernel takes 14 + 0.0208 K, its tail what
-// sk_tail_cost says.
+// whole rounds the more the more of them there are.  A round of the ping-pong kernel takes 14 + 0.0208 K, its tail 1.1 of
+// what sk_tail_cost says (1.0 fits as well; where the two are level the four-wave kernel is the better choice, since a
+// layer whose four projections all run there needs no add + RMSNorm passes: 1024 rows of Llama-3-8B 2855 -> 2811 us).
 // Constants fitted to 30 weight shapes (the projections of Llama-3-8B and 70B, whole and in 2 - 8 shards, Mixtral's,
 // and shapes of no model here: N 2048 - 128256, K 1024 - 28672) at 38 row counts from 385 to 8000, every variant measured
-// in one process, twice: the choice is 0.2 % slower than the best of the five on average, more than 5 % at 4 of 1147
+// in one process, twice: the choice is 0.2 % slower than the best of the five on average, more than 5 % at 8 of 1147
 // points, 12 % at worst; fitted to half of the shapes, 0.3 % on the others.  (Constants fitted to Llama-3-8B's matrices
 // alone: 1.4 %, 110 points and 38 %, and at 46 slower than the rule by tile counts that was here before: 70B qkv at 640
 // rows 113 us against 102, o at 1000 116 against 107, down at 2300 839 against 785; all three are 3 % from it now.)  That
@@ -1412,7 +1413,9 @@ static bool big_plan(int M, int N, int K, bool pp_ok, Plan& p) {
   p.BM = p.BN = 256;
   if (pp_ok) {
     const int T = (M + 255) / 256 * (N / 256), q = T / b->cus, r = T % b->cus, d = sk_choose_d(T, nk, b->cus, sk_min_half());
-    const float tail = d ? sk_tail_cost(r, nk, d) / (float)nk : r > 0 ? 1.f : 0.f;
+    // a grid of tails alone skips the last row tiles' empty 64-row quadrants
+    const float live = q > 0 ? 1.f : .7f + .3f * (float)((M + 63) / 64) / (float)((M + 255) / 256 * 4);
+    const float tail = d ? 1.1f * live * sk_tail_cost(r, nk, d) / (float)nk : r > 0 ? 1.f : 0.f;
     best = (14.f + 0.0208f * (float)K) * ((float)q + tail);
   }
   for (const Tile& t : tiles) {
