@@ -1393,7 +1393,7 @@ static bool mid_plan(int M, int N, int K, Plan& p) {
 // whole rounds the more the more of them there are.  A round of the ping-pong kernel takes 14 + 0.0208 K, its tail 1.1 of
 // what sk_tail_cost says (1.0 fits as well; where the two are level the four-wave kernel is the better choice, since a
 // layer whose four projections all run there needs no add + RMSNorm passes: 1024 rows of Llama-3-8B 2855 -> 2811 us).
-// Constants fitted to 30 weight shapes (the projections of Llama-3-8B and 70B, whole and in 2 - 8 shards, Mixtral's,
+// Constants fitted to 32 weight shapes (the projections of Llama-3-8B and 70B, whole and in 2 - 8 shards, Mixtral's,
 // and shapes of no model here: N 2048 - 128256, K 1024 - 28672) at 38 row counts from 385 to 8000, every variant measured
 // in one process, twice: the choice is 0.2 % slower than the best of the five on average, more than 5 % at 8 of 1147
 // points, 12 % at worst; fitted to half of the shapes, 0.3 % on the others.  (Constants fitted to Llama-3-8B's matrices

@@ -23,8 +23,8 @@
 // (the weights are the MFMA's first operand): a lane holds four neighbouring columns, gate and up of an
 // output sit in one lane, and nothing is staged for the epilogue.
 // Measured (cold weights, us, the LDS-ring tiles -> this kernel): gate_up 28672 x 4096 at 16 / 64 / 100 /
-// 150 / 300 rows 42 -> 37, 49 -> 39, 59 -> 45, 68 -> 51, 134 -> 82; lm_head 128256 x 4096 at 64 / 100 /
-// 150 / 256 / 300 rows 211 -> 168, 247 -> 175, 280 -> 181, 297 -> 251, 548 -> 339; down 4096 x 14336 with
+// 150 rows 42 -> 37, 49 -> 39, 59 -> 45, 68 -> 51; lm_head 128256 x 4096 at 64 / 100 /
+// 150 / 256 rows 211 -> 168, 247 -> 175, 280 -> 181, 297 -> 251; down 4096 x 14336 with
 // its reduce at 100 / 150 / 300 rows 37 -> 34, 46 -> 39, 68 -> 56.
 #include "common.h"
 #include "launch.h"
