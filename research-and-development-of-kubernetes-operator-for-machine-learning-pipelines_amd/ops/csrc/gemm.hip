@@ -1387,26 +1387,27 @@ static bool mid_plan(int M, int N, int K, Plan& p) {
 }
 
 // Above the weight stream's rows: the four-wave kernel's tile height, or the ping-pong kernel with its stream-K tail,
-// by estimated time in us.  A round of 256-row tiles takes 4.5 + 0.021 K; lower tiles cost more per row (192 rows 0.80
-// of it, 160 0.685, 128 0.645: fewer MFMAs per fragment read), and an only round that fills a share f of the CUs runs
-// faster.  A tail of at most half the CUs is cut into K-halves: half a round and the hand-off of the partials, behind
-// whole rounds the more the more of them there are.  A round of the ping-pong kernel takes 14 + 0.0208 K, its tail 1.1 of
+// by estimated time in us.  A round of 256-row tiles takes 6 + 0.0207 K; lower tiles cost more per row (192 rows 0.805
+// of it, 160 0.70, 128 0.632: fewer MFMAs per fragment read), and an only round that fills a share f of the CUs runs
+// faster.  A tail of at most half the CUs is cut into K-halves: half a round and the hand-off of the partials,
+// 15 us.  A round of the ping-pong kernel takes 13.5 + 0.0206 K, its tail 1.1 of
 // what sk_tail_cost says (1.0 fits as well; where the two are level the four-wave kernel is the better choice, since a
 // layer whose four projections all run there needs no add + RMSNorm passes: 1024 rows of Llama-3-8B 2855 -> 2811 us).
-// Constants fitted to 32 weight shapes (the projections of Llama-3-8B and 70B, whole and in 2 - 8 shards, Mixtral's,
-// and shapes of no model here: N 2048 - 128256, K 1024 - 28672) at 38 row counts from 385 to 8000, every variant measured
-// in one process, twice: the choice is 0.2 % slower than the best of the five on average, more than 5 % at 8 of 1147
-// points, 12 % at worst; fitted to half of the shapes, 0.3 % on the others.  (Constants fitted to Llama-3-8B's matrices
-// alone: 1.4 %, 110 points and 38 %, and at 46 slower than the rule by tile counts that was here before: 70B qkv at 640
-// rows 113 us against 102, o at 1000 116 against 107, down at 2300 839 against 785; all three are 3 % from it now.)  That
-// rule, heights 256 and 128 only, was 8.4 % slower than the best (gate_up of Llama-3-8B at 400 / 700 / 1152 rows 138 ->
-// 92, 158 -> 147, 245 -> 219 us, o at 1152 / 2300 / 2600 55 -> 43, 79 -> 62, 83 -> 68).
+// Constants fitted to 39 weight shapes (the projections of Llama-3-8B and 70B, whole and in 2 - 8 shards, Mixtral's,
+// a 1B model's and shapes of no model here: N 1024 - 128256, K 1024 - 28672) at 39 row counts from 385 to 8192, every
+// variant measured in one process, two to four times: the choice is 0.13 % slower than the best of the five on average,
+// more than 5 % at 8 of 1370 points, 12 % at worst; fitted to half of the shapes, 0.3 % on the others.  (Constants fitted
+// to Llama-3-8B's matrices alone: 1.4 %, 110 of 1147 points and 38 %, and at 46 of them slower than the rule by tile
+// counts that was here before: 70B qkv at 640 rows 113 us against 102, o at 1000 116 against 107, down at 2300 839
+// against 785; all three are within 3 % of the best now.)  That rule, heights 256 and 128 only, was 8.4 % slower than the
+// best (gate_up of Llama-3-8B at 400 / 700 / 1152 rows 138 -> 92, 158 -> 147, 245 -> 219 us, o at 1152 / 2300 / 2600
+// 55 -> 43, 79 -> 62, 83 -> 68).
 static bool big_plan(int M, int N, int K, bool pp_ok, Plan& p) {
   const SkBuf* b = sk_buf();
   if (!b || !gemm_w4_ok(M, N, K, K, K)) return false;
   struct Tile { int rows; float round, slope; };
-  constexpr Tile tiles[] = {{256, 1.f, .2f}, {192, .80f, .2f}, {160, .685f, .05f}, {128, .645f, .15f}};
-  const float full = 4.5f + 0.021f * (float)K, C = (float)b->cus;
+  constexpr Tile tiles[] = {{256, 1.f, .3f}, {192, .805f, .25f}, {160, .70f, .1f}, {128, .632f, 0.f}};
+  const float full = 6.f + 0.0207f * (float)K, C = (float)b->cus;
   const int nk = K / kBK;
   float best = 1e30f;
   p.variant = 3;
@@ -1416,7 +1417,7 @@ static bool big_plan(int M, int N, int K, bool pp_ok, Plan& p) {
     // a grid of tails alone skips the last row tiles' empty 64-row quadrants
     const float live = q > 0 ? 1.f : .7f + .3f * (float)((M + 63) / 64) / (float)((M + 255) / 256 * 4);
     const float tail = d ? 1.1f * live * sk_tail_cost(r, nk, d) / (float)nk : r > 0 ? 1.f : 0.f;
-    best = (14.f + 0.0208f * (float)K) * ((float)q + tail);
+    best = (13.5f + 0.0206f * (float)K) * ((float)q + tail);
   }
   for (const Tile& t : tiles) {
     if (t.rows < 256 && !g_half_tile) break;
@@ -1426,7 +1427,7 @@ static bool big_plan(int M, int N, int K, bool pp_ok, Plan& p) {
     const bool halves = r > 0 && gemm_w4_split_ok((int)T, nk);
     const float fill = (halves ? 2.f : 1.f) * (float)r / C, slope = q > 0 ? 0.f : t.slope;
     if (r > 0) us += (halves ? .5f : 1.f) * one * (1.f - slope * (1.f - fill));
-    if (halves) us += q > 0 ? 15.f * fill : 14.f;
+    if (halves) us += q > 0 ? 15.f : 15.5f;
     if (us < best) {
       best = us;
       p.variant = t.rows == 256 ? 5 : 6;

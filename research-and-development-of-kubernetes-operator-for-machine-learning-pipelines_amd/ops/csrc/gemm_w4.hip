@@ -15,7 +15,7 @@
 // outputs per wave (a[0:127]), 12 DMA pieces per K-tile, its own generated loop
 // (MLOP_W4H_KLOOP_*, 64 MFMAs per K-tile), every epilogue shared with the full tile.  BMT = 160 and 192
 // (80 and 96 output rows per wave, loops MLOP_W4_160_* / _192_*) stand between them for grids that both fill
-// badly: whole rounds take 0.685 and 0.80 of the full tile's (gemm.hip big_plan has the choice and its figures).
+// badly: whole rounds take 0.70 and 0.805 of the full tile's (gemm.hip big_plan has the choice and its figures).
 //
 // HIP handles the rest: tile placement (XCD-contiguous bands, as gemm_pp_kernel), per-lane
 // DMA source offsets (rows clamped to the last valid row, XOR swizzle in the source), the
