@@ -501,7 +501,7 @@ int attn_kv_nt(int set) {
 // (35.1), 20 x 800 23.9 (22.4).  Counts a little above one per CU run as long as two (not powers of two, as steps beside
 // prompts have: 104 pairs in 3 shares 36.9 us, in 2 33; 136 pairs in 2 41, in 3 33; 288 pairs whole 77, in 2 66).
 static int even_parts(int base) {
-  constexpr int wgs = 256, two = 384;
+  constexpr int wgs = kCus, two = 384;
   if (base <= wgs / 2) return wgs / base;
   return base == wgs || base >= two ? 1 : (two + base - 1) / base;
 }

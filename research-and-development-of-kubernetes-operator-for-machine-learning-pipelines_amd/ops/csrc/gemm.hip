@@ -1354,7 +1354,7 @@ static bool sk_halves_ok(long T, int nk) {
 // (o 4096 x 4096 at 100 rows 17.5 us against 18.6 in six ranges; down 4096 x 14336 at 16 / 64 rows 24.2 / 29.2
 // against 26.6 / 29.5).
 static bool mid_plan(int M, int N, int K, Plan& p) {
-  constexpr int max_m = 384, fill = 192;
+  constexpr int max_m = 384, fill = kCus * 3 / 4;
   if (M > max_m || K < kBK || K % kBK || N % 8) return false;  // (no K-step: gemm_kernel writes the empty sums)
   if (M <= 64 && g_small_tile != 1) return false;              // one of gemm_kernel's tiles is asked for
   const int m_tiles = M <= 256 ? 1 : 2, rows = (M + m_tiles - 1) / m_tiles;
@@ -1362,7 +1362,7 @@ static bool mid_plan(int M, int N, int K, Plan& p) {
   const int t256 = (N + 255) / 256 * m_tiles, t128 = (N + 127) / 128 * m_tiles, nk = K / kBK;
   int s = 1;
   if (t256 < fill && t128 < fill) {
-    s = std::min({kMaxSplits, 256 / t128, nk / 12});
+    s = std::min({kMaxSplits, kCus / t128, nk / 12});
     if (M <= 64 || t128 * s < fill) return false;
     const int t64 = (N + 63) / 64;
     // where the 64-column tiles need no K ranges, the slabs have to be small beside the weights (12544 x 2048 in two
@@ -1370,7 +1370,7 @@ static bool mid_plan(int M, int N, int K, Plan& p) {
     // tiles fill the CUs with K in a few ranges (8192 x 3584 in four at 80 / 112 / 128 rows 23 / 26.0 / 26.5 us against 24 /
     // 24.2 / 24.5, at 160 / 192 / 256 rows 28.5 / 31.6 / 36.4 against 29.6 / 30.2 / 32.2)
     if (t64 >= 160 && 4l * s * M > K * 3l / 10) return false;
-    if (m_tiles == 1 && t64 < 160 && t64 * std::max(1, 256 / t64) >= 250 && 400l * s * M > K * (M <= 128 ? 43l : 80l)) return false;
+    if (m_tiles == 1 && t64 < 160 && t64 * std::max(1, kCus / t64) >= 250 && 400l * s * M > K * (M <= 128 ? 43l : 80l)) return false;
   }
   // Two row tiles read the weights twice (the second from L2).  Where the four-wave kernel's lower tiles have a grid, they
   // are faster without K ranges, and with them above 320 rows (257 / 384 rows of gate_up 28672 x 4096 80 / 92 us ->

@@ -262,7 +262,7 @@ static void run_mid(const uint16_t* A, int lda, const uint16_t* B, int ldb, uint
   constexpr int per_cu = (int)(163840 / lds) >= 2 ? 2 : 1;
   RopeEpi r = re;
   r.b_nt = gemm_weights_nt(m_tiles);
-  kern<<<std::min(tasks, 256 * per_cu), WM * WN * 64, lds, st>>>(A, lda, B, ldb, C, ldc, ws, M, N, K, k_chunk, m_tiles,
+  kern<<<std::min(tasks, kCus * per_cu), WM * WN * 64, lds, st>>>(A, lda, B, ldb, C, ldc, ws, M, N, K, k_chunk, m_tiles,
                                                                  splits, tasks, r);
 }
 }  // namespace

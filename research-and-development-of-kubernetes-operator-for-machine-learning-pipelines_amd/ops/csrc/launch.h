@@ -10,6 +10,9 @@
 
 namespace mlop {
 
+// compute units of an MI355X, for plans that hold without the stream-K scratch (which knows its device's: SkBuf::cus)
+constexpr int kCus = 256;
+
 void launch_rmsnorm(void* out, const void* x, const void* w, float eps, int M, int H,
                     hipStream_t st);
 void launch_add_rmsnorm(void* out, void* residual, const void* x, const void* w, float eps, int M,
