@@ -72,17 +72,19 @@ if __name__ == "__main__":
 
 
 def _warm_hip() -> None:
-    """Initialise the HIP runtime and this rank's device context on a helper thread WHILE torch
-    imports (~1.4 s of Python and dlopen): the C calls release the GIL, and torch's own first
-    device call then finds the runtime up (first allocation 0.15-0.35 s -> ~0.1 s,
-    scripts/probe_startup.py).  Off for CPU predictors and with MLOP_HIP_WARMUP=0."""
+    """Initialise the HIP runtime and this rank's device context on a helper thread while the rest
+    of the predictor is imported: the C calls release the GIL, and torch's own first device call
+    then finds the runtime up.  Only between libraries: loading one with device code registers its
+    kernels with the runtime, which walks the registered ones when it initialises.  So torch is
+    loaded before, and ``ops.load`` waits for this thread.  Off for CPU predictors and with
+    MLOP_HIP_WARMUP=0."""
     import ctypes
     import importlib.util
 
     try:
-        # torch's OWN copy of the runtime (its lib/ directory, found without importing torch): a
-        # bare "libamdhip64.so" could resolve to the system ROCm copy, and a second HIP runtime
-        # in the process would not be the one torch and _C.so launch on
+        # torch's OWN copy of the runtime (its lib/ directory): a bare "libamdhip64.so" could resolve
+        # to the system ROCm copy, and a second HIP runtime in the process would not be the one torch
+        # and _C.so launch on
         spec = importlib.util.find_spec("torch")
         if spec is None or not spec.origin:
             return
@@ -107,16 +109,18 @@ def start_hip_warmup() -> bool:
 
     rank_launcher.WARMUP_STARTED = True
     STARTUP["hip_warmup_started"] = True
-    threading.Thread(target=_warm_hip, name="hip-warmup", daemon=True).start()
+    t = threading.Thread(target=_warm_hip, name="hip-warmup", daemon=True)
+    ops.before_load.append(t)
+    t.start()
     return True
 
 
-if __name__ == "__main__":
-    start_hip_warmup()
-
-from .sampler import SamplingParams  # noqa: E402 (imports torch: timed below)
+from .. import ops  # noqa: E402 (imports torch: timed below)
+from .sampler import SamplingParams  # noqa: E402
 
 STARTUP["torch_imported_s"] = _since_process_start()
+if __name__ == "__main__":
+    start_hip_warmup()
 
 _DT = {"FP32": np.float32, "FP64": np.float64, "INT64": np.int64, "INT32": np.int32, "FP16": np.float16,
        "BOOL": np.bool_, "UINT8": np.uint8}

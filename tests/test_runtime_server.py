@@ -268,7 +268,7 @@ def test_kernel_time_shares_exported():
 
 
 def test_hip_warmup_loads_torchs_own_runtime():
-    """The predictor's start-up thread initialises HIP while torch imports (server._warm_hip).  It
+    """The predictor's start-up thread initialises HIP while the server is imported (server._warm_hip).  It
     must load torch's OWN libamdhip64 (torch/lib): a second HIP runtime in the process (e.g. the
     system ROCm copy) would not be the one torch and _C.so launch on.  After the server module,
     torch and the extension are loaded, exactly one HIP runtime file is mapped."""
@@ -289,6 +289,42 @@ def test_hip_warmup_loads_torchs_own_runtime():
     maps = ast.literal_eval(out.stdout.strip().splitlines()[-1])
     torch_lib = os.path.join(os.path.dirname(torch.__file__), "lib")
     assert len(maps) == 1 and maps[0].startswith(torch_lib), maps
+
+
+def test_hip_warmup_overlaps_no_library_load():
+    """Loading a library with device code registers its kernels with the HIP runtime, which walks them when it is
+    initialised: the start-up thread begins behind torch's libraries and ends before the extension's load."""
+    import os
+    import subprocess
+    import sys
+
+    code = """
+import os, runpy, sys, threading, time
+begun, order, start = [], [], threading.Thread.start
+def noted(t):
+    if t.name == "hip-warmup":
+        maps = open("/proc/self/maps").read()
+        begun.append("libtorch_hip" in maps and "torch" in sys.modules and hasattr(sys.modules["torch"], "ops"))
+        t._target = lambda: (time.sleep(0.5), order.append("runtime"))
+    start(t)
+threading.Thread.start = noted
+sys.argv = ["server", "--help"]
+try:
+    runpy.run_module("mlopamd.runtime.server", run_name="__main__")
+except SystemExit:
+    pass
+import torch
+from mlopamd import ops
+load = torch.ops.load_library
+torch.ops.load_library = lambda p: (order.append("load"), load(p))
+ops.load()
+print(begun, order)
+"""
+    env = {k: v for k, v in os.environ.items() if k not in ("MLOP_DEVICE", "MLOP_HIP_WARMUP", "MLOP_RUNTIME", "WORLD_SIZE")}
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    env["PYTHONPATH"] = root + os.pathsep + env.get("PYTHONPATH", "")
+    out = subprocess.run([sys.executable, "-c", code], env=env, capture_output=True, text=True, timeout=300)
+    assert out.stdout.strip().endswith("[True] ['runtime', 'load']"), out.stdout[-300:] + out.stderr[-2000:]
 
 
 def test_engine_clock_and_tokens_come_from_one_snapshot():
