@@ -56,8 +56,10 @@ if os.environ.get("MLOP_LAUNCHER_INFO"):  # this rank's pod launcher (rank_launc
     STARTUP["launcher"] = json.loads(os.environ["MLOP_LAUNCHER_INFO"])
 
 if __name__ == "__main__":
+    import faulthandler as _faulthandler
     import sys as _sys
 
+    _faulthandler.enable()  # a crash leaves every thread's Python stack in the pod's log
     # one module object whether reached as __main__ or as a package import (tp_worker /
     # ep_serving import make_app from here): one STARTUP dict, one set of globals
     _sys.modules.setdefault(f"{__package__}.server", _sys.modules[__name__])
