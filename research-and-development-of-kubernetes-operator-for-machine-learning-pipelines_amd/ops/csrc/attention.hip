@@ -513,7 +513,10 @@ static void launch_g(void* out, float* part_o, float* part_ml, const void* q, co
                      int num_tiles, int Hq, int Hkv, float scale_log2, int part_tokens, int nparts,
                      int num_blocks, int* sem, hipStream_t st) {
   const int even = std::min(nparts, even_parts(num_tiles * Hkv));
-  if (num_tiles == 1 || even >= kEnoughParts) nparts = even;  // (seq_part: none needs more)
+  if (num_tiles == 1 || even >= kEnoughParts) {  // (seq_part: none needs more)
+    if (even == 1 && nparts > 1) part_tokens = 1 << 30;  // the only partition has all keys, whatever was planned
+    nparts = even;
+  }
   dim3 grid(num_tiles, Hkv, nparts);
   // K / V pages non-temporal (attn_kv_nt op): each is read once per step by one workgroup
   // (below 8 query tiles the default policy: batch 4 lost 0.7 % with it, batch 16 gained 1.8 %)

@@ -279,6 +279,24 @@ def test_paged_attention_partitions_of_a_longer_limit(gpu, Hq, Hkv, part_tokens,
         assert (out[-2:] == 0).all() and int(m.part_sem.abs().sum()) == 0
 
 
+@pytest.mark.parametrize("Hkv,ctx", [(128, 3000), (255, 3000), (256, 1), (256, 3000), (383, 1500), (400, 700)])
+def test_paged_attention_one_sequence_many_kv_heads(gpu, Hkv, ctx, attn_fused_all):
+    """One sequence whose kv heads alone fill the CUs: planned in several partitions, launched in one that has all keys."""
+    from mlopamd.runtime.attn_meta import plan_partitions
+
+    torch.manual_seed(0)
+    np.random.seed(0)
+    NB = (ctx + 15) // 16 + 2
+    kc = torch.randn(NB, Hkv, 16, 128, device=gpu, dtype=bf)
+    vc = torch.randn(NB, Hkv, 16, 128, device=gpu, dtype=bf)
+    part, nparts = plan_partitions(1, Hkv, max(ctx, 256))
+    assert nparts > 1
+    m, T = make_meta(gpu, [1], [ctx], Hkv, 1, NB, part_tokens=part, nparts=nparts)
+    m.part_sem = torch.zeros(m.tile_seq.numel() * Hkv, dtype=torch.int32, device=gpu)
+    q = torch.randn(T, Hkv, 128, device=gpu, dtype=bf)
+    close(ops.paged_attention(q, kc, vc, m), ref.paged_attention(q, kc, vc, m), atol=2e-2, rtol=2e-2)
+
+
 @pytest.mark.parametrize("fused", [False, True])
 @pytest.mark.parametrize("Hq,Hkv,long,short,padding", [
     (32, 8, [4000], [100] * 20, 0),            # all of the 7 shares that are planned
