@@ -622,7 +622,7 @@ void gemm_grouped_plan(int bm, int bn, int stages, int splits) {
 
 // dense-plan override (scripts/bench_mid_m.py sweeps the mid-M projection tilings in one
 // process): variant (0 = gemm_kernel BM x BN, 1 = 256x256 two-stage, 3 = ping-pong, 5 =
-// four-wave, 6 = four-wave of BM 160 or 192 rows, else half height), BM, BN, K splits (plain gemm_kernel only), LDS
+// four-wave, 6 = four-wave of BM 160, 192 or 224 rows, else half height), BM, BN, K splits (plain gemm_kernel only), LDS
 // ring depth of the small tiles (0 = the default); -1 = the planner's own choice
 static int g_dp[5] = {-1, -1, -1, -1, 0};
 void gemm_dense_plan(int variant, int bm, int bn, int splits, int stages) {
@@ -1338,7 +1338,7 @@ struct Plan {
 //   large M: variant 0 = 256x128 (3-stage ring), 1 = 256x256 (2-stage, 128x64 per
 //   wave: half the LDS + L2 bytes per FLOP), 2 = 256x256 + setprio around MFMAs,
 //   3 = 256x256 two-group ping-pong (gemm_pp_kernel), 5 (default) = the four-wave kernel with
-//   the hand-scheduled asm K-loop (gemm_w4.hip), 256 rows, 6 = its tiles of 128, 160 and 192 rows (big_plan
+//   the hand-scheduled asm K-loop (gemm_w4.hip), 256 rows, 6 = its tiles of 128 - 224 rows (big_plan
 //   chooses between 3, 5 and 6; without its scratch 5 where the grid fills the chip, else 3), 7 = the weight
 //   stream of gemm_mid.hip (mid_plan, up to 384 rows, before all others).  (A four-wave 128x128-per-wave
 //   variant was measured 10-20% slower: profiles/r02_gemm_fourwave_rejected.md.)
@@ -1387,8 +1387,8 @@ static bool mid_plan(int M, int N, int K, Plan& p) {
 }
 
 // Above the weight stream's rows: the four-wave kernel's tile height, or the ping-pong kernel with its stream-K tail,
-// by estimated time in us.  A round of 256-row tiles takes 6 + 0.0207 K; lower tiles cost more per row (192 rows 0.805
-// of it, 160 0.70, 128 0.632: fewer MFMAs per fragment read), and an only round that fills a share f of the CUs runs
+// by estimated time in us.  A round of 256-row tiles takes 6 + 0.0207 K; lower tiles cost more per row (224 rows 0.90
+// of it, 192 0.805, 160 0.70, 128 0.632: fewer MFMAs per fragment read), and an only round that fills a share f of the CUs runs
 // faster.  A tail of at most half the CUs is cut into K-halves: half a round and the hand-off of the partials,
 // 15 us.  A round of the ping-pong kernel takes 13.5 + 0.0206 K, its tail 1.1 of
 // what sk_tail_cost says (1.0 fits as well; where the two are level the four-wave kernel is the better choice, since a
@@ -1399,14 +1399,16 @@ static bool mid_plan(int M, int N, int K, Plan& p) {
 // more than 5 % at 8 of 1370 points, 12 % at worst; fitted to half of the shapes, 0.3 % on the others.  (Constants fitted
 // to Llama-3-8B's matrices alone: 1.4 %, 110 of 1147 points and 38 %, and at 46 of them slower than the rule by tile
 // counts that was here before: 70B qkv at 640 rows 113 us against 102, o at 1000 116 against 107, down at 2300 839
-// against 785; all three are within 3 % of the best now.)  That rule, heights 256 and 128 only, was 8.4 % slower than the
+// against 785; all three are within 3 % of the best now.)  The 224-row tile, measured on 13 of the shapes at 21 row counts:
+// 1.2 % faster on average, 53 of 273 points by more than 2 % (gate_up at 400 / 892 / 1100 rows 99 -> 89, 188 -> 174, 216 ->
+// 209 us), the choice among the heights 0.27 % slower than the best, over 5 % at three points.  That rule, heights 256 and 128 only, was 8.4 % slower than the
 // best (gate_up of Llama-3-8B at 400 / 700 / 1152 rows 138 -> 92, 158 -> 147, 245 -> 219 us, o at 1152 / 2300 / 2600
 // 55 -> 43, 79 -> 62, 83 -> 68).
 static bool big_plan(int M, int N, int K, bool pp_ok, Plan& p) {
   const SkBuf* b = sk_buf();
   if (!b || !gemm_w4_ok(M, N, K, K, K)) return false;
   struct Tile { int rows; float round, slope; };
-  constexpr Tile tiles[] = {{256, 1.f, .3f}, {192, .805f, .25f}, {160, .70f, .1f}, {128, .632f, 0.f}};
+  constexpr Tile tiles[] = {{256, 1.f, .3f}, {224, .90f, .28f}, {192, .805f, .25f}, {160, .70f, .1f}, {128, .632f, 0.f}};
   const float full = 6.f + 0.0207f * (float)K, C = (float)b->cus;
   const int nk = K / kBK;
   float best = 1e30f;
@@ -1557,7 +1559,7 @@ static Plan plan(int M, int N, int K, bool grouped, int n_groups, int rows_per_g
   }
   if (!grouped && g_dp[0] >= 0) {  // bench override (gemm_dense_plan)
     p.variant = g_dp[0];
-    p.BM = p.variant == 0 || (p.variant == 6 && (g_dp[1] == 160 || g_dp[1] == 192)) ? g_dp[1] : p.variant == 6 ? 128 : 256;
+    p.BM = p.variant == 0 || (p.variant == 6 && (g_dp[1] == 160 || g_dp[1] == 192 || g_dp[1] == 224)) ? g_dp[1] : p.variant == 6 ? 128 : 256;
     p.BN = p.variant == 0 ? g_dp[2] : 256;
     p.stages = g_dp[4];
   }
@@ -1912,26 +1914,24 @@ bool launch_gemm_add_rmsnorm(const void* A, int lda, const void* B, void* out, v
 }
 
 // The experts' products: gemm_kernel's tiles, the ping-pong kernel (variant 3) or the four-wave kernel (5).  The latter
-// where the 256-row tiles make three rounds or more (gate_up): with fewer, stream-K's even split of the tail wins (down
-// of 8 experts at 350 / 450 / 1024 rows each 320 / 355 / 791 us against 318 / 375 / 798).
-// gate_up of 8 experts, ping-pong -> four-wave: 75 / 125 / 300 / 350 / 500 / 625 / 1024 rows each 374 -> 353, 376 ->
-// 364, 630 -> 530, 654 -> 604, 828 -> 772, 1047 -> 978, 1606 -> 1479 us, and with the experts 0.6 - 1.4 of that 370
-// -> 351, 375 -> 352, 636 -> 595, 666 -> 646, 877 -> 848, 1072 -> 954, 1620 -> 1481.  Not at 160 - 240 and 368 - 440
-// rows on average, where experts of exactly that size are most of one or two 256-row tiles but not of lower ones, and the
-// ping-pong kernel skips a tile's empty 64-row quadrants (200 rows 397 us against 436, 425 714 against 745).
-// The bands are those of this one shape and of equal experts.  Measured in one process on others (8 experts of half the
-// width, 4 of the same, 16 x 12800 x 4096, 32 x 8192 x 2048, 64 x 2816 x 2048; 43 row counts; equal experts, random
-// tokens, experts 0.6 - 1.4 of the mean, one expert of two fifths of the tokens): outside the bands the choice is at
-// most 6 % slower than ping-pong (at 240 - 256 equal rows) and 13 % faster on average; inside them the four-wave kernel
-// would be 4 - 16 % faster on 4 - 16 experts, by routing, and 10 - 37 % on 32 and 64, at single sizes up to 9 % slower: a
-// choice on the host, from the mean alone, cannot tell.
+// where tiles of 224 rows (one per expert up to 256) make two and a half rounds or more; with fewer, stream-K's even split of the tail wins (down of 8
+// experts at 200 / 407 / 700 rows each on average 200 / 341 / 547 us against 222 / 361 / 586; at 1024 805 against 770).
+// gate_up of 8 experts, random tokens, ping-pong -> four-wave: 300 / 368 / 407 / 440 / 512 / 700 / 1024 rows each 651 -> 537,
+// 681 -> 573, 755 -> 684, 782 -> 733, 921 -> 813, 1130 -> 1000, 1640 -> 1435 us; of 8 experts of half the width at 256 / 300 /
+// 407 rows 295 -> 267, 345 -> 280, 380 -> 345, of 4 at 512 479 -> 417.  (Without the 224-row tile the ping-pong kernel had 368
+// - 440 rows: two 256-row tiles of which a fifth is empty, and three lower ones.)  Not at 160 - 240 rows of up to 8 experts,
+// one tile each: there the weights' latency bounds both, and the ping-pong kernel skips a tile's empty 64-row quadrants (200
+// rows 394 us against 420; 16 x 12800 x 4096 378 against 355, 32 x 8192 x 2048 290 against 254); at 64 - 140 rows they are level.
+// Measured in one process on six shapes (those, 8 experts of half the width, 4 of the same, down), 19 row counts, equal
+// experts, random tokens and experts 0.6 - 1.4 of the mean: where the four-wave kernel is chosen it takes 0.755 - 1.04 of the
+// ping-pong kernel's time (1.11 at 240 - 256 equal rows of 8 x 28672 x 4096).
 static Plan grouped_plan(int M, int N, int K, int n_groups, int max_rows, int a_n) {
   Plan p = plan(M, N, K, true, n_groups, max_rows);
-  const bool quadrants = (max_rows >= 160 && max_rows < 240) || (max_rows >= 368 && max_rows < 440);
+  const bool quadrants = max_rows >= 160 && max_rows < 240 && n_groups <= 8;
+  const int tiles = max_rows <= 256 ? 1 : (max_rows + 223) / 224;
   if (p.variant == 3 && g_gp[0] <= 0 && !quadrants) {
     const SkBuf* b = sk_buf();
-    if (b && (long)n_groups * std::max(1, (max_rows + 128) / 256) * (N / 256) >= 3l * b->cus &&
-        gemm_w4_grouped_ok(M, N, K, n_groups, a_n))
+    if (b && 2l * n_groups * tiles * (N / 256) >= 5l * b->cus && gemm_w4_grouped_ok(M, N, K, n_groups, a_n))
       p.variant = 5;
   }
   return p;

@@ -13,9 +13,10 @@
 // fragments of tile t in registers, so one buffer pair keeps a whole tile in flight.
 // BMT = 128 is the half-height tile (planner variant 6): 64 x 128
 // outputs per wave (a[0:127]), 12 DMA pieces per K-tile, its own generated loop
-// (MLOP_W4H_KLOOP_*, 64 MFMAs per K-tile), every epilogue shared with the full tile.  BMT = 160 and 192
-// (80 and 96 output rows per wave, loops MLOP_W4_160_* / _192_*) stand between them for grids that both fill
-// badly: whole rounds take 0.70 and 0.805 of the full tile's (gemm.hip big_plan has the choice and its figures).
+// (MLOP_W4H_KLOOP_*, 64 MFMAs per K-tile), every epilogue shared with the full tile.  BMT = 160, 192 and 224
+// (80, 96 and 112 output rows per wave, loops MLOP_W4_160_* / _192_* / _224_*) stand between them for grids that both
+// fill badly: whole rounds take 0.70, 0.805 and 0.90 of the full tile's (gemm.hip big_plan has the choice and its
+// figures).
 //
 // HIP handles the rest: tile placement (XCD-contiguous bands, as gemm_pp_kernel), per-lane
 // DMA source offsets (rows clamped to the last valid row, XOR swizzle in the source), the
@@ -93,7 +94,7 @@ __device__ __forceinline__ void gemm_w4_tiles(
   // BMT = 256: 128 x 128 outputs per wave; BMT = 128 (the half-height tile, twice the tiles for
   // the mid-M and QKV grids): 64 x 128 per wave, 4 x 8 accumulators, 12 DMA pieces per K-tile
   constexpr int BM = BMT, BN = 256;
-  static_assert(BMT == 256 || BMT == 192 || BMT == 160 || BMT == 128, "tile heights of the generated K-loops");
+  static_assert(BMT == 256 || BMT == 224 || BMT == 192 || BMT == 160 || BMT == 128, "tile heights of the generated K-loops");
   constexpr int NI = BMT / 32;      // 16-row accumulator blocks per wave
   constexpr int NPC = NI + 8;       // DMA pieces per wave and K-tile (NI of A, 8 of B)
   // epilogue store instructions per wave and tile (the next tile's K-loop waits for its
@@ -308,87 +309,21 @@ __device__ __forceinline__ void gemm_w4_tiles(
     bf16x8 fb0_0, fb0_1, fb0_2, fb0_3, fb0_4, fb0_5, fb0_6, fb0_7;
     bf16x8 fa1_0, fa1_1, fa1_2, fa1_3, fa1_4, fa1_5, fa1_6, fa1_7;
     bf16x8 fb1_0, fb1_1, fb1_2, fb1_3, fb1_4, fb1_5, fb1_6, fb1_7;
-#define MLOP_W4_OPERANDS                                                                                         \
-  : [fa0_0] "=&v"(fa0_0), [fa0_1] "=&v"(fa0_1), [fa0_2] "=&v"(fa0_2), [fa0_3] "=&v"(fa0_3),                      \
-    [fa0_4] "=&v"(fa0_4), [fa0_5] "=&v"(fa0_5), [fa0_6] "=&v"(fa0_6), [fa0_7] "=&v"(fa0_7),                      \
-    [fb0_0] "=&v"(fb0_0), [fb0_1] "=&v"(fb0_1), [fb0_2] "=&v"(fb0_2), [fb0_3] "=&v"(fb0_3),                      \
-    [fb0_4] "=&v"(fb0_4), [fb0_5] "=&v"(fb0_5), [fb0_6] "=&v"(fb0_6), [fb0_7] "=&v"(fb0_7),                      \
-    [fa1_0] "=&v"(fa1_0), [fa1_1] "=&v"(fa1_1), [fa1_2] "=&v"(fa1_2), [fa1_3] "=&v"(fa1_3),                      \
-    [fa1_4] "=&v"(fa1_4), [fa1_5] "=&v"(fa1_5), [fa1_6] "=&v"(fa1_6), [fa1_7] "=&v"(fa1_7),                      \
-    [fb1_0] "=&v"(fb1_0), [fb1_1] "=&v"(fb1_1), [fb1_2] "=&v"(fb1_2), [fb1_3] "=&v"(fb1_3),                      \
-    [fb1_4] "=&v"(fb1_4), [fb1_5] "=&v"(fb1_5), [fb1_6] "=&v"(fb1_6), [fb1_7] "=&v"(fb1_7),                      \
-    [rA0] "+v"(rA0), [rA1] "+v"(rA1), [rB0] "+v"(rB0), [rB1] "+v"(rB1), [koff] "+s"(koff), [dbase] "+s"(dbase), \
-    [iter] "+s"(iter), [m0save] "=&s"(m0save)                                                                    \
-  : [vo0] "v"(vo[0]), [vo1] "v"(vo[1]), [vo2] "v"(vo[2]), [vo3] "v"(vo[3]), [vo4] "v"(vo[4]), [vo5] "v"(vo[5]), \
-    [vo6] "v"(vo[6]), [vo7] "v"(vo[7]), [vo8] "v"(vo[8]), [vo9] "v"(vo[9]), [vo10] "v"(vo[10]),                 \
-    [vo11] "v"(vo[11]), [vo12] "v"(vo[12]), [vo13] "v"(vo[13]), [vo14] "v"(vo[14]), [vo15] "v"(vo[15]),         \
-    [vn0] "v"(vn[0]), [vn1] "v"(vn[1]), [vn2] "v"(vn[2]), [vn3] "v"(vn[3]), [vn4] "v"(vn[4]), [vn5] "v"(vn[5]), \
-    [vn6] "v"(vn[6]), [vn7] "v"(vn[7]), [vn8] "v"(vn[8]), [vn9] "v"(vn[9]), [vn10] "v"(vn[10]),                 \
-    [vn11] "v"(vn[11]), [vn12] "v"(vn[12]), [vn13] "v"(vn[13]), [vn14] "v"(vn[14]), [vn15] "v"(vn[15]),         \
-    [srdA] "s"(srdA), [srdB] "s"(srdB), [k0] "s"(k0), [k1] "s"(k1), [n0] "s"(kn0), [n1] "s"(kn1), [kend] "s"(kend), [first] "s"(s_first), [has_next] "s"(s_next)          \
-  : "memory", "scc", MLOP_W4_AGPR_CLOBBERS
-// the half-height loop: A fragments 0-3, DMA pieces 0-11 (accumulators a[0:127])
-#define MLOP_W4H_OPERANDS                                                                                        \
-  : [fa0_0] "=&v"(fa0_0), [fa0_1] "=&v"(fa0_1), [fa0_2] "=&v"(fa0_2), [fa0_3] "=&v"(fa0_3),                      \
-    [fb0_0] "=&v"(fb0_0), [fb0_1] "=&v"(fb0_1), [fb0_2] "=&v"(fb0_2), [fb0_3] "=&v"(fb0_3),                      \
-    [fb0_4] "=&v"(fb0_4), [fb0_5] "=&v"(fb0_5), [fb0_6] "=&v"(fb0_6), [fb0_7] "=&v"(fb0_7),                      \
-    [fa1_0] "=&v"(fa1_0), [fa1_1] "=&v"(fa1_1), [fa1_2] "=&v"(fa1_2), [fa1_3] "=&v"(fa1_3),                      \
-    [fb1_0] "=&v"(fb1_0), [fb1_1] "=&v"(fb1_1), [fb1_2] "=&v"(fb1_2), [fb1_3] "=&v"(fb1_3),                      \
-    [fb1_4] "=&v"(fb1_4), [fb1_5] "=&v"(fb1_5), [fb1_6] "=&v"(fb1_6), [fb1_7] "=&v"(fb1_7),                      \
-    [rA0] "+v"(rA0), [rA1] "+v"(rA1), [rB0] "+v"(rB0), [rB1] "+v"(rB1), [koff] "+s"(koff), [dbase] "+s"(dbase), \
-    [iter] "+s"(iter), [m0save] "=&s"(m0save)                                                                    \
-  : [vo0] "v"(vo[0]), [vo1] "v"(vo[1]), [vo2] "v"(vo[2]), [vo3] "v"(vo[3]), [vo4] "v"(vo[4]), [vo5] "v"(vo[5]), \
-    [vo6] "v"(vo[6]), [vo7] "v"(vo[7]), [vo8] "v"(vo[8]), [vo9] "v"(vo[9]), [vo10] "v"(vo[10]),                 \
-    [vo11] "v"(vo[11]), [vn0] "v"(vn[0]), [vn1] "v"(vn[1]), [vn2] "v"(vn[2]), [vn3] "v"(vn[3]),                 \
-    [vn4] "v"(vn[4]), [vn5] "v"(vn[5]), [vn6] "v"(vn[6]), [vn7] "v"(vn[7]), [vn8] "v"(vn[8]), [vn9] "v"(vn[9]), \
-    [vn10] "v"(vn[10]), [vn11] "v"(vn[11]), [srdA] "s"(srdA), [srdB] "s"(srdB), [k0] "s"(k0), [k1] "s"(k1), [n0] "s"(kn0), [n1] "s"(kn1), [kend] "s"(kend),               \
-    [first] "s"(s_first), [has_next] "s"(s_next)                                                                 \
-  : "memory", "scc", MLOP_W4_AGPR_CLOBBERS
-// 160 rows: A fragments 0-4, DMA pieces 0-12
-#define MLOP_W4_160_OPERANDS                                                                                    \
-  : [fa0_0] "=&v"(fa0_0), [fa0_1] "=&v"(fa0_1), [fa0_2] "=&v"(fa0_2), [fa0_3] "=&v"(fa0_3),                     \
-    [fa0_4] "=&v"(fa0_4), [fb0_0] "=&v"(fb0_0), [fb0_1] "=&v"(fb0_1), [fb0_2] "=&v"(fb0_2),                     \
-    [fb0_3] "=&v"(fb0_3), [fb0_4] "=&v"(fb0_4), [fb0_5] "=&v"(fb0_5), [fb0_6] "=&v"(fb0_6),                     \
-    [fb0_7] "=&v"(fb0_7), [fa1_0] "=&v"(fa1_0), [fa1_1] "=&v"(fa1_1), [fa1_2] "=&v"(fa1_2),                     \
-    [fa1_3] "=&v"(fa1_3), [fa1_4] "=&v"(fa1_4), [fb1_0] "=&v"(fb1_0), [fb1_1] "=&v"(fb1_1),                     \
-    [fb1_2] "=&v"(fb1_2), [fb1_3] "=&v"(fb1_3), [fb1_4] "=&v"(fb1_4), [fb1_5] "=&v"(fb1_5),                     \
-    [fb1_6] "=&v"(fb1_6), [fb1_7] "=&v"(fb1_7), [rA0] "+v"(rA0), [rA1] "+v"(rA1), [rB0] "+v"(rB0),              \
-    [rB1] "+v"(rB1), [koff] "+s"(koff), [dbase] "+s"(dbase), [iter] "+s"(iter), [m0save] "=&s"(m0save)          \
-  : [vo0] "v"(vo[0]), [vo1] "v"(vo[1]), [vo2] "v"(vo[2]), [vo3] "v"(vo[3]), [vo4] "v"(vo[4]), [vo5] "v"(vo[5]), \
-    [vo6] "v"(vo[6]), [vo7] "v"(vo[7]), [vo8] "v"(vo[8]), [vo9] "v"(vo[9]), [vo10] "v"(vo[10]),                 \
-    [vo11] "v"(vo[11]), [vo12] "v"(vo[12]), [vn0] "v"(vn[0]), [vn1] "v"(vn[1]), [vn2] "v"(vn[2]),               \
-    [vn3] "v"(vn[3]), [vn4] "v"(vn[4]), [vn5] "v"(vn[5]), [vn6] "v"(vn[6]), [vn7] "v"(vn[7]), [vn8] "v"(vn[8]), \
-    [vn9] "v"(vn[9]), [vn10] "v"(vn[10]), [vn11] "v"(vn[11]), [vn12] "v"(vn[12]), [srdA] "s"(srdA),             \
-    [srdB] "s"(srdB), [k0] "s"(k0), [k1] "s"(k1), [n0] "s"(kn0), [n1] "s"(kn1), [kend] "s"(kend), [first] "s"(s_first), [has_next] "s"(s_next)                            \
-  : "memory", "scc", MLOP_W4_AGPR_CLOBBERS
-// 192 rows: A fragments 0-5, DMA pieces 0-13
-#define MLOP_W4_192_OPERANDS                                                                                    \
-  : [fa0_0] "=&v"(fa0_0), [fa0_1] "=&v"(fa0_1), [fa0_2] "=&v"(fa0_2), [fa0_3] "=&v"(fa0_3),                     \
-    [fa0_4] "=&v"(fa0_4), [fa0_5] "=&v"(fa0_5), [fb0_0] "=&v"(fb0_0), [fb0_1] "=&v"(fb0_1),                     \
-    [fb0_2] "=&v"(fb0_2), [fb0_3] "=&v"(fb0_3), [fb0_4] "=&v"(fb0_4), [fb0_5] "=&v"(fb0_5),                     \
-    [fb0_6] "=&v"(fb0_6), [fb0_7] "=&v"(fb0_7), [fa1_0] "=&v"(fa1_0), [fa1_1] "=&v"(fa1_1),                     \
-    [fa1_2] "=&v"(fa1_2), [fa1_3] "=&v"(fa1_3), [fa1_4] "=&v"(fa1_4), [fa1_5] "=&v"(fa1_5),                     \
-    [fb1_0] "=&v"(fb1_0), [fb1_1] "=&v"(fb1_1), [fb1_2] "=&v"(fb1_2), [fb1_3] "=&v"(fb1_3),                     \
-    [fb1_4] "=&v"(fb1_4), [fb1_5] "=&v"(fb1_5), [fb1_6] "=&v"(fb1_6), [fb1_7] "=&v"(fb1_7), [rA0] "+v"(rA0),    \
-    [rA1] "+v"(rA1), [rB0] "+v"(rB0), [rB1] "+v"(rB1), [koff] "+s"(koff), [dbase] "+s"(dbase),                  \
-    [iter] "+s"(iter), [m0save] "=&s"(m0save)                                                                   \
-  : [vo0] "v"(vo[0]), [vo1] "v"(vo[1]), [vo2] "v"(vo[2]), [vo3] "v"(vo[3]), [vo4] "v"(vo[4]), [vo5] "v"(vo[5]), \
-    [vo6] "v"(vo[6]), [vo7] "v"(vo[7]), [vo8] "v"(vo[8]), [vo9] "v"(vo[9]), [vo10] "v"(vo[10]),                 \
-    [vo11] "v"(vo[11]), [vo12] "v"(vo[12]), [vo13] "v"(vo[13]), [vn0] "v"(vn[0]), [vn1] "v"(vn[1]),             \
-    [vn2] "v"(vn[2]), [vn3] "v"(vn[3]), [vn4] "v"(vn[4]), [vn5] "v"(vn[5]), [vn6] "v"(vn[6]), [vn7] "v"(vn[7]), \
-    [vn8] "v"(vn[8]), [vn9] "v"(vn[9]), [vn10] "v"(vn[10]), [vn11] "v"(vn[11]), [vn12] "v"(vn[12]),             \
-    [vn13] "v"(vn[13]), [srdA] "s"(srdA), [srdB] "s"(srdB), [k0] "s"(k0), [k1] "s"(k1), [n0] "s"(kn0), [n1] "s"(kn1), [kend] "s"(kend), [first] "s"(s_first),             \
-    [has_next] "s"(s_next)                                                                                      \
-  : "memory", "scc", MLOP_W4_AGPR_CLOBBERS
     // one generated K-loop per count of VMEM ops between the prefetched K-tiles and the loop: the
     // previous epilogue's NS stores (+ the two row-sum DMAs of W4_RS, issued above)
     constexpr int NQ = NS + (RS || GROUPED ? 2 : 0);
     if constexpr (BMT == 256) {
       static_assert(NQ == 32 || NQ == 16 || NQ == 34 || NQ == 18, "one generated K-loop per VMEM count");
-      if constexpr (NQ == 32) asm volatile(MLOP_W4_KLOOP_S32_P0_ASM MLOP_W4_OPERANDS);
-      else if constexpr (NQ == 16) asm volatile(MLOP_W4_KLOOP_S16_P0_ASM MLOP_W4_OPERANDS);
-      else if constexpr (NQ == 34) asm volatile(MLOP_W4_KLOOP_S34_P0_ASM MLOP_W4_OPERANDS);
-      else asm volatile(MLOP_W4_KLOOP_S18_P0_ASM MLOP_W4_OPERANDS);
+      if constexpr (NQ == 32) asm volatile(MLOP_W4_KLOOP_S32_P0_ASM MLOP_W4_256_OPERANDS);
+      else if constexpr (NQ == 16) asm volatile(MLOP_W4_KLOOP_S16_P0_ASM MLOP_W4_256_OPERANDS);
+      else if constexpr (NQ == 34) asm volatile(MLOP_W4_KLOOP_S34_P0_ASM MLOP_W4_256_OPERANDS);
+      else asm volatile(MLOP_W4_KLOOP_S18_P0_ASM MLOP_W4_256_OPERANDS);
+    } else if constexpr (BMT == 224) {
+      static_assert(NQ == 28 || NQ == 14 || NQ == 30 || NQ == 16, "one generated K-loop per VMEM count");
+      if constexpr (NQ == 28) asm volatile(MLOP_W4_224_KLOOP_S28_ASM MLOP_W4_224_OPERANDS);
+      else if constexpr (NQ == 14) asm volatile(MLOP_W4_224_KLOOP_S14_ASM MLOP_W4_224_OPERANDS);
+      else if constexpr (NQ == 30) asm volatile(MLOP_W4_224_KLOOP_S30_ASM MLOP_W4_224_OPERANDS);
+      else asm volatile(MLOP_W4_224_KLOOP_S16_ASM MLOP_W4_224_OPERANDS);
     } else if constexpr (BMT == 192) {
       static_assert(NQ == 24 || NQ == 12 || NQ == 26 || NQ == 14, "one generated K-loop per VMEM count");
       if constexpr (NQ == 24) asm volatile(MLOP_W4_192_KLOOP_S24_ASM MLOP_W4_192_OPERANDS);
@@ -403,15 +338,11 @@ __device__ __forceinline__ void gemm_w4_tiles(
       else asm volatile(MLOP_W4_160_KLOOP_S12_ASM MLOP_W4_160_OPERANDS);
     } else {
       static_assert(NQ == 16 || NQ == 8 || NQ == 18 || NQ == 10, "one generated K-loop per VMEM count");
-      if constexpr (NQ == 16) asm volatile(MLOP_W4H_KLOOP_S16_ASM MLOP_W4H_OPERANDS);
-      else if constexpr (NQ == 8) asm volatile(MLOP_W4H_KLOOP_S8_ASM MLOP_W4H_OPERANDS);
-      else if constexpr (NQ == 18) asm volatile(MLOP_W4H_KLOOP_S18_ASM MLOP_W4H_OPERANDS);
-      else asm volatile(MLOP_W4H_KLOOP_S10_ASM MLOP_W4H_OPERANDS);
+      if constexpr (NQ == 16) asm volatile(MLOP_W4H_KLOOP_S16_ASM MLOP_W4_128_OPERANDS);
+      else if constexpr (NQ == 8) asm volatile(MLOP_W4H_KLOOP_S8_ASM MLOP_W4_128_OPERANDS);
+      else if constexpr (NQ == 18) asm volatile(MLOP_W4H_KLOOP_S18_ASM MLOP_W4_128_OPERANDS);
+      else asm volatile(MLOP_W4H_KLOOP_S10_ASM MLOP_W4_128_OPERANDS);
     }
-#undef MLOP_W4_OPERANDS
-#undef MLOP_W4H_OPERANDS
-#undef MLOP_W4_160_OPERANDS
-#undef MLOP_W4_192_OPERANDS
 
     // read-out: the K-loop accumulates C^T, so acc(i, j)[r] of lane l is
     //   C[m0 + wm*BMT/2 + 16i + (l & 15)][n0 + wn*128 + 16j + 4(l >> 4) + r]
@@ -768,10 +699,11 @@ __global__ void __launch_bounds__(256, 1) gemm_w4_kernel(
 
 // The experts' products of a prompt.  What the grid loses is rows of partial tiles and the last round, and both hang on
 // the routing, which only the device knows: the height is chosen here, by estimated time in rounds of 256-row tiles (a
-// round of the lower ones .79 / .69, K-halves .59; W: the weights' rounds at one tile per expert, which bound the lower
+// round of the lower ones .89 / .79 / .69, K-halves .59; W: the weights' rounds at one tile per expert, which bound the lower
 // tiles).  gate_up of 8 experts, 256 / 192 / 160 rows: 300 rows each 738 / 619 / 532 us, 350 747 / 595 / 691, 500 779 /
 // 836 / 911, 550 1021 / 836 / 941, 1024 1497 / 1561 / 1598 (1.29 PFLOP/s); over 22 sizes, even and with the experts
-// 0.6 - 1.4 of the mean, the choice is within 1 % of the best of the three on average.  One XCD's workgroups share
+// 0.6 - 1.4 of the mean, the choice is within 1 % of the best of these three on average.  With 224 rows 407 each take 663
+// us where the ping-pong kernel took 735 and the three heights 714 - 745.  One XCD's workgroups share
 // panels and stay in step; each XCD's K walk starts at another eighth, and nothing is loaded between tiles that the
 // stores and the next tile's DMAs would be waited for with (offsets in LDS, gathered rows two tiles ahead): 1661 / 1577
 // / 1501 us before at 1024 rows, 800 before and 745 after at 450.
@@ -783,7 +715,7 @@ __global__ void __launch_bounds__(256, 1) gemm_w4_grouped_kernel(
   const int lane = threadIdx.x & 63, G = gridDim.x, nk = K / 64;
   const int rows = lane < n_groups ? offsets[lane + 1] - offsets[lane] : 0;
   // (16 bits each: M K < 2^30 and K >= 192 keep every count below 2^16)
-  uint32_t a = (uint32_t)((rows + 255) / 256) | (uint32_t)((rows + 191) / 192) << 16, b = (uint32_t)((rows + 159) / 160);
+  uint32_t a = (uint32_t)((rows + 255) / 256) | (uint32_t)((rows + 191) / 192) << 16, b = (uint32_t)((rows + 159) / 160) | (uint32_t)((rows + 223) / 224) << 16;
 #pragma unroll
   for (int d = 1; d < 64; d <<= 1) {
     a += __shfl_xor(a, d);
@@ -796,11 +728,14 @@ __global__ void __launch_bounds__(256, 1) gemm_w4_grouped_kernel(
     return (float)(T / G) + (r == 0 ? 0.f : 2 * r <= G && nk % 2 == 0 && ws != nullptr ? .59f : 1.f);
   };
   const float W = (float)(__popcll(__ballot(rows > 0)) * n_tiles_x) / (float)G;
-  const float t256 = rounds(a & 0xffff), t192 = fmaxf(.79f * rounds(a >> 16), .88f * W), t160 = fmaxf(.69f * rounds(b), .81f * W);
-  const int h = __builtin_amdgcn_readfirstlane(t256 <= t192 && t256 <= t160 ? 256 : t192 <= t160 ? 192 : 160);
+  const float t256 = rounds(a & 0xffff), t224 = fmaxf(.89f * rounds(b >> 16), .94f * W);
+  const float t192 = fmaxf(.79f * rounds(a >> 16), .88f * W), t160 = fmaxf(.69f * rounds(b & 0xffff), .81f * W);
+  const float upper = fminf(t256, t224), lower = fminf(t192, t160);
+  const int h = __builtin_amdgcn_readfirstlane(upper <= lower ? (t256 <= t224 ? 256 : 224) : t192 <= t160 ? 192 : 160);
 #define MLOP_W4_GROUPED(h_)                                                                                           \
   gemm_w4_tiles<EPI, h_, true>(A, lda, B, ldb, C, ldc, M, N, K, n_tiles_x, 0, 1, re, 0, 0, ws, cnt, offsets, n_groups)
   if (h == 256) MLOP_W4_GROUPED(256);
+  else if (h == 224) MLOP_W4_GROUPED(224);
   else if (h == 192) MLOP_W4_GROUPED(192);
   else MLOP_W4_GROUPED(160);
 #undef MLOP_W4_GROUPED
@@ -921,6 +856,7 @@ bool run_w4(int epi, const uint16_t* A, int lda, const uint16_t* B, int ldb, uin
             int K, hipStream_t st, const RopeEpi& re, int bm) {
   if (bm == 128) return run_w4_h<128>(epi, A, lda, B, ldb, C, ldc, M, N, K, st, re);
   if (bm == 160) return run_w4_h<160>(epi, A, lda, B, ldb, C, ldc, M, N, K, st, re);
+  if (bm == 224) return run_w4_h<224>(epi, A, lda, B, ldb, C, ldc, M, N, K, st, re);
   if (bm == 192) return run_w4_h<192>(epi, A, lda, B, ldb, C, ldc, M, N, K, st, re);
   if (bm == 256) return run_w4_h<256>(epi, A, lda, B, ldb, C, ldc, M, N, K, st, re);
   return false;

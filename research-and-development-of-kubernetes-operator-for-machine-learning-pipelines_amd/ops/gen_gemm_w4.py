@@ -27,8 +27,8 @@ Schedule of iteration t (MFMA slot m = 0..127; H0 = k-half 0 of tile t, H1 = k-h
   m 40..100  16 LDS-DMA pieces of tile t+2 into buffer t&1 (one per 4 MFMAs)
   m  102     vmcnt(16) + s_barrier (B2): tile t+1 (issued one iteration ago) has landed
   m 103..127 ds_read k-half-0 fragments of tile t+1 (FB0, FA0) from buffer (t+1)&1
-Lower tiles (128, 160, 192 rows: 64, 80, 96 MFMAs per K-tile, 12 - 14 pieces and 12 - 14 reads per half) have the same
-phases at their own slots (SCHED_H, SCHED_160, SCHED_192).  The K offset of the DMA runs through an operand: it starts
+Lower tiles (128, 160, 192, 224 rows: 64, 80, 96, 112 MFMAs per K-tile, 12 - 15 pieces and 12 - 15 reads per half) have the
+same phases at their own slots (SCHED_H, SCHED_160, SCHED_192, SCHED_224).  The K offset of the DMA runs through an operand: it starts
 where the caller says and wraps to 0 at %[kend], so that tiles may walk K from different steps.
 MFMA order: H0 = (i, j) row-major over FA0[i] x FB0[j]; H1 = the same over FA1 x FB1.
 lgkmcnt waits are derived here from the in-order LDS return queue (each MFMA waits only
@@ -94,6 +94,8 @@ SCHED_160 = Sched(rd1=[1 + k for k in range(13)], b1=22, dma=[23 + round(2.5 * k
                   rd0=[58 + round(k * 15 / 12) for k in range(13)], toggle1=21, bm=160)
 SCHED_192 = Sched(rd1=[1 + round(k * 16 / 13) for k in range(14)], b1=26, dma=[27 + 3 * k for k in range(14)], b2=70,
                   rd0=[71 + round(k * 18 / 13) for k in range(14)], toggle1=22, bm=192)
+SCHED_224 = Sched(rd1=[1 + round(k * 24 / 14) for k in range(15)], b1=32, dma=[34 + round(3.5 * k) for k in range(15)], b2=86,
+                  rd0=[87 + round(k * 22 / 14) for k in range(15)], toggle1=28, bm=224)
 
 
 def frag(name, i):
@@ -277,6 +279,22 @@ def readout(i: int) -> list[str]:
     return [f"v_accvgpr_read_b32 %{k}, a{32 * i + k}" for k in range(32)]
 
 
+def operands(sc: Sched) -> list[str]:
+    """Operand and clobber lists of a height's K-loop statements: fragments and address registers out, the DMA offsets of
+    this tile and the next in."""
+    frags = [f"fa{h}_{i}" for h in (0, 1) for i in range(sc.nfa)] + [f"fb{h}_{j}" for h in (0, 1) for j in range(NFB)]
+    outs = ([f'[{f}] "=&v"({f})' for f in frags] + [f'[{r}] "+v"({r})' for r in ("rA0", "rA1", "rB0", "rB1")]
+            + [f'[{r}] "+s"({r})' for r in ("koff", "dbase", "iter")] + ['[m0save] "=&s"(m0save)'])
+    ins = ([f'[{v}{k}] "v"({v}[{k}])' for v in ("vo", "vn") for k in range(sc.npc)]
+           + [f'[{n}] "s"({v})' for n, v in (("srdA", "srdA"), ("srdB", "srdB"), ("k0", "k0"), ("k1", "k1"), ("n0", "kn0"),
+                                             ("n1", "kn1"), ("kend", "kend"), ("first", "s_first"), ("has_next", "s_next"))])
+    rows = []
+    for sep, ops in ((":", outs), (":", ins)):
+        for k in range(0, len(ops), 6):
+            rows.append(("  " + sep if k == 0 else "    ") + " " + ", ".join(ops[k:k + 6]) + ("," if k + 6 < len(ops) else ""))
+    return rows + ['  : "memory", "scc", MLOP_W4_AGPR_CLOBBERS']
+
+
 def render() -> str:
     out = ["// GENERATED by mlopamd/ops/gen_gemm_w4.py -- do not edit by hand.",
            "// The K-loop of gemm_w4_kernel (csrc/gemm_w4.hip): see the generator's docstring.",
@@ -299,7 +317,7 @@ def render() -> str:
         out.append('  ""')
         out.append("")
     # the heights between: 4 stores per 16-row block and wave (SiLU-mul 2), the same four counts
-    for sc in (SCHED_160, SCHED_192):
+    for sc in (SCHED_160, SCHED_192, SCHED_224):
         for ns in (4 * sc.nfa, 2 * sc.nfa, 4 * sc.nfa + 2, 2 * sc.nfa + 2):
             out.append(f"#define MLOP_W4_{sc.bm}_KLOOP_S{ns}_ASM \\")
             for ln in kloop(ns, sc):
@@ -312,6 +330,10 @@ def render() -> str:
             out.append(f'  "{ln}\\n" \\')
         out.append('  ""')
         out.append("")
+    for sc in (SCHED_H, SCHED_160, SCHED_192, SCHED_224, *SCHEDS):
+        out.append(f"#define MLOP_W4_{sc.bm}_OPERANDS \\")
+        rows = operands(sc)
+        out += [f"{ln} \\" for ln in rows[:-1]] + [rows[-1], ""]
     clob = ", ".join(f'"a{r}"' for r in range(256))
     out.append(f"#define MLOP_W4_AGPR_CLOBBERS {clob}")
     out.append("")

@@ -10,7 +10,7 @@ pytestmark = pytest.mark.gpu
 bf = torch.bfloat16
 
 
-@pytest.fixture(params=[160, 192])
+@pytest.fixture(params=[160, 192, 224])
 def height(gpu, request):
     ops._sk_reserve(torch.device(gpu))
     torch.ops.mlop.gemm_dense_plan(6, request.param, 256, -1)
@@ -96,7 +96,7 @@ def test_norm_chain(gpu, height, M):
 
 
 # a tile with rows past M, then another on the same workgroup, at short K (the next tile's first K-tile is in flight)
-@pytest.mark.parametrize("variant,bm", [(6, 128), (6, 160), (6, 192), (5, 256)])
+@pytest.mark.parametrize("variant,bm", [(6, 128), (6, 160), (6, 192), (6, 224), (5, 256)])
 @pytest.mark.parametrize("tiles,off", [(1, 1), (2, 17), (5, 3)])
 @pytest.mark.parametrize("K", [192, 448])
 def test_tile_after_a_partial_one(gpu, variant, bm, tiles, off, K):
