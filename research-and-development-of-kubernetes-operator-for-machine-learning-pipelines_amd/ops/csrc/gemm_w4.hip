@@ -236,10 +236,10 @@ __device__ __forceinline__ void gemm_w4_tiles(
     uint32_t vo[NPC], vn[NPC];
     dma_offsets(m0, n0, m_end, b0, kb, rows_lds + slot_i * 64, vo);
     const bool next = it + G < n_items;
-    // the K walk starts at another eighth per XCD (GROUPED): tiles in step would otherwise all read the columns of the
+    // the K walk starts at another eighth per XCD (w4_k_walk): tiles in step would otherwise all read the columns of the
     // same few memory channels
     auto k_at = [&](int len, int j) {
-      const int k = (GROUPED ? xcd * len / 8 : 0) + j;
+      const int k = ((re.k_walk * xcd) & 7) * len / 8 + j;
       return (uint32_t)__builtin_amdgcn_readfirstlane((k >= len ? k - len : k) * 128);
     };
     const uint32_t k0 = k_at(nkl, 0), k1 = k_at(nkl, 1), kend = __builtin_amdgcn_readfirstlane(nkl * 128);
@@ -755,6 +755,18 @@ bool gemm_w4_ok(int M, int N, int K, int lda, int ldb, int ldc) {
          (long)M * lda * 2 < (1l << 31) && (long)N * ldb * 2 < (1l << 31) && (long)M * (ldc > 0 ? ldc : N) * 2 < (1l << 31);
 }
 
+// Each XCD's K walk from another eighth on (XCD x from eighth k_walk x mod 8; 0: all in step): where rows are a multiple of 4 KB apart, tiles in step ask for the same few
+// memory channels.  Not where XCDs share weights (several bands of tiles a round) that the 256 MB cache behind the L2s
+// does not hold: out of step each of them reads HBM.  Cold weights, M 1024 - 6000 (us): 16384 x 16384 1150 -> 1114 at 3000 rows,
+// 8192 x 14336 325 -> 317 at 2048, 8192 x 8192 179 -> 176, 28672 x 4096 640 -> 630 at 4096; without the first condition 5120 x
+// 13824 is 1.5 % slower at 1024 - 3000 rows and 2.5 % faster above, without the second 8192 x 28672 4 % slower, 8192 x
+// 20480 3 %.  In a step (Llama-3-8B widths) o and down together 105 -> 99 us each at 1500 rows, 415 -> 402 at 8000.
+// Neighbours five eighths apart: 0.5 - 1.5 % of a step better than one apart at 1500 rows and in mixed steps, level elsewhere; the
+// experts' products (one apart) gain 1 - 3 % so at 1500 - 1800 tokens and lose 1.4 % at 4500, and stay.
+static int w4_k_walk(int N, int K, int band_tiles, int cus) {
+  return K % 2048 == 0 && ((long)N * K * 2 <= (256l << 20) || band_tiles >= cus) ? 5 : 0;
+}
+
 template <int EPI, int BMT>
 static bool run_w4_t(const uint16_t* A, int lda, const uint16_t* B, int ldb, uint16_t* C, int ldc, int M, int N,
                      int K, hipStream_t st, const RopeEpi& re) {
@@ -798,6 +810,7 @@ static bool run_w4_t(const uint16_t* A, int lda, const uint16_t* B, int ldb, uin
   grid = std::min(grid, cus);
   RopeEpi re2 = re;
   re2.ws_nt = gemm_slab_nt(-1);
+  re2.k_walk = w4_k_walk(N, K, gm * gx, cus);
   if constexpr ((EPI & W4_ADD_SS) != 0) {  // one band ticket per BMT-row band (launch_w4_chain checks gy)
     float* w2 = nullptr;
     int c3 = 0;
@@ -827,6 +840,7 @@ static void run_w4_grouped_t(const uint16_t* A, int lda, const uint16_t* B, int 
   const long most = (long)(N / 256) * ((M + 159) / 160 + n_groups);  // every expert's last tile partial
   RopeEpi re2 = re;
   re2.ws_nt = gemm_slab_nt(-1);
+  re2.k_walk = 1;  // (an expert's column tiles are walked by one XCD)
   kern<<<(int)std::min<long>(most, cus), 256, lds, st>>>(A, lda, B, ldb, C, ldc, M, N, K, N / 256, re2, ws, cnt, offsets,
                                                           n_groups);
 }

@@ -78,6 +78,8 @@ struct RopeEpi {
   // gemm_kernel: split-K slabs stored non-temporal (not left dirty in L2 for the kernel boundary's
   // write-back; MI355X_MICROARCH.md "boundary"); set by run_cfg (gemm_slab_nt)
   int ws_nt = 0;
+  // four-wave kernel: XCD x walks K from eighth k_walk x mod 8 (gemm_w4.hip w4_k_walk)
+  int k_walk = 0;
   // mid norm chain (gemm.hip mid_chain_finish): 1 = the finishing split reads the partials with
   // plain loads behind one agent acquire, 0 = with sc1 loads only (gemm_mid_chain op 2 / 1)
   int mid_acq = 0;

@@ -44,6 +44,21 @@ def test_tiles(gpu, height, tiles, off, N, K, epi):
     assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
 
 
+# K a multiple of 2048 and not, halves of it, several bands of tiles; weights that the cache behind the L2s holds and not
+@pytest.mark.parametrize("M,N,K", [(130, 512, 2048), (130, 512, 2112), (700, 4096, 2048), (1300, 6144, 4096), (257, 16384, 10240),
+                                   (1000, 8192, 18432)])
+def test_k_walk(gpu, height, M, N, K):
+    """XCDs start at different eighths of K: the same sums in another order, and the same ones every time."""
+    torch.manual_seed(M + K)
+    x = torch.randn(M, K, device=gpu, dtype=bf)
+    w = (0.05 * torch.randn(N, K, device=gpu)).to(bf)
+    outs = [ops.gemm(x, w) for _ in range(3)]
+    y = x.float() @ w.float().t()
+    bound = 2.0 ** -8 * y.abs() + 2 * 2.0 ** -20 * (x.float().abs() @ w.float().abs().t())
+    assert ((outs[0].float() - y).abs() <= bound + 1e-6).all()
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+
+
 @pytest.mark.parametrize("M", [300, 1500])
 def test_rope(gpu, height, M):
     from mlopamd.models.layers import rope_table
