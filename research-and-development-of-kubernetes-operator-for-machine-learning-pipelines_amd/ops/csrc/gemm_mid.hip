@@ -5,16 +5,13 @@
 // What bounds it: reading B once (every weight byte from HBM, ~6.5 TB/s at best); A is small and comes
 // from L2, once per workgroup.  The LDS-ring tiles of gemm.hip keep one ring for both operands: at 128
 // rows two thirds of what is in flight is A, and the loop waits out the HBM latency of the rest.  Here
-//   * the operands have rings of their own: half of the waves load A two or three K-steps ahead (L2), the
+//   * the operands have rings of their own: half of the waves load A two to five K-steps ahead (L2), the
 //     other half load B as many steps ahead as the 160 KB of LDS hold.  vmcnt retires in order, so one
 //     wave cannot run two depths;
 //   * column tile bx starts its walk of K at step bx % nk and wraps around.  Weight rows are a multiple of
 //     4 KB apart: tiles that walk K in step ask for the same offset of every row, that is for the same
 //     few memory channels (B alone, gate_up of Llama-3-8B: 43.8 -> 36.8 us);
-//   * the next K-step's first half of fragments is read while this one's second half multiplies.  The
-//     second half's reads stand before the first half's MFMAs as well, but the compiler waits for all LDS
-//     reads in between (lgkmcnt(0): the epilogue's scalar loads share the counter), so half of the LDS
-//     reads (three quarters of a step's time) overlap MFMAs inside a wave, the other half only across waves;
+//   * the next half K-step's fragments are read while this half multiplies (kBehind below);
 //   * a workgroup walks its tiles without draining the rings: the next tile's first K-steps load under
 //     this one's last (lm_head: four tiles per workgroup).
 // Tiles are 256 columns where such tiles fill the chip (A is read half as often), else 128; rows are the
@@ -58,6 +55,12 @@ __global__ void __launch_bounds__(WM * WN * 64) gemm_mid_kernel(
     float* __restrict__ ws, int M, int N, int K, int k_chunk, int m_tiles, int n_splits, int n_tasks, RopeEpi re) {
   constexpr int NW = WM * WN, HW = NW / 2;   // half of the waves issue A, half B
   constexpr int WTM = BM / WM, WTN = BN / WN, TM = WTM / 16, TN = WTN / 16;
+  // Each half's reads stand behind the first MFMA of the half before: the compiler waits for every LDS read in flight before
+  // a fragment's first use, so reads that stand before it overlap with nothing.  Not for 64 rows, where two workgroups
+  // share a CU and overlap each other, and 256 x 256, which would spill.  (Cold weights, us, reads before -> behind with the
+  // rings as deep for A as for B: gate_up 28672 x 4096 at 100 / 150 / 192 rows 50 -> 47, 56 -> 51.5, 62 -> 59, down of
+  // Llama-3-70B 8192 x 28672 at 150 / 300 107 -> 100, 191 -> 182, its gate_up at 100 / 224 153 -> 148, 220 -> 213.)
+  constexpr bool kBehind = BM > 64 && BM + BN < 512;
   constexpr int PA = BM / 8 / HW, PB = BN / 8 / HW;  // 1-KiB pieces per issuing wave and K-step
   static_assert(BM % (8 * HW) == 0 && BN % (8 * HW) == 0 && WTM % 16 == 0 && WTN % 16 == 0, "tile");
   static_assert((SA - 1) * PA < 64 && (SB - 1) * PB < 64, "vmcnt");
@@ -117,11 +120,19 @@ __global__ void __launch_bounds__(WM * WN * 64) gemm_mid_kernel(
     if (is_b) {
       uint16_t* base = ringB + i_buf * (BN * 64);
       i_buf = i_buf == SB - 1 ? 0 : i_buf + 1;
+#define MLOP_LOAD_B(aux) \
+  __builtin_amdgcn_global_load_lds((const void*)(src[i] + k), (lds_void_t*)(base + (iw + HW * i) * 512), 16, 0, aux)
+      if (kBehind && nt) {
 #pragma unroll
-      for (int i = 0; i < PB; ++i) {
-        if (nt) __builtin_amdgcn_global_load_lds((const void*)(src[i] + k), (lds_void_t*)(base + (iw + HW * i) * 512), 16, 0, 2);
-        else __builtin_amdgcn_global_load_lds((const void*)(src[i] + k), (lds_void_t*)(base + (iw + HW * i) * 512), 16, 0, 0);
+        for (int i = 0; i < PB; ++i) MLOP_LOAD_B(2);
+      } else {
+#pragma unroll
+        for (int i = 0; i < PB; ++i) {  // (64 rows: a branch per load is 1 - 3 % faster than one for all, above that 1 - 4 % slower)
+          if (!kBehind && nt) MLOP_LOAD_B(2);
+          else MLOP_LOAD_B(0);
+        }
       }
+#undef MLOP_LOAD_B
     } else {
       uint16_t* base = ringA + i_buf * (BM * 64);
       i_buf = i_buf == SA - 1 ? 0 : i_buf + 1;
@@ -156,12 +167,21 @@ __global__ void __launch_bounds__(WM * WN * 64) gemm_mid_kernel(
 #pragma unroll
     for (int i = 0; i < TM; ++i) fa[kk][i] = *reinterpret_cast<const bf16x8*>(sA + i * 1024);
   };
-  auto multiply = [&](auto kk_) {
+  auto multiply = [&](auto kk_, auto&& behind) {
     constexpr int kk = decltype(kk_)::value;
+    acc[0][0] = mfma16(fb[kk][0], fa[kk][0], acc[0][0]);
+    behind();
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
-      for (int j = 0; j < TN; ++j) acc[i][j] = mfma16(fb[kk][j], fa[kk][i], acc[i][j]);
+      for (int j = i == 0; j < TN; ++j) acc[i][j] = mfma16(fb[kk][j], fa[kk][i], acc[i][j]);
+  };
+  auto read_behind = [&](auto kk_, bool more) {
+    if constexpr (kBehind) {
+      __builtin_amdgcn_sched_barrier(0);
+      if (more) read(kk_);
+      __builtin_amdgcn_sched_barrier(0);
+    }
   };
   using H0 = std::integral_constant<int, 0>;
   using H1 = std::integral_constant<int, 1>;
@@ -222,19 +242,25 @@ __global__ void __launch_bounds__(WM * WN * 64) gemm_mid_kernel(
   raw_barrier();
   read(H0{});
   for (int s = 0; s < total; ++s) {
-    read(H1{});
-    multiply(H0{});
+    if constexpr (!kBehind) read(H1{});
+    multiply(H0{}, [&]() { read_behind(H1{}, true); });
     if (s + 1 < total) {
-      if (is_b) wait_stages<SB - 2, PB>(total - 2 - s);
-      else wait_stages<SA - 2, PA>(total - 2 - s);
+      if (s + (SA > SB ? SA : SB) <= total) {
+        if (is_b) wait_vmcnt<(SB - 2) * PB>();
+        else wait_vmcnt<(SA - 2) * PA>();
+      } else if (is_b) {
+        wait_stages<SB - 2, PB>(total - 2 - s);
+      } else {
+        wait_stages<SA - 2, PA>(total - 2 - s);
+      }
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this wave has step s in registers
       raw_barrier();                                      // step s + 1 landed; step s's buffers are free
       issue();
       rbufA = rbufA == SA - 1 ? 0 : rbufA + 1;
       rbufB = rbufB == SB - 1 ? 0 : rbufB + 1;
-      read(H0{});
+      if constexpr (!kBehind) read(H0{});
     }
-    multiply(H1{});
+    multiply(H1{}, [&]() { read_behind(H0{}, s + 1 < total); });
     if (++c_kt == c_nk) {
       epilogue();
 #pragma unroll
@@ -274,14 +300,16 @@ void launch_mid(int epi, int bm, int bn, const uint16_t* A, int lda, const uint1
     if (epi == 0) return run_mid<m, n, wm, wn, sa, sb, 0>(A, lda, B, ldb, C, ldc, ws, M, N, K, splits, k_chunk, st, re); \
     return run_mid<m, n, wm, wn, sa, sb, 1>(A, lda, B, ldb, C, ldc, ws, M, N, K, splits, k_chunk, st, re);               \
   }
-  // ring depths: what fits 160 KB, B before A (64 x 128: half of it, two workgroups per CU)
+  // ring depths: what fits 160 KB (64 x 128: half of it, two workgroups per CU).  With 128 columns as deep for A as for B: with
+  // A two or three deep and the rest for B 0 - 4 % slower (qkv, gate_up and down at 100 - 160 rows; 8192 x 28672 at 112 - 128 rows 2 %
+  // faster); not 224 rows, where it made no difference.
   MLOP_MID(64, 128, 2, 4, 2, 4)
-  MLOP_MID(96, 128, 2, 4, 3, 7)
-  MLOP_MID(128, 128, 2, 4, 3, 7)
-  MLOP_MID(160, 128, 2, 4, 3, 6)
-  MLOP_MID(192, 128, 2, 4, 3, 5)
+  MLOP_MID(96, 128, 2, 4, 5, 6)
+  MLOP_MID(128, 128, 2, 4, 5, 5)
+  MLOP_MID(160, 128, 2, 4, 4, 5)
+  MLOP_MID(192, 128, 2, 4, 4, 4)
   MLOP_MID(224, 128, 2, 4, 2, 6)
-  MLOP_MID(256, 128, 4, 2, 2, 6)
+  MLOP_MID(256, 128, 4, 2, 3, 4)
   MLOP_MID(64, 256, 2, 4, 3, 4)
   MLOP_MID(96, 256, 2, 4, 2, 4)
   MLOP_MID(128, 256, 2, 4, 3, 3)
