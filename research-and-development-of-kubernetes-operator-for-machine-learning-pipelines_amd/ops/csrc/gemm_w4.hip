@@ -761,8 +761,7 @@ bool gemm_w4_ok(int M, int N, int K, int lda, int ldb, int ldc) {
 // 8192 x 14336 325 -> 317 at 2048, 8192 x 8192 179 -> 176, 28672 x 4096 640 -> 630 at 4096; without the first condition 5120 x
 // 13824 is 1.5 % slower at 1024 - 3000 rows and 2.5 % faster above, without the second 8192 x 28672 4 % slower, 8192 x
 // 20480 3 %.  In a step (Llama-3-8B widths) o and down together 105 -> 99 us each at 1500 rows, 415 -> 402 at 8000.
-// Neighbours five eighths apart: 0.5 - 1.5 % of a step better than one apart at 1500 rows and in mixed steps, level elsewhere; the
-// experts' products (one apart) gain 1 - 3 % so at 1500 - 1800 tokens and lose 1.4 % at 4500, and stay.
+// Neighbours five eighths apart: 0.5 - 1.5 % of a step better than one apart at 1500 rows and in mixed steps, level elsewhere.
 static int w4_k_walk(int N, int K, int band_tiles, int cus) {
   return K % 2048 == 0 && ((long)N * K * 2 <= (256l << 20) || band_tiles >= cus) ? 5 : 0;
 }
@@ -840,7 +839,10 @@ static void run_w4_grouped_t(const uint16_t* A, int lda, const uint16_t* B, int 
   const long most = (long)(N / 256) * ((M + 159) / 160 + n_groups);  // every expert's last tile partial
   RopeEpi re2 = re;
   re2.ws_nt = gemm_slab_nt(-1);
-  re2.k_walk = 1;  // (an expert's column tiles are walked by one XCD)
+  // (an expert's column tiles are walked by one XCD: no condition as in w4_k_walk.  Steps of three Mixtral layers, neighbours
+  // five eighths apart for one: 1500 / 1800 tokens, 375 / 450 rows per expert, 3761 -> 3674, 4144 -> 4076 us, two prompts of 900
+  // 3769 -> 3690; level at 525 rows, at 900 - 1500 7576 -> 7624, 12059 -> 12156)
+  re2.k_walk = M <= 512l * n_groups ? 5 : 1;
   kern<<<(int)std::min<long>(most, cus), 256, lds, st>>>(A, lda, B, ldb, C, ldc, M, N, K, N / 256, re2, ws, cnt, offsets,
                                                           n_groups);
 }
