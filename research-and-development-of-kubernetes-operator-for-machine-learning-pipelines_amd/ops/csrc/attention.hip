@@ -184,7 +184,7 @@ __global__ void __launch_bounds__(256, 3) paged_attn_kernel(
     const int* __restrict__ tile_seq, const int* __restrict__ tile_q0,
     const int* __restrict__ q_start, const int* __restrict__ q_len,
     const int* __restrict__ ctx_len, int Hq, int Hkv, float scale_log2, int part_tokens,
-    int nparts, int even, int num_blocks, int* __restrict__ sem) {
+    int nparts, int even, int num_blocks, int tiles, int* __restrict__ sem) {
   constexpr int QT = 16 / G;
   // (3 waves per SIMD: 154 VGPRs; asked for two fewer the compiler keeps O in AGPRs and copies it for every rescale)
   // wave w stages its page pair's V image (2 x 16 token rows x 256 B = 8 KB) inside sm_o[w]
@@ -195,17 +195,20 @@ __global__ void __launch_bounds__(256, 3) paged_attn_kernel(
   __shared__ float sm_l[4][16];
   __shared__ int sm_last;
 
-  // kv heads fastest: a page holds the heads' 4-KB blocks one behind the other, and whatever workgroups run at a time read
-  // them all.  Tiles fastest, a launch ended on two heads, a quarter of every page (a step of 200 x 1500 keys 2562 ->
-  // 2507 us, 700 x 500 4119 -> 4084, 64 x 4000 1963 -> 1923, 100 x 1000 and fewer as before).
-  const int lin = blockIdx.x + gridDim.x * blockIdx.y, tile = lin / Hkv, kvh = lin % Hkv, part = blockIdx.z;
+  // From 32 tiles on the kv heads are the fastest index: a page holds the heads' 4-KB blocks one behind the other, and whatever
+  // workgroups run at a time read them all.  With tiles fastest a launch ended on two heads, a quarter of every page (a
+  // step of 40 x 8000 keys 2620 -> 2518 us, 48 x 7000 2472 -> 2408, 200 x 1500 2562 -> 2507, 700 x 500 4119 -> 4084, 20 x 17500 2839 ->
+  // 2816, 100 x 1000 the same).  Few long sequences in shares lose a little: 8 x 20000 1388 -> 1400, 13 x 2056 937 -> 940.
+  const bool by_head = tiles >= 32;
+  const int lin = blockIdx.x + tiles * blockIdx.y, part = blockIdx.z;
+  const int tile = by_head ? lin / Hkv : blockIdx.x, kvh = by_head ? lin % Hkv : blockIdx.y;
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   const int s = tile_seq[tile], q0 = tile_q0[tile];
   const int* bt = block_tables + (size_t)s * bt_stride;
   const int ql = q_len[s], ctx = ctx_len[s], qs = q_start[s];
   const int last_q = min(q0 + QT, ql) - 1;           // last valid query of the tile
   const int kv_end = last_q >= 0 ? ctx - ql + last_q + 1 : 0;
-  part_tokens = seq_part(kv_end, part_tokens, nparts, even, tile_seq, ctx_len, gridDim.x, Hkv);
+  part_tokens = seq_part(kv_end, part_tokens, nparts, even, tile_seq, ctx_len, tiles, Hkv);
   const int p_begin = part * part_tokens;
   const int p_end = min(kv_end, p_begin + part_tokens);
   if (p_begin >= p_end) {                            // reducer skips empty partitions
@@ -527,7 +530,7 @@ static void launch_g(void* out, float* part_o, float* part_ml, const void* q, co
   auto kern = nt == 3 ? paged_attn_kernel<G, 3> : nt ? paged_attn_kernel<G, 1> : paged_attn_kernel<G, 0>;
   kern<<<grid, 256, 0, st>>>((uint16_t*)out, part_o, part_ml, (const uint16_t*)q, (const uint16_t*)kc,
                              (const uint16_t*)vc, bt, bt_stride, tile_seq, tile_q0, q_start, q_len, ctx_len,
-                             Hq, Hkv, scale_log2, part_tokens, nparts, even, num_blocks, sem);
+                             Hq, Hkv, scale_log2, part_tokens, nparts, even, num_blocks, num_tiles, sem);
   if (nparts > 1 && sem == nullptr) {
     attn_reduce_kernel<G><<<dim3(num_tiles, Hkv), 256, 0, st>>>(
         (uint16_t*)out, part_o, part_ml, tile_seq, tile_q0, q_start, q_len, ctx_len, Hq, Hkv,
