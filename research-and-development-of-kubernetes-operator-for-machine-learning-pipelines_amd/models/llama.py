@@ -241,9 +241,11 @@ class LlamaModel:
             return ops.rmsnorm(residual, self.final_norm, eps), None
         return None, ops.ss_init(residual, ss)
 
-    def logits_local(self, hidden: torch.Tensor) -> torch.Tensor:
-        """[n, H] -> this rank's vocab shard of the logits [n, V/TP] (model dtype)."""
-        return linear(hidden, self.lm_head)
+    def logits_local(self, hidden: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
+        """[n, H] -> this rank's vocab shard of the logits [n, V/TP] (model dtype), in ``out`` where given."""
+        return linear(hidden, self.lm_head, out)
+
+    logits_out = True  # logits_local takes ``out``
 
     def logits(self, hidden: torch.Tensor) -> torch.Tensor:
         """[n, H] -> full-vocab logits [n, V] in the model dtype (bf16 on GPU: the

@@ -203,8 +203,8 @@ def fill_buckets(listed) -> list[int]:
     1024, 300 take 2193 in 320 and 2634 in 512, 150 take 1431 in 160 and 1683 in 256, 90 take 1139 in 96
     and 1221 in 128, 40 take 982 in 48 and 1016 in 64; 20 take the same in 24 as in 32, so nothing is
     added there.  The weight stream's tiles grow by 32 rows (by 16 where the weights alone count), large
-    tiles fill by 64 or so.  A graph costs its warm-up and capture (1.5 ms for these 6 layers) and its own
-    rows of logits, which is why the steps widen above 1024.  Lists with wider gaps stay as they are."""
+    tiles fill by 64 or so.  A graph costs its warm-up and capture (1.5 ms for these 6 layers), which is
+    why the steps widen above 1024.  Lists with wider gaps stay as they are."""
     out = sorted(set(listed))
     for a, b in zip(out[:-1], out[1:]):
         if b > 2 * a:
@@ -1408,6 +1408,7 @@ class Engine:
         empty = np.zeros(0, dtype=np.int32)
         t0 = time.perf_counter()
         verbose = False
+        widest = None  # logits of the largest graph, captured first
         with torch.cuda.stream(stream):
             for bi, b in enumerate(sorted(self.buckets, reverse=True)):
                 self.meta.fill_decode(empty, empty, np.zeros(0, dtype=np.int64), pad_to=b)
@@ -1424,9 +1425,14 @@ class Engine:
                 if verbose:
                     print(f"[engine] capturing decode graph {bi + 1}/{len(self.buckets)} (batch {b}) "
                           f"at {time.perf_counter() - t0:.1f} s", file=sys.stderr, flush=True)
+                # one graph replays at a time and its logits are read before the next does: the smaller graphs write
+                # theirs into the largest one's buffer where the model can
+                shared = bi and getattr(m, "logits_out", False)
                 g = torch.cuda.CUDAGraph()
                 with torch.cuda.graph(g, pool=self.graph_pool, stream=stream):
-                    logits = m.logits_local(m.forward(ids, meta, self.kv))
+                    hidden = m.forward(ids, meta, self.kv)
+                    logits = m.logits_local(hidden, out=widest[:b]) if shared else m.logits_local(hidden)
+                widest = logits if bi == 0 else widest
                 self.graphs[b] = (g, logits)
         torch.cuda.current_stream(self.device).wait_stream(stream)
         torch.cuda.synchronize(self.device)
