@@ -162,7 +162,7 @@ class LlamaModel:
         M = ids.shape[0]
         # TP > 1: the decode (GEMV) form only, its residual adds riding in the all-reduces
         dmax = ops.decode_chain_max_m()  # the GEMV (<= 4 rows) / weight-streaming MFMA (<= 64) forms
-        chain = (tp.size == 1 or M <= dmax) and self._chain_ok(M)
+        chain = (tp.size == 1 or M <= dmax) and self._chain_ok(M, meta.like)
         ss = None  # norm chain: x is None and ss holds the residual's row partials
         if chain and M <= dmax:
             # decode form: the QKV GEMV takes the embedding rows' factors itself (ss unused)
@@ -175,14 +175,14 @@ class LlamaModel:
                                        self.n_q)
             else:
                 q = ops.qkv_rope_cache_rs(residual, L["qkv"], meta.positions, self.cos_sin, meta.slots, kv.k[i],
-                                          kv.v[i], self.n_q, ss, eps)
+                                          kv.v[i], self.n_q, ss, eps, meta.like > 0)
             a = ops.paged_attention(q, kv.k[i], kv.v[i], meta)
             nxt = self.layers[i + 1]["in_norm"] if i + 1 < len(self.layers) else self.final_norm
             if chain and tp.size > 1:
                 x, ss = self._chain_layer_tp(i, a.view(a.shape[0], -1), residual, i + 1 == len(self.layers), eps, ss)
                 continue
             if chain:
-                x, ss = self._chain_layer(i, a.view(a.shape[0], -1), residual, i + 1 == len(self.layers), eps)
+                x, ss = self._chain_layer(i, a.view(a.shape[0], -1), residual, i + 1 == len(self.layers), eps, meta.like > 0)
                 continue
             if tp.size == 1:
                 x = self.attn_out_mlp(i, a.view(a.shape[0], -1), residual, nxt, eps)
@@ -200,29 +200,30 @@ class LlamaModel:
         return row_parallel_add_norm(act, self.layers[i]["down"], self.ps.tp, residual, next_norm, eps)
 
     # --------------------------------------------------------- norm chain --
-    def _chain_ok(self, M: int) -> bool:
+    def _chain_ok(self, M: int, like: int = 0) -> bool:
         """Large-M TP=1 layers without add + RMSNorm passes: every GEMM of the chain on the
-        four-wave kernel (ops.norm_chain_ok) and unit norm weights (folded into qkv / gate_up)."""
+        four-wave kernel (ops.norm_chain_ok) and unit norm weights (folded into qkv / gate_up).
+        ``like``: AttnMeta.like."""
         if not self.unit_norms or len(self.layers) < 1:
             return False
         cfg, H = self.cfg, self.cfg.hidden_size
         return ops.norm_chain_ok(M, H, ((self.layers[0]["qkv"].shape[0], H), (H, self.n_q * cfg.head_dim),
                                         (2 * self.inter, H), (H, self.inter)), device=self.device,
-                                 epis=(ops.EPI_ROPE, ops.EPI_NONE, ops.EPI_SILU_MUL, ops.EPI_NONE))
+                                 epis=(ops.EPI_ROPE, ops.EPI_NONE, ops.EPI_SILU_MUL, ops.EPI_NONE), like=like)
 
-    def _chain_layer(self, i, a, residual, last, eps):
+    def _chain_layer(self, i, a, residual, last, eps, any_tile=False):
         """O (+= residual, row partials), gate_up + SiLU on the row-scaled residual, down (+=
         residual, row partials; the last layer's down does the final add + RMSNorm instead).
         Returns (x, ss): x normalised hidden states (last layer) or None with the partials."""
         L = self.layers[i]
         M, H = residual.shape
         ss_post = ops.ss_buffer(M, H, residual.device)
-        ops.gemm_res_ss(a, L["o"], residual, ss_post)
-        act = ops.gemm_rs(residual, L["gate_up"], ss_post, eps, ops.EPI_SILU_MUL)
+        ops.gemm_res_ss(a, L["o"], residual, ss_post, any_tile)
+        act = ops.gemm_rs(residual, L["gate_up"], ss_post, eps, ops.EPI_SILU_MUL, any_tile)
         if last:
             return ops.gemm_add_rmsnorm(act, L["down"], residual, self.final_norm, eps), None
         ss = ops.ss_buffer(M, H, residual.device)
-        ops.gemm_res_ss(act, L["down"], residual, ss)
+        ops.gemm_res_ss(act, L["down"], residual, ss, any_tile)
         return None, ss
 
     def _chain_layer_tp(self, i, a, residual, last, eps, ss):

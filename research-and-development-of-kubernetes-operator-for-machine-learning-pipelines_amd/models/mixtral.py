@@ -41,7 +41,7 @@ class MixtralModel(LlamaModel):
     def _folds(self):
         return (("in_norm", "qkv"),)  # post_norm feeds the router and the experts
 
-    def _chain_ok(self, M: int) -> bool:
+    def _chain_ok(self, M: int, like: int = 0) -> bool:
         return False  # the norm chain is the dense MLP's (gate_up / down on the four-wave kernel)
 
     def mlp(self, i: int, x: torch.Tensor) -> torch.Tensor:

@@ -517,13 +517,15 @@ def decode_chain_max_m() -> int:
     return GEMV_CHAIN_MAX_M
 
 
-def norm_chain_ok(M: int, H: int, shapes, device=None, epis=None) -> bool:
+def norm_chain_ok(M: int, H: int, shapes, device=None, epis=None, like: int = 0) -> bool:
     """True when the chain can run at M rows: hidden size H (ss groups of 128 columns, 16 per
     quad of lanes) and every (N, K) GEMM of the chain on the four-wave kernel, with the band
     tickets' scratch reserved on ``device`` and one ticket per 256-row band (w4_chain_ok checks
     everything launch_w4_chain does, so the chain is decided once per forward and never refused
     after a residual was updated in place).  At M <= 4 every GEMM must take the GEMV form
-    instead (``epis``: each shape's epilogue, default plain)."""
+    instead (``epis``: each shape's epilogue, default plain).  ``like``: the rows of a larger step
+    in whose place this one runs; where that one has the chain, this one has it as soon as the
+    four-wave kernel can run its products, whichever kernel is the faster (``any_tile`` below)."""
     if NORM_CHAIN == "force":
         return H % 128 == 0
     if NORM_CHAIN == "0" or GEMM_BACKEND != "mlop" or H % 256:
@@ -541,7 +543,10 @@ def norm_chain_ok(M: int, H: int, shapes, device=None, epis=None) -> bool:
         # 5-64 rows: the planner's small tiles (O / down finish their split-K and leave the row
         # sums of squares, gate_up / QKV scale their rows: gemm.hip mid_chain_ok)
         return all(bool(torch.ops.mlop.mid_chain_ok(M, N, K, e)) for (N, K), e in zip(shapes, epis))
-    return all(bool(torch.ops.mlop.w4_chain_ok(M, N, K)) for N, K in shapes)
+    if all(bool(torch.ops.mlop.w4_chain_ok(M, N, K)) for N, K in shapes):
+        return True
+    return like > M and all(bool(torch.ops.mlop.w4_chain_ok(like, N, K)) and
+                            bool(torch.ops.mlop.w4_chain_ok(M, N, K, True)) for N, K in shapes)
 
 
 def ss_buffer(M: int, H: int, device) -> torch.Tensor:
@@ -571,13 +576,14 @@ def _rinv_ref(ss: torch.Tensor, M: int, K: int, eps: float) -> torch.Tensor:
     return torch.rsqrt(ss_parts(ss, M, K)[1].view(M, 1) / K + eps)
 
 
-def gemm_res_ss(x, w, residual, ss_out):
+def gemm_res_ss(x, w, residual, ss_out, any_tile: bool = False):
     """residual [M, N] += x @ w^T in place (bf16); ss_out (ss_buffer(M, N)) <- the new residual
-    rows' partial sums of squares and totals.  The four-wave kernel's W4_ADD_SS epilogue on GPU."""
+    rows' partial sums of squares and totals.  The four-wave kernel's W4_ADD_SS epilogue on GPU;
+    ``any_tile``: also where another kernel is the choice for this product."""
     if x.is_cuda and NORM_CHAIN != "force":
         _need_gpu()
         _sk_reserve(x.device)
-        if not torch.ops.mlop.gemm_res_ss(residual, x, w, ss_out):
+        if not torch.ops.mlop.gemm_res_ss(residual, x, w, ss_out, any_tile):
             raise RuntimeError("norm chain: shape not on the four-wave kernel")
         _GEMM_USED[(_mbucket(x.shape[0]), w.shape[0], w.shape[1], EPI_ADD_SS)] = "mlop"
         return residual
@@ -589,7 +595,7 @@ def gemm_res_ss(x, w, residual, ss_out):
     return residual
 
 
-def gemm_rs(x, w, ss, eps: float, epi: int = EPI_NONE):
+def gemm_rs(x, w, ss, eps: float, epi: int = EPI_NONE, any_tile: bool = False):
     """epi(rmsnorm_unit(x) @ w^T) with the row factors from ss (gemm_res_ss's partials): the
     normalisation is applied to the accumulators (W4_RS), x is the raw residual."""
     M, K = x.shape
@@ -598,21 +604,23 @@ def gemm_rs(x, w, ss, eps: float, epi: int = EPI_NONE):
         _need_gpu()
         _sk_reserve(x.device)
         out = torch.empty(M, N if epi == EPI_NONE else N // 2, dtype=x.dtype, device=x.device)
-        if not torch.ops.mlop.gemm_rs(out, x, w, ss, eps, epi):
+        if not torch.ops.mlop.gemm_rs(out, x, w, ss, eps, epi, any_tile):
             raise RuntimeError("norm chain: shape not on the four-wave kernel")
         _GEMM_USED[(_mbucket(M), N, K, epi | EPI_RS)] = "mlop"
         return out
     return gemm((x.float() * _rinv_ref(ss, M, K, eps)).to(x.dtype), w, epi=epi)
 
 
-def qkv_rope_cache_rs(x, w, positions, cos_sin, slots, k_cache, v_cache, n_q_heads: int, ss, eps: float):
+def qkv_rope_cache_rs(x, w, positions, cos_sin, slots, k_cache, v_cache, n_q_heads: int, ss, eps: float,
+                      any_tile: bool = False):
     """qkv_rope_cache of rmsnorm_unit(x) with the row factors from ss (norm chain)."""
     M, K = x.shape
     if x.is_cuda and NORM_CHAIN != "force":
         _need_gpu()
         _sk_reserve(x.device)
         q_out = torch.empty(M, n_q_heads, k_cache.shape[3], dtype=x.dtype, device=x.device)
-        if not torch.ops.mlop.gemm_rs_rope(q_out, k_cache, v_cache, x, w, positions, cos_sin, slots, ss, eps):
+        if not torch.ops.mlop.gemm_rs_rope(q_out, k_cache, v_cache, x, w, positions, cos_sin, slots, ss, eps,
+                                           any_tile):
             raise RuntimeError("norm chain: shape not on the four-wave kernel")
         _GEMM_USED[(_mbucket(M), w.shape[0], K, EPI_ROPE | EPI_RS)] = "mlop"
         return q_out

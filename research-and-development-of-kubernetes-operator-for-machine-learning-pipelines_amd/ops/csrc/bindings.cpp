@@ -368,14 +368,14 @@ bool gemm_rope_supported(int64_t M, int64_t N, int64_t K) {
 // residual [M, N] += a . w^T in place; ss (f32, M * (N / 128 + 1)) = [M, N / 128] per-row,
 // per-128-column partial sums of squares of the new residual, then the [M] row totals; false =
 // the shape does not run on the four-wave kernel
-bool w4_chain_ok_op(int64_t M, int64_t N, int64_t K) { return mlop::w4_chain_ok((int)M, (int)N, (int)K); }
+bool w4_chain_ok_op(int64_t M, int64_t N, int64_t K, bool any) { return mlop::w4_chain_ok((int)M, (int)N, (int)K, any); }
 
 static void check_ss(const Tensor& ss, int64_t M, int64_t H, const char* name) {
   TORCH_CHECK(ss.is_cuda() && ss.scalar_type() == at::kFloat && ss.is_contiguous() &&
                   ss.numel() == M * (H / 128 + 1), name, " must be f32 [M * (H / 128 + 1)] contiguous");
 }
 
-bool gemm_res_ss(Tensor residual, Tensor a, Tensor w, Tensor ss_out) {
+bool gemm_res_ss(Tensor residual, Tensor a, Tensor w, Tensor ss_out, bool any) {
   TORCH_CHECK(a.is_cuda() && a.scalar_type() == at::kBFloat16 && a.dim() == 2 && a.stride(1) == 1 &&
                   a.stride(0) % 8 == 0, "a must be bf16 [M, K], 16-B aligned rows");
   check_bf16(w, "w"); check_bf16(residual, "residual");
@@ -405,12 +405,12 @@ bool gemm_res_ss(Tensor residual, Tensor a, Tensor w, Tensor ss_out) {
     return mlop::launch_mid_res_ss(a.data_ptr(), (int)a.stride(0), w.data_ptr(), residual.data_ptr(),
                                    (int)residual.stride(0), (int)M, (int)N, (int)K, re.ss_tot, cur_stream());
   return mlop::launch_w4_chain(4, a.data_ptr(), (int)a.stride(0), w.data_ptr(), residual.data_ptr(),
-                               (int)residual.stride(0), (int)M, (int)N, (int)K, re, cur_stream());
+                               (int)residual.stride(0), (int)M, (int)N, (int)K, re, cur_stream(), any);
 }
 
 // out = epi(diag(rsqrt(ss / K + eps)) . a . w^T): a is the un-normalised residual, ss_in its
 // partial sums of squares (gemm_res_ss), w the consumer weight with the norm weight folded in
-bool gemm_rs(Tensor out, Tensor a, Tensor w, Tensor ss_in, double eps, int64_t epi) {
+bool gemm_rs(Tensor out, Tensor a, Tensor w, Tensor ss_in, double eps, int64_t epi, bool any) {
   TORCH_CHECK(a.is_cuda() && a.scalar_type() == at::kBFloat16 && a.dim() == 2 && a.stride(1) == 1 &&
                   a.stride(0) % 8 == 0, "a must be bf16 [M, K], 16-B aligned rows");
   check_bf16(w, "w"); check_bf16(out, "out");
@@ -441,12 +441,12 @@ bool gemm_rs(Tensor out, Tensor a, Tensor w, Tensor ss_in, double eps, int64_t e
     return mlop::launch_mid_rs(a.data_ptr(), (int)a.stride(0), w.data_ptr(), out.data_ptr(), (int)out.stride(0),
                                (int)M, (int)N, (int)K, re.ss_in, (float)eps, cur_stream());
   return mlop::launch_w4_chain((int)epi | 8, a.data_ptr(), (int)a.stride(0), w.data_ptr(), out.data_ptr(),
-                               (int)out.stride(0), (int)M, (int)N, (int)K, re, cur_stream());
+                               (int)out.stride(0), (int)M, (int)N, (int)K, re, cur_stream(), any);
 }
 
 // QKV projection of the norm chain: rows scaled as gemm_rs, then RoPE + paged K / staged V
 bool gemm_rs_rope(Tensor q_out, Tensor k_cache, Tensor v_cache, Tensor a, Tensor w, Tensor pos, Tensor cos_sin,
-                  Tensor slots, Tensor ss_in, double eps) {
+                  Tensor slots, Tensor ss_in, double eps, bool any) {
   TORCH_CHECK(a.is_cuda() && a.scalar_type() == at::kBFloat16 && a.dim() == 2 && a.stride(1) == 1 &&
                   a.stride(0) % 8 == 0, "a must be bf16 [M, K], 16-B aligned rows");
   check_bf16(w, "w"); check_bf16(q_out, "q_out"); check_bf16(k_cache, "k_cache");
@@ -490,10 +490,10 @@ bool gemm_rs_rope(Tensor q_out, Tensor k_cache, Tensor v_cache, Tensor a, Tensor
     return mlop::launch_gemm_rope(a.data_ptr(), (int)a.stride(0), w.data_ptr(), (int)M, (int)N, (int)K, re,
                                   cur_stream());  // the slab path: row scale in the RoPE + cache reduce
   }
-  if (!mlop::w4_chain_ok((int)M, (int)N, (int)K)) return false;
+  if (!mlop::w4_chain_ok((int)M, (int)N, (int)K, any)) return false;
   c10::DeviceGuard g(a.device());
   return mlop::launch_w4_chain(3 | 8, a.data_ptr(), (int)a.stride(0), w.data_ptr(), nullptr, 0, (int)M, (int)N,
-                               (int)K, re, cur_stream());
+                               (int)K, re, cur_stream(), any);
 }
 
 // out = rmsnorm(residual += a . w^T) * norm_w through the split-K path; false = not taken
@@ -971,11 +971,11 @@ TORCH_LIBRARY(mlop, m) {
   m.def("vmm_chunks_ready(Tensor flat) -> int", &vmm_chunks_ready);
   m.def("vmm_error(Tensor flat) -> int", &vmm_error);
   m.def("gemm_rope_supported(int M, int N, int K) -> bool", &gemm_rope_supported);
-  m.def("w4_chain_ok(int M, int N, int K) -> bool", &w4_chain_ok_op);
-  m.def("gemm_res_ss(Tensor(a!) residual, Tensor a, Tensor w, Tensor(b!) ss_out) -> bool");
-  m.def("gemm_rs(Tensor(a!) out, Tensor a, Tensor w, Tensor ss_in, float eps, int epi) -> bool");
+  m.def("w4_chain_ok(int M, int N, int K, bool any=False) -> bool", &w4_chain_ok_op);
+  m.def("gemm_res_ss(Tensor(a!) residual, Tensor a, Tensor w, Tensor(b!) ss_out, bool any=False) -> bool");
+  m.def("gemm_rs(Tensor(a!) out, Tensor a, Tensor w, Tensor ss_in, float eps, int epi, bool any=False) -> bool");
   m.def("gemm_rs_rope(Tensor(a!) q_out, Tensor(b!) k_cache, Tensor(c!) v_cache, Tensor a, Tensor w, "
-        "Tensor pos, Tensor cos_sin, Tensor slots, Tensor ss_in, float eps) -> bool");
+        "Tensor pos, Tensor cos_sin, Tensor slots, Tensor ss_in, float eps, bool any=False) -> bool");
   m.def("gemm_rope_cache(Tensor(a!) q_out, Tensor(b!) k_cache, Tensor(c!) v_cache, Tensor a, Tensor w, "
         "Tensor pos, Tensor cos_sin, Tensor slots) -> bool");
   m.def("gemm(Tensor(a!) out, Tensor a, Tensor w, Tensor(b!) ws, int epi, float p0=0., float p1=0., int act_from=0) -> ()");

@@ -1747,20 +1747,34 @@ bool launch_gemm_rope(const void* A, int lda, const void* B, int M, int N, int K
 // first in-place residual update) and never meets a refusal mid-layer: the shape on the
 // four-wave kernel, the stream-K scratch that holds the band tickets reserved, and one ticket
 // per band of BM rows.
-bool w4_chain_ok(int M, int N, int K) {
+// ``any``: also where another kernel is the faster choice for the product, on the best four-wave height.  A decode graph
+// that stands in for one of more rows keeps that one's chain so (ops.norm_chain_ok ``like``).  Llama-3-8B widths, 6 layers:
+// 700 sequences 4143 -> 4172 us and 0.0250 -> 0.0234 from 64 bits, 600 / 760 / 850 / 900 3773 -> 3800, 4045 -> 4065, 4489 ->
+// 4490, 4440 -> 4434 (the norm passes that go pay for the slower down); three layers of the 70B at 300 rows 2653 -> 2708.
+static bool w4_chain_plan(int M, int N, int K, bool any, Plan& p) {
   if (M <= 0 || gemv_takes(M, N, K, EPI_NONE) || gemv_takes(M, N, K, EPI_ROPE)) return false;
   int cus = 0;
   if (!gemm_sk_available(&cus) || cus <= 0) return false;
-  const Plan p = plan(M, N, K, false, 0, 0);
+  p = plan(M, N, K, false, 0, 0);
+  if (any && p.variant != 5 && p.variant != 6) {
+    p = Plan{};
+    p.splits = 1;
+    if (!big_plan(M, N, K, false, p)) return false;
+  }
   return (p.variant == 5 || p.variant == 6) && p.splits == 1 && p.BN == 256 && (M + p.BM - 1) / p.BM <= kSkMaxWg &&
          gemm_w4_ok(M, N, K, K, K, N);
 }
 
+bool w4_chain_ok(int M, int N, int K, bool any) {
+  Plan p{};
+  return w4_chain_plan(M, N, K, any, p);
+}
+
 bool launch_w4_chain(int epi, const void* A, int lda, const void* B, void* C, int ldc, int M, int N, int K,
-                     const RopeEpi& re, hipStream_t st) {
+                     const RopeEpi& re, hipStream_t st, bool any) {
   if (M == 0) return true;
-  if (!w4_chain_ok(M, N, K) || !gemm_w4_ok(M, N, K, lda, K, ldc)) return false;
-  const Plan p = plan(M, N, K, false, 0, 0);
+  Plan p{};
+  if (!w4_chain_plan(M, N, K, any, p) || !gemm_w4_ok(M, N, K, lda, K, ldc)) return false;
   if (!run_w4(epi, (const uint16_t*)A, lda, (const uint16_t*)B, K, (uint16_t*)C, ldc, M, N, K, st, re, p.BM)) return false;
   return true;
 }

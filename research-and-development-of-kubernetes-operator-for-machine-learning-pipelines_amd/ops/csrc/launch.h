@@ -160,9 +160,9 @@ void run_w4_grouped(int epi, const uint16_t* A, int lda, const uint16_t* B, int 
                     int K, hipStream_t st, const RopeEpi& re, const int* offsets, int n_groups);
 // norm chain on the four-wave kernel (epi flags: 4 = C += A.B^T with ss partials, 8 = rows scaled
 // by re.ss_in; 4, 0|8, 1|8, 3|8 are built): true when every such GEMM of this shape runs there
-bool w4_chain_ok(int M, int N, int K);
+bool w4_chain_ok(int M, int N, int K, bool any = false);
 bool launch_w4_chain(int epi, const void* A, int lda, const void* B, void* C, int ldc, int M, int N, int K,
-                     const RopeEpi& re, hipStream_t st);
+                     const RopeEpi& re, hipStream_t st, bool any = false);
 // 5-384 rows, weights in a ring of their own (gemm_mid.hip): tile bm x bn as gemm.hip's mid_plan gives it
 void launch_mid(int epi, int bm, int bn, const uint16_t* A, int lda, const uint16_t* B, int ldb, uint16_t* C, int ldc,
                 float* ws, int M, int N, int K, int splits, int k_chunk, hipStream_t st, const RopeEpi& re);

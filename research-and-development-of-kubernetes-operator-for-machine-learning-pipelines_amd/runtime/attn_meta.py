@@ -58,6 +58,9 @@ class AttnMeta:
     x_rows: int = 0
     x_max: int = 0
     x_window: int = 0
+    # rows of the larger step in whose place this one runs (a decode graph between the listed sizes; 0: none): what that
+    # one keeps in 32 bits between its products, this one does too
+    like: int = 0
 
 
 # 128-token partitions: one 32-token page pair per wave at batch 1 (256: 312 tok/s, 128: 322,

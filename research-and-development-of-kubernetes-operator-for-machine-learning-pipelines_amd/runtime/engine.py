@@ -327,7 +327,7 @@ class Engine:
         self.buckets = sorted(b for b in cfg.graph_buckets if b <= cfg.max_num_seqs) or [cfg.max_num_seqs]
         if self.buckets[-1] < cfg.max_num_seqs:
             self.buckets.append(cfg.max_num_seqs)
-        self.buckets = fill_buckets(self.buckets)
+        self.listed_buckets, self.buckets = self.buckets, fill_buckets(self.buckets)
         self.G = model.n_q // model.n_kv
         self.meta = MetaBuffers(max(cfg.max_num_batched_tokens, cfg.max_num_seqs),
                                 cfg.max_num_seqs + self.buckets[-1], self.max_blocks_per_seq,
@@ -1416,6 +1416,8 @@ class Engine:
                 m.moe_capacity_tokens = b  # EP: every rank's graph of bucket b exchanges b rows
                 part, nparts = plan_partitions(b, m.n_kv, self.max_model_len)
                 meta = self.meta.meta(b, b, b, part, nparts)
+                if b not in self.listed_buckets:  # what the listed graph computes in 32 bits stays so in this one
+                    meta.like = next(n for n in self.listed_buckets if n > b)
                 ids = self.meta.ids_d[:b]
                 # decode fills (fill_decode) give every row, padding included, its own logits row
                 # in order: logits_idx is the identity, so the graph skips the row gather

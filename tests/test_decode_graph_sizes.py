@@ -62,3 +62,22 @@ def test_step_in_an_added_size(gpu, model, n):
     rows = ((a - b).norm(dim=1) / b.norm(dim=1)).sort().values
     # a token whose second and third expert are level may go either way (mixtral): all rows but one in twenty
     assert float(rows[int(len(rows) * 0.95) if cfg.num_experts else -1]) < 0.06
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("model", ["llama3-8b", "llama3-70b"])
+def test_added_size_keeps_the_norm_chain(gpu, model):
+    """Where the listed graph has the norm chain (row factors in 32 bits on the accumulators, sums into the residual), every
+    added size below it has it too: a step is not rounded once more because it runs in fewer rows."""
+    m = build_model(get_config(model, num_layers=1), device=gpu, seed=1)
+    rows, layer = set(), m._chain_layer
+
+    def spy(i, a, *args):
+        rows.add(a.shape[0])
+        return layer(i, a, *args)
+
+    m._chain_layer = spy
+    eng = Engine(m, EngineConfig(max_num_seqs=1024, max_num_batched_tokens=2048, max_model_len=256, num_kv_blocks=64))
+    assert 1024 in rows and set(eng.graphs) == set(fill_buckets(LISTED))
+    for b in eng.graphs:
+        assert b in rows or next(n for n in LISTED if n >= b) not in rows, (b, sorted(rows))

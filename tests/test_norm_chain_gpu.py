@@ -283,3 +283,36 @@ def test_checkpoint_norms_folded_chain_matches_hf(gpu, w4, tmp_path, monkeypatch
         lg = hf(torch.tensor(prompts, device=gpu)).logits[:, -1].float()
     for row, o in zip(lg, outs):
         assert row[o[0]] >= row.max() - 0.05 * row.abs().max(), (int(row.argmax()), o[0])
+
+
+@pytest.mark.parametrize("M", [320, 513, 576, 704, 705, 896])
+def test_chain_where_another_kernel_is_the_choice(gpu, M):
+    """Rows at which the planner gives a long-K product to another kernel: refused by default, and with ``any_tile`` on the
+    four-wave kernel as everywhere else."""
+    ops._sk_reserve(torch.device(gpu))
+    N, K = (8192, 8192) if M == 320 else (H, I)
+    assert not torch.ops.mlop.w4_chain_ok(M, N, K) and torch.ops.mlop.w4_chain_ok(M, N, K, True)
+    torch.manual_seed(M)
+    a, r = torch.randn(M, K, device=gpu, dtype=bf), torch.randn(M, N, device=gpu, dtype=bf)
+    w = (0.02 * torch.randn(N, K, device=gpu)).to(bf)
+    exp = r.float() + a.float() @ w.float().t()
+    sums = 2.0 ** -20 * (a.float().abs() @ w.float().abs().t())  # fp32 sums in another order
+    ss, r0 = ops.ss_buffer(M, N, gpu).fill_(float("nan")), r.clone()
+    with pytest.raises(RuntimeError, match="four-wave"):
+        ops.gemm_res_ss(a, w, r, ss)
+    assert torch.equal(r, r0)
+    ops.gemm_res_ss(a, w, r, ss, True)
+    assert ((r.float() - exp).abs() <= 2.0 ** -8 * exp.abs() + 2 * sums + 1e-6).all()  # one rounding
+    part, tot = ops.ss_parts(ss, M, N)
+    close(part, r.float().pow(2).view(M, N // 128, 128).sum(-1), atol=1e-3, rtol=1e-4)
+    close(tot, r.float().pow(2).sum(-1), atol=1e-2, rtol=1e-4)
+    # and the consumer of the row factors
+    x = (3 * torch.randn(M, K, device=gpu)).to(bf)
+    ss = ops.ss_buffer(M, K, gpu).fill_(float("nan"))
+    ops.ss_parts(ss, M, K)[1].copy_(x.float().pow(2).sum(-1))
+    with pytest.raises(RuntimeError, match="four-wave"):
+        ops.gemm_rs(x, w, ss, EPS)
+    y = ops.gemm_rs(x, w, ss, EPS, any_tile=True)
+    xf = x.float() * torch.rsqrt(x.float().pow(2).mean(-1, keepdim=True) + EPS)
+    bound = 2.0 ** -8 * (xf @ w.float().t()).abs() + 2.0 ** -19 * (xf.abs() @ w.float().abs().t())
+    assert ((y.float() - xf @ w.float().t()).abs() <= bound + 1e-6).all()
