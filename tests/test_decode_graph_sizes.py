@@ -81,3 +81,20 @@ def test_added_size_keeps_the_norm_chain(gpu, model):
     assert 1024 in rows and set(eng.graphs) == set(fill_buckets(LISTED))
     for b in eng.graphs:
         assert b in rows or next(n for n in LISTED if n >= b) not in rows, (b, sorted(rows))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("model", ["llama3-8b", "mixtral-8x7b"])
+def test_added_sizes_are_not_run_before_their_capture(gpu, model):
+    """An engine starts with one run of the model per listed size; the added ones are captured only."""
+    m = build_model(get_config(model, num_layers=1), device=gpu, seed=1)
+    ran, caught, forward = [], [], m.forward
+
+    def spy(ids, *args):
+        (caught if torch.cuda.is_current_stream_capturing() else ran).append(ids.shape[0])
+        return forward(ids, *args)
+
+    m.forward = spy
+    Engine(m, EngineConfig(max_num_seqs=512, max_num_batched_tokens=2048, max_model_len=256, num_kv_blocks=64))
+    listed = [b for b in LISTED if b <= 512]
+    assert sorted(ran) == listed and sorted(caught) == fill_buckets(listed)
