@@ -1423,7 +1423,8 @@ class Engine:
         t0 = time.perf_counter()
         verbose = False
         widest = None  # logits of the largest graph, captured first
-        added = [] if not self._native_products() else [b for b in self.buckets if b not in self.listed_buckets]
+        alone = self._native_products()
+        added = [b for b in self.buckets if b not in self.listed_buckets] if alone else []
         order = sorted((b for b in self.buckets if b not in added), reverse=True) + added[::-1]
         with torch.cuda.stream(stream):
             for bi, b in enumerate(order):
@@ -1437,11 +1438,12 @@ class Engine:
                 ids = self.meta.ids_d[:b]
                 # decode fills (fill_decode) give every row, padding included, its own logits row
                 # in order: logits_idx is the identity, so the graph skips the row gather
-                if b not in added:  # warm-up (allocator, autotune, lazy init); the device runs it during the capture
+                if b not in added:  # warm-up (allocator, autotune, lazy init); the device may run it during the capture
                     self.meta.upload(b, b)
                     m.logits_local(m.forward(ids, meta, self.kv))
-                if bi == 0:  # the widest warm-up's memory is the graphs' now
+                if bi == 0 or not alone:  # (a communicator's watchdog may ask for its events, which a capture forbids)
                     torch.cuda.synchronize(self.device)
+                if bi == 0:  # the widest warm-up's memory is the graphs' now
                     torch.cuda.empty_cache()
                 if verbose:
                     print(f"[engine] capturing decode graph {bi + 1}/{len(order)} (batch {b}) "
