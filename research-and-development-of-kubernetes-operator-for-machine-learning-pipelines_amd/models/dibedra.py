@@ -182,9 +182,12 @@ class DibedraModel:
                                   **self._layer(i, x, meta, kv))
         return x
 
-    def logits_local(self, hidden: torch.Tensor) -> torch.Tensor:
-        """[n, padded width] -> logits [n, vocab] (model dtype)."""
-        return linear(hidden, self.head)[:, :self.cfg.vocab_size]
+    def logits_local(self, hidden: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
+        """[n, padded width] -> logits [n, vocab] (model dtype; of ``logits_buffer`` rows ``out`` where given)."""
+        return linear(hidden, self.head, out)[:, :self.cfg.vocab_size]
+
+    def logits_buffer(self, rows: int) -> torch.Tensor:
+        return torch.empty(rows, self.head.shape[0], dtype=self.dtype, device=self.device)
 
     logits = logits_local
 

@@ -153,9 +153,12 @@ class KosesunModel:
                                store=not last)
         return x
 
-    def logits_local(self, hidden: torch.Tensor) -> torch.Tensor:
-        """[n, W] -> soft-capped logits [n, vocab] in fp32."""
-        return ops.softcap(linear(hidden, self.head), self.cfg.logit_softcap)[:, :self.cfg.vocab_size]
+    def logits_local(self, hidden: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
+        """[n, W] -> soft-capped logits [n, vocab] in fp32 (of ``logits_buffer`` rows ``out`` where given)."""
+        return ops.softcap(linear(hidden, self.head), self.cfg.logit_softcap, out)[:, :self.cfg.vocab_size]
+
+    def logits_buffer(self, rows: int) -> torch.Tensor:
+        return torch.empty(rows, self.head.shape[0], dtype=torch.float32, device=self.device)
 
     logits = logits_local
 

@@ -246,7 +246,9 @@ class LlamaModel:
         """[n, H] -> this rank's vocab shard of the logits [n, V/TP] (model dtype), in ``out`` where given."""
         return linear(hidden, self.lm_head, out)
 
-    logits_out = True  # logits_local takes ``out``
+    def logits_buffer(self, rows: int) -> torch.Tensor:
+        """What ``logits_local`` may write into, for up to ``rows`` rows."""
+        return torch.empty(rows, self.lm_head.shape[0], dtype=self.dtype, device=self.device)
 
     def logits(self, hidden: torch.Tensor) -> torch.Tensor:
         """[n, H] -> full-vocab logits [n, V] in the model dtype (bf16 on GPU: the

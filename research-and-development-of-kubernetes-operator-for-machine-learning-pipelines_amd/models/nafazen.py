@@ -191,10 +191,16 @@ class NafazenModel:
                                   **run(i, x, meta, kv))
         return x
 
-    def logits_local(self, hidden: torch.Tensor) -> torch.Tensor:
-        """[n, padded width] -> logits [n, vocab], soft-capped in fp32 (no cap: as the product leaves them)."""
-        lg = linear(hidden, self.head)
-        return (ops.softcap(lg, self.cfg.logit_softcap) if self.cfg.logit_softcap else lg)[:, :self.cfg.vocab_size]
+    def logits_local(self, hidden: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
+        """[n, padded width] -> logits [n, vocab], soft-capped in fp32 (no cap: as the product leaves them); of
+        ``logits_buffer`` rows ``out`` where given."""
+        cap = self.cfg.logit_softcap
+        lg = linear(hidden, self.head, None if cap else out)
+        return (ops.softcap(lg, cap, out) if cap else lg)[:, :self.cfg.vocab_size]
+
+    def logits_buffer(self, rows: int) -> torch.Tensor:
+        return torch.empty(rows, self.head.shape[0], device=self.device,
+                           dtype=torch.float32 if self.cfg.logit_softcap else self.dtype)
 
     logits = logits_local
 

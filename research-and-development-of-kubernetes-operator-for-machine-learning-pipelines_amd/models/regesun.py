@@ -172,9 +172,12 @@ class RegesunModel:
                                   store=not last)
         return x
 
-    def logits_local(self, hidden: torch.Tensor) -> torch.Tensor:
-        """[n, W] -> logits [n, vocab] (model dtype)."""
-        return linear(hidden, self.head)[:, :self.cfg.vocab_size]
+    def logits_local(self, hidden: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
+        """[n, W] -> logits [n, vocab] (model dtype; of ``logits_buffer`` rows ``out`` where given)."""
+        return linear(hidden, self.head, out)[:, :self.cfg.vocab_size]
+
+    def logits_buffer(self, rows: int) -> torch.Tensor:
+        return torch.empty(rows, self.head.shape[0], dtype=self.dtype, device=self.device)
 
     logits = logits_local
 

@@ -794,12 +794,12 @@ def gelu_tanh(x):
     return x
 
 
-def softcap(x, cap: float):
+def softcap(x, cap: float, out: torch.Tensor | None = None):
     """cap * tanh(x / cap), fp32."""
     if not x.is_cuda:
-        return ref.softcap(x, cap)
+        return ref.softcap(x, cap) if out is None else out.copy_(ref.softcap(x, cap))
     _need_gpu()
-    out = torch.empty(x.shape, dtype=torch.float32, device=x.device)
+    out = torch.empty(x.shape, dtype=torch.float32, device=x.device) if out is None else out
     torch.ops.mlop.softcap(out, x, cap)
     return out
 

@@ -1268,7 +1268,7 @@ class Engine:
         # the device is not waited for: a caller may feed the next step while this one runs
         if self.model.ps.tp.size == 1 and idx == list(range(len(idx))):
             rows = logits[:len(idx)]
-            return rows if portions or self.graphs.get(bucket) is None else rows.clone()  # (a graph's buffer is its own)
+            return rows if portions or self.graphs.get(bucket) is None else rows.clone()  # (the graphs' one buffer)
         at_d = torch.tensor(idx, pin_memory=logits.is_cuda).to(logits.device, non_blocking=True)
         return logits[at_d]
 
@@ -1422,7 +1422,9 @@ class Engine:
         empty = np.zeros(0, dtype=np.int32)
         t0 = time.perf_counter()
         verbose = False
-        widest = None  # logits of the largest graph, captured first
+        # one graph replays at a time and its logits are read before the next does: all write into one buffer
+        buf = m.logits_buffer(self.buckets[-1]) if hasattr(m, "logits_buffer") else None
+        logits_of = lambda h, b: m.logits_local(h) if buf is None else m.logits_local(h, out=buf[:b])  # noqa: E731
         alone = self._native_products()
         added = [b for b in self.buckets if b not in self.listed_buckets] if alone else []
         order = sorted((b for b in self.buckets if b not in added), reverse=True) + added[::-1]
@@ -1440,7 +1442,7 @@ class Engine:
                 # in order: logits_idx is the identity, so the graph skips the row gather
                 if b not in added:  # warm-up (allocator, autotune, lazy init); the device may run it during the capture
                     self.meta.upload(b, b)
-                    m.logits_local(m.forward(ids, meta, self.kv))
+                    logits_of(m.forward(ids, meta, self.kv), b)
                 if bi == 0 or not alone:  # (a communicator's watchdog may ask for its events, which a capture forbids)
                     torch.cuda.synchronize(self.device)
                 if bi == 0:  # the widest warm-up's memory is the graphs' now
@@ -1448,17 +1450,12 @@ class Engine:
                 if verbose:
                     print(f"[engine] capturing decode graph {bi + 1}/{len(order)} (batch {b}) "
                           f"at {time.perf_counter() - t0:.1f} s", file=sys.stderr, flush=True)
-                # one graph replays at a time and its logits are read before the next does: the smaller graphs write
-                # theirs into the largest one's buffer where the model can
-                shared = bi and getattr(m, "logits_out", False)
                 g = torch.cuda.CUDAGraph()
                 g.capture_begin(pool=self.graph_pool)
                 try:
-                    hidden = m.forward(ids, meta, self.kv)
-                    logits = m.logits_local(hidden, out=widest[:b]) if shared else m.logits_local(hidden)
+                    logits = logits_of(m.forward(ids, meta, self.kv), b)
                 finally:
                     g.capture_end()
-                widest = logits if bi == 0 else widest
                 self.graphs[b] = (g, logits)
         torch.cuda.current_stream(self.device).wait_stream(stream)
         torch.cuda.synchronize(self.device)
