@@ -134,6 +134,37 @@ def _row_errors(a, b):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("model", HYBRID)
+@pytest.mark.parametrize("n", [33, 81, 193, 321])
+def test_hybrid_step_in_an_added_size(gpu, model, n):
+    """The models with recurrent layers, four layers of them; the same steps with and without graphs, twice one after the
+    other (the second reads the state that the first left)."""
+    m = build_model(get_config(model, num_layers=4), device=gpu, seed=1)
+    got, eng = _steps(m, n, True, [n, n])
+    want, _ = _steps(m, n, False, [n, n])
+    assert min(g for g in eng.graphs if g >= n) not in LISTED
+    for a, b in zip(got, want):
+        assert a.shape == (n, m.cfg.vocab_size) and bool(torch.isfinite(a).all())
+        # twice the layers of BOUND; a token whose experts are level may go either way
+        assert float(_row_errors(a, b)[int(n * 0.95)]) < 2 ** 0.5 * BOUND
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("model", ["llama3-8b", "mixtral-8x7b"])
+@pytest.mark.parametrize("n", [385, 577, 705, 833, 1025, 1537])
+def test_step_in_a_large_added_size(gpu, model, n):
+    """The steps of 64 and of 256 rows, as test_step_in_an_added_size."""
+    m = build_model(get_config(model, num_layers=2), device=gpu, seed=1)
+    if m.cfg.num_experts:
+        for L in m.layers:
+            L["router"].mul_(8)
+    (a,), eng = _steps(m, n, True, [n], (*LISTED, 2048), 2048)
+    (b,), _ = _steps(m, n, False, [n], (*LISTED, 2048), 2048)
+    assert min(g for g in eng.graphs if g >= n) not in (*LISTED, 2048)
+    assert float(_row_errors(a, b)[int(n * 0.95) if m.cfg.num_experts else -1]) < BOUND
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("model", ["llama3-8b", "kosesun-1b"])
 def test_logits_outlive_the_next_step(gpu, model):
     """All graphs write into one buffer: what ``feed`` returned stays as it was while steps of other sizes run."""
