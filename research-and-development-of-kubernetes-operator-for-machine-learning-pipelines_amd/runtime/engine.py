@@ -229,7 +229,10 @@ class EngineConfig:
     kv_fraction: float = 0.5  # pages for this share of max_num_seqs x max_model_len (mean context;
                               # preemption covers the tail) - same policy as controller/placement.py
     use_graphs: bool = True
+    # decode graph sizes; sizes between neighbours at most a factor of two apart are captured as well (fill_buckets),
+    # unless fill_graph_buckets is off: then these, up to max_num_seqs, and max_num_seqs
     graph_buckets: tuple = (1, 2, 4, 8, 16, 32, 64, 128, 256, 512, 1024)
+    fill_graph_buckets: bool = True
     prefill_min_batch: int = 1
     max_decode_gap: int = 0
     mixed_prefill: bool = True    # prefill chunks ride in the decode step (one forward)
@@ -327,7 +330,9 @@ class Engine:
         self.buckets = sorted(b for b in cfg.graph_buckets if b <= cfg.max_num_seqs) or [cfg.max_num_seqs]
         if self.buckets[-1] < cfg.max_num_seqs:
             self.buckets.append(cfg.max_num_seqs)
-        self.listed_buckets, self.buckets = self.buckets, fill_buckets(self.buckets)
+        self.listed_buckets = self.buckets
+        if cfg.fill_graph_buckets:
+            self.buckets = fill_buckets(self.buckets)
         self.G = model.n_q // model.n_kv
         self.meta = MetaBuffers(max(cfg.max_num_batched_tokens, cfg.max_num_seqs),
                                 cfg.max_num_seqs + self.buckets[-1], self.max_blocks_per_seq,

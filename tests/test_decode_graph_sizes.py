@@ -35,6 +35,14 @@ def test_fill_buckets_waste():
         assert b - n < max(16, n // 3)
 
 
+@pytest.mark.parametrize("fill", [True, False])
+def test_exactly_the_listed_sizes(fill):
+    m = build_model(get_config("tiny-llama"), device="cpu", dtype=torch.float32)
+    eng = Engine(m, EngineConfig(max_num_seqs=80, max_num_batched_tokens=128, max_model_len=64, num_kv_blocks=16,
+                                 graph_buckets=(32, 64, 128), fill_graph_buckets=fill))
+    assert eng.buckets == ([32, 48, 64, 80] if fill else [32, 64, 80])
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("model", ["llama3-8b", "mixtral-8x7b"])
 @pytest.mark.parametrize("n", [33, 81, 129, 193, 257, 321])
