@@ -299,6 +299,11 @@ std::vector<int64_t> gemm_plan(int64_t M, int64_t N, int64_t K) {
   return {p[0], p[1], p[2], p[3], p[4]};
 }
 
+int64_t gemm_grouped_height(at::IntArrayRef rows, int64_t N, int64_t K, int64_t cus) {
+  TORCH_CHECK(!rows.empty() && rows.size() <= 64 && N >= 256 && K >= 64 && cus > 0, "rows of 1 - 64 experts, N >= 256, K >= 64, cus");
+  return mlop::gemm_grouped_height(rows.data(), (int)rows.size(), (int)N, (int)K, (int)cus);
+}
+
 int64_t gemm_grouped_variant(int64_t M, int64_t N, int64_t K, int64_t groups, int64_t rows, int64_t a_n) {
   return mlop::gemm_grouped_variant((int)M, (int)N, (int)K, (int)groups, (int)rows, (int)a_n);
 }
@@ -934,6 +939,7 @@ TORCH_LIBRARY(mlop, m) {
   m.def("ep_destroy(int h) -> ()", &ep_destroy);
   m.def("gemm_workspace(int M, int N, int K, int epi) -> int", &gemm_workspace);
   m.def("gemm_plan(int M, int N, int K) -> int[]", &gemm_plan);
+  m.def("gemm_grouped_height(int[] rows, int N, int K, int cus=256) -> int", &gemm_grouped_height);
   m.def("gemm_grouped_variant(int M, int N, int K, int groups, int rows, int a_n) -> int", &gemm_grouped_variant);
   m.def("gemm_big_variant(int set=-1) -> int", &gemm_big_variant);
   m.def("gemm_half_tile(int set=-1) -> int", &gemm_half_tile);

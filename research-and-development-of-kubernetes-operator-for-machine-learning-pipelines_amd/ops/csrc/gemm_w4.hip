@@ -697,10 +697,36 @@ __global__ void __launch_bounds__(256, 1) gemm_w4_kernel(
                                  nullptr, 0);
 }
 
+// Tile height of the experts' products, by estimated time in rounds of 256-row tiles (a round of the lower ones .89 / .79 /
+// .69, K-halves .59; W: the weights' rounds at one tile per expert, which bound the lower tiles).  tNNN: row tiles of that height
+// over all experts, experts: those with rows, G: workgroups.
+__host__ __device__ __forceinline__ int w4_grouped_height(int t256, int t224, int t192, int t160, int experts, int n_tiles_x, int G,
+                                                          int nk, bool halves) {
+  auto rounds = [&](int t) {
+    const int T = t * n_tiles_x, r = T % G;
+    return (float)(T / G) + (r == 0 ? 0.f : 2 * r <= G && nk % 2 == 0 && halves ? .59f : 1.f);
+  };
+  const float W = (float)(experts * n_tiles_x) / (float)G;
+  const float e256 = rounds(t256), e224 = fmaxf(.89f * rounds(t224), .94f * W);
+  const float e192 = fmaxf(.79f * rounds(t192), .88f * W), e160 = fmaxf(.69f * rounds(t160), .81f * W);
+  const float upper = fminf(e256, e224), lower = fminf(e192, e160);
+  return upper <= lower ? (e256 <= e224 ? 256 : 224) : e192 <= e160 ? 192 : 160;
+}
+
+// The same for given counts of rows (tests).
+int gemm_grouped_height(const int64_t* rows, int n_groups, int N, int K, int cus) {
+  int t[4] = {}, experts = 0, total = 0;
+  for (int g = 0; g < n_groups; ++g) {
+    const int r = (int)rows[g];
+    t[0] += (r + 255) / 256, t[1] += (r + 223) / 224, t[2] += (r + 191) / 192, t[3] += (r + 159) / 160;
+    experts += r > 0, total += r;
+  }
+  const int G = (int)std::min<long>((long)(N / 256) * ((total + 159) / 160 + n_groups), cus);  // run_w4_grouped_t's grid
+  return w4_grouped_height(t[0], t[1], t[2], t[3], experts, N / 256, G, K / 64, true);
+}
+
 // The experts' products of a prompt.  What the grid loses is rows of partial tiles and the last round, and both hang on
-// the routing, which only the device knows: the height is chosen here, by estimated time in rounds of 256-row tiles (a
-// round of the lower ones .89 / .79 / .69, K-halves .59; W: the weights' rounds at one tile per expert, which bound the lower
-// tiles).  gate_up of 8 experts, 256 / 192 / 160 rows: 300 rows each 738 / 619 / 532 us, 350 747 / 595 / 691, 500 779 /
+// the routing, which only the device knows: the height is chosen here (w4_grouped_height).  gate_up of 8 experts, 256 / 192 / 160 rows: 300 rows each 738 / 619 / 532 us, 350 747 / 595 / 691, 500 779 /
 // 836 / 911, 550 1021 / 836 / 941, 1024 1497 / 1561 / 1598 (1.29 PFLOP/s); over 22 sizes, even and with the experts
 // 0.6 - 1.4 of the mean, the choice is within 1 % of the best of these three on average.  With 224 rows 407 each take 663
 // us where the ping-pong kernel took 735 and the three heights 714 - 745.  One XCD's workgroups share
@@ -723,15 +749,8 @@ __global__ void __launch_bounds__(256, 1) gemm_w4_grouped_kernel(
   }
   a = __builtin_amdgcn_readfirstlane(a);
   b = __builtin_amdgcn_readfirstlane(b);
-  auto rounds = [&](uint32_t t) {
-    const int T = (int)t * n_tiles_x, r = T % G;
-    return (float)(T / G) + (r == 0 ? 0.f : 2 * r <= G && nk % 2 == 0 && ws != nullptr ? .59f : 1.f);
-  };
-  const float W = (float)(__popcll(__ballot(rows > 0)) * n_tiles_x) / (float)G;
-  const float t256 = rounds(a & 0xffff), t224 = fmaxf(.89f * rounds(b >> 16), .94f * W);
-  const float t192 = fmaxf(.79f * rounds(a >> 16), .88f * W), t160 = fmaxf(.69f * rounds(b & 0xffff), .81f * W);
-  const float upper = fminf(t256, t224), lower = fminf(t192, t160);
-  const int h = __builtin_amdgcn_readfirstlane(upper <= lower ? (t256 <= t224 ? 256 : 224) : t192 <= t160 ? 192 : 160);
+  const int h = __builtin_amdgcn_readfirstlane(w4_grouped_height(a & 0xffff, b >> 16, a >> 16, b & 0xffff,
+                                                                 __popcll(__ballot(rows > 0)), n_tiles_x, G, nk, ws != nullptr));
 #define MLOP_W4_GROUPED(h_)                                                                                           \
   gemm_w4_tiles<EPI, h_, true>(A, lda, B, ldb, C, ldc, M, N, K, n_tiles_x, 0, 1, re, 0, 0, ws, cnt, offsets, n_groups)
   if (h == 256) MLOP_W4_GROUPED(256);

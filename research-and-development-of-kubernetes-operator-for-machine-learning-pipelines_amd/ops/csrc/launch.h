@@ -138,6 +138,8 @@ void gemm_plan(int M, int N, int K, int out[5]);
 bool gemm_weights_nt(int m_tiles);
 // the experts' product of M routed rows, max_rows of them per expert on average, from a_n rows: gemm.hip grouped_plan
 int gemm_grouped_variant(int M, int N, int K, int n_groups, int max_rows, int a_n);
+// tile height that the four-wave kernel chooses for experts of so many rows on cus CUs (tests)
+int gemm_grouped_height(const int64_t* rows, int n_groups, int N, int K, int cus);
 // large-M kernel variant of the GEMM planner (gemm.hip plan(): 0 256x128, 1/2 256x256
 // 8-wave, 3 ping-pong, 5 four-wave asm K-loop); set >= 0 overrides (in-process A/B), returns the current value
 int gemm_big_variant(int set);

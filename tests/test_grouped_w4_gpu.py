@@ -18,6 +18,27 @@ COUNTS = {
     "even-250": [250, 256, 249, 255, 251, 256, 240, 256],
     "skewed": [1500, 3, 17, 0, 64, 5, 90, 700],
     "single-row": [0, 0, 0, 1, 0, 0, 0, 0],
+    "even-224": [224] * G,
+    "even-448": [448] * G,
+    "seven-448": [448] * 7 + [0],
+    "224-edges": [223, 0, 447, 225, 448, 449, 672, 0],
+    "above-512-each": [0, 896, 224, 672, 896, 1120, 0, 672],  # the K walk of larger prompts
+}
+# the height that each leads to at K = 192 / 448 / 1536, and whether its tail is cut into K-halves there
+HEIGHTS = {
+    "even-150": ("160", "160", "160"),
+    "one-row-over": ("256", "256", "256"),
+    "one-expert": ("160", "160", "160 halves"),
+    "first-and-last": ("160", "160", "160 halves"),
+    "even-190": ("192", "192", "192"),
+    "even-250": ("256", "256", "256"),
+    "skewed": ("224", "224", "192 halves"),
+    "single-row": ("160", "160", "160 halves"),
+    "even-224": ("224", "224", "224"),
+    "even-448": ("224", "224", "224"),
+    "seven-448": ("224", "224", "224 halves"),
+    "224-edges": ("224", "224", "224"),
+    "above-512-each": ("224", "224", "224 halves"),
 }
 
 
@@ -27,6 +48,17 @@ def glu(z, lim):
         return g, u, g * g.sigmoid() * u
     gc, uc = g.clamp(max=lim[1]), u.clamp(-lim[1], lim[1])
     return gc, uc + 1, gc * (lim[0] * gc).sigmoid() * (uc + 1)
+
+
+@pytest.mark.parametrize("name", COUNTS)
+def test_heights(gpu, name):
+    """Each routing leads to the height it stands for, and all four are there, with K-halves where a height may have them."""
+    cus, got = torch.cuda.get_device_properties(gpu).multi_processor_count, []
+    for K in (192, 448, 1536):
+        h = torch.ops.mlop.gemm_grouped_height(COUNTS[name], N, K, cus)
+        tail = sum(-(-c // h) for c in COUNTS[name]) * (N // 256) % cus
+        got.append(f"{h} halves" if K // 64 % 2 == 0 and 0 < 2 * tail <= cus else str(h))
+    assert tuple(got) == HEIGHTS[name]
 
 
 @pytest.mark.parametrize("counts", COUNTS.values(), ids=COUNTS.keys())
