@@ -195,11 +195,16 @@ __global__ void __launch_bounds__(256, 3) paged_attn_kernel(
   __shared__ float sm_l[4][16];
   __shared__ int sm_last;
 
-  // From 32 tiles on the kv heads are the fastest index: a page holds the heads' 4-KB blocks one behind the other, and whatever
-  // workgroups run at a time read them all.  With tiles fastest a launch ended on two heads, a quarter of every page (a
-  // step of 40 x 8000 keys 2620 -> 2518 us, 48 x 7000 2472 -> 2408, 200 x 1500 2562 -> 2507, 700 x 500 4119 -> 4084, 20 x 17500 2839 ->
-  // 2816, 100 x 1000 the same).  Few long sequences in shares lose a little: 8 x 20000 1388 -> 1400, 13 x 2056 937 -> 940.
-  const bool by_head = tiles >= 32;
+  // From 32 tiles of 8 kv heads on the heads are the fastest index: a page holds the heads' 4-KB blocks one behind the other,
+  // and whatever workgroups run at a time read them all.  With tiles fastest a launch ended on two heads, a quarter of every page (a
+  // step of 40 x 8000 keys 2620 -> 2518 us, 48 x 7000 2472 -> 2408, 200 x 1500 2562 -> 2507, 700 x 500 4119 -> 4084).  Fewer heads are
+  // less of a page's stripes than that anyhow, and one tile's heads end together: 2 and 4 heads (a tensor-parallel
+  // shard's) lose 1 - 3 % at 24 - 200 tiles on average and 8 % at worst (4 heads, 36 tiles of 4000 keys 64.4 -> 68.1 us), and gain
+  // 1 - 5 % from 250 - 300 on.  Kernel times by heads fastest over tiles fastest, contexts of 500 - 20000, means over 4 - 24
+  // launches: 8 heads 1.00 at 24 tiles, 0.99 at 28, 1.01 / 0.98 / 0.96 / 0.94 / 0.96 at 32 / 40 / 64 / 80 / 150, 1.02 at 300 - 700; 16 and 32 heads
+  // 0.97 - 1.0 from 32 on; 4 heads 1.02 / 1.02 / 1.01 / 0.98 / 0.95 at 32 / 64 / 150 / 300 / 700.  A few long sequences in shares
+  // lose a little too: steps of 8 x 20000 1388 -> 1400, 13 x 2056 937 -> 940.
+  const bool by_head = Hkv > 1 && tiles >= (Hkv >= 8 ? 32 : 256);
   const int lin = blockIdx.x + tiles * blockIdx.y, part = blockIdx.z;
   const int tile = by_head ? lin / Hkv : blockIdx.x, kvh = by_head ? lin % Hkv : blockIdx.y;
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;

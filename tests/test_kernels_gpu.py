@@ -297,6 +297,28 @@ def test_paged_attention_one_sequence_many_kv_heads(gpu, Hkv, ctx, attn_fused_al
     close(ops.paged_attention(q, kc, vc, m), ref.paged_attention(q, kc, vc, m), atol=2e-2, rtol=2e-2)
 
 
+@pytest.mark.parametrize("Hq,Hkv,tiles", [(32, 8, 31), (32, 8, 32), (16, 16, 33), (8, 2, 32), (16, 4, 255), (16, 4, 256), (8, 2, 257),
+                                          (28, 7, 256), (4, 1, 256)])
+def test_paged_attention_tile_and_head_order(gpu, Hq, Hkv, tiles, attn_fused_all):
+    """Where the launch's fastest index turns from the tiles to the kv heads, whole and in shares."""
+    from mlopamd.runtime.attn_meta import plan_partitions
+
+    torch.manual_seed(0)
+    np.random.seed(0)
+    lens = [(7 * i) % 190 for i in range(tiles)]
+    NB = sum((c + 15) // 16 for c in lens) + 8
+    kc = torch.randn(NB, Hkv, 16, 128, device=gpu, dtype=bf)
+    vc = torch.randn(NB, Hkv, 16, 128, device=gpu, dtype=bf)
+    q = torch.randn(tiles, Hq, 128, device=gpu, dtype=bf)
+    for part, nparts in ((192, 1), plan_partitions(tiles, Hkv, 4096)):
+        m, T = make_meta(gpu, [1] * tiles, lens, Hkv, Hq // Hkv, NB, part_tokens=part, nparts=nparts)
+        m.part_sem = torch.zeros(tiles * Hkv, dtype=torch.int32, device=gpu)
+        out = torch.full_like(q, float("nan"))
+        ops.paged_attention(q, kc, vc, m, out=out)
+        close(out, ref.paged_attention(q, kc, vc, m), atol=2e-2, rtol=2e-2)
+        assert int(m.part_sem.abs().sum()) == 0
+
+
 @pytest.mark.parametrize("fused", [False, True])
 @pytest.mark.parametrize("Hq,Hkv,long,short,padding", [
     (32, 8, [4000], [100] * 20, 0),            # all of the 7 shares that are planned
