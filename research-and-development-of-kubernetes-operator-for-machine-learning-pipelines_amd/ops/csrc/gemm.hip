@@ -1393,17 +1393,19 @@ static bool mid_plan(int M, int N, int K, Plan& p) {
 // 15 us.  A round of the ping-pong kernel takes 13.5 + 0.0206 K, its tail 1.1 of
 // what sk_tail_cost says (1.0 fits as well; where the two are level the four-wave kernel is the better choice, since a
 // layer whose four projections all run there needs no add + RMSNorm passes: 1024 rows of Llama-3-8B 2855 -> 2811 us).
-// Constants fitted to 39 weight shapes (the projections of Llama-3-8B and 70B, whole and in 2 - 8 shards, Mixtral's,
-// a 1B model's and shapes of no model here: N 1024 - 128256, K 1024 - 28672) at 39 row counts from 385 to 8192, every
-// variant measured in one process, two to four times: the choice is 0.13 % slower than the best of the five on average,
-// more than 5 % at 8 of 1370 points, 12 % at worst; fitted to half of the shapes, 0.3 % on the others.  (Constants fitted
-// to Llama-3-8B's matrices alone: 1.4 %, 110 of 1147 points and 38 %, and at 46 of them slower than the rule by tile
-// counts that was here before: 70B qkv at 640 rows 113 us against 102, o at 1000 116 against 107, down at 2300 839
-// against 785; all three are within 3 % of the best now.)  The 224-row tile, measured on 13 of the shapes at 21 row counts:
-// 1.2 % faster on average, 53 of 273 points by more than 2 % (gate_up at 400 / 892 / 1100 rows 99 -> 89, 188 -> 174, 216 ->
-// 209 us), the choice among the heights 0.27 % slower than the best, over 5 % at three points.  That rule, heights 256 and 128 only, was 8.4 % slower than the
-// best (gate_up of Llama-3-8B at 400 / 700 / 1152 rows 138 -> 92, 158 -> 147, 245 -> 219 us, o at 1152 / 2300 / 2600
-// 55 -> 43, 79 -> 62, 83 -> 68).
+// Constants of the ping-pong kernel and of 256, 192, 160 and 128 rows fitted to 39 weight shapes (the projections of
+// Llama-3-8B and 70B, whole and in 2 - 8 shards, Mixtral's, a 1B model's and shapes of no model here: N 1024 - 128256, K
+// 1024 - 28672) at 39 row counts from 385 to 8192, every variant measured in one process, two to four times: the choice was
+// 0.13 % slower than the best of those five on average, more than 5 % at 8 of 1370 points, 12 % at worst; fitted to half of
+// the shapes, 0.3 % on the others.  (Constants fitted to Llama-3-8B's matrices alone: 1.4 %, 110 of 1147 points and 38 %, and
+// at 46 of them slower than the rule by tile counts that was here before: 70B qkv at 640 rows 113 us against 102, o at 1000
+// 116 against 107, down at 2300 839 against 785.  The rule by tile counts, heights 256 and 128 only, was 8.4 % slower than
+// the best on average: gate_up of Llama-3-8B at 400 / 700 / 1152 rows 138 -> 92, 158 -> 147, 245 -> 219 us, o at 1152 / 2300 /
+// 2600 55 -> 43, 79 -> 62, 83 -> 68.)
+// With the 224-row tile, 15 shapes at up to 30 row counts from 400 to 8000: it is the best at 62 of 352 points, by more than
+// 2 % at 46 and 0.9 % on average (gate_up of Llama-3-8B at 400 / 892 rows 92 -> 84, 178 -> 165 us, 8192 x 8192 at 5200 495 -> 459);
+// the choice is 0.48 % slower than the best of all six, more than 5 % at 11 points (8192 x 28672 at 400 - 512 rows up to 13 %,
+// 10240 x 8192 at 6600 10 %).
 static bool big_plan(int M, int N, int K, bool pp_ok, Plan& p) {
   const SkBuf* b = sk_buf();
   if (!b || !gemm_w4_ok(M, N, K, K, K)) return false;
@@ -1424,8 +1426,10 @@ static bool big_plan(int M, int N, int K, bool pp_ok, Plan& p) {
   for (const Tile& t : tiles) {
     if (t.rows < 256 && !g_half_tile) break;
     const long T = (long)((M + t.rows - 1) / t.rows) * (N / 256), q = T / b->cus, r = T % b->cus;
-    // (from five whole rounds on the 224-row tile gives its 2 % of a round back in clock: 3700 rows of Llama-3-8B, gate_up
-    // 665 -> 671 us with it and the layer's other kernels 2.5 % slower beside it)
+    // (From five whole rounds on the 224-row tile counts more.  By itself it does not need to: over 56 products of five
+    // rounds and more the choice is 0.18 % slower than the best height with .90 throughout, 0.23 % with .925.  It is for steps: a
+    // prompt of 3700 tokens of Llama-3-8B, seven rounds, took 8417 us with that tile in gate_up and 8336 with 256 rows, gate_up
+    // itself 671 and 665, the kernels beside it 2.5 % longer; why was not measured.)
     const float one = full * (t.rows == 224 && q >= 5 ? .925f : t.round);
     float us = (float)q * one;
     const bool halves = r > 0 && gemm_w4_split_ok((int)T, nk);
@@ -1947,9 +1951,10 @@ bool launch_gemm_add_rmsnorm(const void* A, int lda, const void* B, void* out, v
 // - 440 rows: two 256-row tiles of which a fifth is empty, and three lower ones.)  Not at 160 - 240 rows of up to 8 experts,
 // one tile each: there the weights' latency bounds both, and the ping-pong kernel skips a tile's empty 64-row quadrants (200
 // rows 394 us against 420; 16 x 12800 x 4096 378 against 355, 32 x 8192 x 2048 290 against 254); at 64 - 140 rows they are level.
-// Measured in one process on six shapes (those, 8 experts of half the width, 4 of the same, down), 19 row counts, equal
-// experts, random tokens and experts 0.6 - 1.4 of the mean: where the four-wave kernel is chosen it takes 0.755 - 1.04 of the
-// ping-pong kernel's time (1.11 at 240 - 256 equal rows of 8 x 28672 x 4096).
+// Measured in one process on six shapes (those, 8 experts of half the width, 4 of the same, 64 x 2816 x 2048), 16 row counts,
+// equal experts, random tokens, experts 0.6 - 1.4 of the mean and one with two fifths: where the four-wave kernel is chosen it
+// is 19 % faster than the ping-pong kernel on average, slower at 7 of 320 points and by 8 % at worst (8 x 28672 x 4096 at 240 -
+// 256 equal rows by 3 - 4 % there, by 11 % in a run before).
 static Plan grouped_plan(int M, int N, int K, int n_groups, int max_rows, int a_n) {
   Plan p = plan(M, N, K, true, n_groups, max_rows);
   const bool quadrants = max_rows >= 160 && max_rows < 240 && n_groups <= 8;

@@ -774,13 +774,15 @@ bool gemm_w4_ok(int M, int N, int K, int lda, int ldb, int ldc) {
          (long)M * lda * 2 < (1l << 31) && (long)N * ldb * 2 < (1l << 31) && (long)M * (ldc > 0 ? ldc : N) * 2 < (1l << 31);
 }
 
-// Each XCD's K walk from another eighth on (XCD x from eighth k_walk x mod 8; 0: all in step): where rows are a multiple of 4 KB apart, tiles in step ask for the same few
-// memory channels.  Not where XCDs share weights (several bands of tiles a round) that the 256 MB cache behind the L2s
-// does not hold: out of step each of them reads HBM.  Cold weights, M 1024 - 6000 (us): 16384 x 16384 1150 -> 1114 at 3000 rows,
-// 8192 x 14336 325 -> 317 at 2048, 8192 x 8192 179 -> 176, 28672 x 4096 640 -> 630 at 4096; without the first condition 5120 x
-// 13824 is 1.5 % slower at 1024 - 3000 rows and 2.5 % faster above, without the second 8192 x 28672 4 % slower, 8192 x
-// 20480 3 %.  In a step (Llama-3-8B widths) o and down together 105 -> 99 us each at 1500 rows, 415 -> 402 at 8000.
-// Neighbours five eighths apart: 0.5 - 1.5 % of a step better than one apart at 1500 rows and in mixed steps, level elsewhere.
+// Each XCD's K walk from another eighth on (XCD x from eighth k_walk x mod 8; 0: all in step): where rows are a multiple of
+// 4 KB apart, tiles in step ask for the same few memory channels.  Not where XCDs share weights (several bands of tiles a
+// round) that the 256 MB cache behind the L2s does not hold: out of step each of them reads HBM.  Cold weights, 21 shapes at
+// 640 - 7000 rows: where the rule walks apart 0.992 of the time in step (0.91 - 1.03; 16384 x 16384 0.94 - 0.97, 8192 x 14336
+// at 1500 - 2300 rows 0.92, 12288 x 4096 at 1500 and 8192 x 8192 at 1500 the worst); the shapes that the first condition
+// leaves out 0.998 (0.97 - 1.04), those of the second 0.92 - 1.0 at up to 2300 rows and 1.02 - 1.03 above (8192 x 28672 and
+// x 20480; one line, since few steps have such weights at few rows).  In a step (Llama-3-8B widths) o and down together 105 ->
+// 99 us each at 1500 rows, 415 -> 402 at 8000.  Neighbours five eighths apart: 0.5 - 1.5 % of a step better than one apart
+// at 1500 rows and in mixed steps, level elsewhere and in products alone.
 static int w4_k_walk(int N, int K, int band_tiles, int cus) {
   return K % 2048 == 0 && ((long)N * K * 2 <= (256l << 20) || band_tiles >= cus) ? 5 : 0;
 }
@@ -858,9 +860,10 @@ static void run_w4_grouped_t(const uint16_t* A, int lda, const uint16_t* B, int 
   const long most = (long)(N / 256) * ((M + 159) / 160 + n_groups);  // every expert's last tile partial
   RopeEpi re2 = re;
   re2.ws_nt = gemm_slab_nt(-1);
-  // (an expert's column tiles are walked by one XCD: no condition as in w4_k_walk.  Steps of three Mixtral layers, neighbours
-  // five eighths apart for one: 1500 / 1800 tokens, 375 / 450 rows per expert, 3761 -> 3674, 4144 -> 4076 us, two prompts of 900
-  // 3769 -> 3690; level at 525 rows, at 900 - 1500 7576 -> 7624, 12059 -> 12156)
+  // (an expert's column tiles are walked by one XCD: no condition as in w4_k_walk.  Seven shapes of 4 - 32 experts, 260 - 500 rows
+  // each, equal and random: neighbours five eighths apart take 0.98 of the time of one eighth apart (0.92 - 1.02), 560 - 1500
+  // rows 0.995 (0.96 - 1.016).  Steps of three Mixtral layers: 1500 / 1800 tokens, 375 / 450 rows per expert, 3761 -> 3674,
+  // 4144 -> 4076 us, two prompts of 900 3769 -> 3690; at 900 - 1500 rows 7576 -> 7624, 12059 -> 12156, so one apart there.)
   re2.k_walk = M <= 512l * n_groups ? 5 : 1;
   kern<<<(int)std::min<long>(most, cus), 256, lds, st>>>(A, lda, B, ldb, C, ldc, M, N, K, N / 256, re2, ws, cnt, offsets,
                                                           n_groups);
