@@ -176,7 +176,7 @@ __device__ __forceinline__ void combine_parts(const float* part_o, const float* 
   for (int j = 0; j < 4; ++j) ov[j] = pack2(a[2 * j] * inv, a[2 * j + 1] * inv);
 }
 
-template <int G, int NT>  // NT bit 0: K / V loads non-temporal, bit 1: the output stores
+template <int G, int NT, bool BY_HEAD>  // NT bit 0: K / V loads non-temporal, bit 1: the output stores
 __global__ void __launch_bounds__(256, 3) paged_attn_kernel(
     uint16_t* __restrict__ out, float* __restrict__ part_o, float* __restrict__ part_ml,
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ kc,
@@ -184,7 +184,7 @@ __global__ void __launch_bounds__(256, 3) paged_attn_kernel(
     const int* __restrict__ tile_seq, const int* __restrict__ tile_q0,
     const int* __restrict__ q_start, const int* __restrict__ q_len,
     const int* __restrict__ ctx_len, int Hq, int Hkv, float scale_log2, int part_tokens,
-    int nparts, int even, int num_blocks, int tiles, int* __restrict__ sem) {
+    int nparts, int even, int num_blocks, int* __restrict__ sem) {
   constexpr int QT = 16 / G;
   // (3 waves per SIMD: 154 VGPRs; asked for two fewer the compiler keeps O in AGPRs and copies it for every rescale)
   // wave w stages its page pair's V image (2 x 16 token rows x 256 B = 8 KB) inside sm_o[w]
@@ -195,25 +195,14 @@ __global__ void __launch_bounds__(256, 3) paged_attn_kernel(
   __shared__ float sm_l[4][16];
   __shared__ int sm_last;
 
-  // From 32 tiles of 8 kv heads on the heads are the fastest index: a page holds the heads' 4-KB blocks one behind the other,
-  // and whatever workgroups run at a time read them all.  With tiles fastest a launch ended on two heads, a quarter of every page (a
-  // step of 40 x 8000 keys 2620 -> 2518 us, 48 x 7000 2472 -> 2408, 200 x 1500 2562 -> 2507, 700 x 500 4119 -> 4084).  Fewer heads are
-  // less of a page's stripes than that anyhow, and one tile's heads end together: 2 and 4 heads (a tensor-parallel
-  // shard's) lose 1 - 3 % at 24 - 200 tiles on average and 8 % at worst (4 heads, 36 tiles of 4000 keys 64.4 -> 68.1 us), and gain
-  // 1 - 5 % from 250 - 300 on.  Kernel times by heads fastest over tiles fastest, contexts of 500 - 20000, means over 4 - 24
-  // launches: 8 heads 1.00 at 24 tiles, 0.99 at 28, 1.01 / 0.98 / 0.96 / 0.94 / 0.96 at 32 / 40 / 64 / 80 / 150, 1.02 at 300 - 700; 16 and 32 heads
-  // 0.97 - 1.0 from 32 on; 4 heads 1.02 / 1.02 / 1.01 / 0.98 / 0.95 at 32 / 64 / 150 / 300 / 700.  A few long sequences in shares
-  // lose a little too: steps of 8 x 20000 1388 -> 1400, 13 x 2056 937 -> 940.
-  const bool by_head = Hkv > 1 && tiles >= (Hkv >= 8 ? 32 : 256);
-  const int lin = blockIdx.x + tiles * blockIdx.y, part = blockIdx.z;
-  const int tile = by_head ? lin / Hkv : blockIdx.x, kvh = by_head ? lin % Hkv : blockIdx.y;
+  const int tile = BY_HEAD ? blockIdx.y : blockIdx.x, kvh = BY_HEAD ? blockIdx.x : blockIdx.y, part = blockIdx.z;
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   const int s = tile_seq[tile], q0 = tile_q0[tile];
   const int* bt = block_tables + (size_t)s * bt_stride;
   const int ql = q_len[s], ctx = ctx_len[s], qs = q_start[s];
   const int last_q = min(q0 + QT, ql) - 1;           // last valid query of the tile
   const int kv_end = last_q >= 0 ? ctx - ql + last_q + 1 : 0;
-  part_tokens = seq_part(kv_end, part_tokens, nparts, even, tile_seq, ctx_len, tiles, Hkv);
+  part_tokens = seq_part(kv_end, part_tokens, nparts, even, tile_seq, ctx_len, BY_HEAD ? gridDim.y : gridDim.x, Hkv);
   const int p_begin = part * part_tokens;
   const int p_end = min(kv_end, p_begin + part_tokens);
   if (p_begin >= p_end) {                            // reducer skips empty partitions
@@ -528,14 +517,30 @@ static void launch_g(void* out, float* part_o, float* part_ml, const void* q, co
     if (even == 1 && nparts > 1) part_tokens = 1 << 30;  // the only partition has all keys, whatever was planned
     nparts = even;
   }
-  dim3 grid(num_tiles, Hkv, nparts);
+  // Above 32 tiles of 8 kv heads the heads are the grid's fastest index: a page holds the heads' 4-KB blocks one behind the
+  // other, and whatever workgroups run at a time read them all.  With tiles fastest a launch ended on two heads, a quarter of
+  // every page (a step of 40 x 8000 keys 2620 -> 2518 us, 48 x 7000 2472 -> 2408, 200 x 1500 2562 -> 2507, 700 x 500 4119 -> 4084).
+  // 32 tiles of 8 heads are one workgroup per CU, no order to gain from (32 x 800 23.5 us, heads fastest 23.9).  Fewer heads are
+  // less of a page than that anyhow, and one tile's heads end together: 2 and 4 heads (a tensor-parallel shard's) lose 1 -
+  // 3 % at 24 - 200 tiles on average and 8 % at worst (4 heads, 36 tiles of 4000 keys 63.0 -> 67.0 us), and gain 1 - 5 % from 250 -
+  // 300 on.  Kernel times by heads fastest over tiles fastest, contexts of 500 - 20000, means over 4 - 24 launches: 8 heads 1.00
+  // at 24 tiles, 0.99 at 28, 1.01 / 0.97 / 0.98 / 0.96 / 0.94 / 0.96 at 32 / 36 / 40 / 64 / 80 / 150, 1.02 at 300 - 700 of equal lengths
+  // and 0.99 of unequal ones; 16 and 32 heads 0.97 - 1.0 from 32 on; 4 heads 1.02 / 1.02 / 1.01 / 0.98 / 0.95 at 32 / 64 / 150 / 300 /
+  // 700.  A kernel of its own for each order: chosen inside, by a division of the linear index, it cost every launch 0.2 us
+  // (7 x 1000 keys 12.05 -> 12.3).
+  const bool by_head = Hkv > 1 && num_tiles >= (Hkv >= 8 ? 33 : 256) && num_tiles <= 65535;  // (the grid's second dimension)
+  const dim3 grid = by_head ? dim3(Hkv, num_tiles, nparts) : dim3(num_tiles, Hkv, nparts);
   // K / V pages non-temporal (attn_kv_nt op): each is read once per step by one workgroup
   // (below 8 query tiles the default policy: batch 4 lost 0.7 % with it, batch 16 gained 1.8 %)
   const int nt = num_tiles >= 8 ? g_attn_kv_nt : 0;
-  auto kern = nt == 3 ? paged_attn_kernel<G, 3> : nt ? paged_attn_kernel<G, 1> : paged_attn_kernel<G, 0>;
+  auto pick = [&](auto h) {
+    constexpr bool H = decltype(h)::value;
+    return nt == 3 ? paged_attn_kernel<G, 3, H> : nt ? paged_attn_kernel<G, 1, H> : paged_attn_kernel<G, 0, H>;
+  };
+  auto kern = by_head ? pick(std::true_type{}) : pick(std::false_type{});
   kern<<<grid, 256, 0, st>>>((uint16_t*)out, part_o, part_ml, (const uint16_t*)q, (const uint16_t*)kc,
                              (const uint16_t*)vc, bt, bt_stride, tile_seq, tile_q0, q_start, q_len, ctx_len,
-                             Hq, Hkv, scale_log2, part_tokens, nparts, even, num_blocks, num_tiles, sem);
+                             Hq, Hkv, scale_log2, part_tokens, nparts, even, num_blocks, sem);
   if (nparts > 1 && sem == nullptr) {
     attn_reduce_kernel<G><<<dim3(num_tiles, Hkv), 256, 0, st>>>(
         (uint16_t*)out, part_o, part_ml, tile_seq, tile_q0, q_start, q_len, ctx_len, Hq, Hkv,

@@ -297,7 +297,7 @@ def test_paged_attention_one_sequence_many_kv_heads(gpu, Hkv, ctx, attn_fused_al
     close(ops.paged_attention(q, kc, vc, m), ref.paged_attention(q, kc, vc, m), atol=2e-2, rtol=2e-2)
 
 
-@pytest.mark.parametrize("Hq,Hkv,tiles", [(32, 8, 31), (32, 8, 32), (16, 16, 33), (8, 2, 32), (16, 4, 255), (16, 4, 256), (8, 2, 257),
+@pytest.mark.parametrize("Hq,Hkv,tiles", [(32, 8, 32), (32, 8, 33), (16, 16, 33), (8, 2, 32), (16, 4, 255), (16, 4, 256), (8, 2, 257),
                                           (28, 7, 256), (4, 1, 256)])
 def test_paged_attention_tile_and_head_order(gpu, Hq, Hkv, tiles, attn_fused_all):
     """Where the launch's fastest index turns from the tiles to the kv heads, whole and in shares."""
