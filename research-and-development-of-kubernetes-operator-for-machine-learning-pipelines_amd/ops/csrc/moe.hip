@@ -584,8 +584,9 @@ void launch_moe_dispatch_small_sigmoid(float* topw, int* topi, void* xp, int* of
 //     order and co-residency are not assumed) counts the T*k slots per local expert and writes
 //     offsets, inv (slot -> permuted row) and arow (permuted row -> token row).
 // There is no gathered copy: the grouped gate_up GEMM reads x rows through arow.  Rows inside
-// an expert come in ticket order (LDS atomics), which changes no value: each row's product is
-// independent of its position and the combine gathers by inv.
+// an expert come in ticket order (LDS atomics): the combine gathers by inv, and a row's product is
+// the same sum wherever the row stands, in fp32 and in an order that on the large tiles hangs on its
+// tile (K-halves, the XCDs' K walks): the last bit may differ from call to call.
 constexpr int kMidT = 16384;
 static int g_mid_max_t = kMidT;  // moe_mid_max_tokens op: in-process A/B of the range
 // moe_mid_tok op: tokens per workgroup (2, 4 or 8; the router row is loaded once per

@@ -199,7 +199,7 @@ class Sequence:
 def fill_buckets(listed) -> list[int]:
     """Decode graph sizes: the listed ones and, between neighbours at most a factor of two apart, those
     where a step becomes cheaper.  A graph's products compute all of its rows: of Llama-3-8B's widths
-    (6 layers, contexts of 500) 700 sequences take 4117 us in a graph of 704 rows and 4781 in one of
+    (6 layers, contexts of 500) 700 sequences take 4150 us in a graph of 704 rows and 4781 in one of
     1024, 300 take 2193 in 320 and 2634 in 512, 150 take 1431 in 160 and 1683 in 256, 90 take 1139 in 96
     and 1221 in 128, 40 take 982 in 48 and 1016 in 64; 20 take the same in 24 as in 32, so nothing is
     added there.  The weight stream's tiles grow by 32 rows (by 16 where the weights alone count), large

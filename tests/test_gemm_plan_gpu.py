@@ -101,9 +101,9 @@ def test_small_tile_switch(gpu, M, N):
         torch.ops.mlop.gemm_small_tile(prev)
 
 
-@pytest.mark.parametrize("bm,rows", [(-1, 128), (0, 128), (64, 128), (128, 128), (160, 160), (192, 192), (256, 128)])
+@pytest.mark.parametrize("bm,rows", [(-1, 128), (0, 128), (64, 128), (128, 128), (160, 160), (192, 192), (224, 224), (256, 128)])
 def test_four_wave_override(gpu, bm, rows):
-    """Variant 6 takes any tile height, as ever: the two between as they are, the half height for all others."""
+    """Variant 6 takes any tile height, as ever: the three between as they are, the half height for all others."""
     ops._sk_reserve(torch.device(gpu))
     x = torch.randn(300, 256, device=gpu, dtype=bf)
     w = (0.05 * torch.randn(512, 256, device=gpu)).to(bf)
