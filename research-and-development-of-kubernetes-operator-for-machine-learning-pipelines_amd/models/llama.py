@@ -161,7 +161,7 @@ class LlamaModel:
         residual = h
         M = ids.shape[0]
         # TP > 1: the decode (GEMV) form only, its residual adds riding in the all-reduces
-        dmax = ops.decode_chain_max_m()  # the GEMV (<= 4 rows) / weight-streaming MFMA (<= 64) forms
+        dmax = ops.decode_chain_max_m() if tp.size == 1 else ops.GEMV_CHAIN_MAX_M  # the GEMV / weight-streaming MFMA forms
         chain = (tp.size == 1 or M <= dmax) and self._chain_ok(M, meta.like)
         ss = None  # norm chain: x is None and ss holds the residual's row partials
         if chain and M <= dmax:

@@ -509,8 +509,8 @@ GEMV_CHAIN_MAX_M = 4  # = gemv.hip gemv_chain_max_m (the GEMV form; the torch re
 
 
 def decode_chain_max_m() -> int:
-    """Rows the decode form of the norm chain takes: the GEMV up to 4 rows, then the
-    weight-streaming MFMA kernel (gemm_ws.hip) up to ``gemm_ws_max_m`` (64; the
+    """Rows the decode form of the norm chain takes: the GEMV up to 4 rows and the
+    weight-streaming MFMA kernel (gemm_ws.hip) up to ``gemm_ws_max_m`` (16; the
     ``gemm_ws_max_m`` op is its A/B switch).  Without the extension (CPU): the GEMV bound."""
     if _loaded:
         return int(torch.ops.mlop.decode_chain_max_m())

@@ -380,6 +380,12 @@ static void check_ss(const Tensor& ss, int64_t M, int64_t H, const char* name) {
                   ss.numel() == M * (H / 128 + 1), name, " must be f32 [M * (H / 128 + 1)] contiguous");
 }
 
+// sizes of the decode form of the chain: the GEMV's rows, and above them what the weight-streaming kernel takes
+static bool decode_form(int64_t M, int64_t N, int64_t K, int64_t epi) {
+  return M <= mlop::gemv_chain_max_m() ||
+         (M <= mlop::decode_chain_max_m() && mlop::decode_chain_takes((int)M, (int)N, (int)K, (int)epi));
+}
+
 bool gemm_res_ss(Tensor residual, Tensor a, Tensor w, Tensor ss_out, bool any) {
   TORCH_CHECK(a.is_cuda() && a.scalar_type() == at::kBFloat16 && a.dim() == 2 && a.stride(1) == 1 &&
                   a.stride(0) % 8 == 0, "a must be bf16 [M, K], 16-B aligned rows");
@@ -390,11 +396,11 @@ bool gemm_res_ss(Tensor residual, Tensor a, Tensor w, Tensor ss_out, bool any) {
                   residual.stride(0) % 8 == 0, "residual [M, N]");
   TORCH_CHECK(N % 128 == 0, "N % 128");
   check_ss(ss_out, M, N, "ss");
-  if (M <= mlop::decode_chain_max_m()) {  // decode sizes: the GEMV (M <= 4) / weight-streaming MFMA chain
+  if (decode_form(M, N, K, 0)) {  // the GEMV / weight-streaming MFMA chain
                  // (EPI_RES); its consumers take their row factors from the residual itself, so ss_out is not written
     if (residual.stride(0) != N || !mlop::decode_chain_takes((int)M, (int)N, (int)K, 0)) return false;
     c10::DeviceGuard g(a.device());
-    if (M <= mlop::gemv_chain_max_m())
+    if (!mlop::chain_on_ws((int)M, (int)N, (int)K, 5))
       mlop::launch_gemv_res(a.data_ptr(), (int)a.stride(0), w.data_ptr(), residual.data_ptr(), (int)M, (int)N,
                             (int)K, cur_stream());
     else
@@ -426,10 +432,10 @@ bool gemm_rs(Tensor out, Tensor a, Tensor w, Tensor ss_in, double eps, int64_t e
                   out.stride(0) % 8 == 0, "out [M, N or N/2]");
   TORCH_CHECK(K % 128 == 0, "K % 128");
   check_ss(ss_in, M, K, "ss");
-  if (M <= mlop::decode_chain_max_m()) {  // decode sizes: PRO_RS, row factors from the streamed chunks (ss_in unused)
+  if (decode_form(M, N, K, epi)) {  // PRO_RS, row factors from the streamed chunks (ss_in unused)
     if (!mlop::decode_chain_takes((int)M, (int)N, (int)K, (int)epi)) return false;
     c10::DeviceGuard g(a.device());
-    if (M <= mlop::gemv_chain_max_m())
+    if (!mlop::chain_on_ws((int)M, (int)N, (int)K, (int)epi))
       mlop::launch_gemv_rs(a.data_ptr(), (int)a.stride(0), w.data_ptr(), out.data_ptr(), (int)out.stride(0), (int)M,
                            (int)N, (int)K, (int)epi, mlop::RopeEpi{}, (float)eps, cur_stream());
     else
@@ -471,10 +477,10 @@ bool gemm_rs_rope(Tensor q_out, Tensor k_cache, Tensor v_cache, Tensor a, Tensor
   mlop::RopeEpi re{(uint16_t*)q_out.data_ptr(), (uint16_t*)k_cache.data_ptr(),
                    (uint16_t*)v_cache.data_ptr(), pos.data_ptr<int>(), cos_sin.data_ptr<float>(),
                    slots.data_ptr<int>(), (int)Hq, (int)Hkv, (int)BS};
-  if (M <= mlop::decode_chain_max_m()) {  // decode sizes: PRO_RS + the RoPE / paged K/V epilogue (ss_in unused)
+  if (decode_form(M, N, K, 3)) {  // PRO_RS + the RoPE / paged K/V epilogue (ss_in unused)
     if (!mlop::decode_chain_takes((int)M, (int)N, (int)K, 3)) return false;
     c10::DeviceGuard g(a.device());
-    if (M <= mlop::gemv_chain_max_m())
+    if (!mlop::chain_on_ws((int)M, (int)N, (int)K, 3))
       mlop::launch_gemv_rs(a.data_ptr(), (int)a.stride(0), w.data_ptr(), nullptr, 0, (int)M, (int)N, (int)K, 3, re,
                            (float)eps, cur_stream());
     else

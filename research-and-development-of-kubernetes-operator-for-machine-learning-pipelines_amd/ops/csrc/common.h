@@ -29,6 +29,15 @@ __device__ __forceinline__ void raw_barrier() {
   asm volatile("" ::: "memory");
 }
 
+// One LDS-DMA instruction (16 B per lane to lds + 16 lane) in its buffer form.  The global form counts as a flat access, behind
+// which the compiler waits for every load in flight (vmcnt(0)) before it uses a register of any of them; this one it counts.
+__device__ __forceinline__ void lds_dma16(__amdgpu_buffer_rsrc_t rs, uint32_t lds, uint32_t offset, int aux_nt) {
+#ifdef __HIP_DEVICE_COMPILE__
+  if (aux_nt) __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void_t*)(uintptr_t)lds, 16, offset, 0, 0, 2);
+  else __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void_t*)(uintptr_t)lds, 16, offset, 0, 0, 0);
+#endif
+}
+
 template <int N>
 __device__ __forceinline__ void wait_vmcnt() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");

@@ -1712,7 +1712,7 @@ static bool rope_tiles(const Plan& p) { return p.variant != 7 && (p.BM == 256 ||
 
 bool gemm_rope_supported(int M, int N, int K) {
   if (M <= 0 || N % 128 || K % kBK) return false;
-  if (gemv_takes(M, N, K, EPI_ROPE)) return true;  // decode M <= 8: gemv.hip
+  if (gemv_takes(M, N, K, EPI_ROPE) || ws_prefer(M, N, K, EPI_ROPE)) return true;  // decode: gemv.hip, gemm_ws.hip
   const Plan p = rope_plan(M, N, K);
   return rope_tiles(p) || rope_slabs_ok(p, M, N);
 }
@@ -1721,12 +1721,12 @@ bool launch_gemm_rope(const void* A, int lda, const void* B, int M, int N, int K
                       hipStream_t st) {
   if (M == 0) return true;
   if (!gemm_rope_supported(M, N, K)) return false;
-  if (gemv_takes(M, N, K, EPI_ROPE) && lda % 8 == 0) {
-    launch_gemv_rope(A, lda, B, M, N, K, re, st);
+  if (ws_prefer(M, N, K, EPI_ROPE) && lda % 8 == 0) {  // up to 16 rows: the weight-streaming MFMA kernel
+    launch_ws(A, lda, B, K, nullptr, 0, M, N, K, EPI_ROPE, false, re, 0.f, st);
     return true;
   }
-  if (ws_prefer(M, N, K, EPI_ROPE) && lda % 8 == 0) {  // 5-16 rows: the weight-streaming MFMA kernel
-    launch_ws(A, lda, B, K, nullptr, 0, M, N, K, EPI_ROPE, false, re, 0.f, st);
+  if (gemv_takes(M, N, K, EPI_ROPE) && lda % 8 == 0) {
+    launch_gemv_rope(A, lda, B, M, N, K, re, st);
     return true;
   }
   Plan p = rope_plan(M, N, K);
@@ -1882,6 +1882,10 @@ void launch_gemm(const void* A, int lda, const void* B, int ldb, void* C, int ld
   re.act = epi_act(epi);
   const int epi0 = epi;
   if (re.act) epi = EPI_NONE;
+  if (ws_prefer(M, N, K, epi) && lda % 8 == 0 && ldb % 8 == 0) {
+    launch_ws(A, lda, B, ldb, C, ldc, M, N, K, epi, false, re, 0.f, st);
+    return;
+  }
   if (gemv_takes(M, N, K, epi) && lda % 8 == 0 && ldb % 8 == 0) {
     launch_gemv(A, lda, B, ldb, C, ldc, M, N, K, epi0, st, p0, p1, act_n0);
     return;
@@ -1914,7 +1918,7 @@ bool launch_gemm_add_rmsnorm(const void* A, int lda, const void* B, void* out, v
   if (M == 0) return true;
   if (gemv_takes(M, N, K, EPI_NONE)) return false;  // decode sizes: GEMV + add_rmsnorm (or the norm chain)
   if (ws_prefer(M, N, K, EPI_NONE) && lda % 8 == 0) {
-    // 5-16 rows of an O-size projection: the weight-streaming MFMA kernel adds into the residual
+    // up to 16 rows: the weight-streaming MFMA kernel adds into the residual
     // in place (bf16(res + bf16(y)), norm.hip's rounding), then one RMSNorm pass
     launch_ws(A, lda, B, K, residual, N, M, N, K, 5, false, RopeEpi{}, 0.f, st);
     launch_rmsnorm(out, residual, w, eps, M, N, st);

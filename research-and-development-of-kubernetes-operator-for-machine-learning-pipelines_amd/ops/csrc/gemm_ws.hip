@@ -1,32 +1,36 @@
-// K2 at 5-64 rows (batch 5-64 decode): the weight-streaming MFMA GEMM.
+// K2 at 1-16 rows (decode of up to 16 sequences, the head of a prompt): the weight-streaming MFMA GEMM.
 //
 //   C[M, N] = A[M, K] . B[N, K]^T      (A activations, B weights [out, in], both bf16)
 //
-// Between the GEMV (gemv.hip, M <= 4: dot2 on VALU) and the LDS-ring MFMA tiles (gemm.hip),
-// a decode projection at 5-64 rows is still pure weight streaming (every weight byte read once,
-// ~M / 2 FLOP per byte), but too many dot products for the VALU.  This kernel keeps the GEMV's
-// structure -- many waves, each streaming its weight rows straight into registers with
-// non-temporal 16-B loads, several K-steps in flight, no LDS ring, no split-K slabs -- and
-// does the arithmetic on the matrix cores:
-//   * one workgroup = 16 x RB weight rows over the WHOLE K; its 4 waves take one K quarter
-//     each (LDS combine at the end), so even O (N = 4096) runs 1024 streaming waves;
-//   * a wave's B fragment of one K-step IS the MFMA operand: lane l loads 16 B of weight row
-//     (l & 15) at k-chunk (l >> 4) (v_mfma_f32_16x16x32_bf16 B layout, common.h), 16 rows x
-//     64 contiguous B per load, the next step continuing the same rows; A fragments come the
-//     same way through the cached path (A is a few hundred KiB, L2-resident);
-//   * U K-steps in flight per wave (a U-slot register ring: step s's slot is reloaded with
-//     step s + U right after its MFMAs), MT = ceil(M / 16) MFMAs per weight fragment.
-// Epilogues (the decode norm chain of gemv.hip, so a layer has no add + RMSNorm launch):
-//   WS_NONE      bf16 store;
+// What bounds it: every weight byte comes from HBM once, at 6.8 TB/s at best; at 4 rows a CU also takes in A once for every
+// 16 weight rows.  Between the GEMV (gemv.hip: a quarter of its time at 4 rows is dot products) and the LDS-ring tiles (gemm.hip:
+// K ranges whose fp32 sums a second launch adds) this kernel keeps the GEMV's way of loading and multiplies on the matrix cores:
+//   * a workgroup has 16 (or 32) weight rows over the WHOLE K; its 8 waves take steps of 128 k in turn and meet in LDS once,
+//     at the end: no slabs, no second launch, and the epilogue has whole sums;
+//   * weights go straight to registers, non-temporal, one load instruction 8 rows x 128 B (whole lines).  The MFMA wants
+//     16 rows from it: its row v holds the chunks 2 g + (v & 1) of weight row v / 2, is multiplied with the even and with the odd
+//     chunks of A, and the halves that belong together are added at the end.  Twice the MFMAs, of which a CU has ten times what the
+//     stream needs; 16 rows x 64 B per instruction, each line in two halves, ran at 6.3 TB/s instead of 6.8 (gate_up of
+//     Llama-3-8B, weights alone: 37.3 -> 34.7 us), and needed the cached path;
+//   * A comes as a wave-private LDS image per step, by LDS-DMA of 4 rows x 256 B.  As MFMA fragments straight from memory its
+//     16-B pieces of 16 rows cost a lookup each: 28672 x 4096 at 16 rows 55.8 -> 41.9 us, 4096 x 14336 28.8 -> 24.3;
+//   * workgroups start their walk of K at steps that differ.  Rows are a multiple of 4 KB apart: in step they ask the same few
+//     channels (28672 x 4096, 32 rows per workgroup, 50.6 -> 38.7 us; 16 rows 37.6 -> 36.3).
+// What is left: at 16 rows 4096 x 14336 takes 22.9 us, with half of A's image 19.8: weights and A share what a CU can have in
+// flight.  The epilogue is 0.8 us of a launch of one workgroup per CU.  Tried and slower: A kept in registers for all tiles of a
+// workgroup (28672 x 4096 39.5 us), four steps in flight (VGPRs for one workgroup fewer), 4 or 16 waves.
+// Epilogues (the decode norm chain, so that a layer has no add + RMSNorm launch):
+//   WS_NONE      bf16 store (with an activation, RopeEpi::act);
 //   WS_RES       residual (C) += y in place, bf16(res + bf16(y)) (norm.hip's add rounding);
-//   WS_SILU_MUL  RB = 2: rows 32b.. (gate) and 32b+16.. (up) of the 16-interleaved gate_up;
-//   WS_ROPE      RB = 2: a q / k head's rotate-half row pair blocks (d, d + 64), rotated and
-//                stored to q_out / the paged K cache; V rows straight into their page rows;
-// prologue RS (QKV / gate_up of the chain, norm weights folded into B): A is the raw
-// residual; each row's sum of squares accumulates from the very A fragments the MFMAs read
-// (4 v_dot2 per fragment) and rsqrt(mean + eps) scales the finished sums.
+//   WS_SILU_MUL  gate rows 32b.. and their up rows 32b+16.. of the 16-interleaved gate_up;
+//   WS_ROPE      a q / k head's rotate-half rows (d, d + 64), rotated and stored to q_out / the paged K cache; V rows straight
+//                into their page rows;
+// prologue RS (QKV / gate_up of the chain, norm weights folded into B): A is the raw residual; each row's sum of squares
+// accumulates from the fragments the MFMAs read and rsqrt(mean + eps) scales the finished sums.
 #include "common.h"
 #include "launch.h"
+
+#include <type_traits>
 
 namespace mlop {
 
@@ -41,227 +45,305 @@ __device__ __forceinline__ float ws_dot2(uint32_t a, uint32_t b, float c) {
                                         false);
 }
 
-__device__ __forceinline__ float ws_sq8(const bf16x8& v, float c) {
-  const u32x4 w = __builtin_bit_cast(u32x4, v);
+__device__ __forceinline__ float ws_sq8(const u32x4& w, float c) {
   c = ws_dot2(w.x, w.x, c);
   c = ws_dot2(w.y, w.y, c);
   c = ws_dot2(w.z, w.z, c);
   return ws_dot2(w.w, w.w, c);
 }
 
-template <int MT, int RB, int U, int EPI, bool RS, bool NT = true>
-__global__ void __launch_bounds__(256) gemm_ws_kernel(const uint16_t* __restrict__ A, int lda,
-                                                      const uint16_t* __restrict__ B, int ldb,
-                                                      uint16_t* __restrict__ C, int ldc, int M, int K,
-                                                      RopeEpi re, float eps) {
-  static_assert(EPI != WS_SILU_MUL || RB % 2 == 0, "gate / up row block pairs");
-  static_assert(EPI != WS_ROPE || RB == 2, "rotate-half row blocks");
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+// A fragments of one 16-row tile and step (256 B of every row): f[2 h + x] = chunk 8 h + 2 (lane >> 4) + x of row m, in the
+// image [row][16 x 16 B] with chunk c of row r at slot c ^ (r & 15).  `N`: vector memory operations younger than the image's.
+template <int N>
+__device__ __forceinline__ void ws_frags(uint32_t row, uint32_t x0, uint32_t x1, uint32_t x2, uint32_t x3, u32x4 (&f)[4]) {
+  asm volatile(
+      "s_waitcnt vmcnt(%8)\n"
+      "ds_read_b128 %0, %4\n"
+      "ds_read_b128 %1, %5\n"
+      "ds_read_b128 %2, %6\n"
+      "ds_read_b128 %3, %7\n"
+      "s_waitcnt lgkmcnt(0)"
+      : "=&v"(f[0]), "=&v"(f[1]), "=&v"(f[2]), "=&v"(f[3])
+      : "v"(row + x0), "v"(row + x1), "v"(row + x2), "v"(row + x3), "n"(N)
+      : "memory");
+}
+
+template <int AR, int G, int NW, int U, int EPI, bool RS>
+__global__ void __launch_bounds__(NW * 64) gemm_ws_kernel(const uint16_t* __restrict__ A, int lda,
+                                                          const uint16_t* __restrict__ B, int ldb,
+                                                          uint16_t* __restrict__ C, int ldc, int M, int K,
+                                                          RopeEpi re, float eps) {
+  static_assert(G % 2 == 0, "gate / up and rotate-half pairs of row groups");
+  static_assert(AR == 4 || AR == 8 || AR % 16 == 0, "rows of A staged");
+  constexpr int MT = (AR + 15) / 16, H2 = G / 2, T = NW * 64, D = 128;
+  constexpr int AI = AR / 4;            // LDS-DMA instructions (4 rows x 256 B) per step
+  constexpr int IMG = AR * 256;         // bytes of a step's A image
+  extern __shared__ __attribute__((aligned(256))) uint8_t ws_lds[];
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int blk = blockIdx.x;
-  constexpr int D = 128;
-  // first weight row of each of this workgroup's RB 16-row blocks
-  int rbase[RB];
+  // first weight row of the workgroup, and row group g's distance from it
+  int row0, far;  // groups 0 .. H2 - 1: row0 + 8 g; H2 .. G - 1: row0 + far + 8 (g - H2)
   bool rope_blk = false;
-  if constexpr (EPI == WS_SILU_MUL) {  // RB / 2 (gate, up) 16-row group pairs
-#pragma unroll
-    for (int g = 0; g < RB / 2; ++g) {
-      rbase[2 * g] = 32 * (blk * (RB / 2) + g);
-      rbase[2 * g + 1] = rbase[2 * g] + 16;
-    }
-  } else if constexpr (EPI == WS_ROPE) {
-    const int rope_blocks = (re.Hq + re.Hkv) * 4;  // 4 blocks of 16 dim pairs per q / k head
+  if constexpr (EPI == WS_SILU_MUL) {  // gate rows, and their up rows 16 further
+    row0 = H2 == 2 ? 32 * blk : 32 * (blk >> 1) + 8 * (blk & 1);
+    far = 16;
+  } else if constexpr (EPI == WS_ROPE) {  // a q / k head's dims d .. and d + 64 ..; plain v rows
+    constexpr int BPH = 8 / H2;  // workgroups per head
+    const int rope_blocks = (re.Hq + re.Hkv) * BPH;
     rope_blk = blk < rope_blocks;
-    if (rope_blk) {
-      rbase[0] = (blk >> 2) * D + (blk & 3) * 16;
-      rbase[1] = rbase[0] + D / 2;
-    } else {
-      rbase[0] = (re.Hq + re.Hkv) * D + (blk - rope_blocks) * 32;
-      rbase[1] = rbase[0] + 16;
-    }
+    row0 = rope_blk ? (blk / BPH) * D + (blk % BPH) * 8 * H2 : (re.Hq + re.Hkv) * D + (blk - rope_blocks) * 8 * G;
+    far = rope_blk ? D / 2 : 8 * H2;
   } else {
-#pragma unroll
-    for (int rb = 0; rb < RB; ++rb) rbase[rb] = blk * 16 * RB + 16 * rb;
+    row0 = blk * 8 * G;
+    far = 8 * H2;
   }
 
-  const int kq = K >> 2;                        // this wave's K quarter
-  const int k0 = wv * kq + (lane >> 4) * 8;     // + the lane's 8-element chunk of a 32-k step
-  const bf16x8* bp[RB];
-#pragma unroll
-  for (int rb = 0; rb < RB; ++rb)
-    bp[rb] = reinterpret_cast<const bf16x8*>(B + (size_t)(rbase[rb] + (lane & 15)) * ldb + k0);
-  const bf16x8* ap[MT];
-#pragma unroll
-  for (int t = 0; t < MT; ++t)  // rows past M read row M - 1: their outputs are never stored
-    ap[t] = reinterpret_cast<const bf16x8*>(A + (size_t)min(16 * t + (lane & 15), M - 1) * lda + k0);
+  // outputs of this thread: with one row tile, at most one (or one pair), whose old residual value, slot and position
+  // load ahead of the weights
+  constexpr int PAIR = EPI == WS_SILU_MUL || EPI == WS_ROPE, GO = PAIR ? H2 : G, OUTS = MT * 16 * GO * 8;
+  const int ot = threadIdx.x;
+  const int oj = ot & 7, og = (ot >> 3) % GO, om = ot / (8 * GO);
+  uint16_t res_pf = 0;
+  int pos_pf = 0, slot_pf = -1;
+  float cos_pf = 0.f, sin_pf = 0.f;
+  const bool out_pf = OUTS <= T && ot < OUTS && om < M;
+  if constexpr (EPI == WS_RES) {
+    if (out_pf) res_pf = C[(size_t)om * ldc + row0 + 8 * og + oj];
+  }
+  if constexpr (EPI == WS_ROPE) {
+    if (out_pf) {
+      slot_pf = re.slots[om];
+      pos_pf = re.pos[om];
+    }
+  }
 
-  f32x4 acc[MT][RB];
+  // Weight loads cover 8 rows x 128 B: MFMA row v = lane & 15 holds chunks 2 g4 + (v & 1) of row v >> 1, so two neighbouring
+  // lanes read 32 B, and a product with the even chunks of A counts for even v, one with the odd chunks for odd v.
+  const int v = lane & 15, g4 = lane >> 4;
+  const char* const Bw = reinterpret_cast<const char*>(B + (size_t)row0 * ldb);
+  uint32_t bo[G], ao[AI];
+#pragma unroll
+  for (int g = 0; g < G; ++g) bo[g] = (uint32_t)((g < H2 ? 8 * g : far + 8 * (g - H2)) + (v >> 1)) * ldb * 2 + g4 * 32 + (v & 1) * 16;
+#pragma unroll
+  for (int i = 0; i < AI; ++i) {  // (rows past M: the last one again, never stored)
+    const int r = 4 * i + g4;
+    ao[i] = (uint32_t)min(r, M - 1) * lda * 2 + ((v ^ (r & 15)) << 4);
+  }
+  // steps of 128 k (256 B of a row): the waves take them in turn, from one that differs by workgroup on
+  const int n_steps = K >> 7, rounds = n_steps / NW, rot = (blk >> 3) * 5 % n_steps;
+  // (a generic pointer's low 32 bits are the LDS offset)
+  const uint32_t img = (uint32_t)(uintptr_t)ws_lds + wv * (U * IMG);
+  const int mr16 = AR < 16 ? lane & (AR - 1) : v;
+  const uint32_t arow = img + mr16 * 256;
+  const uint32_t x0 = ((2 * g4) ^ mr16) << 4, x1 = ((2 * g4 + 1) ^ mr16) << 4, x2 = ((8 + 2 * g4) ^ mr16) << 4, x3 = ((9 + 2 * g4) ^ mr16) << 4;
+
+  f32x4 acc[MT][G][2];
 #pragma unroll
   for (int t = 0; t < MT; ++t)
 #pragma unroll
-    for (int rb = 0; rb < RB; ++rb) acc[t][rb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int g = 0; g < G; ++g) acc[t][g][0] = acc[t][g][1] = f32x4{0.f, 0.f, 0.f, 0.f};
   float ss[MT];
 #pragma unroll
   for (int t = 0; t < MT; ++t) ss[t] = 0.f;
 
-  // step s = 32 k: element offset 32 s = 4 s bf16x8 vectors
-  bf16x8 bq[U][RB], aq[U][MT];
+  u32x4 bq[U][2][G];
+  const auto rsA = __builtin_amdgcn_make_buffer_rsrc((void*)A, 0, ((M - 1) * lda + K) * 2, 0x00020000);
+  constexpr int OPS = AI + 2 * G;  // vector memory operations of a step
   auto load = [&](int u, int s) {
+    int p = s * NW + wv + rot;
+    p -= p >= n_steps ? n_steps : 0;
+    const uint32_t k = (uint32_t)p * 256;
 #pragma unroll
-    for (int rb = 0; rb < RB; ++rb) {
-      if constexpr (NT) bq[u][rb] = __builtin_nontemporal_load(bp[rb] + 4 * s);
-      else bq[u][rb] = bp[rb][4 * s];
-    }
+    for (int i = 0; i < AI; ++i)
+      lds_dma16(rsA, img + u * IMG + i * 1024, ao[i] + k, 0);
+    asm volatile("" ::: "memory");
 #pragma unroll
-    for (int t = 0; t < MT; ++t) aq[u][t] = ap[t][4 * s];
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int g = 0; g < G; ++g)
+        bq[u][h][g] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(Bw + (bo[g] + k + h * 128)));
+    asm volatile("" ::: "memory");
   };
-  auto consume = [&](int u) {
-#pragma unroll
-    for (int t = 0; t < MT; ++t)
-#pragma unroll
-      for (int rb = 0; rb < RB; ++rb) acc[t][rb] = mfma16(aq[u][t], bq[u][rb], acc[t][rb]);
-    if constexpr (RS) {
-#pragma unroll
-      for (int t = 0; t < MT; ++t) ss[t] = ws_sq8(aq[u][t], ss[t]);
-    }
-  };
-  // a multiple of U (ws_takes).  The steady-state body reloads unconditionally (a guarded
-  // reload made the compiler drain every load, vmcnt(0), at the top of each pass), so each
-  // slot's MFMAs wait only for that slot: vmcnt((U - 1) x loads per step)
-  const int steps = kq >> 5;
-#pragma unroll
-  for (int u = 0; u < U; ++u) load(u, u);
-  for (int s0 = 0; s0 < steps - U; s0 += U) {
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      consume(u);
-      load(u, s0 + u + U);
-    }
-  }
-#pragma unroll
-  for (int u = 0; u < U; ++u) consume(u);
-
-  // combine the 4 K quarters: red[w][(t RB + rb) 4 + r][lane]; RS: the row sums of squares
-  __shared__ float red[4][MT * RB * 4][64];
-  __shared__ float red_ss[4][MT][16];
-#pragma unroll
-  for (int t = 0; t < MT; ++t)
-#pragma unroll
-    for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) red[wv][(t * RB + rb) * 4 + r][lane] = acc[t][rb][r];
-  if constexpr (RS) {
+  // `younger`: steps loaded after this one
+  auto consume = [&](auto younger, int u) {
 #pragma unroll
     for (int t = 0; t < MT; ++t) {
-      const float v = sum_x16_x32(ss[t]);  // lanes l, l^16, l^32, l^48: the four k-chunks of row l & 15
-      if (lane < 16) red_ss[wv][t][lane] = v;
+      u32x4 f[4];
+      ws_frags<decltype(younger)::value * OPS + 2 * G>(arow + u * IMG + t * 4096, x0, x1, x2, x3, f);
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+#pragma unroll
+          for (int g = 0; g < G; ++g)
+            acc[t][g][x] = mfma16(__builtin_bit_cast(bf16x8, bq[u][h][g]), __builtin_bit_cast(bf16x8, f[2 * h + x]), acc[t][g][x]);
+          if constexpr (RS) ss[t] = ws_sq8(f[2 * h + x], ss[t]);
+        }
+    }
+  };
+  using Y0 = std::integral_constant<int, 0>;
+  auto load_cs = [&]() {
+    if constexpr (EPI == WS_ROPE) {
+      if (out_pf && rope_blk) {
+        const float* cs = re.cos_sin + (size_t)pos_pf * D + (row0 % D) + 8 * og + oj;
+        cos_pf = cs[0];
+        sin_pf = cs[D / 2];
+      }
+    }
+  };
+  int s0 = 0;
+  if (rounds >= U) {
+    // whole passes of the ring without a branch (behind a guarded load the compiler waits for all that are in flight)
+#pragma unroll
+    for (int u = 0; u < U; ++u) load(u, u);
+    load_cs();
+    for (; s0 + 2 * U <= rounds; s0 += U) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        consume(std::integral_constant<int, U - 1>{}, u);
+        load(u, s0 + U + u);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) consume(Y0{}, u);
+    s0 += U;
+  } else {
+    load_cs();
+  }
+  for (; s0 < rounds; ++s0) {
+    load(0, s0);
+    consume(Y0{}, 0);
+  }
+  if (wv < n_steps - rounds * NW) {
+    load(0, rounds);
+    consume(Y0{}, 0);
+  }
+  wait_vmcnt<0>();
+  __syncthreads();  // the images' space now takes the waves' sums
+
+  float (*red)[MT][G][16][8] = reinterpret_cast<float (*)[MT][G][16][8]>(ws_lds);
+  float (*red_ss)[MT][16] = reinterpret_cast<float (*)[MT][16]>(ws_lds + NW * MT * G * 512);
+#pragma unroll
+  for (int t = 0; t < MT; ++t) {
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      const float2 y = {acc[t][g][0][0] + acc[t][g][1][1], acc[t][g][0][2] + acc[t][g][1][3]};
+      *reinterpret_cast<float2*>(&red[wv][t][g][v][2 * g4]) = y;
+    }
+    if constexpr (RS) {
+      const float sum = sum_x16_x32(ss[t]);
+      if (lane < 16) red_ss[wv][t][lane] = sum;
     }
   }
   __syncthreads();
 
-  // thread (w', ln) finishes fragment element r = w' of every (t, rb) block: output row
-  // m = 16 t + 4 (ln >> 4) + r, weight row rbase[rb] + (ln & 15)
-  const int r = wv, ln = lane, col = ln & 15;
+#pragma unroll 1
+  for (int o = ot; o < OUTS; o += T) {
+    const int j = o & 7, g = (o >> 3) % GO, m = o / (8 * GO), t = m >> 4, mr = m & 15;
+    if (m >= M) return;
+    float y = 0.f, z = 0.f;
 #pragma unroll
-  for (int t = 0; t < MT; ++t) {
-    const int m = 16 * t + 4 * (ln >> 4) + r;
-    float y[RB];
-#pragma unroll
-    for (int rb = 0; rb < RB; ++rb) {
-      const int idx = (t * RB + rb) * 4 + r;
-      y[rb] = (red[0][idx][ln] + red[1][idx][ln]) + (red[2][idx][ln] + red[3][idx][ln]);
+    for (int w = 0; w < NW; ++w) {
+      y += red[w][t][g][mr][j];
+      if constexpr (PAIR) z += red[w][t][g + H2][mr][j];
     }
-    if (m >= M) continue;
     if constexpr (RS) {
-      const int mr = m & 15;
-      const float tot = (red_ss[0][t][mr] + red_ss[1][t][mr]) + (red_ss[2][t][mr] + red_ss[3][t][mr]);
-      const float inv = rsqrtf(tot / (float)K + eps);
+      float tot = 0.f;
 #pragma unroll
-      for (int rb = 0; rb < RB; ++rb) y[rb] *= inv;
+      for (int w = 0; w < NW; ++w) tot += red_ss[w][t][mr];
+      const float inv = rsqrtf(tot / (float)K + eps);
+      y *= inv;
+      z *= inv;
     }
     if constexpr (EPI == WS_SILU_MUL) {
-#pragma unroll
-      for (int g = 0; g < RB / 2; ++g)
-        C[(size_t)m * ldc + (blk * (RB / 2) + g) * 16 + col] = f2bf(glu_out(re, y[2 * g], y[2 * g + 1]));
+      C[(size_t)m * ldc + blk * 8 * H2 + 8 * g + j] = f2bf(glu_out(re, y, z));
     } else if constexpr (EPI == WS_ROPE) {
-      const int slot = re.slots[m];
+      const int slot = OUTS <= T ? slot_pf : re.slots[m];
       const int pblk = slot >= 0 ? slot / re.BS : 0, poff = slot >= 0 ? slot % re.BS : 0;
       if (rope_blk) {
-        const int h = rbase[0] / D, d = rbase[0] % D + col;  // d < 64
-        const float* cs = re.cos_sin + (size_t)re.pos[m] * D;
-        const float c = cs[d], s = cs[D / 2 + d];
-        const float x = bf2f(f2bf(y[0])), z = bf2f(f2bf(y[1]));
-        const uint16_t oa = f2bf(x * c - z * s), ob = f2bf(z * c + x * s);
+        const int hd = row0 / D, d = row0 % D + 8 * g + j;
+        float c = cos_pf, s = sin_pf;
+        if constexpr (OUTS > T) {
+          const float* cs = re.cos_sin + (size_t)re.pos[m] * D + d;
+          c = cs[0];
+          s = cs[D / 2];
+        }
+        const float x = bf2f(f2bf(y)), w = bf2f(f2bf(z));
+        const uint16_t oa = f2bf(x * c - w * s), ob = f2bf(w * c + x * s);
         uint16_t* dst;
-        if (h < re.Hq) {
-          dst = re.q_out + ((size_t)m * re.Hq + h) * D;
+        if (hd < re.Hq) {
+          dst = re.q_out + ((size_t)m * re.Hq + hd) * D;
         } else {
           if (slot < 0) continue;
-          dst = re.k_cache + (((size_t)pblk * re.Hkv + (h - re.Hq)) * re.BS + poff) * D;
+          dst = re.k_cache + (((size_t)pblk * re.Hkv + (hd - re.Hq)) * re.BS + poff) * D;
         }
         dst[d] = oa;
         dst[D / 2 + d] = ob;
       } else if (slot >= 0) {
-#pragma unroll
-        for (int rb = 0; rb < RB; ++rb) {
-          const int vr = rbase[rb] + col - (re.Hq + re.Hkv) * D;  // v row 0 .. Hkv * 128
-          re.v_cache[(((size_t)pblk * re.Hkv + vr / D) * re.BS + poff) * D + vr % D] = f2bf(y[rb]);
-        }
-      }
-    } else if constexpr (EPI == WS_RES) {
-#pragma unroll
-      for (int rb = 0; rb < RB; ++rb) {
-        uint16_t* p = C + (size_t)m * ldc + rbase[rb] + col;
-        *p = f2bf(bf2f(*p) + bf2f(f2bf(y[rb])));
+        const int vr = row0 - (re.Hq + re.Hkv) * D + 8 * g + j;  // v row 0 .. Hkv * 128, and the one far from it
+        uint16_t* v0 = re.v_cache + (((size_t)pblk * re.Hkv + vr / D) * re.BS + poff) * D + vr % D;
+        const int vz = vr + far;
+        v0[0] = f2bf(y);
+        re.v_cache[(((size_t)pblk * re.Hkv + vz / D) * re.BS + poff) * D + vz % D] = f2bf(z);
       }
     } else {
-#pragma unroll
-      for (int rb = 0; rb < RB; ++rb) C[(size_t)m * ldc + rbase[rb] + col] = f2bf(y[rb]);
+      uint16_t* p = C + (size_t)m * ldc + row0 + 8 * g + j;  // (plain rows: far = 8 H2)
+      if constexpr (EPI == WS_RES) *p = f2bf(bf2f(OUTS <= T ? res_pf : *p) + bf2f(f2bf(y)));
+      else *p = f2bf(act_out(re, y, row0 + 8 * g + j));
     }
   }
 }
 
-// rows the weight-streaming kernel takes, (gemv_chain_max_m, g_ws_max_m]: 0 = off (default, the
-// decode chain stays at the GEMV's 4 rows).  Measured slower than the planner's LDS-ring small
-// tiles on gate_up / down at every M and on all shapes at M >= 32 (profiles/r06_small_m_ws.md);
-// the gemm_ws_max_m op turns it on for A/B runs
-int g_ws_max_m = 0;
+// rows up to which this kernel is taken, in the decode chain and outside (gemm_ws_max_m op; 0: never)
+int g_ws_max_m = 16;
 
-// A/B plan of the sweep (gemm_ws_plan op, scripts/bench_ws.py): row blocks per workgroup (plain: 1 / 2 /
-// 4, SiLU-mul: 2 / 4; 0 = default 1 / 2), K-steps in flight (4 / 8; 0 = 8 where K allows) and
-// non-temporal (1) or cached (0, default: 64 B per row per load, the two halves of a line on
-// consecutive loads, which the cached path merges in L2 -- 1.3-1.9x faster than nt at o / qkv)
-// weight loads.  The RoPE / residual / row-scale forms keep the defaults.
-int g_ws_rb = 0, g_ws_u = 0, g_ws_nt = 0;
+// A / B plan (gemm_ws_plan op, 0 = by shape): 16-row blocks per workgroup (1 / 2) and K-steps in flight per wave (1 / 2)
+int g_ws_rb = 0, g_ws_u = 0;
 
-template <int MT, int RB, int EPI, bool RS, int U, bool NT>
-void launch_ws_k(const uint16_t* A, int lda, const uint16_t* B, int ldb, uint16_t* C, int ldc, int M, int N, int K,
-                 const RopeEpi& re, float eps, hipStream_t st) {
-  gemm_ws_kernel<MT, RB, U, EPI, RS, NT><<<N / (16 * RB), 256, 0, st>>>(A, lda, B, ldb, C, ldc, M, K, re, eps);
+template <int AR, int G, int U, int EPI, bool RS>
+void run_ws_k(const uint16_t* A, int lda, const uint16_t* B, int ldb, uint16_t* C, int ldc, int M, int N, int K,
+              const RopeEpi& re, float eps, hipStream_t st) {
+  constexpr int MT = (AR + 15) / 16, NW = 8;
+  constexpr size_t ring = (size_t)NW * U * AR * 256, red = (size_t)NW * MT * (G * 512 + 64), lds = ring > red ? ring : red;
+  static_assert(lds <= 163840, "LDS");
+  auto kern = gemm_ws_kernel<AR, G, NW, U, EPI, RS>;
+  static const bool attr =
+      hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess;
+  (void)attr;
+  kern<<<N / (8 * G), NW * 64, lds, st>>>(A, lda, B, ldb, C, ldc, M, K, re, eps);
 }
 
-template <int MT, int RB, int EPI, bool RS>
-void run_ws_mt(const uint16_t* A, int lda, const uint16_t* B, int ldb, uint16_t* C, int ldc, int M, int N, int K,
+template <int AR, int EPI, bool RS>
+void run_ws_ar(const uint16_t* A, int lda, const uint16_t* B, int ldb, uint16_t* C, int ldc, int M, int N, int K,
                const RopeEpi& re, float eps, hipStream_t st) {
-  const bool u8 = (K >> 2) % (32 * 8) == 0 && g_ws_u != 4;
-  constexpr bool SWEEP = !RS && (EPI == WS_NONE || EPI == WS_SILU_MUL);
-  if (SWEEP && g_ws_nt) {
-    if (u8) launch_ws_k<MT, RB, EPI, RS, 8, true>(A, lda, B, ldb, C, ldc, M, N, K, re, eps, st);
-    else launch_ws_k<MT, RB, EPI, RS, 4, true>(A, lda, B, ldb, C, ldc, M, N, K, re, eps, st);
-    return;
+  // 32 weight rows take in half as much of A as 16 do, on half as many workgroups: where 16 make a second round of the CUs
+  // and 32 do not (6144 x 4096 at 4 rows 10.6 -> 10.3 us, at 16 13.4 -> 11.8; 5120 x 5120 at 8 14.5 -> 13.2), and from 9 rows on
+  // unless they end in a round half empty (28672 x 4096 at 16 rows 42 -> 39, lm_head 128256 x 4096 184 -> 158; but 10240 x
+  // 8192, 320 workgroups, 34.4 -> 37.2).  Up to 8 rows A costs little: 28672 x 4096 at 8 36.2 against 38.2.
+  const int w32 = N / 32;
+  const bool wide = N % 32 == 0 && (g_ws_rb ? g_ws_rb == 2 : N / 16 > kCus && (w32 <= kCus || (M > 8 && w32 >= 7 * kCus / 4)));
+  // two steps per wave in flight where there are as many and the images leave a second workgroup its LDS (lm_head at 4 rows
+  // 152.2 -> 148.8 us; 16384 x 512 at 4, one step per wave, 5.3 -> 7.0; at 16 rows down 4096 x 14336 23.4 -> 24.0)
+  const bool two = g_ws_u ? g_ws_u == 2 : AR <= 8 && K >= 2048;
+#define MLOP_WS(G, U) return run_ws_k<AR, G, U, EPI, RS>(A, lda, B, ldb, C, ldc, M, N, K, re, eps, st)
+  if constexpr (AR <= 32) {
+    if (wide && two) MLOP_WS(4, 2);
+    if (two) MLOP_WS(2, 2);
   }
-  if (u8) launch_ws_k<MT, RB, EPI, RS, 8, false>(A, lda, B, ldb, C, ldc, M, N, K, re, eps, st);
-  else launch_ws_k<MT, RB, EPI, RS, 4, false>(A, lda, B, ldb, C, ldc, M, N, K, re, eps, st);
+  if (wide) MLOP_WS(4, 1);
+  MLOP_WS(2, 1);
+#undef MLOP_WS
 }
 
-template <int RB, int EPI, bool RS>
+template <int EPI, bool RS>
 void run_ws(const uint16_t* A, int lda, const uint16_t* B, int ldb, uint16_t* C, int ldc, int M, int N, int K,
             const RopeEpi& re, float eps, hipStream_t st) {
-  switch ((M + 15) >> 4) {
-    case 1: run_ws_mt<1, RB, EPI, RS>(A, lda, B, ldb, C, ldc, M, N, K, re, eps, st); break;
-    case 2: run_ws_mt<2, RB, EPI, RS>(A, lda, B, ldb, C, ldc, M, N, K, re, eps, st); break;
-    case 3: run_ws_mt<3, RB, EPI, RS>(A, lda, B, ldb, C, ldc, M, N, K, re, eps, st); break;
-    default: run_ws_mt<4, RB, EPI, RS>(A, lda, B, ldb, C, ldc, M, N, K, re, eps, st); break;
-  }
+  if (M <= 4) run_ws_ar<4, EPI, RS>(A, lda, B, ldb, C, ldc, M, N, K, re, eps, st);
+  else if (M <= 8) run_ws_ar<8, EPI, RS>(A, lda, B, ldb, C, ldc, M, N, K, re, eps, st);
+  else if (M <= 16) run_ws_ar<16, EPI, RS>(A, lda, B, ldb, C, ldc, M, N, K, re, eps, st);
+  else if (M <= 32) run_ws_ar<32, EPI, RS>(A, lda, B, ldb, C, ldc, M, N, K, re, eps, st);
+  else if (M <= 48) run_ws_ar<48, EPI, RS>(A, lda, B, ldb, C, ldc, M, N, K, re, eps, st);
+  else run_ws_ar<64, EPI, RS>(A, lda, B, ldb, C, ldc, M, N, K, re, eps, st);
 }
 
 }  // namespace
@@ -271,54 +353,61 @@ int gemm_ws_max_m(int set) {
   return g_ws_max_m;
 }
 
-// Outside the chain, the plain decode projections take this kernel where it measured faster
-// than the planner's small tiles (profiles/r06_small_m_ws.md): the O-size (33 MB) and QKV-size
-// (50 MB) matrices at 5-8 rows.  Cold-weight microbench: o 8.4 vs 15.9 us, qkv 12.4 vs 17.8 (the
-// QKV form also does RoPE + the paged K/V stores, so the rope_cache slab reduce launch goes);
-// in the model the planner's O runs nearer 9 us, so end to end batch 8 gains 1.7 % and batch
-// 16 is within noise (-1 %): 8 rows.  gate_up / down and 32+ rows stay on the planner.  The
-// gemm_ws_small_m op (0 = off) is the A/B switch.
-int g_ws_small_m = 8;
+// and outside the chain: gemm_ws_small_m op, QKV + RoPE gemm_ws_rope_m
+int g_ws_small_m = 16, g_ws_rope_m = 16;
 
 int gemm_ws_small_m(int set) {
   if (set >= 0) g_ws_small_m = set > 64 ? 64 : set;
   return g_ws_small_m;
 }
 
-// QKV + RoPE takes the weight-streaming kernel up to g_ws_rope_m rows (gemm_ws_rope_m op): it
-// replaces the planner's split-K tile AND the rope_cache slab-reduce launch after it
-int g_ws_rope_m = 8;
 int gemm_ws_rope_m(int set) {
   if (set >= 0) g_ws_rope_m = set > 64 ? 64 : set;
   return g_ws_rope_m;
 }
 
-bool ws_prefer(int M, int N, int K, int epi) {
-  if (M <= gemv_chain_max_m() || (long)N * K > 32L * 1024 * 1024 || K % 512) return false;
-  if (epi == WS_ROPE) return M <= g_ws_rope_m && N % 128 == 0;
-  return M <= g_ws_small_m && (epi == WS_NONE || epi == WS_RES) && N % 16 == 0;
-}
-
-void gemm_ws_plan(int rb, int u, int nt) {
-  g_ws_rb = rb == 1 || rb == 2 || rb == 4 ? rb : 0;
-  g_ws_u = u == 4 || u == 8 ? u : 0;
-  g_ws_nt = nt != 0;
-}
-
-// Shapes this path takes: gemv_max_m() < M <= ws max (default 64), K a multiple of 512 (four K
-// quarters of whole 4-step rings), 16-B aligned rows, whole 16-row blocks (plain / residual),
-// whole 32-row gate / up groups (SiLU-mul), a QKV projection of 128-wide heads (RoPE).
-bool ws_takes(int M, int N, int K, int epi) {
-  if (M <= gemv_chain_max_m() || M > g_ws_max_m || K % 512 || N < 16) return false;
+// shapes this kernel can take: whole steps of 128 k, whole 16-row blocks (gate / up: 32-row groups; RoPE: 128-wide heads)
+static bool ws_shape(int M, int N, int K, int epi) {
+  if (M < 1 || M > 64 || K % 128 || K < 128 || K > (1 << 18) || N < 16) return false;
   if (epi == WS_SILU_MUL) return N % 32 == 0;
   if (epi == WS_ROPE) return N % 128 == 0;
   return (epi == WS_NONE || epi == WS_RES) && N % 16 == 0;
 }
 
+// Where it is the faster choice.  Against the GEMV (one to four rows): from 3 rows on, two where the matrix is not narrow, one
+// where it is large (us, GEMV -> here: 6144 x 4096 at 2 / 4 rows 11.3 -> 10.5, 15.1 -> 10.5; 28672 x 4096 at 1 / 2 / 4 36.6 -> 37.2,
+// 36.0 -> 36.5, 43.3 -> 36; 4096 x 14336 at 4 24.4 -> 19.9; 128256 x 4096 at 1 / 4 160 -> 155, 171 -> 150; 128256 x 8192 at 1 336 ->
+// 307; 2048 x 4096 at 2 / 4 6.0 -> 6.6, 7.2 -> 6.2; 1024 x 4096 at 4 5.4 -> 5.8).  Against the planner's tiles and their K ranges' sums (5 to
+// 16): everywhere but where few rows have a long K (6144 x 4096 at 5 / 16 17.7 -> 10.9, 17.7 -> 11.7; 4096 x 4096 with its norm pass 12.1
+// -> 7.6, 12.1 -> 8.5; 8192 x 28672 at 8 105 -> 73; 28672 x 4096 at 8 / 16 39.4 -> 36, 39.6 -> 39; 1024 x 14336 at 8 12.6 -> 16.2, 2048 x 8192
+// at 16 12.4 -> 12.0).  At 24 and 32 rows A is what a CU takes in: 28672 x 4096 40.4 -> 48.5, 4096 x 14336 25 -> 28.
+static bool ws_fast(int M, int N, int K) {
+  if (M == 1) return (long)N * K >= 200L * 1000 * 1000;
+  if (M <= 4) return N >= (M == 2 ? 3072 : 2048);
+  return (long)N * K >= 1 << 20 && (N >= 3072 || K <= 9216);  // (smaller ones are launches, whichever the kernel)
+}
+
+bool ws_prefer(int M, int N, int K, int epi) {
+  return M <= std::min(g_ws_max_m, epi == WS_ROPE ? g_ws_rope_m : g_ws_small_m) && ws_shape(M, N, K, epi) && ws_fast(M, N, K);
+}
+
+// (the third argument chose a form of the weight loads that is no more)
+void gemm_ws_plan(int rb, int u, int) {
+  g_ws_rb = rb == 1 ? 1 : rb == 2 || rb == 4 ? 2 : 0;
+  g_ws_u = u == 1 ? 1 : u > 1 ? 2 : 0;
+}
+
+bool ws_takes(int M, int N, int K, int epi) { return M <= g_ws_max_m && ws_shape(M, N, K, epi); }
+
 int decode_chain_max_m() { return g_ws_max_m > gemv_chain_max_m() ? g_ws_max_m : gemv_chain_max_m(); }
 
+// the chain's product of this shape on this kernel rather than the GEMV
+bool chain_on_ws(int M, int N, int K, int epi) {
+  return ws_takes(M, N, K, epi) && (M > gemv_chain_max_m() || ws_fast(M, N, K));
+}
+
 bool decode_chain_takes(int M, int N, int K, int epi) {
-  return M <= gemv_chain_max_m() ? gemv_chain_takes(M, N, K, epi) : ws_takes(M, N, K, epi);
+  return gemv_chain_takes(M, N, K, epi) || (ws_takes(M, N, K, epi) && ((long)N * K >= 1 << 20));
 }
 
 void launch_ws(const void* A, int lda, const void* B, int ldb, void* C, int ldc, int M, int N, int K, int epi,
@@ -327,19 +416,16 @@ void launch_ws(const void* A, int lda, const void* B, int ldb, void* C, int ldc,
   auto* b = (const uint16_t*)B;
   auto* c = (uint16_t*)C;
   if (epi == WS_SILU_MUL) {
-    if (rs) run_ws<2, WS_SILU_MUL, true>(a, lda, b, ldb, c, ldc, M, N, K, re, eps, st);
-    else if (g_ws_rb == 4 && N % 64 == 0) run_ws<4, WS_SILU_MUL, false>(a, lda, b, ldb, c, ldc, M, N, K, re, eps, st);
-    else run_ws<2, WS_SILU_MUL, false>(a, lda, b, ldb, c, ldc, M, N, K, re, eps, st);
+    if (rs) run_ws<WS_SILU_MUL, true>(a, lda, b, ldb, c, ldc, M, N, K, re, eps, st);
+    else run_ws<WS_SILU_MUL, false>(a, lda, b, ldb, c, ldc, M, N, K, re, eps, st);
   } else if (epi == WS_ROPE) {
-    if (rs) run_ws<2, WS_ROPE, true>(a, lda, b, ldb, c, ldc, M, N, K, re, eps, st);
-    else run_ws<2, WS_ROPE, false>(a, lda, b, ldb, c, ldc, M, N, K, re, eps, st);
+    if (rs) run_ws<WS_ROPE, true>(a, lda, b, ldb, c, ldc, M, N, K, re, eps, st);
+    else run_ws<WS_ROPE, false>(a, lda, b, ldb, c, ldc, M, N, K, re, eps, st);
   } else if (epi == WS_RES) {
-    run_ws<1, WS_RES, false>(a, lda, b, ldb, c, ldc, M, N, K, re, eps, st);
+    run_ws<WS_RES, false>(a, lda, b, ldb, c, ldc, M, N, K, re, eps, st);
   } else {
-    if (rs) run_ws<1, WS_NONE, true>(a, lda, b, ldb, c, ldc, M, N, K, re, eps, st);
-    else if (g_ws_rb == 4 && N % 64 == 0) run_ws<4, WS_NONE, false>(a, lda, b, ldb, c, ldc, M, N, K, re, eps, st);
-    else if (g_ws_rb == 2 && N % 32 == 0) run_ws<2, WS_NONE, false>(a, lda, b, ldb, c, ldc, M, N, K, re, eps, st);
-    else run_ws<1, WS_NONE, false>(a, lda, b, ldb, c, ldc, M, N, K, re, eps, st);
+    if (rs) run_ws<WS_NONE, true>(a, lda, b, ldb, c, ldc, M, N, K, re, eps, st);
+    else run_ws<WS_NONE, false>(a, lda, b, ldb, c, ldc, M, N, K, re, eps, st);
   }
 }
 

@@ -306,8 +306,7 @@ __global__ void __launch_bounds__(256) gemv_kernel(const uint16_t* __restrict__ 
 }
 
 int gemv_max_m() {
-  // measured (scripts/history INDEX run38): the GEMV wins every decode projection at M <= 4 in
-  // the running model; at M = 8 the 64-row MFMA tiles stream gate_up / down faster
+  // (at 2 - 4 rows most products are faster on gemm_ws.hip, asked first: ws_fast there)
   return 4;
 }
 
@@ -450,10 +449,7 @@ void launch_gemv_grouped(const void* A, const void* B, void* C, const int* offse
 // QKV and gate_up read the raw residual and scale each row's sums by rsqrt(mean(a^2) + eps)
 // taken from the chunks they stream anyway (PRO_RS).  A decode layer is then five launches
 // and no add + RMSNorm pass: the GEMV form of gemm_w4.hip's large-M chain (W4_ADD_SS / W4_RS).
-// rows the chain's GEMV form takes (above gemv_max_m() the GEMV takes nothing anyway).
-// Measured (scripts/history INDEX r4_chain8): the GEMV with the chain at 6 / 8 rows streams
-// 1,419 / 1,612 tok/s against the MFMA path's 1,522 / 1,936 (its split-K reduce already
-// carries the add + RMSNorm), so 4 stays.
+// rows the chain's GEMV form takes (above gemv_max_m() the GEMV takes nothing anyway)
 int gemv_chain_max_m() { return 4; }
 
 bool gemv_chain_takes(int M, int N, int K, int epi) {

@@ -196,7 +196,7 @@ struct NormPro {
 // decode norm chain (gemv.hip PRO_RS / EPI_RES, M <= 4): C = epi(rowscale(A) . B^T) with
 // rowscale = rsqrt(mean(A_row^2) + eps) (norm weights folded into B); residual += A . B^T
 bool gemv_chain_takes(int M, int N, int K, int epi);
-// weight-streaming MFMA GEMM (gemm_ws.hip) at gemv_chain_max_m() < M <= gemm_ws_max_m() (64):
+// weight-streaming MFMA GEMM (gemm_ws.hip), M <= gemm_ws_max_m() (16):
 // epi 0 plain, 1 SiLU-mul, 3 RoPE + paged K/V (re), 5 residual += (C in place); rs: A is the raw
 // residual, rows scaled by rsqrt(mean(a^2) + eps) (norm weights folded into B)
 bool ws_takes(int M, int N, int K, int epi);
@@ -204,7 +204,7 @@ int gemm_ws_max_m(int set);
 void gemm_ws_plan(int rb, int u, int nt);
 int gemm_ws_small_m(int set);
 int gemm_ws_rope_m(int set);  // rows up to which QKV + RoPE takes the weight-streaming kernel
-// the plain (non-chain) decode projections this kernel takes instead of the planner
+// the decode projections outside the chain that this kernel takes instead of the GEMV or the planner's tiles
 bool ws_prefer(int M, int N, int K, int epi);
 // mid-M norm chain on the planner's small tiles (gemm.hip): epi 0 = O / down (split-K, the
 // last split adds into the residual and leaves the row sums of squares), 1 = gate_up (SiLU-mul,
@@ -215,10 +215,11 @@ bool launch_mid_res_ss(const void* A, int lda, const void* B, void* residual, in
                        float* ss_tot, hipStream_t st);
 bool launch_mid_rs(const void* A, int lda, const void* B, void* out, int ldo, int M, int N, int K,
                    const float* ss_tot, float eps, hipStream_t st);
-// the decode norm chain's forms: the GEMV up to gemv_chain_max_m() rows, then the weight-
-// streaming MFMA kernel up to gemm_ws_max_m()
+// the decode norm chain's forms: the GEMV up to gemv_chain_max_m() rows, the weight-streaming MFMA kernel up to
+// gemm_ws_max_m(); chain_on_ws: the latter is this product's choice
 int decode_chain_max_m();
 bool decode_chain_takes(int M, int N, int K, int epi);
+bool chain_on_ws(int M, int N, int K, int epi);
 void launch_ws(const void* A, int lda, const void* B, int ldb, void* C, int ldc, int M, int N, int K, int epi,
                bool rs, const RopeEpi& re, float eps, hipStream_t st);
 int gemv_chain_max_m();
