@@ -14,10 +14,9 @@
 // from the first one's accumulator registers (cdna_hip_programming.md §3
 // "An accumulator tile as the next MFMA's operand", with a permuted k order).
 // Decode kernel token order of a page pair (A, B; pair token t = 16*page + offset):
-// lane group g = lane>>4 owns the 8 CONSECUTIVE pair tokens 8g..8g+7 - the first S
-// MFMA produces 8g..8g+3 of every group, the second 8g+4..8g+7 (its K rows are
-// loaded in that permuted row order) - so each lane's V^T fragment is two transposed
-// 4-row reads of the pair's LDS image and P^T = {S1 rows, S2 rows} as before.
+// lane group g = lane>>4 owns the 8 CONSECUTIVE pair tokens 8g..8g+7 (K rows are
+// loaded in a row order that makes it so: load_k) - so each lane's V^T fragment is two transposed
+// 4-row reads of the pair's LDS image and P^T comes from the S registers as before.
 //
 // MFMA rows: 16 q-rows per tile = (16/G query tokens) x (G heads of one kv head).
 // A workgroup = 4 waves = one (tile, kv head, kv partition); the waves split
@@ -25,9 +24,8 @@
 // Partitions > 1 (long context, small batch: fill 256 CUs) write fp32 partials
 // that attn_reduce_kernel combines.
 //
-// Memory-bound: each K byte is loaded once per tile straight into VGPRs ("GEMV / M <= 16" row
-// of the glds table, cdna_hip_programming.md §5); each V byte once into the wave's LDS image
-// by LDS-DMA (the transpose needs it in LDS).
+// Memory-bound: each K byte is loaded once per tile straight into VGPRs, 8 token rows x 128 B an instruction; each V
+// byte once into the wave's LDS image by LDS-DMA (the transpose needs it in LDS).
 //
 // REQUIREMENT: the cache is zero-initialised at allocation (masked lanes multiply
 // p = 0 with whatever the unused slots hold; NaN garbage would poison O).
@@ -225,14 +223,16 @@ __global__ void __launch_bounds__(256, 3) paged_attn_kernel(
   const int head = kvh * G + (r % G);
   const int pos_r = row_ok ? ctx - ql + qi : -1;
 
-  bf16x8 qf[4];
+  bf16x8 qf[2][2];  // [half of the head's dims][even / odd 16-B chunks]
   {
     const uint16_t* qrow = q + ((size_t)(qs + (row_ok ? qi : 0)) * Hq + head) * kD;
 #pragma unroll
-    for (int kk = 0; kk < 4; ++kk) {
-      bf16x8 v = *reinterpret_cast<const bf16x8*>(qrow + kk * 32 + g4 * 8);
-      qf[kk] = row_ok ? v : bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
-    }
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int x = 0; x < 2; ++x) {
+        bf16x8 v = *reinterpret_cast<const bf16x8*>(qrow + h * 64 + g4 * 16 + x * 8);
+        qf[h][x] = row_ok ? v : bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+      }
   }
 
   f32x4 o[8];
@@ -250,39 +250,42 @@ __global__ void __launch_bounds__(256, 3) paged_attn_kernel(
   // clamp: a corrupt block table must not become an out-of-bounds fault
   auto page_of = [&](int raw) { return min(max(raw, 0), num_blocks - 1); };
   // the pair's 32 token rows of this kv head by LDS-DMA into this wave's V image
-  auto issue_v = [&](int pa, int pb) {
-    const uint16_t* vA = vc + pa * page_stride + (size_t)kvh * kBS * kD;
-    const uint16_t* vB = vc + pb * page_stride + (size_t)kvh * kBS * kD;
-    const uint32_t dst = vimg;
+  uint32_t vo[4];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int trow = (4 * i + g4) & 15;
-      const uint16_t* src = (i < 4 ? vA : vB) + trow * kD + ((r ^ vswz(trow)) << 3);
-      __builtin_amdgcn_global_load_lds((const void*)src, (lds_void_t*)(uintptr_t)(dst + 1024u * i), 16, 0,
-                                       (NT & 1) ? 2 /* nt */ : 0);
-    }
+  for (int i = 0; i < 4; ++i) vo[i] = (4 * i + g4) * (2 * kD) + ((r ^ vswz(4 * i + g4)) << 4);
+  auto issue_v = [&](int pa, int pb) {
+    const uint16_t* vh = vc + (size_t)kvh * kBS * kD;
+    const auto rA = __builtin_amdgcn_make_buffer_rsrc((void*)(vh + pa * page_stride), 0, kBS * kD * 2, 0x00020000);
+    const auto rB = __builtin_amdgcn_make_buffer_rsrc((void*)(vh + pb * page_stride), 0, kBS * kD * 2, 0x00020000);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) lds_dma16(rA, vimg + 1024u * i, vo[i], NT & 1);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) lds_dma16(rB, vimg + 4096u + 1024u * i, vo[i], NT & 1);
   };
-  // K rows of MFMA row r: pair tokens 8*(r>>2) + (r&3) (first S MFMA) and +4 (second)
-  bf16x8 ka[4], kb[4];
+  // K: instruction (t, h) loads half h (128 B, a whole line) of 8 token rows.  MFMA row r holds the chunks 2 g4 + (r & 1) of
+  // the half of pair token 8 (r >> 2) + 2 t + ((r >> 1) & 1); multiplied with Q's even chunks its even rows count, with the
+  // odd ones its odd rows, and a lane's accumulators 0 and 2 of the one and 1 and 3 of the other make its tokens
+  // 8 g4 + 2 t and + 1.  (Twice the MFMAs, of which there are plenty.)
+  bf16x8 kf[4][2];
   auto load_k = [&](int pa, int pb) {
     const uint16_t* kP = kc + (r >> 3 ? pb : pa) * page_stride + (size_t)kvh * kBS * kD;
-    const uint16_t* kR = kP + (8 * ((r >> 2) & 1) + (r & 3)) * kD;
+    const uint16_t* kR = kP + (8 * ((r >> 2) & 1) + ((r >> 1) & 1)) * kD + g4 * 16 + (r & 1) * 8;
 #pragma unroll
-    for (int kk = 0; kk < 4; ++kk) {
-      if constexpr ((NT & 1) != 0) {
-        ka[kk] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(kR + kk * 32 + g4 * 8));
-        kb[kk] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(kR + 4 * kD + kk * 32 + g4 * 8));
-      } else {
-        ka[kk] = *reinterpret_cast<const bf16x8*>(kR + kk * 32 + g4 * 8);
-        kb[kk] = *reinterpret_cast<const bf16x8*>(kR + 4 * kD + kk * 32 + g4 * 8);
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const bf16x8* p = reinterpret_cast<const bf16x8*>(kR + 2 * t * kD + h * 64);
+        if constexpr ((NT & 1) != 0) kf[t][h] = __builtin_nontemporal_load(p);
+        else kf[t][h] = *p;
       }
-    }
   };
   // A pair's K loads (registers) and V image (LDS) are issued a pair ahead: K(p + 4) as soon as the S MFMAs have
   // taken K(p), V(p + 4) as soon as the transposed reads have taken V(p).  The workgroups of a launch run in step, and
   // memory stood still while they all multiplied (100 sequences of 1000 keys 96.7 -> 90.2 us, 64 of 4000 217 -> 196).
-  // K is in flight under the softmax and P.V; V only from its issue to the loop's top, where the compiler waits for
-  // everything (vmcnt(0) before the first S MFMA: it does not count loads into registers apart from the LDS-DMA).
+  // Each is waited for alone, by count: with the global form of LDS-DMA the compiler waited for K and V together at the
+  // loop's top, and with 16 rows x 64 B per K instruction (one MFMA each) every line was asked for twice.  Both together, us per
+  // launch, 8 kv heads: 7 x 1000 keys 12.2 -> 10.4, 13 x 2500 34.8 -> 29.7, 20 x 800 22.2 -> 15.6, 100 x 1000 83.1 -> 74.5, 300 x
+  // 600 130 -> 122, 700 x 500 243 -> 234 (6.1 TB/s).
   int pgA = 0, pgB = 0, rawA = 0, rawB = 0;  // page ids of the pair whose K is loading; the next pair's as read
   auto load_pages = [&](int pp) {  // (past the end: entries of the row, never used)
     rawA = bt[min(2 * pp, bt_stride - 1)];
@@ -306,14 +309,21 @@ __global__ void __launch_bounds__(256, 3) paged_attn_kernel(
   }
   auto pair = [&](auto more_) {
     constexpr bool more = decltype(more_)::value;
-    // S^T[token][row]: lane holds row r, tokens 4*g4 + i of each page
-    f32x4 sa = {0.f, 0.f, 0.f, 0.f}, sb = {0.f, 0.f, 0.f, 0.f};
+    // S^T[token][row]: lane holds row r, tokens 8 g4 + i of the pair
+    float sc[8];
 #pragma unroll
-    for (int kk = 0; kk < 4; ++kk) {
-      sa = mfma16(ka[kk], qf[kk], sa);
-      sb = mfma16(kb[kk], qf[kk], sb);
+    for (int t = 0; t < 4; ++t) {
+      f32x4 e = {0.f, 0.f, 0.f, 0.f}, d = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        e = mfma16(kf[t][h], qf[h][0], e);
+        d = mfma16(kf[t][h], qf[h][1], d);
+      }
+      sc[2 * t] = e[0] + d[1];
+      sc[2 * t + 1] = e[2] + d[3];
     }
-    asm volatile("" : "+v"(sa), "+v"(sb)::"memory");  // the next K loads stay behind the MFMAs that read this pair's
+    // the next K loads stay behind the MFMAs that read this pair's
+    asm volatile("" : "+v"(sc[0]), "+v"(sc[1]), "+v"(sc[2]), "+v"(sc[3]), "+v"(sc[4]), "+v"(sc[5]), "+v"(sc[6]), "+v"(sc[7])::"memory");
     if constexpr (more) {
       take_pages(pp + 4);
       load_k(pgA, pgB);
@@ -321,36 +331,27 @@ __global__ void __launch_bounds__(256, 3) paged_attn_kernel(
       load_pages(pp + 8);
       asm volatile("" ::: "memory");
     }
-    const int tokA = pp * 32 + g4 * 8, tokB = tokA + 4;
-    float pa[4], pb[4];
+    const int tok = pp * 32 + g4 * 8;
     float mx = kNegBig;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int ta = tokA + i, tb = tokB + i;
-      pa[i] = (ta < p_end && ta <= pos_r) ? sa[i] * scale_log2 : -INFINITY;
-      pb[i] = (tb < p_end && tb <= pos_r) ? sb[i] * scale_log2 : -INFINITY;
-      mx = fmaxf(mx, fmaxf(pa[i], pb[i]));
+    for (int i = 0; i < 8; ++i) {
+      sc[i] = (tok + i < p_end && tok + i <= pos_r) ? sc[i] * scale_log2 : -INFINITY;
+      mx = fmaxf(mx, sc[i]);
     }
     mx = max_x16_x32(mx);
     const float m_new = fmaxf(m, mx);
     const float alpha = fast_exp2(m - m_new);
     m = m_new;
     float rs = 0.f;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      pa[i] = fast_exp2(pa[i] - m_new);
-      pb[i] = fast_exp2(pb[i] - m_new);
-      rs += pa[i] + pb[i];
-    }
-    l = l * alpha + rs;
     bf16x8 pf;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      pf[i] = (short)f2bf(pa[i]);
-      pf[4 + i] = (short)f2bf(pb[i]);
+    for (int i = 0; i < 8; ++i) {
+      sc[i] = fast_exp2(sc[i] - m_new);
+      rs += sc[i];
+      pf[i] = (short)f2bf(sc[i]);
     }
-    // this wave's V image has landed: at least the eight K loads are younger (the wait at the loop's top covers it
-    // as long as the compiler puts one there)
+    l = l * alpha + rs;
+    // this wave's V image has landed: at least the eight K loads are younger
     if constexpr (more) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     const uint32_t b0 = vimg + vt_base(lane);
@@ -530,9 +531,9 @@ static void launch_g(void* out, float* part_o, float* part_ml, const void* q, co
   // (7 x 1000 keys 12.05 -> 12.3).
   const bool by_head = Hkv > 1 && num_tiles >= (Hkv >= 8 ? 33 : 256) && num_tiles <= 65535;  // (the grid's second dimension)
   const dim3 grid = by_head ? dim3(Hkv, num_tiles, nparts) : dim3(num_tiles, Hkv, nparts);
-  // K / V pages non-temporal (attn_kv_nt op): each is read once per step by one workgroup
-  // (below 8 query tiles the default policy: batch 4 lost 0.7 % with it, batch 16 gained 1.8 %)
-  const int nt = num_tiles >= 8 ? g_attn_kv_nt : 0;
+  // K / V pages non-temporal (attn_kv_nt op): each is read once per step by one workgroup (1 x 24000 keys 22.5 -> 20.8 us, 3 x
+  // 24000 55.1 -> 51.0; while a line of K was read in two halves few tiles were faster cached)
+  const int nt = g_attn_kv_nt;
   auto pick = [&](auto h) {
     constexpr bool H = decltype(h)::value;
     return nt == 3 ? paged_attn_kernel<G, 3, H> : nt ? paged_attn_kernel<G, 1, H> : paged_attn_kernel<G, 0, H>;
