@@ -174,7 +174,8 @@ def paged_attention(q, k_cache, v_cache, meta, out: torch.Tensor | None = None):
             sem = _no_sem(q.device)
         torch.ops.mlop.paged_attention(out, meta.part_o, meta.part_ml, sem, q, k_cache, v_cache,
                                        meta.block_tables, meta.tile_seq, meta.tile_q0, meta.q_start,
-                                       meta.q_len, meta.ctx_len, scale, meta.part_tokens, meta.nparts)
+                                       meta.q_len, meta.ctx_len, scale, meta.part_tokens, meta.nparts,
+                                       getattr(meta, "load", None))
     pts = getattr(meta, "ptile_seq", None)
     if pts is not None and pts.numel():
         # prompt chunks: K7 flash prefill (128 q-rows per workgroup, K/V via LDS-DMA)

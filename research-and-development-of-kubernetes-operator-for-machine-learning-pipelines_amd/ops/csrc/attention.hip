@@ -104,15 +104,22 @@ constexpr int kEnoughParts = 8;
 // 40 x 200 67 -> 28 us, 1 x 24000 beside 20 x 500 195 -> 102, 10 x 4000 beside 10 x 100 70 -> 43).  From kEnoughParts shares
 // on, further slabs cost what shorter walks save (2 x 16000 beside 2 x 200 in 8 shares 38.7 us, in 31 45.5).  Every
 // workgroup of the launch and the reduction sum the same integers.
-__device__ __forceinline__ int seq_part(int kv_end, int part_tokens, int nparts, int even, const int* tile_seq,
-                                        const int* ctx_len, int tiles, int Hkv) {
+__device__ __forceinline__ int seq_part(int kv_end, int part_tokens, int nparts, int even, int even_from, const int* load,
+                                        const int* tile_seq, const int* ctx_len, int tiles, int Hkv) {
   constexpr int min_part = 128;  // attn_meta.MIN_PART
   constexpr int long_part = 512;
   if (nparts == 1) return part_tokens;
+  // (by the mean where the host has summed them: a launch of which some sequences are cut is slower than either)
+  if (even_from > 0 && (load != nullptr ? load[0] < (long)even_from * load[1] : kv_end < even_from)) even = 1;
   int n = even;
   if (even < nparts && kv_end > long_part * 3 / 2 * even) {  // (two long shares or more)
     float sum = 0.f;  // (below 2^24 exact, above the same everywhere)
     int live = 0;
+    if (load != nullptr) {
+      sum = threadIdx.x & 63 ? 0.f : (float)load[0];
+      live = load[1];
+      tiles = 0;
+    }
     for (int i = 0; i < tiles; i += 256) {
       const int l = i + (threadIdx.x & 63);
       int c[4];
@@ -182,7 +189,7 @@ __global__ void __launch_bounds__(256, 3) paged_attn_kernel(
     const int* __restrict__ tile_seq, const int* __restrict__ tile_q0,
     const int* __restrict__ q_start, const int* __restrict__ q_len,
     const int* __restrict__ ctx_len, int Hq, int Hkv, float scale_log2, int part_tokens,
-    int nparts, int even, int num_blocks, int* __restrict__ sem) {
+    int nparts, int even, int even_from, int num_blocks, int* __restrict__ sem, const int* __restrict__ load) {
   constexpr int QT = 16 / G;
   // (3 waves per SIMD: 154 VGPRs; asked for two fewer the compiler keeps O in AGPRs and copies it for every rescale)
   // wave w stages its page pair's V image (2 x 16 token rows x 256 B = 8 KB) inside sm_o[w]
@@ -200,7 +207,7 @@ __global__ void __launch_bounds__(256, 3) paged_attn_kernel(
   const int ql = q_len[s], ctx = ctx_len[s], qs = q_start[s];
   const int last_q = min(q0 + QT, ql) - 1;           // last valid query of the tile
   const int kv_end = last_q >= 0 ? ctx - ql + last_q + 1 : 0;
-  part_tokens = seq_part(kv_end, part_tokens, nparts, even, tile_seq, ctx_len, BY_HEAD ? gridDim.y : gridDim.x, Hkv);
+  part_tokens = seq_part(kv_end, part_tokens, nparts, even, even_from, load, tile_seq, ctx_len, BY_HEAD ? gridDim.y : gridDim.x, Hkv);
   const int p_begin = part * part_tokens;
   const int p_end = min(kv_end, p_begin + part_tokens);
   if (p_begin >= p_end) {                            // reducer skips empty partitions
@@ -468,14 +475,14 @@ __global__ void __launch_bounds__(256) attn_reduce_kernel(
     const float* __restrict__ part_ml, const int* __restrict__ tile_seq,
     const int* __restrict__ tile_q0, const int* __restrict__ q_start,
     const int* __restrict__ q_len, const int* __restrict__ ctx_len, int Hq, int Hkv,
-    int part_tokens, int nparts, int even) {
+    int part_tokens, int nparts, int even, int even_from, const int* __restrict__ load) {
   constexpr int QT = 16 / G;
   const int tile = blockIdx.x, kvh = blockIdx.y;
   const int s = tile_seq[tile], q0 = tile_q0[tile];
   const int ql = q_len[s], ctx = ctx_len[s], qs = q_start[s];
   const int last_q = min(q0 + QT, ql) - 1;
   const int kv_end = last_q >= 0 ? ctx - ql + last_q + 1 : 0;
-  part_tokens = seq_part(kv_end, part_tokens, nparts, even, tile_seq, ctx_len, gridDim.x, Hkv);
+  part_tokens = seq_part(kv_end, part_tokens, nparts, even, even_from, load, tile_seq, ctx_len, gridDim.x, Hkv);
   const int nvalid = min(nparts, (kv_end + part_tokens - 1) / part_tokens);
   const int rr = threadIdx.x >> 4, c = (threadIdx.x & 15) * 8;
   const int qi = q0 + rr / G;
@@ -496,15 +503,34 @@ int attn_kv_nt(int set) {
   return g_attn_kv_nt;
 }
 
-// Partitions of a sequence in a launch of `base` (tile, kv head) pairs of like lengths: the CUs filled once.  A partition
-// more costs its slab, a ticket and its share of the combine; the metadata plans up to four workgroups per CU, with
-// which 1 x 24000 keys took 47 us (27.6 with 32 partitions), 3 x 24000 64 (58), 7 x 1000 14.1 (12.2), 13 x 2500 34.6
-// (35.1), 20 x 800 23.9 (22.4).  Counts a little above one per CU run as long as two (not powers of two, as steps beside
-// prompts have: 104 pairs in 3 shares 36.9 us, in 2 33; 136 pairs in 2 41, in 3 33; 288 pairs whole 77, in 2 66).
-static int even_parts(int base) {
-  constexpr int wgs = kCus, two = 384;
-  if (base <= wgs / 2) return wgs / base;
-  return base == wgs || base >= two ? 1 : (two + base - 1) / base;
+// Partitions of a sequence in a launch of `base` (tile, kv head) pairs of like lengths, and the keys from which on a sequence
+// is cut into them.  A CU reads its pages at up to 35 GB/s however many workgroups it has, all of them together 6.3 TB/s.  So in
+// units of the launch's bytes at that rate, w workgroups of equal shares take a 256 / w for the a = w / 256 that every CU has and
+// max(180, w % 256) / w for the rest: 136 pairs whole 1.32, in 2 / 3 / 4 shares 1.60 / 1.07 / 1.27 (measured, 17 x 4000 keys 57.1, 64.0,
+// 51.4, 56.2 us); 192 1.0, 1.14, 1.20, 1.0 (24 x 4000 68.2, 75.5, 76.0, 70.2); 264 1.65, 1.31, 1.20, 1.14 (33 x 4000 111, 103, 101, 98.9).
+// A cut costs its slabs, tickets and combining, 2.6 - 4.2 us, which short contexts do not earn back: 16 x 300 keys whole 7.6
+// us, in 2 shares 8.8, 16 x 1000 17.1 and 15.5; 24 x 300 8.5, 11.2; 20 x 1000 18.9, 19.2 in 3.
+struct EvenParts {
+  int n, from;
+};
+static EvenParts even_parts(int base, int nparts) {
+  // few pairs: the CUs filled once (1 x 24000 keys 47 us in four workgroups per CU, 27.6 so; a share has 128 keys at least)
+  if (base <= kCus / 4) return {std::min(nparts, kCus / base), 0};
+  auto model = [&](int n) {
+    const int w = n * base, a = w / kCus, r = w % kCus;
+    return (float)(a * kCus + (r ? std::max(180, r) : 0)) / (float)w;
+  };
+  const int most = std::min(nparts, 4);
+  int n = 1;
+  float best = model(1);
+  for (int i = 2; i <= most; ++i) {
+    const float t = model(i) + .05f + .01f * (float)i;
+    if (t < best - .01f * (n == 1)) best = t, n = i;
+  }
+  if (n == 1) return {1, 0};
+  // a key of `base` pairs is base / 12300 us of the launch; above 256 pairs unequal lengths hide part of a whole launch's end
+  const float gain = std::max(model(1) - model(n), .01f) * (base > kCus ? .6f : 1.f);
+  return {n, (int)std::min(1e6f, (n == 4 ? 4.2f : 2.6f) * 12300.f / ((float)base * gain))};
 }
 
 template <int G>
@@ -512,8 +538,9 @@ static void launch_g(void* out, float* part_o, float* part_ml, const void* q, co
                      const void* vc, const int* bt, int bt_stride, const int* tile_seq,
                      const int* tile_q0, const int* q_start, const int* q_len, const int* ctx_len,
                      int num_tiles, int Hq, int Hkv, float scale_log2, int part_tokens, int nparts,
-                     int num_blocks, int* sem, hipStream_t st) {
-  const int even = std::min(nparts, even_parts(num_tiles * Hkv));
+                     int num_blocks, int* sem, const int* load, hipStream_t st) {
+  const EvenParts ep = even_parts(num_tiles * Hkv, nparts);
+  const int even = ep.n, even_from = ep.from;
   if (num_tiles == 1 || even >= kEnoughParts) {  // (seq_part: none needs more)
     if (even == 1 && nparts > 1) part_tokens = 1 << 30;  // the only partition has all keys, whatever was planned
     nparts = even;
@@ -541,11 +568,11 @@ static void launch_g(void* out, float* part_o, float* part_ml, const void* q, co
   auto kern = by_head ? pick(std::true_type{}) : pick(std::false_type{});
   kern<<<grid, 256, 0, st>>>((uint16_t*)out, part_o, part_ml, (const uint16_t*)q, (const uint16_t*)kc,
                              (const uint16_t*)vc, bt, bt_stride, tile_seq, tile_q0, q_start, q_len, ctx_len,
-                             Hq, Hkv, scale_log2, part_tokens, nparts, even, num_blocks, sem);
+                             Hq, Hkv, scale_log2, part_tokens, nparts, even, even_from, num_blocks, sem, load);
   if (nparts > 1 && sem == nullptr) {
     attn_reduce_kernel<G><<<dim3(num_tiles, Hkv), 256, 0, st>>>(
         (uint16_t*)out, part_o, part_ml, tile_seq, tile_q0, q_start, q_len, ctx_len, Hq, Hkv,
-        part_tokens, nparts, even);
+        part_tokens, nparts, even, even_from, load);
   }
 }
 
@@ -554,13 +581,13 @@ void launch_paged_attention(void* out, float* part_o, float* part_ml, const void
                             const int* tile_seq, const int* tile_q0, const int* q_start,
                             const int* q_len, const int* ctx_len, int num_tiles, int Hq, int Hkv,
                             float scale_log2, int part_tokens, int nparts, int num_blocks,
-                            int* sem, hipStream_t st) {
+                            int* sem, const int* load, hipStream_t st) {
   if (num_tiles == 0) return;
   const int G = Hq / Hkv;
 #define MLOP_ATTN_CASE(GG)                                                                        \
   case GG:                                                                                        \
     launch_g<GG>(out, part_o, part_ml, q, kc, vc, bt, bt_stride, tile_seq, tile_q0, q_start,     \
-                 q_len, ctx_len, num_tiles, Hq, Hkv, scale_log2, part_tokens, nparts, num_blocks, sem, st);   \
+                 q_len, ctx_len, num_tiles, Hq, Hkv, scale_log2, part_tokens, nparts, num_blocks, sem, load, st);   \
     break;
   switch (G) {
     MLOP_ATTN_CASE(1)

@@ -184,7 +184,7 @@ int64_t attn_fused_max_pairs(int64_t n) {
 void paged_attention(Tensor out, Tensor part_o, Tensor part_ml, Tensor part_sem, Tensor q, Tensor k_cache,
                      Tensor v_cache, Tensor block_tables, Tensor tile_seq, Tensor tile_q0,
                      Tensor q_start, Tensor q_len, Tensor ctx_len, double scale,
-                     int64_t part_tokens, int64_t nparts) {
+                     int64_t part_tokens, int64_t nparts, const std::optional<Tensor>& load) {
   check_bf16(out, "out"); check_bf16(q, "q"); check_bf16(k_cache, "k_cache");
   check_bf16(v_cache, "v_cache");
   check_i32(block_tables, "block_tables"); check_i32(tile_seq, "tile_seq");
@@ -226,6 +226,10 @@ void paged_attention(Tensor out, Tensor part_o, Tensor part_ml, Tensor part_sem,
     TORCH_CHECK(part_sem.numel() >= (int64_t)num_tiles * Hkv, "part_sem too small");
     sem = part_sem.data_ptr<int>();
   }
+  if (load) {  // {keys, tiles that have any} of the launch's sequences, summed over its tiles
+    check_i32(*load, "load");
+    TORCH_CHECK(load->numel() >= 2, "load");
+  }
   c10::DeviceGuard g(q.device());
   const float scale_log2 = (float)(scale * 1.4426950408889634);
   mlop::launch_paged_attention(
@@ -234,7 +238,7 @@ void paged_attention(Tensor out, Tensor part_o, Tensor part_ml, Tensor part_sem,
       v_cache.data_ptr(), block_tables.data_ptr<int>(), (int)block_tables.stride(0),
       tile_seq.data_ptr<int>(), tile_q0.data_ptr<int>(), q_start.data_ptr<int>(),
       q_len.data_ptr<int>(), ctx_len.data_ptr<int>(), num_tiles, Hq, Hkv, scale_log2,
-      (int)part_tokens, (int)nparts, (int)k_cache.size(0), sem, cur_stream());
+      (int)part_tokens, (int)nparts, (int)k_cache.size(0), sem, load ? load->data_ptr<int>() : nullptr, cur_stream());
 }
 
 // ---- lazily backed KV arenas (vmm.hip)
@@ -1026,7 +1030,7 @@ TORCH_LIBRARY(mlop, m) {
   m.def("paged_attention(Tensor(a!) out, Tensor(b!) part_o, Tensor(c!) part_ml, Tensor(d!) part_sem, Tensor q, "
         "Tensor k_cache, Tensor v_cache, Tensor block_tables, Tensor tile_seq, Tensor tile_q0, "
         "Tensor q_start, Tensor q_len, Tensor ctx_len, float scale, int part_tokens, "
-        "int nparts) -> ()");
+        "int nparts, Tensor? load=None) -> ()");
 }
 
 TORCH_LIBRARY_IMPL(mlop, CUDA, m) {

@@ -35,7 +35,7 @@ void launch_paged_attention(void* out, float* part_o, float* part_ml, const void
                             const int* tile_seq, const int* tile_q0, const int* q_start,
                             const int* q_len, const int* ctx_len, int num_tiles, int Hq, int Hkv,
                             float scale_log2, int part_tokens, int nparts, int num_blocks,
-                            int* sem, hipStream_t st);
+                            int* sem, const int* load, hipStream_t st);
 int flash_persist(int set);  // 0: one workgroup per flash item; n: persistent grid, n per CU
 int flash_stream(int set);   // 1: the persistent grid streams K / V pairs and Q across tiles
 int gemm_grouped_balance(int set);  // 1: equal row ranges per expert m-tile; 2: + the 16-row MFMA skip

@@ -61,6 +61,9 @@ class AttnMeta:
     # rows of the larger step in whose place this one runs (a decode graph between the listed sizes; 0: none): what that
     # one keeps in 32 bits between its products, this one does too
     like: int = 0
+    # int32 [2]: keys of the decode tiles' sequences, summed over the tiles, and the tiles that have any (None: the kernel
+    # sums them itself)
+    load: torch.Tensor | None = None
 
 
 # 128-token partitions: one 32-token page pair per wave at batch 1 (256: 312 tok/s, 128: 322,
@@ -144,7 +147,7 @@ class MetaBuffers:
         self._pwork = np.zeros(self.max_tiles, dtype=np.int32)  # per flash tile: keys it reads
         sizes = [("positions", max_tokens), ("slots", max_tokens), ("tile_seq", self.max_tiles),
                  ("tile_q0", self.max_tiles), ("ptile_seq", self.max_tiles), ("ptile_q0", self.max_tiles),
-                 ("q_start", max_seqs), ("q_len", max_seqs), ("ctx_len", max_seqs)]
+                 ("q_start", max_seqs), ("q_len", max_seqs), ("ctx_len", max_seqs), ("load", 2)]
         self.chunk = self.step_chunk = chunk
         self.n_items = self.n_crows = 0  # recurrent chunk items / rows of the last fill
         self.expand_window = expand_window
@@ -251,7 +254,8 @@ class MetaBuffers:
             ptile_seq=self.view_d("ptile_seq", num_ptiles), ptile_q0=self.view_d("ptile_q0", num_ptiles),
             q_start=self.view_d("q_start"), q_len=self.view_d("q_len"), ctx_len=self.view_d("ctx_len"),
             part_tokens=part_tokens, nparts=nparts, part_o=self.part_o, part_ml=self.part_ml,
-            logits_idx=self.lidx_d[:n_logits], num_tokens=num_tokens, part_sem=self.part_sem, **self._chunk_views())
+            logits_idx=self.lidx_d[:n_logits], num_tokens=num_tokens, part_sem=self.part_sem,
+            load=self.view_d("load", 2), **self._chunk_views())
 
     def _chunk_views(self) -> dict:
         d = {}
@@ -273,6 +277,7 @@ class MetaBuffers:
         hold the pages covering ctx_lens.  want_logits[i] (default all): emit a
         logits row for sequence i's last token; a list of token offsets emits those.  Returns (T, num_tiles, n_logits);
         the flash-tile count is left in ``self.npt``."""
+        self.view_h("load")[:2] = 0
         return self._fill_ragged(0, 0, 0, rows, q_lens, ctx_lens, token_ids_per_seq, want_logits)
 
     def fill_mixed(self, d_rows: np.ndarray, d_ctx: np.ndarray, d_last: np.ndarray,
@@ -296,7 +301,7 @@ class MetaBuffers:
             self.step_chunk = self.chunk * (2 if sum(int(q) for q in q_lens) >= 64 * self.chunk else 1)
         max_flash_q = 0
         qs_h, ql_h, cl_h = self.view_h("q_start"), self.view_h("q_len"), self.view_h("ctx_len")
-        qt = self.qt
+        qt, load_h = self.qt, self.view_h("load")
         for i, row in enumerate(rows):
             ql, cl = int(q_lens[i]), int(ctx_lens[i])
             qs_h[row], ql_h[row], cl_h[row] = t, ql, cl
@@ -315,6 +320,7 @@ class MetaBuffers:
                 ntile = (ql + qt - 1) // qt
                 ts_h[nt:nt + ntile] = row
                 tq_h[nt:nt + ntile] = np.arange(ntile, dtype=np.int32) * qt
+                load_h[:2] += (ntile * cl, ntile)
                 nt += ntile
             if self.chunk and ql > 1:
                 n = -(-ql // self.step_chunk)
@@ -357,6 +363,7 @@ class MetaBuffers:
         qs_h[rows] = np.arange(B, dtype=np.int32)
         ql_h[rows] = 1
         cl_h[rows] = ctx_lens
+        self.view_h("load")[:2] = (int(np.sum(ctx_lens)), B)
         self.ids_hn[:B] = last_tokens
         self.lidx_hn[:B] = np.arange(B)  # the identity: decode graphs skip the gather (Engine.capture_graphs)
         if pad_to > B:
