@@ -439,7 +439,10 @@ bool gemm_rs(Tensor out, Tensor a, Tensor w, Tensor ss_in, double eps, int64_t e
   if (decode_form(M, N, K, epi)) {  // PRO_RS, row factors from the streamed chunks (ss_in unused)
     if (!mlop::decode_chain_takes((int)M, (int)N, (int)K, (int)epi)) return false;
     c10::DeviceGuard g(a.device());
-    if (!mlop::chain_on_ws((int)M, (int)N, (int)K, (int)epi))
+    if (epi == 1 && mlop::chain_on_mid((int)M, (int)N, (int)K))
+      mlop::launch_mid_self(a.data_ptr(), (int)a.stride(0), w.data_ptr(), out.data_ptr(), (int)out.stride(0), (int)M, (int)N,
+                            (int)K, (float)eps, cur_stream());
+    else if (!mlop::chain_on_ws((int)M, (int)N, (int)K, (int)epi))
       mlop::launch_gemv_rs(a.data_ptr(), (int)a.stride(0), w.data_ptr(), out.data_ptr(), (int)out.stride(0), (int)M,
                            (int)N, (int)K, (int)epi, mlop::RopeEpi{}, (float)eps, cur_stream());
     else

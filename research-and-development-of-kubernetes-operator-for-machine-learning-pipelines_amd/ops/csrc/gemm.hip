@@ -1358,7 +1358,7 @@ static bool mid_plan(int M, int N, int K, Plan& p) {
   if (M > max_m || K < kBK || K % kBK || N % 8) return false;  // (no K-step: gemm_kernel writes the empty sums)
   if (M <= 64 && g_small_tile != 1) return false;              // one of gemm_kernel's tiles is asked for
   const int m_tiles = M <= 256 ? 1 : 2, rows = (M + m_tiles - 1) / m_tiles;
-  const int bm = rows <= 64 ? 64 : (rows + 31) / 32 * 32;
+  const int bm = (rows + 31) / 32 * 32;
   const int t256 = (N + 255) / 256 * m_tiles, t128 = (N + 127) / 128 * m_tiles, nk = K / kBK;
   int s = 1;
   if (t256 < fill && t128 < fill) {
@@ -1721,7 +1721,7 @@ bool launch_gemm_rope(const void* A, int lda, const void* B, int M, int N, int K
                       hipStream_t st) {
   if (M == 0) return true;
   if (!gemm_rope_supported(M, N, K)) return false;
-  if (ws_prefer(M, N, K, EPI_ROPE) && lda % 8 == 0) {  // up to 16 rows: the weight-streaming MFMA kernel
+  if (ws_prefer(M, N, K, EPI_ROPE) && lda % 8 == 0) {  // up to 32 rows: the weight-streaming MFMA kernel
     launch_ws(A, lda, B, K, nullptr, 0, M, N, K, EPI_ROPE, false, re, 0.f, st);
     return true;
   }
@@ -1853,6 +1853,22 @@ bool launch_mid_rs(const void* A, int lda, const void* B, void* out, int ldo, in
   launch_plan<EPI_SILU_MUL, false>(p, (const uint16_t*)A, lda, (const uint16_t*)B, K, (uint16_t*)out, ldo, nullptr,
                                    M, N, K, nullptr, 0, st, re);
   return true;
+}
+
+// gate_up of the decode norm chain on the weight stream: out = SiLU-mul(diag(rsqrt(mean(a^2) + eps)) . A . B^T), the rows'
+// factors from the rows themselves
+bool mid_self_ok(int M, int N, int K) {
+  Plan p{};
+  return N % 32 == 0 && M <= 64 && g_dp[0] < 0 && mid_plan(M, N, K, p) && p.splits == 1;
+}
+
+void launch_mid_self(const void* A, int lda, const void* B, void* out, int ldo, int M, int N, int K, float eps, hipStream_t st) {
+  Plan p{};
+  mid_plan(M, N, K, p);
+  RopeEpi re{};
+  re.ss_inv_k = 1.f / (float)K;
+  re.ss_eps = eps;
+  launch_mid(2, p.BM, p.BN, (const uint16_t*)A, lda, (const uint16_t*)B, K, (uint16_t*)out, ldo, nullptr, M, N, K, 1, K, st, re);
 }
 
 void gemm_plan(int M, int N, int K, int out[5]) {

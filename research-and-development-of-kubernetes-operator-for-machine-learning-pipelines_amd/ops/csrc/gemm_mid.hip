@@ -20,7 +20,7 @@
 // (the weights are the MFMA's first operand): a lane holds four neighbouring columns, gate and up of an
 // output sit in one lane, and nothing is staged for the epilogue.
 // Measured (cold weights, us, the LDS-ring tiles -> this kernel): gate_up 28672 x 4096 at 16 / 64 / 100 /
-// 150 rows 42 -> 37, 49 -> 39, 59 -> 45, 68 -> 51; lm_head 128256 x 4096 at 64 / 100 /
+// 150 rows 42 -> 37, 49 -> 39, 59 -> 45, 68 -> 51 (24 rows, 32-row tiles: 39.5 -> 36.7); lm_head 128256 x 4096 at 64 / 100 /
 // 150 / 256 rows 211 -> 168, 247 -> 175, 280 -> 181, 297 -> 251; down 4096 x 14336 with
 // its reduce at 100 / 150 / 300 rows 37 -> 34, 46 -> 39, 68 -> 56.
 #include "common.h"
@@ -35,6 +35,19 @@ namespace {
 
 __device__ __forceinline__ int mid_swz(int r) { return (r >> 1) & 7; }
 
+// c + the squares of eight bf16
+__device__ __forceinline__ float mid_sq8(const bf16x8& v, float c) {
+  typedef __attribute__((ext_vector_type(2))) __bf16 bf2;
+  const u32x4 w = __builtin_bit_cast(u32x4, v);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const uint32_t x = w[e];  // (bit_cast of the element itself reads the vector's first)
+    const bf2 p = __builtin_bit_cast(bf2, x);
+    c = __builtin_amdgcn_fdot2_f32_bf16(p, p, c, false);
+  }
+  return c;
+}
+
 // s_waitcnt vmcnt(min(n, MAX) * PER) for a wave-uniform n
 template <int MAX, int PER>
 __device__ __forceinline__ void wait_stages(int n) {
@@ -47,20 +60,21 @@ __device__ __forceinline__ void wait_stages(int n) {
 }
 
 // Tasks (column tile, row tile, K range), row tile fastest; a workgroup takes lid, lid + G, ...  SA / SB: ring
-// depths in K-steps of 64.  EPI 0: plain (with an activation, RopeEpi::act), 1: gate / up; several K ranges leave
-// fp32 slabs [range][M][N] in ws instead, non-temporal always (a second form of the stores cost 3 % at 200 rows).
-template <int BM, int BN, int WM, int WN, int SA, int SB, int EPI>
+// depths in K-steps of 64.  EPI 0: plain (with an activation, RopeEpi::act), 1: gate / up, 2: gate / up of A's rows scaled by
+// their RMSNorm factors, whose sums of squares a wave adds up from its own fragments (one K range: it sees whole rows); several
+// K ranges leave fp32 slabs [range][M][N] in ws instead, non-temporal always (a second form of the stores cost 3 % at 200 rows).
+template <int BM, int BN, int WM, int WN, int SA, int SB, int EPI, bool BEHIND>
 __global__ void __launch_bounds__(WM * WN * 64) gemm_mid_kernel(
     const uint16_t* __restrict__ A, int lda, const uint16_t* __restrict__ B, int ldb, uint16_t* __restrict__ C, int ldc,
     float* __restrict__ ws, int M, int N, int K, int k_chunk, int m_tiles, int n_splits, int n_tasks, RopeEpi re) {
   constexpr int NW = WM * WN, HW = NW / 2;   // half of the waves issue A, half B
   constexpr int WTM = BM / WM, WTN = BN / WN, TM = WTM / 16, TN = WTN / 16;
   // Each half's reads stand behind the first MFMA of the half before: the compiler waits for every LDS read in flight before
-  // a fragment's first use, so reads that stand before it overlap with nothing.  Not for 64 rows, where two workgroups
+  // a fragment's first use, so reads that stand before it overlap with nothing.  Not where two workgroups of 64 rows
   // share a CU and overlap each other, and 256 x 256, which would spill.  (Cold weights, us, reads before -> behind with the
   // rings as deep for A as for B: gate_up 28672 x 4096 at 100 / 150 / 192 rows 50 -> 47, 56 -> 51.5, 62 -> 59, down of
   // Llama-3-70B 8192 x 28672 at 150 / 300 107 -> 100, 191 -> 182, its gate_up at 100 / 224 153 -> 148, 220 -> 213.)
-  constexpr bool kBehind = BM > 64 && BM + BN < 512;
+  constexpr bool kBehind = BEHIND;
   constexpr int PA = BM / 8 / HW, PB = BN / 8 / HW;  // 1-KiB pieces per issuing wave and K-step
   static_assert(BM % (8 * HW) == 0 && BN % (8 * HW) == 0 && WTM % 16 == 0 && WTN % 16 == 0, "tile");
   static_assert((SA - 1) * PA < 64 && (SB - 1) * PB < 64, "vmcnt");
@@ -147,6 +161,9 @@ __global__ void __launch_bounds__(WM * WN * 64) gemm_mid_kernel(
   const int depth = is_b ? SB : SA;
   for (int s = 0; s < depth; ++s) issue();
 
+  float ss[TM];
+#pragma unroll
+  for (int i = 0; i < TM; ++i) ss[i] = 0.f;
   f32x4 acc[TM][TN];
 #pragma unroll
   for (int i = 0; i < TM; ++i)
@@ -172,9 +189,11 @@ __global__ void __launch_bounds__(WM * WN * 64) gemm_mid_kernel(
     acc[0][0] = mfma16(fb[kk][0], fa[kk][0], acc[0][0]);
     behind();
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
+    for (int i = 0; i < TM; ++i) {
 #pragma unroll
       for (int j = i == 0; j < TN; ++j) acc[i][j] = mfma16(fb[kk][j], fa[kk][i], acc[i][j]);
+      if constexpr (EPI == 2) ss[i] = mid_sq8(fa[kk][i], ss[i]);
+    }
   };
   auto read_behind = [&](auto kk_, bool more) {
     if constexpr (kBehind) {
@@ -222,7 +241,9 @@ __global__ void __launch_bounds__(WM * WN * 64) gemm_mid_kernel(
       } else {
         static_assert(EPI == 0 || TN % 2 == 0, "gate / up pairs");
         // (launch_mid_rs: the row's RMSNorm factor first)
-        const float f = re.ss_in != nullptr ? rsqrtf(re.ss_in[m] * re.ss_inv_k + re.ss_eps) : 1.f;
+        float f;
+        if constexpr (EPI == 2) f = rsqrtf(sum_x16_x32(ss[i]) * re.ss_inv_k + re.ss_eps);
+        else f = re.ss_in != nullptr ? rsqrtf(re.ss_in[m] * re.ss_inv_k + re.ss_eps) : 1.f;
 #pragma unroll
         for (int j = 0; j < TN; j += 2) {
           const int n = nc + j * 16;
@@ -264,9 +285,11 @@ __global__ void __launch_bounds__(WM * WN * 64) gemm_mid_kernel(
     if (++c_kt == c_nk) {
       epilogue();
 #pragma unroll
-      for (int i = 0; i < TM; ++i)
+      for (int i = 0; i < TM; ++i) {
+        ss[i] = 0.f;
 #pragma unroll
         for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
       c_kt = 0;
       c_task += G;
       if (c_task < n_tasks) place(c_task, c_bx, c_by, c_bz, c_nk);
@@ -274,12 +297,12 @@ __global__ void __launch_bounds__(WM * WN * 64) gemm_mid_kernel(
   }
 }
 
-template <int BM, int BN, int WM, int WN, int SA, int SB, int EPI>
+template <int BM, int BN, int WM, int WN, int SA, int SB, int EPI, bool BEHIND>
 static void run_mid(const uint16_t* A, int lda, const uint16_t* B, int ldb, uint16_t* C, int ldc, float* ws, int M, int N,
                     int K, int splits, int k_chunk, hipStream_t st, const RopeEpi& re) {
   constexpr size_t lds = (size_t)(SA * BM + SB * BN) * 128;
   static_assert(lds <= 163840, "LDS budget");
-  auto kern = gemm_mid_kernel<BM, BN, WM, WN, SA, SB, EPI>;
+  auto kern = gemm_mid_kernel<BM, BN, WM, WN, SA, SB, EPI, BEHIND>;
   static const bool attr =
       hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess;
   (void)attr;
@@ -295,29 +318,41 @@ static void run_mid(const uint16_t* A, int lda, const uint16_t* B, int ldb, uint
 
 void launch_mid(int epi, int bm, int bn, const uint16_t* A, int lda, const uint16_t* B, int ldb, uint16_t* C, int ldc,
                 float* ws, int M, int N, int K, int splits, int k_chunk, hipStream_t st, const RopeEpi& re) {
-#define MLOP_MID(m, n, wm, wn, sa, sb)                                                                                  \
-  if (bm == m && bn == n) {                                                                                             \
-    if (epi == 0) return run_mid<m, n, wm, wn, sa, sb, 0>(A, lda, B, ldb, C, ldc, ws, M, N, K, splits, k_chunk, st, re); \
-    return run_mid<m, n, wm, wn, sa, sb, 1>(A, lda, B, ldb, C, ldc, ws, M, N, K, splits, k_chunk, st, re);               \
+#define MLOP_MID_(m, n, wm, wn, sa, sb, e, behind) \
+  return run_mid<m, n, wm, wn, sa, sb, e, behind>(A, lda, B, ldb, C, ldc, ws, M, N, K, splits, k_chunk, st, re)
+#define MLOP_MID(m, n, wm, wn, sa, sb, behind)               \
+  if (bm == m && bn == n) {                                  \
+    if (epi == 0) MLOP_MID_(m, n, wm, wn, sa, sb, 0, behind); \
+    if (epi == 1) MLOP_MID_(m, n, wm, wn, sa, sb, 1, behind); \
+    if constexpr (m <= 64) MLOP_MID_(m, n, wm, wn, sa, sb, 2, behind); \
   }
-  // ring depths: what fits 160 KB (64 x 128: half of it, two workgroups per CU).  With 128 columns as deep for A as for B: with
+  // ring depths: what fits 160 KB (half of it where two workgroups share a CU).  With 128 columns as deep for A as for B: with
   // A two or three deep and the rest for B 0 - 4 % slower (qkv, gate_up and down at 100 - 160 rows; 8192 x 28672 at 112 - 128 rows 2 %
-  // faster); not 224 rows, where it made no difference.
-  MLOP_MID(64, 128, 2, 4, 2, 4)
-  MLOP_MID(96, 128, 2, 4, 5, 6)
-  MLOP_MID(128, 128, 2, 4, 5, 5)
-  MLOP_MID(160, 128, 2, 4, 4, 5)
-  MLOP_MID(192, 128, 2, 4, 4, 4)
-  MLOP_MID(224, 128, 2, 4, 2, 6)
-  MLOP_MID(256, 128, 4, 2, 3, 4)
-  MLOP_MID(64, 256, 2, 4, 3, 4)
-  MLOP_MID(96, 256, 2, 4, 2, 4)
-  MLOP_MID(128, 256, 2, 4, 3, 3)
-  MLOP_MID(160, 256, 2, 4, 3, 3)
-  MLOP_MID(192, 256, 2, 4, 2, 3)
-  MLOP_MID(224, 256, 2, 4, 2, 3)
-  MLOP_MID(256, 256, 2, 4, 2, 3)
+  // faster); not 224 rows, where it made no difference.  64 x 128: the whole of it for grids of one workgroup per CU (28672 x 4096
+  // at 33 / 64 rows 39.9 -> 37.7, 40.9 -> 39.3 us, 24576 x 3072 at 33 33.9 -> 30.3), half for larger ones (40960 x 4096 at 33 66
+  // against 72).  32 rows: half (28672 x 4096 at 24 rows 39.5 -> 36.7 us, with the whole 38.4).
+  const long tasks = (long)((N + bn - 1) / bn) * ((M + bm - 1) / bm) * splits;
+  MLOP_MID(32, 128, 2, 4, 3, 4, true)
+  if (tasks <= kCus) {
+    MLOP_MID(64, 128, 2, 4, 4, 6, true)
+  }
+  MLOP_MID(64, 128, 2, 4, 2, 4, false)
+  MLOP_MID(96, 128, 2, 4, 5, 6, true)
+  MLOP_MID(128, 128, 2, 4, 5, 5, true)
+  MLOP_MID(160, 128, 2, 4, 4, 5, true)
+  MLOP_MID(192, 128, 2, 4, 4, 4, true)
+  MLOP_MID(224, 128, 2, 4, 2, 6, true)
+  MLOP_MID(256, 128, 4, 2, 3, 4, true)
+  MLOP_MID(32, 256, 2, 4, 2, 4, true)
+  MLOP_MID(64, 256, 2, 4, 3, 4, false)
+  MLOP_MID(96, 256, 2, 4, 2, 4, true)
+  MLOP_MID(128, 256, 2, 4, 3, 3, true)
+  MLOP_MID(160, 256, 2, 4, 3, 3, true)
+  MLOP_MID(192, 256, 2, 4, 2, 3, true)
+  MLOP_MID(224, 256, 2, 4, 2, 3, true)
+  MLOP_MID(256, 256, 2, 4, 2, 3, false)
 #undef MLOP_MID
+#undef MLOP_MID_
   throw std::runtime_error("gemm_mid: no such tile");
 }
 

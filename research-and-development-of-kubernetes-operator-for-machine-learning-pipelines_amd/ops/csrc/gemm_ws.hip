@@ -353,8 +353,10 @@ int gemm_ws_max_m(int set) {
   return g_ws_max_m;
 }
 
-// and outside the chain: gemm_ws_small_m op, QKV + RoPE gemm_ws_rope_m
-int g_ws_small_m = 16, g_ws_rope_m = 16;
+// and outside the chain: gemm_ws_small_m op, QKV + RoPE gemm_ws_rope_m.  The latter to 32 rows: its RoPE + cache epilogue
+// spares the launch that sums the planner's K ranges (6144 x 4096 at 20 / 32 rows 16.1 + 4 -> 13.0, 16.4 + 4 -> 14.2 us; 10240 x
+// 8192 at 24 / 32 43.8 + 4 -> 41.2, 44.2 + 4 -> 46.1; 3072 x 2048 at 32 9.3 + 3 -> 6.5)
+int g_ws_small_m = 16, g_ws_rope_m = 32;
 
 int gemm_ws_small_m(int set) {
   if (set >= 0) g_ws_small_m = set > 64 ? 64 : set;
@@ -388,7 +390,8 @@ static bool ws_fast(int M, int N, int K) {
 }
 
 bool ws_prefer(int M, int N, int K, int epi) {
-  return M <= std::min(g_ws_max_m, epi == WS_ROPE ? g_ws_rope_m : g_ws_small_m) && ws_shape(M, N, K, epi) && ws_fast(M, N, K);
+  const int bound = epi == WS_ROPE ? (g_ws_max_m ? g_ws_rope_m : 0) : std::min(g_ws_max_m, g_ws_small_m);
+  return M <= bound && ws_shape(M, N, K, epi) && ws_fast(M, N, K);
 }
 
 // (the third argument chose a form of the weight loads that is no more)
@@ -405,6 +408,10 @@ int decode_chain_max_m() { return g_ws_max_m > gemv_chain_max_m() ? g_ws_max_m :
 bool chain_on_ws(int M, int N, int K, int epi) {
   return ws_takes(M, N, K, epi) && (M > gemv_chain_max_m() || ws_fast(M, N, K));
 }
+
+// and gate_up on gemm_mid.hip's stream, where that takes it: above 8 rows A is what a CU of this kernel takes in (28672 x
+// 4096 at 16 rows 42.3 -> 37.1 us, at 9 39.6 -> 37.0; at 8 35.8 here, 36.8 there)
+bool chain_on_mid(int M, int N, int K) { return M > 8 && M <= g_ws_max_m && mid_self_ok(M, N, K); }
 
 bool decode_chain_takes(int M, int N, int K, int epi) {
   return gemv_chain_takes(M, N, K, epi) || (ws_takes(M, N, K, epi) && ((long)N * K >= 1 << 20));

@@ -213,6 +213,8 @@ int gemm_mid_chain(int set);
 bool mid_chain_ok(int M, int N, int K, int epi);
 bool launch_mid_res_ss(const void* A, int lda, const void* B, void* residual, int ldr, int M, int N, int K,
                        float* ss_tot, hipStream_t st);
+bool mid_self_ok(int M, int N, int K);
+void launch_mid_self(const void* A, int lda, const void* B, void* out, int ldo, int M, int N, int K, float eps, hipStream_t st);
 bool launch_mid_rs(const void* A, int lda, const void* B, void* out, int ldo, int M, int N, int K,
                    const float* ss_tot, float eps, hipStream_t st);
 // the decode norm chain's forms: the GEMV up to gemv_chain_max_m() rows, the weight-streaming MFMA kernel up to
@@ -220,6 +222,7 @@ bool launch_mid_rs(const void* A, int lda, const void* B, void* out, int ldo, in
 int decode_chain_max_m();
 bool decode_chain_takes(int M, int N, int K, int epi);
 bool chain_on_ws(int M, int N, int K, int epi);
+bool chain_on_mid(int M, int N, int K);
 void launch_ws(const void* A, int lda, const void* B, int ldb, void* C, int ldc, int M, int N, int K, int epi,
                bool rs, const RopeEpi& re, float eps, hipStream_t st);
 int gemv_chain_max_m();
