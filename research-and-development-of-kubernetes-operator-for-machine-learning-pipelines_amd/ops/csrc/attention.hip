@@ -658,7 +658,7 @@ __device__ __forceinline__ void flash32_item(
   constexpr int STAGES = 3;
   constexpr int STAGE = 4 * kBS * kD;    // bf16 per stage: K page A | K page B | V page A | V page B
   constexpr int PAGE = kBS * kD;
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int s = ptile_seq[tile], q0 = ptile_q0[tile];
   const int ql = q_len[s], ctx = ctx_len[s], qs = q_start[s];
   const int last_q = min(q0 + QB, ql) - 1;
@@ -694,55 +694,61 @@ __device__ __forceinline__ void flash32_item(
   const int kkey = wid * 4 + (lane >> 4);
   // K image: chunk c of key k at slot c ^ k on BOTH pages (the 32x32 A-operand reads take keys
   // {0-3, 12-15} of one page and {4-11} of the other per 16-lane group: 16 distinct slots)
-  const int k_off = kvh * PAGE + kkey * kD + (((lane & 15) ^ (kkey & 15)) << 3);
-  const int v_off = kvh * PAGE + kkey * kD + (((lane & 15) ^ vswz(kkey)) << 3);
-  auto page_of = [&](int idx) { return idx < n_pages ? min(max(bt[idx], 0), num_blocks - 1) : -1; };
-  auto issue_pages = [&](int buf, int pgA, int pgB) {
-    if (pgB < 0) pgB = pgA;
-    uint16_t* base = smem + buf * STAGE + wid * 512;
-    __builtin_amdgcn_global_load_lds((const void*)(kc + pgA * page_stride + k_off), (lds_void_t*)(base), 16, 0, 0);
-    __builtin_amdgcn_global_load_lds((const void*)(kc + pgB * page_stride + k_off), (lds_void_t*)(base + PAGE), 16, 0, 0);
-    __builtin_amdgcn_global_load_lds((const void*)(vc + pgA * page_stride + v_off), (lds_void_t*)(base + 2 * PAGE), 16, 0, 0);
-    __builtin_amdgcn_global_load_lds((const void*)(vc + pgB * page_stride + v_off), (lds_void_t*)(base + 3 * PAGE), 16, 0, 0);
+  const uint32_t k_off = 2u * (uint32_t)(kkey * kD + (((lane & 15) ^ (kkey & 15)) << 3));
+  const uint32_t v_off = 2u * (uint32_t)(kkey * kD + (((lane & 15) ^ vswz(kkey)) << 3));
+  const uint16_t* kh = kc + kvh * PAGE;
+  const uint16_t* vh = vc + kvh * PAGE;
+  struct Pages {
+    int a, b;
   };
+  auto pages_of = [&](int pp) { return Pages{bt[min(2 * pp, n_pages - 1)], bt[min(2 * pp + 1, n_pages - 1)]}; };
+  // a pair's two pages of K / of V into slot st of their ring
+  const uint32_t ring = (uint32_t)(uintptr_t)smem + wid * 1024;
+  auto issue = [&](const uint16_t* head, uint32_t off, uint32_t slot, Pages pg) {
+    auto page = [&](int id) {
+      return __builtin_amdgcn_make_buffer_rsrc((void*)(head + min(max(id, 0), num_blocks - 1) * page_stride), 0, 2 * PAGE, 0x00020000);
+    };
+    lds_dma16(page(pg.a), ring + slot, off, 0);
+    lds_dma16(page(pg.b), ring + slot + 2 * PAGE, off, 0);
+  };
+  constexpr uint32_t SLOT = 4 * PAGE, RING_V = STAGES * SLOT;  // bytes
   // K fragment t of this lane: key col of the pair (page col >> 4, row col & 15), chunk 2t + h at
   // slot (2t + h) ^ (col & 15): byte k_b0 ^ 32 t
   const int k15 = col & 15;
   const uint32_t k_b0 = (uint32_t)(uintptr_t)smem + (uint32_t)((col >> 4) * PAGE * 2 + k15 * 256 + ((h ^ k15) << 4));
-  const uint32_t v_b0 = (uint32_t)(uintptr_t)smem + 2 * PAGE * 2 + vt32_base(lane);
-
-  // S^T of the pair in ring slot ST: K fragment t at k_b0 ^ 32 t, four reads in flight (inline
-  // asm with counted waits: as plain loads the compiler reused one register set and waited
-  // lgkmcnt(0) in front of every MFMA, one LDS latency per fragment)
-  auto qk = [&](auto st_tag) {
-    constexpr uint32_t so = (uint32_t)(decltype(st_tag)::value * STAGE * 2);
-    uint32_t kb = k_b0;
-    asm volatile("" : "+v"(kb));
-    auto kread = [&](int t, bf16x8& f) {
-      asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(f) : "v"(kb ^ (32u * t)), "n"(so));
-    };
-    f32x16 sc;
+  const uint32_t v_b0 = (uint32_t)(uintptr_t)smem + RING_V + vt32_base(lane);
+  // The fragment reads are inline asm with counted waits: as plain loads the compiler reused one register set and waited
+  // lgkmcnt(0) before every MFMA, and, for V, vmcnt(0) (it cannot tell them from the LDS-DMA in flight).  No scalar load may
+  // be in flight beside them (it would be counted): page ids are loaded where a step's last read has landed.
+#define MLOP_KREAD(t, f, so) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(f) : "v"(k_b0 ^ (32u * (t))), "n"(so))
+#define MLOP_WAIT_K(n, f) asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(f) : "n"(n))
+  // both pages' fragments of dim block dblk: (lo, hi) of page A, of page B; vx: a ring slot's bytes
+#define MLOP_VREAD(dblk, r, vx, so)                                                                                    \
+  asm volatile("ds_read_b64_tr_b16 %0, %4 offset:%6\nds_read_b64_tr_b16 %1, %5 offset:%7\n"                           \
+               "ds_read_b64_tr_b16 %2, %4 offset:%8\nds_read_b64_tr_b16 %3, %5 offset:%9\n"                           \
+               : "=&v"(r[0]), "=&v"(r[1]), "=&v"(r[2]), "=&v"(r[3])                                                   \
+               : "v"((v_b0 ^ (64u * (dblk))) + (vx)), "v"((v_b0 ^ (64u * (dblk)) ^ 32u) + (vx)), "n"(so),             \
+                 "n"((so) + 2048u), "n"((so) + 4096u), "n"((so) + 6144u))
+#define MLOP_WAIT_V(n, r) \
+  asm volatile("s_waitcnt lgkmcnt(%4)" : "+v"(r[0]), "+v"(r[1]), "+v"(r[2]), "+v"(r[3]) : "n"(n))
+  auto frag = [&](const v4s16& lo, const v4s16& hi) {
+    bf16x8 f;
 #pragma unroll
-    for (int e = 0; e < 16; ++e) sc[e] = 0.f;
-    bf16x8 kf[4];
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // nothing else (SMEM) in the counts below
-#pragma unroll
-    for (int t = 0; t < 4; ++t) kread(t, kf[t]);
-#pragma unroll
-    for (int t = 0; t < 8; ++t) {
-      bf16x8& f = kf[t & 3];
-      if (t <= 4) asm volatile("s_waitcnt lgkmcnt(3)" : "+v"(f));
-      else if (t == 5) asm volatile("s_waitcnt lgkmcnt(2)" : "+v"(f));
-      else if (t == 6) asm volatile("s_waitcnt lgkmcnt(1)" : "+v"(f));
-      else asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(f));
-      sc = mfma32(f, qf[t], sc);
-      if (t + 4 < 8) kread(t + 4, kf[t & 3]);
+    for (int e = 0; e < 4; ++e) {
+      f[e] = lo[e];
+      f[4 + e] = hi[e];
     }
-    return sc;
+    return f;
   };
-  // online softmax on the lane's 16 keys of its q column (raw score units; the scale folds into
-  // the exponent's FMA) -> P^T fragments of the two k-steps; O and l rescaled when the max moved
-  auto softmax = [&](f32x16 sc, int pp, bf16x8 (&pf)[2]) {
+
+  float alpha = 1.f, mc = -m * scale_log2;
+  bool resc = false;
+  // Row max of a pair's scores (raw units; the scale folds into the exponent's FMA).  Deferred rescale: the running max
+  // moves only when some row's new max exceeds it by more than 2^kRescaleLog2 in exp2 units (always on a row's first
+  // keys: m starts at -1e30); otherwise P stays scaled against the old max, <= 2^8, which bf16 P and f32 O / l carry
+  // exactly as well.  The halves of a row's keys meet only when it does.  O takes the factor (resc) once the pair before
+  // has been added to it.
+  auto row_max = [&](f32x16& sc, int pp) {
     if (pp * 32 + 31 > wg_min_pos) {  // a pair crossing the workgroup's causal diagonal
       // (a side effect keeps this a branch: if-converted, the 47 compare / select / add of the
       // mask ran on every pair, a third of the loop's VALU)
@@ -753,109 +759,196 @@ __device__ __forceinline__ void flash32_item(
         sc[r] = tok <= pos_r ? sc[r] : -INFINITY;
       }
     }
-    float mx = fmaxf(fmaxf(sc[0], sc[1]), sc[2]);
-#pragma unroll
-    for (int r = 3; r < 15; r += 2) mx = fmaxf(fmaxf(mx, sc[r]), sc[r + 1]);
-    mx = fmaxf(mx, sc[15]);
-    {
+    const float a = fmaxf(fmaxf(sc[0], sc[1]), sc[2]), b = fmaxf(fmaxf(sc[3], sc[4]), sc[5]);
+    const float c = fmaxf(fmaxf(sc[6], sc[7]), sc[8]), d = fmaxf(fmaxf(sc[9], sc[10]), sc[11]);
+    const float e = fmaxf(fmaxf(sc[12], sc[13]), sc[14]);
+    float mx = fmaxf(fmaxf(fmaxf(a, b), c), fmaxf(fmaxf(d, e), sc[15]));
+    if (__ballot(fmaf(mx, scale_log2, mc) > kRescaleLog2)) {
       const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
       mx = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
-    }
-    // deferred rescale (cdna_hip_programming.md T13): the running max moves only when some row's
-    // new max exceeds it by more than 2^kRescaleLog2 in exp2 units (always on a row's first
-    // keys: m starts at -1e30); otherwise P stays scaled against the old max, <= 2^8, which
-    // bf16 P and f32 O / l carry exactly as well.  The decision covers this pair's P and is
-    // taken before it is exponentiated, with the previous pair's P.V complete, so O, l and P
-    // all see the same factor.
-    float alpha = 1.f;
-    if (__ballot((mx - m) * scale_log2 > kRescaleLog2)) {
       const float m_new = fmaxf(m, mx);
       alpha = fast_exp2((m - m_new) * scale_log2);
       m = m_new;
+      mc = -m * scale_log2;
+      l *= alpha;
+      resc = true;
+    }
+  };
+  auto rescale = [&]() {
+    if (resc) {
+      asm volatile("");
 #pragma unroll
       for (int d = 0; d < 4; ++d) o[d] *= alpha;
-      l *= alpha;
+      resc = false;
     }
-    const float mc = -m * scale_log2;
-    float rs = 0.f;
-    u32x4 w[2];
-#pragma unroll
-    for (int r = 0; r < 16; r += 2) {
-      const float p0 = fast_exp2(fmaf(sc[r], scale_log2, mc)), p1 = fast_exp2(fmaf(sc[r + 1], scale_log2, mc));
-      rs += p0 + p1;
-      w[r >> 3][(r & 7) >> 1] = cvt_pk_bf16(p0, p1);
-    }
-    pf[0] = __builtin_bit_cast(bf16x8, w[0]);
-    pf[1] = __builtin_bit_cast(bf16x8, w[1]);
-    l += rs;
   };
-  // O^T += V^T . P^T from ring slot ST; the V^T fragment of (dblk, page) = two transposed reads.
-  // The reads are inline asm: as builtins the compiler put s_waitcnt vmcnt(0) in front of them
-  // (it cannot tell them from the in-flight LDS-DMA of the next pairs), which exposed the
-  // latency of the DMA just issued on every pair.  The ring protocol (vmcnt + barrier at the
-  // top of the step) already covers this pair; the asm waits below count only these reads.
-  auto pv = [&](auto st_tag, const bf16x8 (&pf)[2]) {
-    constexpr uint32_t so = (uint32_t)(decltype(st_tag)::value * STAGE * 2);
-    uint32_t vb = v_b0;
-    asm volatile("" : "+v"(vb));
-    // both pages' fragments of dim block dblk: 4 reads, results in (lo, hi) of f0 (page A), f1
-    auto issue = [&](int dblk, v4s16 (&r)[4]) {
-      const uint32_t a0 = vb ^ (64u * dblk), a1 = a0 ^ 32u;
-      asm volatile(
-          "ds_read_b64_tr_b16 %0, %4 offset:%6\n"
-          "ds_read_b64_tr_b16 %1, %5 offset:%7\n"
-          "ds_read_b64_tr_b16 %2, %4 offset:%8\n"
-          "ds_read_b64_tr_b16 %3, %5 offset:%9\n"
-          : "=&v"(r[0]), "=&v"(r[1]), "=&v"(r[2]), "=&v"(r[3])
-          : "v"(a0), "v"(a1), "n"(so), "n"(so + 2048u), "n"(so + 4096u), "n"(so + 6144u));
-    };
-    auto frag = [&](const v4s16& lo, const v4s16& hi) {
-      bf16x8 f;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        f[e] = lo[e];
-        f[4 + e] = hi[e];
-      }
-      return f;
-    };
-    v4s16 ra[4], rb[4];
-    issue(0, ra);
-#pragma unroll
-    for (int dblk = 0; dblk < 4; ++dblk) {
-      v4s16 (&cur)[4] = (dblk & 1) ? rb : ra;
-      v4s16 (&nxt)[4] = (dblk & 1) ? ra : rb;
-      if (dblk < 3) {
-        issue(dblk + 1, nxt);
-        asm volatile("s_waitcnt lgkmcnt(4)" : "+v"(cur[0]), "+v"(cur[1]), "+v"(cur[2]), "+v"(cur[3]));
-      } else {
-        asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(cur[0]), "+v"(cur[1]), "+v"(cur[2]), "+v"(cur[3]));
-      }
-      o[dblk] = mfma32(frag(cur[0], cur[1]), pf[0], o[dblk]);
-      o[dblk] = mfma32(frag(cur[2], cur[3]), pf[1], o[dblk]);
+  // P of element r of the lane's 16 keys of its q column; every second makes a dword of the P^T fragments
+  // (r = 16: the last of them; a pair is packed behind the next element's exponential, which a VALU instruction could not
+  // read at once)
+  float rs, pe[2];
+  auto soft = [&](int r, const f32x16& sc, u32x4 (&w)[2]) {
+    float p = 0.f;
+    if (r < 16) p = fast_exp2(fmaf(sc[r], scale_log2, mc));
+    if (r > 0 && r % 2 == 0) {
+      rs = r == 2 ? pe[0] + pe[1] : rs + (pe[0] + pe[1]);
+      asm volatile("v_cvt_pk_bf16_f32 %0, %2, %3" : "=v"(w[(r - 2) >> 3][((r - 2) & 7) >> 1]), "+v"(rs) : "v"(pe[0]), "v"(pe[1]));
     }
+    if (r < 16) pe[r & 1] = p;
+    else l += rs;
+  };
+  auto zero = []() {
+    f32x16 z;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) z[e] = 0.f;
+    return z;
   };
 
-  issue_pages(0, page_of(0), page_of(1));
-  if (n_pairs > 1) issue_pages(1, page_of(2), page_of(3));
-  int nxtA = page_of(4), nxtB = page_of(5);
-  auto pair_step = [&](auto st_tag, int pp) {
-    constexpr int ST = decltype(st_tag)::value;
-    if (pp + 1 < n_pairs) wait_vmcnt<4>(); else wait_vmcnt<0>();
-    raw_barrier();  // pair pp visible to every wave; ring slot (pp - 1) % 3 free
-    if (pp + 2 < n_pairs) {
-      issue_pages((ST + 2) % STAGES, nxtA, nxtB);
-      nxtA = page_of(2 * pp + 6);
-      nxtB = page_of(2 * pp + 7);
+#define MLOP_SLOT(t)                 \
+  __builtin_amdgcn_sched_barrier(0); \
+  soft(t, sc, wn);                   \
+  __builtin_amdgcn_sched_barrier(0)
+  // Step pp: S(pp + 1) = K . Q^T and O += V^T . P(pp - 1)^T, 16 MFMAs, with an element of P(pp)'s softmax behind each, so
+  // that a wave's matrix and vector work overlap, and not only those of a SIMD's waves.  K is a pair ahead of the softmax
+  // and V a pair behind it: rings of their own.  (pp = 0: no P before.)
+  auto step = [&](auto p_, auto first_, int pp, f32x16& sc, f32x16& sn, const u32x4 (&wp)[2], u32x4 (&wn)[2], Pages p1,
+                  Pages p3) {
+    constexpr int P = decltype(p_)::value;
+    constexpr bool FIRST = decltype(first_)::value;
+    constexpr uint32_t ks = (P + 1) % 3 * SLOT, vs = (P + 2) % 3 * SLOT;
+    if (pp + 2 < n_pairs) wait_vmcnt<4>(); else wait_vmcnt<2>();
+    raw_barrier();  // K of pp + 1 and V of pp - 1 visible to every wave; the slots of K pp and V pp - 2 free
+    issue(vh, v_off, RING_V + ks, p1);
+    if (pp + 3 < n_pairs) issue(kh, k_off, P % 3 * SLOT, p3);
+    row_max(sc, pp);
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the page ids
+    bf16x8 kf[4];
+    v4s16 va[4], vb[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) MLOP_KREAD(t, kf[t], ks);
+    // (reads in flight at each wait: K 4 - 7 behind K 0 - 3, then V's blocks of four)
+    sn = zero();
+    MLOP_WAIT_K(3, kf[0]); sn = mfma32(kf[0], qf[0], sn); MLOP_KREAD(4, kf[0], ks); MLOP_SLOT(0);
+    MLOP_WAIT_K(3, kf[1]); sn = mfma32(kf[1], qf[1], sn); MLOP_KREAD(5, kf[1], ks); MLOP_SLOT(1);
+    MLOP_WAIT_K(3, kf[2]); sn = mfma32(kf[2], qf[2], sn); MLOP_KREAD(6, kf[2], ks); MLOP_SLOT(2);
+    MLOP_WAIT_K(3, kf[3]); sn = mfma32(kf[3], qf[3], sn); MLOP_KREAD(7, kf[3], ks); MLOP_SLOT(3);
+    if constexpr (FIRST) {
+      MLOP_WAIT_K(3, kf[0]); sn = mfma32(kf[0], qf[4], sn); MLOP_SLOT(4); MLOP_SLOT(5);
+      MLOP_WAIT_K(2, kf[1]); sn = mfma32(kf[1], qf[5], sn); MLOP_SLOT(6); MLOP_SLOT(7); MLOP_SLOT(8);
+      MLOP_WAIT_K(1, kf[2]); sn = mfma32(kf[2], qf[6], sn); MLOP_SLOT(9); MLOP_SLOT(10); MLOP_SLOT(11);
+      MLOP_WAIT_K(0, kf[3]); sn = mfma32(kf[3], qf[7], sn); MLOP_SLOT(12); MLOP_SLOT(13); MLOP_SLOT(14); MLOP_SLOT(15);
+    } else {
+      MLOP_WAIT_K(3, kf[0]); sn = mfma32(kf[0], qf[4], sn); MLOP_VREAD(0, va, 0, vs); MLOP_SLOT(4);
+      MLOP_WAIT_K(6, kf[1]); sn = mfma32(kf[1], qf[5], sn); MLOP_SLOT(5);
+      MLOP_WAIT_K(5, kf[2]); sn = mfma32(kf[2], qf[6], sn); MLOP_VREAD(1, vb, 0, vs); MLOP_SLOT(6);
+      MLOP_WAIT_K(8, kf[3]); sn = mfma32(kf[3], qf[7], sn); MLOP_SLOT(7);
+      const bf16x8 p0f = __builtin_bit_cast(bf16x8, wp[0]), p1f = __builtin_bit_cast(bf16x8, wp[1]);
+      MLOP_WAIT_V(4, va); o[0] = mfma32(frag(va[0], va[1]), p0f, o[0]); MLOP_SLOT(8);
+      o[0] = mfma32(frag(va[2], va[3]), p1f, o[0]); MLOP_VREAD(2, va, 0, vs); MLOP_SLOT(9);
+      MLOP_WAIT_V(4, vb); o[1] = mfma32(frag(vb[0], vb[1]), p0f, o[1]); MLOP_SLOT(10);
+      o[1] = mfma32(frag(vb[2], vb[3]), p1f, o[1]); MLOP_VREAD(3, vb, 0, vs); MLOP_SLOT(11);
+      MLOP_WAIT_V(4, va); o[2] = mfma32(frag(va[0], va[1]), p0f, o[2]); MLOP_SLOT(12);
+      o[2] = mfma32(frag(va[2], va[3]), p1f, o[2]); MLOP_SLOT(13);
+      MLOP_WAIT_V(0, vb); o[3] = mfma32(frag(vb[0], vb[1]), p0f, o[3]); MLOP_SLOT(14);
+      o[3] = mfma32(frag(vb[2], vb[3]), p1f, o[3]); MLOP_SLOT(15);
     }
-    bf16x8 pf[2];
-    softmax(qk(st_tag), pp, pf);
-    pv(st_tag, pf);
+    soft(16, sc, wn);
+    rescale();
   };
-  for (int pp = 0; pp < n_pairs; pp += STAGES) {
-    pair_step(std::integral_constant<int, 0>{}, pp);
-    if (pp + 1 < n_pairs) pair_step(std::integral_constant<int, 1>{}, pp + 1);
-    if (pp + 2 < n_pairs) pair_step(std::integral_constant<int, 2>{}, pp + 2);
+  // The last pair: its softmax under O += V^T . P^T of the pair before, then its own
+  auto finish = [&](f32x16& sc, const u32x4 (&wp)[2]) {
+    u32x4 wn[2];
+    v4s16 va[4], vb[4];
+    wait_vmcnt<0>();
+    raw_barrier();
+    row_max(sc, n_pairs - 1);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    const uint32_t v1 = (uint32_t)((n_pairs + 1) % 3) * SLOT, v0 = (uint32_t)((n_pairs + 2) % 3) * SLOT;
+    if (n_pairs > 1) {
+      MLOP_VREAD(0, va, v1, 0); MLOP_VREAD(1, vb, v1, 0);
+      const bf16x8 p0f = __builtin_bit_cast(bf16x8, wp[0]), p1f = __builtin_bit_cast(bf16x8, wp[1]);
+      MLOP_WAIT_V(4, va); o[0] = mfma32(frag(va[0], va[1]), p0f, o[0]); MLOP_SLOT(0); MLOP_SLOT(1);
+      o[0] = mfma32(frag(va[2], va[3]), p1f, o[0]); MLOP_VREAD(2, va, v1, 0); MLOP_SLOT(2); MLOP_SLOT(3);
+      MLOP_WAIT_V(4, vb); o[1] = mfma32(frag(vb[0], vb[1]), p0f, o[1]); MLOP_SLOT(4); MLOP_SLOT(5);
+      o[1] = mfma32(frag(vb[2], vb[3]), p1f, o[1]); MLOP_VREAD(3, vb, v1, 0); MLOP_SLOT(6); MLOP_SLOT(7);
+      MLOP_WAIT_V(4, va); o[2] = mfma32(frag(va[0], va[1]), p0f, o[2]); MLOP_SLOT(8); MLOP_SLOT(9);
+      o[2] = mfma32(frag(va[2], va[3]), p1f, o[2]); MLOP_SLOT(10); MLOP_SLOT(11);
+      MLOP_WAIT_V(0, vb); o[3] = mfma32(frag(vb[0], vb[1]), p0f, o[3]); MLOP_SLOT(12); MLOP_SLOT(13);
+      o[3] = mfma32(frag(vb[2], vb[3]), p1f, o[3]); MLOP_SLOT(14); MLOP_SLOT(15);
+    } else {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) soft(r, sc, wn);
+    }
+    soft(16, sc, wn);
+    rescale();
+    const bf16x8 p0f = __builtin_bit_cast(bf16x8, wn[0]), p1f = __builtin_bit_cast(bf16x8, wn[1]);
+    MLOP_VREAD(0, va, v0, 0); MLOP_VREAD(1, vb, v0, 0);
+    MLOP_WAIT_V(4, va); o[0] = mfma32(frag(va[0], va[1]), p0f, o[0]); o[0] = mfma32(frag(va[2], va[3]), p1f, o[0]);
+    MLOP_VREAD(2, va, v0, 0);
+    MLOP_WAIT_V(4, vb); o[1] = mfma32(frag(vb[0], vb[1]), p0f, o[1]); o[1] = mfma32(frag(vb[2], vb[3]), p1f, o[1]);
+    MLOP_VREAD(3, vb, v0, 0);
+    MLOP_WAIT_V(4, va); o[2] = mfma32(frag(va[0], va[1]), p0f, o[2]); o[2] = mfma32(frag(va[2], va[3]), p1f, o[2]);
+    MLOP_WAIT_V(0, vb); o[3] = mfma32(frag(vb[0], vb[1]), p0f, o[3]); o[3] = mfma32(frag(vb[2], vb[3]), p1f, o[3]);
+  };
+#undef MLOP_SLOT
+  // S of pair 0
+  auto qk0 = [&]() {
+    bf16x8 kf[8];
+    f32x16 sc = zero();
+#pragma unroll
+    for (int t = 0; t < 8; ++t) MLOP_KREAD(t, kf[t], 0);
+    MLOP_WAIT_K(7, kf[0]); sc = mfma32(kf[0], qf[0], sc);
+    MLOP_WAIT_K(6, kf[1]); sc = mfma32(kf[1], qf[1], sc);
+    MLOP_WAIT_K(5, kf[2]); sc = mfma32(kf[2], qf[2], sc);
+    MLOP_WAIT_K(4, kf[3]); sc = mfma32(kf[3], qf[3], sc);
+    MLOP_WAIT_K(3, kf[4]); sc = mfma32(kf[4], qf[4], sc);
+    MLOP_WAIT_K(2, kf[5]); sc = mfma32(kf[5], qf[5], sc);
+    MLOP_WAIT_K(1, kf[6]); sc = mfma32(kf[6], qf[6], sc);
+    MLOP_WAIT_K(0, kf[7]); sc = mfma32(kf[7], qf[7], sc);
+    return sc;
+  };
+
+  Pages g[6];  // ids of pair p in g[p % 6] (past the last page: the last)
+#pragma unroll
+  for (int i = 0; i < 5; ++i) g[i] = pages_of(i);
+  issue(kh, k_off, 0, g[0]);
+  if (n_pairs > 1) issue(kh, k_off, SLOT, g[1]);
+  issue(vh, v_off, RING_V, g[0]);
+  if (n_pairs > 2) issue(kh, k_off, 2 * SLOT, g[2]);
+  if (n_pairs > 2) wait_vmcnt<6>(); else if (n_pairs > 1) wait_vmcnt<4>(); else wait_vmcnt<2>();
+  raw_barrier();
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the page ids
+  f32x16 sa = qk0(), sb;
+  u32x4 wa[2], wb[2];
+  const int last = n_pairs - 1;
+  if (last > 0) {
+    int pp = 0;
+#define MLOP_STEP(P, FIRST, SC, SN, WP, WN)                                                                             \
+  step(std::integral_constant<int, P>{}, std::bool_constant<FIRST>{}, pp, SC, SN, WP, WN, g[(P + 1) % 6], g[(P + 3) % 6]); \
+  g[(P + 5) % 6] = pages_of(pp + 5);                                                                                    \
+  if (++pp >= last) break
+    do {
+      MLOP_STEP(0, true, sa, sb, wb, wa);
+      for (;;) {
+        MLOP_STEP(1, false, sb, sa, wa, wb);
+        MLOP_STEP(2, false, sa, sb, wb, wa);
+        MLOP_STEP(3, false, sb, sa, wa, wb);
+        MLOP_STEP(4, false, sa, sb, wb, wa);
+        MLOP_STEP(5, false, sb, sa, wa, wb);
+        MLOP_STEP(0, false, sa, sb, wb, wa);
+      }
+    } while (false);
+#undef MLOP_STEP
   }
+  {
+    f32x16 sc = last & 1 ? sb : sa;
+    const u32x4 wp[2] = {last & 1 ? wa[0] : wb[0], last & 1 ? wa[1] : wb[1]};
+    finish(sc, wp);
+  }
+#undef MLOP_KREAD
+#undef MLOP_WAIT_K
+#undef MLOP_VREAD
+#undef MLOP_WAIT_V
 
   // the two lane halves' partial row sums; O^T element r of dim block d is dim
   // 32 d + 8 (r >> 2) + 4 h + (r & 3) of q row R

@@ -1,0 +1,61 @@
+"""Flash prefill (attention.hip flash32_item) where its pipeline begins and ends: one pair of pages up to more than two rounds
+of its unrolled loop, last pairs of one key to 32, rows that move the running max at every pair."""
+import numpy as np
+import pytest
+import torch
+
+from mlopamd import ops
+from mlopamd.ops import reference as ref
+
+pytestmark = pytest.mark.gpu
+bf = torch.bfloat16
+
+
+def launch(gpu, q_lens, ctx_lens, Hq, Hkv, grow):
+    """Every sequence a prefill of q_lens tokens behind ctx_lens - q_lens cached ones, pages scattered."""
+    G, rng, S = Hq // Hkv, np.random.default_rng(len(q_lens) + Hq), len(q_lens)
+    pages = [(c + 15) // 16 for c in ctx_lens]
+    NB = sum(pages) + 3
+    ids = rng.permutation(np.arange(1, NB))
+    bt = np.zeros((S, max(pages)), np.int32)
+    seq, q0 = [], []
+    for i, n in enumerate(pages):
+        bt[i, :n] = ids[sum(pages[:i]):sum(pages[:i]) + n]
+        first = list(range(0, q_lens[i], 128 // G))
+        seq += [i] * len(first)
+        q0 += first[::-1]
+
+    class Meta:
+        pass
+
+    m, d = Meta(), lambda a: torch.tensor(np.asarray(a), dtype=torch.int32, device=gpu)
+    m.block_tables, m.ctx_len, m.q_len = d(bt), d(ctx_lens), d(q_lens)
+    m.q_start = d(np.concatenate([[0], np.cumsum(q_lens)[:-1]]))
+    m.tile_seq = m.tile_q0 = d(np.zeros(0))
+    m.ptile_seq, m.ptile_q0 = d(seq), d(q0)
+    m.part_tokens, m.nparts = max(ctx_lens), 1
+    m.part_o = m.part_ml = torch.empty(1, device=gpu)
+    torch.manual_seed(S)
+    q = torch.randn(sum(q_lens), Hq, 128, device=gpu, dtype=bf)
+    kc, vc = (torch.randn(NB, Hkv, 16, 128, device=gpu, dtype=bf) for _ in range(2))
+    if grow:  # larger keys the later they stand
+        for i, n in enumerate(pages):
+            at = torch.arange(n, device=gpu).view(n, 1, 1, 1)
+            kc[bt[i, :n]] = (kc[bt[i, :n]].float() * 1.25 ** (at % 24)).to(bf)
+    out = ops.paged_attention(q, kc, vc, m)
+    exp = ref.paged_attention(q, kc, vc, m)
+    # P in bf16 (2^-9 of each addend, which the row's sum does not share) and the result's rounding; |V| < 5
+    torch.testing.assert_close(out.float(), exp.float(), atol=2.0 ** -6, rtol=2.0 ** -6)
+
+
+@pytest.mark.parametrize("grow", [False, True])
+@pytest.mark.parametrize("Hq,Hkv", [(8, 8), (8, 2), (16, 2)])
+def test_every_number_of_pairs(gpu, Hq, Hkv, grow):
+    ctx = [32 * p + r for p in range(14) for r in (1, 16, 17, 32)]
+    launch(gpu, [min(c, 1 + 7 * i % 23) for i, c in enumerate(ctx)], ctx, Hq, Hkv, grow)
+
+
+@pytest.mark.parametrize("Hq,Hkv", [(8, 8), (8, 2), (16, 2)])
+def test_whole_prompts(gpu, Hq, Hkv):
+    n = [1, 15, 31, 32, 33, 63, 64, 65, 97, 127, 128, 129, 190, 255, 257, 449]
+    launch(gpu, n, n, Hq, Hkv, False)
