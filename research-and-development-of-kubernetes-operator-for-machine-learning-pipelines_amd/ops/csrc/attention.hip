@@ -604,9 +604,9 @@ void launch_paged_attention(void* out, float* part_o, float* part_ml, const void
 // K7 flash prefill on the 32x32x16 MFMA (cdna_hip_programming.md "Fused attention prefill":
 // swapped QK^T, an accumulator tile as the next MFMA's operand).  One workgroup = 128 MFMA
 // q-rows (128/G query tokens x the G heads of one kv head) against EVERY key of its causal
-// range, so every K/V byte fetched from L2 feeds all 128 q-rows.  K/V page pairs (32 keys, 16 KB)
-// stream through a 3-deep LDS ring by LDS-DMA (global_load_lds, counted vmcnt, one raw barrier
-// per pair), swizzled through the SOURCE address:
+// range, so every K/V byte fetched from L2 feeds all 128 q-rows.  Page pairs (32 keys, 8 KB of K, 8 of V)
+// stream through LDS rings of three by LDS-DMA (buffer form, counted vmcnt, one raw barrier per pair),
+// swizzled through the SOURCE address:
 //   K page [16 keys][16 x 16 B]: chunk c of key k at slot c ^ k       (ds_read_b128)
 //   V page [16 keys][16 x 16 B]: chunk c of key k at slot c ^ vswz(k) (ds_read_b64_tr_b16)
 // both conflict-free for the fragment reads below (SQ_LDS_BANK_CONFLICT = 0).  Per wave 32
@@ -619,11 +619,15 @@ void launch_paged_attention(void* out, float* part_o, float* part_ml, const void
 //     8s .. 8s+7 -> bf16 = the k-step s fragment, k order permuted), V^T by two
 //     ds_read_b64_tr_b16 per fragment from the token-major image (keys 16s + 4h + 0..3 and
 //     + 8, dims 32 dblk + (l & 31)).
-// Half the MFMA issue slots of a 16x16x32 form for the same FLOPs (an MFMA holds the SIMD's
-// vector issue for 8 cycles either way, MI355X_MICROARCH.md constants) and a quarter of its
-// cross-lane max steps: +4 % at 1 x 8192, +19 % at 4 x 2048 and 16 x 512 over the round-4
-// 16x16x32 kernel (profiles/r05_flash32.md).  Two workgroups per CU (up to 256 VGPRs) beat
-// three (168) by 1-5 %.
+// Half the MFMA issue slots of a 16x16x32 form for the same FLOPs and a quarter of its cross-lane max
+// steps: +4 % at 1 x 8192, +19 % at 4 x 2048 and 16 x 512 over the 16x16x32 kernel.
+// What bounds it at long contexts: power.  With the three phases of a pair one behind the other, matrix and
+// vector work overlapped only between a SIMD's waves, at 1.73 GHz and half of its cycles with an MFMA in them;
+// now each wave has the softmax of one pair between the MFMAs of S of the next and O of the one before (step),
+// with a quarter fewer vector instructions.  us, before -> now: 2048 queries of 64 heads at 11048 keys
+// 670 -> 613 (1097 TFLOP/s), 512 at 4000 93.4 -> 82; 32 heads, 2048 at 8000 248 -> 224, prompts of 1 x 2048
+// 57 -> 50.7, 2 x 900 33.4 -> 30, 3 x 333 14.2 -> 13, 1 x 8192 550 -> 525; many short ones, where the start of a
+// workgroup counts and two of 194 registers share a CU that had three of 168: 16 x 500 61 -> 62, 64 x 100 36.5 -> 38.5.
 using f32x16 = __attribute__((ext_vector_type(16))) float;
 constexpr float kRescaleLog2 = 8.f;  // flash32 deferred-rescale threshold (exp2 units)
 // two floats -> one dword of two bf16 in ONE v_cvt_pk_bf16_f32 (pack2's two scalar casts
@@ -1192,7 +1196,7 @@ __global__ void __launch_bounds__(256, 2) flash32_stream_kernel(
     raw_barrier();  // pair visible to every wave; the stage consumed one step ago is free
     issue_next(std::integral_constant<int, (ST + 2) % 3>{});
     if (pp == 0 && nxt.tile >= 0) q_issue(nxt);  // the next tile's Q under this tile's pairs
-    // S^T = K . Q^T of this pair (flash32_item's qk)
+    // S^T = K . Q^T of this pair
     f32x16 sc;
     {
       uint32_t kb = k_b0;
@@ -1216,7 +1220,7 @@ __global__ void __launch_bounds__(256, 2) flash32_stream_kernel(
           asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(kf[t & 3]) : "v"(kb ^ (32u * (t + 4))), "n"(so));
       }
     }
-    // online softmax (flash32_item's, deferred rescale)
+    // online softmax (deferred rescale)
     bf16x8 pf[2];
     {
       if (pp * 32 + 31 > cur.wg_min_pos) {
@@ -1256,7 +1260,7 @@ __global__ void __launch_bounds__(256, 2) flash32_stream_kernel(
       pf[1] = __builtin_bit_cast(bf16x8, w[1]);
       l += rs;
     }
-    // O^T += V^T . P^T (flash32_item's pv)
+    // O^T += V^T . P^T
     {
       uint32_t vb = v_b0;
       asm volatile("" : "+v"(vb));
