@@ -601,35 +601,33 @@ void launch_paged_attention(void* out, float* part_o, float* part_ml, const void
 }
 
 // ---------------------------------------------------------------------------
-// K7 flash prefill on the 32x32x16 MFMA (cdna_hip_programming.md "Fused attention prefill":
+// K7 flash prefill on the 16x16x32 MFMA (cdna_hip_programming.md "Fused attention prefill":
 // swapped QK^T, an accumulator tile as the next MFMA's operand).  One workgroup = 128 MFMA
 // q-rows (128/G query tokens x the G heads of one kv head) against EVERY key of its causal
 // range, so every K/V byte fetched from L2 feeds all 128 q-rows.  Page pairs (32 keys, 8 KB of K, 8 of V)
-// stream through LDS rings of three by LDS-DMA (buffer form, counted vmcnt, one raw barrier per pair),
+// stream through LDS rings of four by LDS-DMA (buffer form, counted vmcnt, one raw barrier per pair),
 // swizzled through the SOURCE address:
-//   K page [16 keys][16 x 16 B]: chunk c of key k at slot c ^ k       (ds_read_b128)
-//   V page [16 keys][16 x 16 B]: chunk c of key k at slot c ^ vswz(k) (ds_read_b64_tr_b16)
-// both conflict-free for the fragment reads below (SQ_LDS_BANK_CONFLICT = 0).  Per wave 32
-// q-rows, ONE per lane column:
-//   S^T [32 keys x 32 q] = K . Q^T: 8 MFMAs (A = K rows by ds_read_b128, B = Q^T in registers);
-//     lane l holds the 16 keys (r & 3) + 8 (r >> 2) + 4 h (h = l >> 5) of q column l & 31, so
-//     the row max is 15 lane-local max + ONE permlane32 swap, the row sum lane-local (the two
-//     halves' partial sums meet once, in the epilogue);
-//   O^T [128 d x 32 q] += V^T . P^T: 8 MFMAs, P^T straight from the S registers (registers
-//     8s .. 8s+7 -> bf16 = the k-step s fragment, k order permuted), V^T by two
-//     ds_read_b64_tr_b16 per fragment from the token-major image (keys 16s + 4h + 0..3 and
-//     + 8, dims 32 dblk + (l & 31)).
-// Half the MFMA issue slots of a 16x16x32 form for the same FLOPs and a quarter of its cross-lane max
-// steps: +4 % at 1 x 8192, +19 % at 4 x 2048 and 16 x 512 over the 16x16x32 kernel.
-// What bounds it at long contexts: power.  With the three phases of a pair one behind the other, matrix and
-// vector work overlapped only between a SIMD's waves, at 1.73 GHz and half of its cycles with an MFMA in them;
-// now each wave has the softmax of one pair between the MFMAs of S of the next and O of the one before (step),
-// with a quarter fewer vector instructions.  us, before -> now: 2048 queries of 64 heads at 11048 keys
-// 670 -> 613 (1097 TFLOP/s), 512 at 4000 93.4 -> 82; 32 heads, 2048 at 8000 248 -> 224, prompts of 1 x 2048
-// 57 -> 50.7, 2 x 900 33.4 -> 30, 3 x 333 14.2 -> 13, 1 x 8192 550 -> 525; many short ones, where the start of a
-// workgroup counts and two of 194 registers share a CU that had three of 168: 16 x 500 61 -> 62, 64 x 100 36.5 -> 38.5.
+//   K pair [32 keys][16 x 16 B]: chunk c of key k at slot c ^ (4 (k >> 3) + (k & 3)) (ds_read_b128)
+//   V pair [32 keys][16 x 16 B]: chunk c of key k at slot c ^ vswz(k & 15)           (ds_read_b64_tr_b16)
+// both conflict-free for the fragment reads below.  Per wave 32 q-rows, two per lane column (qb):
+//   S^T [2 x 16 keys][2 x 16 q] = K . Q^T: 16 MFMAs (A = K rows by ds_read_b128, B = Q^T in registers); the
+//     rows of A are keys 8 (i >> 2) + (i & 3) and + 4, so lane group g4 holds keys 8 g4 + 0 .. 7 of q column
+//     l & 15: the row max and sum are lane-local, the quarters meet where the max moves and in the epilogue;
+//   O^T [128 d][2 x 16 q] += V^T . P^T: 16 MFMAs, P^T straight from the S registers (bf16, 32 keys = one MFMA),
+//     V^T by two ds_read_b64_tr_b16 per fragment from the token-major image.
+// What bounds it at long contexts: power (1.7 GHz).  With a pair's three phases one behind the other (32x32x16 MFMAs),
+// matrix and vector work overlapped only between a SIMD's waves; now each wave has the softmax of one pair between
+// the MFMAs of S of the next and O of the one before (step), with a quarter fewer vector instructions, and the
+// 16x16x32 MFMA does the same FLOPs on less power (registers only, all CUs: 2020 TFLOP/s against 1795).  A wave in its
+// MFMAs goes before the SIMD's other one, which then does its waiting in the shadow (2048 x 11048 586 -> 570, 2 x 900
+// 30.6 -> 28.2, 1 x 2048 47.7 -> 49).  us, phases in turn -> software pipeline -> now: 2048 queries of 64 heads at 11048
+// keys 670 -> 613 -> 565 (1190 TFLOP/s), 512 at 4000 94 -> 82 -> 77; 32 heads, 2048 at 8000 250 -> 224 -> 205, prompts of
+// 1 x 8192 550 -> 525 -> 464, 1 x 2048 57 -> 50.7 -> 49, 2 x 900 33.4 -> 30 -> 28.2, 3 x 333 14.2 -> 13 -> 12.5; many
+// short ones, where the start of a workgroup counts and two of 214 registers share a CU that had three of 168, 16 x
+// 500 61 -> 62 -> 60.5, 64 x 100 36 -> 38.5 -> 37.5.
 using f32x16 = __attribute__((ext_vector_type(16))) float;
-constexpr float kRescaleLog2 = 8.f;  // flash32 deferred-rescale threshold (exp2 units)
+constexpr int kFlashRing = 4;  // pairs in flash_item's rings
+constexpr float kRescaleLog2 = 8.f;  // flash prefill's deferred-rescale threshold (exp2 units)
 // two floats -> one dword of two bf16 in ONE v_cvt_pk_bf16_f32 (pack2's two scalar casts
 // become two cvt + shift + or)
 __device__ __forceinline__ uint32_t cvt_pk_bf16(float lo, float hi) {
@@ -650,16 +648,36 @@ __device__ __forceinline__ uint32_t vt32_base(int lane) {
   return 256u * t + 16u * (c ^ vswz(t)) + 8u * (p & 1);
 }
 
+// s_waitcnt lgkmcnt(W) for the reads of a (and b), then c += a . b, or c = a . b, in place.  As builtins the compiler gives the
+// results registers of their own, 64 of the output's beside the 64 they replace, and pads each MFMA behind an asm wait.  It
+// does not know this asm for an MFMA: vector instructions that read c wait for mfma16_settle or stand behind eight more MFMAs,
+// as does the next one on c.
+template <int W, bool ZERO = false>
+__device__ __forceinline__ void mfma16_into(f32x4& c, const bf16x8& a, const bf16x8& b) {
+  if constexpr (ZERO) {
+    if constexpr (W >= 0) asm volatile("s_waitcnt lgkmcnt(%3)\nv_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=&v"(c) : "v"(a), "v"(b), "n"(W));
+    else asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=&v"(c) : "v"(a), "v"(b));
+  } else {
+    if constexpr (W >= 0) asm volatile("s_waitcnt lgkmcnt(%3)\nv_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b), "n"(W));
+    else asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));
+  }
+}
+__device__ __forceinline__ void mfma16_settle(f32x4 (&c)[8][2]) {
+  asm volatile("s_nop 15\ns_nop 3"
+               : "+v"(c[0][0]), "+v"(c[0][1]), "+v"(c[1][0]), "+v"(c[1][1]), "+v"(c[2][0]), "+v"(c[2][1]), "+v"(c[3][0]), "+v"(c[3][1]),
+                 "+v"(c[4][0]), "+v"(c[4][1]), "+v"(c[5][0]), "+v"(c[5][1]), "+v"(c[6][0]), "+v"(c[6][1]), "+v"(c[7][0]), "+v"(c[7][1]));
+}
+
 // one flash tile (128 q-rows of ONE kv head against its whole causal key range)
 template <int G>
-__device__ __forceinline__ void flash32_item(
+__device__ __forceinline__ void flash_item(
     uint16_t* smem, int tile, int kvh, uint16_t* __restrict__ out, const uint16_t* __restrict__ q,
     const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc, const int* __restrict__ block_tables,
     int bt_stride, const int* __restrict__ ptile_seq, const int* __restrict__ ptile_q0,
     const int* __restrict__ q_start, const int* __restrict__ q_len, const int* __restrict__ ctx_len, int Hq,
     int Hkv, float scale_log2, int num_blocks) {
   constexpr int QB = 128 / G;            // query tokens per workgroup
-  constexpr int STAGES = 3;
+  constexpr int STAGES = kFlashRing;
   constexpr int STAGE = 4 * kBS * kD;    // bf16 per stage: K page A | K page B | V page A | V page B
   constexpr int PAGE = kBS * kD;
   const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -670,215 +688,238 @@ __device__ __forceinline__ void flash32_item(
   const int n_pairs = (kv_end + 31) >> 5;
   const int n_pages = (kv_end + kBS - 1) / kBS;
   const int wg_min_pos = ctx - ql + q0;
-  const int col = lane & 31, h = lane >> 5;
+  const int r16 = lane & 15, g4 = lane >> 4;
 
-  // this lane's q row (MFMA column): R = 32 wid + col
-  const int R = 32 * wid + col;
-  const int qi = q0 + R / G;
-  const bool q_ok = qi < ql;
-  const int pos_r = q_ok ? ctx - ql + qi : -1;
-  bf16x8 qf[8];
-  {
-    const uint16_t* qrow = q + ((size_t)(qs + (q_ok ? qi : 0)) * Hq + kvh * G + R % G) * kD + 8 * h;
+  // this lane's two q rows (MFMA columns): R = 32 wid + 16 qb + r16
+  int qi[2], pos_r[2];
+  bool q_ok[2];
+  bf16x8 qf[2][4];
+  float m[2], l[2], mc[2], alpha[2];
 #pragma unroll
-    for (int t = 0; t < 8; ++t) {
-      const bf16x8 v = *reinterpret_cast<const bf16x8*>(qrow + 16 * t);
-      qf[t] = q_ok ? v : bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+  for (int b = 0; b < 2; ++b) {
+    const int R = 32 * wid + 16 * b + r16;
+    qi[b] = q0 + R / G;
+    q_ok[b] = qi[b] < ql;
+    pos_r[b] = q_ok[b] ? ctx - ql + qi[b] : -1;
+    const uint16_t* qrow = q + ((size_t)(qs + (q_ok[b] ? qi[b] : 0)) * Hq + kvh * G + R % G) * kD + 8 * g4;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const bf16x8 v = *reinterpret_cast<const bf16x8*>(qrow + 32 * t);
+      qf[b][t] = q_ok[b] ? v : bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
     }
+    m[b] = kNegBig, l[b] = 0.f, mc[b] = -kNegBig * scale_log2, alpha[b] = 1.f;
   }
-  f32x16 o[4];
+  f32x4 o[8][2];
 #pragma unroll
-  for (int d = 0; d < 4; ++d)
+  for (int d = 0; d < 8; ++d)
 #pragma unroll
-    for (int e = 0; e < 16; ++e) o[d][e] = 0.f;
-  float m = kNegBig, l = 0.f;
+    for (int b = 0; b < 2; ++b) o[d][b] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   const int* bt = block_tables + (size_t)s * bt_stride;
-  const size_t page_stride = (size_t)Hkv * PAGE;
+  const uint32_t page_bytes = (uint32_t)Hkv * (2 * PAGE);
   const int kkey = wid * 4 + (lane >> 4);
-  // K image: chunk c of key k at slot c ^ k on BOTH pages (the 32x32 A-operand reads take keys
-  // {0-3, 12-15} of one page and {4-11} of the other per 16-lane group: 16 distinct slots)
-  const uint32_t k_off = 2u * (uint32_t)(kkey * kD + (((lane & 15) ^ (kkey & 15)) << 3));
-  const uint32_t v_off = 2u * (uint32_t)(kkey * kD + (((lane & 15) ^ vswz(kkey)) << 3));
+  const int ksw = (kkey >> 3) * 4 + (kkey & 3);  // (page B: + 8)
+  const uint32_t k_off[2] = {2u * (uint32_t)(kkey * kD + ((r16 ^ ksw) << 3)), 2u * (uint32_t)(kkey * kD + ((r16 ^ ksw ^ 8) << 3))};
+  const uint32_t v_off[1] = {2u * (uint32_t)(kkey * kD + ((r16 ^ vswz(kkey)) << 3))};
   const uint16_t* kh = kc + kvh * PAGE;
   const uint16_t* vh = vc + kvh * PAGE;
-  struct Pages {
+  struct Ids {
     int a, b;
   };
-  auto pages_of = [&](int pp) { return Pages{bt[min(2 * pp, n_pages - 1)], bt[min(2 * pp + 1, n_pages - 1)]}; };
-  // a pair's two pages of K / of V into slot st of their ring
+  struct Pages {
+    uint64_t a, b;
+  };
+  // ids of pair pp (past the last page: the last), and their bytes from the first page (clamped: a corrupt block table must
+  // not become an out-of-bounds fault)
+  auto id_at = [&](uint32_t i) { return *reinterpret_cast<const int*>((const char*)bt + 4u * i); };
+  auto ids_of = [&](int pp) {
+    const uint32_t i = min(2 * pp, n_pages - 1);
+    return Ids{id_at(i), id_at(min((int)i + 1, n_pages - 1))};
+  };
+  auto at = [&](int id) { return (uint64_t)(uint32_t)min(max(id, 0), num_blocks - 1) * page_bytes; };
+  auto pages_of = [&](Ids i) { return Pages{at(i.a), at(i.b)}; };
+  // a pair's two pages of K / of V into a slot of their ring
   const uint32_t ring = (uint32_t)(uintptr_t)smem + wid * 1024;
-  auto issue = [&](const uint16_t* head, uint32_t off, uint32_t slot, Pages pg) {
-    auto page = [&](int id) {
-      return __builtin_amdgcn_make_buffer_rsrc((void*)(head + min(max(id, 0), num_blocks - 1) * page_stride), 0, 2 * PAGE, 0x00020000);
-    };
-    lds_dma16(page(pg.a), ring + slot, off, 0);
-    lds_dma16(page(pg.b), ring + slot + 2 * PAGE, off, 0);
+  auto issue = [&](const uint16_t* head, uint32_t off_a, uint32_t off_b, uint32_t slot, Pages pg) {
+    auto page = [&](uint64_t at) { return __builtin_amdgcn_make_buffer_rsrc((void*)((const char*)head + at), 0, 2 * PAGE, 0x00020000); };
+    lds_dma16(page(pg.a), ring + slot, off_a, 0);
+    lds_dma16(page(pg.b), ring + slot + 2 * PAGE, off_b, 0);
   };
   constexpr uint32_t SLOT = 4 * PAGE, RING_V = STAGES * SLOT;  // bytes
-  // K fragment t of this lane: key col of the pair (page col >> 4, row col & 15), chunk 2t + h at
-  // slot (2t + h) ^ (col & 15): byte k_b0 ^ 32 t
-  const int k15 = col & 15;
-  const uint32_t k_b0 = (uint32_t)(uintptr_t)smem + (uint32_t)((col >> 4) * PAGE * 2 + k15 * 256 + ((h ^ k15) << 4));
-  const uint32_t v_b0 = (uint32_t)(uintptr_t)smem + RING_V + vt32_base(lane);
+  // K fragment (kb, t): key row 8 (r16 >> 2) + (r16 & 3) + 4 kb of the pair, chunk 4t + g4 at slot
+  // (4t + g4) ^ r16: byte (k_b0 ^ 64 t) + 1024 kb
+  const uint32_t k_b0 = (uint32_t)(uintptr_t)smem + (uint32_t)((8 * (r16 >> 2) + (r16 & 3)) * 256 + ((g4 ^ r16) << 4));
+  const uint32_t v_b0 = (uint32_t)(uintptr_t)smem + RING_V + vt_base(lane);
   // The fragment reads are inline asm with counted waits: as plain loads the compiler reused one register set and waited
   // lgkmcnt(0) before every MFMA, and, for V, vmcnt(0) (it cannot tell them from the LDS-DMA in flight).  No scalar load may
   // be in flight beside them (it would be counted): page ids are loaded where a step's last read has landed.
-#define MLOP_KREAD(t, f, so) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(f) : "v"(k_b0 ^ (32u * (t))), "n"(so))
-#define MLOP_WAIT_K(n, f) asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(f) : "n"(n))
-  // both pages' fragments of dim block dblk: (lo, hi) of page A, of page B; vx: a ring slot's bytes
-#define MLOP_VREAD(dblk, r, vx, so)                                                                                    \
-  asm volatile("ds_read_b64_tr_b16 %0, %4 offset:%6\nds_read_b64_tr_b16 %1, %5 offset:%7\n"                           \
-               "ds_read_b64_tr_b16 %2, %4 offset:%8\nds_read_b64_tr_b16 %3, %5 offset:%9\n"                           \
-               : "=&v"(r[0]), "=&v"(r[1]), "=&v"(r[2]), "=&v"(r[3])                                                   \
-               : "v"((v_b0 ^ (64u * (dblk))) + (vx)), "v"((v_b0 ^ (64u * (dblk)) ^ 32u) + (vx)), "n"(so),             \
-                 "n"((so) + 2048u), "n"((so) + 4096u), "n"((so) + 6144u))
-#define MLOP_WAIT_V(n, r) \
-  asm volatile("s_waitcnt lgkmcnt(%4)" : "+v"(r[0]), "+v"(r[1]), "+v"(r[2]), "+v"(r[3]) : "n"(n))
-  auto frag = [&](const v4s16& lo, const v4s16& hi) {
+  // (f = 2 t + kb)
+#define MLOP_KREAD(f, r, so) \
+  asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(r) : "v"(k_b0 ^ (64u * ((f) >> 1))), "n"((so) + 1024u * ((f) & 1)))
+  // dims 16 d .. + 15 of keys 8 g4 + 0 .. 3 and + 4 .. 7; vx: a ring slot's bytes
+#define MLOP_VREAD(d, r, vx, so)                                                                                        \
+  asm volatile("ds_read_b64_tr_b16 %0, %2 offset:%4\nds_read_b64_tr_b16 %1, %3 offset:%5"                               \
+               : "=&v"(r[0]), "=&v"(r[1])                                                                               \
+               : "v"((v_b0 ^ (32u * (d))) + (vx)), "v"((v_b0 ^ (32u * (d)) ^ 16u) + (vx)), "n"(so), "n"((so) + 1024u))
+  auto frag = [&](const v4s16 (&r)[2]) {
     bf16x8 f;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      f[e] = lo[e];
-      f[4 + e] = hi[e];
+      f[e] = r[0][e];
+      f[4 + e] = r[1][e];
     }
     return f;
   };
 
-  float alpha = 1.f, mc = -m * scale_log2;
   bool resc = false;
+  using Sc = f32x4[2][2];  // S^T [kb][qb]: keys 8 g4 + 4 kb + 0 .. 3 of q row qb
   // Row max of a pair's scores (raw units; the scale folds into the exponent's FMA).  Deferred rescale: the running max
   // moves only when some row's new max exceeds it by more than 2^kRescaleLog2 in exp2 units (always on a row's first
   // keys: m starts at -1e30); otherwise P stays scaled against the old max, <= 2^8, which bf16 P and f32 O / l carry
-  // exactly as well.  The halves of a row's keys meet only when it does.  O takes the factor (resc) once the pair before
+  // exactly as well.  The quarters of a row's keys meet only when it does.  O takes the factor (resc) once the pair before
   // has been added to it.
-  auto row_max = [&](f32x16& sc, int pp) {
+  auto row_max = [&](Sc& sc, int pp) {
     if (pp * 32 + 31 > wg_min_pos) {  // a pair crossing the workgroup's causal diagonal
       // (a side effect keeps this a branch: if-converted, the 47 compare / select / add of the
       // mask ran on every pair, a third of the loop's VALU)
       asm volatile("");
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int tok = pp * 32 + (r & 3) + 8 * (r >> 2) + 4 * h;
-        sc[r] = tok <= pos_r ? sc[r] : -INFINITY;
-      }
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+          const int tok = pp * 32 + 8 * g4 + k;
+          sc[k >> 2][b][k & 3] = tok <= pos_r[b] ? sc[k >> 2][b][k & 3] : -INFINITY;
+        }
     }
-    const float a = fmaxf(fmaxf(sc[0], sc[1]), sc[2]), b = fmaxf(fmaxf(sc[3], sc[4]), sc[5]);
-    const float c = fmaxf(fmaxf(sc[6], sc[7]), sc[8]), d = fmaxf(fmaxf(sc[9], sc[10]), sc[11]);
-    const float e = fmaxf(fmaxf(sc[12], sc[13]), sc[14]);
-    float mx = fmaxf(fmaxf(fmaxf(a, b), c), fmaxf(fmaxf(d, e), sc[15]));
-    if (__ballot(fmaf(mx, scale_log2, mc) > kRescaleLog2)) {
-      const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
-      mx = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
-      const float m_new = fmaxf(m, mx);
-      alpha = fast_exp2((m - m_new) * scale_log2);
-      m = m_new;
-      mc = -m * scale_log2;
-      l *= alpha;
+    float mx[2];
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      const float x = fmaxf(fmaxf(sc[0][b][0], sc[0][b][1]), sc[0][b][2]), y = fmaxf(fmaxf(sc[0][b][3], sc[1][b][0]), sc[1][b][1]);
+      mx[b] = fmaxf(fmaxf(x, y), fmaxf(sc[1][b][2], sc[1][b][3]));
+    }
+    if (__ballot(fmaf(mx[0], scale_log2, mc[0]) > kRescaleLog2) | __ballot(fmaf(mx[1], scale_log2, mc[1]) > kRescaleLog2)) {
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+        const float m_new = fmaxf(m[b], max_x16_x32(mx[b]));
+        alpha[b] = fast_exp2((m[b] - m_new) * scale_log2);
+        m[b] = m_new;
+        mc[b] = -m_new * scale_log2;
+        l[b] *= alpha[b];
+      }
       resc = true;
     }
   };
   auto rescale = [&]() {
     if (resc) {
-      asm volatile("");
+      mfma16_settle(o);
 #pragma unroll
-      for (int d = 0; d < 4; ++d) o[d] *= alpha;
+      for (int d = 0; d < 8; ++d)
+#pragma unroll
+        for (int b = 0; b < 2; ++b) o[d][b] *= alpha[b];
       resc = false;
     }
   };
-  // P of element r of the lane's 16 keys of its q column; every second makes a dword of the P^T fragments
-  // (r = 16: the last of them; a pair is packed behind the next element's exponential, which a VALU instruction could not
-  // read at once)
+  // P of element r of the lane's 2 x 8; every second makes a dword of the P^T fragments (r = 16: the last of them; a pair is
+  // packed behind the next element's exponential, which a VALU instruction could not read at once)
   float rs, pe[2];
-  auto soft = [&](int r, const f32x16& sc, u32x4 (&w)[2]) {
+  auto soft = [&](int r, const Sc& sc, u32x4 (&w)[2]) {
     float p = 0.f;
-    if (r < 16) p = fast_exp2(fmaf(sc[r], scale_log2, mc));
+    if (r < 16) p = fast_exp2(fmaf(sc[(r >> 2) & 1][r >> 3][r & 3], scale_log2, mc[r >> 3]));
     if (r > 0 && r % 2 == 0) {
-      rs = r == 2 ? pe[0] + pe[1] : rs + (pe[0] + pe[1]);
-      asm volatile("v_cvt_pk_bf16_f32 %0, %2, %3" : "=v"(w[(r - 2) >> 3][((r - 2) & 7) >> 1]), "+v"(rs) : "v"(pe[0]), "v"(pe[1]));
+      const int e = r - 2;
+      rs = e % 8 == 0 ? pe[0] + pe[1] : rs + (pe[0] + pe[1]);
+      asm volatile("v_cvt_pk_bf16_f32 %0, %2, %3" : "=v"(w[e >> 3][(e & 7) >> 1]), "+v"(rs) : "v"(pe[0]), "v"(pe[1]));
+      if (e % 8 == 6) l[e >> 3] += rs;
     }
     if (r < 16) pe[r & 1] = p;
-    else l += rs;
-  };
-  auto zero = []() {
-    f32x16 z;
-#pragma unroll
-    for (int e = 0; e < 16; ++e) z[e] = 0.f;
-    return z;
   };
 
 #define MLOP_SLOT(t)                 \
   __builtin_amdgcn_sched_barrier(0); \
   soft(t, sc, wn);                   \
   __builtin_amdgcn_sched_barrier(0)
-  // Step pp: S(pp + 1) = K . Q^T and O += V^T . P(pp - 1)^T, 16 MFMAs, with an element of P(pp)'s softmax behind each, so
-  // that a wave's matrix and vector work overlap, and not only those of a SIMD's waves.  K is a pair ahead of the softmax
-  // and V a pair behind it: rings of their own.  (pp = 0: no P before.)
-  auto step = [&](auto p_, auto first_, int pp, f32x16& sc, f32x16& sn, const u32x4 (&wp)[2], u32x4 (&wn)[2], Pages p1,
-                  Pages p3) {
+  // S += K . Q^T of fragment f (its wait, its two MFMAs with an element between, the next read), and O += V^T . P^T of d
+#define MLOP_QK(f, n, t)                                                   \
+  mfma16_into<n, ((f) < 2)>(sn[(f) & 1][0], kf[f], qf[0][(f) >> 1]);       \
+  MLOP_SLOT(t);                                                            \
+  mfma16_into<-1, ((f) < 2)>(sn[(f) & 1][1], kf[f], qf[1][(f) >> 1])
+#define MLOP_PV(d, n, t)                        \
+  mfma16_into<n>(o[d][0], frag(vf[d]), p0f);    \
+  MLOP_SLOT(t);                                 \
+  mfma16_into<-1>(o[d][1], frag(vf[d]), p1f)
+  // Step pp: S(pp + 1) = K . Q^T and O += V^T . P(pp - 1)^T, 32 MFMAs, with an element of P(pp)'s softmax behind every
+  // second, so that a wave's matrix and vector work overlap, and not only those of a SIMD's waves.  K is a pair ahead of the
+  // softmax and V a pair behind it: rings of their own.  (pp = 0: no P before.)
+  auto step = [&](auto p_, auto first_, int pp, Sc& sc, Sc& sn, const u32x4 (&wp)[2], u32x4 (&wn)[2], Pages p1, Ids i3, Pages& p3) {
     constexpr int P = decltype(p_)::value;
     constexpr bool FIRST = decltype(first_)::value;
-    constexpr uint32_t ks = (P + 1) % 3 * SLOT, vs = (P + 2) % 3 * SLOT;
+    constexpr uint32_t ks = (P + 1) % STAGES * SLOT, vs = (P + STAGES - 1) % STAGES * SLOT;
     if (pp + 2 < n_pairs) wait_vmcnt<4>(); else wait_vmcnt<2>();
     raw_barrier();  // K of pp + 1 and V of pp - 1 visible to every wave; the slots of K pp and V pp - 2 free
-    issue(vh, v_off, RING_V + ks, p1);
-    if (pp + 3 < n_pairs) issue(kh, k_off, P % 3 * SLOT, p3);
+    issue(vh, v_off[0], v_off[0], RING_V + ks, p1);
+    p3 = pages_of(i3);
+    if (pp + 3 < n_pairs) issue(kh, k_off[0], k_off[1], (P + 3) % STAGES * SLOT, p3);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the page ids
+    bf16x8 kf[8];
+    v4s16 vf[8][2];
+#pragma unroll
+    for (int f = 0; f < 8; ++f) MLOP_KREAD(f, kf[f], ks);
     row_max(sc, pp);
     __builtin_amdgcn_sched_barrier(0);
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the page ids
-    bf16x8 kf[4];
-    v4s16 va[4], vb[4];
-#pragma unroll
-    for (int t = 0; t < 4; ++t) MLOP_KREAD(t, kf[t], ks);
-    // (reads in flight at each wait: K 4 - 7 behind K 0 - 3, then V's blocks of four)
-    sn = zero();
-    MLOP_WAIT_K(3, kf[0]); sn = mfma32(kf[0], qf[0], sn); MLOP_KREAD(4, kf[0], ks); MLOP_SLOT(0);
-    MLOP_WAIT_K(3, kf[1]); sn = mfma32(kf[1], qf[1], sn); MLOP_KREAD(5, kf[1], ks); MLOP_SLOT(1);
-    MLOP_WAIT_K(3, kf[2]); sn = mfma32(kf[2], qf[2], sn); MLOP_KREAD(6, kf[2], ks); MLOP_SLOT(2);
-    MLOP_WAIT_K(3, kf[3]); sn = mfma32(kf[3], qf[3], sn); MLOP_KREAD(7, kf[3], ks); MLOP_SLOT(3);
+    // (reads in flight at each wait: the K behind this one, then V's by twos)
+    __builtin_amdgcn_s_setprio(1);
+    MLOP_QK(0, 7, 0);
     if constexpr (FIRST) {
-      MLOP_WAIT_K(3, kf[0]); sn = mfma32(kf[0], qf[4], sn); MLOP_SLOT(4); MLOP_SLOT(5);
-      MLOP_WAIT_K(2, kf[1]); sn = mfma32(kf[1], qf[5], sn); MLOP_SLOT(6); MLOP_SLOT(7); MLOP_SLOT(8);
-      MLOP_WAIT_K(1, kf[2]); sn = mfma32(kf[2], qf[6], sn); MLOP_SLOT(9); MLOP_SLOT(10); MLOP_SLOT(11);
-      MLOP_WAIT_K(0, kf[3]); sn = mfma32(kf[3], qf[7], sn); MLOP_SLOT(12); MLOP_SLOT(13); MLOP_SLOT(14); MLOP_SLOT(15);
+      MLOP_QK(1, 6, 1); MLOP_SLOT(2);
+      MLOP_QK(2, 5, 3); MLOP_SLOT(4);
+      MLOP_QK(3, 4, 5); MLOP_SLOT(6);
+      MLOP_QK(4, 3, 7); MLOP_SLOT(8);
+      MLOP_QK(5, 2, 9); MLOP_SLOT(10);
+      MLOP_QK(6, 1, 11); MLOP_SLOT(12);
+      MLOP_QK(7, 0, 13); MLOP_SLOT(14); MLOP_SLOT(15);
     } else {
-      MLOP_WAIT_K(3, kf[0]); sn = mfma32(kf[0], qf[4], sn); MLOP_VREAD(0, va, 0, vs); MLOP_SLOT(4);
-      MLOP_WAIT_K(6, kf[1]); sn = mfma32(kf[1], qf[5], sn); MLOP_SLOT(5);
-      MLOP_WAIT_K(5, kf[2]); sn = mfma32(kf[2], qf[6], sn); MLOP_VREAD(1, vb, 0, vs); MLOP_SLOT(6);
-      MLOP_WAIT_K(8, kf[3]); sn = mfma32(kf[3], qf[7], sn); MLOP_SLOT(7);
+      MLOP_QK(1, 6, 1); MLOP_VREAD(0, vf[0], 0, vs);
+      MLOP_QK(2, 7, 2); MLOP_VREAD(1, vf[1], 0, vs);
+      MLOP_QK(3, 8, 3); MLOP_VREAD(2, vf[2], 0, vs);
+      MLOP_QK(4, 9, 4); MLOP_VREAD(3, vf[3], 0, vs);
+      MLOP_QK(5, 10, 5); MLOP_VREAD(4, vf[4], 0, vs);
+      MLOP_QK(6, 11, 6); MLOP_VREAD(5, vf[5], 0, vs);
+      MLOP_QK(7, 12, 7);
       const bf16x8 p0f = __builtin_bit_cast(bf16x8, wp[0]), p1f = __builtin_bit_cast(bf16x8, wp[1]);
-      MLOP_WAIT_V(4, va); o[0] = mfma32(frag(va[0], va[1]), p0f, o[0]); MLOP_SLOT(8);
-      o[0] = mfma32(frag(va[2], va[3]), p1f, o[0]); MLOP_VREAD(2, va, 0, vs); MLOP_SLOT(9);
-      MLOP_WAIT_V(4, vb); o[1] = mfma32(frag(vb[0], vb[1]), p0f, o[1]); MLOP_SLOT(10);
-      o[1] = mfma32(frag(vb[2], vb[3]), p1f, o[1]); MLOP_VREAD(3, vb, 0, vs); MLOP_SLOT(11);
-      MLOP_WAIT_V(4, va); o[2] = mfma32(frag(va[0], va[1]), p0f, o[2]); MLOP_SLOT(12);
-      o[2] = mfma32(frag(va[2], va[3]), p1f, o[2]); MLOP_SLOT(13);
-      MLOP_WAIT_V(0, vb); o[3] = mfma32(frag(vb[0], vb[1]), p0f, o[3]); MLOP_SLOT(14);
-      o[3] = mfma32(frag(vb[2], vb[3]), p1f, o[3]); MLOP_SLOT(15);
+      MLOP_PV(0, 10, 8); MLOP_VREAD(6, vf[6], 0, vs);
+      MLOP_PV(1, 10, 9); MLOP_VREAD(7, vf[7], 0, vs);
+      MLOP_PV(2, 10, 10);
+      MLOP_PV(3, 8, 11);
+      MLOP_PV(4, 6, 12);
+      MLOP_PV(5, 4, 13);
+      MLOP_PV(6, 2, 14);
+      MLOP_PV(7, 0, 15);
     }
+    __builtin_amdgcn_s_setprio(0);
     soft(16, sc, wn);
     rescale();
   };
   // The last pair: its softmax under O += V^T . P^T of the pair before, then its own
-  auto finish = [&](f32x16& sc, const u32x4 (&wp)[2]) {
+  auto finish = [&](Sc& sc, const u32x4 (&wp)[2]) {
     u32x4 wn[2];
-    v4s16 va[4], vb[4];
+    v4s16 vf[8][2];
     wait_vmcnt<0>();
     raw_barrier();
+    const uint32_t v1 = (uint32_t)((n_pairs + STAGES - 2) % STAGES) * SLOT, v0 = (uint32_t)((n_pairs + STAGES - 1) % STAGES) * SLOT;
     row_max(sc, n_pairs - 1);
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    const uint32_t v1 = (uint32_t)((n_pairs + 1) % 3) * SLOT, v0 = (uint32_t)((n_pairs + 2) % 3) * SLOT;
     if (n_pairs > 1) {
-      MLOP_VREAD(0, va, v1, 0); MLOP_VREAD(1, vb, v1, 0);
+#pragma unroll
+      for (int d = 0; d < 6; ++d) MLOP_VREAD(d, vf[d], v1, 0);
       const bf16x8 p0f = __builtin_bit_cast(bf16x8, wp[0]), p1f = __builtin_bit_cast(bf16x8, wp[1]);
-      MLOP_WAIT_V(4, va); o[0] = mfma32(frag(va[0], va[1]), p0f, o[0]); MLOP_SLOT(0); MLOP_SLOT(1);
-      o[0] = mfma32(frag(va[2], va[3]), p1f, o[0]); MLOP_VREAD(2, va, v1, 0); MLOP_SLOT(2); MLOP_SLOT(3);
-      MLOP_WAIT_V(4, vb); o[1] = mfma32(frag(vb[0], vb[1]), p0f, o[1]); MLOP_SLOT(4); MLOP_SLOT(5);
-      o[1] = mfma32(frag(vb[2], vb[3]), p1f, o[1]); MLOP_VREAD(3, vb, v1, 0); MLOP_SLOT(6); MLOP_SLOT(7);
-      MLOP_WAIT_V(4, va); o[2] = mfma32(frag(va[0], va[1]), p0f, o[2]); MLOP_SLOT(8); MLOP_SLOT(9);
-      o[2] = mfma32(frag(va[2], va[3]), p1f, o[2]); MLOP_SLOT(10); MLOP_SLOT(11);
-      MLOP_WAIT_V(0, vb); o[3] = mfma32(frag(vb[0], vb[1]), p0f, o[3]); MLOP_SLOT(12); MLOP_SLOT(13);
-      o[3] = mfma32(frag(vb[2], vb[3]), p1f, o[3]); MLOP_SLOT(14); MLOP_SLOT(15);
+      MLOP_PV(0, 10, 0); MLOP_VREAD(6, vf[6], v1, 0); MLOP_SLOT(1);
+      MLOP_PV(1, 10, 2); MLOP_VREAD(7, vf[7], v1, 0); MLOP_SLOT(3);
+      MLOP_PV(2, 10, 4); MLOP_SLOT(5);
+      MLOP_PV(3, 8, 6); MLOP_SLOT(7);
+      MLOP_PV(4, 6, 8); MLOP_SLOT(9);
+      MLOP_PV(5, 4, 10); MLOP_SLOT(11);
+      MLOP_PV(6, 2, 12); MLOP_SLOT(13);
+      MLOP_PV(7, 0, 14); MLOP_SLOT(15);
     } else {
 #pragma unroll
       for (int r = 0; r < 16; ++r) soft(r, sc, wn);
@@ -886,92 +927,103 @@ __device__ __forceinline__ void flash32_item(
     soft(16, sc, wn);
     rescale();
     const bf16x8 p0f = __builtin_bit_cast(bf16x8, wn[0]), p1f = __builtin_bit_cast(bf16x8, wn[1]);
-    MLOP_VREAD(0, va, v0, 0); MLOP_VREAD(1, vb, v0, 0);
-    MLOP_WAIT_V(4, va); o[0] = mfma32(frag(va[0], va[1]), p0f, o[0]); o[0] = mfma32(frag(va[2], va[3]), p1f, o[0]);
-    MLOP_VREAD(2, va, v0, 0);
-    MLOP_WAIT_V(4, vb); o[1] = mfma32(frag(vb[0], vb[1]), p0f, o[1]); o[1] = mfma32(frag(vb[2], vb[3]), p1f, o[1]);
-    MLOP_VREAD(3, vb, v0, 0);
-    MLOP_WAIT_V(4, va); o[2] = mfma32(frag(va[0], va[1]), p0f, o[2]); o[2] = mfma32(frag(va[2], va[3]), p1f, o[2]);
-    MLOP_WAIT_V(0, vb); o[3] = mfma32(frag(vb[0], vb[1]), p0f, o[3]); o[3] = mfma32(frag(vb[2], vb[3]), p1f, o[3]);
+#define MLOP_PV1(d, n)                       \
+  mfma16_into<n>(o[d][0], frag(vf[d]), p0f); \
+  mfma16_into<-1>(o[d][1], frag(vf[d]), p1f)
+#pragma unroll
+    for (int d = 0; d < 6; ++d) MLOP_VREAD(d, vf[d], v0, 0);
+    MLOP_PV1(0, 10); MLOP_VREAD(6, vf[6], v0, 0);
+    MLOP_PV1(1, 10); MLOP_VREAD(7, vf[7], v0, 0);
+    MLOP_PV1(2, 10);
+    MLOP_PV1(3, 8);
+    MLOP_PV1(4, 6);
+    MLOP_PV1(5, 4);
+    MLOP_PV1(6, 2);
+    MLOP_PV1(7, 0);
+#undef MLOP_PV1
   };
 #undef MLOP_SLOT
+#undef MLOP_QK
+#undef MLOP_PV
   // S of pair 0
-  auto qk0 = [&]() {
+  auto qk0 = [&](Sc& sc) {
     bf16x8 kf[8];
-    f32x16 sc = zero();
 #pragma unroll
-    for (int t = 0; t < 8; ++t) MLOP_KREAD(t, kf[t], 0);
-    MLOP_WAIT_K(7, kf[0]); sc = mfma32(kf[0], qf[0], sc);
-    MLOP_WAIT_K(6, kf[1]); sc = mfma32(kf[1], qf[1], sc);
-    MLOP_WAIT_K(5, kf[2]); sc = mfma32(kf[2], qf[2], sc);
-    MLOP_WAIT_K(4, kf[3]); sc = mfma32(kf[3], qf[3], sc);
-    MLOP_WAIT_K(3, kf[4]); sc = mfma32(kf[4], qf[4], sc);
-    MLOP_WAIT_K(2, kf[5]); sc = mfma32(kf[5], qf[5], sc);
-    MLOP_WAIT_K(1, kf[6]); sc = mfma32(kf[6], qf[6], sc);
-    MLOP_WAIT_K(0, kf[7]); sc = mfma32(kf[7], qf[7], sc);
-    return sc;
+    for (int f = 0; f < 8; ++f) MLOP_KREAD(f, kf[f], 0);
+#define MLOP_QK0(f, n)                                               \
+  mfma16_into<n, ((f) < 2)>(sc[(f) & 1][0], kf[f], qf[0][(f) >> 1]); \
+  mfma16_into<-1, ((f) < 2)>(sc[(f) & 1][1], kf[f], qf[1][(f) >> 1])
+    MLOP_QK0(0, 7); MLOP_QK0(1, 6); MLOP_QK0(2, 5); MLOP_QK0(3, 4); MLOP_QK0(4, 3); MLOP_QK0(5, 2); MLOP_QK0(6, 1); MLOP_QK0(7, 0);
+#undef MLOP_QK0
+    asm volatile("s_nop 15" : "+v"(sc[0][0]), "+v"(sc[0][1]), "+v"(sc[1][0]), "+v"(sc[1][1]));
   };
 
-  Pages g[6];  // ids of pair p in g[p % 6] (past the last page: the last)
+  // pages of the pairs pp + 1 .. pp + 3, ids of pp + 3 and pp + 4 (pair p in g[p % 4], ids[p % 2])
+  Pages g[4];
+  Ids ids[2] = {ids_of(4), ids_of(3)};
 #pragma unroll
-  for (int i = 0; i < 5; ++i) g[i] = pages_of(i);
-  issue(kh, k_off, 0, g[0]);
-  if (n_pairs > 1) issue(kh, k_off, SLOT, g[1]);
-  issue(vh, v_off, RING_V, g[0]);
-  if (n_pairs > 2) issue(kh, k_off, 2 * SLOT, g[2]);
+  for (int i = 0; i < 3; ++i) g[i] = pages_of(ids_of(i));
+  issue(kh, k_off[0], k_off[1], 0, g[0]);
+  if (n_pairs > 1) issue(kh, k_off[0], k_off[1], SLOT, g[1]);
+  issue(vh, v_off[0], v_off[0], RING_V, g[0]);
+  if (n_pairs > 2) issue(kh, k_off[0], k_off[1], 2 * SLOT, g[2]);
   if (n_pairs > 2) wait_vmcnt<6>(); else if (n_pairs > 1) wait_vmcnt<4>(); else wait_vmcnt<2>();
   raw_barrier();
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the page ids
-  f32x16 sa = qk0(), sb;
+  Sc sa, sb;
   u32x4 wa[2], wb[2];
+  qk0(sa);
   const int last = n_pairs - 1;
+#define MLOP_STEP(P, FIRST, SC, SN, WP, WN)                                                                             \
+  step(std::integral_constant<int, P>{}, std::bool_constant<FIRST>{}, pp, SC, SN, WP, WN, g[(P + 1) % 4], ids[(P + 1) % 2], \
+       g[(P + 3) % 4]);                                                                                                 \
+  ids[(P + 1) % 2] = ids_of(pp + 5);                                                                                    \
+  ++pp
   if (last > 0) {
     int pp = 0;
-#define MLOP_STEP(P, FIRST, SC, SN, WP, WN)                                                                             \
-  step(std::integral_constant<int, P>{}, std::bool_constant<FIRST>{}, pp, SC, SN, WP, WN, g[(P + 1) % 6], g[(P + 3) % 6]); \
-  g[(P + 5) % 6] = pages_of(pp + 5);                                                                                    \
-  if (++pp >= last) break
-    do {
-      MLOP_STEP(0, true, sa, sb, wb, wa);
-      for (;;) {
-        MLOP_STEP(1, false, sb, sa, wa, wb);
-        MLOP_STEP(2, false, sa, sb, wb, wa);
-        MLOP_STEP(3, false, sb, sa, wa, wb);
-        MLOP_STEP(4, false, sa, sb, wb, wa);
-        MLOP_STEP(5, false, sb, sa, wa, wb);
-        MLOP_STEP(0, false, sa, sb, wb, wa);
-      }
-    } while (false);
-#undef MLOP_STEP
-  }
-  {
-    f32x16 sc = last & 1 ? sb : sa;
-    const u32x4 wp[2] = {last & 1 ? wa[0] : wb[0], last & 1 ? wa[1] : wb[1]};
-    finish(sc, wp);
-  }
-#undef MLOP_KREAD
-#undef MLOP_WAIT_K
-#undef MLOP_VREAD
-#undef MLOP_WAIT_V
-
-  // the two lane halves' partial row sums; O^T element r of dim block d is dim
-  // 32 d + 8 (r >> 2) + 4 h + (r & 3) of q row R
-  {
-    const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(l), __float_as_uint(l), false, false);
-    l = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
-  }
-  if (!q_ok) return;
-  const float inv = l > 0.f ? 1.f / l : 0.f;
-  uint16_t* orow = out + ((size_t)(qs + qi) * Hq + kvh * G + R % G) * kD + 4 * h;
-#pragma unroll
-  for (int d = 0; d < 4; ++d)
-#pragma unroll
-    for (int b = 0; b < 4; ++b) {
-      u32x2 v;
-      v[0] = pack2(o[d][4 * b] * inv, o[d][4 * b + 1] * inv);
-      v[1] = pack2(o[d][4 * b + 2] * inv, o[d][4 * b + 3] * inv);
-      *reinterpret_cast<u32x2*>(orow + 32 * d + 8 * b) = v;
+    MLOP_STEP(0, true, sa, sb, wb, wa);
+    while (pp + 4 <= last) {
+      MLOP_STEP(1, false, sb, sa, wa, wb);
+      MLOP_STEP(2, false, sa, sb, wb, wa);
+      MLOP_STEP(3, false, sb, sa, wa, wb);
+      MLOP_STEP(0, false, sa, sb, wb, wa);
     }
+    if (pp < last) {
+      MLOP_STEP(1, false, sb, sa, wa, wb);
+      if (pp < last) {
+        MLOP_STEP(2, false, sa, sb, wb, wa);
+        if (pp < last) {
+          MLOP_STEP(3, false, sb, sa, wa, wb);
+        }
+      }
+    }
+  }
+#undef MLOP_STEP
+  Sc sl;
+  const bool odd = last & 1;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) sl[i >> 1][i & 1][e] = odd ? sb[i >> 1][i & 1][e] : sa[i >> 1][i & 1][e];
+  const u32x4 wl[2] = {odd ? wa[0] : wb[0], odd ? wa[1] : wb[1]};
+  finish(sl, wl);
+#undef MLOP_KREAD
+#undef MLOP_VREAD
+
+  mfma16_settle(o);
+  // the four lane groups' partial row sums; O^T element e of dim block d is dim 16 d + 4 g4 + e of q row b
+#pragma unroll
+  for (int b = 0; b < 2; ++b) {
+    const float sum = sum_x16_x32(l[b]);
+    if (!q_ok[b]) continue;
+    const float inv = sum > 0.f ? 1.f / sum : 0.f;
+    uint16_t* orow = out + ((size_t)(qs + qi[b]) * Hq + kvh * G + (32 * wid + 16 * b + r16) % G) * kD + 4 * g4;
+#pragma unroll
+    for (int d = 0; d < 8; ++d) {
+      const f32x4 y = o[d][b] * inv;
+      *reinterpret_cast<u32x2*>(orow + 16 * d) = u32x2{pack2(y[0], y[1]), pack2(y[2], y[3])};
+    }
+  }
 }
 
 // STREAM (flash_stream op): the persistent grid's tiles as ONE stream of K / V page pairs per
@@ -983,6 +1035,9 @@ __device__ __forceinline__ void flash32_item(
 //     read into registers at tile i+1's start (80 KB of LDS: 2 workgroups per CU);
 //   * the loop is unrolled by the ring depth, so every step's stage is a constant (LDS read
 //     offsets in the instruction) and tile boundaries are a branch inside a step.
+// On the 32x32x16 MFMA: per wave 32 q-rows, ONE per lane column; S^T [32 keys x 32 q]: lane l holds keys (r & 3) + 8 (r >> 2)
+// + 4 h (h = l >> 5) of q column l & 31; O^T [128 d x 32 q], P^T from registers 8s .. 8s + 7 of S as the k-step s fragment,
+// V^T keys 16 s + 4 h + 0..3 and + 8, dims 32 dblk + (l & 31).
 // Every vector memory operation of a wave is counted (4 LDS-DMAs per pair, 8 Q DMAs per tile,
 // 16 O stores per tile: buffer stores, rows past the prompt dropped by the range check, so the
 // count never depends on the data), and a pair's wait is vmcnt(operations issued after its DMAs):
@@ -1329,17 +1384,17 @@ __global__ void __launch_bounds__(256, 2) flash32_stream_kernel(
 // mirror on every slot (16 x 512: positions p, 15 - p, p, 15 - p), and the launch holds whole
 // rounds instead of ~2 k one-item workgroups.
 template <int G, int WPC, bool PERSIST>
-__global__ void __launch_bounds__(256, WPC) flash32_prefill_kernel(
+__global__ void __launch_bounds__(256, WPC) flash_prefill_kernel(
     uint16_t* __restrict__ out, const uint16_t* __restrict__ q, const uint16_t* __restrict__ kc,
     const uint16_t* __restrict__ vc, const int* __restrict__ block_tables, int bt_stride,
     const int* __restrict__ ptile_seq, const int* __restrict__ ptile_q0,
     const int* __restrict__ q_start, const int* __restrict__ q_len,
     const int* __restrict__ ctx_len, int Hq, int Hkv, float scale_log2, int num_blocks, int num_ptiles) {
-  constexpr int STAGES = 3;
+  constexpr int STAGES = kFlashRing;
   constexpr int STAGE = 4 * kBS * kD;    // bf16 per stage: K page A | K page B | V page A | V page B
   __shared__ __attribute__((aligned(256))) uint16_t smem[STAGES * STAGE];
   if constexpr (!PERSIST) {
-    flash32_item<G>(smem, blockIdx.x / Hkv, blockIdx.x % Hkv, out, q, kc, vc, block_tables, bt_stride, ptile_seq,
+    flash_item<G>(smem, blockIdx.x / Hkv, blockIdx.x % Hkv, out, q, kc, vc, block_tables, bt_stride, ptile_seq,
                     ptile_q0, q_start, q_len, ctx_len, Hq, Hkv, scale_log2, num_blocks);
   } else {
     const int kvh = blockIdx.x % Hkv, j = blockIdx.x / Hkv, S = gridDim.x / Hkv;
@@ -1347,14 +1402,14 @@ __global__ void __launch_bounds__(256, WPC) flash32_prefill_kernel(
       const int t = r * S + ((r & 1) ? S - 1 - j : j);
       if (t >= num_ptiles) continue;  // a partial last round: every slot still leaves the loop
       if (r > 0) __syncthreads();      // the previous tile's last ring reads before this tile's DMAs
-      flash32_item<G>(smem, t, kvh, out, q, kc, vc, block_tables, bt_stride, ptile_seq, ptile_q0, q_start, q_len,
+      flash_item<G>(smem, t, kvh, out, q, kc, vc, block_tables, bt_stride, ptile_seq, ptile_q0, q_start, q_len,
                       ctx_len, Hq, Hkv, scale_log2, num_blocks);
     }
   }
 }
 
 // flash_persist op: 0 = one workgroup per (tile, kv head) item; n = the persistent grid of n
-// workgroups per CU (flash32_prefill_kernel PERSIST); n >= 64: exactly n / 64 slots per kv head
+// workgroups per CU (flash_prefill_kernel PERSIST); n >= 64: exactly n / 64 slots per kv head
 // (tests: several rounds on a few tiles).  Off by default: +3-5 % at 16 x 512 in the host's
 // per-sequence order, nothing or -1-2 % at 1024+ tokens in the LPT order the engine uses there
 // (profiles/r06_flash_persist.md).
@@ -1365,7 +1420,7 @@ int flash_persist(int set) {
 }
 
 // flash_stream op: 1 = the persistent grid runs flash32_stream_kernel (cross-tile K / V ring and
-// Q prefetch, 2 workgroups per CU) instead of flash32_item per tile; 0 = off
+// Q prefetch, 2 workgroups per CU) instead of flash_item per tile; 0 = off
 static int g_flash_stream = 0;
 int flash_stream(int set) {
   if (set >= 0) g_flash_stream = set;
@@ -1398,11 +1453,11 @@ void launch_flash_prefill(void* out, const void* q, const void* kc, const void* 
           (uint16_t*)out, (const uint16_t*)q, (const uint16_t*)kc, (const uint16_t*)vc, bt, bt_stride,   \
           ptile_seq, ptile_q0, q_start, q_len, ctx_len, Hq, Hkv, scale_log2, num_blocks, num_ptiles);    \
     else if (persist)                                                                                    \
-      flash32_prefill_kernel<GG, 2, true><<<grid, 256, 0, st>>>(                                         \
+      flash_prefill_kernel<GG, 2, true><<<grid, 256, 0, st>>>(                                         \
           (uint16_t*)out, (const uint16_t*)q, (const uint16_t*)kc, (const uint16_t*)vc, bt, bt_stride,   \
           ptile_seq, ptile_q0, q_start, q_len, ctx_len, Hq, Hkv, scale_log2, num_blocks, num_ptiles);    \
     else                                                                                                 \
-      flash32_prefill_kernel<GG, 2, false><<<grid, 256, 0, st>>>(                                        \
+      flash_prefill_kernel<GG, 2, false><<<grid, 256, 0, st>>>(                                        \
           (uint16_t*)out, (const uint16_t*)q, (const uint16_t*)kc, (const uint16_t*)vc, bt, bt_stride,   \
           ptile_seq, ptile_q0, q_start, q_len, ctx_len, Hq, Hkv, scale_log2, num_blocks, num_ptiles);    \
     break;

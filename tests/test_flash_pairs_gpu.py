@@ -1,4 +1,4 @@
-"""Flash prefill (attention.hip flash32_item) where its pipeline begins and ends: one pair of pages up to more than two rounds
+"""Flash prefill (attention.hip flash_item) where its pipeline begins and ends: one pair of pages up to more than two rounds
 of its unrolled loop, last pairs of one key to 32, rows that move the running max at every pair."""
 import numpy as np
 import pytest
