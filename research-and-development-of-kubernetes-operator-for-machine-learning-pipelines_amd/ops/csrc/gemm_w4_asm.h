@@ -109,783 +109,813 @@
   "s_waitcnt vmcnt(48)\n" \
   "L_w4_go_%=:\n" \
   "s_barrier\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
   "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
   "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
   "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
-  "s_waitcnt lgkmcnt(7)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
   "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
   "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
   "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
   "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
   "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
+  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
+  "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
   "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
-  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
-  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
-  "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], 0\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], 0\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], 0\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], 0\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb0_0], %[fa0_7], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb0_1], %[fa0_7], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], 0\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb0_2], %[fa0_7], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb0_3], %[fa0_7], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], 0\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], 0\n" \
   "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb0_6], %[fa0_7], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb0_7], %[fa0_7], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], 0\n" \
   "buffer_load_dwordx4 %[vo6], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
   "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "buffer_load_dwordx4 %[vo14], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "buffer_load_dwordx4 %[vo15], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
   "s_waitcnt vmcnt(16)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb1_0], %[fa1_7], a[224:227]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb1_1], %[fa1_7], a[228:231]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb1_2], %[fa1_7], a[232:235]\n" \
   "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb1_3], %[fa1_7], a[236:239]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb1_4], %[fa1_7], a[240:243]\n" \
-  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb1_5], %[fa1_7], a[244:247]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
+  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
   "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb1_6], %[fa1_7], a[248:251]\n" \
-  "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb1_7], %[fa1_7], a[252:255]\n" \
+  "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
   "s_cmp_eq_u32 %[iter], 0\n" \
   "s_cbranch_scc1 L_w4_after_%=\n" \
   "L_w4_loop_%=:\n" \
-  "s_waitcnt lgkmcnt(7)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
   "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
   "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
   "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
   "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
   "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb0_0], %[fa0_7], a[224:227]\n" \
   "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb0_1], %[fa0_7], a[228:231]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
   "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb0_2], %[fa0_7], a[232:235]\n" \
   "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb0_3], %[fa0_7], a[236:239]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], a[240:243]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], a[244:247]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
   "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], a[240:243]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], a[244:247]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
   "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb0_6], %[fa0_7], a[248:251]\n" \
   "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb0_7], %[fa0_7], a[252:255]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
   "buffer_load_dwordx4 %[vo6], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
   "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "buffer_load_dwordx4 %[vo14], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "buffer_load_dwordx4 %[vo15], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
   "s_waitcnt vmcnt(16)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb1_0], %[fa1_7], a[224:227]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb1_1], %[fa1_7], a[228:231]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb1_2], %[fa1_7], a[232:235]\n" \
   "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb1_3], %[fa1_7], a[236:239]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb1_4], %[fa1_7], a[240:243]\n" \
-  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb1_5], %[fa1_7], a[244:247]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
+  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
   "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb1_6], %[fa1_7], a[248:251]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb1_7], %[fa1_7], a[252:255]\n" \
   "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
   "s_sub_u32 %[iter], %[iter], 1\n" \
   "s_cmp_lg_u32 %[iter], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb1_7], %[fa1_7], a[252:255]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
   "s_cbranch_scc1 L_w4_loop_%=\n" \
   "L_w4_after_%=:\n" \
-  "s_waitcnt lgkmcnt(7)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
   "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
   "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
   "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
   "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
   "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
   "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
   "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb0_0], %[fa0_7], a[224:227]\n" \
   "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb0_1], %[fa0_7], a[228:231]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
   "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb0_2], %[fa0_7], a[232:235]\n" \
   "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb0_3], %[fa0_7], a[236:239]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
   "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], a[240:243]\n" \
   "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], a[244:247]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
   "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb0_6], %[fa0_7], a[248:251]\n" \
   "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb0_7], %[fa0_7], a[252:255]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
   "s_waitcnt lgkmcnt(7)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "s_waitcnt lgkmcnt(6)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "s_waitcnt lgkmcnt(5)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(4)\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "s_waitcnt lgkmcnt(2)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
   "s_waitcnt vmcnt(0)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
   "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
   "s_waitcnt lgkmcnt(7)\n" \
   "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "s_waitcnt lgkmcnt(7)\n" \
   "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb1_0], %[fa1_7], a[224:227]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb1_1], %[fa1_7], a[228:231]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb1_2], %[fa1_7], a[232:235]\n" \
   "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb1_3], %[fa1_7], a[236:239]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb1_4], %[fa1_7], a[240:243]\n" \
-  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb1_5], %[fa1_7], a[244:247]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
+  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
   "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb1_6], %[fa1_7], a[248:251]\n" \
-  "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb1_7], %[fa1_7], a[252:255]\n" \
-  "s_waitcnt lgkmcnt(7)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
   "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
   "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
   "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
   "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
   "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
   "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
   "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb0_0], %[fa0_7], a[224:227]\n" \
   "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb0_1], %[fa0_7], a[228:231]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
   "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb0_2], %[fa0_7], a[232:235]\n" \
   "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb0_3], %[fa0_7], a[236:239]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
   "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], a[240:243]\n" \
   "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], a[244:247]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
   "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb0_6], %[fa0_7], a[248:251]\n" \
   "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb0_7], %[fa0_7], a[252:255]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
   "s_waitcnt lgkmcnt(7)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "s_waitcnt lgkmcnt(6)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "s_waitcnt lgkmcnt(5)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(4)\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
   "s_waitcnt lgkmcnt(2)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
   "s_waitcnt lgkmcnt(1)\n" \
   "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb1_0], %[fa1_7], a[224:227]\n" \
   "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb1_1], %[fa1_7], a[228:231]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
   "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb1_2], %[fa1_7], a[232:235]\n" \
   "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb1_3], %[fa1_7], a[236:239]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
   "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb1_4], %[fa1_7], a[240:243]\n" \
   "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb1_5], %[fa1_7], a[244:247]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
   "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb1_6], %[fa1_7], a[248:251]\n" \
   "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb1_7], %[fa1_7], a[252:255]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
   "s_barrier\n" \
   "s_cmp_eq_u32 %[has_next], 0\n" \
   "s_cbranch_scc1 L_w4_end_%=\n" \
@@ -1099,783 +1129,813 @@
   "s_waitcnt vmcnt(32)\n" \
   "L_w4_go_%=:\n" \
   "s_barrier\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
   "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
   "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
   "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
-  "s_waitcnt lgkmcnt(7)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
   "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
   "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
   "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
   "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
   "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
+  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
+  "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
   "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
-  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
-  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
-  "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], 0\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], 0\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], 0\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], 0\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb0_0], %[fa0_7], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb0_1], %[fa0_7], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], 0\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb0_2], %[fa0_7], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb0_3], %[fa0_7], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], 0\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], 0\n" \
   "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb0_6], %[fa0_7], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb0_7], %[fa0_7], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], 0\n" \
   "buffer_load_dwordx4 %[vo6], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
   "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "buffer_load_dwordx4 %[vo14], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "buffer_load_dwordx4 %[vo15], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
   "s_waitcnt vmcnt(16)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb1_0], %[fa1_7], a[224:227]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb1_1], %[fa1_7], a[228:231]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb1_2], %[fa1_7], a[232:235]\n" \
   "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb1_3], %[fa1_7], a[236:239]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb1_4], %[fa1_7], a[240:243]\n" \
-  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb1_5], %[fa1_7], a[244:247]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
+  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
   "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb1_6], %[fa1_7], a[248:251]\n" \
-  "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb1_7], %[fa1_7], a[252:255]\n" \
+  "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
   "s_cmp_eq_u32 %[iter], 0\n" \
   "s_cbranch_scc1 L_w4_after_%=\n" \
   "L_w4_loop_%=:\n" \
-  "s_waitcnt lgkmcnt(7)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
   "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
   "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
   "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
   "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
   "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb0_0], %[fa0_7], a[224:227]\n" \
   "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb0_1], %[fa0_7], a[228:231]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
   "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb0_2], %[fa0_7], a[232:235]\n" \
   "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb0_3], %[fa0_7], a[236:239]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], a[240:243]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], a[244:247]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
   "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], a[240:243]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], a[244:247]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
   "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb0_6], %[fa0_7], a[248:251]\n" \
   "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb0_7], %[fa0_7], a[252:255]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
   "buffer_load_dwordx4 %[vo6], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
   "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "buffer_load_dwordx4 %[vo14], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "buffer_load_dwordx4 %[vo15], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
   "s_waitcnt vmcnt(16)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb1_0], %[fa1_7], a[224:227]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb1_1], %[fa1_7], a[228:231]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb1_2], %[fa1_7], a[232:235]\n" \
   "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb1_3], %[fa1_7], a[236:239]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb1_4], %[fa1_7], a[240:243]\n" \
-  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb1_5], %[fa1_7], a[244:247]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
+  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
   "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb1_6], %[fa1_7], a[248:251]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb1_7], %[fa1_7], a[252:255]\n" \
   "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
   "s_sub_u32 %[iter], %[iter], 1\n" \
   "s_cmp_lg_u32 %[iter], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb1_7], %[fa1_7], a[252:255]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
   "s_cbranch_scc1 L_w4_loop_%=\n" \
   "L_w4_after_%=:\n" \
-  "s_waitcnt lgkmcnt(7)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
   "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
   "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
   "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
   "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
   "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
   "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
   "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb0_0], %[fa0_7], a[224:227]\n" \
   "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb0_1], %[fa0_7], a[228:231]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
   "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb0_2], %[fa0_7], a[232:235]\n" \
   "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb0_3], %[fa0_7], a[236:239]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
   "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], a[240:243]\n" \
   "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], a[244:247]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
   "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb0_6], %[fa0_7], a[248:251]\n" \
   "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb0_7], %[fa0_7], a[252:255]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
   "s_waitcnt lgkmcnt(7)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "s_waitcnt lgkmcnt(6)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "s_waitcnt lgkmcnt(5)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(4)\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "s_waitcnt lgkmcnt(2)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
   "s_waitcnt vmcnt(0)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
   "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
   "s_waitcnt lgkmcnt(7)\n" \
   "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "s_waitcnt lgkmcnt(7)\n" \
   "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb1_0], %[fa1_7], a[224:227]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb1_1], %[fa1_7], a[228:231]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb1_2], %[fa1_7], a[232:235]\n" \
   "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb1_3], %[fa1_7], a[236:239]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb1_4], %[fa1_7], a[240:243]\n" \
-  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb1_5], %[fa1_7], a[244:247]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
+  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
   "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb1_6], %[fa1_7], a[248:251]\n" \
-  "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb1_7], %[fa1_7], a[252:255]\n" \
-  "s_waitcnt lgkmcnt(7)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
   "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
   "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
   "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
   "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
   "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
   "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
   "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb0_0], %[fa0_7], a[224:227]\n" \
   "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb0_1], %[fa0_7], a[228:231]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
   "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb0_2], %[fa0_7], a[232:235]\n" \
   "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb0_3], %[fa0_7], a[236:239]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
   "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], a[240:243]\n" \
   "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], a[244:247]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
   "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb0_6], %[fa0_7], a[248:251]\n" \
   "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb0_7], %[fa0_7], a[252:255]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
   "s_waitcnt lgkmcnt(7)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "s_waitcnt lgkmcnt(6)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "s_waitcnt lgkmcnt(5)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(4)\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
   "s_waitcnt lgkmcnt(2)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
   "s_waitcnt lgkmcnt(1)\n" \
   "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb1_0], %[fa1_7], a[224:227]\n" \
   "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb1_1], %[fa1_7], a[228:231]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
   "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb1_2], %[fa1_7], a[232:235]\n" \
   "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb1_3], %[fa1_7], a[236:239]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
   "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb1_4], %[fa1_7], a[240:243]\n" \
   "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb1_5], %[fa1_7], a[244:247]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
   "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb1_6], %[fa1_7], a[248:251]\n" \
   "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb1_7], %[fa1_7], a[252:255]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
   "s_barrier\n" \
   "s_cmp_eq_u32 %[has_next], 0\n" \
   "s_cbranch_scc1 L_w4_end_%=\n" \
@@ -2089,783 +2149,813 @@
   "s_waitcnt vmcnt(50)\n" \
   "L_w4_go_%=:\n" \
   "s_barrier\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
   "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
   "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
   "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
-  "s_waitcnt lgkmcnt(7)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
   "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
   "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
   "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
   "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
   "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
+  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
+  "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
   "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
-  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
-  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
-  "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], 0\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], 0\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], 0\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], 0\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb0_0], %[fa0_7], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb0_1], %[fa0_7], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], 0\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb0_2], %[fa0_7], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb0_3], %[fa0_7], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], 0\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], 0\n" \
   "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb0_6], %[fa0_7], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb0_7], %[fa0_7], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], 0\n" \
   "buffer_load_dwordx4 %[vo6], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
   "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "buffer_load_dwordx4 %[vo14], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "buffer_load_dwordx4 %[vo15], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
   "s_waitcnt vmcnt(16)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb1_0], %[fa1_7], a[224:227]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb1_1], %[fa1_7], a[228:231]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb1_2], %[fa1_7], a[232:235]\n" \
   "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb1_3], %[fa1_7], a[236:239]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb1_4], %[fa1_7], a[240:243]\n" \
-  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb1_5], %[fa1_7], a[244:247]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
+  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
   "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb1_6], %[fa1_7], a[248:251]\n" \
-  "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb1_7], %[fa1_7], a[252:255]\n" \
+  "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
   "s_cmp_eq_u32 %[iter], 0\n" \
   "s_cbranch_scc1 L_w4_after_%=\n" \
   "L_w4_loop_%=:\n" \
-  "s_waitcnt lgkmcnt(7)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
   "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
   "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
   "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
   "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
   "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb0_0], %[fa0_7], a[224:227]\n" \
   "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb0_1], %[fa0_7], a[228:231]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
   "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb0_2], %[fa0_7], a[232:235]\n" \
   "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb0_3], %[fa0_7], a[236:239]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], a[240:243]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], a[244:247]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
   "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], a[240:243]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], a[244:247]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
   "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb0_6], %[fa0_7], a[248:251]\n" \
   "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb0_7], %[fa0_7], a[252:255]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
   "buffer_load_dwordx4 %[vo6], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
   "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "buffer_load_dwordx4 %[vo14], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "buffer_load_dwordx4 %[vo15], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
   "s_waitcnt vmcnt(16)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb1_0], %[fa1_7], a[224:227]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb1_1], %[fa1_7], a[228:231]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb1_2], %[fa1_7], a[232:235]\n" \
   "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb1_3], %[fa1_7], a[236:239]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb1_4], %[fa1_7], a[240:243]\n" \
-  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb1_5], %[fa1_7], a[244:247]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
+  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
   "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb1_6], %[fa1_7], a[248:251]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb1_7], %[fa1_7], a[252:255]\n" \
   "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
   "s_sub_u32 %[iter], %[iter], 1\n" \
   "s_cmp_lg_u32 %[iter], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb1_7], %[fa1_7], a[252:255]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
   "s_cbranch_scc1 L_w4_loop_%=\n" \
   "L_w4_after_%=:\n" \
-  "s_waitcnt lgkmcnt(7)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
   "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
   "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
   "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
   "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
   "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
   "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
   "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb0_0], %[fa0_7], a[224:227]\n" \
   "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb0_1], %[fa0_7], a[228:231]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
   "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb0_2], %[fa0_7], a[232:235]\n" \
   "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb0_3], %[fa0_7], a[236:239]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
   "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], a[240:243]\n" \
   "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], a[244:247]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
   "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb0_6], %[fa0_7], a[248:251]\n" \
   "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb0_7], %[fa0_7], a[252:255]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
   "s_waitcnt lgkmcnt(7)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "s_waitcnt lgkmcnt(6)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "s_waitcnt lgkmcnt(5)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(4)\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "s_waitcnt lgkmcnt(2)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
   "s_waitcnt vmcnt(0)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
   "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
   "s_waitcnt lgkmcnt(7)\n" \
   "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "s_waitcnt lgkmcnt(7)\n" \
   "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb1_0], %[fa1_7], a[224:227]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb1_1], %[fa1_7], a[228:231]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb1_2], %[fa1_7], a[232:235]\n" \
   "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb1_3], %[fa1_7], a[236:239]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb1_4], %[fa1_7], a[240:243]\n" \
-  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb1_5], %[fa1_7], a[244:247]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
+  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
   "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb1_6], %[fa1_7], a[248:251]\n" \
-  "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb1_7], %[fa1_7], a[252:255]\n" \
-  "s_waitcnt lgkmcnt(7)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
   "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
   "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
   "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
   "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
   "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
   "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
   "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb0_0], %[fa0_7], a[224:227]\n" \
   "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb0_1], %[fa0_7], a[228:231]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
   "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb0_2], %[fa0_7], a[232:235]\n" \
   "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb0_3], %[fa0_7], a[236:239]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
   "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], a[240:243]\n" \
   "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], a[244:247]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
   "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb0_6], %[fa0_7], a[248:251]\n" \
   "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb0_7], %[fa0_7], a[252:255]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
   "s_waitcnt lgkmcnt(7)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "s_waitcnt lgkmcnt(6)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "s_waitcnt lgkmcnt(5)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(4)\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
   "s_waitcnt lgkmcnt(2)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
   "s_waitcnt lgkmcnt(1)\n" \
   "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb1_0], %[fa1_7], a[224:227]\n" \
   "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb1_1], %[fa1_7], a[228:231]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
   "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb1_2], %[fa1_7], a[232:235]\n" \
   "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb1_3], %[fa1_7], a[236:239]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
   "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb1_4], %[fa1_7], a[240:243]\n" \
   "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb1_5], %[fa1_7], a[244:247]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
   "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb1_6], %[fa1_7], a[248:251]\n" \
   "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb1_7], %[fa1_7], a[252:255]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
   "s_barrier\n" \
   "s_cmp_eq_u32 %[has_next], 0\n" \
   "s_cbranch_scc1 L_w4_end_%=\n" \
@@ -3079,783 +3169,813 @@
   "s_waitcnt vmcnt(34)\n" \
   "L_w4_go_%=:\n" \
   "s_barrier\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
   "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
   "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
   "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
-  "s_waitcnt lgkmcnt(7)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
   "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
   "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
   "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
   "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
   "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
+  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
+  "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
   "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
-  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
-  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
-  "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], 0\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], 0\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], 0\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], 0\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb0_0], %[fa0_7], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb0_1], %[fa0_7], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], 0\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb0_2], %[fa0_7], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb0_3], %[fa0_7], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], 0\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], 0\n" \
   "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb0_6], %[fa0_7], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb0_7], %[fa0_7], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], 0\n" \
   "buffer_load_dwordx4 %[vo6], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
   "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "buffer_load_dwordx4 %[vo14], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "buffer_load_dwordx4 %[vo15], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
   "s_waitcnt vmcnt(16)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb1_0], %[fa1_7], a[224:227]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb1_1], %[fa1_7], a[228:231]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb1_2], %[fa1_7], a[232:235]\n" \
   "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb1_3], %[fa1_7], a[236:239]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb1_4], %[fa1_7], a[240:243]\n" \
-  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb1_5], %[fa1_7], a[244:247]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
+  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
   "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb1_6], %[fa1_7], a[248:251]\n" \
-  "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb1_7], %[fa1_7], a[252:255]\n" \
+  "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
   "s_cmp_eq_u32 %[iter], 0\n" \
   "s_cbranch_scc1 L_w4_after_%=\n" \
   "L_w4_loop_%=:\n" \
-  "s_waitcnt lgkmcnt(7)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
   "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
   "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
   "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
   "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
   "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb0_0], %[fa0_7], a[224:227]\n" \
   "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb0_1], %[fa0_7], a[228:231]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
   "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb0_2], %[fa0_7], a[232:235]\n" \
   "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb0_3], %[fa0_7], a[236:239]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], a[240:243]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], a[244:247]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
   "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], a[240:243]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], a[244:247]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
   "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb0_6], %[fa0_7], a[248:251]\n" \
   "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb0_7], %[fa0_7], a[252:255]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
   "buffer_load_dwordx4 %[vo6], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
   "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "buffer_load_dwordx4 %[vo14], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "buffer_load_dwordx4 %[vo15], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
   "s_waitcnt vmcnt(16)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb1_0], %[fa1_7], a[224:227]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb1_1], %[fa1_7], a[228:231]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb1_2], %[fa1_7], a[232:235]\n" \
   "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb1_3], %[fa1_7], a[236:239]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb1_4], %[fa1_7], a[240:243]\n" \
-  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb1_5], %[fa1_7], a[244:247]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
+  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
   "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb1_6], %[fa1_7], a[248:251]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb1_7], %[fa1_7], a[252:255]\n" \
   "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
   "s_sub_u32 %[iter], %[iter], 1\n" \
   "s_cmp_lg_u32 %[iter], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb1_7], %[fa1_7], a[252:255]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
   "s_cbranch_scc1 L_w4_loop_%=\n" \
   "L_w4_after_%=:\n" \
-  "s_waitcnt lgkmcnt(7)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
   "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
   "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
   "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
   "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
   "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
   "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
   "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb0_0], %[fa0_7], a[224:227]\n" \
   "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb0_1], %[fa0_7], a[228:231]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
   "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb0_2], %[fa0_7], a[232:235]\n" \
   "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb0_3], %[fa0_7], a[236:239]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
   "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], a[240:243]\n" \
   "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], a[244:247]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
   "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb0_6], %[fa0_7], a[248:251]\n" \
   "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb0_7], %[fa0_7], a[252:255]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
   "s_waitcnt lgkmcnt(7)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "s_waitcnt lgkmcnt(6)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "s_waitcnt lgkmcnt(5)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(4)\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "s_waitcnt lgkmcnt(2)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
   "s_waitcnt vmcnt(0)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
   "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
   "s_waitcnt lgkmcnt(7)\n" \
   "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "s_waitcnt lgkmcnt(7)\n" \
   "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb1_0], %[fa1_7], a[224:227]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb1_1], %[fa1_7], a[228:231]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb1_2], %[fa1_7], a[232:235]\n" \
   "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb1_3], %[fa1_7], a[236:239]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb1_4], %[fa1_7], a[240:243]\n" \
-  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb1_5], %[fa1_7], a[244:247]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
+  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
   "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb1_6], %[fa1_7], a[248:251]\n" \
-  "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb1_7], %[fa1_7], a[252:255]\n" \
-  "s_waitcnt lgkmcnt(7)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
   "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
   "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
   "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
   "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
   "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
   "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
   "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb0_0], %[fa0_7], a[224:227]\n" \
   "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb0_1], %[fa0_7], a[228:231]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
   "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb0_2], %[fa0_7], a[232:235]\n" \
   "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb0_3], %[fa0_7], a[236:239]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
   "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], a[240:243]\n" \
   "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], a[244:247]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
   "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb0_6], %[fa0_7], a[248:251]\n" \
   "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb0_7], %[fa0_7], a[252:255]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
   "s_waitcnt lgkmcnt(7)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "s_waitcnt lgkmcnt(6)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "s_waitcnt lgkmcnt(5)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(4)\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
   "s_waitcnt lgkmcnt(2)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
   "s_waitcnt lgkmcnt(1)\n" \
   "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb1_0], %[fa1_7], a[224:227]\n" \
   "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb1_1], %[fa1_7], a[228:231]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
   "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb1_2], %[fa1_7], a[232:235]\n" \
   "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb1_3], %[fa1_7], a[236:239]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
   "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb1_4], %[fa1_7], a[240:243]\n" \
   "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb1_5], %[fa1_7], a[244:247]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
   "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb1_6], %[fa1_7], a[248:251]\n" \
   "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb1_7], %[fa1_7], a[252:255]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
   "s_barrier\n" \
   "s_cmp_eq_u32 %[has_next], 0\n" \
   "s_cbranch_scc1 L_w4_end_%=\n" \
@@ -4045,467 +4165,497 @@
   "s_waitcnt vmcnt(28)\n" \
   "L_w4_go_%=:\n" \
   "s_barrier\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
   "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
   "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
   "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
   "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(15)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
+  "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
+  "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
-  "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
-  "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
   "buffer_load_dwordx4 %[vo4], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
   "buffer_load_dwordx4 %[vo5], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
   "s_waitcnt vmcnt(12)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "s_cmp_eq_u32 %[iter], 0\n" \
   "s_cbranch_scc1 L_w4_after_%=\n" \
   "L_w4_loop_%=:\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
   "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
   "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
   "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
   "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "s_waitcnt lgkmcnt(15)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "buffer_load_dwordx4 %[vo4], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
   "buffer_load_dwordx4 %[vo5], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
   "s_waitcnt vmcnt(12)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "s_sub_u32 %[iter], %[iter], 1\n" \
   "s_cmp_lg_u32 %[iter], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "s_cbranch_scc1 L_w4_loop_%=\n" \
   "L_w4_after_%=:\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
   "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
   "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
   "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
   "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "s_waitcnt lgkmcnt(15)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "s_waitcnt lgkmcnt(2)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
   "s_waitcnt vmcnt(0)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "s_waitcnt lgkmcnt(4)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
   "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
+  "s_waitcnt lgkmcnt(4)\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
   "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
   "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
   "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
   "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "s_waitcnt lgkmcnt(15)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "s_waitcnt lgkmcnt(2)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "s_waitcnt lgkmcnt(1)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "s_barrier\n" \
   "s_cmp_eq_u32 %[has_next], 0\n" \
   "s_cbranch_scc1 L_w4_end_%=\n" \
@@ -4671,467 +4821,497 @@
   "s_waitcnt vmcnt(20)\n" \
   "L_w4_go_%=:\n" \
   "s_barrier\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
   "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
   "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
   "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
   "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(15)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
+  "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
+  "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
-  "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
-  "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
   "buffer_load_dwordx4 %[vo4], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
   "buffer_load_dwordx4 %[vo5], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
   "s_waitcnt vmcnt(12)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "s_cmp_eq_u32 %[iter], 0\n" \
   "s_cbranch_scc1 L_w4_after_%=\n" \
   "L_w4_loop_%=:\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
   "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
   "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
   "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
   "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "s_waitcnt lgkmcnt(15)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "buffer_load_dwordx4 %[vo4], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
   "buffer_load_dwordx4 %[vo5], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
   "s_waitcnt vmcnt(12)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "s_sub_u32 %[iter], %[iter], 1\n" \
   "s_cmp_lg_u32 %[iter], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "s_cbranch_scc1 L_w4_loop_%=\n" \
   "L_w4_after_%=:\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
   "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
   "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
   "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
   "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "s_waitcnt lgkmcnt(15)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "s_waitcnt lgkmcnt(2)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
   "s_waitcnt vmcnt(0)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "s_waitcnt lgkmcnt(4)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
   "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
+  "s_waitcnt lgkmcnt(4)\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
   "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
   "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
   "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
   "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "s_waitcnt lgkmcnt(15)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "s_waitcnt lgkmcnt(2)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "s_waitcnt lgkmcnt(1)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "s_barrier\n" \
   "s_cmp_eq_u32 %[has_next], 0\n" \
   "s_cbranch_scc1 L_w4_end_%=\n" \
@@ -5297,467 +5477,497 @@
   "s_waitcnt vmcnt(30)\n" \
   "L_w4_go_%=:\n" \
   "s_barrier\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
   "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
   "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
   "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
   "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(15)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
+  "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
+  "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
-  "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
-  "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
   "buffer_load_dwordx4 %[vo4], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
   "buffer_load_dwordx4 %[vo5], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
   "s_waitcnt vmcnt(12)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "s_cmp_eq_u32 %[iter], 0\n" \
   "s_cbranch_scc1 L_w4_after_%=\n" \
   "L_w4_loop_%=:\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
   "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
   "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
   "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
   "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "s_waitcnt lgkmcnt(15)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "buffer_load_dwordx4 %[vo4], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
   "buffer_load_dwordx4 %[vo5], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
   "s_waitcnt vmcnt(12)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "s_sub_u32 %[iter], %[iter], 1\n" \
   "s_cmp_lg_u32 %[iter], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "s_cbranch_scc1 L_w4_loop_%=\n" \
   "L_w4_after_%=:\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
   "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
   "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
   "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
   "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "s_waitcnt lgkmcnt(15)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "s_waitcnt lgkmcnt(2)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
   "s_waitcnt vmcnt(0)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "s_waitcnt lgkmcnt(4)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
   "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
+  "s_waitcnt lgkmcnt(4)\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
   "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
   "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
   "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
   "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "s_waitcnt lgkmcnt(15)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "s_waitcnt lgkmcnt(2)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "s_waitcnt lgkmcnt(1)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "s_barrier\n" \
   "s_cmp_eq_u32 %[has_next], 0\n" \
   "s_cbranch_scc1 L_w4_end_%=\n" \
@@ -5923,467 +6133,497 @@
   "s_waitcnt vmcnt(22)\n" \
   "L_w4_go_%=:\n" \
   "s_barrier\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
   "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
   "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
   "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
   "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(15)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
+  "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
+  "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
-  "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
-  "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
   "buffer_load_dwordx4 %[vo4], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
   "buffer_load_dwordx4 %[vo5], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
   "s_waitcnt vmcnt(12)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "s_cmp_eq_u32 %[iter], 0\n" \
   "s_cbranch_scc1 L_w4_after_%=\n" \
   "L_w4_loop_%=:\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
   "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
   "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
   "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
   "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "s_waitcnt lgkmcnt(15)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "buffer_load_dwordx4 %[vo4], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
   "buffer_load_dwordx4 %[vo5], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
   "s_waitcnt vmcnt(12)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "s_sub_u32 %[iter], %[iter], 1\n" \
   "s_cmp_lg_u32 %[iter], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "s_cbranch_scc1 L_w4_loop_%=\n" \
   "L_w4_after_%=:\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
   "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
   "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
   "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
   "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "s_waitcnt lgkmcnt(15)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "s_waitcnt lgkmcnt(2)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
   "s_waitcnt vmcnt(0)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "s_waitcnt lgkmcnt(4)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
   "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
+  "s_waitcnt lgkmcnt(4)\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
   "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
   "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
   "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
   "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "s_waitcnt lgkmcnt(15)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "s_waitcnt lgkmcnt(2)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "s_waitcnt lgkmcnt(1)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "s_barrier\n" \
   "s_cmp_eq_u32 %[has_next], 0\n" \
   "s_cbranch_scc1 L_w4_end_%=\n" \
@@ -6556,6 +6796,7 @@
   "L_w4_go_%=:\n" \
   "s_barrier\n" \
   "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
   "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
   "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
   "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
@@ -6563,86 +6804,92 @@
   "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
   "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
   "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
   "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
   "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
   "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
   "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
   "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
   "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
   "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
   "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdB], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdB], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
   "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
@@ -6659,140 +6906,147 @@
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
   "s_waitcnt vmcnt(13)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
   "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "s_cmp_eq_u32 %[iter], 0\n" \
   "s_cbranch_scc1 L_w4_after_%=\n" \
   "L_w4_loop_%=:\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
   "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
   "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
   "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
   "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
   "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
   "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
   "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
   "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdB], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdB], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
   "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
@@ -6809,126 +7063,133 @@
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
   "s_waitcnt vmcnt(13)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
   "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
   "s_sub_u32 %[iter], %[iter], 1\n" \
   "s_cmp_lg_u32 %[iter], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "s_cbranch_scc1 L_w4_loop_%=\n" \
   "L_w4_after_%=:\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
   "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
   "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
   "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
   "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
   "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
   "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
   "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
   "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
   "s_waitcnt lgkmcnt(4)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
@@ -6939,118 +7200,125 @@
   "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
   "s_waitcnt lgkmcnt(2)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
   "s_waitcnt vmcnt(0)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
   "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
   "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
   "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "s_waitcnt lgkmcnt(7)\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
+  "s_waitcnt lgkmcnt(6)\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
   "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
   "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
   "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
   "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
   "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
   "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
   "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
   "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
   "s_waitcnt lgkmcnt(4)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
@@ -7061,41 +7329,41 @@
   "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
   "s_waitcnt lgkmcnt(2)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
   "s_waitcnt lgkmcnt(1)\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "s_barrier\n" \
   "s_cmp_eq_u32 %[has_next], 0\n" \
   "s_cbranch_scc1 L_w4_end_%=\n" \
@@ -7274,6 +7542,7 @@
   "L_w4_go_%=:\n" \
   "s_barrier\n" \
   "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
   "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
   "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
   "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
@@ -7281,86 +7550,92 @@
   "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
   "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
   "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
   "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
   "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
   "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
   "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
   "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
   "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
   "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
   "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdB], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdB], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
   "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
@@ -7377,140 +7652,147 @@
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
   "s_waitcnt vmcnt(13)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
   "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "s_cmp_eq_u32 %[iter], 0\n" \
   "s_cbranch_scc1 L_w4_after_%=\n" \
   "L_w4_loop_%=:\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
   "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
   "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
   "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
   "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
   "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
   "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
   "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
   "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdB], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdB], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
   "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
@@ -7527,126 +7809,133 @@
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
   "s_waitcnt vmcnt(13)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
   "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
   "s_sub_u32 %[iter], %[iter], 1\n" \
   "s_cmp_lg_u32 %[iter], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "s_cbranch_scc1 L_w4_loop_%=\n" \
   "L_w4_after_%=:\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
   "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
   "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
   "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
   "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
   "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
   "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
   "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
   "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
   "s_waitcnt lgkmcnt(4)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
@@ -7657,118 +7946,125 @@
   "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
   "s_waitcnt lgkmcnt(2)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
   "s_waitcnt vmcnt(0)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
   "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
   "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
   "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "s_waitcnt lgkmcnt(7)\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
+  "s_waitcnt lgkmcnt(6)\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
   "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
   "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
   "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
   "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
   "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
   "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
   "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
   "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
   "s_waitcnt lgkmcnt(4)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
@@ -7779,41 +8075,41 @@
   "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
   "s_waitcnt lgkmcnt(2)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
   "s_waitcnt lgkmcnt(1)\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "s_barrier\n" \
   "s_cmp_eq_u32 %[has_next], 0\n" \
   "s_cbranch_scc1 L_w4_end_%=\n" \
@@ -7992,6 +8288,7 @@
   "L_w4_go_%=:\n" \
   "s_barrier\n" \
   "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
   "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
   "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
   "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
@@ -7999,86 +8296,92 @@
   "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
   "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
   "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
   "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
   "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
   "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
   "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
   "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
   "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
   "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
   "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdB], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdB], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
   "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
@@ -8095,140 +8398,147 @@
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
   "s_waitcnt vmcnt(13)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
   "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "s_cmp_eq_u32 %[iter], 0\n" \
   "s_cbranch_scc1 L_w4_after_%=\n" \
   "L_w4_loop_%=:\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
   "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
   "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
   "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
   "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
   "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
   "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
   "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
   "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdB], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdB], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
   "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
@@ -8245,126 +8555,133 @@
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
   "s_waitcnt vmcnt(13)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
   "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
   "s_sub_u32 %[iter], %[iter], 1\n" \
   "s_cmp_lg_u32 %[iter], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "s_cbranch_scc1 L_w4_loop_%=\n" \
   "L_w4_after_%=:\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
   "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
   "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
   "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
   "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
   "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
   "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
   "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
   "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
   "s_waitcnt lgkmcnt(4)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
@@ -8375,118 +8692,125 @@
   "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
   "s_waitcnt lgkmcnt(2)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
   "s_waitcnt vmcnt(0)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
   "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
   "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
   "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "s_waitcnt lgkmcnt(7)\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
+  "s_waitcnt lgkmcnt(6)\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
   "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
   "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
   "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
   "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
   "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
   "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
   "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
   "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
   "s_waitcnt lgkmcnt(4)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
@@ -8497,41 +8821,41 @@
   "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
   "s_waitcnt lgkmcnt(2)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
   "s_waitcnt lgkmcnt(1)\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "s_barrier\n" \
   "s_cmp_eq_u32 %[has_next], 0\n" \
   "s_cbranch_scc1 L_w4_end_%=\n" \
@@ -8710,6 +9034,7 @@
   "L_w4_go_%=:\n" \
   "s_barrier\n" \
   "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
   "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
   "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
   "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
@@ -8717,86 +9042,92 @@
   "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
   "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
   "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
   "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
   "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
   "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
   "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
   "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
   "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
   "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
   "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdB], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdB], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
   "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
@@ -8813,140 +9144,147 @@
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
   "s_waitcnt vmcnt(13)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
   "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "s_cmp_eq_u32 %[iter], 0\n" \
   "s_cbranch_scc1 L_w4_after_%=\n" \
   "L_w4_loop_%=:\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
   "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
   "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
   "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
   "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
   "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
   "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
   "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
   "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdB], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdB], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
   "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
@@ -8963,126 +9301,133 @@
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
   "s_waitcnt vmcnt(13)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
   "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
   "s_sub_u32 %[iter], %[iter], 1\n" \
   "s_cmp_lg_u32 %[iter], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "s_cbranch_scc1 L_w4_loop_%=\n" \
   "L_w4_after_%=:\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
   "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
   "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
   "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
   "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
   "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
   "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
   "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
   "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
   "s_waitcnt lgkmcnt(4)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
@@ -9093,118 +9438,125 @@
   "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
   "s_waitcnt lgkmcnt(2)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
   "s_waitcnt vmcnt(0)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
   "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
   "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
   "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "s_waitcnt lgkmcnt(7)\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
+  "s_waitcnt lgkmcnt(6)\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
   "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
   "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
   "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
   "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
   "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
   "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
   "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
   "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
   "s_waitcnt lgkmcnt(4)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
@@ -9215,41 +9567,41 @@
   "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
   "s_waitcnt lgkmcnt(2)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
   "s_waitcnt lgkmcnt(1)\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "s_barrier\n" \
   "s_cmp_eq_u32 %[has_next], 0\n" \
   "s_cbranch_scc1 L_w4_end_%=\n" \
@@ -9434,6 +9786,8 @@
   "L_w4_go_%=:\n" \
   "s_barrier\n" \
   "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
   "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
   "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
@@ -9441,617 +9795,643 @@
   "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
   "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
-  "s_waitcnt lgkmcnt(5)\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
   "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(15)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(15)\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
   "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
   "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
   "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
   "s_mov_b32 m0, %[dbase]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], 0\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], 0\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], 0\n" \
-  "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
+  "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
   "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
   "s_waitcnt vmcnt(14)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
   "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
   "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
   "s_cmp_eq_u32 %[iter], 0\n" \
   "s_cbranch_scc1 L_w4_after_%=\n" \
   "L_w4_loop_%=:\n" \
-  "s_waitcnt lgkmcnt(5)\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(15)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(15)\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
   "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
   "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
   "s_mov_b32 m0, %[dbase]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
   "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
   "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
-  "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
   "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
   "s_waitcnt vmcnt(14)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
   "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
   "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
   "s_sub_u32 %[iter], %[iter], 1\n" \
   "s_cmp_lg_u32 %[iter], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
   "s_cbranch_scc1 L_w4_loop_%=\n" \
   "L_w4_after_%=:\n" \
-  "s_waitcnt lgkmcnt(5)\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(15)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(15)\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
   "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
   "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
   "s_waitcnt lgkmcnt(15)\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
   "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
   "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
   "s_waitcnt lgkmcnt(5)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "s_waitcnt lgkmcnt(4)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "s_waitcnt lgkmcnt(2)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
   "s_waitcnt vmcnt(0)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
   "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "s_waitcnt lgkmcnt(8)\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "s_waitcnt lgkmcnt(8)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
   "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
-  "s_waitcnt lgkmcnt(5)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(15)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(15)\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
   "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
   "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
   "s_waitcnt lgkmcnt(15)\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
   "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
   "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
   "s_waitcnt lgkmcnt(5)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "s_waitcnt lgkmcnt(4)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(2)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "s_waitcnt lgkmcnt(1)\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
   "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
   "s_barrier\n" \
   "s_cmp_eq_u32 %[has_next], 0\n" \
   "s_cbranch_scc1 L_w4_end_%=\n" \
@@ -10242,6 +10622,8 @@
   "L_w4_go_%=:\n" \
   "s_barrier\n" \
   "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
   "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
   "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
@@ -10249,617 +10631,643 @@
   "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
   "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
-  "s_waitcnt lgkmcnt(5)\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
   "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(15)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(15)\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
   "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
   "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
   "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
   "s_mov_b32 m0, %[dbase]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], 0\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], 0\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], 0\n" \
-  "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
+  "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
   "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
   "s_waitcnt vmcnt(14)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
   "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
   "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
   "s_cmp_eq_u32 %[iter], 0\n" \
   "s_cbranch_scc1 L_w4_after_%=\n" \
   "L_w4_loop_%=:\n" \
-  "s_waitcnt lgkmcnt(5)\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(15)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(15)\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
   "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
   "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
   "s_mov_b32 m0, %[dbase]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
   "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
   "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
-  "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
   "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
   "s_waitcnt vmcnt(14)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
   "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
   "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
   "s_sub_u32 %[iter], %[iter], 1\n" \
   "s_cmp_lg_u32 %[iter], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
   "s_cbranch_scc1 L_w4_loop_%=\n" \
   "L_w4_after_%=:\n" \
-  "s_waitcnt lgkmcnt(5)\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(15)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(15)\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
   "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
   "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
   "s_waitcnt lgkmcnt(15)\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
   "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
   "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
   "s_waitcnt lgkmcnt(5)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "s_waitcnt lgkmcnt(4)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "s_waitcnt lgkmcnt(2)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
   "s_waitcnt vmcnt(0)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
   "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "s_waitcnt lgkmcnt(8)\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "s_waitcnt lgkmcnt(8)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
   "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
-  "s_waitcnt lgkmcnt(5)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(15)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(15)\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
   "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
   "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
   "s_waitcnt lgkmcnt(15)\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
   "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
   "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
   "s_waitcnt lgkmcnt(5)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "s_waitcnt lgkmcnt(4)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(2)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "s_waitcnt lgkmcnt(1)\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
   "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
   "s_barrier\n" \
   "s_cmp_eq_u32 %[has_next], 0\n" \
   "s_cbranch_scc1 L_w4_end_%=\n" \
@@ -11050,6 +11458,8 @@
   "L_w4_go_%=:\n" \
   "s_barrier\n" \
   "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
   "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
   "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
@@ -11057,617 +11467,643 @@
   "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
   "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
-  "s_waitcnt lgkmcnt(5)\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
   "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(15)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(15)\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
   "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
   "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
   "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
   "s_mov_b32 m0, %[dbase]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], 0\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], 0\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], 0\n" \
-  "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
+  "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
   "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
   "s_waitcnt vmcnt(14)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
   "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
   "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
   "s_cmp_eq_u32 %[iter], 0\n" \
   "s_cbranch_scc1 L_w4_after_%=\n" \
   "L_w4_loop_%=:\n" \
-  "s_waitcnt lgkmcnt(5)\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(15)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(15)\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
   "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
   "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
   "s_mov_b32 m0, %[dbase]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
   "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
   "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
-  "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
   "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
   "s_waitcnt vmcnt(14)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
   "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
   "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
   "s_sub_u32 %[iter], %[iter], 1\n" \
   "s_cmp_lg_u32 %[iter], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
   "s_cbranch_scc1 L_w4_loop_%=\n" \
   "L_w4_after_%=:\n" \
-  "s_waitcnt lgkmcnt(5)\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(15)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(15)\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
   "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
   "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
   "s_waitcnt lgkmcnt(15)\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
   "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
   "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
   "s_waitcnt lgkmcnt(5)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "s_waitcnt lgkmcnt(4)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "s_waitcnt lgkmcnt(2)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
   "s_waitcnt vmcnt(0)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
   "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "s_waitcnt lgkmcnt(8)\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "s_waitcnt lgkmcnt(8)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
   "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
-  "s_waitcnt lgkmcnt(5)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(15)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(15)\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
   "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
   "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
   "s_waitcnt lgkmcnt(15)\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
   "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
   "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
   "s_waitcnt lgkmcnt(5)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "s_waitcnt lgkmcnt(4)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(2)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "s_waitcnt lgkmcnt(1)\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
   "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
   "s_barrier\n" \
   "s_cmp_eq_u32 %[has_next], 0\n" \
   "s_cbranch_scc1 L_w4_end_%=\n" \
@@ -11858,6 +12294,8 @@
   "L_w4_go_%=:\n" \
   "s_barrier\n" \
   "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
   "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
   "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
@@ -11865,617 +12303,643 @@
   "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
   "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
-  "s_waitcnt lgkmcnt(5)\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
   "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(15)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(15)\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
   "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
   "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
   "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
   "s_mov_b32 m0, %[dbase]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], 0\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], 0\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], 0\n" \
-  "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
+  "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
   "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
   "s_waitcnt vmcnt(14)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
   "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
   "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
   "s_cmp_eq_u32 %[iter], 0\n" \
   "s_cbranch_scc1 L_w4_after_%=\n" \
   "L_w4_loop_%=:\n" \
-  "s_waitcnt lgkmcnt(5)\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(15)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(15)\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
   "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
   "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
   "s_mov_b32 m0, %[dbase]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
   "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
   "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
-  "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
   "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
   "s_waitcnt vmcnt(14)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
   "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
   "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
   "s_sub_u32 %[iter], %[iter], 1\n" \
   "s_cmp_lg_u32 %[iter], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
   "s_cbranch_scc1 L_w4_loop_%=\n" \
   "L_w4_after_%=:\n" \
-  "s_waitcnt lgkmcnt(5)\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(15)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(15)\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
   "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
   "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
   "s_waitcnt lgkmcnt(15)\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
   "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
   "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
   "s_waitcnt lgkmcnt(5)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "s_waitcnt lgkmcnt(4)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "s_waitcnt lgkmcnt(2)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
   "s_waitcnt vmcnt(0)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
   "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "s_waitcnt lgkmcnt(8)\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "s_waitcnt lgkmcnt(8)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
   "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
-  "s_waitcnt lgkmcnt(5)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(15)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(15)\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
   "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
   "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
   "s_waitcnt lgkmcnt(15)\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
   "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
   "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
   "s_waitcnt lgkmcnt(5)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "s_waitcnt lgkmcnt(4)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "s_waitcnt lgkmcnt(2)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "s_waitcnt lgkmcnt(1)\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
   "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
   "s_barrier\n" \
   "s_cmp_eq_u32 %[has_next], 0\n" \
   "s_cbranch_scc1 L_w4_end_%=\n" \
@@ -12671,705 +13135,733 @@
   "s_waitcnt vmcnt(43)\n" \
   "L_w4_go_%=:\n" \
   "s_barrier\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
   "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
   "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
-  "s_waitcnt lgkmcnt(6)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
   "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "s_waitcnt lgkmcnt(10)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
+  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
   "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
   "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], 0\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], 0\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], 0\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], 0\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], 0\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], 0\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], 0\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], 0\n" \
   "buffer_load_dwordx4 %[vo6], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
   "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
   "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "buffer_load_dwordx4 %[vo14], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
   "s_waitcnt vmcnt(15)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
   "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
   "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
   "s_cmp_eq_u32 %[iter], 0\n" \
   "s_cbranch_scc1 L_w4_after_%=\n" \
   "L_w4_loop_%=:\n" \
-  "s_waitcnt lgkmcnt(6)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "s_waitcnt lgkmcnt(10)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
   "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
   "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
   "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
   "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
   "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
   "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
   "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
   "buffer_load_dwordx4 %[vo6], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
   "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
   "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "buffer_load_dwordx4 %[vo14], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
   "s_waitcnt vmcnt(15)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
   "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
   "s_sub_u32 %[iter], %[iter], 1\n" \
   "s_cmp_lg_u32 %[iter], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
   "s_cbranch_scc1 L_w4_loop_%=\n" \
   "L_w4_after_%=:\n" \
-  "s_waitcnt lgkmcnt(6)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "s_waitcnt lgkmcnt(10)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
   "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
   "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
   "s_waitcnt lgkmcnt(15)\n" \
   "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
   "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
   "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
   "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
   "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
   "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
   "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
   "s_waitcnt lgkmcnt(6)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "s_waitcnt lgkmcnt(5)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
   "s_waitcnt lgkmcnt(4)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
   "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "s_waitcnt lgkmcnt(2)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
   "s_waitcnt vmcnt(0)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
   "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
   "s_waitcnt lgkmcnt(8)\n" \
   "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "s_waitcnt lgkmcnt(7)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
   "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
   "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
   "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
-  "s_waitcnt lgkmcnt(6)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "s_waitcnt lgkmcnt(10)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
   "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
   "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
   "s_waitcnt lgkmcnt(15)\n" \
   "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
   "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
   "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
   "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
   "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
   "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
   "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
   "s_waitcnt lgkmcnt(6)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "s_waitcnt lgkmcnt(5)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
   "s_waitcnt lgkmcnt(4)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
   "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "s_waitcnt lgkmcnt(2)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
   "s_waitcnt lgkmcnt(1)\n" \
   "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
   "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
   "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
   "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
   "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
   "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
   "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
   "s_barrier\n" \
   "s_cmp_eq_u32 %[has_next], 0\n" \
   "s_cbranch_scc1 L_w4_end_%=\n" \
@@ -13571,705 +14063,733 @@
   "s_waitcnt vmcnt(29)\n" \
   "L_w4_go_%=:\n" \
   "s_barrier\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
   "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
   "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
-  "s_waitcnt lgkmcnt(6)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
   "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "s_waitcnt lgkmcnt(10)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
+  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
   "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
   "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], 0\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], 0\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], 0\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], 0\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], 0\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], 0\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], 0\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], 0\n" \
   "buffer_load_dwordx4 %[vo6], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
   "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
   "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "buffer_load_dwordx4 %[vo14], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
   "s_waitcnt vmcnt(15)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
   "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
   "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
   "s_cmp_eq_u32 %[iter], 0\n" \
   "s_cbranch_scc1 L_w4_after_%=\n" \
   "L_w4_loop_%=:\n" \
-  "s_waitcnt lgkmcnt(6)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "s_waitcnt lgkmcnt(10)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
   "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
   "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
   "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
   "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
   "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
   "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
   "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
   "buffer_load_dwordx4 %[vo6], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
   "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
   "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "buffer_load_dwordx4 %[vo14], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
   "s_waitcnt vmcnt(15)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
   "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
   "s_sub_u32 %[iter], %[iter], 1\n" \
   "s_cmp_lg_u32 %[iter], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
   "s_cbranch_scc1 L_w4_loop_%=\n" \
   "L_w4_after_%=:\n" \
-  "s_waitcnt lgkmcnt(6)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "s_waitcnt lgkmcnt(10)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
   "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
   "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
   "s_waitcnt lgkmcnt(15)\n" \
   "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
   "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
   "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
   "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
   "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
   "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
   "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
   "s_waitcnt lgkmcnt(6)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "s_waitcnt lgkmcnt(5)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
   "s_waitcnt lgkmcnt(4)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
   "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "s_waitcnt lgkmcnt(2)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
   "s_waitcnt vmcnt(0)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
   "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
   "s_waitcnt lgkmcnt(8)\n" \
   "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "s_waitcnt lgkmcnt(7)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
   "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
   "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
   "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
-  "s_waitcnt lgkmcnt(6)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "s_waitcnt lgkmcnt(10)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
   "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
   "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
   "s_waitcnt lgkmcnt(15)\n" \
   "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
   "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
   "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
   "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
   "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
   "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
   "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
   "s_waitcnt lgkmcnt(6)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "s_waitcnt lgkmcnt(5)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
   "s_waitcnt lgkmcnt(4)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
   "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "s_waitcnt lgkmcnt(2)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
   "s_waitcnt lgkmcnt(1)\n" \
   "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
   "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
   "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
   "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
   "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
   "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
   "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
   "s_barrier\n" \
   "s_cmp_eq_u32 %[has_next], 0\n" \
   "s_cbranch_scc1 L_w4_end_%=\n" \
@@ -14471,705 +14991,733 @@
   "s_waitcnt vmcnt(45)\n" \
   "L_w4_go_%=:\n" \
   "s_barrier\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
   "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
   "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
-  "s_waitcnt lgkmcnt(6)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
   "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "s_waitcnt lgkmcnt(10)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
+  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
   "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
   "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], 0\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], 0\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], 0\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], 0\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], 0\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], 0\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], 0\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], 0\n" \
   "buffer_load_dwordx4 %[vo6], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
   "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
   "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "buffer_load_dwordx4 %[vo14], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
   "s_waitcnt vmcnt(15)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
   "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
   "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
   "s_cmp_eq_u32 %[iter], 0\n" \
   "s_cbranch_scc1 L_w4_after_%=\n" \
   "L_w4_loop_%=:\n" \
-  "s_waitcnt lgkmcnt(6)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "s_waitcnt lgkmcnt(10)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
   "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
   "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
   "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
   "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
   "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
   "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
   "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
   "buffer_load_dwordx4 %[vo6], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
   "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
   "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "buffer_load_dwordx4 %[vo14], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
   "s_waitcnt vmcnt(15)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
   "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
   "s_sub_u32 %[iter], %[iter], 1\n" \
   "s_cmp_lg_u32 %[iter], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
   "s_cbranch_scc1 L_w4_loop_%=\n" \
   "L_w4_after_%=:\n" \
-  "s_waitcnt lgkmcnt(6)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "s_waitcnt lgkmcnt(10)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
   "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
   "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
   "s_waitcnt lgkmcnt(15)\n" \
   "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
   "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
   "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
   "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
   "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
   "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
   "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
   "s_waitcnt lgkmcnt(6)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "s_waitcnt lgkmcnt(5)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
   "s_waitcnt lgkmcnt(4)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
   "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "s_waitcnt lgkmcnt(2)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
   "s_waitcnt vmcnt(0)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
   "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
   "s_waitcnt lgkmcnt(8)\n" \
   "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "s_waitcnt lgkmcnt(7)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
   "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
   "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
   "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
-  "s_waitcnt lgkmcnt(6)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "s_waitcnt lgkmcnt(10)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
   "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
   "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
   "s_waitcnt lgkmcnt(15)\n" \
   "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
   "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
   "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
   "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
   "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
   "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
   "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
   "s_waitcnt lgkmcnt(6)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "s_waitcnt lgkmcnt(5)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
   "s_waitcnt lgkmcnt(4)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
   "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "s_waitcnt lgkmcnt(2)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
   "s_waitcnt lgkmcnt(1)\n" \
   "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
   "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
   "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
   "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
   "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
   "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
   "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
   "s_barrier\n" \
   "s_cmp_eq_u32 %[has_next], 0\n" \
   "s_cbranch_scc1 L_w4_end_%=\n" \
@@ -15371,705 +15919,733 @@
   "s_waitcnt vmcnt(31)\n" \
   "L_w4_go_%=:\n" \
   "s_barrier\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
   "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
   "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
-  "s_waitcnt lgkmcnt(6)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
   "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "s_waitcnt lgkmcnt(10)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
+  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
   "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
   "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], 0\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], 0\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], 0\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], 0\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], 0\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], 0\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], 0\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], 0\n" \
   "buffer_load_dwordx4 %[vo6], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
   "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
   "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "buffer_load_dwordx4 %[vo14], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
   "s_waitcnt vmcnt(15)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
   "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
   "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
   "s_cmp_eq_u32 %[iter], 0\n" \
   "s_cbranch_scc1 L_w4_after_%=\n" \
   "L_w4_loop_%=:\n" \
-  "s_waitcnt lgkmcnt(6)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "s_waitcnt lgkmcnt(10)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
   "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
   "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
-  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
-  "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
   "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
   "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
   "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
   "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
-  "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
   "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
   "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
   "buffer_load_dwordx4 %[vo6], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
   "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
-  "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
+  "s_add_u32 m0, m0, 0x1000\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
   "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "buffer_load_dwordx4 %[vo14], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
   "s_waitcnt vmcnt(15)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
   "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
   "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
   "s_sub_u32 %[iter], %[iter], 1\n" \
   "s_cmp_lg_u32 %[iter], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
   "s_cbranch_scc1 L_w4_loop_%=\n" \
   "L_w4_after_%=:\n" \
-  "s_waitcnt lgkmcnt(6)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "s_waitcnt lgkmcnt(10)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
   "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
   "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
   "s_waitcnt lgkmcnt(15)\n" \
   "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
   "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
   "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
   "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
   "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
   "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
   "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
   "s_waitcnt lgkmcnt(6)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "s_waitcnt lgkmcnt(5)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
   "s_waitcnt lgkmcnt(4)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
   "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "s_waitcnt lgkmcnt(2)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
   "s_waitcnt vmcnt(0)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
   "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
   "s_waitcnt lgkmcnt(8)\n" \
   "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "s_waitcnt lgkmcnt(7)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
   "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
   "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
   "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
-  "s_waitcnt lgkmcnt(6)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "s_waitcnt lgkmcnt(10)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
   "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
   "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
   "s_waitcnt lgkmcnt(15)\n" \
   "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
   "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
   "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
   "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
   "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
   "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
   "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
   "s_waitcnt lgkmcnt(6)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
   "s_waitcnt lgkmcnt(5)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
   "s_waitcnt lgkmcnt(4)\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
   "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "s_waitcnt lgkmcnt(2)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
   "s_waitcnt lgkmcnt(1)\n" \
   "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
   "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
   "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
   "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
   "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
   "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
   "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
   "s_barrier\n" \
   "s_cmp_eq_u32 %[has_next], 0\n" \
   "s_cbranch_scc1 L_w4_end_%=\n" \

@@ -30,7 +30,7 @@ Schedule of iteration t (MFMA slot m = 0..127; H0 = k-half 0 of tile t, H1 = k-h
 Lower tiles (128, 160, 192, 224 rows: 64, 80, 96, 112 MFMAs per K-tile, 12 - 15 pieces and 12 - 15 reads per half) have the
 same phases at their own slots (SCHED_H, SCHED_160, SCHED_192, SCHED_224).  The K offset of the DMA runs through an operand: it starts
 where the caller says and wraps to 0 at %[kend], so that tiles may walk K from different steps.
-MFMA order: H0 = (i, j) row-major over FA0[i] x FB0[j]; H1 = the same over FA1 x FB1.
+MFMA order: H0 = order() over FA0[i] x FB0[j]; H1 = the same over FA1 x FB1.
 lgkmcnt waits are derived here from the in-order LDS return queue (each MFMA waits only
 for the fragments it reads).  The last two iterations are peeled: t = nk-2 issues no DMA
 (B2 waits vmcnt(0)), t = nk-1 issues neither DMA nor next-tile reads.
@@ -141,13 +141,47 @@ class Stream:
         self.queue = []
 
 
+def order(sc: Sched):
+    """(i, j) of a k-half's MFMAs: strips of two A fragments (an odd one alone, first), the columns there and back, the
+    strip's two in turn up and down, so that an MFMA shares a fragment with the one before it and mostly another with the
+    one before that.  The last strip walks its columns upwards: FB1 is read again in that order.
+
+    Sustained products are bound by power, and operands that stay take less of it: registers only, all CUs, row by row
+    2101 TFLOP/s, row snake 2130, blocks of 2 x 2 2150, of 4 x 4 2128, so (and along a Hilbert curve) 2166."""
+    strips = [[0]] if sc.nfa % 2 else []
+    strips += [[i, i + 1] for i in range(sc.nfa % 2, sc.nfa, 2)]
+    out = []
+    for n, strip in enumerate(strips):
+        cols = range(NFB) if (len(strips) - 1 - n) % 2 == 0 else range(NFB - 1, -1, -1)
+        for c, j in enumerate(cols):
+            out += [(i, j) for i in (strip if c % 2 == 0 else strip[::-1])]
+    return out
+
+
 def reads_k1(sc: Sched):
-    """ds_reads of the k-half-1 fragments (FB1 then FA1) of the current tile."""
+    """ds_reads of the k-half-1 fragments (FB1 then FA1) of the current tile, in the order of their last readers."""
     return [(("fb1_", j), "rB1", j * 2048) for j in range(NFB)] + [(("fa1_", i), "rA1", i * 2048) for i in range(sc.nfa)]
 
 
 def reads_k0(sc: Sched):
-    return [(("fb0_", j), "rB0", j * 2048) for j in range(NFB)] + [(("fa0_", i), "rA0", i * 2048) for i in range(sc.nfa)]
+    """ds_reads of the k-half-0 fragments, in the order of their first readers."""
+    seq = []
+    for i, j in order(sc):
+        seq += [f for f in (("fb0_", j), ("fa0_", i)) if f not in seq]
+    return [(f, "rB0" if f[0] == "fb0_" else "rA0", f[1] * 2048) for f in seq]
+
+
+def check_reuse(sc: Sched):
+    """A fragment is read again at least eight MFMAs behind its last reader."""
+    half = sc.nmma // 2
+    last = {}
+    for m, (i, j) in enumerate(order(sc)):
+        for f in (("fa0_", i), ("fb0_", j)):
+            last[f] = m
+        for f in (("fa1_", i), ("fb1_", j)):
+            last[f] = half + m - sc.nmma  # of the K-tile before
+    for slots, ops in ((sc.rd0, reads_k0(sc)), (sc.rd1, reads_k1(sc))):
+        assert all(m - last[op[0]] >= 8 for m, op in zip(slots, ops))
 
 
 def body(s: Stream, sc: Sched, kind: str, first: bool = False):
@@ -156,6 +190,8 @@ def body(s: Stream, sc: Sched, kind: str, first: bool = False):
     dma = kind == "steady"
     nxt = kind != "last"
     NM = sc.nmma
+    check_reuse(sc)
+    seq = order(sc)
     slots: dict[int, list] = {m: [] for m in range(NM + 1)}
     for m, op in zip(sc.rd1, reads_k1(sc)):
         slots[m].append(("read", op))
@@ -198,7 +234,7 @@ def body(s: Stream, sc: Sched, kind: str, first: bool = False):
         if m == NM:
             break
         h, mm = divmod(m, NM // 2)
-        i, j = divmod(mm, NFB)
+        i, j = seq[mm]
         a, b = (("fa0_", i), ("fb0_", j)) if h == 0 else (("fa1_", i), ("fb1_", j))
         s.need(a, b)
         s.emit(mfma(NFB * i + j, frag(*a), frag(*b), zero_c=first and h == 0))
