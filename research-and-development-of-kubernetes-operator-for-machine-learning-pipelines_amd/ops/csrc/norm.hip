@@ -132,21 +132,24 @@ __global__ void __launch_bounds__(256) rmsnorm_wave_kernel(uint16_t* __restrict_
   }
 }
 
-// fewer rows: the block form's 8-wave fan-out per row wins (at batch 1 the wave form measured
-// 345 vs 351 tok/s, scripts/history INDEX r4_norm1)
-constexpr int kWaveRowsMinM = 256;
+// Rows from which a wave takes a row of H, against the block form's 8 waves (add + norm behind a producer, us, block / wave).
+// Narrow rows: from 256 on (512: 2.5 / 1.75 at 640 rows, 6.9 / 4.3 at 6000; 1024: 3.3 / 2.8, 12.5 / 11.2).  2048: the block
+// form until the pass is bound by memory (256 rows 2.1 / 3.0, 890 3.4 / 4.8, 2300 6.6 / 10.0, 4000 12.1 / 11.8).  4096: where
+// its rows no longer fit the chip at once (256 rows 3.5 / 4.7, 500 5.4 / 5.9, 640 6.5 / 6.7, 1000 8.9 / 8.4, 1600 13.0 / 11.9,
+// 6000 28.9 / 29.4).  8192: never (a lane's 32 loads are 128 registers: 256 rows 5.4 / 8.0, 890 12.6 / 13.3, 2300 23.1 / 25.2,
+// 8000 100 / 107).  At one row the wave form made a decode step 2 % slower.
+static int wave_rows(int H) { return H <= 1024 ? 256 : H == 2048 ? 3200 : H == 4096 ? 700 : 1 << 30; }
 
 template <bool ADD>
 static bool dispatch_wave(uint16_t* out, uint16_t* residual, const uint16_t* x, const uint16_t* w,
                           float eps, int M, int H, hipStream_t st) {
-  if (M < kWaveRowsMinM || H % 512) return false;
+  if (H % 512 || M < wave_rows(H)) return false;
   const int g = cdiv(M, 4);
   switch (H / 512) {
     case 1: rmsnorm_wave_kernel<1, ADD><<<g, 256, 0, st>>>(out, residual, x, w, eps, M, H); return true;
     case 2: rmsnorm_wave_kernel<2, ADD><<<g, 256, 0, st>>>(out, residual, x, w, eps, M, H); return true;
     case 4: rmsnorm_wave_kernel<4, ADD><<<g, 256, 0, st>>>(out, residual, x, w, eps, M, H); return true;
     case 8: rmsnorm_wave_kernel<8, ADD><<<g, 256, 0, st>>>(out, residual, x, w, eps, M, H); return true;
-    case 16: rmsnorm_wave_kernel<16, ADD><<<g, 256, 0, st>>>(out, residual, x, w, eps, M, H); return true;
     default: return false;
   }
 }
