@@ -501,10 +501,10 @@ def qkv_rope_cache(x, w, positions, cos_sin, slots, k_cache, v_cache, n_q_heads:
 NORM_CHAIN = "1"
 
 
-# The decode (M <= 4) form of the chain runs on the GEMV (gemv.hip EPI_RES / PRO_RS): O and down
-# add into the residual in place, QKV and gate_up take each row's factor from the residual
-# chunks they stream, so a layer has no add + RMSNorm launch.  False keeps the decode norms (the
-# GPU tests' A/B).
+# The decode form of the chain (``decode_chain_max_m`` rows) runs on the GEMV (gemv.hip EPI_RES / PRO_RS), the
+# weight-streaming MFMA kernel (gemm_ws.hip) and, gate_up above 8 rows, the weight stream (gemm_mid.hip): O and down add into
+# the residual in place, QKV and gate_up take each row's factor from the residual chunks they stream, so a layer has no add
+# + RMSNorm launch.  False keeps the decode norms (the GPU tests' A/B).
 GEMV_CHAIN = True
 GEMV_CHAIN_MAX_M = 4  # = gemv.hip gemv_chain_max_m (the GEMV form; the torch reference's decode form)
 
@@ -523,7 +523,7 @@ def norm_chain_ok(M: int, H: int, shapes, device=None, epis=None, like: int = 0)
     quad of lanes) and every (N, K) GEMM of the chain on the four-wave kernel, with the band
     tickets' scratch reserved on ``device`` and one ticket per 256-row band (w4_chain_ok checks
     everything launch_w4_chain does, so the chain is decided once per forward and never refused
-    after a residual was updated in place).  At M <= 4 every GEMM must take the GEMV form
+    after a residual was updated in place).  Up to ``decode_chain_max_m`` rows every GEMM must take the decode form
     instead (``epis``: each shape's epilogue, default plain).  ``like``: the rows of a larger step
     in whose place this one runs; where that one has the chain, this one has it as soon as the
     four-wave kernel can run its products, whichever kernel is the faster (``any_tile`` below)."""
