@@ -109,812 +109,842 @@
   "s_waitcnt vmcnt(48)\n" \
   "L_w4_go_%=:\n" \
   "s_barrier\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
-  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
-  "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
   "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
   "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
   "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
   "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
   "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
   "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
   "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
   "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], 0\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
+  "s_waitcnt lgkmcnt(8)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb0_0], %[fa0_7], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb0_1], %[fa0_7], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
   "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb0_2], %[fa0_7], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb0_3], %[fa0_7], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
   "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb0_6], %[fa0_7], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb0_7], %[fa0_7], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "buffer_load_dwordx4 %[vo6], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
   "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
   "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
   "buffer_load_dwordx4 %[vo14], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb0_0], %[fa0_7], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb1_0], %[fa1_7], a[224:227]\n" \
   "buffer_load_dwordx4 %[vo15], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb0_1], %[fa0_7], 0\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb1_1], %[fa1_7], a[228:231]\n" \
   "s_waitcnt vmcnt(16)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], 0\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb1_0], %[fa1_7], a[224:227]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb1_1], %[fa1_7], a[228:231]\n" \
   "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], 0\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
   "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb0_2], %[fa0_7], 0\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb1_2], %[fa1_7], a[232:235]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb0_3], %[fa0_7], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb1_3], %[fa1_7], a[236:239]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], 0\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], 0\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb1_4], %[fa1_7], a[240:243]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb1_5], %[fa1_7], a[244:247]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], 0\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
-  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb0_6], %[fa0_7], 0\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb1_6], %[fa1_7], a[248:251]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb0_7], %[fa0_7], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb1_7], %[fa1_7], a[252:255]\n" \
-  "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], 0\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
   "s_cmp_eq_u32 %[iter], 0\n" \
   "s_cbranch_scc1 L_w4_after_%=\n" \
   "L_w4_loop_%=:\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
   "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
   "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
   "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
   "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
   "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
   "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "s_waitcnt lgkmcnt(8)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb0_0], %[fa0_7], a[224:227]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb0_1], %[fa0_7], a[228:231]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
   "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb0_2], %[fa0_7], a[232:235]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb0_3], %[fa0_7], a[236:239]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], a[240:243]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], a[244:247]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
   "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb0_6], %[fa0_7], a[248:251]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb0_7], %[fa0_7], a[252:255]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "buffer_load_dwordx4 %[vo6], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
   "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
   "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
   "buffer_load_dwordx4 %[vo14], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb0_0], %[fa0_7], a[224:227]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb1_0], %[fa1_7], a[224:227]\n" \
   "buffer_load_dwordx4 %[vo15], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb0_1], %[fa0_7], a[228:231]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb1_1], %[fa1_7], a[228:231]\n" \
   "s_waitcnt vmcnt(16)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb1_0], %[fa1_7], a[224:227]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb1_1], %[fa1_7], a[228:231]\n" \
   "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
   "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb0_2], %[fa0_7], a[232:235]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb1_2], %[fa1_7], a[232:235]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb0_3], %[fa0_7], a[236:239]\n" \
   "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb1_3], %[fa1_7], a[236:239]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
   "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], a[240:243]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb1_4], %[fa1_7], a[240:243]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], a[244:247]\n" \
   "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb1_5], %[fa1_7], a[244:247]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
-  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb0_6], %[fa0_7], a[248:251]\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb1_6], %[fa1_7], a[248:251]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb0_7], %[fa0_7], a[252:255]\n" \
   "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb1_7], %[fa1_7], a[252:255]\n" \
-  "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "s_sub_u32 %[iter], %[iter], 1\n" \
   "s_cmp_lg_u32 %[iter], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
   "s_cbranch_scc1 L_w4_loop_%=\n" \
   "L_w4_after_%=:\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb0_0], %[fa0_7], a[224:227]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb0_1], %[fa0_7], a[228:231]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb0_2], %[fa0_7], a[232:235]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb0_3], %[fa0_7], a[236:239]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], a[240:243]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], a[244:247]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb0_6], %[fa0_7], a[248:251]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb0_7], %[fa0_7], a[252:255]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
-  "s_waitcnt lgkmcnt(7)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "s_waitcnt lgkmcnt(6)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "s_waitcnt lgkmcnt(5)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "s_waitcnt lgkmcnt(2)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "s_waitcnt lgkmcnt(8)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "s_waitcnt lgkmcnt(7)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "s_waitcnt lgkmcnt(6)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "s_waitcnt lgkmcnt(5)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
+  "s_waitcnt lgkmcnt(4)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "s_waitcnt lgkmcnt(3)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
+  "s_waitcnt lgkmcnt(2)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
+  "s_waitcnt lgkmcnt(1)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb0_0], %[fa0_7], a[224:227]\n" \
+  "s_waitcnt lgkmcnt(0)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb1_0], %[fa1_7], a[224:227]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb0_1], %[fa0_7], a[228:231]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb1_1], %[fa1_7], a[228:231]\n" \
   "s_waitcnt vmcnt(0)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "s_waitcnt lgkmcnt(7)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "s_waitcnt lgkmcnt(7)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb1_0], %[fa1_7], a[224:227]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb1_1], %[fa1_7], a[228:231]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb1_2], %[fa1_7], a[232:235]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb1_3], %[fa1_7], a[236:239]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb1_4], %[fa1_7], a[240:243]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb1_5], %[fa1_7], a[244:247]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
-  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb1_6], %[fa1_7], a[248:251]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb1_7], %[fa1_7], a[252:255]\n" \
-  "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb0_0], %[fa0_7], a[224:227]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb0_1], %[fa0_7], a[228:231]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb0_2], %[fa0_7], a[232:235]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb0_3], %[fa0_7], a[236:239]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], a[240:243]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], a[244:247]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb0_2], %[fa0_7], a[232:235]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb1_2], %[fa1_7], a[232:235]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb0_3], %[fa0_7], a[236:239]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb1_3], %[fa1_7], a[236:239]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], a[240:243]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb1_4], %[fa1_7], a[240:243]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], a[244:247]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb1_5], %[fa1_7], a[244:247]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb0_6], %[fa0_7], a[248:251]\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb1_6], %[fa1_7], a[248:251]\n" \
   "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb0_7], %[fa0_7], a[252:255]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb1_7], %[fa1_7], a[252:255]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
-  "s_waitcnt lgkmcnt(7)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "s_waitcnt lgkmcnt(6)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "s_waitcnt lgkmcnt(5)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "s_waitcnt lgkmcnt(2)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "s_waitcnt lgkmcnt(8)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "s_waitcnt lgkmcnt(7)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "s_waitcnt lgkmcnt(6)\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "s_waitcnt lgkmcnt(1)\n" \
+  "s_waitcnt lgkmcnt(5)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
+  "s_waitcnt lgkmcnt(4)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "s_waitcnt lgkmcnt(3)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
+  "s_waitcnt lgkmcnt(2)\n" \
   "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
+  "s_waitcnt lgkmcnt(1)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb0_0], %[fa0_7], a[224:227]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb1_0], %[fa1_7], a[224:227]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb0_1], %[fa0_7], a[228:231]\n" \
   "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb1_1], %[fa1_7], a[228:231]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
   "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
   "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb0_2], %[fa0_7], a[232:235]\n" \
   "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb1_2], %[fa1_7], a[232:235]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb0_3], %[fa0_7], a[236:239]\n" \
   "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb1_3], %[fa1_7], a[236:239]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
   "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
   "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], a[240:243]\n" \
   "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb1_4], %[fa1_7], a[240:243]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], a[244:247]\n" \
   "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb1_5], %[fa1_7], a[244:247]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
   "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb0_6], %[fa0_7], a[248:251]\n" \
   "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb1_6], %[fa1_7], a[248:251]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb0_7], %[fa0_7], a[252:255]\n" \
   "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb1_7], %[fa1_7], a[252:255]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
   "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
   "s_barrier\n" \
   "s_cmp_eq_u32 %[has_next], 0\n" \
@@ -1129,812 +1159,842 @@
   "s_waitcnt vmcnt(32)\n" \
   "L_w4_go_%=:\n" \
   "s_barrier\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
-  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
-  "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
   "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
   "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
   "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
   "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
   "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
   "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
   "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
   "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], 0\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
+  "s_waitcnt lgkmcnt(8)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb0_0], %[fa0_7], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb0_1], %[fa0_7], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
   "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb0_2], %[fa0_7], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb0_3], %[fa0_7], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
   "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb0_6], %[fa0_7], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb0_7], %[fa0_7], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "buffer_load_dwordx4 %[vo6], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
   "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
   "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
   "buffer_load_dwordx4 %[vo14], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb0_0], %[fa0_7], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb1_0], %[fa1_7], a[224:227]\n" \
   "buffer_load_dwordx4 %[vo15], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb0_1], %[fa0_7], 0\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb1_1], %[fa1_7], a[228:231]\n" \
   "s_waitcnt vmcnt(16)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], 0\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb1_0], %[fa1_7], a[224:227]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb1_1], %[fa1_7], a[228:231]\n" \
   "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], 0\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
   "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb0_2], %[fa0_7], 0\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb1_2], %[fa1_7], a[232:235]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb0_3], %[fa0_7], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb1_3], %[fa1_7], a[236:239]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], 0\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], 0\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb1_4], %[fa1_7], a[240:243]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb1_5], %[fa1_7], a[244:247]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], 0\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
-  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb0_6], %[fa0_7], 0\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb1_6], %[fa1_7], a[248:251]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb0_7], %[fa0_7], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb1_7], %[fa1_7], a[252:255]\n" \
-  "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], 0\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
   "s_cmp_eq_u32 %[iter], 0\n" \
   "s_cbranch_scc1 L_w4_after_%=\n" \
   "L_w4_loop_%=:\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
   "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
   "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
   "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
   "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
   "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
   "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "s_waitcnt lgkmcnt(8)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb0_0], %[fa0_7], a[224:227]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb0_1], %[fa0_7], a[228:231]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
   "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb0_2], %[fa0_7], a[232:235]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb0_3], %[fa0_7], a[236:239]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], a[240:243]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], a[244:247]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
   "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb0_6], %[fa0_7], a[248:251]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb0_7], %[fa0_7], a[252:255]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "buffer_load_dwordx4 %[vo6], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
   "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
   "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
   "buffer_load_dwordx4 %[vo14], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb0_0], %[fa0_7], a[224:227]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb1_0], %[fa1_7], a[224:227]\n" \
   "buffer_load_dwordx4 %[vo15], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb0_1], %[fa0_7], a[228:231]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb1_1], %[fa1_7], a[228:231]\n" \
   "s_waitcnt vmcnt(16)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb1_0], %[fa1_7], a[224:227]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb1_1], %[fa1_7], a[228:231]\n" \
   "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
   "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb0_2], %[fa0_7], a[232:235]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb1_2], %[fa1_7], a[232:235]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb0_3], %[fa0_7], a[236:239]\n" \
   "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb1_3], %[fa1_7], a[236:239]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
   "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], a[240:243]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb1_4], %[fa1_7], a[240:243]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], a[244:247]\n" \
   "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb1_5], %[fa1_7], a[244:247]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
-  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb0_6], %[fa0_7], a[248:251]\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb1_6], %[fa1_7], a[248:251]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb0_7], %[fa0_7], a[252:255]\n" \
   "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb1_7], %[fa1_7], a[252:255]\n" \
-  "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "s_sub_u32 %[iter], %[iter], 1\n" \
   "s_cmp_lg_u32 %[iter], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
   "s_cbranch_scc1 L_w4_loop_%=\n" \
   "L_w4_after_%=:\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb0_0], %[fa0_7], a[224:227]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb0_1], %[fa0_7], a[228:231]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb0_2], %[fa0_7], a[232:235]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb0_3], %[fa0_7], a[236:239]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], a[240:243]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], a[244:247]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb0_6], %[fa0_7], a[248:251]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb0_7], %[fa0_7], a[252:255]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
-  "s_waitcnt lgkmcnt(7)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "s_waitcnt lgkmcnt(6)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "s_waitcnt lgkmcnt(5)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "s_waitcnt lgkmcnt(2)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "s_waitcnt lgkmcnt(8)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "s_waitcnt lgkmcnt(7)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "s_waitcnt lgkmcnt(6)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "s_waitcnt lgkmcnt(5)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
+  "s_waitcnt lgkmcnt(4)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "s_waitcnt lgkmcnt(3)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
+  "s_waitcnt lgkmcnt(2)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
+  "s_waitcnt lgkmcnt(1)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb0_0], %[fa0_7], a[224:227]\n" \
+  "s_waitcnt lgkmcnt(0)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb1_0], %[fa1_7], a[224:227]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb0_1], %[fa0_7], a[228:231]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb1_1], %[fa1_7], a[228:231]\n" \
   "s_waitcnt vmcnt(0)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "s_waitcnt lgkmcnt(7)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "s_waitcnt lgkmcnt(7)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb1_0], %[fa1_7], a[224:227]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb1_1], %[fa1_7], a[228:231]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb1_2], %[fa1_7], a[232:235]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb1_3], %[fa1_7], a[236:239]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb1_4], %[fa1_7], a[240:243]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb1_5], %[fa1_7], a[244:247]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
-  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb1_6], %[fa1_7], a[248:251]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb1_7], %[fa1_7], a[252:255]\n" \
-  "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb0_0], %[fa0_7], a[224:227]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb0_1], %[fa0_7], a[228:231]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb0_2], %[fa0_7], a[232:235]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb0_3], %[fa0_7], a[236:239]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], a[240:243]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], a[244:247]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb0_2], %[fa0_7], a[232:235]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb1_2], %[fa1_7], a[232:235]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb0_3], %[fa0_7], a[236:239]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb1_3], %[fa1_7], a[236:239]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], a[240:243]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb1_4], %[fa1_7], a[240:243]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], a[244:247]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb1_5], %[fa1_7], a[244:247]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb0_6], %[fa0_7], a[248:251]\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb1_6], %[fa1_7], a[248:251]\n" \
   "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb0_7], %[fa0_7], a[252:255]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb1_7], %[fa1_7], a[252:255]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
-  "s_waitcnt lgkmcnt(7)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "s_waitcnt lgkmcnt(6)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "s_waitcnt lgkmcnt(5)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "s_waitcnt lgkmcnt(2)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "s_waitcnt lgkmcnt(8)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "s_waitcnt lgkmcnt(7)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "s_waitcnt lgkmcnt(6)\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "s_waitcnt lgkmcnt(1)\n" \
+  "s_waitcnt lgkmcnt(5)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
+  "s_waitcnt lgkmcnt(4)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "s_waitcnt lgkmcnt(3)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
+  "s_waitcnt lgkmcnt(2)\n" \
   "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
+  "s_waitcnt lgkmcnt(1)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb0_0], %[fa0_7], a[224:227]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb1_0], %[fa1_7], a[224:227]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb0_1], %[fa0_7], a[228:231]\n" \
   "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb1_1], %[fa1_7], a[228:231]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
   "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
   "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb0_2], %[fa0_7], a[232:235]\n" \
   "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb1_2], %[fa1_7], a[232:235]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb0_3], %[fa0_7], a[236:239]\n" \
   "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb1_3], %[fa1_7], a[236:239]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
   "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
   "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], a[240:243]\n" \
   "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb1_4], %[fa1_7], a[240:243]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], a[244:247]\n" \
   "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb1_5], %[fa1_7], a[244:247]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
   "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb0_6], %[fa0_7], a[248:251]\n" \
   "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb1_6], %[fa1_7], a[248:251]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb0_7], %[fa0_7], a[252:255]\n" \
   "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb1_7], %[fa1_7], a[252:255]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
   "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
   "s_barrier\n" \
   "s_cmp_eq_u32 %[has_next], 0\n" \
@@ -2149,812 +2209,842 @@
   "s_waitcnt vmcnt(50)\n" \
   "L_w4_go_%=:\n" \
   "s_barrier\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
-  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
-  "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
   "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
   "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
   "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
   "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
   "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
   "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
   "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
   "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], 0\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
+  "s_waitcnt lgkmcnt(8)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb0_0], %[fa0_7], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb0_1], %[fa0_7], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
   "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb0_2], %[fa0_7], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb0_3], %[fa0_7], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
   "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb0_6], %[fa0_7], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb0_7], %[fa0_7], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "buffer_load_dwordx4 %[vo6], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
   "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
   "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
   "buffer_load_dwordx4 %[vo14], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb0_0], %[fa0_7], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb1_0], %[fa1_7], a[224:227]\n" \
   "buffer_load_dwordx4 %[vo15], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb0_1], %[fa0_7], 0\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb1_1], %[fa1_7], a[228:231]\n" \
   "s_waitcnt vmcnt(16)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], 0\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb1_0], %[fa1_7], a[224:227]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb1_1], %[fa1_7], a[228:231]\n" \
   "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], 0\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
   "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb0_2], %[fa0_7], 0\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb1_2], %[fa1_7], a[232:235]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb0_3], %[fa0_7], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb1_3], %[fa1_7], a[236:239]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], 0\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], 0\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb1_4], %[fa1_7], a[240:243]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb1_5], %[fa1_7], a[244:247]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], 0\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
-  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb0_6], %[fa0_7], 0\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb1_6], %[fa1_7], a[248:251]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb0_7], %[fa0_7], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb1_7], %[fa1_7], a[252:255]\n" \
-  "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], 0\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
   "s_cmp_eq_u32 %[iter], 0\n" \
   "s_cbranch_scc1 L_w4_after_%=\n" \
   "L_w4_loop_%=:\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
   "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
   "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
   "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
   "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
   "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
   "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "s_waitcnt lgkmcnt(8)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb0_0], %[fa0_7], a[224:227]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb0_1], %[fa0_7], a[228:231]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
   "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb0_2], %[fa0_7], a[232:235]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb0_3], %[fa0_7], a[236:239]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], a[240:243]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], a[244:247]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
   "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb0_6], %[fa0_7], a[248:251]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb0_7], %[fa0_7], a[252:255]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "buffer_load_dwordx4 %[vo6], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
   "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
   "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
   "buffer_load_dwordx4 %[vo14], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb0_0], %[fa0_7], a[224:227]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb1_0], %[fa1_7], a[224:227]\n" \
   "buffer_load_dwordx4 %[vo15], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb0_1], %[fa0_7], a[228:231]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb1_1], %[fa1_7], a[228:231]\n" \
   "s_waitcnt vmcnt(16)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb1_0], %[fa1_7], a[224:227]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb1_1], %[fa1_7], a[228:231]\n" \
   "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
   "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb0_2], %[fa0_7], a[232:235]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb1_2], %[fa1_7], a[232:235]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb0_3], %[fa0_7], a[236:239]\n" \
   "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb1_3], %[fa1_7], a[236:239]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
   "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], a[240:243]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb1_4], %[fa1_7], a[240:243]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], a[244:247]\n" \
   "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb1_5], %[fa1_7], a[244:247]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
-  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb0_6], %[fa0_7], a[248:251]\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb1_6], %[fa1_7], a[248:251]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb0_7], %[fa0_7], a[252:255]\n" \
   "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb1_7], %[fa1_7], a[252:255]\n" \
-  "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "s_sub_u32 %[iter], %[iter], 1\n" \
   "s_cmp_lg_u32 %[iter], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
   "s_cbranch_scc1 L_w4_loop_%=\n" \
   "L_w4_after_%=:\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb0_0], %[fa0_7], a[224:227]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb0_1], %[fa0_7], a[228:231]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb0_2], %[fa0_7], a[232:235]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb0_3], %[fa0_7], a[236:239]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], a[240:243]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], a[244:247]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb0_6], %[fa0_7], a[248:251]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb0_7], %[fa0_7], a[252:255]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
-  "s_waitcnt lgkmcnt(7)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "s_waitcnt lgkmcnt(6)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "s_waitcnt lgkmcnt(5)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "s_waitcnt lgkmcnt(2)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "s_waitcnt lgkmcnt(8)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "s_waitcnt lgkmcnt(7)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "s_waitcnt lgkmcnt(6)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "s_waitcnt lgkmcnt(5)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
+  "s_waitcnt lgkmcnt(4)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "s_waitcnt lgkmcnt(3)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
+  "s_waitcnt lgkmcnt(2)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
+  "s_waitcnt lgkmcnt(1)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb0_0], %[fa0_7], a[224:227]\n" \
+  "s_waitcnt lgkmcnt(0)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb1_0], %[fa1_7], a[224:227]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb0_1], %[fa0_7], a[228:231]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb1_1], %[fa1_7], a[228:231]\n" \
   "s_waitcnt vmcnt(0)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "s_waitcnt lgkmcnt(7)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "s_waitcnt lgkmcnt(7)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb1_0], %[fa1_7], a[224:227]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb1_1], %[fa1_7], a[228:231]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb1_2], %[fa1_7], a[232:235]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb1_3], %[fa1_7], a[236:239]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb1_4], %[fa1_7], a[240:243]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb1_5], %[fa1_7], a[244:247]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
-  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb1_6], %[fa1_7], a[248:251]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb1_7], %[fa1_7], a[252:255]\n" \
-  "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb0_0], %[fa0_7], a[224:227]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb0_1], %[fa0_7], a[228:231]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb0_2], %[fa0_7], a[232:235]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb0_3], %[fa0_7], a[236:239]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], a[240:243]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], a[244:247]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb0_2], %[fa0_7], a[232:235]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb1_2], %[fa1_7], a[232:235]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb0_3], %[fa0_7], a[236:239]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb1_3], %[fa1_7], a[236:239]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], a[240:243]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb1_4], %[fa1_7], a[240:243]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], a[244:247]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb1_5], %[fa1_7], a[244:247]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb0_6], %[fa0_7], a[248:251]\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb1_6], %[fa1_7], a[248:251]\n" \
   "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb0_7], %[fa0_7], a[252:255]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb1_7], %[fa1_7], a[252:255]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
-  "s_waitcnt lgkmcnt(7)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "s_waitcnt lgkmcnt(6)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "s_waitcnt lgkmcnt(5)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "s_waitcnt lgkmcnt(2)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "s_waitcnt lgkmcnt(8)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "s_waitcnt lgkmcnt(7)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "s_waitcnt lgkmcnt(6)\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "s_waitcnt lgkmcnt(1)\n" \
+  "s_waitcnt lgkmcnt(5)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
+  "s_waitcnt lgkmcnt(4)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "s_waitcnt lgkmcnt(3)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
+  "s_waitcnt lgkmcnt(2)\n" \
   "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
+  "s_waitcnt lgkmcnt(1)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb0_0], %[fa0_7], a[224:227]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb1_0], %[fa1_7], a[224:227]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb0_1], %[fa0_7], a[228:231]\n" \
   "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb1_1], %[fa1_7], a[228:231]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
   "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
   "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb0_2], %[fa0_7], a[232:235]\n" \
   "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb1_2], %[fa1_7], a[232:235]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb0_3], %[fa0_7], a[236:239]\n" \
   "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb1_3], %[fa1_7], a[236:239]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
   "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
   "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], a[240:243]\n" \
   "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb1_4], %[fa1_7], a[240:243]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], a[244:247]\n" \
   "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb1_5], %[fa1_7], a[244:247]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
   "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb0_6], %[fa0_7], a[248:251]\n" \
   "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb1_6], %[fa1_7], a[248:251]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb0_7], %[fa0_7], a[252:255]\n" \
   "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb1_7], %[fa1_7], a[252:255]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
   "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
   "s_barrier\n" \
   "s_cmp_eq_u32 %[has_next], 0\n" \
@@ -3169,812 +3259,842 @@
   "s_waitcnt vmcnt(34)\n" \
   "L_w4_go_%=:\n" \
   "s_barrier\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
-  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
-  "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
   "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
   "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
   "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
   "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
   "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
   "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
   "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
   "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], 0\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
+  "s_waitcnt lgkmcnt(8)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb0_0], %[fa0_7], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb0_1], %[fa0_7], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
   "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb0_2], %[fa0_7], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb0_3], %[fa0_7], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
   "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb0_6], %[fa0_7], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb0_7], %[fa0_7], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "buffer_load_dwordx4 %[vo6], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
   "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
   "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
   "buffer_load_dwordx4 %[vo14], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb0_0], %[fa0_7], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb1_0], %[fa1_7], a[224:227]\n" \
   "buffer_load_dwordx4 %[vo15], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb0_1], %[fa0_7], 0\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb1_1], %[fa1_7], a[228:231]\n" \
   "s_waitcnt vmcnt(16)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], 0\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb1_0], %[fa1_7], a[224:227]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb1_1], %[fa1_7], a[228:231]\n" \
   "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], 0\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
   "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb0_2], %[fa0_7], 0\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb1_2], %[fa1_7], a[232:235]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb0_3], %[fa0_7], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb1_3], %[fa1_7], a[236:239]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], 0\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], 0\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb1_4], %[fa1_7], a[240:243]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb1_5], %[fa1_7], a[244:247]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], 0\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
-  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb0_6], %[fa0_7], 0\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb1_6], %[fa1_7], a[248:251]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb0_7], %[fa0_7], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb1_7], %[fa1_7], a[252:255]\n" \
-  "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], 0\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
   "s_cmp_eq_u32 %[iter], 0\n" \
   "s_cbranch_scc1 L_w4_after_%=\n" \
   "L_w4_loop_%=:\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
   "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
   "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
   "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
   "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
   "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
   "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "s_waitcnt lgkmcnt(8)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb0_0], %[fa0_7], a[224:227]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb0_1], %[fa0_7], a[228:231]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
   "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb0_2], %[fa0_7], a[232:235]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb0_3], %[fa0_7], a[236:239]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], a[240:243]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], a[244:247]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
   "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb0_6], %[fa0_7], a[248:251]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb0_7], %[fa0_7], a[252:255]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "buffer_load_dwordx4 %[vo6], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
   "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
   "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
   "buffer_load_dwordx4 %[vo14], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb0_0], %[fa0_7], a[224:227]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb1_0], %[fa1_7], a[224:227]\n" \
   "buffer_load_dwordx4 %[vo15], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb0_1], %[fa0_7], a[228:231]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb1_1], %[fa1_7], a[228:231]\n" \
   "s_waitcnt vmcnt(16)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb1_0], %[fa1_7], a[224:227]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb1_1], %[fa1_7], a[228:231]\n" \
   "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
   "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb0_2], %[fa0_7], a[232:235]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb1_2], %[fa1_7], a[232:235]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb0_3], %[fa0_7], a[236:239]\n" \
   "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb1_3], %[fa1_7], a[236:239]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
   "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], a[240:243]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb1_4], %[fa1_7], a[240:243]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], a[244:247]\n" \
   "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb1_5], %[fa1_7], a[244:247]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
-  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb0_6], %[fa0_7], a[248:251]\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb1_6], %[fa1_7], a[248:251]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb0_7], %[fa0_7], a[252:255]\n" \
   "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb1_7], %[fa1_7], a[252:255]\n" \
-  "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "s_sub_u32 %[iter], %[iter], 1\n" \
   "s_cmp_lg_u32 %[iter], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
   "s_cbranch_scc1 L_w4_loop_%=\n" \
   "L_w4_after_%=:\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb0_0], %[fa0_7], a[224:227]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb0_1], %[fa0_7], a[228:231]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb0_2], %[fa0_7], a[232:235]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb0_3], %[fa0_7], a[236:239]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], a[240:243]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], a[244:247]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb0_6], %[fa0_7], a[248:251]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb0_7], %[fa0_7], a[252:255]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
-  "s_waitcnt lgkmcnt(7)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "s_waitcnt lgkmcnt(6)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "s_waitcnt lgkmcnt(5)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "s_waitcnt lgkmcnt(2)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "s_waitcnt lgkmcnt(8)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "s_waitcnt lgkmcnt(7)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "s_waitcnt lgkmcnt(6)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "s_waitcnt lgkmcnt(5)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
+  "s_waitcnt lgkmcnt(4)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "s_waitcnt lgkmcnt(3)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
+  "s_waitcnt lgkmcnt(2)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
+  "s_waitcnt lgkmcnt(1)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb0_0], %[fa0_7], a[224:227]\n" \
+  "s_waitcnt lgkmcnt(0)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb1_0], %[fa1_7], a[224:227]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb0_1], %[fa0_7], a[228:231]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb1_1], %[fa1_7], a[228:231]\n" \
   "s_waitcnt vmcnt(0)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "s_waitcnt lgkmcnt(7)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "s_waitcnt lgkmcnt(7)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb1_0], %[fa1_7], a[224:227]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb1_1], %[fa1_7], a[228:231]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb1_2], %[fa1_7], a[232:235]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb1_3], %[fa1_7], a[236:239]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb1_4], %[fa1_7], a[240:243]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb1_5], %[fa1_7], a[244:247]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
-  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb1_6], %[fa1_7], a[248:251]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb1_7], %[fa1_7], a[252:255]\n" \
-  "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb0_0], %[fa0_7], a[224:227]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb0_1], %[fa0_7], a[228:231]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb0_2], %[fa0_7], a[232:235]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb0_3], %[fa0_7], a[236:239]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], a[240:243]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], a[244:247]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb0_2], %[fa0_7], a[232:235]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb1_2], %[fa1_7], a[232:235]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb0_3], %[fa0_7], a[236:239]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb1_3], %[fa1_7], a[236:239]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], a[240:243]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb1_4], %[fa1_7], a[240:243]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], a[244:247]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb1_5], %[fa1_7], a[244:247]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb0_6], %[fa0_7], a[248:251]\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb1_6], %[fa1_7], a[248:251]\n" \
   "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb0_7], %[fa0_7], a[252:255]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb1_7], %[fa1_7], a[252:255]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
-  "s_waitcnt lgkmcnt(7)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "s_waitcnt lgkmcnt(6)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "s_waitcnt lgkmcnt(5)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "ds_read_b128 %[fa0_7], %[rA0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "ds_read_b128 %[fa1_7], %[rA1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "s_waitcnt lgkmcnt(2)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "s_waitcnt lgkmcnt(8)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "s_waitcnt lgkmcnt(7)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "s_waitcnt lgkmcnt(6)\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "s_waitcnt lgkmcnt(1)\n" \
+  "s_waitcnt lgkmcnt(5)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
+  "s_waitcnt lgkmcnt(4)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "s_waitcnt lgkmcnt(3)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
+  "s_waitcnt lgkmcnt(2)\n" \
   "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
+  "s_waitcnt lgkmcnt(1)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb0_0], %[fa0_7], a[224:227]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "v_mfma_f32_16x16x32_bf16 a[224:227], %[fb1_0], %[fa1_7], a[224:227]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb0_1], %[fa0_7], a[228:231]\n" \
   "v_mfma_f32_16x16x32_bf16 a[228:231], %[fb1_1], %[fa1_7], a[228:231]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
   "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
   "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb0_2], %[fa0_7], a[232:235]\n" \
   "v_mfma_f32_16x16x32_bf16 a[232:235], %[fb1_2], %[fa1_7], a[232:235]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb0_3], %[fa0_7], a[236:239]\n" \
   "v_mfma_f32_16x16x32_bf16 a[236:239], %[fb1_3], %[fa1_7], a[236:239]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
   "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
   "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb0_4], %[fa0_7], a[240:243]\n" \
   "v_mfma_f32_16x16x32_bf16 a[240:243], %[fb1_4], %[fa1_7], a[240:243]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb0_5], %[fa0_7], a[244:247]\n" \
   "v_mfma_f32_16x16x32_bf16 a[244:247], %[fb1_5], %[fa1_7], a[244:247]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
   "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb0_6], %[fa0_7], a[248:251]\n" \
   "v_mfma_f32_16x16x32_bf16 a[248:251], %[fb1_6], %[fa1_7], a[248:251]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb0_7], %[fa0_7], a[252:255]\n" \
   "v_mfma_f32_16x16x32_bf16 a[252:255], %[fb1_7], %[fa1_7], a[252:255]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
   "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
   "s_barrier\n" \
   "s_cmp_eq_u32 %[has_next], 0\n" \
@@ -4165,496 +4285,506 @@
   "s_waitcnt vmcnt(28)\n" \
   "L_w4_go_%=:\n" \
   "s_barrier\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
   "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
   "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
   "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
   "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
   "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
   "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
   "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
   "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
   "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
   "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
   "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
   "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
   "buffer_load_dwordx4 %[vo4], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
   "buffer_load_dwordx4 %[vo5], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
   "s_waitcnt vmcnt(12)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
   "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "s_cmp_eq_u32 %[iter], 0\n" \
   "s_cbranch_scc1 L_w4_after_%=\n" \
   "L_w4_loop_%=:\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
   "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
   "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
   "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
   "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
   "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
   "buffer_load_dwordx4 %[vo4], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
   "buffer_load_dwordx4 %[vo5], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
   "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
   "s_waitcnt vmcnt(12)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
   "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "s_sub_u32 %[iter], %[iter], 1\n" \
   "s_cmp_lg_u32 %[iter], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "s_cbranch_scc1 L_w4_loop_%=\n" \
   "L_w4_after_%=:\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
   "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
   "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
   "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
   "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "s_waitcnt lgkmcnt(8)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(7)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(6)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
   "s_waitcnt lgkmcnt(2)\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "s_waitcnt lgkmcnt(1)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "s_waitcnt lgkmcnt(0)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
   "s_waitcnt vmcnt(0)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "s_waitcnt lgkmcnt(8)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(7)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(6)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
   "s_waitcnt lgkmcnt(2)\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "s_waitcnt lgkmcnt(1)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
   "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "s_barrier\n" \
   "s_cmp_eq_u32 %[has_next], 0\n" \
@@ -4821,496 +4951,506 @@
   "s_waitcnt vmcnt(20)\n" \
   "L_w4_go_%=:\n" \
   "s_barrier\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
   "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
   "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
   "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
   "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
   "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
   "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
   "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
   "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
   "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
   "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
   "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
   "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
   "buffer_load_dwordx4 %[vo4], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
   "buffer_load_dwordx4 %[vo5], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
   "s_waitcnt vmcnt(12)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
   "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "s_cmp_eq_u32 %[iter], 0\n" \
   "s_cbranch_scc1 L_w4_after_%=\n" \
   "L_w4_loop_%=:\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
   "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
   "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
   "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
   "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
   "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
   "buffer_load_dwordx4 %[vo4], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
   "buffer_load_dwordx4 %[vo5], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
   "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
   "s_waitcnt vmcnt(12)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
   "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "s_sub_u32 %[iter], %[iter], 1\n" \
   "s_cmp_lg_u32 %[iter], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "s_cbranch_scc1 L_w4_loop_%=\n" \
   "L_w4_after_%=:\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
   "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
   "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
   "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
   "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "s_waitcnt lgkmcnt(8)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(7)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(6)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
   "s_waitcnt lgkmcnt(2)\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "s_waitcnt lgkmcnt(1)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "s_waitcnt lgkmcnt(0)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
   "s_waitcnt vmcnt(0)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "s_waitcnt lgkmcnt(8)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(7)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(6)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
   "s_waitcnt lgkmcnt(2)\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "s_waitcnt lgkmcnt(1)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
   "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "s_barrier\n" \
   "s_cmp_eq_u32 %[has_next], 0\n" \
@@ -5477,496 +5617,506 @@
   "s_waitcnt vmcnt(30)\n" \
   "L_w4_go_%=:\n" \
   "s_barrier\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
   "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
   "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
   "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
   "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
   "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
   "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
   "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
   "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
   "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
   "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
   "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
   "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
   "buffer_load_dwordx4 %[vo4], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
   "buffer_load_dwordx4 %[vo5], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
   "s_waitcnt vmcnt(12)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
   "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "s_cmp_eq_u32 %[iter], 0\n" \
   "s_cbranch_scc1 L_w4_after_%=\n" \
   "L_w4_loop_%=:\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
   "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
   "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
   "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
   "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
   "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
   "buffer_load_dwordx4 %[vo4], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
   "buffer_load_dwordx4 %[vo5], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
   "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
   "s_waitcnt vmcnt(12)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
   "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "s_sub_u32 %[iter], %[iter], 1\n" \
   "s_cmp_lg_u32 %[iter], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "s_cbranch_scc1 L_w4_loop_%=\n" \
   "L_w4_after_%=:\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
   "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
   "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
   "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
   "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "s_waitcnt lgkmcnt(8)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(7)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(6)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
   "s_waitcnt lgkmcnt(2)\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "s_waitcnt lgkmcnt(1)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "s_waitcnt lgkmcnt(0)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
   "s_waitcnt vmcnt(0)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "s_waitcnt lgkmcnt(8)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(7)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(6)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
   "s_waitcnt lgkmcnt(2)\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "s_waitcnt lgkmcnt(1)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
   "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "s_barrier\n" \
   "s_cmp_eq_u32 %[has_next], 0\n" \
@@ -6133,496 +6283,506 @@
   "s_waitcnt vmcnt(22)\n" \
   "L_w4_go_%=:\n" \
   "s_barrier\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
   "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
   "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
   "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
   "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
   "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
   "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
   "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
   "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
   "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
   "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
   "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
   "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
   "buffer_load_dwordx4 %[vo4], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
   "buffer_load_dwordx4 %[vo5], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
   "s_waitcnt vmcnt(12)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
   "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "s_cmp_eq_u32 %[iter], 0\n" \
   "s_cbranch_scc1 L_w4_after_%=\n" \
   "L_w4_loop_%=:\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
   "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
   "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
   "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
   "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
   "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
   "buffer_load_dwordx4 %[vo4], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
   "buffer_load_dwordx4 %[vo5], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
   "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
   "s_waitcnt vmcnt(12)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
   "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "s_sub_u32 %[iter], %[iter], 1\n" \
   "s_cmp_lg_u32 %[iter], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "s_cbranch_scc1 L_w4_loop_%=\n" \
   "L_w4_after_%=:\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
   "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
   "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
   "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
   "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
   "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
   "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "s_waitcnt lgkmcnt(8)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(7)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(6)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
   "s_waitcnt lgkmcnt(2)\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "s_waitcnt lgkmcnt(1)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "s_waitcnt lgkmcnt(0)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
   "s_waitcnt vmcnt(0)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "s_waitcnt lgkmcnt(8)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(7)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(6)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
   "s_waitcnt lgkmcnt(2)\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "s_waitcnt lgkmcnt(1)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
   "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "s_barrier\n" \
   "s_cmp_eq_u32 %[has_next], 0\n" \
@@ -6795,574 +6955,590 @@
   "s_waitcnt vmcnt(33)\n" \
   "L_w4_go_%=:\n" \
   "s_barrier\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
   "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo5], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
   "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
   "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
   "s_waitcnt vmcnt(13)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "s_cmp_eq_u32 %[iter], 0\n" \
   "s_cbranch_scc1 L_w4_after_%=\n" \
   "L_w4_loop_%=:\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
   "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
   "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
   "buffer_load_dwordx4 %[vo5], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
   "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
   "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
   "s_waitcnt vmcnt(13)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "s_sub_u32 %[iter], %[iter], 1\n" \
   "s_cmp_lg_u32 %[iter], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "s_cbranch_scc1 L_w4_loop_%=\n" \
   "L_w4_after_%=:\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
   "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
   "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "s_waitcnt lgkmcnt(2)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(8)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(7)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "s_waitcnt lgkmcnt(5)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "s_waitcnt lgkmcnt(4)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "s_waitcnt lgkmcnt(3)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "s_waitcnt lgkmcnt(2)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "s_waitcnt lgkmcnt(1)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "s_waitcnt lgkmcnt(0)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
   "s_waitcnt vmcnt(0)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "s_waitcnt lgkmcnt(7)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "s_waitcnt lgkmcnt(6)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "s_waitcnt lgkmcnt(2)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "s_waitcnt lgkmcnt(1)\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(8)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(7)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "s_waitcnt lgkmcnt(5)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "s_waitcnt lgkmcnt(4)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "s_waitcnt lgkmcnt(3)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "s_waitcnt lgkmcnt(2)\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "s_waitcnt lgkmcnt(1)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "s_barrier\n" \
   "s_cmp_eq_u32 %[has_next], 0\n" \
@@ -7541,574 +7717,590 @@
   "s_waitcnt vmcnt(23)\n" \
   "L_w4_go_%=:\n" \
   "s_barrier\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
   "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo5], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
   "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
   "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
   "s_waitcnt vmcnt(13)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "s_cmp_eq_u32 %[iter], 0\n" \
   "s_cbranch_scc1 L_w4_after_%=\n" \
   "L_w4_loop_%=:\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
   "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
   "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
   "buffer_load_dwordx4 %[vo5], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
   "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
   "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
   "s_waitcnt vmcnt(13)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "s_sub_u32 %[iter], %[iter], 1\n" \
   "s_cmp_lg_u32 %[iter], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "s_cbranch_scc1 L_w4_loop_%=\n" \
   "L_w4_after_%=:\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
   "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
   "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "s_waitcnt lgkmcnt(2)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(8)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(7)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "s_waitcnt lgkmcnt(5)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "s_waitcnt lgkmcnt(4)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "s_waitcnt lgkmcnt(3)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "s_waitcnt lgkmcnt(2)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "s_waitcnt lgkmcnt(1)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "s_waitcnt lgkmcnt(0)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
   "s_waitcnt vmcnt(0)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "s_waitcnt lgkmcnt(7)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "s_waitcnt lgkmcnt(6)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "s_waitcnt lgkmcnt(2)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "s_waitcnt lgkmcnt(1)\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(8)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(7)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "s_waitcnt lgkmcnt(5)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "s_waitcnt lgkmcnt(4)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "s_waitcnt lgkmcnt(3)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "s_waitcnt lgkmcnt(2)\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "s_waitcnt lgkmcnt(1)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "s_barrier\n" \
   "s_cmp_eq_u32 %[has_next], 0\n" \
@@ -8287,574 +8479,590 @@
   "s_waitcnt vmcnt(35)\n" \
   "L_w4_go_%=:\n" \
   "s_barrier\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
   "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo5], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
   "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
   "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
   "s_waitcnt vmcnt(13)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "s_cmp_eq_u32 %[iter], 0\n" \
   "s_cbranch_scc1 L_w4_after_%=\n" \
   "L_w4_loop_%=:\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
   "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
   "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
   "buffer_load_dwordx4 %[vo5], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
   "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
   "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
   "s_waitcnt vmcnt(13)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "s_sub_u32 %[iter], %[iter], 1\n" \
   "s_cmp_lg_u32 %[iter], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "s_cbranch_scc1 L_w4_loop_%=\n" \
   "L_w4_after_%=:\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
   "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
   "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "s_waitcnt lgkmcnt(2)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(8)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(7)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "s_waitcnt lgkmcnt(5)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "s_waitcnt lgkmcnt(4)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "s_waitcnt lgkmcnt(3)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "s_waitcnt lgkmcnt(2)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "s_waitcnt lgkmcnt(1)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "s_waitcnt lgkmcnt(0)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
   "s_waitcnt vmcnt(0)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "s_waitcnt lgkmcnt(7)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "s_waitcnt lgkmcnt(6)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "s_waitcnt lgkmcnt(2)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "s_waitcnt lgkmcnt(1)\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(8)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(7)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "s_waitcnt lgkmcnt(5)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "s_waitcnt lgkmcnt(4)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "s_waitcnt lgkmcnt(3)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "s_waitcnt lgkmcnt(2)\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "s_waitcnt lgkmcnt(1)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "s_barrier\n" \
   "s_cmp_eq_u32 %[has_next], 0\n" \
@@ -9033,574 +9241,590 @@
   "s_waitcnt vmcnt(25)\n" \
   "L_w4_go_%=:\n" \
   "s_barrier\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
   "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo5], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
   "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
   "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
   "s_waitcnt vmcnt(13)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "s_cmp_eq_u32 %[iter], 0\n" \
   "s_cbranch_scc1 L_w4_after_%=\n" \
   "L_w4_loop_%=:\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
   "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
   "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
   "buffer_load_dwordx4 %[vo5], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
   "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
   "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
   "s_waitcnt vmcnt(13)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "s_sub_u32 %[iter], %[iter], 1\n" \
   "s_cmp_lg_u32 %[iter], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "s_cbranch_scc1 L_w4_loop_%=\n" \
   "L_w4_after_%=:\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
   "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
   "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "s_waitcnt lgkmcnt(2)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(8)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(7)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "s_waitcnt lgkmcnt(5)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "s_waitcnt lgkmcnt(4)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "s_waitcnt lgkmcnt(3)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "s_waitcnt lgkmcnt(2)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "s_waitcnt lgkmcnt(1)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "s_waitcnt lgkmcnt(0)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
   "s_waitcnt vmcnt(0)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "s_waitcnt lgkmcnt(7)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "s_waitcnt lgkmcnt(6)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "s_waitcnt lgkmcnt(2)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "s_waitcnt lgkmcnt(1)\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(8)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(7)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "s_waitcnt lgkmcnt(5)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "s_waitcnt lgkmcnt(4)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "s_waitcnt lgkmcnt(3)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "s_waitcnt lgkmcnt(2)\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "s_waitcnt lgkmcnt(1)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "s_barrier\n" \
   "s_cmp_eq_u32 %[has_next], 0\n" \
@@ -9785,370 +10009,382 @@
   "s_waitcnt vmcnt(38)\n" \
   "L_w4_go_%=:\n" \
   "s_barrier\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
   "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
   "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
   "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
   "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
   "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
   "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
   "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
   "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
   "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
   "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], 0\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
   "s_waitcnt vmcnt(14)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], 0\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], 0\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], 0\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
   "s_cmp_eq_u32 %[iter], 0\n" \
   "s_cbranch_scc1 L_w4_after_%=\n" \
   "L_w4_loop_%=:\n" \
   "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
   "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
   "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
   "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
   "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
   "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
   "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
   "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
   "s_waitcnt vmcnt(14)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "s_sub_u32 %[iter], %[iter], 1\n" \
   "s_cmp_lg_u32 %[iter], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
@@ -10156,281 +10392,287 @@
   "L_w4_after_%=:\n" \
   "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
   "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
   "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
   "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
   "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
-  "s_waitcnt lgkmcnt(5)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
   "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
   "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
   "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "s_waitcnt lgkmcnt(7)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "s_waitcnt lgkmcnt(6)\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "s_waitcnt lgkmcnt(2)\n" \
+  "s_waitcnt lgkmcnt(5)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "s_waitcnt lgkmcnt(4)\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "s_waitcnt lgkmcnt(3)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "s_waitcnt lgkmcnt(2)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "s_waitcnt lgkmcnt(1)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
+  "s_waitcnt lgkmcnt(0)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
   "s_waitcnt vmcnt(0)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "s_waitcnt lgkmcnt(8)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "s_waitcnt lgkmcnt(8)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
   "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
   "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
   "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
   "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
   "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
-  "s_waitcnt lgkmcnt(5)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
   "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
   "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
   "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "s_waitcnt lgkmcnt(7)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "s_waitcnt lgkmcnt(6)\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "s_waitcnt lgkmcnt(2)\n" \
+  "s_waitcnt lgkmcnt(5)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "s_waitcnt lgkmcnt(4)\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
   "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "s_waitcnt lgkmcnt(1)\n" \
+  "s_waitcnt lgkmcnt(3)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "s_waitcnt lgkmcnt(2)\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "s_waitcnt lgkmcnt(1)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
   "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
   "s_barrier\n" \
   "s_cmp_eq_u32 %[has_next], 0\n" \
@@ -10621,370 +10863,382 @@
   "s_waitcnt vmcnt(26)\n" \
   "L_w4_go_%=:\n" \
   "s_barrier\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
   "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
   "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
   "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
   "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
   "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
   "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
   "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
   "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
   "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
   "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], 0\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
   "s_waitcnt vmcnt(14)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], 0\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], 0\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], 0\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
   "s_cmp_eq_u32 %[iter], 0\n" \
   "s_cbranch_scc1 L_w4_after_%=\n" \
   "L_w4_loop_%=:\n" \
   "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
   "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
   "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
   "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
   "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
   "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
   "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
   "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
   "s_waitcnt vmcnt(14)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "s_sub_u32 %[iter], %[iter], 1\n" \
   "s_cmp_lg_u32 %[iter], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
@@ -10992,281 +11246,287 @@
   "L_w4_after_%=:\n" \
   "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
   "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
   "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
   "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
   "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
-  "s_waitcnt lgkmcnt(5)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
   "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
   "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
   "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "s_waitcnt lgkmcnt(7)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "s_waitcnt lgkmcnt(6)\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "s_waitcnt lgkmcnt(2)\n" \
+  "s_waitcnt lgkmcnt(5)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "s_waitcnt lgkmcnt(4)\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "s_waitcnt lgkmcnt(3)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "s_waitcnt lgkmcnt(2)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "s_waitcnt lgkmcnt(1)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
+  "s_waitcnt lgkmcnt(0)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
   "s_waitcnt vmcnt(0)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "s_waitcnt lgkmcnt(8)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "s_waitcnt lgkmcnt(8)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
   "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
   "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
   "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
   "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
   "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
-  "s_waitcnt lgkmcnt(5)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
   "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
   "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
   "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "s_waitcnt lgkmcnt(7)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "s_waitcnt lgkmcnt(6)\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "s_waitcnt lgkmcnt(2)\n" \
+  "s_waitcnt lgkmcnt(5)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "s_waitcnt lgkmcnt(4)\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
   "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "s_waitcnt lgkmcnt(1)\n" \
+  "s_waitcnt lgkmcnt(3)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "s_waitcnt lgkmcnt(2)\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "s_waitcnt lgkmcnt(1)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
   "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
   "s_barrier\n" \
   "s_cmp_eq_u32 %[has_next], 0\n" \
@@ -11457,370 +11717,382 @@
   "s_waitcnt vmcnt(40)\n" \
   "L_w4_go_%=:\n" \
   "s_barrier\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
   "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
   "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
   "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
   "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
   "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
   "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
   "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
   "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
   "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
   "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], 0\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
   "s_waitcnt vmcnt(14)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], 0\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], 0\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], 0\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
   "s_cmp_eq_u32 %[iter], 0\n" \
   "s_cbranch_scc1 L_w4_after_%=\n" \
   "L_w4_loop_%=:\n" \
   "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
   "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
   "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
   "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
   "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
   "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
   "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
   "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
   "s_waitcnt vmcnt(14)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "s_sub_u32 %[iter], %[iter], 1\n" \
   "s_cmp_lg_u32 %[iter], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
@@ -11828,281 +12100,287 @@
   "L_w4_after_%=:\n" \
   "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
   "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
   "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
   "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
   "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
-  "s_waitcnt lgkmcnt(5)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
   "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
   "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
   "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "s_waitcnt lgkmcnt(7)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "s_waitcnt lgkmcnt(6)\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "s_waitcnt lgkmcnt(2)\n" \
+  "s_waitcnt lgkmcnt(5)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "s_waitcnt lgkmcnt(4)\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "s_waitcnt lgkmcnt(3)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "s_waitcnt lgkmcnt(2)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "s_waitcnt lgkmcnt(1)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
+  "s_waitcnt lgkmcnt(0)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
   "s_waitcnt vmcnt(0)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "s_waitcnt lgkmcnt(8)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "s_waitcnt lgkmcnt(8)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
   "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
   "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
   "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
   "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
   "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
-  "s_waitcnt lgkmcnt(5)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
   "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
   "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
   "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "s_waitcnt lgkmcnt(7)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "s_waitcnt lgkmcnt(6)\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "s_waitcnt lgkmcnt(2)\n" \
+  "s_waitcnt lgkmcnt(5)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "s_waitcnt lgkmcnt(4)\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
   "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "s_waitcnt lgkmcnt(1)\n" \
+  "s_waitcnt lgkmcnt(3)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "s_waitcnt lgkmcnt(2)\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "s_waitcnt lgkmcnt(1)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
   "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
   "s_barrier\n" \
   "s_cmp_eq_u32 %[has_next], 0\n" \
@@ -12293,370 +12571,382 @@
   "s_waitcnt vmcnt(28)\n" \
   "L_w4_go_%=:\n" \
   "s_barrier\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
   "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
   "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
   "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
   "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
   "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
   "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
   "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
   "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
   "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
   "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], 0\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
   "s_waitcnt vmcnt(14)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], 0\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], 0\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], 0\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
   "s_cmp_eq_u32 %[iter], 0\n" \
   "s_cbranch_scc1 L_w4_after_%=\n" \
   "L_w4_loop_%=:\n" \
   "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
   "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
   "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
   "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "s_waitcnt lgkmcnt(14)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
   "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
   "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "buffer_load_dwordx4 %[vo6], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
   "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
   "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
   "s_waitcnt vmcnt(14)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "s_sub_u32 %[iter], %[iter], 1\n" \
   "s_cmp_lg_u32 %[iter], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
@@ -12664,281 +12954,287 @@
   "L_w4_after_%=:\n" \
   "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
   "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
   "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
   "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
   "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
-  "s_waitcnt lgkmcnt(5)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
   "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
   "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
   "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "s_waitcnt lgkmcnt(7)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "s_waitcnt lgkmcnt(6)\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "s_waitcnt lgkmcnt(2)\n" \
+  "s_waitcnt lgkmcnt(5)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "s_waitcnt lgkmcnt(4)\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "s_waitcnt lgkmcnt(3)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "s_waitcnt lgkmcnt(2)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "s_waitcnt lgkmcnt(1)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
+  "s_waitcnt lgkmcnt(0)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
   "s_waitcnt vmcnt(0)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "s_waitcnt lgkmcnt(8)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "s_waitcnt lgkmcnt(8)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
   "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
   "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
   "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
   "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
   "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
   "s_waitcnt lgkmcnt(14)\n" \
   "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
   "s_waitcnt lgkmcnt(14)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
-  "s_waitcnt lgkmcnt(5)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
   "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
   "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
   "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "s_waitcnt lgkmcnt(7)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "s_waitcnt lgkmcnt(6)\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
   "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "s_waitcnt lgkmcnt(2)\n" \
+  "s_waitcnt lgkmcnt(5)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "s_waitcnt lgkmcnt(4)\n" \
   "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
   "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
   "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
   "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
   "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
   "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
   "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
   "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
   "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
   "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
   "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
   "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
   "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
   "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "s_waitcnt lgkmcnt(1)\n" \
+  "s_waitcnt lgkmcnt(3)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "s_waitcnt lgkmcnt(2)\n" \
   "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "s_waitcnt lgkmcnt(1)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
   "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
   "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
   "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
   "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
   "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
   "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
   "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
   "s_barrier\n" \
   "s_cmp_eq_u32 %[has_next], 0\n" \
@@ -13135,732 +13431,756 @@
   "s_waitcnt vmcnt(43)\n" \
   "L_w4_go_%=:\n" \
   "s_barrier\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
   "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
   "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
   "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
   "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
   "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
   "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
   "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
-  "s_waitcnt lgkmcnt(9)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
   "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
   "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
   "buffer_load_dwordx4 %[vo6], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], 0\n" \
   "buffer_load_dwordx4 %[vo14], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
   "s_waitcnt vmcnt(15)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], 0\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
   "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], 0\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], 0\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], 0\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], 0\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], 0\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
-  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], 0\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], 0\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
   "s_cmp_eq_u32 %[iter], 0\n" \
   "s_cbranch_scc1 L_w4_after_%=\n" \
   "L_w4_loop_%=:\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
   "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "s_waitcnt lgkmcnt(9)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
   "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
   "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
   "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
   "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
   "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
   "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
   "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
   "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
   "buffer_load_dwordx4 %[vo6], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
   "buffer_load_dwordx4 %[vo14], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
   "s_waitcnt vmcnt(15)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
   "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
   "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
   "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
-  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
   "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "s_sub_u32 %[iter], %[iter], 1\n" \
   "s_cmp_lg_u32 %[iter], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
   "s_cbranch_scc1 L_w4_loop_%=\n" \
   "L_w4_after_%=:\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
   "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "s_waitcnt lgkmcnt(9)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
-  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
-  "s_waitcnt lgkmcnt(6)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "s_waitcnt lgkmcnt(5)\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "s_waitcnt lgkmcnt(2)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "s_waitcnt lgkmcnt(8)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "s_waitcnt lgkmcnt(7)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "s_waitcnt lgkmcnt(6)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "s_waitcnt lgkmcnt(5)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "s_waitcnt lgkmcnt(4)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "s_waitcnt lgkmcnt(3)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
+  "s_waitcnt lgkmcnt(2)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "s_waitcnt lgkmcnt(1)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
+  "s_waitcnt lgkmcnt(0)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
   "s_waitcnt vmcnt(0)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "s_waitcnt lgkmcnt(8)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "s_waitcnt lgkmcnt(7)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
-  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "s_waitcnt lgkmcnt(9)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
-  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
   "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
   "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
   "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
-  "s_waitcnt lgkmcnt(6)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "s_waitcnt lgkmcnt(5)\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "s_waitcnt lgkmcnt(2)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "s_waitcnt lgkmcnt(8)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "s_waitcnt lgkmcnt(7)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "s_waitcnt lgkmcnt(6)\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "s_waitcnt lgkmcnt(1)\n" \
+  "s_waitcnt lgkmcnt(5)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "s_waitcnt lgkmcnt(4)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "s_waitcnt lgkmcnt(3)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
+  "s_waitcnt lgkmcnt(2)\n" \
   "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "s_waitcnt lgkmcnt(1)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
   "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
   "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
   "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
   "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
   "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
   "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
   "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
   "s_barrier\n" \
   "s_cmp_eq_u32 %[has_next], 0\n" \
@@ -14063,732 +14383,756 @@
   "s_waitcnt vmcnt(29)\n" \
   "L_w4_go_%=:\n" \
   "s_barrier\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
   "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
   "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
   "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
   "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
   "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
   "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
   "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
-  "s_waitcnt lgkmcnt(9)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
   "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
   "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
   "buffer_load_dwordx4 %[vo6], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], 0\n" \
   "buffer_load_dwordx4 %[vo14], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
   "s_waitcnt vmcnt(15)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], 0\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
   "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], 0\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], 0\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], 0\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], 0\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], 0\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
-  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], 0\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], 0\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
   "s_cmp_eq_u32 %[iter], 0\n" \
   "s_cbranch_scc1 L_w4_after_%=\n" \
   "L_w4_loop_%=:\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
   "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "s_waitcnt lgkmcnt(9)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
   "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
   "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
   "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
   "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
   "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
   "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
   "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
   "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
   "buffer_load_dwordx4 %[vo6], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
   "buffer_load_dwordx4 %[vo14], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
   "s_waitcnt vmcnt(15)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
   "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
   "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
   "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
-  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
   "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "s_sub_u32 %[iter], %[iter], 1\n" \
   "s_cmp_lg_u32 %[iter], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
   "s_cbranch_scc1 L_w4_loop_%=\n" \
   "L_w4_after_%=:\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
   "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "s_waitcnt lgkmcnt(9)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
-  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
-  "s_waitcnt lgkmcnt(6)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "s_waitcnt lgkmcnt(5)\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "s_waitcnt lgkmcnt(2)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "s_waitcnt lgkmcnt(8)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "s_waitcnt lgkmcnt(7)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "s_waitcnt lgkmcnt(6)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "s_waitcnt lgkmcnt(5)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "s_waitcnt lgkmcnt(4)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "s_waitcnt lgkmcnt(3)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
+  "s_waitcnt lgkmcnt(2)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "s_waitcnt lgkmcnt(1)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
+  "s_waitcnt lgkmcnt(0)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
   "s_waitcnt vmcnt(0)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "s_waitcnt lgkmcnt(8)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "s_waitcnt lgkmcnt(7)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
-  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "s_waitcnt lgkmcnt(9)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
-  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
   "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
   "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
   "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
-  "s_waitcnt lgkmcnt(6)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "s_waitcnt lgkmcnt(5)\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "s_waitcnt lgkmcnt(2)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "s_waitcnt lgkmcnt(8)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "s_waitcnt lgkmcnt(7)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "s_waitcnt lgkmcnt(6)\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "s_waitcnt lgkmcnt(1)\n" \
+  "s_waitcnt lgkmcnt(5)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "s_waitcnt lgkmcnt(4)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "s_waitcnt lgkmcnt(3)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
+  "s_waitcnt lgkmcnt(2)\n" \
   "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "s_waitcnt lgkmcnt(1)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
   "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
   "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
   "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
   "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
   "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
   "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
   "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
   "s_barrier\n" \
   "s_cmp_eq_u32 %[has_next], 0\n" \
@@ -14991,732 +15335,756 @@
   "s_waitcnt vmcnt(45)\n" \
   "L_w4_go_%=:\n" \
   "s_barrier\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
   "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
   "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
   "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
   "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
   "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
   "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
   "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
-  "s_waitcnt lgkmcnt(9)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
   "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
   "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
   "buffer_load_dwordx4 %[vo6], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], 0\n" \
   "buffer_load_dwordx4 %[vo14], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
   "s_waitcnt vmcnt(15)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], 0\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
   "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], 0\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], 0\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], 0\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], 0\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], 0\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
-  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], 0\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], 0\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
   "s_cmp_eq_u32 %[iter], 0\n" \
   "s_cbranch_scc1 L_w4_after_%=\n" \
   "L_w4_loop_%=:\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
   "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "s_waitcnt lgkmcnt(9)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
   "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
   "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
   "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
   "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
   "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
   "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
   "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
   "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
   "buffer_load_dwordx4 %[vo6], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
   "buffer_load_dwordx4 %[vo14], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
   "s_waitcnt vmcnt(15)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
   "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
   "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
   "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
-  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
   "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "s_sub_u32 %[iter], %[iter], 1\n" \
   "s_cmp_lg_u32 %[iter], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
   "s_cbranch_scc1 L_w4_loop_%=\n" \
   "L_w4_after_%=:\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
   "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "s_waitcnt lgkmcnt(9)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
-  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
-  "s_waitcnt lgkmcnt(6)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "s_waitcnt lgkmcnt(5)\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "s_waitcnt lgkmcnt(2)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "s_waitcnt lgkmcnt(8)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "s_waitcnt lgkmcnt(7)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "s_waitcnt lgkmcnt(6)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "s_waitcnt lgkmcnt(5)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "s_waitcnt lgkmcnt(4)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "s_waitcnt lgkmcnt(3)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
+  "s_waitcnt lgkmcnt(2)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "s_waitcnt lgkmcnt(1)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
+  "s_waitcnt lgkmcnt(0)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
   "s_waitcnt vmcnt(0)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "s_waitcnt lgkmcnt(8)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "s_waitcnt lgkmcnt(7)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
-  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "s_waitcnt lgkmcnt(9)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
-  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
   "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
   "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
   "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
-  "s_waitcnt lgkmcnt(6)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "s_waitcnt lgkmcnt(5)\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "s_waitcnt lgkmcnt(2)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "s_waitcnt lgkmcnt(8)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "s_waitcnt lgkmcnt(7)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "s_waitcnt lgkmcnt(6)\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "s_waitcnt lgkmcnt(1)\n" \
+  "s_waitcnt lgkmcnt(5)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "s_waitcnt lgkmcnt(4)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "s_waitcnt lgkmcnt(3)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
+  "s_waitcnt lgkmcnt(2)\n" \
   "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "s_waitcnt lgkmcnt(1)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
   "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
   "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
   "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
   "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
   "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
   "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
   "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
   "s_barrier\n" \
   "s_cmp_eq_u32 %[has_next], 0\n" \
@@ -15919,732 +16287,756 @@
   "s_waitcnt vmcnt(31)\n" \
   "L_w4_go_%=:\n" \
   "s_barrier\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
   "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
   "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
   "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
   "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
+  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
   "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
   "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
   "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], 0\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], 0\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], 0\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], 0\n" \
-  "s_waitcnt lgkmcnt(9)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], 0\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
-  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
   "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], 0\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], 0\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], 0\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], 0\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
   "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], 0\n" \
   "buffer_load_dwordx4 %[vo6], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], 0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], 0\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], 0\n" \
   "buffer_load_dwordx4 %[vo14], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], 0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
   "s_waitcnt vmcnt(15)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], 0\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
   "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], 0\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], 0\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], 0\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], 0\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], 0\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
-  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], 0\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], 0\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
   "s_cmp_eq_u32 %[iter], 0\n" \
   "s_cbranch_scc1 L_w4_after_%=\n" \
   "L_w4_loop_%=:\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
   "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "s_waitcnt lgkmcnt(9)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
   "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
   "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
   "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
   "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
   "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
   "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
   "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "s_barrier\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
   "s_mov_b32 m0, %[dbase]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
   "buffer_load_dwordx4 %[vo0], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
   "buffer_load_dwordx4 %[vo1], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
   "buffer_load_dwordx4 %[vo2], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
   "buffer_load_dwordx4 %[vo3], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
   "buffer_load_dwordx4 %[vo4], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
   "buffer_load_dwordx4 %[vo5], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
   "buffer_load_dwordx4 %[vo6], %[srdA], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
   "buffer_load_dwordx4 %[vo7], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
   "buffer_load_dwordx4 %[vo8], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
   "buffer_load_dwordx4 %[vo9], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
   "buffer_load_dwordx4 %[vo10], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
   "buffer_load_dwordx4 %[vo11], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
   "buffer_load_dwordx4 %[vo12], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
   "buffer_load_dwordx4 %[vo13], %[srdB], %[koff] offen lds\n" \
   "s_add_u32 m0, m0, 0x1000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
   "buffer_load_dwordx4 %[vo14], %[srdB], %[koff] offen lds\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
   "s_add_u32 %[koff], %[koff], 0x80\n" \
   "s_cmp_eq_u32 %[koff], %[kend]\n" \
   "s_cselect_b32 %[koff], 0, %[koff]\n" \
   "s_xor_b32 %[dbase], %[dbase], 0x10000\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
   "s_waitcnt vmcnt(15)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
+  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
   "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
   "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
   "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
   "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
   "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
-  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
   "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
   "s_sub_u32 %[iter], %[iter], 1\n" \
   "s_cmp_lg_u32 %[iter], 0\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
   "s_cbranch_scc1 L_w4_loop_%=\n" \
   "L_w4_after_%=:\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
   "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "s_waitcnt lgkmcnt(9)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
-  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
-  "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
-  "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
-  "s_waitcnt lgkmcnt(6)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "s_waitcnt lgkmcnt(5)\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "s_waitcnt lgkmcnt(2)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "s_waitcnt lgkmcnt(8)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "s_waitcnt lgkmcnt(7)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "s_waitcnt lgkmcnt(6)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
+  "s_waitcnt lgkmcnt(5)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "s_waitcnt lgkmcnt(4)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
   "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "s_waitcnt lgkmcnt(3)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
+  "s_waitcnt lgkmcnt(2)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "s_waitcnt lgkmcnt(1)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
+  "s_waitcnt lgkmcnt(0)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
   "s_waitcnt vmcnt(0)\n" \
   "s_barrier\n" \
   "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]\n" \
   "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
-  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
-  "s_waitcnt lgkmcnt(8)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
-  "s_waitcnt lgkmcnt(7)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
-  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
-  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
-  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
-  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
-  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
-  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
-  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
-  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
-  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
-  "s_waitcnt lgkmcnt(13)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
-  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
-  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
-  "s_waitcnt lgkmcnt(12)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
-  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
-  "s_waitcnt lgkmcnt(11)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
-  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
-  "s_waitcnt lgkmcnt(10)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
-  "s_waitcnt lgkmcnt(9)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
-  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
-  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
-  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
-  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
-  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
-  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
-  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
-  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
-  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
-  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
-  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
-  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
-  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
-  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
   "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]\n" \
   "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
-  "s_waitcnt lgkmcnt(15)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
   "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
+  "ds_read_b128 %[fa0_0], %[rA0] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "ds_read_b128 %[fa1_0], %[rA1] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
+  "ds_read_b128 %[fa0_1], %[rA0] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "ds_read_b128 %[fb0_0], %[rB0] offset:0\n" \
   "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
+  "ds_read_b128 %[fb1_0], %[rB1] offset:0\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
+  "ds_read_b128 %[fa1_1], %[rA1] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "ds_read_b128 %[fb0_1], %[rB0] offset:2048\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
+  "ds_read_b128 %[fb1_1], %[rB1] offset:2048\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "ds_read_b128 %[fb0_2], %[rB0] offset:4096\n" \
   "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
+  "ds_read_b128 %[fb1_2], %[rB1] offset:4096\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
   "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
+  "ds_read_b128 %[fb0_3], %[rB0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
+  "ds_read_b128 %[fb1_3], %[rB1] offset:6144\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "ds_read_b128 %[fb0_4], %[rB0] offset:8192\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
+  "ds_read_b128 %[fb1_4], %[rB1] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
   "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
+  "ds_read_b128 %[fb0_5], %[rB0] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
-  "s_waitcnt lgkmcnt(6)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_5], %[rB1] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb0_0], %[fa0_0], a[0:3]\n" \
+  "ds_read_b128 %[fa0_2], %[rA0] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[0:3], %[fb1_0], %[fa1_0], a[0:3]\n" \
-  "s_waitcnt lgkmcnt(5)\n" \
+  "ds_read_b128 %[fb0_6], %[rB0] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb0_0], %[fa0_1], a[32:35]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[32:35], %[fb1_0], %[fa1_1], a[32:35]\n" \
-  "s_waitcnt lgkmcnt(4)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "ds_read_b128 %[fb1_6], %[rB1] offset:12288\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb0_1], %[fa0_1], a[36:39]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
   "v_mfma_f32_16x16x32_bf16 a[36:39], %[fb1_1], %[fa1_1], a[36:39]\n" \
+  "ds_read_b128 %[fb0_7], %[rB0] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb0_1], %[fa0_0], a[4:7]\n" \
+  "ds_read_b128 %[fb1_7], %[rB1] offset:14336\n" \
+  "v_mfma_f32_16x16x32_bf16 a[4:7], %[fb1_1], %[fa1_0], a[4:7]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb0_2], %[fa0_0], a[8:11]\n" \
+  "ds_read_b128 %[fa1_2], %[rA1] offset:4096\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[8:11], %[fb1_2], %[fa1_0], a[8:11]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb0_2], %[fa0_1], a[40:43]\n" \
+  "ds_read_b128 %[fa0_3], %[rA0] offset:6144\n" \
   "v_mfma_f32_16x16x32_bf16 a[40:43], %[fb1_2], %[fa1_1], a[40:43]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb0_3], %[fa0_1], a[44:47]\n" \
+  "ds_read_b128 %[fa1_3], %[rA1] offset:6144\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
   "v_mfma_f32_16x16x32_bf16 a[44:47], %[fb1_3], %[fa1_1], a[44:47]\n" \
+  "ds_read_b128 %[fa0_4], %[rA0] offset:8192\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb0_3], %[fa0_0], a[12:15]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[12:15], %[fb1_3], %[fa1_0], a[12:15]\n" \
+  "ds_read_b128 %[fa1_4], %[rA1] offset:8192\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb0_4], %[fa0_0], a[16:19]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[16:19], %[fb1_4], %[fa1_0], a[16:19]\n" \
+  "ds_read_b128 %[fa0_5], %[rA0] offset:10240\n" \
+  "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb0_4], %[fa0_1], a[48:51]\n" \
+  "ds_read_b128 %[fa1_5], %[rA1] offset:10240\n" \
   "v_mfma_f32_16x16x32_bf16 a[48:51], %[fb1_4], %[fa1_1], a[48:51]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb0_5], %[fa0_1], a[52:55]\n" \
+  "ds_read_b128 %[fa0_6], %[rA0] offset:12288\n" \
+  "s_waitcnt lgkmcnt(13)\n" \
   "v_mfma_f32_16x16x32_bf16 a[52:55], %[fb1_5], %[fa1_1], a[52:55]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb0_5], %[fa0_0], a[20:23]\n" \
+  "ds_read_b128 %[fa1_6], %[rA1] offset:12288\n" \
+  "v_mfma_f32_16x16x32_bf16 a[20:23], %[fb1_5], %[fa1_0], a[20:23]\n" \
+  "s_waitcnt lgkmcnt(12)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb0_6], %[fa0_0], a[24:27]\n" \
+  "s_waitcnt lgkmcnt(11)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[24:27], %[fb1_6], %[fa1_0], a[24:27]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb0_6], %[fa0_1], a[56:59]\n" \
   "v_mfma_f32_16x16x32_bf16 a[56:59], %[fb1_6], %[fa1_1], a[56:59]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "s_waitcnt lgkmcnt(10)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb0_7], %[fa0_1], a[60:63]\n" \
+  "s_waitcnt lgkmcnt(9)\n" \
   "v_mfma_f32_16x16x32_bf16 a[60:63], %[fb1_7], %[fa1_1], a[60:63]\n" \
-  "s_waitcnt lgkmcnt(3)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
-  "s_waitcnt lgkmcnt(2)\n" \
-  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
-  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb0_7], %[fa0_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[28:31], %[fb1_7], %[fa1_0], a[28:31]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb0_7], %[fa0_2], a[92:95]\n" \
+  "s_waitcnt lgkmcnt(8)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[92:95], %[fb1_7], %[fa1_2], a[92:95]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb0_6], %[fa0_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[88:91], %[fb1_6], %[fa1_2], a[88:91]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb0_5], %[fa0_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[84:87], %[fb1_5], %[fa1_2], a[84:87]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb0_4], %[fa0_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[80:83], %[fb1_4], %[fa1_2], a[80:83]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb0_3], %[fa0_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[76:79], %[fb1_3], %[fa1_2], a[76:79]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb0_2], %[fa0_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[72:75], %[fb1_2], %[fa1_2], a[72:75]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb0_1], %[fa0_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[68:71], %[fb1_1], %[fa1_2], a[68:71]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb0_0], %[fa0_2], a[64:67]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[64:67], %[fb1_0], %[fa1_2], a[64:67]\n" \
+  "s_waitcnt lgkmcnt(7)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb0_0], %[fa0_3], a[96:99]\n" \
+  "s_waitcnt lgkmcnt(6)\n" \
   "v_mfma_f32_16x16x32_bf16 a[96:99], %[fb1_0], %[fa1_3], a[96:99]\n" \
-  "s_waitcnt lgkmcnt(1)\n" \
+  "s_waitcnt lgkmcnt(5)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb0_0], %[fa0_4], a[128:131]\n" \
+  "s_waitcnt lgkmcnt(4)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[128:131], %[fb1_0], %[fa1_4], a[128:131]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb0_1], %[fa0_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[132:135], %[fb1_1], %[fa1_4], a[132:135]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb0_1], %[fa0_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[100:103], %[fb1_1], %[fa1_3], a[100:103]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb0_2], %[fa0_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[104:107], %[fb1_2], %[fa1_3], a[104:107]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb0_2], %[fa0_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[136:139], %[fb1_2], %[fa1_4], a[136:139]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb0_3], %[fa0_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[140:143], %[fb1_3], %[fa1_4], a[140:143]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb0_3], %[fa0_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[108:111], %[fb1_3], %[fa1_3], a[108:111]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb0_4], %[fa0_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[112:115], %[fb1_4], %[fa1_3], a[112:115]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb0_4], %[fa0_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[144:147], %[fb1_4], %[fa1_4], a[144:147]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb0_5], %[fa0_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[148:151], %[fb1_5], %[fa1_4], a[148:151]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb0_5], %[fa0_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[116:119], %[fb1_5], %[fa1_3], a[116:119]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb0_6], %[fa0_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[120:123], %[fb1_6], %[fa1_3], a[120:123]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb0_6], %[fa0_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[152:155], %[fb1_6], %[fa1_4], a[152:155]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb0_7], %[fa0_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[156:159], %[fb1_7], %[fa1_4], a[156:159]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb0_7], %[fa0_3], a[124:127]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[124:127], %[fb1_7], %[fa1_3], a[124:127]\n" \
+  "s_waitcnt lgkmcnt(3)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb0_0], %[fa0_5], a[160:163]\n" \
+  "s_waitcnt lgkmcnt(2)\n" \
   "v_mfma_f32_16x16x32_bf16 a[160:163], %[fb1_0], %[fa1_5], a[160:163]\n" \
+  "s_waitcnt lgkmcnt(1)\n" \
+  "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb0_0], %[fa0_6], a[192:195]\n" \
   "s_waitcnt lgkmcnt(0)\n" \
   "v_mfma_f32_16x16x32_bf16 a[192:195], %[fb1_0], %[fa1_6], a[192:195]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb0_1], %[fa0_6], a[196:199]\n" \
   "v_mfma_f32_16x16x32_bf16 a[196:199], %[fb1_1], %[fa1_6], a[196:199]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb0_1], %[fa0_5], a[164:167]\n" \
   "v_mfma_f32_16x16x32_bf16 a[164:167], %[fb1_1], %[fa1_5], a[164:167]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb0_2], %[fa0_5], a[168:171]\n" \
   "v_mfma_f32_16x16x32_bf16 a[168:171], %[fb1_2], %[fa1_5], a[168:171]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb0_2], %[fa0_6], a[200:203]\n" \
   "v_mfma_f32_16x16x32_bf16 a[200:203], %[fb1_2], %[fa1_6], a[200:203]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb0_3], %[fa0_6], a[204:207]\n" \
   "v_mfma_f32_16x16x32_bf16 a[204:207], %[fb1_3], %[fa1_6], a[204:207]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb0_3], %[fa0_5], a[172:175]\n" \
   "v_mfma_f32_16x16x32_bf16 a[172:175], %[fb1_3], %[fa1_5], a[172:175]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb0_4], %[fa0_5], a[176:179]\n" \
   "v_mfma_f32_16x16x32_bf16 a[176:179], %[fb1_4], %[fa1_5], a[176:179]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb0_4], %[fa0_6], a[208:211]\n" \
   "v_mfma_f32_16x16x32_bf16 a[208:211], %[fb1_4], %[fa1_6], a[208:211]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb0_5], %[fa0_6], a[212:215]\n" \
   "v_mfma_f32_16x16x32_bf16 a[212:215], %[fb1_5], %[fa1_6], a[212:215]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb0_5], %[fa0_5], a[180:183]\n" \
   "v_mfma_f32_16x16x32_bf16 a[180:183], %[fb1_5], %[fa1_5], a[180:183]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb0_6], %[fa0_5], a[184:187]\n" \
   "v_mfma_f32_16x16x32_bf16 a[184:187], %[fb1_6], %[fa1_5], a[184:187]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb0_6], %[fa0_6], a[216:219]\n" \
   "v_mfma_f32_16x16x32_bf16 a[216:219], %[fb1_6], %[fa1_6], a[216:219]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb0_7], %[fa0_6], a[220:223]\n" \
   "v_mfma_f32_16x16x32_bf16 a[220:223], %[fb1_7], %[fa1_6], a[220:223]\n" \
+  "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb0_7], %[fa0_5], a[188:191]\n" \
   "v_mfma_f32_16x16x32_bf16 a[188:191], %[fb1_7], %[fa1_5], a[188:191]\n" \
   "s_barrier\n" \
   "s_cmp_eq_u32 %[has_next], 0\n" \

@@ -21,16 +21,17 @@ Geometry (one workgroup = 4 waves = one 256 x 256 output tile, BK = 64):
     p = w + 4i, i = 0..15: i < 8 A rows 8p.., else B rows 8(p - 32)..) and 32 ds_read_b128
     (A and B fragments for both 32-deep K halves) against 128 MFMAs.
 
-Schedule of iteration t (MFMA slot m = 0..127; H0 = k-half 0 of tile t, H1 = k-half 1):
-  m  1..31   ds_read k-half-1 fragments of tile t (FB1[0..7], FA1[0..7]) from buffer t&1
+Schedule of iteration t (MFMA slot m = 0..127):
+  m  1..31   ds_read what is left of tile t (FB*[6], FB*[7], FA*[2..7]) from buffer t&1
   m  38      lgkmcnt(0) + s_barrier (B1): every wave is done reading buffer t&1
   m 40..100  16 LDS-DMA pieces of tile t+2 into buffer t&1 (one per 4 MFMAs)
   m  102     vmcnt(16) + s_barrier (B2): tile t+1 (issued one iteration ago) has landed
-  m 103..127 ds_read k-half-0 fragments of tile t+1 (FB0, FA0) from buffer (t+1)&1
-Lower tiles (128, 160, 192, 224 rows: 64, 80, 96, 112 MFMAs per K-tile, 12 - 15 pieces and 12 - 15 reads per half) have the
-same phases at their own slots (SCHED_H, SCHED_160, SCHED_192, SCHED_224).  The K offset of the DMA runs through an operand: it starts
-where the caller says and wraps to 0 at %[kend], so that tiles may walk K from different steps.
-MFMA order: H0 = order() over FA0[i] x FB0[j]; H1 = the same over FA1 x FB1.
+  m 103..127 ds_read what tile t+1 begins with (FA*[0], FA*[1], FB*[0..5]) from buffer (t+1)&1, each
+             fragment eight MFMAs behind its last reader
+Lower tiles (128, 160, 192, 224 rows: 64, 80, 96, 112 MFMAs per K-tile, 12 - 15 pieces, 16 reads at the end and 8 - 14 at the
+start) have the same phases at their own slots (SCHED_H, SCHED_160, SCHED_192, SCHED_224).  The K offset of the DMA runs through an operand:
+it starts where the caller says and wraps to 0 at %[kend], so that tiles may walk K from different steps.
+MFMA order: order(), both k-halves of an accumulator one behind the other.
 lgkmcnt waits are derived here from the in-order LDS return queue (each MFMA waits only
 for the fragments it reads).  The last two iterations are peeled: t = nk-2 issues no DMA
 (B2 waits vmcnt(0)), t = nk-1 issues neither DMA nor next-tile reads.
@@ -45,9 +46,9 @@ Half-height variant (BM = 128, round 5): the same schedule shape over 64 MFMAs p
 each wave owns 64 x 128 outputs (4 x 8 accumulators, 128 AGPRs), the A operand is 128 rows
 (4 fragments per k-half, 4 of the 12 LDS-DMA pieces per wave), so a grid has twice the tiles
 (QKV at M = 4088: 768 tiles = 3 whole rounds of the 256 CUs instead of 1.5; O at 1536-2560 rows
-one full round instead of K-half tails).  Slots: rd1 at 1..12, B1 at 20 (8 MFMAs of slack for
-the reads' return), 12 DMAs at 21..43, B2 at 45, rd0 at 46..57 (6 MFMAs of slack before the next
-K-tile's first MFMA); the fragment-reuse distance (>= 8 MFMAs) holds as in the full tile.
+one full round instead of K-half tails).  Slots: reads at 1..12, B1 at 20 (8 MFMAs of slack for
+the reads' return), 12 DMAs at 21..43, B2 at 45, reads from 46 on; the fragment-reuse distance (>= 8
+MFMAs) holds as in the full tile.
 
 Run ``python -m mlopamd.ops.gen_gemm_w4`` to regenerate the header (committed; the build
 does not run Python).
@@ -64,10 +65,11 @@ NFB = 8           # B fragments per k-half (8 x 16 columns: the wave's 128 colum
 class Sched:
     """Slot placement of one K-tile iteration (slot m = before MFMA m) for a tile of ``bm`` rows:
     ``nfa`` = bm / 32 A fragments per wave and k-half, ``na`` = bm / 32 A pieces of the ``npc``
-    LDS-DMA pieces per wave, ``nmma`` MFMAs per K-tile."""
+    LDS-DMA pieces per wave, ``nmma`` MFMAs per K-tile.  ``head`` / ``tail``: (slot, fragment) of the
+    reads of this tile's rest and of the next tile's beginning."""
 
-    def __init__(self, rd1, b1, dma, b2, rd0, toggle1=60, pol_a="", pol_b="", bm=256):
-        self.rd1, self.b1, self.dma, self.b2, self.rd0, self.toggle1 = rd1, b1, dma, b2, rd0, toggle1
+    def __init__(self, b1, dma, b2, pol_a="", pol_b="", bm=256):
+        self.b1, self.dma, self.b2 = b1, dma, b2
         self.pol = {"srdA": pol_a, "srdB": pol_b}  # cache-policy bits of each operand's LDS-DMA
         self.bm = bm
         self.nfa = bm // 32
@@ -75,27 +77,66 @@ class Sched:
         self.npc = self.na + 8
         self.nmma = 2 * self.nfa * NFB
         self.loopctl = self.nmma - 1
-        nrd = NFB + self.nfa
-        assert len(rd1) == nrd and len(rd0) == nrd and len(dma) == self.npc
-        assert max(rd1) < b1 < min(dma) and b2 < min(rd0) and max(rd0) <= self.nmma - 1 and toggle1 > max(rd1)
+        assert len(dma) == self.npc and b1 < min(dma)
         self.dma_before_b2 = sum(1 for m in dma if m < b2)
+        self.seq = [(i, j, h) for i, j in order(self.nfa) for h in (0, 1)]
+        first, last = {}, {}
+        for m, (i, j, h) in enumerate(self.seq):
+            for f in ((f"fa{h}_", i), (f"fb{h}_", j)):
+                first.setdefault(f, m)
+                last[f] = m
+        begin = [f for f in first if f[1] < (2 if f[0][1] == "a" else 6)]  # in the order of first readers
+        rest = [f for f in first if f not in begin]
+        # the first whose register is free eight MFMAs behind its last reader, one a slot (what is left, at the last)
+        self.tail, m = [], b2 + 1
+        while begin:
+            ready = [f for f in begin if last[f] + 8 <= m]
+            for f in ready if m == self.nmma - 1 else ready[:1]:
+                self.tail.append((m, f))
+                begin.remove(f)
+            m += 1
+            assert m <= self.nmma
+        # spread up to seven MFMAs before B1
+        self.head, m, n = [], 1, len(rest)
+        while rest:
+            ready = [f for f in rest if last[f] + 8 - self.nmma <= m]
+            if ready and m >= 1 + len(self.head) * (b1 - 8) // n:
+                self.head.append((m, ready[0]))
+                rest.remove(ready[0])
+            m += 1
+            assert m <= b1 - 6
+        assert all(m < first[f] - 4 for m, f in self.head)
+
+
+def order(nfa):
+    """(i, j) of a K-tile's MFMA pairs: strips of two A fragments (an odd one alone, third), the columns there and back, the
+    strip's two in turn up and down, so that a pair shares a fragment with the one before it and mostly another with the
+    one before that.  The last strip walks its columns upwards, as the next tile's first does: a column's fragments are
+    read again between the two.
+
+    Sustained products are bound by power, and operands that stay take less of it.  Registers only, all CUs, TFLOP/s: one
+    k-half row by row and then the other 2101, row snake 2130, blocks of 2 x 2 2150, of 4 x 4 2128, strips of two (and a Hilbert curve)
+    2166; in another session strips of two 2090, with both k-halves of an accumulator one behind the other 2164 (row by row 2153)."""
+    strips = [[0, 1]] + ([[2]] if nfa % 2 else [])
+    strips += [[i, i + 1] for i in range(2 + nfa % 2, nfa, 2)]
+    out = []
+    for n, strip in enumerate(strips):
+        cols = range(NFB) if n % 2 == 0 or strip is strips[-1] else range(NFB - 1, -1, -1)
+        for c, j in enumerate(cols):
+            out += [(i, j) for i in (strip if c % 2 == 0 else strip[::-1])]
+    return out
 
 
 # All 16 DMAs between the barriers (one per 4 MFMAs), next-tile reads packed at the end.
 # Measured and dropped (profiles/r03_gemm_w4.md): B2 at MFMA 86 with one DMA per 3 MFMAs (within
 # 1 %), and non-temporal weight / activation DMAs (2-8 % slower).
-SCHEDS = [Sched(rd1=[1 + 2 * k for k in range(16)], b1=38, dma=[40 + 4 * k for k in range(16)], b2=102,
-                rd0=[103 + round(k * 24 / 15) for k in range(16)])]
-# the half-height tile (BM = 128): 64 MFMAs, 12 fragment reads per k-half, 12 DMA pieces
-SCHED_H = Sched(rd1=[1 + k for k in range(12)], b1=20, dma=[21 + 2 * k for k in range(12)], b2=45,
-                rd0=[46 + k for k in range(12)], toggle1=19, bm=128)
-# the heights between: 80 / 96 MFMAs, 13 / 14 fragment reads per k-half and DMA pieces
-SCHED_160 = Sched(rd1=[1 + k for k in range(13)], b1=22, dma=[23 + round(2.5 * k) for k in range(13)], b2=57,
-                  rd0=[58 + round(k * 15 / 12) for k in range(13)], toggle1=21, bm=160)
-SCHED_192 = Sched(rd1=[1 + round(k * 16 / 13) for k in range(14)], b1=26, dma=[27 + 3 * k for k in range(14)], b2=70,
-                  rd0=[71 + round(k * 18 / 13) for k in range(14)], toggle1=22, bm=192)
-SCHED_224 = Sched(rd1=[1 + round(k * 24 / 14) for k in range(15)], b1=32, dma=[34 + round(3.5 * k) for k in range(15)], b2=86,
-                  rd0=[87 + round(k * 22 / 14) for k in range(15)], toggle1=28, bm=224)
+SCHEDS = [Sched(b1=38, dma=[40 + 4 * k for k in range(16)], b2=102)]
+# the half-height tile (BM = 128): 64 MFMAs, 12 DMA pieces
+SCHED_H = Sched(b1=20, dma=[21 + 2 * k for k in range(12)], b2=45, bm=128)
+# the heights between: 80 / 96 / 112 MFMAs, 13 / 14 / 15 DMA pieces
+SCHED_160 = Sched(b1=22, dma=[23 + round(2.5 * k) for k in range(13)], b2=57, bm=160)
+SCHED_192 = Sched(b1=26, dma=[27 + 3 * k for k in range(14)], b2=70, bm=192)
+SCHED_224 = Sched(b1=32, dma=[34 + round(3.5 * k) for k in range(15)], b2=86, bm=224)
 
 
 def frag(name, i):
@@ -141,60 +182,20 @@ class Stream:
         self.queue = []
 
 
-def order(sc: Sched):
-    """(i, j) of a k-half's MFMAs: strips of two A fragments (an odd one alone, first), the columns there and back, the
-    strip's two in turn up and down, so that an MFMA shares a fragment with the one before it and mostly another with the
-    one before that.  The last strip walks its columns upwards: FB1 is read again in that order.
-
-    Sustained products are bound by power, and operands that stay take less of it: registers only, all CUs, row by row
-    2101 TFLOP/s, row snake 2130, blocks of 2 x 2 2150, of 4 x 4 2128, so (and along a Hilbert curve) 2166."""
-    strips = [[0]] if sc.nfa % 2 else []
-    strips += [[i, i + 1] for i in range(sc.nfa % 2, sc.nfa, 2)]
-    out = []
-    for n, strip in enumerate(strips):
-        cols = range(NFB) if (len(strips) - 1 - n) % 2 == 0 else range(NFB - 1, -1, -1)
-        for c, j in enumerate(cols):
-            out += [(i, j) for i in (strip if c % 2 == 0 else strip[::-1])]
-    return out
-
-
-def reads_k1(sc: Sched):
-    """ds_reads of the k-half-1 fragments (FB1 then FA1) of the current tile, in the order of their last readers."""
-    return [(("fb1_", j), "rB1", j * 2048) for j in range(NFB)] + [(("fa1_", i), "rA1", i * 2048) for i in range(sc.nfa)]
-
-
-def reads_k0(sc: Sched):
-    """ds_reads of the k-half-0 fragments, in the order of their first readers."""
-    seq = []
-    for i, j in order(sc):
-        seq += [f for f in (("fb0_", j), ("fa0_", i)) if f not in seq]
-    return [(f, "rB0" if f[0] == "fb0_" else "rA0", f[1] * 2048) for f in seq]
-
-
-def check_reuse(sc: Sched):
-    """A fragment is read again at least eight MFMAs behind its last reader."""
-    half = sc.nmma // 2
-    last = {}
-    for m, (i, j) in enumerate(order(sc)):
-        for f in (("fa0_", i), ("fb0_", j)):
-            last[f] = m
-        for f in (("fa1_", i), ("fb1_", j)):
-            last[f] = half + m - sc.nmma  # of the K-tile before
-    for slots, ops in ((sc.rd0, reads_k0(sc)), (sc.rd1, reads_k1(sc))):
-        assert all(m - last[op[0]] >= 8 for m, op in zip(slots, ops))
+def read_of(f):
+    """(fragment, address register, offset) of a fragment's ds_read."""
+    return f, f"r{f[0][1].upper()}{f[0][2]}", f[1] * 2048
 
 
 def body(s: Stream, sc: Sched, kind: str, first: bool = False):
     """One K-tile iteration. kind: steady (DMA t+2, reads t+1), nodma (reads t+1), last.
-    first: the tile's K-tile 0 -- the H0 MFMAs start the accumulators from 0 (no zeroing pass)."""
+    first: the tile's K-tile 0 -- its k-half-0 MFMAs start the accumulators from 0 (no zeroing pass)."""
     dma = kind == "steady"
     nxt = kind != "last"
     NM = sc.nmma
-    check_reuse(sc)
-    seq = order(sc)
     slots: dict[int, list] = {m: [] for m in range(NM + 1)}
-    for m, op in zip(sc.rd1, reads_k1(sc)):
-        slots[m].append(("read", op))
+    for m, f in sc.head:
+        slots[m].append(("read", read_of(f)))
     if dma:
         slots[sc.b1].append(("b1",))
         slots[sc.dma[0] - 1].append(("emit", "s_mov_b32 m0, %[dbase]"))
@@ -207,14 +208,12 @@ def body(s: Stream, sc: Sched, kind: str, first: bool = False):
         slots[sc.dma[-1] + 1].append(("emit", "s_cmp_eq_u32 %[koff], %[kend]"))
         slots[sc.dma[-1] + 1].append(("emit", "s_cselect_b32 %[koff], 0, %[koff]"))
         slots[sc.dma[-1] + 1].append(("emit", "s_xor_b32 %[dbase], %[dbase], 0x10000"))
-    slots[sc.toggle1].append(("emit", "v_xor_b32_e32 %[rA1], 0x10000, %[rA1]"))
-    slots[sc.toggle1].append(("emit", "v_xor_b32_e32 %[rB1], 0x10000, %[rB1]"))
     if nxt:
         slots[sc.b2].append(("b2", sc.dma_before_b2 if dma else 0))
-        slots[sc.b2].append(("emit", "v_xor_b32_e32 %[rA0], 0x10000, %[rA0]"))
-        slots[sc.b2].append(("emit", "v_xor_b32_e32 %[rB0], 0x10000, %[rB0]"))
-        for m, op in zip(sc.rd0, reads_k0(sc)):
-            slots[m].append(("read", op))
+        for r in ("rA0", "rB0", "rA1", "rB1"):  # to the next tile's buffer
+            slots[sc.b2].append(("emit", f"v_xor_b32_e32 %[{r}], 0x10000, %[{r}]"))
+        for m, f in sc.tail:
+            slots[m].append(("read", read_of(f)))
     if kind == "steady" and not first:
         slots[sc.loopctl].append(("emit", "s_sub_u32 %[iter], %[iter], 1"))
         slots[sc.loopctl].append(("emit", "s_cmp_lg_u32 %[iter], 0"))
@@ -233,9 +232,8 @@ def body(s: Stream, sc: Sched, kind: str, first: bool = False):
                 s.emit("s_barrier")
         if m == NM:
             break
-        h, mm = divmod(m, NM // 2)
-        i, j = seq[mm]
-        a, b = (("fa0_", i), ("fb0_", j)) if h == 0 else (("fa1_", i), ("fb1_", j))
+        i, j, h = sc.seq[m]
+        a, b = (f"fa{h}_", i), (f"fb{h}_", j)
         s.need(a, b)
         s.emit(mfma(NFB * i + j, frag(*a), frag(*b), zero_c=first and h == 0))
 
@@ -281,8 +279,8 @@ def kloop(n_stores: int, sc: Sched) -> list[str]:
     s.emit(f"s_waitcnt vmcnt({sc.npc + n_stores})")
     s.emit("L_w4_go_%=:")
     s.emit("s_barrier")
-    for dst, addr, off in reads_k0(sc):
-        s.read(dst, addr, off)
+    for _, f in sc.tail:
+        s.read(*read_of(f))
     q0 = list(s.queue)
     body(s, sc, "steady", first=True)
     assert suffix(s.queue, q0)
