@@ -46,7 +46,7 @@ Half-height variant (BM = 128, round 5): the same schedule shape over 64 MFMAs p
 each wave owns 64 x 128 outputs (4 x 8 accumulators, 128 AGPRs), the A operand is 128 rows
 (4 fragments per k-half, 4 of the 12 LDS-DMA pieces per wave), so a grid has twice the tiles
 (QKV at M = 4088: 768 tiles = 3 whole rounds of the 256 CUs instead of 1.5; O at 1536-2560 rows
-one full round instead of K-half tails).  Slots: reads at 1..12, B1 at 20 (8 MFMAs of slack for
+one full round instead of K-half tails).  Slots: reads at 2..11, B1 at 20 (8 MFMAs of slack for
 the reads' return), 12 DMAs at 21..43, B2 at 45, reads from 46 on; the fragment-reuse distance (>= 8
 MFMAs) holds as in the full tile.
 
@@ -116,7 +116,9 @@ def order(nfa):
 
     Sustained products are bound by power, and operands that stay take less of it.  Registers only, all CUs, TFLOP/s: one
     k-half row by row and then the other 2101, row snake 2130, blocks of 2 x 2 2150, of 4 x 4 2128, strips of two (and a Hilbert curve)
-    2166; in another session strips of two 2090, with both k-halves of an accumulator one behind the other 2164 (row by row 2153)."""
+    2166; in another session strips of two 2090, with both k-halves of an accumulator one behind the other 2164 (row by row 2153).
+    The kernel with one k-half after the other, and with both together, us: 8000 x 28672 x 4096 1305 / 1277, 2048 x 8192 x 28672
+    663 / 646, 704 x 128256 x 4096 596 / 587, 999 x 28672 x 4096 191 / 187.5."""
     strips = [[0, 1]] + ([[2]] if nfa % 2 else [])
     strips += [[i, i + 1] for i in range(2 + nfa % 2, nfa, 2)]
     out = []
