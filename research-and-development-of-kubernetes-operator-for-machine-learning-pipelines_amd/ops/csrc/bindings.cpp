@@ -500,7 +500,7 @@ bool gemm_rs_rope(Tensor q_out, Tensor k_cache, Tensor v_cache, Tensor a, Tensor
   re.ss_eps = (float)eps;
   if (mlop::mid_chain_ok((int)M, (int)N, (int)K, 3)) {  // 5-64 rows
     c10::DeviceGuard g(a.device());
-    if (mlop::ws_prefer((int)M, (int)N, (int)K, 3)) {  // row scale computed from the streamed rows
+    if (mlop::gemm_on_ws((int)M, (int)N, (int)K, 3)) {  // row scale computed from the streamed rows
       mlop::launch_ws(a.data_ptr(), (int)a.stride(0), w.data_ptr(), (int)K, nullptr, 0, (int)M, (int)N, (int)K, 3,
                       true, re, (float)eps, cur_stream());
       return true;

@@ -1696,6 +1696,12 @@ int gemm_rope_split(int set) {
   return g_rope_split_k;
 }
 
+// The weight-streaming kernel (gemm_ws.hip) has this product: where its rule says so, and above the GEMV's rows no switch
+// asks for another form (a plan, one of the small tiles, weights through the caches, which that kernel does not have).
+bool gemm_on_ws(int M, int N, int K, int epi) {
+  return g_dp[0] < 0 && (M <= gemv_chain_max_m() || (g_small_tile == 1 && gemm_weights_nt(1))) && ws_prefer(M, N, K, epi);
+}
+
 static Plan rope_plan(int M, int N, int K) {
   Plan p = plan(M, N, K, false, 0, 0);
   if (p.variant == 7 && p.splits == 1) p = plan(M, N, K, false, 0, 0, false);  // no slabs, and no RoPE epilogue
@@ -1712,7 +1718,7 @@ static bool rope_tiles(const Plan& p) { return p.variant != 7 && (p.BM == 256 ||
 
 bool gemm_rope_supported(int M, int N, int K) {
   if (M <= 0 || N % 128 || K % kBK) return false;
-  if (gemv_takes(M, N, K, EPI_ROPE) || ws_prefer(M, N, K, EPI_ROPE)) return true;  // decode: gemv.hip, gemm_ws.hip
+  if (gemv_takes(M, N, K, EPI_ROPE) || gemm_on_ws(M, N, K, EPI_ROPE)) return true;  // decode: gemv.hip, gemm_ws.hip
   const Plan p = rope_plan(M, N, K);
   return rope_tiles(p) || rope_slabs_ok(p, M, N);
 }
@@ -1721,7 +1727,7 @@ bool launch_gemm_rope(const void* A, int lda, const void* B, int M, int N, int K
                       hipStream_t st) {
   if (M == 0) return true;
   if (!gemm_rope_supported(M, N, K)) return false;
-  if (ws_prefer(M, N, K, EPI_ROPE) && lda % 8 == 0) {  // up to 32 rows: the weight-streaming MFMA kernel
+  if (gemm_on_ws(M, N, K, EPI_ROPE) && lda % 8 == 0) {  // up to 32 rows: the weight-streaming MFMA kernel
     launch_ws(A, lda, B, K, nullptr, 0, M, N, K, EPI_ROPE, false, re, 0.f, st);
     return true;
   }
@@ -1807,7 +1813,7 @@ bool mid_chain_ok(int M, int N, int K, int epi) {
   int cus = 0;
   if (!gemm_sk_available(&cus)) return false;
   if (epi == EPI_ROPE) {
-    if (ws_prefer(M, N, K, EPI_ROPE)) return K % 512 == 0;
+    if (gemm_on_ws(M, N, K, EPI_ROPE)) return K % 512 == 0;
     const Plan p = rope_plan(M, N, K);
     return !rope_tiles(p) && rope_slabs_ok(p, M, N);
   }
@@ -1898,7 +1904,7 @@ void launch_gemm(const void* A, int lda, const void* B, int ldb, void* C, int ld
   re.act = epi_act(epi);
   const int epi0 = epi;
   if (re.act) epi = EPI_NONE;
-  if (ws_prefer(M, N, K, epi) && lda % 8 == 0 && ldb % 8 == 0) {
+  if (gemm_on_ws(M, N, K, epi) && lda % 8 == 0 && ldb % 8 == 0) {
     launch_ws(A, lda, B, ldb, C, ldc, M, N, K, epi, false, re, 0.f, st);
     return;
   }
@@ -1933,7 +1939,7 @@ bool launch_gemm_add_rmsnorm(const void* A, int lda, const void* B, void* out, v
                              int K, hipStream_t st) {
   if (M == 0) return true;
   if (gemv_takes(M, N, K, EPI_NONE)) return false;  // decode sizes: GEMV + add_rmsnorm (or the norm chain)
-  if (ws_prefer(M, N, K, EPI_NONE) && lda % 8 == 0) {
+  if (gemm_on_ws(M, N, K, EPI_NONE) && lda % 8 == 0) {
     // up to 16 rows: the weight-streaming MFMA kernel adds into the residual
     // in place (bf16(res + bf16(y)), norm.hip's rounding), then one RMSNorm pass
     launch_ws(A, lda, B, K, residual, N, M, N, K, 5, false, RopeEpi{}, 0.f, st);

@@ -206,6 +206,8 @@ int gemm_ws_small_m(int set);
 int gemm_ws_rope_m(int set);  // rows up to which QKV + RoPE takes the weight-streaming kernel
 // the decode projections outside the chain that this kernel takes instead of the GEMV or the planner's tiles
 bool ws_prefer(int M, int N, int K, int epi);
+// and no switch asks for another form (gemm.hip)
+bool gemm_on_ws(int M, int N, int K, int epi);
 // mid-M norm chain on the planner's small tiles (gemm.hip): epi 0 = O / down (split-K, the
 // last split adds into the residual and leaves the row sums of squares), 1 = gate_up (SiLU-mul,
 // row-scaled), 3 = QKV + RoPE (row-scaled slab reduce, or the ws kernel at 5-8 rows)
