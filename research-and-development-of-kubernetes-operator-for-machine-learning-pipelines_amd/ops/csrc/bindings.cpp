@@ -293,7 +293,7 @@ bool gemm_sk_reserve() { return mlop::gemm_sk_reserve(); }
 int64_t gemm_sk_workgroups(int64_t M, int64_t N, int64_t K) { return mlop::gemm_sk_workgroups((int)M, (int)N, (int)K); }
 
 int64_t gemm_workspace(int64_t M, int64_t N, int64_t K, int64_t epi) {
-  if (epi == 2) return mlop::gemm_workspace_floats((int)M, (int)N, (int)K, 0);  // GEMM + add + RMSNorm: split-K slabs
+  if (epi == 2) return mlop::gemm_workspace_floats((int)M, (int)N, (int)K, 0, true);  // GEMM + add + RMSNorm
   return mlop::gemm_workspace_floats((int)M, (int)N, (int)K, (int)epi);
 }
 

@@ -1878,6 +1878,10 @@ void launch_mid_self(const void* A, int lda, const void* B, void* out, int ldo, 
 }
 
 void gemm_plan(int M, int N, int K, int out[5]) {
+  if (gemm_on_ws(M, N, K, EPI_NONE)) {
+    out[0] = -2, out[1] = out[2] = 0, out[3] = out[4] = 1;
+    return;
+  }
   if (gemv_takes(M, N, K, EPI_NONE)) {
     out[0] = -1, out[1] = out[2] = out[4] = 0, out[3] = 1;
     return;
@@ -1887,9 +1891,11 @@ void gemm_plan(int M, int N, int K, int out[5]) {
   out[4] = (p.variant == 0 || p.variant == 7) && gemm_weights_nt((M + p.BM - 1) / p.BM);
 }
 
-long gemm_workspace_floats(int M, int N, int K, int epi) {
+// fp32 slabs of the K ranges: of a plain product, and (add_norm) of one with the residual add + RMSNorm behind it, for which 0
+// also says that there is no such form; the weight-streaming kernel's has none, but A's rows may not suit it
+long gemm_workspace_floats(int M, int N, int K, int epi, bool add_norm) {
   if (epi_act(epi)) epi = EPI_NONE;
-  if (gemv_takes(M, N, K, epi)) return 0;
+  if (gemv_takes(M, N, K, epi) || (!add_norm && gemm_on_ws(M, N, K, epi))) return 0;
   const Plan p = plan(M, N, K, false, 0, 0);
   return p.splits > 1 ? (long)p.splits * M * N : 0;
 }
