@@ -1697,9 +1697,9 @@ int gemm_rope_split(int set) {
 }
 
 // The weight-streaming kernel (gemm_ws.hip) has this product: where its rule says so, and above the GEMV's rows no switch
-// asks for another form (a plan, one of the small tiles, weights through the caches, which that kernel does not have).
+// asks for a plan or one of the small tiles.
 bool gemm_on_ws(int M, int N, int K, int epi) {
-  return g_dp[0] < 0 && (M <= gemv_chain_max_m() || (g_small_tile == 1 && gemm_weights_nt(1))) && ws_prefer(M, N, K, epi);
+  return g_dp[0] < 0 && (M <= gemv_chain_max_m() || g_small_tile == 1) && ws_prefer(M, N, K, epi);
 }
 
 static Plan rope_plan(int M, int N, int K) {
@@ -1879,7 +1879,7 @@ void launch_mid_self(const void* A, int lda, const void* B, void* out, int ldo, 
 
 void gemm_plan(int M, int N, int K, int out[5]) {
   if (gemm_on_ws(M, N, K, EPI_NONE)) {
-    out[0] = -2, out[1] = out[2] = 0, out[3] = out[4] = 1;
+    out[0] = -2, out[1] = out[2] = 0, out[3] = 1, out[4] = gemm_weights_nt(1);
     return;
   }
   if (gemv_takes(M, N, K, EPI_NONE)) {

@@ -68,7 +68,7 @@ __device__ __forceinline__ void ws_frags(uint32_t row, uint32_t x0, uint32_t x1,
       : "memory");
 }
 
-template <int AR, int G, int NW, int U, int EPI, bool RS>
+template <int AR, int G, int NW, int U, int EPI, bool RS, bool NT>
 __global__ void __launch_bounds__(NW * 64) gemm_ws_kernel(const uint16_t* __restrict__ A, int lda,
                                                           const uint16_t* __restrict__ B, int ldb,
                                                           uint16_t* __restrict__ C, int ldc, int M, int K,
@@ -160,8 +160,10 @@ __global__ void __launch_bounds__(NW * 64) gemm_ws_kernel(const uint16_t* __rest
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
-      for (int g = 0; g < G; ++g)
-        bq[u][h][g] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(Bw + (bo[g] + k + h * 128)));
+      for (int g = 0; g < G; ++g) {
+        const u32x4* p = reinterpret_cast<const u32x4*>(Bw + (bo[g] + k + h * 128));
+        bq[u][h][g] = NT ? __builtin_nontemporal_load(p) : *p;
+      }
     asm volatile("" ::: "memory");
   };
   // `younger`: steps loaded after this one
@@ -300,13 +302,13 @@ int g_ws_max_m = 16;
 // A / B plan (gemm_ws_plan op, 0 = by shape): 16-row blocks per workgroup (1 / 2) and K-steps in flight per wave (1 / 2)
 int g_ws_rb = 0, g_ws_u = 0;
 
-template <int AR, int G, int U, int EPI, bool RS>
+template <int AR, int G, int U, int EPI, bool RS, bool NT = true>
 void run_ws_k(const uint16_t* A, int lda, const uint16_t* B, int ldb, uint16_t* C, int ldc, int M, int N, int K,
               const RopeEpi& re, float eps, hipStream_t st) {
   constexpr int MT = (AR + 15) / 16, NW = 8;
   constexpr size_t ring = (size_t)NW * U * AR * 256, red = (size_t)NW * MT * (G * 512 + 64), lds = ring > red ? ring : red;
   static_assert(lds <= 163840, "LDS");
-  auto kern = gemm_ws_kernel<AR, G, NW, U, EPI, RS>;
+  auto kern = gemm_ws_kernel<AR, G, NW, U, EPI, RS, NT>;
   static const bool attr =
       hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess;
   (void)attr;
@@ -325,7 +327,13 @@ void run_ws_ar(const uint16_t* A, int lda, const uint16_t* B, int ldb, uint16_t*
   // two steps per wave in flight where there are as many and the images leave a second workgroup its LDS (lm_head at 4 rows
   // 152.2 -> 148.8 us; 16384 x 512 at 4, one step per wave, 5.3 -> 7.0; at 16 rows down 4096 x 14336 23.4 -> 24.0)
   const bool two = g_ws_u ? g_ws_u == 2 : AR <= 8 && K >= 2048;
-#define MLOP_WS(G, U) return run_ws_k<AR, G, U, EPI, RS>(A, lda, B, ldb, C, ldc, M, N, K, re, eps, st)
+#define MLOP_WS(G, U, ...) return run_ws_k<AR, G, U, EPI, RS __VA_ARGS__>(A, lda, B, ldb, C, ldc, M, N, K, re, eps, st)
+  if constexpr (AR <= 32) {  // weights through the caches (gemm_small_nt op); the same sums, whatever is in flight
+    if (!gemm_weights_nt(1)) {
+      if (wide) MLOP_WS(4, 1, , false);
+      MLOP_WS(2, 1, , false);
+    }
+  }
   if constexpr (AR <= 32) {
     if (wide && two) MLOP_WS(4, 2);
     if (two) MLOP_WS(2, 2);

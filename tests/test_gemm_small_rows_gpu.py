@@ -26,7 +26,7 @@ def switches(gpu):
     o.gemm_dense_plan(-1, -1, -1, -1)
 
 
-@pytest.mark.parametrize("switch", [("gemm_small_tile", 32), ("gemm_small_nt", 6), ("gemm_dense_plan", 0, 64, 64, 2)], ids=lambda s: s[0])
+@pytest.mark.parametrize("switch", [("gemm_small_tile", 32), ("gemm_dense_plan", 0, 64, 64, 2)], ids=lambda s: s[0])
 @pytest.mark.parametrize("M", [5, 9, 16])
 @pytest.mark.parametrize("N,K", [(6144, 4096), (4096, 4096)])
 def test_switches_are_followed(gpu, switches, M, N, K, switch):
@@ -43,6 +43,19 @@ def test_switches_are_followed(gpu, switches, M, N, K, switch):
     on = outs()
     torch.ops.mlop.gemm_ws_max_m(0)
     assert all(torch.equal(a, b) for a, b in zip(on, outs()))
+
+
+@pytest.mark.parametrize("M", [2, 4, 8, 16])
+@pytest.mark.parametrize("N,K", [(6144, 4096), (4096, 1152), (8192, 2176)])
+def test_cache_policy_changes_no_bit(gpu, switches, M, N, K):
+    """gemm_small_nt is where the weights go, not which kernel multiplies: one and two steps in flight, 16 and 32 rows."""
+    o, outs = torch.ops.mlop, []
+    x, w = operands(gpu, M, N, K)
+    for nt in (7, 6):
+        o.gemm_small_nt(nt)
+        assert o.gemm_plan(M, N, K) == [-2, 0, 0, 1, nt & 1]
+        outs.append([ops.gemm(x, w), ops.gemm(x, w, epi=ops.EPI_SILU_MUL)])
+    assert all(torch.equal(a, b) for a, b in zip(*outs))
 
 
 @pytest.mark.parametrize("M,N,K", [(1, 4096, 4096), (1, 128256, 4096), (2, 6144, 4096), (2, 2048, 4096), (4, 1024, 4096), (4, 4096, 14336),
