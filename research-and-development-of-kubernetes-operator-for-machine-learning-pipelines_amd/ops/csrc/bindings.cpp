@@ -553,6 +553,8 @@ bool gemm_ws(Tensor out, Tensor a, Tensor w, int64_t epi, bool rs, double eps) {
   return true;
 }
 
+// whether a product of this shape goes to the weight-streaming kernel (epi 0 plain, 1 gate / up, 3 RoPE + cache, 5 residual add)
+bool gemm_on_ws(int64_t M, int64_t N, int64_t K, int64_t epi) { return mlop::gemm_on_ws((int)M, (int)N, (int)K, (int)epi); }
 int64_t gemm_ws_max_m(int64_t set) { return mlop::gemm_ws_max_m((int)set); }
 void gemm_ws_plan(int64_t rb, int64_t u, int64_t nt) { mlop::gemm_ws_plan((int)rb, (int)u, (int)nt); }
 int64_t gemm_ws_small_m(int64_t set) { return mlop::gemm_ws_small_m((int)set); }
@@ -963,6 +965,7 @@ TORCH_LIBRARY(mlop, m) {
   m.def("gemm_split_target(int set=-1) -> int", &gemm_split_target);
   m.def("gemm_grouped_narrow(int set=-1) -> int", &gemm_grouped_narrow);
   m.def("gemm_ws_max_m(int set=-1) -> int", &gemm_ws_max_m);
+  m.def("gemm_on_ws(int M, int N, int K, int epi) -> bool", &gemm_on_ws);
   m.def("decode_chain_max_m() -> int", &decode_chain_max_m);
   m.def("gemm_ws_plan(int rb, int u, int nt) -> ()", &gemm_ws_plan);
   m.def("gemm_ws_small_m(int set=-1) -> int", &gemm_ws_small_m);

@@ -1696,10 +1696,20 @@ int gemm_rope_split(int set) {
   return g_rope_split_k;
 }
 
+// The weight stream of gemm_mid.hip has all tasks of this product in flight at once, each over the whole K.
+static bool mid_one_round(int M, int N, int K) {
+  Plan p{};
+  return mid_plan(M, N, K, p) && p.splits == 1 && (N + p.BN - 1) / p.BN <= kCus;
+}
+
 // The weight-streaming kernel (gemm_ws.hip) has this product: where its rule says so, and above the GEMV's rows no switch
-// asks for a plan or one of the small tiles.
+// asks for a plan or one of the small tiles.  From 9 rows on not where the weight stream's tasks make one round and its own
+// workgroups (of 32 rows there) leave one unfilled: 28672 x 4096 / 8192 at 16 rows 39.7 / 76.7 us against 37.3 / 73.7, 30016 x
+// 5120 54.1 / 48.4, 50304 x 4096 67.7 / 64.6; 24576 and 65536 columns, whole rounds, 0.92 - 1.02 of the weight stream.
 bool gemm_on_ws(int M, int N, int K, int epi) {
-  return g_dp[0] < 0 && (M <= gemv_chain_max_m() || g_small_tile == 1) && ws_prefer(M, N, K, epi);
+  if (g_dp[0] >= 0 || (M > gemv_chain_max_m() && g_small_tile != 1)) return false;
+  if (M > 8 && N % (32 * kCus) && mid_one_round(M, N, K)) return false;
+  return ws_prefer(M, N, K, epi);
 }
 
 static Plan rope_plan(int M, int N, int K) {
@@ -1945,7 +1955,7 @@ bool launch_gemm_add_rmsnorm(const void* A, int lda, const void* B, void* out, v
                              int K, hipStream_t st) {
   if (M == 0) return true;
   if (gemv_takes(M, N, K, EPI_NONE)) return false;  // decode sizes: GEMV + add_rmsnorm (or the norm chain)
-  if (gemm_on_ws(M, N, K, EPI_NONE) && lda % 8 == 0) {
+  if (gemm_on_ws(M, N, K, 5) && lda % 8 == 0) {
     // up to 16 rows: the weight-streaming MFMA kernel adds into the residual
     // in place (bf16(res + bf16(y)), norm.hip's rounding), then one RMSNorm pass
     launch_ws(A, lda, B, K, residual, N, M, N, K, 5, false, RopeEpi{}, 0.f, st);

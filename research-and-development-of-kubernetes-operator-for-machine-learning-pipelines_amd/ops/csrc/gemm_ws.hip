@@ -320,10 +320,11 @@ void run_ws_ar(const uint16_t* A, int lda, const uint16_t* B, int ldb, uint16_t*
                const RopeEpi& re, float eps, hipStream_t st) {
   // 32 weight rows take in half as much of A as 16 do, on half as many workgroups: where 16 make a second round of the CUs
   // and 32 do not (6144 x 4096 at 4 rows 10.6 -> 10.3 us, at 16 13.4 -> 11.8; 5120 x 5120 at 8 14.5 -> 13.2), and from 9 rows on
-  // unless they end in a round half empty (28672 x 4096 at 16 rows 42 -> 39, lm_head 128256 x 4096 184 -> 158; but 10240 x
-  // 8192, 320 workgroups, 34.4 -> 37.2).  Up to 8 rows A costs little: 28672 x 4096 at 8 36.2 against 38.2.
+  // where 16 make more than three (28672 x 4096 at 16 rows 42 -> 39, lm_head 128256 x 4096 184 -> 158; 13824 x 4096 24.0 -> 21.7,
+  // x 5120 31.8 -> 28.3; but 12288 x 4096, 768 workgroups of 16, 19.7 -> 21.2, 10240 x 8192 33.6 -> 36.8).  Up to 8 rows A costs
+  // little: 28672 x 4096 at 8 36.2 against 38.2.
   const int w32 = N / 32;
-  const bool wide = N % 32 == 0 && (g_ws_rb ? g_ws_rb == 2 : N / 16 > kCus && (w32 <= kCus || (M > 8 && w32 >= 7 * kCus / 4)));
+  const bool wide = N % 32 == 0 && (g_ws_rb ? g_ws_rb == 2 : N / 16 > kCus && (w32 <= kCus || (M > 8 && N / 16 > 3 * kCus)));
   // two steps per wave in flight where there are as many and the images leave a second workgroup its LDS (lm_head at 4 rows
   // 152.2 -> 148.8 us; 16384 x 512 at 4, one step per wave, 5.3 -> 7.0; at 16 rows down 4096 x 14336 23.4 -> 24.0)
   const bool two = g_ws_u ? g_ws_u == 2 : AR <= 8 && K >= 2048;
@@ -387,19 +388,34 @@ static bool ws_shape(int M, int N, int K, int epi) {
 // Where it is the faster choice.  Against the GEMV (one to four rows): from 3 rows on, two where the matrix is not narrow, one
 // where it is large (us, GEMV -> here: 6144 x 4096 at 2 / 4 rows 11.3 -> 10.5, 15.1 -> 10.5; 28672 x 4096 at 1 / 2 / 4 36.6 -> 37.2,
 // 36.0 -> 36.5, 43.3 -> 36; 4096 x 14336 at 4 24.4 -> 19.9; 128256 x 4096 at 1 / 4 160 -> 155, 171 -> 150; 128256 x 8192 at 1 336 ->
-// 307; 2048 x 4096 at 2 / 4 6.0 -> 6.6, 7.2 -> 6.2; 1024 x 4096 at 4 5.4 -> 5.8).  Against the planner's tiles and their K ranges' sums (5 to
-// 16): everywhere but where few rows have a long K (6144 x 4096 at 5 / 16 17.7 -> 10.9, 17.7 -> 11.7; 4096 x 4096 with its norm pass 12.1
-// -> 7.6, 12.1 -> 8.5; 8192 x 28672 at 8 105 -> 73; 28672 x 4096 at 8 / 16 39.4 -> 36, 39.6 -> 39; 1024 x 14336 at 8 12.6 -> 16.2, 2048 x 8192
-// at 16 12.4 -> 12.0).  At 24 and 32 rows A is what a CU takes in: 28672 x 4096 40.4 -> 48.5, 4096 x 14336 25 -> 28.
-static bool ws_fast(int M, int N, int K) {
-  if (M == 1) return (long)N * K >= 200L * 1000 * 1000;
-  if (M <= 4) return N >= (M == 2 ? 3072 : 2048);
-  return (long)N * K >= 1 << 20 && (N >= 3072 || K <= 9216);  // (smaller ones are launches, whichever the kernel)
+// 307; 2048 x 4096 at 2 / 4 6.0 -> 6.6, 7.2 -> 6.2; 1024 x 4096 at 4 5.4 -> 5.8).  At two
+// rows not where the last of a few rounds of workgroups is nearly empty, short K aside (4256 x 4736 9.8 -> 10.6, 8480 x 11136 32.8
+// -> 36.0, 12704 x 8192 33.6 -> 37.0).
+//   Against the planner's tiles and their K ranges' sums (5 to 16 rows), where a workgroup's walk of the whole K is no longer
+// than those: it takes in 16 weight rows and A, and few workgroups cannot make up for it.  Measured at 5 - 16 rows on 120 shapes,
+// here over there: narrow ones (128 - 1024 columns) at K 6144 0.80 - 0.98, at 8192 0.82 / 0.92 / 0.99 / 1.05 at 5 / 9 / 12 / 16 rows, at 9216
+// 0.94 / 1.02 / 1.10 / 1.17; 1280 - 2048 columns at 8192 0.80 - 0.98, at 9216 0.90 / 0.95 / 1.02 / 1.07; 3072 x 14336 0.88 / 0.95 / 1.01 /
+// 1.06, 3072 x 28672 0.96 / 1.05 / 1.11 / 1.17, 4096 x 28672 0.91 / 0.94 / 0.99 / 1.03; 5120 - 22016 columns 0.46 - 0.98, but 4112 -
+// 5104, a second round for a few workgroups, 0.98 / 1.06 / 1.1 at K 9000 / 10000 / 14000 and 5 - 8 rows, 1.02 / 1.06 / 1.16 at 7300 / 9000 /
+// 11000 and 11.  Short K under many columns are launches of thousands of short workgroups: 16384 x 256 / 512 / 1024 1.10 / 1.12 / 1.0, 65536 x 256 / 512 / 768 /
+// 1024 1.30 / 1.15 / 1.04 / 0.9.  At 24 and 32 rows A is what a CU takes in: 28672 x 4096 40.4 -> 48.5, 4096 x 14336 25 -> 28.
+static bool ws_fast(int M, int N, int K, int epi) {
+  const long nk = (long)N * K, mk = (long)M * K;
+  const int w = N / 16;  // workgroups of 16 rows
+  if (M == 1) return nk >= 200L * 1000 * 1000;
+  if (M == 2) return N >= 3072 && (K <= 2560 || w % kCus == 0 || w < kCus || w > 4 * kCus || w % kCus >= (w < 2 * kCus ? 64 : 128));
+  if (M <= 4) return N >= 2048;
+  if (nk < 1 << 20) return false;  // (launches, whichever the kernel)
+  if (epi == WS_RES || epi == WS_ROPE) return N >= 3072 || K <= 9216;
+  if (N >= 16384 && K < 1024) return false;
+  if (w > kCus && w < kCus + 64) return K <= (M > 8 ? 7168 : 9216);
+  if (N >= 3072) return mk <= 190L * (N - 2100);
+  return K <= 9216 && 1024L * M + 5L * K <= (N < 1280 ? 53760 : 57500);
 }
 
 bool ws_prefer(int M, int N, int K, int epi) {
   const int bound = epi == WS_ROPE ? (g_ws_max_m ? g_ws_rope_m : 0) : std::min(g_ws_max_m, g_ws_small_m);
-  return M <= bound && ws_shape(M, N, K, epi) && ws_fast(M, N, K);
+  return M <= bound && ws_shape(M, N, K, epi) && ws_fast(M, N, K, epi);
 }
 
 // (the third argument chose a form of the weight loads that is no more)
@@ -414,7 +430,7 @@ int decode_chain_max_m() { return g_ws_max_m > gemv_chain_max_m() ? g_ws_max_m :
 
 // the chain's product of this shape on this kernel rather than the GEMV
 bool chain_on_ws(int M, int N, int K, int epi) {
-  return ws_takes(M, N, K, epi) && (M > gemv_chain_max_m() || ws_fast(M, N, K));
+  return ws_takes(M, N, K, epi) && (M > gemv_chain_max_m() || ws_fast(M, N, K, epi));
 }
 
 // and gate_up on gemm_mid.hip's stream, where that takes it: above 8 rows A is what a CU of this kernel takes in (28672 x

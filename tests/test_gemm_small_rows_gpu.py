@@ -59,7 +59,7 @@ def test_cache_policy_changes_no_bit(gpu, switches, M, N, K):
 
 
 @pytest.mark.parametrize("M,N,K", [(1, 4096, 4096), (1, 128256, 4096), (2, 6144, 4096), (2, 2048, 4096), (4, 1024, 4096), (4, 4096, 14336),
-                                   (5, 6144, 4096), (16, 28672, 4096), (16, 6144, 4160), (16, 256, 1024), (17, 6144, 4096)])
+                                   (5, 6144, 4096), (16, 24576, 4096), (16, 6144, 4160), (16, 256, 1024), (17, 6144, 4096)])
 def test_plan_says_what_runs(gpu, switches, M, N, K):
     """gemm_plan's -2 is where a plain product is the weight-streaming kernel's, bit for bit, with no slabs reserved; without
     that kernel it names another form, whose product is in another order."""
@@ -71,9 +71,9 @@ def test_plan_says_what_runs(gpu, switches, M, N, K):
         assert o.gemm_ws(z, x, w, 0, False, 0.0) and torch.equal(y, z)
         assert o.gemm_workspace(M, N, K, 0) == 0
         o.gemm_ws_max_m(0)
-        assert o.gemm_plan(M, N, K)[0] == (-1 if M <= 4 else 0 if N < 28672 else 7)
+        assert o.gemm_plan(M, N, K)[0] == (-1 if M <= 4 else 0 if N < 24449 else 7)
     else:
         o.gemm_ws_max_m(0)
         assert o.gemm_plan(M, N, K)[0] == variant and torch.equal(ops.gemm(x, w), y)
-    assert (variant == -2) == ((M, N, K) in [(1, 128256, 4096), (2, 6144, 4096), (4, 4096, 14336), (5, 6144, 4096), (16, 28672, 4096),
+    assert (variant == -2) == ((M, N, K) in [(1, 128256, 4096), (2, 6144, 4096), (4, 4096, 14336), (5, 6144, 4096), (16, 24576, 4096),
                                              (16, 6144, 4096)])
