@@ -399,6 +399,10 @@ static bool ws_shape(int M, int N, int K, int epi) {
 // 5104, a second round for a few workgroups, 0.98 / 1.06 / 1.1 at K 9000 / 10000 / 14000 and 5 - 8 rows, 1.02 / 1.06 / 1.16 at 7300 / 9000 /
 // 11000 and 11.  Short K under many columns are launches of thousands of short workgroups: 16384 x 256 / 512 / 1024 1.10 / 1.12 / 1.0, 65536 x 256 / 512 / 768 /
 // 1024 1.30 / 1.15 / 1.04 / 0.9.  At 24 and 32 rows A is what a CU takes in: 28672 x 4096 40.4 -> 48.5, 4096 x 14336 25 -> 28.
+//   With the residual add and a norm behind it, the planner's K ranges have the norm in the launch that sums them and this kernel a
+// launch of its own: 512 x 2048 / 4096 / 8192 at 16 rows 0.97 / 1.17 / 1.38 (at 5 0.89 / 1.01 / 1.13), 1024 x 4096 1.14 (1.01), 2048 x 4096 /
+// 8192 1.0 / 1.16 (0.89 / 0.98), 3072 x 8192 / 9216 1.0 / 1.09 (0.87 / 0.96), 3584 and 4096 x 14336 1.03 (0.93), 4352 x 3328 /
+// 5120 / 14336 1.0 / 1.05 / 1.19, 5120 and more columns 0.54 - 0.86.
 static bool ws_fast(int M, int N, int K, int epi) {
   const long nk = (long)N * K, mk = (long)M * K;
   const int w = N / 16;  // workgroups of 16 rows
@@ -406,9 +410,15 @@ static bool ws_fast(int M, int N, int K, int epi) {
   if (M == 2) return N >= 3072 && (K <= 2560 || w % kCus == 0 || w < kCus || w > 4 * kCus || w % kCus >= (w < 2 * kCus ? 64 : 128));
   if (M <= 4) return N >= 2048;
   if (nk < 1 << 20) return false;  // (launches, whichever the kernel)
-  if (epi == WS_RES || epi == WS_ROPE) return N >= 3072 || K <= 9216;
+  if (epi == WS_ROPE) return N >= 3072 || K <= 9216;
+  const bool second = w > kCus && w < kCus + 64;  // (workgroups of a second round that leave most CUs idle)
+  if (epi == WS_RES) {
+    if (second) return K <= 3072;
+    if (N >= 3072) return N >= 5120 || (N >= 3584 ? mk <= 45L * N : mk < 36L * N);
+    return K <= 2048 || (K <= 9216 && mk <= (N <= 1536 ? 24L : 28L) * N);
+  }
   if (N >= 16384 && K < 1024) return false;
-  if (w > kCus && w < kCus + 64) return K <= (M > 8 ? 7168 : 9216);
+  if (second) return K <= (M > 8 ? 7168 : 9216);
   if (N >= 3072) return mk <= 190L * (N - 2100);
   return K <= 9216 && 1024L * M + 5L * K <= (N < 1280 ? 53760 : 57500);
 }
