@@ -403,20 +403,26 @@ static bool ws_shape(int M, int N, int K, int epi) {
 // launch of its own: 512 x 2048 / 4096 / 8192 at 16 rows 0.97 / 1.17 / 1.38 (at 5 0.89 / 1.01 / 1.13), 1024 x 4096 1.14 (1.01), 2048 x 4096 /
 // 8192 1.0 / 1.16 (0.89 / 0.98), 3072 x 8192 / 9216 1.0 / 1.09 (0.87 / 0.96), 3584 and 4096 x 14336 1.03 (0.93), 4352 x 3328 /
 // 5120 / 14336 1.0 / 1.05 / 1.19, 5120 and more columns 0.54 - 0.86.
+//   QKV + RoPE at 17 - 32 rows, where A is most of what a CU takes in, against K ranges and the launch that sums, rotates and stores them
+// (34 numbers of heads, K 512 - 8192): K up to 4096 0.5 - 1.0; 768 - 2048 columns at 17 / 24 / 32 rows with K 5120 0.95 / 1.0 / 1.05, 6144
+// 0.97 / 1.04 / 1.1, 8192 1.03 / 1.12 / 1.2; 3072 0.9 / 0.94 / 1.03 with 8192; 4352 - 5376 columns, a second round for few, 1.0 - 1.1 from
+// 5120 on; 5632 - 8192 0.8 - 0.98; more at K 5120 - 7168 0.92 / 0.97 / 1.05, at 8192 0.88 / 0.94 / 1.0.
 static bool ws_fast(int M, int N, int K, int epi) {
   const long nk = (long)N * K, mk = (long)M * K;
   const int w = N / 16;  // workgroups of 16 rows
   if (M == 1) return nk >= 200L * 1000 * 1000;
   if (M == 2) return N >= 3072 && (K <= 2560 || w % kCus == 0 || w < kCus || w > 4 * kCus || w % kCus >= (w < 2 * kCus ? 64 : 128));
   if (M <= 4) return N >= 2048;
-  if (nk < 1 << 20) return false;  // (launches, whichever the kernel)
-  if (epi == WS_ROPE) return N >= 3072 || K <= 9216;
+  if (nk < 1 << 20) return epi == WS_ROPE && M <= 8 && K % 512 == 0;  // (launches, whichever the kernel; here one less)
   const bool second = w > kCus && w < kCus + 64;  // (workgroups of a second round that leave most CUs idle)
   if (epi == WS_RES) {
     if (second) return K <= 3072;
     if (N >= 3072) return N >= 5120 || (N >= 3584 ? mk <= 45L * N : mk < 36L * N);
     return K <= 2048 || (K <= 9216 && mk <= (N <= 1536 ? 24L : 28L) * N);
   }
+  if (epi == WS_ROPE && M > 16)
+    return K <= 4096 || (N <= 4096 ? K <= 8192 && mk <= (N < 3072 ? 60L : 64L) * N : N >= 5632 && (N <= 8192 || K % 4096 == 0 || mk <= 150000));
+  if (epi == WS_ROPE && N <= 1280) return K <= 9216 && mk <= 100000;
   if (N >= 16384 && K < 1024) return false;
   if (second) return K <= (M > 8 ? 7168 : 9216);
   if (N >= 3072) return mk <= 190L * (N - 2100);
