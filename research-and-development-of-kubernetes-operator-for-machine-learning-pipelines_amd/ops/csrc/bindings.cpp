@@ -389,6 +389,13 @@ static bool decode_form(int64_t M, int64_t N, int64_t K, int64_t epi) {
   return M <= mlop::gemv_chain_max_m() ||
          (M <= mlop::decode_chain_max_m() && mlop::decode_chain_takes((int)M, (int)N, (int)K, (int)epi));
 }
+// and whether they take these rows: above the GEMV's, where both kernels read them by LDS-DMA
+static bool decode_rows(const Tensor& a) {
+  return a.size(0) <= mlop::gemv_chain_max_m() || mlop::ws_rows_ok(a.data_ptr(), (int)a.stride(0));
+}
+static bool decode_on_ws(const Tensor& a, int64_t N, int64_t K, int64_t epi) {
+  return mlop::chain_on_ws((int)a.size(0), (int)N, (int)K, (int)epi) && mlop::ws_rows_ok(a.data_ptr(), (int)a.stride(0));
+}
 
 bool gemm_res_ss(Tensor residual, Tensor a, Tensor w, Tensor ss_out, bool any) {
   TORCH_CHECK(a.is_cuda() && a.scalar_type() == at::kBFloat16 && a.dim() == 2 && a.stride(1) == 1 &&
@@ -402,9 +409,9 @@ bool gemm_res_ss(Tensor residual, Tensor a, Tensor w, Tensor ss_out, bool any) {
   check_ss(ss_out, M, N, "ss");
   if (decode_form(M, N, K, 0)) {  // the GEMV / weight-streaming MFMA chain
                  // (EPI_RES); its consumers take their row factors from the residual itself, so ss_out is not written
-    if (residual.stride(0) != N || !mlop::decode_chain_takes((int)M, (int)N, (int)K, 0)) return false;
+    if (residual.stride(0) != N || !decode_rows(a) || !mlop::decode_chain_takes((int)M, (int)N, (int)K, 0)) return false;
     c10::DeviceGuard g(a.device());
-    if (!mlop::chain_on_ws((int)M, (int)N, (int)K, 5))
+    if (!decode_on_ws(a, N, K, 5))
       mlop::launch_gemv_res(a.data_ptr(), (int)a.stride(0), w.data_ptr(), residual.data_ptr(), (int)M, (int)N,
                             (int)K, cur_stream());
     else
@@ -437,12 +444,12 @@ bool gemm_rs(Tensor out, Tensor a, Tensor w, Tensor ss_in, double eps, int64_t e
   TORCH_CHECK(K % 128 == 0, "K % 128");
   check_ss(ss_in, M, K, "ss");
   if (decode_form(M, N, K, epi)) {  // PRO_RS, row factors from the streamed chunks (ss_in unused)
-    if (!mlop::decode_chain_takes((int)M, (int)N, (int)K, (int)epi)) return false;
+    if (!decode_rows(a) || !mlop::decode_chain_takes((int)M, (int)N, (int)K, (int)epi)) return false;
     c10::DeviceGuard g(a.device());
     if (epi == 1 && mlop::chain_on_mid((int)M, (int)N, (int)K))
       mlop::launch_mid_self(a.data_ptr(), (int)a.stride(0), w.data_ptr(), out.data_ptr(), (int)out.stride(0), (int)M, (int)N,
                             (int)K, (float)eps, cur_stream());
-    else if (!mlop::chain_on_ws((int)M, (int)N, (int)K, (int)epi))
+    else if (!decode_on_ws(a, N, K, epi))
       mlop::launch_gemv_rs(a.data_ptr(), (int)a.stride(0), w.data_ptr(), out.data_ptr(), (int)out.stride(0), (int)M,
                            (int)N, (int)K, (int)epi, mlop::RopeEpi{}, (float)eps, cur_stream());
     else
@@ -485,9 +492,9 @@ bool gemm_rs_rope(Tensor q_out, Tensor k_cache, Tensor v_cache, Tensor a, Tensor
                    (uint16_t*)v_cache.data_ptr(), pos.data_ptr<int>(), cos_sin.data_ptr<float>(),
                    slots.data_ptr<int>(), (int)Hq, (int)Hkv, (int)BS};
   if (decode_form(M, N, K, 3)) {  // PRO_RS + the RoPE / paged K/V epilogue (ss_in unused)
-    if (!mlop::decode_chain_takes((int)M, (int)N, (int)K, 3)) return false;
+    if (!decode_rows(a) || !mlop::decode_chain_takes((int)M, (int)N, (int)K, 3)) return false;
     c10::DeviceGuard g(a.device());
-    if (!mlop::chain_on_ws((int)M, (int)N, (int)K, 3))
+    if (!decode_on_ws(a, N, K, 3))
       mlop::launch_gemv_rs(a.data_ptr(), (int)a.stride(0), w.data_ptr(), nullptr, 0, (int)M, (int)N, (int)K, 3, re,
                            (float)eps, cur_stream());
     else
@@ -500,7 +507,7 @@ bool gemm_rs_rope(Tensor q_out, Tensor k_cache, Tensor v_cache, Tensor a, Tensor
   re.ss_eps = (float)eps;
   if (mlop::mid_chain_ok((int)M, (int)N, (int)K, 3)) {  // 5-64 rows
     c10::DeviceGuard g(a.device());
-    if (mlop::gemm_on_ws((int)M, (int)N, (int)K, 3)) {  // row scale computed from the streamed rows
+    if (mlop::gemm_on_ws((int)M, (int)N, (int)K, 3) && mlop::ws_rows_ok(a.data_ptr(), (int)a.stride(0))) {  // row scale computed from the streamed rows
       mlop::launch_ws(a.data_ptr(), (int)a.stride(0), w.data_ptr(), (int)K, nullptr, 0, (int)M, (int)N, (int)K, 3,
                       true, re, (float)eps, cur_stream());
       return true;
@@ -546,7 +553,7 @@ bool gemm_ws(Tensor out, Tensor a, Tensor w, int64_t epi, bool rs, double eps) {
   TORCH_CHECK(out.dim() == 2 && out.size(0) == M && out.size(1) == (epi == 1 ? N / 2 : N) && out.stride(1) == 1,
               "out [M, N or N/2]");
   TORCH_CHECK(!(rs && epi == 5), "residual form has no row scale");
-  if (!mlop::ws_takes((int)M, (int)N, (int)K, (int)epi)) return false;
+  if (!mlop::ws_rows_ok(a.data_ptr(), (int)a.stride(0)) || !mlop::ws_takes((int)M, (int)N, (int)K, (int)epi)) return false;
   c10::DeviceGuard g(a.device());
   mlop::launch_ws(a.data_ptr(), (int)a.stride(0), w.data_ptr(), (int)K, out.data_ptr(), (int)out.stride(0), (int)M,
                   (int)N, (int)K, (int)epi, rs, mlop::RopeEpi{}, (float)eps, cur_stream());

@@ -77,3 +77,31 @@ def test_plan_says_what_runs(gpu, switches, M, N, K):
         assert o.gemm_plan(M, N, K)[0] == variant and torch.equal(ops.gemm(x, w), y)
     assert (variant == -2) == ((M, N, K) in [(1, 128256, 4096), (2, 6144, 4096), (4, 4096, 14336), (5, 6144, 4096), (16, 24576, 4096),
                                              (16, 6144, 4096)])
+
+
+@pytest.mark.parametrize("M", [2, 3, 4])
+def test_rows_off_16_bytes_stay_on_the_gemv(gpu, switches, M):
+    """Rows that begin 8 bytes off a multiple of 16 are not for LDS-DMA: QKV + RoPE and the chain's products of up to 4 rows are
+    the GEMV's there, bit for bit, and the chain's of more rows are refused."""
+    from mlopamd.models.layers import rope_table
+
+    o, K, hq, hkv = torch.ops.mlop, 4096, 32, 8
+    N = (hq + 2 * hkv) * 128
+    x, w = operands(gpu, 8, 8, K + 8)[0][:, 4:4 + K], operands(gpu, 1, N, K)[1]
+    assert x.data_ptr() % 16 == 8 and x.stride(0) % 8 == 0
+    cs = rope_table(128, 64, 10000.0, device=gpu)
+    pos, slots = torch.arange(M, device=gpu, dtype=torch.int32), torch.arange(M, device=gpu, dtype=torch.int32)
+
+    def outs(a):
+        kc, vc = (torch.zeros(2, hkv, 16, 128, device=gpu, dtype=bf) for _ in range(2))
+        r, ss = torch.ones(M, K, device=gpu, dtype=bf), ops.ss_buffer(M, K, gpu)
+        q = ops.qkv_rope_cache(a, w, pos, cs, slots, kc, vc, hq)
+        q2 = ops.qkv_rope_cache_rs(a, w, pos, cs, slots, kc.clone(), vc.clone(), hq, ss, 1e-5)
+        ops.gemm_res_ss(a, w[:K], r, ss)
+        return q, kc, vc, q2, r, ops.gemm_rs(a, w, ss, 1e-5, ops.EPI_SILU_MUL)
+
+    here = outs(x[:M])
+    with pytest.raises(RuntimeError):
+        ops.gemm_rs(x, w, ops.ss_buffer(8, K, gpu), 1e-5, ops.EPI_SILU_MUL)
+    o.gemm_ws_max_m(0)
+    assert all(torch.equal(a, b) for a, b in zip(here, outs(x[:M].clone())))
