@@ -163,6 +163,7 @@ class LlamaModel:
         # TP > 1: the decode (GEMV) form only, its residual adds riding in the all-reduces
         dmax = ops.decode_chain_max_m() if tp.size == 1 else ops.GEMV_CHAIN_MAX_M  # the GEMV / weight-streaming MFMA forms
         chain = (tp.size == 1 or M <= dmax) and self._chain_ok(M, meta.like)
+        any_tile = meta.like > 0 and M > dmax  # (the decode form has no row sums to keep)
         ss = None  # norm chain: x is None and ss holds the residual's row partials
         if chain and M <= dmax:
             # decode form: the QKV GEMV takes the embedding rows' factors itself (ss unused)
@@ -175,14 +176,14 @@ class LlamaModel:
                                        self.n_q)
             else:
                 q = ops.qkv_rope_cache_rs(residual, L["qkv"], meta.positions, self.cos_sin, meta.slots, kv.k[i],
-                                          kv.v[i], self.n_q, ss, eps, meta.like > 0)
+                                          kv.v[i], self.n_q, ss, eps, any_tile)
             a = ops.paged_attention(q, kv.k[i], kv.v[i], meta)
             nxt = self.layers[i + 1]["in_norm"] if i + 1 < len(self.layers) else self.final_norm
             if chain and tp.size > 1:
                 x, ss = self._chain_layer_tp(i, a.view(a.shape[0], -1), residual, i + 1 == len(self.layers), eps, ss)
                 continue
             if chain:
-                x, ss = self._chain_layer(i, a.view(a.shape[0], -1), residual, i + 1 == len(self.layers), eps, meta.like > 0)
+                x, ss = self._chain_layer(i, a.view(a.shape[0], -1), residual, i + 1 == len(self.layers), eps, any_tile)
                 continue
             if tp.size == 1:
                 x = self.attn_out_mlp(i, a.view(a.shape[0], -1), residual, nxt, eps)

@@ -384,10 +384,11 @@ static void check_ss(const Tensor& ss, int64_t M, int64_t H, const char* name) {
                   ss.numel() == M * (H / 128 + 1), name, " must be f32 [M * (H / 128 + 1)] contiguous");
 }
 
-// sizes of the decode form of the chain: the GEMV's rows, and above them what the weight-streaming kernel takes
-static bool decode_form(int64_t M, int64_t N, int64_t K, int64_t epi) {
+// sizes of the decode form of the chain: the GEMV's rows, and above them what the weight-streaming kernel takes, unless the
+// four-wave form with its row sums is asked for (any)
+static bool decode_form(int64_t M, int64_t N, int64_t K, int64_t epi, bool any) {
   return M <= mlop::gemv_chain_max_m() ||
-         (M <= mlop::decode_chain_max_m() && mlop::decode_chain_takes((int)M, (int)N, (int)K, (int)epi));
+         (!any && M <= mlop::decode_chain_max_m() && mlop::decode_chain_takes((int)M, (int)N, (int)K, (int)epi));
 }
 // and whether they take these rows: above the GEMV's, where both kernels read them by LDS-DMA
 static bool decode_rows(const Tensor& a) {
@@ -407,7 +408,7 @@ bool gemm_res_ss(Tensor residual, Tensor a, Tensor w, Tensor ss_out, bool any) {
                   residual.stride(0) % 8 == 0, "residual [M, N]");
   TORCH_CHECK(N % 128 == 0, "N % 128");
   check_ss(ss_out, M, N, "ss");
-  if (decode_form(M, N, K, 0)) {  // the GEMV / weight-streaming MFMA chain
+  if (decode_form(M, N, K, 0, any)) {  // the GEMV / weight-streaming MFMA chain
                  // (EPI_RES); its consumers take their row factors from the residual itself, so ss_out is not written
     if (residual.stride(0) != N || !decode_rows(a) || !mlop::decode_chain_takes((int)M, (int)N, (int)K, 0)) return false;
     c10::DeviceGuard g(a.device());
@@ -443,7 +444,7 @@ bool gemm_rs(Tensor out, Tensor a, Tensor w, Tensor ss_in, double eps, int64_t e
                   out.stride(0) % 8 == 0, "out [M, N or N/2]");
   TORCH_CHECK(K % 128 == 0, "K % 128");
   check_ss(ss_in, M, K, "ss");
-  if (decode_form(M, N, K, epi)) {  // PRO_RS, row factors from the streamed chunks (ss_in unused)
+  if (decode_form(M, N, K, epi, any)) {  // PRO_RS, row factors from the streamed chunks (ss_in unused)
     if (!decode_rows(a) || !mlop::decode_chain_takes((int)M, (int)N, (int)K, (int)epi)) return false;
     c10::DeviceGuard g(a.device());
     if (epi == 1 && mlop::chain_on_mid((int)M, (int)N, (int)K))
@@ -491,7 +492,7 @@ bool gemm_rs_rope(Tensor q_out, Tensor k_cache, Tensor v_cache, Tensor a, Tensor
   mlop::RopeEpi re{(uint16_t*)q_out.data_ptr(), (uint16_t*)k_cache.data_ptr(),
                    (uint16_t*)v_cache.data_ptr(), pos.data_ptr<int>(), cos_sin.data_ptr<float>(),
                    slots.data_ptr<int>(), (int)Hq, (int)Hkv, (int)BS};
-  if (decode_form(M, N, K, 3)) {  // PRO_RS + the RoPE / paged K/V epilogue (ss_in unused)
+  if (decode_form(M, N, K, 3, any)) {  // PRO_RS + the RoPE / paged K/V epilogue (ss_in unused)
     if (!decode_rows(a) || !mlop::decode_chain_takes((int)M, (int)N, (int)K, 3)) return false;
     c10::DeviceGuard g(a.device());
     if (!decode_on_ws(a, N, K, 3))

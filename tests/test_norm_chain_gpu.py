@@ -316,3 +316,24 @@ def test_chain_where_another_kernel_is_the_choice(gpu, M):
     xf = x.float() * torch.rsqrt(x.float().pow(2).mean(-1, keepdim=True) + EPS)
     bound = 2.0 ** -8 * (xf @ w.float().t()).abs() + 2.0 ** -19 * (xf.abs() @ w.float().abs().t())
     assert ((y.float() - xf @ w.float().t()).abs() <= bound + 1e-6).all()
+
+
+@pytest.mark.parametrize("M", [5, 9, 16])
+def test_any_tile_at_decode_rows(gpu, M):
+    """``any_tile`` is the four-wave form, which leaves the row sums and takes them, also at rows that the decode form has."""
+    ops._sk_reserve(torch.device(gpu))
+    torch.manual_seed(M)
+    a, r = torch.randn(M, H, device=gpu, dtype=bf), torch.randn(M, H, device=gpu, dtype=bf)
+    w = (0.02 * torch.randn(H, H, device=gpu)).to(bf)
+    exp, ss = r.float() + a.float() @ w.float().t(), ops.ss_buffer(M, H, gpu).fill_(float("nan"))
+    ops.gemm_res_ss(a, w, r, ss, True)
+    sums = 2.0 ** -20 * (a.float().abs() @ w.float().abs().t())  # fp32 sums in another order
+    assert ((r.float() - exp).abs() <= 2.0 ** -8 * exp.abs() + 2 * sums + 1e-6).all()
+    part, tot = ops.ss_parts(ss, M, H)
+    close(part, r.float().pow(2).view(M, H // 128, 128).sum(-1), atol=1e-3, rtol=1e-4)
+    close(tot, r.float().pow(2).sum(-1), atol=1e-2, rtol=1e-4)
+    tot.mul_(4)  # what they hold is what scales the rows
+    y = ops.gemm_rs(r, w, ss, EPS, any_tile=True)
+    xf = r.float() * torch.rsqrt(4 * r.float().pow(2).mean(-1, keepdim=True) + EPS)
+    bound = 2.0 ** -8 * (xf @ w.float().t()).abs() + 2.0 ** -19 * (xf.abs() @ w.float().abs().t())
+    assert ((y.float() - xf @ w.float().t()).abs() <= bound + 1e-6).all()
