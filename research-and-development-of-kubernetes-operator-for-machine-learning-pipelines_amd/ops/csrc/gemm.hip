@@ -1805,8 +1805,8 @@ bool launch_w4_chain(int epi, const void* A, int lda, const void* B, void* C, in
 // (epi 0) split K and the tile's last split adds into the residual and leaves the row sums of
 // squares (mid_chain_finish); gate_up (epi 1, one K range) scales its accumulator rows by the
 // RMSNorm factor in its SiLU epilogue; QKV + RoPE (epi 3) takes the factor in the split-K slab
-// reduce of the RoPE + cache kernel, or in the weight-streaming kernel's row-scale prologue at
-// 5-8 rows (which computes it from the rows it streams).
+// reduce of the RoPE + cache kernel, or in the weight-streaming kernel's row-scale prologue at up
+// to 32 rows (which computes it from the rows it streams).
 // gemm_mid_chain op: 0 off (default), 1 on (sc1 hand-off), 2 on (acquire hand-off).  Off by
 // default: the in-kernel finish adds ~3.5 us to each O / down call (two ticket round trips,
 // write-through partials, the band's row totals) against the ~5 us splitk_add_rmsnorm launch it
@@ -1824,7 +1824,7 @@ bool mid_chain_ok(int M, int N, int K, int epi) {
   int cus = 0;
   if (!gemm_sk_available(&cus)) return false;
   if (epi == EPI_ROPE) {
-    if (gemm_on_ws(M, N, K, EPI_ROPE)) return K % 512 == 0;
+    if (gemm_on_ws(M, N, K, EPI_ROPE)) return true;  // (whole steps of 128 k are part of its rule)
     const Plan p = rope_plan(M, N, K);
     return !rope_tiles(p) && rope_slabs_ok(p, M, N);
   }

@@ -212,7 +212,7 @@ inline bool ws_rows_ok(const void* A, int lda) { return lda % 8 == 0 && reinterp
 bool gemm_on_ws(int M, int N, int K, int epi);
 // mid-M norm chain on the planner's small tiles (gemm.hip): epi 0 = O / down (split-K, the
 // last split adds into the residual and leaves the row sums of squares), 1 = gate_up (SiLU-mul,
-// row-scaled), 3 = QKV + RoPE (row-scaled slab reduce, or the ws kernel at 5-8 rows)
+// row-scaled), 3 = QKV + RoPE (row-scaled slab reduce, or the ws kernel at up to 32 rows)
 int gemm_mid_chain(int set);
 bool mid_chain_ok(int M, int N, int K, int epi);
 bool launch_mid_res_ss(const void* A, int lda, const void* B, void* residual, int ldr, int M, int N, int K,

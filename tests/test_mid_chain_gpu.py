@@ -150,3 +150,36 @@ def test_llama_decode_mid_chain_on_off(gpu, mid, batch):
                 best = int(lg.argmax())
                 assert t == best or float(lg[best] - lg[t]) < 0.1 * float(lg.std()), (on, len(toks), best, t)
                 toks.append(t)
+
+
+@pytest.mark.parametrize("M", [17, 24, 32])
+@pytest.mark.parametrize("hq,hkv,K", [(18, 3, 2304), (32, 8, 4096), (44, 4, 2688)])
+def test_mid_rs_rope_on_the_weight_streaming_kernel(gpu, M, hq, hkv, K):
+    """QKV + RoPE of the mid chain where that kernel has it (it is on, as in serving): its row factors are those of the rows it
+    streams, K of whole 128, not only of whole 512; what ss holds is not read."""
+    from mlopamd.models.layers import rope_table
+
+    o, D, BS = torch.ops.mlop, 128, 16
+    ops._sk_reserve(torch.device(gpu))
+    N, NB = (hq + 2 * hkv) * D, 8
+    prev = o.gemm_mid_chain(-1)
+    o.gemm_mid_chain(1)
+    try:
+        assert o.gemm_on_ws(M, N, K, 3) and o.mid_chain_ok(M, N, K, 3)
+        torch.manual_seed(M + K)
+        x, w = (3 * torch.randn(M, K, device=gpu)).to(bf), (0.02 * torch.randn(N, K, device=gpu)).to(bf)
+        cs = rope_table(D, 512, 1e4, device=gpu)
+        pos = torch.randint(0, 512, (M,), device=gpu, dtype=torch.int32)
+        slots = torch.randperm(NB * BS, device=gpu)[:M].to(torch.int32)
+        slots[M // 2] = -1
+        kc, vc = (torch.zeros(NB, hkv, BS, D, device=gpu, dtype=bf) for _ in range(2))
+        q = ops.qkv_rope_cache_rs(x, w, pos, cs, slots, kc, vc, hq, ops.ss_buffer(M, K, gpu).fill_(float("nan")), EPS)
+    finally:
+        o.gemm_mid_chain(prev)
+    kr, vr = torch.zeros_like(kc).cpu(), torch.zeros_like(vc).cpu()
+    qkv = (_unit_norm(x) @ w.float().t()).cpu()
+    qr = ref.rope_cache(qkv, pos.cpu(), cs.cpu(), slots.cpu(), kr, vr, hq)
+    # the projections' bf16 rounding through a rotation of two of them, and the result's own
+    tol = dict(rtol=2.0 ** -8, atol=2.0 ** -7 * float(qkv.abs().max()))
+    for a, b in ((q, qr), (kc, kr), (vc, vr)):
+        torch.testing.assert_close(a.float().cpu(), b.float(), **tol)
