@@ -180,7 +180,7 @@ def paged_attention(q, k_cache, v_cache, meta, out: torch.Tensor | None = None):
     if pts is not None and pts.numel():
         # prompt chunks: K7 flash prefill (128 q-rows per workgroup, K/V via LDS-DMA)
         torch.ops.mlop.flash_prefill(out, q, k_cache, v_cache, meta.block_tables, pts, meta.ptile_q0,
-                                     meta.q_start, meta.q_len, meta.ctx_len, scale)
+                                     meta.q_start, meta.q_len, meta.ctx_len, scale, getattr(meta, "pkeys", 0))
     return out
 
 

@@ -1026,6 +1026,241 @@ __device__ __forceinline__ void flash_item(
   }
 }
 
+// The same tile with a pair's three phases (S, softmax, O) one behind the other, on the 32x32x16 MFMA, K and V pair in one ring
+// of three: 160 registers and 48 KB, three workgroups per CU where flash_item has two, and half as much to run before the first
+// score and after the last.  For short tiles (flash_in_turn).  Per wave 32 q-rows, one per lane column: S^T [32 keys x 32 q], lane
+// l holds keys (r & 3) + 8 (r >> 2) + 4 h (h = l >> 5) of q column l & 31; O^T [128 d x 32 q], P^T from registers 8 s .. 8 s + 7 of
+// S as the k-step s fragment, V^T keys 16 s + 4 h + 0 .. 3 and + 8, dims 32 dblk + (l & 31).
+template <int G>
+__device__ __forceinline__ void flash_item_in_turn(
+    uint16_t* smem, int tile, int kvh, uint16_t* __restrict__ out, const uint16_t* __restrict__ q,
+    const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc, const int* __restrict__ block_tables,
+    int bt_stride, const int* __restrict__ ptile_seq, const int* __restrict__ ptile_q0,
+    const int* __restrict__ q_start, const int* __restrict__ q_len, const int* __restrict__ ctx_len, int Hq,
+    int Hkv, float scale_log2, int num_blocks) {
+  constexpr int QB = 128 / G;            // query tokens per workgroup
+  constexpr int STAGES = 3;
+  constexpr int STAGE = 4 * kBS * kD;    // bf16 per stage: K page A | K page B | V page A | V page B
+  constexpr int PAGE = kBS * kD;
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  const int s = ptile_seq[tile], q0 = ptile_q0[tile];
+  const int ql = q_len[s], ctx = ctx_len[s], qs = q_start[s];
+  const int last_q = min(q0 + QB, ql) - 1;
+  const int kv_end = ctx - ql + last_q + 1;
+  const int n_pairs = (kv_end + 31) >> 5;
+  const int n_pages = (kv_end + kBS - 1) / kBS;
+  const int wg_min_pos = ctx - ql + q0;
+  const int col = lane & 31, h = lane >> 5;
+
+  // this lane's q row (MFMA column): R = 32 wid + col
+  const int R = 32 * wid + col;
+  const int qi = q0 + R / G;
+  const bool q_ok = qi < ql;
+  const int pos_r = q_ok ? ctx - ql + qi : -1;
+  bf16x8 qf[8];
+  {
+    const uint16_t* qrow = q + ((size_t)(qs + (q_ok ? qi : 0)) * Hq + kvh * G + R % G) * kD + 8 * h;
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+      const bf16x8 v = *reinterpret_cast<const bf16x8*>(qrow + 16 * t);
+      qf[t] = q_ok ? v : bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+    }
+  }
+  f32x16 o[4];
+#pragma unroll
+  for (int d = 0; d < 4; ++d)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) o[d][e] = 0.f;
+  float m = kNegBig, l = 0.f;
+
+  const int* bt = block_tables + (size_t)s * bt_stride;
+  const size_t page_stride = (size_t)Hkv * PAGE;
+  const int kkey = wid * 4 + (lane >> 4);
+  // K image: chunk c of key k at slot c ^ k on BOTH pages (the 32x32 A-operand reads take keys
+  // {0-3, 12-15} of one page and {4-11} of the other per 16-lane group: 16 distinct slots)
+  const int k_off = kvh * PAGE + kkey * kD + (((lane & 15) ^ (kkey & 15)) << 3);
+  const int v_off = kvh * PAGE + kkey * kD + (((lane & 15) ^ vswz(kkey)) << 3);
+  auto page_of = [&](int idx) { return idx < n_pages ? min(max(bt[idx], 0), num_blocks - 1) : -1; };
+  auto issue_pages = [&](int buf, int pgA, int pgB) {
+    if (pgB < 0) pgB = pgA;
+    uint16_t* base = smem + buf * STAGE + wid * 512;
+    __builtin_amdgcn_global_load_lds((const void*)(kc + pgA * page_stride + k_off), (lds_void_t*)(base), 16, 0, 0);
+    __builtin_amdgcn_global_load_lds((const void*)(kc + pgB * page_stride + k_off), (lds_void_t*)(base + PAGE), 16, 0, 0);
+    __builtin_amdgcn_global_load_lds((const void*)(vc + pgA * page_stride + v_off), (lds_void_t*)(base + 2 * PAGE), 16, 0, 0);
+    __builtin_amdgcn_global_load_lds((const void*)(vc + pgB * page_stride + v_off), (lds_void_t*)(base + 3 * PAGE), 16, 0, 0);
+  };
+  // K fragment t of this lane: key col of the pair (page col >> 4, row col & 15), chunk 2t + h at
+  // slot (2t + h) ^ (col & 15): byte k_b0 ^ 32 t
+  const int k15 = col & 15;
+  const uint32_t k_b0 = (uint32_t)(uintptr_t)smem + (uint32_t)((col >> 4) * PAGE * 2 + k15 * 256 + ((h ^ k15) << 4));
+  const uint32_t v_b0 = (uint32_t)(uintptr_t)smem + 2 * PAGE * 2 + vt32_base(lane);
+
+  // S^T of the pair in ring slot ST: K fragment t at k_b0 ^ 32 t, four reads in flight (inline
+  // asm with counted waits: as plain loads the compiler reused one register set and waited
+  // lgkmcnt(0) in front of every MFMA, one LDS latency per fragment)
+  auto qk = [&](auto st_tag) {
+    constexpr uint32_t so = (uint32_t)(decltype(st_tag)::value * STAGE * 2);
+    uint32_t kb = k_b0;
+    asm volatile("" : "+v"(kb));
+    auto kread = [&](int t, bf16x8& f) {
+      asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(f) : "v"(kb ^ (32u * t)), "n"(so));
+    };
+    f32x16 sc;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) sc[e] = 0.f;
+    bf16x8 kf[4];
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // nothing else (SMEM) in the counts below
+#pragma unroll
+    for (int t = 0; t < 4; ++t) kread(t, kf[t]);
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+      bf16x8& f = kf[t & 3];
+      if (t <= 4) asm volatile("s_waitcnt lgkmcnt(3)" : "+v"(f));
+      else if (t == 5) asm volatile("s_waitcnt lgkmcnt(2)" : "+v"(f));
+      else if (t == 6) asm volatile("s_waitcnt lgkmcnt(1)" : "+v"(f));
+      else asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(f));
+      sc = mfma32(f, qf[t], sc);
+      if (t + 4 < 8) kread(t + 4, kf[t & 3]);
+    }
+    return sc;
+  };
+  // online softmax on the lane's 16 keys of its q column (raw score units; the scale folds into
+  // the exponent's FMA) -> P^T fragments of the two k-steps; O and l rescaled when the max moved
+  auto softmax = [&](f32x16 sc, int pp, bf16x8 (&pf)[2]) {
+    if (pp * 32 + 31 > wg_min_pos) {  // a pair crossing the workgroup's causal diagonal
+      // (a side effect keeps this a branch: if-converted, the 47 compare / select / add of the
+      // mask ran on every pair, a third of the loop's VALU)
+      asm volatile("");
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int tok = pp * 32 + (r & 3) + 8 * (r >> 2) + 4 * h;
+        sc[r] = tok <= pos_r ? sc[r] : -INFINITY;
+      }
+    }
+    float mx = fmaxf(fmaxf(sc[0], sc[1]), sc[2]);
+#pragma unroll
+    for (int r = 3; r < 15; r += 2) mx = fmaxf(fmaxf(mx, sc[r]), sc[r + 1]);
+    mx = fmaxf(mx, sc[15]);
+    {
+      const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+      mx = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
+    }
+    // deferred rescale (cdna_hip_programming.md T13): the running max moves only when some row's
+    // new max exceeds it by more than 2^kRescaleLog2 in exp2 units (always on a row's first
+    // keys: m starts at -1e30); otherwise P stays scaled against the old max, <= 2^8, which
+    // bf16 P and f32 O / l carry exactly as well.  The decision covers this pair's P and is
+    // taken before it is exponentiated, with the previous pair's P.V complete, so O, l and P
+    // all see the same factor.
+    float alpha = 1.f;
+    if (__ballot((mx - m) * scale_log2 > kRescaleLog2)) {
+      const float m_new = fmaxf(m, mx);
+      alpha = fast_exp2((m - m_new) * scale_log2);
+      m = m_new;
+#pragma unroll
+      for (int d = 0; d < 4; ++d) o[d] *= alpha;
+      l *= alpha;
+    }
+    const float mc = -m * scale_log2;
+    float rs = 0.f;
+    u32x4 w[2];
+#pragma unroll
+    for (int r = 0; r < 16; r += 2) {
+      const float p0 = fast_exp2(fmaf(sc[r], scale_log2, mc)), p1 = fast_exp2(fmaf(sc[r + 1], scale_log2, mc));
+      rs += p0 + p1;
+      w[r >> 3][(r & 7) >> 1] = cvt_pk_bf16(p0, p1);
+    }
+    pf[0] = __builtin_bit_cast(bf16x8, w[0]);
+    pf[1] = __builtin_bit_cast(bf16x8, w[1]);
+    l += rs;
+  };
+  // O^T += V^T . P^T from ring slot ST; the V^T fragment of (dblk, page) = two transposed reads.
+  // The reads are inline asm: as builtins the compiler put s_waitcnt vmcnt(0) in front of them
+  // (it cannot tell them from the in-flight LDS-DMA of the next pairs), which exposed the
+  // latency of the DMA just issued on every pair.  The ring protocol (vmcnt + barrier at the
+  // top of the step) already covers this pair; the asm waits below count only these reads.
+  auto pv = [&](auto st_tag, const bf16x8 (&pf)[2]) {
+    constexpr uint32_t so = (uint32_t)(decltype(st_tag)::value * STAGE * 2);
+    uint32_t vb = v_b0;
+    asm volatile("" : "+v"(vb));
+    // both pages' fragments of dim block dblk: 4 reads, results in (lo, hi) of f0 (page A), f1
+    auto issue = [&](int dblk, v4s16 (&r)[4]) {
+      const uint32_t a0 = vb ^ (64u * dblk), a1 = a0 ^ 32u;
+      asm volatile(
+          "ds_read_b64_tr_b16 %0, %4 offset:%6\n"
+          "ds_read_b64_tr_b16 %1, %5 offset:%7\n"
+          "ds_read_b64_tr_b16 %2, %4 offset:%8\n"
+          "ds_read_b64_tr_b16 %3, %5 offset:%9\n"
+          : "=&v"(r[0]), "=&v"(r[1]), "=&v"(r[2]), "=&v"(r[3])
+          : "v"(a0), "v"(a1), "n"(so), "n"(so + 2048u), "n"(so + 4096u), "n"(so + 6144u));
+    };
+    auto frag = [&](const v4s16& lo, const v4s16& hi) {
+      bf16x8 f;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        f[e] = lo[e];
+        f[4 + e] = hi[e];
+      }
+      return f;
+    };
+    v4s16 ra[4], rb[4];
+    issue(0, ra);
+#pragma unroll
+    for (int dblk = 0; dblk < 4; ++dblk) {
+      v4s16 (&cur)[4] = (dblk & 1) ? rb : ra;
+      v4s16 (&nxt)[4] = (dblk & 1) ? ra : rb;
+      if (dblk < 3) {
+        issue(dblk + 1, nxt);
+        asm volatile("s_waitcnt lgkmcnt(4)" : "+v"(cur[0]), "+v"(cur[1]), "+v"(cur[2]), "+v"(cur[3]));
+      } else {
+        asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(cur[0]), "+v"(cur[1]), "+v"(cur[2]), "+v"(cur[3]));
+      }
+      o[dblk] = mfma32(frag(cur[0], cur[1]), pf[0], o[dblk]);
+      o[dblk] = mfma32(frag(cur[2], cur[3]), pf[1], o[dblk]);
+    }
+  };
+
+  issue_pages(0, page_of(0), page_of(1));
+  if (n_pairs > 1) issue_pages(1, page_of(2), page_of(3));
+  int nxtA = page_of(4), nxtB = page_of(5);
+  auto pair_step = [&](auto st_tag, int pp) {
+    constexpr int ST = decltype(st_tag)::value;
+    if (pp + 1 < n_pairs) wait_vmcnt<4>(); else wait_vmcnt<0>();
+    raw_barrier();  // pair pp visible to every wave; ring slot (pp - 1) % 3 free
+    if (pp + 2 < n_pairs) {
+      issue_pages((ST + 2) % STAGES, nxtA, nxtB);
+      nxtA = page_of(2 * pp + 6);
+      nxtB = page_of(2 * pp + 7);
+    }
+    bf16x8 pf[2];
+    softmax(qk(st_tag), pp, pf);
+    pv(st_tag, pf);
+  };
+  for (int pp = 0; pp < n_pairs; pp += STAGES) {
+    pair_step(std::integral_constant<int, 0>{}, pp);
+    if (pp + 1 < n_pairs) pair_step(std::integral_constant<int, 1>{}, pp + 1);
+    if (pp + 2 < n_pairs) pair_step(std::integral_constant<int, 2>{}, pp + 2);
+  }
+
+  // the two lane halves' partial row sums; O^T element r of dim block d is dim
+  // 32 d + 8 (r >> 2) + 4 h + (r & 3) of q row R
+  {
+    const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(l), __float_as_uint(l), false, false);
+    l = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
+  }
+  if (!q_ok) return;
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  uint16_t* orow = out + ((size_t)(qs + qi) * Hq + kvh * G + R % G) * kD + 4 * h;
+#pragma unroll
+  for (int d = 0; d < 4; ++d)
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+      u32x2 v;
+      v[0] = pack2(o[d][4 * b] * inv, o[d][4 * b + 1] * inv);
+      v[1] = pack2(o[d][4 * b + 2] * inv, o[d][4 * b + 3] * inv);
+      *reinterpret_cast<u32x2*>(orow + 32 * d + 8 * b) = v;
+    }
+}
+
 // STREAM (flash_stream op): the persistent grid's tiles as ONE stream of K / V page pairs per
 // workgroup, so a tile's fixed cost hides under the previous tile's pairs (the 29 us fixed term
 // of profiles/r06_flash_persist.md):
@@ -1383,17 +1618,21 @@ __global__ void __launch_bounds__(256, 2) flash32_stream_kernel(
 // ones.  The host's per-sequence latest-first tile order then pairs a heavy tile with its light
 // mirror on every slot (16 x 512: positions p, 15 - p, p, 15 - p), and the launch holds whole
 // rounds instead of ~2 k one-item workgroups.
-template <int G, int WPC, bool PERSIST>
+template <int G, int WPC, bool PERSIST, bool IN_TURN>
 __global__ void __launch_bounds__(256, WPC) flash_prefill_kernel(
     uint16_t* __restrict__ out, const uint16_t* __restrict__ q, const uint16_t* __restrict__ kc,
     const uint16_t* __restrict__ vc, const int* __restrict__ block_tables, int bt_stride,
     const int* __restrict__ ptile_seq, const int* __restrict__ ptile_q0,
     const int* __restrict__ q_start, const int* __restrict__ q_len,
     const int* __restrict__ ctx_len, int Hq, int Hkv, float scale_log2, int num_blocks, int num_ptiles) {
-  constexpr int STAGES = kFlashRing;
+  constexpr int STAGES = IN_TURN ? 3 : kFlashRing;
   constexpr int STAGE = 4 * kBS * kD;    // bf16 per stage: K page A | K page B | V page A | V page B
   __shared__ __attribute__((aligned(256))) uint16_t smem[STAGES * STAGE];
-  if constexpr (!PERSIST) {
+  if constexpr (IN_TURN) {
+    static_assert(!PERSIST, "one tile per workgroup");
+    flash_item_in_turn<G>(smem, blockIdx.x / Hkv, blockIdx.x % Hkv, out, q, kc, vc, block_tables, bt_stride, ptile_seq,
+                          ptile_q0, q_start, q_len, ctx_len, Hq, Hkv, scale_log2, num_blocks);
+  } else if constexpr (!PERSIST) {
     flash_item<G>(smem, blockIdx.x / Hkv, blockIdx.x % Hkv, out, q, kc, vc, block_tables, bt_stride, ptile_seq,
                     ptile_q0, q_start, q_len, ctx_len, Hq, Hkv, scale_log2, num_blocks);
   } else {
@@ -1427,6 +1666,32 @@ int flash_stream(int set) {
   return g_flash_stream;
 }
 
+// flash_form op: 0 by flash_in_turn, 1 flash_item, 2 flash_item_in_turn
+static int g_flash_form = 0;
+int flash_form(int set) {
+  if (set >= 0) g_flash_form = set;
+  return g_flash_form;
+}
+
+// The form in turn: for launches of short tiles, by their workgroups w and the keys that a tile reads on average (keys: summed over
+// the tiles, 0 where not known).  What the software pipeline gains per pair it has to earn back: a longer way to the first score
+// and from the last, and two workgroups per CU instead of three.  2244 launches (whole prompts alike and unlike, chunks behind
+// cached keys, 1 - 32 kv heads, groups of 1 - 8), time of the pipeline over the form in turn at 48 / 100 / 200 / 320 / 512 keys: up to
+// 224 workgroups 1.04 / 1.01 / 0.95 / 0.91 / 0.87; 225 - 512, one round of either, below 1; 513 - 640 1.16 / 1.05 / 0.95 / 0.93 / 0.92; 641 -
+// 768, one round of it and two of the pipeline, 1.09 / 1.08 / 1.1 / 0.99 / 0.93; 769 - 896 about 1.0 up to 256 keys; 897 - 1024, two rounds
+// of the pipeline, 1.03 / 1.0 / 0.94 / 0.96 / 0.9; 1025 - 1280 1.06 / 1.03 / 1.01 / 0.99 / 1.0; 1281 - 1792 1.03 / 1.02 / 1.03 / 1.0 / 0.99;
+// 1793 - 2560 1.03 / 1.06 / 1.06 / 1.03 / 1.01; more 1.05 / 1.08 / 1.06 / 1.05 / 1.02, 0.97 from 768 keys on.
+static bool flash_in_turn(int num_ptiles, int Hkv, long keys) {
+  const long w = (long)num_ptiles * Hkv, mean = keys / num_ptiles;
+  if (keys <= 0) return false;
+  if (w <= kCus * 7 / 8) return mean <= 80;
+  if (w <= 2 * kCus) return false;
+  if (w <= kCus * 5 / 2) return mean <= 180;
+  if (w <= kCus * 7 / 2) return mean <= 256;
+  if (w <= 4 * kCus) return false;
+  return mean <= std::min(512L, 200 + (w - 4 * kCus) / 5);
+}
+
 static int device_cus() {
   static int cus[16] = {};
   int dev = 0;
@@ -1439,8 +1704,9 @@ static int device_cus() {
 void launch_flash_prefill(void* out, const void* q, const void* kc, const void* vc, const int* bt,
                           int bt_stride, const int* ptile_seq, const int* ptile_q0,
                           const int* q_start, const int* q_len, const int* ctx_len, int num_ptiles,
-                          int Hq, int Hkv, float scale_log2, int num_blocks, hipStream_t st) {
+                          int Hq, int Hkv, float scale_log2, int num_blocks, long keys, hipStream_t st) {
   if (num_ptiles == 0) return;
+  const bool in_turn = g_flash_form ? g_flash_form == 2 : flash_in_turn(num_ptiles, Hkv, keys);
   const int slots = g_flash_persist >= 64 ? g_flash_persist / 64
                     : g_flash_persist > 0 ? std::max(1, g_flash_persist * device_cus() / Hkv) : 0;
   const bool persist = slots > 0 && num_ptiles > slots;
@@ -1453,11 +1719,15 @@ void launch_flash_prefill(void* out, const void* q, const void* kc, const void* 
           (uint16_t*)out, (const uint16_t*)q, (const uint16_t*)kc, (const uint16_t*)vc, bt, bt_stride,   \
           ptile_seq, ptile_q0, q_start, q_len, ctx_len, Hq, Hkv, scale_log2, num_blocks, num_ptiles);    \
     else if (persist)                                                                                    \
-      flash_prefill_kernel<GG, 2, true><<<grid, 256, 0, st>>>(                                         \
+      flash_prefill_kernel<GG, 2, true, false><<<grid, 256, 0, st>>>(                                  \
+          (uint16_t*)out, (const uint16_t*)q, (const uint16_t*)kc, (const uint16_t*)vc, bt, bt_stride,   \
+          ptile_seq, ptile_q0, q_start, q_len, ctx_len, Hq, Hkv, scale_log2, num_blocks, num_ptiles);    \
+    else if (in_turn)                                                                                    \
+      flash_prefill_kernel<GG, 2, false, true><<<grid, 256, 0, st>>>(                                  \
           (uint16_t*)out, (const uint16_t*)q, (const uint16_t*)kc, (const uint16_t*)vc, bt, bt_stride,   \
           ptile_seq, ptile_q0, q_start, q_len, ctx_len, Hq, Hkv, scale_log2, num_blocks, num_ptiles);    \
     else                                                                                                 \
-      flash_prefill_kernel<GG, 2, false><<<grid, 256, 0, st>>>(                                        \
+      flash_prefill_kernel<GG, 2, false, false><<<grid, 256, 0, st>>>(                                 \
           (uint16_t*)out, (const uint16_t*)q, (const uint16_t*)kc, (const uint16_t*)vc, bt, bt_stride,   \
           ptile_seq, ptile_q0, q_start, q_len, ctx_len, Hq, Hkv, scale_log2, num_blocks, num_ptiles);    \
     break;

@@ -139,7 +139,7 @@ void upload(Tensor dst, Tensor src, at::IntArrayRef runs) {
 
 void flash_prefill(Tensor out, Tensor q, Tensor k_cache, Tensor v_cache, Tensor block_tables,
                    Tensor ptile_seq, Tensor ptile_q0, Tensor q_start, Tensor q_len, Tensor ctx_len,
-                   double scale) {
+                   double scale, int64_t keys) {
   check_bf16(out, "out"); check_bf16(q, "q"); check_bf16(k_cache, "k_cache");
   check_bf16(v_cache, "v_cache");
   check_i32(block_tables, "block_tables"); check_i32(ptile_seq, "ptile_seq");
@@ -167,7 +167,7 @@ void flash_prefill(Tensor out, Tensor q, Tensor k_cache, Tensor v_cache, Tensor 
                              ptile_seq.data_ptr<int>(), ptile_q0.data_ptr<int>(),
                              q_start.data_ptr<int>(), q_len.data_ptr<int>(), ctx_len.data_ptr<int>(),
                              (int)ptile_seq.numel(), Hq, Hkv, (float)(scale * 1.4426950408889634),
-                             (int)k_cache.size(0), cur_stream());
+                             (int)k_cache.size(0), (long)keys, cur_stream());
 }
 
 // Largest (tile, kv head) pair count that takes the in-launch split-KV combine: no cap (a cap of
@@ -567,6 +567,7 @@ int64_t gemm_ws_max_m(int64_t set) { return mlop::gemm_ws_max_m((int)set); }
 void gemm_ws_plan(int64_t rb, int64_t u, int64_t nt) { mlop::gemm_ws_plan((int)rb, (int)u, (int)nt); }
 int64_t gemm_ws_small_m(int64_t set) { return mlop::gemm_ws_small_m((int)set); }
 int64_t gemm_ws_rope_m(int64_t set) { return mlop::gemm_ws_rope_m((int)set); }
+int64_t flash_form(int64_t set) { return mlop::flash_form((int)set); }
 int64_t flash_persist(int64_t set) { return mlop::flash_persist((int)set); }
 int64_t flash_stream(int64_t set) { return mlop::flash_stream((int)set); }
 int64_t gemm_grouped_balance(int64_t set) { return mlop::gemm_grouped_balance((int)set); }
@@ -978,6 +979,7 @@ TORCH_LIBRARY(mlop, m) {
   m.def("gemm_ws_plan(int rb, int u, int nt) -> ()", &gemm_ws_plan);
   m.def("gemm_ws_small_m(int set=-1) -> int", &gemm_ws_small_m);
   m.def("gemm_ws_rope_m(int set=-1) -> int", &gemm_ws_rope_m);
+  m.def("flash_form(int set=-1) -> int", &flash_form);
   m.def("flash_persist(int set=-1) -> int", &flash_persist);
   m.def("flash_stream(int set=-1) -> int", &flash_stream);
   m.def("gemm_grouped_balance(int set=-1) -> int", &gemm_grouped_balance);
@@ -1040,7 +1042,7 @@ TORCH_LIBRARY(mlop, m) {
   m.def("upload(Tensor(a!) dst, Tensor src, int[] runs) -> ()");
   m.def("gemm_ws(Tensor(a!) out, Tensor a, Tensor w, int epi, bool rs, float eps) -> bool");
   m.def("flash_prefill(Tensor(a!) out, Tensor q, Tensor k_cache, Tensor v_cache, Tensor block_tables, "
-        "Tensor ptile_seq, Tensor ptile_q0, Tensor q_start, Tensor q_len, Tensor ctx_len, float scale) -> ()");
+        "Tensor ptile_seq, Tensor ptile_q0, Tensor q_start, Tensor q_len, Tensor ctx_len, float scale, int keys=0) -> ()");
   m.def("paged_attention(Tensor(a!) out, Tensor(b!) part_o, Tensor(c!) part_ml, Tensor(d!) part_sem, Tensor q, "
         "Tensor k_cache, Tensor v_cache, Tensor block_tables, Tensor tile_seq, Tensor tile_q0, "
         "Tensor q_start, Tensor q_len, Tensor ctx_len, float scale, int part_tokens, "

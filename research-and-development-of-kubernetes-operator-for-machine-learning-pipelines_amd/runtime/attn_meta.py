@@ -64,6 +64,8 @@ class AttnMeta:
     # int32 [2]: keys of the decode tiles' sequences, summed over the tiles, and the tiles that have any (None: the kernel
     # sums them itself)
     load: torch.Tensor | None = None
+    # keys that the flash tiles read, summed over them (0: not known), by which their kernel's form is chosen
+    pkeys: int = 0
 
 
 # 128-token partitions: one 32-token page pair per wave at batch 1 (256: 312 tok/s, 128: 322,
@@ -143,7 +145,7 @@ class MetaBuffers:
         self.pqt = flash_tile or (128 // group if group <= 8 else 0)
         self.flash_min_q = flash_min_q if self.pqt else 1 << 30
         self.max_tiles = max_tokens  # worst case: one tile per token
-        self.npt = 0                 # flash tiles of the last fill
+        self.npt = self.pkeys = 0    # flash tiles of the last fill, keys that they read
         self._pwork = np.zeros(self.max_tiles, dtype=np.int32)  # per flash tile: keys it reads
         sizes = [("positions", max_tokens), ("slots", max_tokens), ("tile_seq", self.max_tiles),
                  ("tile_q0", self.max_tiles), ("ptile_seq", self.max_tiles), ("ptile_q0", self.max_tiles),
@@ -244,7 +246,7 @@ class MetaBuffers:
         self.hdr_hn[:len(vals)] = vals
 
     def meta(self, num_tokens: int, num_tiles: int, n_logits: int, part_tokens: int, nparts: int,
-             num_ptiles: int = 0) -> AttnMeta:
+             num_ptiles: int = 0, pkeys: int = 0) -> AttnMeta:
         if nparts > 1:
             assert num_tiles * self.n_kv * nparts <= self.wp_capacity, "partial workspace too small"
         return AttnMeta(
@@ -255,7 +257,7 @@ class MetaBuffers:
             q_start=self.view_d("q_start"), q_len=self.view_d("q_len"), ctx_len=self.view_d("ctx_len"),
             part_tokens=part_tokens, nparts=nparts, part_o=self.part_o, part_ml=self.part_ml,
             logits_idx=self.lidx_d[:n_logits], num_tokens=num_tokens, part_sem=self.part_sem,
-            load=self.view_d("load", 2), **self._chunk_views())
+            load=self.view_d("load", 2), pkeys=pkeys, **self._chunk_views())
 
     def _chunk_views(self) -> dict:
         d = {}
@@ -294,7 +296,7 @@ class MetaBuffers:
         pos_h, slot_h = self.view_h("positions"), self.view_h("slots")
         ts_h, tq_h = self.view_h("tile_seq"), self.view_h("tile_q0")
         pts_h, ptq_h = self.view_h("ptile_seq"), self.view_h("ptile_q0")
-        npt, pqt = 0, self.pqt
+        npt, pqt, pkeys = 0, self.pqt, 0
         ni = nr = xr = xm = 0
         if self.chunk:
             # enough chunks to fill the chip either way: longer ones halve the chunk states' traffic
@@ -314,6 +316,7 @@ class MetaBuffers:
                 pts_h[npt:npt + n] = row
                 ptq_h[npt:npt + n] = np.arange(n - 1, -1, -1, dtype=np.int32) * pqt  # latest first
                 self._pwork[npt:npt + n] = (cl - ql + pqt) + ptq_h[npt:npt + n]  # keys each tile reads
+                pkeys += n * (cl - ql) + pqt * (n * (n - 1) // 2) + ql
                 max_flash_q = max(max_flash_q, ql)
                 npt += n
             else:
@@ -342,7 +345,7 @@ class MetaBuffers:
             t += ql
         if npt > 1 and FLASH_LPT and max_flash_q >= FLASH_LPT_MIN_Q:
             order_flash_tiles(pts_h[:npt], ptq_h[:npt], self._pwork[:npt])
-        self.npt = npt
+        self.npt, self.pkeys = npt, pkeys
         self.n_items, self.n_crows = ni, nr
         self.x_rows, self.x_max = xr, xm
         return t, nt, nl
@@ -351,7 +354,7 @@ class MetaBuffers:
         """Vectorised decode fill: one query token per sequence, padded to the
         graph bucket ``pad_to`` with rows that attend to nothing."""
         B = len(rows)
-        self.npt = self.n_items = self.n_crows = self.x_rows = self.x_max = 0
+        self.npt = self.pkeys = self.n_items = self.n_crows = self.x_rows = self.x_max = 0
         pos_h, slot_h = self.view_h("positions"), self.view_h("slots")
         ts_h, tq_h = self.view_h("tile_seq"), self.view_h("tile_q0")
         qs_h, ql_h, cl_h = self.view_h("q_start"), self.view_h("q_len"), self.view_h("ctx_len")

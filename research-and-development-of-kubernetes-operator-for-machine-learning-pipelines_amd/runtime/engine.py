@@ -57,13 +57,13 @@ class StepSync:
       * the step's packed metadata buffer (attn_meta.MetaBuffers: int32 metadata, ids and
         logits index in ONE device buffer, already uploaded by one H2D, decode ids gathered on
         the device from the previous step's tokens) as ONE in-stream device broadcast of its
-        used prefix (header word 9: up to the highest block-table row in use): the K15 IPC
+        used prefix (header word 10: up to the highest block-table row in use): the K15 IPC
         broadcast kernel on GPU (parallel/custom_ar.py: each worker copies the leader's bytes in
         one hop, no host round trip), RCCL / gloo otherwise, ordered after the previous forward
         on every rank's stream.
     STOP / BARRIER steps carry the header only."""
 
-    NHDR = 10
+    NHDR = 11
 
     def __init__(self, group, cpu_group=None):
         import os
@@ -97,9 +97,9 @@ class StepSync:
             return
         dist.broadcast(self.hdr, src=dist.get_global_rank(self.cpu, 0), group=self.cpu)
 
-    def send(self, eng, kind, T, nt, nl, part, nparts, bucket, npt=0, greedy=0):
+    def send(self, eng, kind, T, nt, nl, part, nparts, bucket, npt=0, greedy=0, pkeys=0):
         n = eng.meta.extent(eng.rows_hi)
-        self.hdr[:] = torch.tensor([kind, T, nt, nl, part, nparts, bucket, npt, greedy, n], dtype=torch.int64)
+        self.hdr[:] = torch.tensor([kind, T, nt, nl, part, nparts, bucket, npt, greedy, pkeys, n], dtype=torch.int64)
         self._bcast_header()
         if kind not in (KIND_STOP, KIND_BARRIER):
             self.g.broadcast(eng.meta.dbuf[:n], 0)
@@ -108,8 +108,8 @@ class StepSync:
         self._bcast_header()
         hdr = tuple(self.hdr.tolist())
         if hdr[0] not in (KIND_STOP, KIND_BARRIER):
-            self.g.broadcast(eng.meta.dbuf[:hdr[9]], 0)
-        return hdr[:9]
+            self.g.broadcast(eng.meta.dbuf[:hdr[10]], 0)
+        return hdr[:10]
 
 
 class _Tokens:
@@ -1286,7 +1286,7 @@ class Engine:
         (SURVEY §2.5 CL5); the other ranks run the same ``_execute`` from ``worker_loop``.
         Returns logits, or (TP, all-greedy rows) the chosen token ids already."""
         self._launched = True
-        npt = self.meta.npt  # flash-prefill tiles of the metadata just filled
+        npt, pkeys = self.meta.npt, self.meta.pkeys  # flash-prefill tiles of the metadata just filled, and their keys
         if self.ep_sync is not None:
             kind, T, nt, nl, part, nparts, bucket = self._ep_agree(kind, T, nt, nl, part, nparts, bucket)
         self.meta.upload(T, nl, self.rows_hi)
@@ -1304,13 +1304,13 @@ class Engine:
                 self.meta.ids_d[:B].copy_(toks_d.index_select(0, self._src_d[:B]))
         if self.step_sync is not None:
             t0 = time.perf_counter()
-            self.step_sync.send(self, kind, T, nt, nl, part, nparts, bucket, npt, int(greedy))
+            self.step_sync.send(self, kind, T, nt, nl, part, nparts, bucket, npt, int(greedy), pkeys)
             self.stats["tp_sync_us"] += int(1e6 * (time.perf_counter() - t0))
             self.stats["tp_sync_calls"] += 1
         if self.device.type == "cuda":
             self._meta_ev = torch.cuda.Event()
             self._meta_ev.record()
-        return self._execute(kind, T, nt, nl, part, nparts, bucket, npt, greedy)
+        return self._execute(kind, T, nt, nl, part, nparts, bucket, npt, greedy, pkeys)
 
     def _ep_agree(self, kind, T, nt, nl, part, nparts, bucket):
         """EP lock-step: the group's common step shape.  Someone eager -> everyone eager, MoE
@@ -1330,14 +1330,14 @@ class Engine:
             self.stats["ep_repadded_steps"] += 1
         return kind, b_max, b_max, b_max, part, nparts, b_max
 
-    def _execute(self, kind, T, nt, nl, part, nparts, bucket, npt=0, greedy=0):
+    def _execute(self, kind, T, nt, nl, part, nparts, bucket, npt=0, greedy=0, pkeys=0):
         if self._inject_device_us:  # fault injection: this step is slower on the device only
             torch.ops.mlop.device_delay(self._inject_device_us)
         if kind == KIND_GRAPH:
             graph, logits_buf = self.graphs[bucket]
             graph.replay()
             return self._gather(logits_buf, greedy)
-        meta = self.meta.meta(T, nt, nl, part, nparts, npt)
+        meta = self.meta.meta(T, nt, nl, part, nparts, npt, pkeys)
         hidden = self.model.forward(self.meta.ids_d[:T], meta, self.kv)
         if nl == 0:
             return None

@@ -396,3 +396,32 @@ def test_dead_peer_error_word_fails_the_step():
             eng.step()
     finally:
         model.ps.tp.car = None
+
+
+def test_flash_keys_reach_every_rank():
+    """The keys that a step's flash tiles read (AttnMeta.pkeys), summed as the tiles read them, and in the step's header."""
+    from mlopamd.runtime.attn_meta import MetaBuffers
+    from mlopamd.runtime.engine import KIND_EAGER, StepSync
+
+    mb = MetaBuffers(2048, 8, 64, 4, 2, 1024, "cpu")
+    q, ctx = [17, 100, 32, 5, 200], [17, 130, 32, 9, 700]
+    T, nt, nl = mb.fill(list(range(5)), q, ctx, [[0] * n for n in q])
+    tiles = [c - n + min(a + mb.pqt, n) for n, c in zip(q, ctx) if n >= mb.flash_min_q for a in range(0, n, mb.pqt)]
+    assert (mb.npt, mb.pkeys) == (len(tiles), sum(tiles))
+    assert mb.meta(T, nt, nl, 1024, 1, mb.npt, mb.pkeys).pkeys == sum(tiles) and mb.meta(T, nt, nl, 1024, 1, mb.npt).pkeys == 0
+
+    class Group:
+        rank = 0
+
+        def broadcast(self, buf, src):
+            self.sent = buf
+
+    class Eng:
+        meta, rows_hi = mb, 5
+
+    sync = StepSync(Group())
+    sync.send(Eng, KIND_EAGER, T, nt, nl, 1024, 1, 0, mb.npt, 1, mb.pkeys)
+    n = sync.g.sent.numel()
+    assert sync.recv(Eng) == (KIND_EAGER, T, nt, nl, 1024, 1, 0, mb.npt, 1, sum(tiles)) and sync.g.sent.numel() == n == mb.extent(5)
+    mb.fill_decode(np.array([1], np.int32), np.array([9], np.int32), np.zeros(1, np.int64), pad_to=1)
+    assert mb.npt == mb.pkeys == 0

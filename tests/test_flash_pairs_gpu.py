@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 bf = torch.bfloat16
 
 
-def launch(gpu, q_lens, ctx_lens, Hq, Hkv, grow):
+def launch(gpu, q_lens, ctx_lens, Hq, Hkv, grow, keys=0):
     """Every sequence a prefill of q_lens tokens behind ctx_lens - q_lens cached ones, pages scattered."""
     G, rng, S = Hq // Hkv, np.random.default_rng(len(q_lens) + Hq), len(q_lens)
     pages = [(c + 15) // 16 for c in ctx_lens]
@@ -42,10 +42,12 @@ def launch(gpu, q_lens, ctx_lens, Hq, Hkv, grow):
         for i, n in enumerate(pages):
             at = torch.arange(n, device=gpu).view(n, 1, 1, 1)
             kc[bt[i, :n]] = (kc[bt[i, :n]].float() * 1.25 ** (at % 24)).to(bf)
+    m.pkeys = keys
     out = ops.paged_attention(q, kc, vc, m)
     exp = ref.paged_attention(q, kc, vc, m)
     # P in bf16 (2^-9 of each addend, which the row's sum does not share) and the result's rounding; |V| < 5
     torch.testing.assert_close(out.float(), exp.float(), atol=2.0 ** -6, rtol=2.0 ** -6)
+    return out, lambda: ops.paged_attention(q, kc, vc, m)
 
 
 @pytest.mark.parametrize("grow", [False, True])
@@ -59,3 +61,34 @@ def test_every_number_of_pairs(gpu, Hq, Hkv, grow):
 def test_whole_prompts(gpu, Hq, Hkv):
     n = [1, 15, 31, 32, 33, 63, 64, 65, 97, 127, 128, 129, 190, 255, 257, 449]
     launch(gpu, n, n, Hq, Hkv, False)
+
+
+@pytest.fixture
+def in_turn(gpu):
+    torch.ops.mlop.flash_form(2)
+    yield
+    torch.ops.mlop.flash_form(0)
+
+
+@pytest.mark.parametrize("grow", [False, True])
+@pytest.mark.parametrize("Hq,Hkv", [(8, 8), (8, 4), (8, 2), (16, 2)])
+def test_in_turn(gpu, in_turn, Hq, Hkv, grow):
+    """The form of short tiles, whose rings are three pairs deep, over the same numbers of pairs and lengths."""
+    ctx = [32 * p + r for p in range(11) for r in (1, 16, 17, 32)]
+    launch(gpu, [min(c, 1 + 7 * i % 23) for i, c in enumerate(ctx)], ctx, Hq, Hkv, grow)
+    n = [1, 15, 31, 32, 33, 63, 64, 65, 97, 127, 128, 129, 190, 255, 257, 449]
+    launch(gpu, n, n, Hq, Hkv, grow)
+
+
+@pytest.mark.parametrize("tiles,mean,turn", [(28, 80, True), (28, 81, False), (29, 20, False), (64, 20, False), (65, 20, True), (80, 180, True), (80, 181, False),
+                                             (112, 256, True), (113, 20, False), (128, 20, False), (129, 200, True), (129, 202, False), (400, 512, True), (400, 513, False)])
+def test_which_form(gpu, tiles, mean, turn):
+    """8 kv heads, short prompts of one tile each: the form that the rule names, bit for bit (the two sum in other orders)."""
+    out, again = launch(gpu, [1 + i % 16 for i in range(tiles)], [100 + i for i in range(tiles)], 64, 8, False, keys=tiles * mean)
+    try:
+        torch.ops.mlop.flash_form(2 if turn else 1)
+        assert torch.equal(out, again())
+        torch.ops.mlop.flash_form(1 if turn else 2)
+        assert not torch.equal(out, again())
+    finally:
+        torch.ops.mlop.flash_form(0)
