@@ -976,7 +976,7 @@ TORCH_LIBRARY(mlop, m) {
   m.def("gemm_ws_max_m(int set=-1) -> int", &gemm_ws_max_m);
   m.def("gemm_on_ws(int M, int N, int K, int epi) -> bool", &gemm_on_ws);
   m.def("decode_chain_max_m() -> int", &decode_chain_max_m);
-  m.def("gemm_ws_plan(int rb, int u, int nt) -> ()", &gemm_ws_plan);
+  m.def("gemm_ws_plan(int rb, int u, int nt=1) -> ()", &gemm_ws_plan);
   m.def("gemm_ws_small_m(int set=-1) -> int", &gemm_ws_small_m);
   m.def("gemm_ws_rope_m(int set=-1) -> int", &gemm_ws_rope_m);
   m.def("flash_form(int set=-1) -> int", &flash_form);

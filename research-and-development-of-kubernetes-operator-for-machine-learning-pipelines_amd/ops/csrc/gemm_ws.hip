@@ -299,7 +299,8 @@ __global__ void __launch_bounds__(NW * 64) gemm_ws_kernel(const uint16_t* __rest
 // rows up to which this kernel is taken, in the decode chain and outside (gemm_ws_max_m op; 0: never)
 int g_ws_max_m = 16;
 
-// A / B plan (gemm_ws_plan op, 0 = by shape): 16-row blocks per workgroup (1 / 2) and K-steps in flight per wave (1 / 2)
+// A / B plan (gemm_ws_plan op, 0 = by shape): 16-row blocks per workgroup (1 / 2) and K-steps in flight per wave (1; 2 up to 16
+// rows of A)
 int g_ws_rb = 0, g_ws_u = 0;
 
 template <int AR, int G, int U, int EPI, bool RS, bool NT = true>
@@ -335,7 +336,7 @@ void run_ws_ar(const uint16_t* A, int lda, const uint16_t* B, int ldb, uint16_t*
       MLOP_WS(2, 1, , false);
     }
   }
-  if constexpr (AR <= 32) {
+  if constexpr (AR <= 16) {  // (32 rows and two steps: 28 - 41 registers over)
     if (wide && two) MLOP_WS(4, 2);
     if (two) MLOP_WS(2, 2);
   }
@@ -434,7 +435,7 @@ bool ws_prefer(int M, int N, int K, int epi) {
   return M <= bound && ws_shape(M, N, K, epi) && ws_fast(M, N, K, epi);
 }
 
-// (the third argument chose a form of the weight loads that is no more)
+// (the third argument chose a form of the weight loads: gemm_small_nt does)
 void gemm_ws_plan(int rb, int u, int) {
   g_ws_rb = rb == 1 ? 1 : rb == 2 || rb == 4 ? 2 : 0;
   g_ws_u = u == 1 ? 1 : u > 1 ? 2 : 0;
