@@ -1,13 +1,12 @@
-"""Weight-streaming MFMA GEMM (ops/csrc/gemm_ws.hip) vs the planner's small-M tiles at decode
-batch sizes, Llama-3-8B projections, cold weights (a rotation over > 1 GB of copies, as in
+"""Weight-streaming MFMA GEMM (ops/csrc/gemm_ws.hip) vs what has the product without it (the GEMV, the planner's small-M tiles)
+at decode batch sizes, Llama-3-8B projections, cold weights (a rotation over > 1 GB of copies, as in
 serving where 16 GB of other layers stream between two calls of one matrix), one process,
 interleaved rounds.  Also checks each ws result against the fp32 torch product.
 
-  plain forms:  qkv / o / down plain, gate_up with the SiLU-mul epilogue (ops.gemm vs gemm_ws)
-  --chain:      the decode norm chain's forms too: gate_up / qkv-plain with the row-scale
-                prologue (rs), o / down adding into a residual (epi 5)
+qkv / o / down plain, gate_up with the SiLU-mul epilogue: "planner" is the gemm op with the kernel off, "rule" as it is served,
+"ws_<weight rows>x<steps in flight>" the kernel's plans (two steps up to 16 rows of A).
 
-Usage (GPU box): python scripts/bench_ws.py [--ms 8,16,32,64] [--shapes qkv,o,gate_up,down]
+Usage (GPU box): python scripts/bench_ws.py [--ms 4,8,16,32] [--shapes qkv,o,gate_up,down]
 """
 from __future__ import annotations
 
@@ -45,7 +44,7 @@ def ref_silu_mul(y):
 
 def main():
     ap = argparse.ArgumentParser()
-    ap.add_argument("--ms", default="8,16,32,64")
+    ap.add_argument("--ms", default="4,8,16,32")
     ap.add_argument("--shapes", default="qkv,o,gate_up,down")
     ap.add_argument("--iters", type=int, default=20)
     ap.add_argument("--rounds", type=int, default=2)
@@ -53,8 +52,8 @@ def main():
     ops.load()
     dev = torch.device("cuda")
     ops._sk_reserve(dev)
-    torch.ops.mlop.gemm_ws_max_m(64)  # off by default in serving
-    bf = torch.bfloat16
+    o, bf = torch.ops.mlop, torch.bfloat16
+    served = o.gemm_ws_max_m(-1)
     for M in [int(m) for m in a.ms.split(",")]:
         for name in a.shapes.split(","):
             N, K = PROJ[name]
@@ -71,30 +70,34 @@ def main():
                 return ws[cyc[0]]
 
             # numerics: ws vs fp32 torch
-            ok = bool(torch.ops.mlop.gemm_ws(out, x, ws[0], epi, False, 0.0))
+            o.gemm_ws_max_m(64)
+            ok = bool(o.gemm_ws(out, x, ws[0], epi, False, 0.0))
             err = None
             if ok:
                 exp = x.float() @ ws[0].float().t()
                 if silu:
                     exp = ref_silu_mul(exp)
                 err = float((out.float() - exp).abs().max() / exp.abs().max())
-            runs = {"planner": (None, lambda: ops.gemm(x, nxt(), epi=epi))}
+            o.gemm_ws_max_m(0)
+            slabs = torch.empty(max(1, o.gemm_workspace(M, N, K, epi)), device=dev)
+            # name: (rows that the kernel takes, its plan, call)
+            runs = {"planner": (0, (0, 0), lambda: o.gemm(out, x, nxt(), slabs, epi)),
+                    "rule": (served, (0, 0), lambda: o.gemm(out, x, nxt(), slabs, epi))}
             if ok:
-                for rb in ((2, 4) if silu else (1, 2, 4)):
-                    for u in (4, 8):
-                        for nt in (0, 1):
-                            runs[f"ws_rb{rb}_u{u}_nt{nt}"] = (
-                                (rb, u, nt), lambda: torch.ops.mlop.gemm_ws(out, x, nxt(), epi, False, 0.0))
+                for rb in (1, 2):
+                    for u in ((1, 2) if M <= 16 else (1,)):
+                        runs[f"ws_{16 * rb}x{u}"] = (64, (rb, u), lambda: o.gemm_ws(out, x, nxt(), epi, False, 0.0))
             res = {}
             for _ in range(a.rounds):
-                for k, (plan, fn) in runs.items():
-                    if plan is not None:
-                        torch.ops.mlop.gemm_ws_plan(*plan)
+                for k, (rows, plan, fn) in runs.items():
+                    o.gemm_ws_max_m(rows)
+                    o.gemm_ws_plan(*plan)
                     res[k] = min(res.get(k, 1e9), timeit(fn, a.iters))
-            torch.ops.mlop.gemm_ws_plan(0, 0, 1)
-            best = min((k for k in res if k != "planner"), key=res.get, default=None)
+            o.gemm_ws_plan(0, 0)
+            o.gemm_ws_max_m(served)
+            best = min((k for k in res if k.startswith("ws_")), key=res.get, default=None)
             if best:
-                res = {"planner": res["planner"], "ws_best": res[best], **res}
+                res = {"planner": res["planner"], "rule": res["rule"], "ws_best": res[best], **res}
             wbytes = N * K * 2
             print(json.dumps(dict(shape=name, M=M, ws_taken=ok, rel_err=err, ws_best_plan=best if ok else None,
                                   **{f"{k}_us": round(v, 2) for k, v in res.items()},
