@@ -12,9 +12,9 @@ EPS = 1e-5
 
 @pytest.fixture
 def plan(gpu, request):
-    torch.ops.mlop.gemm_ws_plan(*request.param, 0)
+    torch.ops.mlop.gemm_ws_plan(*request.param)
     yield
-    torch.ops.mlop.gemm_ws_plan(0, 0, 0)
+    torch.ops.mlop.gemm_ws_plan(0, 0)
 
 
 def bound(y, a, w, K):

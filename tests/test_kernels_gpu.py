@@ -630,13 +630,26 @@ def test_gemm_stream_k(gpu, pp_variant, M, N, K, epi):
     close(outs[0], outs[2], atol=0, rtol=0)  # deterministic: fixed slot order in the fixup
 
 
+@pytest.fixture(params=[16, 0], ids=["ws", "gemv"])
+def ws_rows(request):
+    """The weight-streaming kernel as served, which has most products of 2 - 4 rows, and off, which leaves them to the GEMV."""
+    prev = torch.ops.mlop.gemm_ws_max_m(-1)
+    assert prev == 16
+    torch.ops.mlop.gemm_ws_max_m(request.param)
+    yield request.param
+    torch.ops.mlop.gemm_ws_max_m(prev)
+
+
 @pytest.mark.parametrize("M", [1, 2, 3, 4, 5, 8])
 @pytest.mark.parametrize("N,K", [(4096, 4096), (6144, 4096), (4096, 14336), (1280, 8192), (8192, 1024),
-                                 (8192, 3584), (16, 1024)])
-def test_gemv(gpu, M, N, K):
-    """K2 skinny GEMV (gemv.hip, M <= 4; M = 5 / 8 take the MFMA tiles): wave-per-row-pair
-    (N >= 4096) and the 4-waves-split-K form (N = 1280 / 16: 70B TP=8 shards, tiny N), K
-    not a multiple of the unrolled stride (1024, 3584); vs fp32 matmul."""
+                                 (8192, 3584), (16, 1024), (4096, 4160), (6144, 64)])
+def test_gemv(gpu, ws_rows, M, N, K):
+    """K2 skinny GEMV (gemv.hip, M <= 4, where the weight-streaming kernel is not the choice; M = 5 / 8 take that or the MFMA
+    tiles): wave-per-row-pair (N >= 4096) and the 4-waves-split-K form (N = 1280 / 16: 70B TP=8 shards, tiny N), K
+    not a multiple of the unrolled stride (1024, 3584) nor of the other kernel's steps (4160, 64); vs fp32 matmul."""
+    if M <= 4:  # the GEMV where that kernel is off, at one row, in narrow products and where K is not whole steps of 128
+        ws = ws_rows and M > 1 and K % 128 == 0 and N >= (3072 if M == 2 else 2048)
+        assert torch.ops.mlop.gemm_plan(M, N, K)[0] == (-2 if ws else -1)
     torch.manual_seed(M * 7 + N + K)
     x = torch.randn(M, K, device=gpu, dtype=bf)
     w = (0.05 * torch.randn(N, K, device=gpu)).to(bf)
@@ -736,9 +749,10 @@ def test_mid_m_gemm(gpu, M, N, K, epi):
 
 
 @pytest.mark.parametrize("M", [1, 2, 4])
-@pytest.mark.parametrize("I,K", [(14336, 4096), (3584, 8192)])
-def test_gemv_silu_mul(gpu, M, I, K):
+@pytest.mark.parametrize("I,K", [(14336, 4096), (3584, 8192), (3584, 2112)])
+def test_gemv_silu_mul(gpu, ws_rows, M, I, K):
     torch.manual_seed(M + I)
+    assert torch.ops.mlop.gemm_on_ws(M, 2 * I, K, 1) == bool(ws_rows and M > 1 and K % 128 == 0)
     x = torch.randn(M, K, device=gpu, dtype=bf)
     g = (0.05 * torch.randn(I, K, device=gpu)).to(bf)
     u = (0.05 * torch.randn(I, K, device=gpu)).to(bf)
@@ -794,12 +808,13 @@ def test_qkv_rope_fused_in_graph(gpu, consecutive):
 
 
 @pytest.mark.parametrize("M,Hq,Hkv", [(1, 32, 8), (3, 32, 8), (4, 32, 8), (2, 8, 1), (4, 64, 8)])
-def test_gemv_rope_cache(gpu, M, Hq, Hkv):
-    """Decode QKV GEMV with RoPE + paged K/V stores in its epilogue (EPI_ROPE at M <= 8)."""
+def test_gemv_rope_cache(gpu, ws_rows, M, Hq, Hkv):
+    """Decode QKV GEMV with RoPE + paged K/V stores in its epilogue (EPI_ROPE at M <= 4)."""
     from mlopamd.models.layers import rope_table
 
     D, K, BS, NB = 128, 4096, 16, 64
     N = (Hq + 2 * Hkv) * D
+    assert torch.ops.mlop.gemm_on_ws(M, N, K, 3) == bool(ws_rows and M > 2)
     cs = rope_table(D, 8192, 5e5, device=gpu)
     x = torch.randn(M, K, device=gpu, dtype=bf)
     w = (0.02 * torch.randn(N, K, device=gpu)).to(bf)
@@ -1218,19 +1233,19 @@ def test_attention_kv_policy_bit_identical(gpu, case):
 
 @pytest.fixture
 def ws_on():
-    """The weight-streaming MFMA kernel is off in serving (gemm_ws_max_m = 0): on for the test."""
+    """The weight-streaming MFMA kernel has up to 16 rows in serving (gemm_ws_max_m): up to 64, which it can take, for the test."""
     prev = torch.ops.mlop.gemm_ws_max_m(-1)
     torch.ops.mlop.gemm_ws_max_m(64)
     yield
     torch.ops.mlop.gemm_ws_max_m(prev)
-    torch.ops.mlop.gemm_ws_plan(0, 0, 1)
+    torch.ops.mlop.gemm_ws_plan(0, 0)
 
 
-@pytest.mark.parametrize("plan", [(0, 0, 1), (4, 4, 0), (2, 8, 1)], ids=["default", "rb4u4c", "rb2u8nt"])
+@pytest.mark.parametrize("plan", [(0, 0), (1, 2), (2, 1)], ids=["default", "16x2", "32x1"])
 @pytest.mark.parametrize("M", [5, 16, 17, 33, 64])
 @pytest.mark.parametrize("N,K,epi", [(1024, 4096, 0), (2048, 4096, 1), (512, 14336, 0), (4096, 1024, 0)])
 def test_gemm_ws_vs_fp32(gpu, ws_on, plan, M, N, K, epi):
-    """K2 at 5-64 rows, the weight-streaming MFMA kernel (gemm_ws.hip): plain and SiLU-mul
+    """K2 at 5-64 rows (more than serving gives it), the weight-streaming MFMA kernel (gemm_ws.hip): plain and SiLU-mul
     (16-interleaved gate / up rows) against the fp32 product; rows past M are never written."""
     from mlopamd import ops
 

@@ -17,8 +17,8 @@ H, I, EPS = 4096, 14336, 1e-5
 
 @pytest.fixture
 def ws_on():
-    """The decode chain's weight-streaming MFMA form (5-64 rows) is off in serving
-    (gemm_ws_max_m = 0): on for these tests."""
+    """The decode chain's weight-streaming MFMA form has up to 16 rows in serving (gemm_ws_max_m): up
+    to 64, which it can take, for these tests."""
     prev = torch.ops.mlop.gemm_ws_max_m(-1)
     torch.ops.mlop.gemm_ws_max_m(64)
     yield
@@ -148,8 +148,8 @@ def test_llama_forward_chain_on_off(gpu, w4, monkeypatch):
 
 @pytest.mark.parametrize("M", [1, 2, 3, 4, 5, 8, 16, 17, 33, 48, 64])
 def test_gemv_chain_res_rs(gpu, w4, ws_on, M):
-    """Decode form of the chain (M <= 4: gemv.hip EPI_RES / PRO_RS; 5-64 rows: the
-    weight-streaming MFMA kernel, gemm_ws.hip WS_RES / RS): O / down add into the residual in
+    """Decode form of the chain (M <= 4: gemv.hip EPI_RES / PRO_RS or, mostly, the weight-streaming MFMA
+    kernel, gemm_ws.hip WS_RES / RS; 5-64 rows: that one, gate_up of 9 and more on gemm_mid.hip): O / down add into the residual in
     place with norm.hip's rounding, gate_up / plain / QKV + RoPE scale each row by
     rsqrt(mean(a^2) + eps) of the residual they stream.  The ss buffers are NaN: the decode
     form must neither read nor need them (the four-wave form would turn them into NaNs)."""
@@ -196,11 +196,61 @@ def test_gemv_chain_res_rs(gpu, w4, ws_on, M):
     close(vc, vr)
 
 
+@pytest.mark.parametrize("M", [1, 2, 3, 4])
+def test_gemv_chain_on_the_gemv(gpu, w4, M):
+    """The same with the weight-streaming kernel off: every product of the chain on the GEMV, plain and narrow, wide, gate / up,
+    residual and RoPE."""
+    prev = torch.ops.mlop.gemm_ws_max_m(-1)
+    torch.ops.mlop.gemm_ws_max_m(0)
+    try:
+        test_gemv_chain_res_rs(gpu, w4, None, M)
+    finally:
+        torch.ops.mlop.gemm_ws_max_m(prev)
+
+
+@pytest.mark.parametrize("M", [4, 5, 9, 16, 17])
+def test_decode_chain_as_served(gpu, w4, M):
+    """With the bounds that serving has: the decode form to 16 rows, none at 17."""
+    assert ops.decode_chain_max_m() == 16
+    shapes = [((32 + 16) * 128, H), (H, H), (2 * I, H), (H, I)]
+    assert ops.norm_chain_ok(M, H, shapes, gpu, (ops.EPI_ROPE, ops.EPI_NONE, ops.EPI_SILU_MUL, ops.EPI_NONE)) == (M <= 16)
+    if M <= 16:
+        test_gemv_chain_res_rs(gpu, w4, None, M)
+
+
+@pytest.mark.parametrize("batch", [6, 13, 24])
+def test_llama_decode_as_served(gpu, batch):
+    """2-layer Llama-3-8B-wide engine as it serves: decode graphs of 8 and 16 rows with the decode chain, of 32 without it, follow
+    the fp32 dense oracle."""
+    from mlopamd.models import build_model
+    from mlopamd.models.config import get_config
+    from mlopamd.models.reference import dense_logits
+    from mlopamd.runtime.engine import Engine, EngineConfig
+    from mlopamd.runtime.sampler import SamplingParams
+
+    model = build_model(get_config("llama3-8b", num_layers=2), device=gpu, seed=7)
+    g = torch.Generator().manual_seed(batch)
+    prompts = [torch.randint(1000, 100000, (48,), generator=g).tolist() for _ in range(batch)]
+    ops._GEMM_USED.clear()  # before the engine: its graph captures run the decode forwards
+    eng = Engine(model, EngineConfig(max_num_seqs=batch, max_num_batched_tokens=512, max_model_len=128,
+                                     num_kv_blocks=batch * 8 + 1, use_graphs=True))
+    outs = eng.generate(prompts, SamplingParams(max_tokens=4, ignore_eos=True))
+    assert (ops.EPI_ADD_SS in set(k[3] for k in ops._GEMM_USED if k[0] <= 16)) and model._chain_ok(batch) == (batch <= 16)
+    assert ops.EPI_ADD_SS not in set(k[3] for k in ops._GEMM_USED if k[0] == 32)
+    for p, o in zip(prompts[:4], outs):
+        toks = list(p)
+        for t in o:
+            lg = dense_logits(model, toks)[-1]
+            best = int(lg.argmax())
+            assert t == best or float(lg[best] - lg[t]) < 0.1 * float(lg.std()), (len(toks), best, t)
+            toks.append(t)
+
+
 @pytest.mark.parametrize("batch", [1, 3, 4, 8, 24])
 def test_llama_decode_gemv_chain_on_off(gpu, w4, ws_on, monkeypatch, batch):
     """2-layer Llama-3-8B-wide engine, graphs on: decode steps of 1 / 3 / 4 sequences with the
-    GEMV chain, of 8 / 24 with the weight-streaming MFMA chain (five launches per layer, no add
-    + RMSNorm; batch 3 / 24 replay the 4- / 32-row graphs with padding rows) and without the
+    GEMV chain, of 8 / 24 with the weight-streaming MFMA chain (at 24 more than serving gives it;
+    five launches per layer, no add + RMSNorm; batch 3 / 24 replay the 4- / 32-row graphs with padding rows) and without the
     chain all follow the fp32 dense oracle."""
     from mlopamd.models import build_model
     from mlopamd.models.config import get_config
