@@ -93,3 +93,42 @@ def test_ss_init_and_all_reduce_add_fallback():
     exp = (res.float() + y.float()).to(torch.bfloat16)
     out = Group().all_reduce_add(y.clone(), res)
     assert out is res and torch.equal(res, exp)
+
+
+@pytest.mark.parametrize("rows,chain", [(4, True), (5, False), (16, False), (17, False)])
+def test_tensor_parallel_chain_has_the_gemvs_rows(force_chain, monkeypatch, rows, chain):
+    """With more ranks the decode chain has the GEMV's four rows, also where one rank alone has it for more (decode_chain_max_m)."""
+    from mlopamd.models import llama
+    from mlopamd.parallel.comm import Group
+    from mlopamd.runtime.attn_meta import MetaBuffers
+    from mlopamd.runtime.kv_cache import KVCache
+
+    class Two(Group):  # of two ranks that hold the whole weights: a sum over them is what one of them has
+        size = 2
+
+        def __init__(self):
+            pass
+
+        def all_reduce(self, x):
+            return x
+
+        def all_reduce_add(self, x, residual):
+            residual.add_(x)
+
+    monkeypatch.setattr(ops, "decode_chain_max_m", lambda: 16)
+    model = build_model(TINY_LLAMA, device="cpu", dtype=torch.float32, seed=1)
+    kv = KVCache(TINY_LLAMA.num_layers, 40, model.n_kv, TINY_LLAMA.head_dim, "cpu", torch.float32)
+    mb = MetaBuffers(64, rows + 1, 4, model.n_q // model.n_kv, model.n_kv, 64, "cpu")
+    for i in range(rows):
+        mb.bt_h[i, 0] = i + 1
+    mb.fill([*range(rows)], [1] * rows, [1] * rows, [[7 + i] for i in range(rows)])
+    mb.upload()
+    meta = mb.meta(rows, rows, rows, 64, 1)
+    alone = model.forward(mb.ids_d[:rows], meta, kv)
+    used = []
+    of = type(model)._chain_layer_tp
+    monkeypatch.setattr(type(model), "_chain_layer_tp", lambda self, *a: used.append(1) or of(self, *a))
+    monkeypatch.setattr(llama, "row_parallel_add_norm", lambda x, w, tp, r, g, eps: ops.add_rmsnorm(ops.gemm(x, w), r, g, eps))
+    monkeypatch.setattr(model.ps, "tp", Two())
+    torch.testing.assert_close(model.forward(mb.ids_d[:rows], meta, kv), alone, rtol=1e-4, atol=1e-4)
+    assert bool(used) == chain
