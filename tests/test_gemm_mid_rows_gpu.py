@@ -42,6 +42,20 @@ def test_plain(gpu, M, N, K):
     assert bool((out[M:] == 7.0).all())
 
 
+@pytest.mark.parametrize("M", [17, 32])
+@pytest.mark.parametrize("N,K", [(32776, 192), (40824, 1088)])
+def test_few_second_tiles(gpu, M, N, K):
+    """64-row tiles of few rows, where 32-row ones would give some CUs a second one."""
+    assert torch.ops.mlop.gemm_plan(M, N, K)[:3] == [7, 64, 128]
+    a, w = operands(gpu, M, N, K)
+    out = torch.full((M + 1, N), 7.0, device=gpu, dtype=bf)
+    torch.ops.mlop.gemm(out[:M], a, w, torch.empty(1, device=gpu), 0)
+    ad, wd = a.double(), w.double()
+    y = ad @ wd.t()
+    assert bool(((out[:M].double() - y).abs() <= bound(y, ad, wd, K)).all())
+    assert bool((out[M:] == 7.0).all())
+
+
 @pytest.mark.parametrize("M", [9, 16, 32, 33, 64])
 @pytest.mark.parametrize("N,K", [(24608, 128), (24608, 1152), (40960, 384), (49184, 640)])
 def test_gate_up_of_the_residual(gpu, M, N, K):
