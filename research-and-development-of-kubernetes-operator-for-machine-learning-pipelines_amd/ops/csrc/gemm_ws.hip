@@ -408,6 +408,8 @@ static bool ws_shape(int M, int N, int K, int epi) {
 // (34 numbers of heads, K 512 - 8192): K up to 4096 0.5 - 1.0; 768 - 2048 columns at 17 / 24 / 32 rows with K 5120 0.95 / 1.0 / 1.05, 6144
 // 0.97 / 1.04 / 1.1, 8192 1.03 / 1.12 / 1.2; 3072 0.9 / 0.94 / 1.03 with 8192; 4352 - 5376 columns, a second round for few, 1.0 - 1.1 from
 // 5120 on; 5632 - 8192 0.8 - 0.98; more at K 5120 - 7168 0.92 / 0.97 / 1.05, at 8192 0.88 / 0.94 / 1.0.
+// Those are with K of whole 2048, mostly, where the K ranges are slower (3328 x 8192 at 19 rows 0.82); with others 2048 - 3583 columns are
+// level at M K / N = 56 (3072 x 7808 at 25 rows, 63: 1.11), 3584 - 4096 at 48 (4096 x 8064 at 32, 63: 1.11).
 static bool ws_fast(int M, int N, int K, int epi) {
   const long nk = (long)N * K, mk = (long)M * K;
   const int w = N / 16;  // workgroups of 16 rows
@@ -423,7 +425,8 @@ static bool ws_fast(int M, int N, int K, int epi) {
     return K <= 2048 || (K <= 9216 && mk <= (N <= 1536 ? 24L : 28L) * N);
   }
   if (epi == WS_ROPE && M > 16)
-    return K <= 4096 || (N <= 4096 ? K <= 8192 && mk <= (N < 3072 ? 60L : 64L) * N : N >= 5632 && (N <= 8192 || K % 4096 == 0 || mk <= 150000));
+    return K <= 4096 || (N <= 4096 ? K <= 8192 && mk <= (K % 2048 ? (N < 2048 ? 60L : N < 3584 ? 56L : 48L) : N < 3072 ? 60L : 64L) * N
+                                   : N >= 5632 && (N <= 8192 || K % 4096 == 0 || mk <= 150000));
   if (epi == WS_ROPE && N <= 1280) return K <= 9216 && mk <= 100000;
   if (N >= 16384 && K < 1024) return false;
   if (second) return K <= (M > 8 ? 7168 : 9216);
