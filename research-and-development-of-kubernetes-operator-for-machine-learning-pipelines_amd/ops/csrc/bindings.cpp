@@ -390,12 +390,15 @@ static bool decode_form(int64_t M, int64_t N, int64_t K, int64_t epi, bool any) 
   return M <= mlop::gemv_chain_max_m() ||
          (!any && M <= mlop::decode_chain_max_m() && mlop::decode_chain_takes((int)M, (int)N, (int)K, (int)epi));
 }
+static bool rows_for_ws(const Tensor& a) {
+  return mlop::ws_rows_ok(a.data_ptr(), (int)a.stride(0), (int)a.size(0), (int)a.size(1));
+}
 // and whether they take these rows: above the GEMV's, where both kernels read them by LDS-DMA
 static bool decode_rows(const Tensor& a) {
-  return a.size(0) <= mlop::gemv_chain_max_m() || mlop::ws_rows_ok(a.data_ptr(), (int)a.stride(0));
+  return a.size(0) <= mlop::gemv_chain_max_m() || rows_for_ws(a);
 }
 static bool decode_on_ws(const Tensor& a, int64_t N, int64_t K, int64_t epi) {
-  return mlop::chain_on_ws((int)a.size(0), (int)N, (int)K, (int)epi) && mlop::ws_rows_ok(a.data_ptr(), (int)a.stride(0));
+  return mlop::chain_on_ws((int)a.size(0), (int)N, (int)K, (int)epi) && rows_for_ws(a);
 }
 
 bool gemm_res_ss(Tensor residual, Tensor a, Tensor w, Tensor ss_out, bool any) {
@@ -508,7 +511,7 @@ bool gemm_rs_rope(Tensor q_out, Tensor k_cache, Tensor v_cache, Tensor a, Tensor
   re.ss_eps = (float)eps;
   if (mlop::mid_chain_ok((int)M, (int)N, (int)K, 3)) {  // 5-64 rows
     c10::DeviceGuard g(a.device());
-    if (mlop::gemm_on_ws((int)M, (int)N, (int)K, 3) && mlop::ws_rows_ok(a.data_ptr(), (int)a.stride(0))) {  // row scale computed from the streamed rows
+    if (mlop::gemm_on_ws((int)M, (int)N, (int)K, 3) && rows_for_ws(a)) {  // row scale computed from the streamed rows
       mlop::launch_ws(a.data_ptr(), (int)a.stride(0), w.data_ptr(), (int)K, nullptr, 0, (int)M, (int)N, (int)K, 3,
                       true, re, (float)eps, cur_stream());
       return true;
@@ -554,7 +557,7 @@ bool gemm_ws(Tensor out, Tensor a, Tensor w, int64_t epi, bool rs, double eps) {
   TORCH_CHECK(out.dim() == 2 && out.size(0) == M && out.size(1) == (epi == 1 ? N / 2 : N) && out.stride(1) == 1,
               "out [M, N or N/2]");
   TORCH_CHECK(!(rs && epi == 5), "residual form has no row scale");
-  if (!mlop::ws_rows_ok(a.data_ptr(), (int)a.stride(0)) || !mlop::ws_takes((int)M, (int)N, (int)K, (int)epi)) return false;
+  if (!rows_for_ws(a) || !mlop::ws_takes((int)M, (int)N, (int)K, (int)epi)) return false;
   c10::DeviceGuard g(a.device());
   mlop::launch_ws(a.data_ptr(), (int)a.stride(0), w.data_ptr(), (int)K, out.data_ptr(), (int)out.stride(0), (int)M,
                   (int)N, (int)K, (int)epi, rs, mlop::RopeEpi{}, (float)eps, cur_stream());

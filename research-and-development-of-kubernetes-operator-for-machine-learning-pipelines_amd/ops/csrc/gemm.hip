@@ -1740,7 +1740,7 @@ bool launch_gemm_rope(const void* A, int lda, const void* B, int M, int N, int K
                       hipStream_t st) {
   if (M == 0) return true;
   if (!gemm_rope_supported(M, N, K)) return false;
-  if (gemm_on_ws(M, N, K, EPI_ROPE) && ws_rows_ok(A, lda)) {  // up to 32 rows: the weight-streaming MFMA kernel
+  if (gemm_on_ws(M, N, K, EPI_ROPE) && ws_rows_ok(A, lda, M, K)) {  // up to 32 rows: the weight-streaming MFMA kernel
     launch_ws(A, lda, B, K, nullptr, 0, M, N, K, EPI_ROPE, false, re, 0.f, st);
     return true;
   }
@@ -1924,7 +1924,7 @@ void launch_gemm(const void* A, int lda, const void* B, int ldb, void* C, int ld
   re.act = epi_act(epi);
   const int epi0 = epi;
   if (re.act) epi = EPI_NONE;
-  if (gemm_on_ws(M, N, K, epi) && ws_rows_ok(A, lda) && ldb % 8 == 0) {
+  if (gemm_on_ws(M, N, K, epi) && ws_rows_ok(A, lda, M, K) && ldb % 8 == 0) {
     launch_ws(A, lda, B, ldb, C, ldc, M, N, K, epi, false, re, 0.f, st);
     return;
   }
@@ -1959,7 +1959,7 @@ bool launch_gemm_add_rmsnorm(const void* A, int lda, const void* B, void* out, v
                              int K, hipStream_t st) {
   if (M == 0) return true;
   if (gemv_takes(M, N, K, EPI_NONE)) return false;  // decode sizes: GEMV + add_rmsnorm (or the norm chain)
-  if (gemm_on_ws(M, N, K, 5) && ws_rows_ok(A, lda)) {
+  if (gemm_on_ws(M, N, K, 5) && ws_rows_ok(A, lda, M, K)) {
     // up to 16 rows: the weight-streaming MFMA kernel adds into the residual
     // in place (bf16(res + bf16(y)), norm.hip's rounding), then one RMSNorm pass
     launch_ws(A, lda, B, K, residual, N, M, N, K, 5, false, RopeEpi{}, 0.f, st);

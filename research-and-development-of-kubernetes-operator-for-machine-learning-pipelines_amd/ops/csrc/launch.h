@@ -207,8 +207,10 @@ int gemm_ws_small_m(int set);
 int gemm_ws_rope_m(int set);  // rows up to which QKV + RoPE takes the weight-streaming kernel
 // the decode projections outside the chain that this kernel takes instead of the GEMV or the planner's tiles
 bool ws_prefer(int M, int N, int K, int epi);
-// it reads A by LDS-DMA of 16 bytes a lane (the GEMV's loads are free of that)
-inline bool ws_rows_ok(const void* A, int lda) { return lda % 8 == 0 && reinterpret_cast<uintptr_t>(A) % 16 == 0; }
+// it reads A by LDS-DMA of 16 bytes a lane at 32-bit offsets from the first row (the GEMV's loads are free of both)
+inline bool ws_rows_ok(const void* A, int lda, int M, int K) {
+  return lda % 8 == 0 && reinterpret_cast<uintptr_t>(A) % 16 == 0 && (long)(M - 1) * lda + K < 1L << 30;
+}
 // and no switch asks for another form (gemm.hip)
 bool gemm_on_ws(int M, int N, int K, int epi);
 // mid-M norm chain on the planner's small tiles (gemm.hip): epi 0 = O / down (split-K, the

@@ -105,3 +105,21 @@ def test_rows_off_16_bytes_stay_on_the_gemv(gpu, switches, M):
         ops.gemm_rs(x, w, ops.ss_buffer(8, K, gpu), 1e-5, ops.EPI_SILU_MUL)
     o.gemm_ws_max_m(0)
     assert all(torch.equal(a, b) for a, b in zip(here, outs(x[:M].clone())))
+
+
+@pytest.mark.parametrize("M", [3, 4, 8])
+def test_rows_far_apart(gpu, M):
+    """Rows of A that span more than 32 bits of bytes are not for the weight-streaming kernel, whose offsets have that many."""
+    K, N = 512, 4096
+    lda = -(-(1 << 31) // (M - 1)) + 64  # elements: the last row begins beyond 2^32 bytes
+    lda -= lda % 8
+    assert torch.ops.mlop.gemm_on_ws(M, N, K, 0) and (M - 1) * lda * 2 >= 1 << 32
+    x = torch.empty((M - 1) * lda + K, device=gpu, dtype=bf).as_strided((M, K), (lda, 1))
+    dense, w = operands(gpu, M, N, K)
+    x.copy_(dense)
+    y = dense.double() @ w.double().t()
+    # the result's rounding to bf16, and fp32 sums of K products
+    bound = 2.0 ** -8 * y.abs() + K * 2.0 ** -23 * (dense.double().abs() @ w.double().abs().t())
+    out = torch.empty(M, N, device=gpu, dtype=bf)
+    torch.ops.mlop.gemm(out, x, w, torch.empty(1, device=gpu), 0)
+    assert bool(((out.double() - y).abs() <= bound).all())
