@@ -228,7 +228,7 @@ class LlamaModel:
         return None, ss
 
     def _chain_layer_tp(self, i, a, residual, last, eps, ss):
-        """Tensor-parallel decode chain (M <= decode_chain_max_m()): the row-parallel O / down partial sums are
+        """Tensor-parallel decode chain (M <= GEMV_CHAIN_MAX_M): the row-parallel O / down partial sums are
         all-reduced AND added into the replicated residual in one launch (Group.all_reduce_add,
         K15), gate_up and the next QKV take their rows' RMSNorm factors from the residual chunks
         they stream (gemv.hip PRO_RS).  Two add + RMSNorm launches per layer fewer than

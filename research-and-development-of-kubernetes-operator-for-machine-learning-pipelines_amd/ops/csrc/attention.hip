@@ -1261,7 +1261,8 @@ __device__ __forceinline__ void flash_item_in_turn(
     }
 }
 
-// STREAM (flash_stream op): the persistent grid's tiles as ONE stream of K / V page pairs per
+// STREAM (flash_stream op; off: with a pair's phases in turn, as flash_item_in_turn, with which it tied at two workgroups per CU): the
+// persistent grid's tiles as ONE stream of K / V page pairs per
 // workgroup, so a tile's fixed cost hides under the previous tile's pairs (the 29 us fixed term
 // of profiles/r06_flash_persist.md):
 //   * the 3-deep LDS ring runs across tiles: while the last pairs of tile i are consumed, the

@@ -427,7 +427,7 @@ bool gemm_res_ss(Tensor residual, Tensor a, Tensor w, Tensor ss_out, bool any) {
   re.ss_out = ss_out.data_ptr<float>();
   re.ss_tot = re.ss_out + M * (N / 128);
   c10::DeviceGuard g(a.device());
-  if (mlop::mid_chain_ok((int)M, (int)N, (int)K, 0))  // 5-64 rows: the planner's split-K tiles finish themselves
+  if (mlop::mid_chain_ok((int)M, (int)N, (int)K, 0))  // up to 64 rows: the planner's split-K tiles finish themselves
     return mlop::launch_mid_res_ss(a.data_ptr(), (int)a.stride(0), w.data_ptr(), residual.data_ptr(),
                                    (int)residual.stride(0), (int)M, (int)N, (int)K, re.ss_tot, cur_stream());
   return mlop::launch_w4_chain(4, a.data_ptr(), (int)a.stride(0), w.data_ptr(), residual.data_ptr(),
@@ -466,7 +466,7 @@ bool gemm_rs(Tensor out, Tensor a, Tensor w, Tensor ss_in, double eps, int64_t e
   re.ss_inv_k = 1.f / (float)K;
   re.ss_eps = (float)eps;
   c10::DeviceGuard g(a.device());
-  if (mlop::mid_chain_ok((int)M, (int)N, (int)K, (int)epi))  // 5-64 rows: the planner's SiLU tile, row-scaled
+  if (mlop::mid_chain_ok((int)M, (int)N, (int)K, (int)epi))  // up to 64 rows: the planner's SiLU tile, row-scaled
     return mlop::launch_mid_rs(a.data_ptr(), (int)a.stride(0), w.data_ptr(), out.data_ptr(), (int)out.stride(0),
                                (int)M, (int)N, (int)K, re.ss_in, (float)eps, cur_stream());
   return mlop::launch_w4_chain((int)epi | 8, a.data_ptr(), (int)a.stride(0), w.data_ptr(), out.data_ptr(),
@@ -509,7 +509,7 @@ bool gemm_rs_rope(Tensor q_out, Tensor k_cache, Tensor v_cache, Tensor a, Tensor
   re.ss_in = ss_in.data_ptr<float>() + M * (K / 128);
   re.ss_inv_k = 1.f / (float)K;
   re.ss_eps = (float)eps;
-  if (mlop::mid_chain_ok((int)M, (int)N, (int)K, 3)) {  // 5-64 rows
+  if (mlop::mid_chain_ok((int)M, (int)N, (int)K, 3)) {  // up to 64 rows
     c10::DeviceGuard g(a.device());
     if (mlop::gemm_on_ws((int)M, (int)N, (int)K, 3) && rows_for_ws(a)) {  // row scale computed from the streamed rows
       mlop::launch_ws(a.data_ptr(), (int)a.stride(0), w.data_ptr(), (int)K, nullptr, 0, (int)M, (int)N, (int)K, 3,

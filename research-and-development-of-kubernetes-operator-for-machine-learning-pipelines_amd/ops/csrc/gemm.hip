@@ -51,7 +51,7 @@ __device__ __forceinline__ int swz(int r) { return (r >> 1) & 7; }
 
 
 
-// Mid-M norm chain (5-64 rows, launch_mid_res_ss): the O / down projection's split-K GEMM
+// Mid-M norm chain (above the decode form's rows, up to 64; launch_mid_res_ss): the O / down projection's split-K GEMM
 // finishes itself.  Every split stored its fp32 partial write-through (sc1), waited for it,
 // met its workgroup at a barrier, and one lane draws a relaxed agent-scope ticket on the
 // tile's counter; the split that draws the last ticket reads the partials with sc1 loads only
@@ -1408,7 +1408,10 @@ static bool mid_plan(int M, int N, int K, Plan& p) {
 // With the 224-row tile, 15 shapes at up to 30 row counts from 400 to 8000: it is the best at 62 of 352 points, by more than
 // 2 % at 46 and 0.9 % on average (gate_up of Llama-3-8B at 400 / 892 rows 92 -> 84, 178 -> 165 us, 8192 x 8192 at 5200 495 -> 459);
 // the choice is 0.48 % slower than the best of all six, more than 5 % at 11 points (8192 x 28672 at 400 - 512 rows up to 13 %,
-// 10240 x 8192 at 6600 10 %).
+// 10240 x 8192 at 6600 10 %).  All that was before the four-wave kernel's MFMAs had their present order, which made its rounds 2 - 4 %
+// shorter and the ping-pong kernel's not.  Measured since, 18 shapes at 191 points of 390 - 8192 rows: the choice is 0.12 % slower than
+// the best of all six, more than 5 % at 7 points (5120 x 13824 at 423 rows 23 %, 8192 x 28672 at 417 - 466 7 - 11 %, 6144 x 16384 at
+// 418 - 506 8 %, all on the ping-pong kernel then; 2560 x 8192 at 777, 5120 x 5120 at 793 6 %).
 static bool big_plan(int M, int N, int K, bool pp_ok, Plan& p) {
   const SkBuf* b = sk_buf();
   if (!b || !gemm_w4_ok(M, N, K, K, K)) return false;

@@ -728,7 +728,8 @@ int gemm_grouped_height(const int64_t* rows, int n_groups, int N, int K, int cus
 // The experts' products of a prompt.  What the grid loses is rows of partial tiles and the last round, and both hang on
 // the routing, which only the device knows: the height is chosen here (w4_grouped_height).  gate_up of 8 experts, 256 / 192 / 160 rows: 300 rows each 738 / 619 / 532 us, 350 747 / 595 / 691, 500 779 /
 // 836 / 911, 550 1021 / 836 / 941, 1024 1497 / 1561 / 1598 (1.29 PFLOP/s); over 22 sizes, even and with the experts
-// 0.6 - 1.4 of the mean, the choice is within 1 % of the best of these three on average.  With 224 rows 407 each take 663
+// 0.6 - 1.4 of the mean, the choice is within 1 % of the best of these three on average (all
+// measured before the MFMAs had their present order, which the heights share).  With 224 rows 407 each take 663
 // us where the ping-pong kernel took 735 and the three heights 714 - 745.  One XCD's workgroups share
 // panels and stay in step; each XCD's K walk starts at another eighth, and nothing is loaded between tiles that the
 // stores and the next tile's DMAs would be waited for with (offsets in LDS, gathered rows two tiles ahead): 1661 / 1577

@@ -13,10 +13,10 @@
 //     stream needs; 16 rows x 64 B per instruction, each line in two halves, ran at 6.3 TB/s instead of 6.8 (gate_up of
 //     Llama-3-8B, weights alone: 37.3 -> 34.7 us), and needed the cached path;
 //   * A comes as a wave-private LDS image per step, by LDS-DMA of 4 rows x 256 B.  As MFMA fragments straight from memory its
-//     16-B pieces of 16 rows cost a lookup each: 28672 x 4096 at 16 rows 55.8 -> 41.9 us, 4096 x 14336 28.8 -> 24.3;
+//     16-B pieces of 16 rows cost a lookup each: 28672 x 4096 at 16 rows 55.8 -> 41.9 us, 4096 x 14336 28.8 -> 24.3 (then);
 //   * workgroups start their walk of K at steps that differ.  Rows are a multiple of 4 KB apart: in step they ask the same few
 //     channels (28672 x 4096, 32 rows per workgroup, 50.6 -> 38.7 us; 16 rows 37.6 -> 36.3).
-// What is left: at 16 rows 4096 x 14336 takes 22.9 us, with half of A's image 19.8: weights and A share what a CU can have in
+// What is left: 4096 x 14336 takes 20.1 / 20.9 / 22.2 / 23.4 us at 4 / 8 / 13 / 16 rows (into a residual the same), at 16 with half of A's image 19.8: weights and A share what a CU can have in
 // flight.  The epilogue is 0.8 us of a launch of one workgroup per CU.  Tried and slower: A kept in registers for all tiles of a
 // workgroup (28672 x 4096 39.5 us), four steps in flight (VGPRs for one workgroup fewer), 4 or 16 waves.
 // Epilogues (the decode norm chain, so that a layer has no add + RMSNorm launch):

@@ -194,7 +194,7 @@ void launch_gemv_rope(const void* A, int lda, const void* B, int M, int N, int K
 struct NormPro {
   float eps = 0.f;
 };
-// decode norm chain (gemv.hip PRO_RS / EPI_RES, M <= 4): C = epi(rowscale(A) . B^T) with
+// the decode norm chain's GEMV form (gemv.hip PRO_RS / EPI_RES, M <= 4; the others: decode_chain_takes): C = epi(rowscale(A) . B^T) with
 // rowscale = rsqrt(mean(A_row^2) + eps) (norm weights folded into B); residual += A . B^T
 bool gemv_chain_takes(int M, int N, int K, int epi);
 // weight-streaming MFMA GEMM (gemm_ws.hip), M <= gemm_ws_max_m() (16):

@@ -1,6 +1,7 @@
 """Shares of a sequence's keys in decode attention (attention.hip even_parts / seq_part): launches of 72 to 376 (sequence, kv
-head) pairs, two padding tiles among them, on either side of the lengths from which they are cut (376: of 888 keys on average), alike and with one long sequence, with the host's sums of the
-lengths (AttnMeta.load) and without, combined in the launch and by a second one."""
+head) pairs, two padding tiles among them, on either side of the lengths from which they are cut (376: of 888 keys on average),
+alike and with one long sequence, with the host's sums of the lengths (AttnMeta.load) and without, combined in the launch and
+by a second one."""
 import numpy as np
 import pytest
 import torch
