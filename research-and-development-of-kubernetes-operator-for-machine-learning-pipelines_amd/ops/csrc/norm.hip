@@ -132,24 +132,42 @@ __global__ void __launch_bounds__(256) rmsnorm_wave_kernel(uint16_t* __restrict_
   }
 }
 
-// Rows from which a wave takes a row of H, against the block form's 8 waves (add + norm behind a producer, us, block / wave).
-// Narrow rows: from 256 on (512: 2.5 / 1.75 at 640 rows, 6.9 / 4.3 at 6000; 1024: 3.3 / 2.8, 12.5 / 11.2).  2048: the block
-// form until the pass is bound by memory (256 rows 2.1 / 3.0, 890 3.4 / 4.8, 2300 6.6 / 10.0, 4000 12.1 / 11.8).  4096: where
-// its rows no longer fit the chip at once (256 rows 3.5 / 4.7, 500 5.4 / 5.9, 640 6.5 / 6.7, 1000 8.9 / 8.4, 1600 13.0 / 11.9,
-// 6000 28.9 / 29.4).  8192: never (a lane's 32 loads are 128 registers: 256 rows 5.4 / 8.0, 890 12.6 / 13.3, 2300 23.1 / 25.2,
-// 8000 100 / 107).  At one row the wave form made a decode step 2 % slower.
-static int wave_rows(int H) { return H <= 1024 ? 256 : H == 2048 ? 3200 : H == 4096 ? 700 : 1 << 30; }
+// Where a wave takes a row of H, against the block form's 8 waves (behind a producer, us, block / wave; without the add in brackets).
+// Narrow rows: from 256 on (512: 2.5 / 1.75 at 640 rows, 6.9 / 4.3 at 6000; 1024: 3.3 / 2.8, 12.5 / 11.2).  2048: with the add the
+// block form until the pass is bound by memory (320 rows 2.8 / 3.1, 1150 5.4 / 5.7, 2300 level, 4000 12.1 / 11.8), without it the
+// wave form from 400 on (320 level, 640 (3.3 / 3.1), 1000 (4.15 / 3.95), 1700 (3 % of 4.8)).  4096: where its rows no longer fit the
+// chip at once (320 rows 3.7 / 4.6 (3.2 / 3.6), 640 5.7 / 6.6 (4.8 / 4.9), 1000 level (level), 1600 13.0 / 11.9, 6000 28.9 / 29.4).
+// 8192: the block form (a lane's 32 loads are 128 registers: 320 rows 6.2 / 9.0 (4.9 / 6.2), 1150 16.0 / 19.4 (11.5 / 12.4), 8000 100 /
+// 107).  The wave form has four rows in a workgroup: from 769 to 1024 rows every CU has one and it is at its best where the
+// block form makes another round (2048: 800 rows 4.4 / 4.2, 1000 5.2 / 4.9; 8192: from 705 on, 740 (9.35 / 8.95), 930 (11.7 / 9.6), 1000 (11.8 / 10.1), with the
+// add 13.2 / 13.9 still).  At one row the wave form made a decode step 2 % slower.
+static bool wave_rows(int M, int H, bool add) {
+  const bool one_each = M > 3 * kCus && M <= 4 * kCus;
+  switch (H) {
+    case 512: case 1024: return M >= 256;
+    case 2048: return M >= (add ? 3200 : 400) || one_each;
+    case 4096: return M >= 700;
+    case 8192: return !add && M > kCus * 11 / 4 && M <= 4 * kCus;
+    default: return false;
+  }
+}
 
 template <bool ADD>
 static bool dispatch_wave(uint16_t* out, uint16_t* residual, const uint16_t* x, const uint16_t* w,
                           float eps, int M, int H, hipStream_t st) {
-  if (H % 512 || M < wave_rows(H)) return false;
+  if (!wave_rows(M, H, ADD)) return false;
   const int g = cdiv(M, 4);
   switch (H / 512) {
     case 1: rmsnorm_wave_kernel<1, ADD><<<g, 256, 0, st>>>(out, residual, x, w, eps, M, H); return true;
     case 2: rmsnorm_wave_kernel<2, ADD><<<g, 256, 0, st>>>(out, residual, x, w, eps, M, H); return true;
     case 4: rmsnorm_wave_kernel<4, ADD><<<g, 256, 0, st>>>(out, residual, x, w, eps, M, H); return true;
     case 8: rmsnorm_wave_kernel<8, ADD><<<g, 256, 0, st>>>(out, residual, x, w, eps, M, H); return true;
+    case 16:
+      if constexpr (!ADD) {
+        rmsnorm_wave_kernel<16, ADD><<<g, 256, 0, st>>>(out, residual, x, w, eps, M, H);
+        return true;
+      }
+      return false;
     default: return false;
   }
 }

@@ -21,3 +21,10 @@ def test_either_side(gpu, M, H):
     assert torch.equal(r, r_ref)
     torch.testing.assert_close(y.float(), y_ref.float(), **tol)
     torch.testing.assert_close(ops.rmsnorm(x, w, 1e-5).float(), ref.rmsnorm(x, w, 1e-5).float(), **tol)
+
+
+# where every CU has one workgroup of four rows: its ends, and the rows of 2048 without an add that begin before them
+@pytest.mark.parametrize("M,H", [(399, 2048), (401, 2048), (768, 2048), (769, 2048), (1024, 2048), (1025, 2048), (704, 8192), (705, 8192), (1022, 8192),
+                                 (1024, 8192)])
+def test_one_workgroup_each(gpu, M, H):
+    test_either_side(gpu, M, H)
