@@ -270,8 +270,12 @@ class ProcessLauncher:
         try:
             with open(f.name, "rb") as fh:
                 fh.seek(0, 2)
-                fh.seek(max(0, fh.tell() - 4096))
-                lines = [ln for ln in fh.read().decode("utf-8", "replace").splitlines() if ln.strip()]
+                fh.seek(max(0, fh.tell() - 65536))
+                text = fh.read().decode("utf-8", "replace")
+            at = text.find("Fatal Python error")  # faulthandler's dump: what matters stands first, the last line lists modules
+            if at >= 0:
+                return text[at:at + 8 * n]
+            lines = [ln for ln in text.splitlines() if ln.strip()]
             return (lines[-1] if lines else "")[-n:]
         except OSError:
             return ""

@@ -327,6 +327,22 @@ print(begun, order)
     assert out.stdout.strip().endswith("[True] ['runtime', 'load']"), out.stdout[-300:] + out.stderr[-2000:]
 
 
+def test_reason_of_a_crashed_predictor(tmp_path):
+    """A process that a signal ended leaves faulthandler's dump, whose last line only lists modules: the reason begins with
+    the error and the stacks.  Another one's reason is its log's last line."""
+    from types import SimpleNamespace
+
+    from mlopamd.controller.local import ProcessLauncher
+
+    log = tmp_path / "log"
+    pod = SimpleNamespace(extra={"log": SimpleNamespace(name=str(log))})
+    dump = "Fatal Python error: Segmentation fault\n\nCurrent thread 0x1 (most recent call first):\n  File \"a.py\", line 1 in f\n\n"
+    log.write_text("first words\n" + dump + "Extension modules: " + ", ".join(f"m{i}" for i in range(200)) + " (total: 200)\n")
+    assert ProcessLauncher._log_tail(pod).startswith(dump)
+    log.write_text("first words\nValueError: no such model\n\n")
+    assert ProcessLauncher._log_tail(pod) == "ValueError: no such model"
+
+
 def test_engine_clock_and_tokens_come_from_one_snapshot():
     """the HTTP served rate pairs the engine clock with the token total taken
     at that same instant (one collector over one tuple), never a token count from another step."""
