@@ -20,7 +20,6 @@ from . import reference as ref
 
 _LIB = Path(__file__).resolve().parent / "_C.so"
 _loaded = False
-before_load: list = []  # threads inside the HIP runtime: load() lets them end, since loading registers kernels there
 
 
 class StaleExtension(RuntimeError):
@@ -43,8 +42,6 @@ def load(build_if_missing: bool = True) -> bool:
         from .build import build
 
         build()
-    for t in before_load:
-        t.join()
     torch.ops.load_library(str(_LIB))
     got = torch.ops.mlop.src_hash()
     if got != want:

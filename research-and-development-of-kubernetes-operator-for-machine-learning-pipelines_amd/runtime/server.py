@@ -74,12 +74,12 @@ if __name__ == "__main__":
 
 
 def _warm_hip() -> None:
-    """Initialise the HIP runtime and this rank's device context on a helper thread while the rest
-    of the predictor is imported: the C calls release the GIL, and torch's own first device call
-    then finds the runtime up.  Only between libraries: loading one with device code registers its
-    kernels with the runtime, which walks the registered ones when it initialises.  So torch is
-    loaded before, and ``ops.load`` waits for this thread.  Off for CPU predictors and with
-    MLOP_HIP_WARMUP=0."""
+    """Initialise the HIP runtime and this rank's device context on a helper thread: torch's own first
+    device call then finds the runtime up.  Between libraries: loading one with device code registers its
+    kernels with the runtime, which walks the registered ones when it initialises.  And beside nothing
+    else: a predictor ended twice with signal 11 while the rest of it was imported meanwhile (the second
+    time aiohttp, which has no device code; the cause is not known), so the importing thread waits.  Off for CPU
+    predictors and with MLOP_HIP_WARMUP=0."""
     import ctypes
     import importlib.util
 
@@ -99,7 +99,7 @@ def _warm_hip() -> None:
 
 
 def start_hip_warmup() -> bool:
-    """Start ``_warm_hip`` on a daemon thread in a process that will itself run a GPU engine:
+    """Run ``_warm_hip`` on a thread of its own, to its end, in a process that will itself run a GPU engine:
     the predictor's ``__main__`` once it is known not to be a multi-rank launcher (above), never
     on import as a library.  Off for CPU / sklearn predictors and with MLOP_HIP_WARMUP=0."""
     if (os.environ.get("MLOP_DEVICE", "cuda") == "cpu" or os.environ.get("MLOP_HIP_WARMUP", "1") == "0"
@@ -112,8 +112,8 @@ def start_hip_warmup() -> bool:
     rank_launcher.WARMUP_STARTED = True
     STARTUP["hip_warmup_started"] = True
     t = threading.Thread(target=_warm_hip, name="hip-warmup", daemon=True)
-    ops.before_load.append(t)
     t.start()
+    t.join()  # (40 ms of a start of 0.97 s that it would share with imports)
     return True
 
 

@@ -327,6 +327,21 @@ print(begun, order)
     assert out.stdout.strip().endswith("[True] ['runtime', 'load']"), out.stdout[-300:] + out.stderr[-2000:]
 
 
+def test_nothing_runs_beside_the_hip_warmup(monkeypatch):
+    """The runtime is up, or the attempt over, when start_hip_warmup returns: imports go on behind it."""
+    import time
+
+    from mlopamd.runtime import rank_launcher, server
+
+    done = []
+    for k in ("MLOP_DEVICE", "MLOP_HIP_WARMUP", "MLOP_RUNTIME"):
+        monkeypatch.delenv(k, raising=False)
+    monkeypatch.setattr(server, "_warm_hip", lambda: (time.sleep(0.2), done.append(1)))
+    monkeypatch.setattr(rank_launcher, "WARMUP_STARTED", False)
+    monkeypatch.setattr(server, "STARTUP", {})
+    assert server.start_hip_warmup() and done
+
+
 def test_reason_of_a_crashed_predictor(tmp_path):
     """A process that a signal ended leaves faulthandler's dump, whose last line only lists modules: the reason begins with
     the error and the stacks.  Another one's reason is its log's last line."""
