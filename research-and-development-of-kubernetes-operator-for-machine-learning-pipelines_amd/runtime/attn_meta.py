@@ -8,7 +8,7 @@ see new values on every replay without re-capture.
 Sequence-indexed arrays (q_start, q_len, ctx_len, block_tables) are indexed by
 a stable *row* (the sequence's slot in [0, max_seqs)), so the host only
 touches the rows that changed; tiles (16 MFMA q-rows = 16/G query tokens)
-point at rows.  Rows with a prompt chunk of at least ``flash_min_q`` tokens
+point at rows, in any order.  Rows with a prompt chunk of at least ``flash_min_q`` tokens
 get flash-prefill tiles instead (128 q-rows = 128/G tokens each, ordered
 longest-first over the whole step so the longest causal ranges start first).
 """
@@ -98,6 +98,21 @@ def order_flash_tiles(seq: np.ndarray, q0: np.ndarray, work: np.ndarray) -> None
     seq[:] = seq[o]
     q0[:] = q0[o]
     work[:] = work[o]
+
+
+# Decode tiles longest first, where a launch has more (sequence, kv head) pairs than the card CUs: a CU holds three of the
+# kernel's workgroups, so from then on some CUs have more of them than others, and above 768 the last ones start when the first
+# have ended; with the longest first what starts late or shares a CU is short.  us per launch, in the order of the rows -> longest
+# first, 8 kv heads: 33 x 1000 keys 28.9 -> 28.2, 64 x 1000 44.8 -> 42.4, 100 x 1000 73.5 -> 66.7, 200 x 1000 132.5 -> 126.5 (lengths
+# 0.75 - 1.25 of the mean), 700 x 500 222 -> 223; log-normal lengths (sigma 0.8) 128 x 700 72.9 -> 65.4, 256 x 1024 186 -> 153,
+# 700 x 400 193 -> 175.  Not below: 20 x 800 16.9 and 17.0, 2 kv heads 48 x 2000 22.9 and 23.3, 96 x 1000 21.0 and 21.2.  (Above it
+# 2 heads 150 x 1500 45.0 -> 43.9, 200 x 1000 38.3 -> 38.9.)  Costs the host 2 us at 100 sequences, 12 at 1000.
+DECODE_LPT_PAIRS = 256
+
+
+def order_decode_rows(rows: np.ndarray, ctx_lens: np.ndarray) -> np.ndarray:
+    """``rows`` by descending context length.  A tile finds its token by its row (q_start), so their order is free."""
+    return rows[np.argsort(ctx_lens)[::-1]]
 
 
 def plan_partitions(num_tiles: int, n_kv: int, max_ctx: int, min_part: int | None = None,
@@ -361,7 +376,7 @@ class MetaBuffers:
         p = (ctx_lens - 1).astype(np.int32)
         pos_h[:B] = p
         slot_h[:B] = self.bt_h[rows, p // BLOCK_SIZE] * BLOCK_SIZE + p % BLOCK_SIZE
-        ts_h[:B] = rows
+        ts_h[:B] = order_decode_rows(rows, ctx_lens) if B * self.n_kv > DECODE_LPT_PAIRS else rows
         tq_h[:B] = 0
         qs_h[rows] = np.arange(B, dtype=np.int32)
         ql_h[rows] = 1

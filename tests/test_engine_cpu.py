@@ -425,3 +425,24 @@ def test_flash_keys_reach_every_rank():
     assert sync.recv(Eng) == (KIND_EAGER, T, nt, nl, 1024, 1, 0, mb.npt, 1, sum(tiles)) and sync.g.sent.numel() == n == mb.extent(5)
     mb.fill_decode(np.array([1], np.int32), np.array([9], np.int32), np.zeros(1, np.int64), pad_to=1)
     assert mb.npt == mb.pkeys == 0
+
+
+@pytest.mark.parametrize("n", [1, 31, 32, 33, 100])
+def test_decode_tiles_longest_first(n):
+    """Decode tiles in the order of the rows up to one (sequence, kv head) pair per CU, above it longest first; every other array
+    stays in the order of the batch, and padding behind all of them."""
+    from mlopamd.runtime.attn_meta import MetaBuffers
+
+    mb = MetaBuffers(128, 128, 64, 4, 8, 1024, "cpu")
+    mb.bt_h[:] = np.arange(mb.bt_h.size, dtype=np.int32).reshape(mb.bt_h.shape)
+    rng = np.random.default_rng(n)
+    rows, ctx = rng.permutation(120)[:n].astype(np.int32), rng.integers(1, 1024, n).astype(np.int32)
+    mb.fill_decode(rows, ctx, np.arange(n), pad_to=n + 2)
+    tiles = mb.view_h("tile_seq")[:n].tolist()
+    assert tiles == rows.tolist() if 8 * n <= 256 else sorted(tiles) == sorted(rows.tolist())
+    if 8 * n > 256:
+        assert (np.diff(mb.view_h("ctx_len")[tiles]) <= 0).all()
+    assert mb.view_h("tile_seq")[n:n + 2].tolist() == [126, 127] and not mb.view_h("tile_q0")[:n + 2].any()
+    assert mb.view_h("q_start")[rows].tolist() == list(range(n)) == mb.ids_hn[:n].tolist()
+    assert mb.view_h("positions")[:n].tolist() == (ctx - 1).tolist()
+    assert mb.view_h("slots")[:n].tolist() == [int(mb.bt_h[r, (c - 1) // 16]) * 16 + (c - 1) % 16 for r, c in zip(rows, ctx)]
