@@ -622,18 +622,22 @@ void gemm_grouped_plan(int bm, int bn, int stages, int splits) {
 
 // dense-plan override (scripts/bench_mid_m.py sweeps the mid-M projection tilings in one
 // process): variant (0 = gemm_kernel BM x BN, 1 = 256x256 two-stage, 3 = ping-pong, 5 =
-// four-wave, 6 = four-wave of BM 160, 192 or 224 rows, else half height), BM, BN, K splits (plain gemm_kernel only), LDS
+// four-wave, 6 = four-wave of BM 160, 192 or 224 rows, else half height, 8 = four-wave of BM rows over K ranges, behind
+// gemm_add_rmsnorm only; one range: no such form), BM, BN, K splits (0 and 8 only), LDS
 // ring depth of the small tiles (0 = the default); -1 = the planner's own choice
 static int g_dp[5] = {-1, -1, -1, -1, 0};
+static int g_slab[2] = {0, 0};  // variant 8's tile height (0: slab_plan's choice) and ranges
 void gemm_dense_plan(int variant, int bm, int bn, int splits, int stages) {
-  if (variant >= 0 && variant != 0 && variant != 1 && variant != 3 && variant != 5 && variant != 6)
-    throw std::runtime_error("gemm_dense_plan: variant must be 0, 1, 3, 5 or 6");
+  if (variant >= 0 && variant != 0 && variant != 1 && variant != 3 && variant != 5 && variant != 6 && variant != 8)
+    throw std::runtime_error("gemm_dense_plan: variant must be 0, 1, 3, 5, 6 or 8");
   if (variant == 0) {
     static const int ok[][2] = {{16, 32}, {16, 64}, {32, 32}, {32, 64}, {64, 32}, {64, 64}, {96, 64}, {128, 64}, {192, 64}, {256, 64}, {256, 128}};
     bool found = false;
     for (const auto& t : ok) found = found || (t[0] == bm && t[1] == bn);
     if (!found) throw std::runtime_error("gemm_dense_plan: no dense config for this tile");
   }
+  g_slab[0] = variant == 8 ? bm : 0, g_slab[1] = splits;
+  if (variant == 8) variant = -1;  // (the plain plans keep their choice)
   g_dp[0] = variant, g_dp[1] = bm, g_dp[2] = bn, g_dp[3] = splits, g_dp[4] = stages > 0 ? stages : 0;
 }
 
@@ -1412,11 +1416,11 @@ static bool mid_plan(int M, int N, int K, Plan& p) {
 // shorter and the ping-pong kernel's not.  Measured since, 18 shapes at 191 points of 390 - 8192 rows: the choice is 0.12 % slower than
 // the best of all six, more than 5 % at 7 points (5120 x 13824 at 423 rows 23 %, 8192 x 28672 at 417 - 466 7 - 11 %, 6144 x 16384 at
 // 418 - 506 8 %, all on the ping-pong kernel then; 2560 x 8192 at 777, 5120 x 5120 at 793 6 %).
-static bool big_plan(int M, int N, int K, bool pp_ok, Plan& p) {
+struct W4Tile { int rows; float round, slope; };
+constexpr W4Tile kW4Tiles[] = {{256, 1.f, .3f}, {224, .90f, .28f}, {192, .805f, .25f}, {160, .70f, .1f}, {128, .632f, 0.f}};
+static bool big_plan(int M, int N, int K, bool pp_ok, Plan& p, float* us_out = nullptr) {
   const SkBuf* b = sk_buf();
   if (!b || !gemm_w4_ok(M, N, K, K, K)) return false;
-  struct Tile { int rows; float round, slope; };
-  constexpr Tile tiles[] = {{256, 1.f, .3f}, {224, .90f, .28f}, {192, .805f, .25f}, {160, .70f, .1f}, {128, .632f, 0.f}};
   const float full = 6.f + 0.0207f * (float)K, C = (float)b->cus;
   const int nk = K / kBK;
   float best = 1e30f;
@@ -1429,7 +1433,7 @@ static bool big_plan(int M, int N, int K, bool pp_ok, Plan& p) {
     const float tail = d ? 1.1f * live * sk_tail_cost(r, nk, d) / (float)nk : r > 0 ? 1.f : 0.f;
     best = (13.5f + 0.0206f * (float)K) * ((float)q + tail);
   }
-  for (const Tile& t : tiles) {
+  for (const W4Tile& t : kW4Tiles) {
     if (t.rows < 256 && !g_half_tile) break;
     const long T = (long)((M + t.rows - 1) / t.rows) * (N / 256), q = T / b->cus, r = T % b->cus;
     // (From five whole rounds on the 224-row tile counts more.  By itself it does not need to: over 56 products of five
@@ -1448,6 +1452,7 @@ static bool big_plan(int M, int N, int K, bool pp_ok, Plan& p) {
       p.BM = t.rows;
     }
   }
+  if (us_out) *us_out = best;
   return true;
 }
 
@@ -1910,8 +1915,52 @@ void gemm_plan(int M, int N, int K, int out[5]) {
 
 // fp32 slabs of the K ranges: of a plain product, and (add_norm) of one with the residual add + RMSNorm behind it, for which 0
 // also says that there is no such form; the weight-streaming kernel's has none, but A's rows may not suit it
+// GEMM + residual add + RMSNorm above 256 rows: the four-wave kernel over K in 2 - 8 ranges, one workgroup per (tile, range), its
+// fp32 slabs summed by the pass that adds and norms anyway.  A grid of few tiles fills the CUs with whole tiles so: what the
+// K-half hand-over and the stream-K tail send through one workgroup of a tile (a CU takes in 50 GB/s of what is not in its L2) is read by
+// all CUs, and the 128-row tiles, which halves need to fill the chip and whose loop waits for its loads (48 KB a K-tile in
+// 0.73 us, of its 0.78), give way to taller ones.  us, GEMM + add + norm as it was -> so: 4096 x 14336 at 390 / 600 / 892 rows 71 -> 57, 100 -> 72,
+// 113 -> 91, 4096 x 4096 at 390 / 640 38.4 -> 31, 42 -> 36, 8192 x 8192 at 330 80 -> 62, 8192 x 28672 at 390 217 -> 176.  (Slabs stored
+// non-temporal: 101 instead of 91.)
+// By estimated time: a range takes what big_plan says of its K, 4.5 us for 4-byte stores; the pass 3.1 us and its bytes at 8.3
+// TB/s, the plain pass 3 and 6.  14 shapes and 250 drawn ones at 257 - 3000 rows: the choice of tile and ranges is 1 % off the best.
+// Up to 320 rows the weight stream is the faster of small matrices (257 x 4096 x 7168 33.1 us, slabs 36.1; 270 x 5120 x 13824
+// 68.8 and 60.9), so it is of narrow ones with K in 8 ranges (334 x 1536 x
+// 19008, 144 workgroups, 41.5 and 45.6); K below 1536 is too short to cut (266 x 1024 x 1088 14.9 and 19.1), as are grids of less
+// than 96 workgroups (335 x 768 x 1984 16.7 and 19.3).
+static bool slab_plan(int M, int N, int K, int& bm, int& splits) {
+  if (g_slab[0] > 0) {  // bench override (gemm_dense_plan)
+    bm = g_slab[0];
+    splits = g_slab[1];
+    return splits > 1;
+  }
+  const SkBuf* b = sk_buf();
+  if (!b || g_dp[0] >= 0 || M <= 256 || K < 1536 || !gemm_w4_ok(M, N, K, K, K) || (long)M * N * 4 >= (1l << 31)) return false;
+  if (M < 320 && (long)N * K < 60l << 20) return false;
+  const int nk = K / kBK;
+  const float C = (float)b->cus, mn = (float)M * (float)N * 1e-6f;
+  float best = 1e30f;
+  int wgs = 0;
+  for (const W4Tile& t : kW4Tiles) {
+    const int T = (M + t.rows - 1) / t.rows * (N / 256);
+    for (int s = 2; s <= kMaxSplits && s * T <= b->cus && nk / s >= 6; ++s) {
+      if (s * T < 96) continue;
+      const float one = (6.f + 0.0207f * (float)((nk + s - 1) / s * kBK)) * t.round;
+      const float us = one * (1.f - t.slope * (1.f - (float)(T * s) / C)) + 4.5f + 3.1f + mn * (4.f * (float)s + 6.f) / 8.3f;
+      if (us < best) best = us, bm = t.rows, splits = s, wgs = s * T;
+    }
+  }
+  if (wgs == 0) return false;
+  Plan p = plan(M, N, K, false, 0, 0);
+  if (p.variant == 7) return wgs >= 160;
+  if (p.splits > 1) return true;
+  float us = 0.f;
+  return big_plan(M, N, K, true, p, &us) && best * 1.03f + (K < 2600 ? 2.f : 0.f) < us + 3.f + mn * 8.f / 6.f;
+}
+
 long gemm_workspace_floats(int M, int N, int K, int epi, bool add_norm) {
   if (epi_act(epi)) epi = EPI_NONE;
+  if (int bm, s; add_norm && slab_plan(M, N, K, bm, s)) return (long)s * M * N;
   if (gemv_takes(M, N, K, epi) || (!add_norm && gemm_on_ws(M, N, K, epi))) return 0;
   const Plan p = plan(M, N, K, false, 0, 0);
   return p.splits > 1 ? (long)p.splits * M * N : 0;
@@ -1969,12 +2018,17 @@ bool launch_gemm_add_rmsnorm(const void* A, int lda, const void* B, void* out, v
     launch_rmsnorm(out, residual, w, eps, M, N, st);
     return true;
   }
-  int splits;
-  const Plan p = plan(M, N, K, false, 0, 0);
-  if (p.splits <= 1 || p.splits > kMaxSplits || (long)p.splits * M * N > ws_floats || N % 8) return false;
-  launch_plan<EPI_NONE, false>(p, (const uint16_t*)A, lda, (const uint16_t*)B, K, nullptr, N, ws,
-                               M, N, K, nullptr, 0, st);
-  splits = p.splits;
+  int splits, bm;
+  if (slab_plan(M, N, K, bm, splits) && (long)splits * M * N <= ws_floats && gemm_w4_ok(M, N, K, lda, K) &&
+      K / kBK / splits >= 3 && (long)M * N * 4 < (1l << 31)) {
+    run_w4_slab((const uint16_t*)A, lda, (const uint16_t*)B, K, ws, M, N, K, splits, bm, st);
+  } else {
+    const Plan p = plan(M, N, K, false, 0, 0);
+    if (p.splits <= 1 || p.splits > kMaxSplits || (long)p.splits * M * N > ws_floats || N % 8) return false;
+    launch_plan<EPI_NONE, false>(p, (const uint16_t*)A, lda, (const uint16_t*)B, K, nullptr, N, ws,
+                                 M, N, K, nullptr, 0, st);
+    splits = p.splits;
+  }
   const int nvec = N / 8;
   int vpt = 1;
   while (vpt < 8 && nvec / vpt > 512) vpt <<= 1;

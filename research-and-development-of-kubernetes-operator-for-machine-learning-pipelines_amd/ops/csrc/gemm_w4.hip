@@ -36,8 +36,9 @@ namespace mlop {
 namespace {
 // epilogue = base (bits 0-1) | flags: W4_ADD_SS (plain base only) C += A.B^T in place with the
 // per-row sum-of-squares partials of the new C; W4_RS rows scaled by the RMSNorm factor from
-// re.ss_in (launch.h RopeEpi; the norm chain of launch_w4_chain)
-enum { W4_NONE = 0, W4_SILU_MUL = 1, W4_ROPE = 3, W4_ADD_SS = 4, W4_RS = 8 };
+// re.ss_in (launch.h RopeEpi; the norm chain of launch_w4_chain).  W4_SLAB: K in ranges, fp32 slabs [range][M][N] in C
+// (run_w4_slab; one item per workgroup, nothing prefetched behind it)
+enum { W4_NONE = 0, W4_SILU_MUL = 1, W4_SLAB = 2, W4_ROPE = 3, W4_ADD_SS = 4, W4_RS = 8 };
 using i32x4 = __attribute__((ext_vector_type(4))) int;
 typedef __attribute__((address_space(3))) uint16_t lds_u16;
 
@@ -178,6 +179,13 @@ __device__ __forceinline__ void gemm_w4_tiles(
   // i < NI A rows 8p.., else B rows 8(p - 4 NI).. (B starts at LDS byte 128 BMT); lane -> row
   // 8p + lane / 8, LDS slot lane % 8 holds source chunk (lane % 8) ^ swz(row)
   auto item = [&](int i, int& m0, int& n0, int& m_end, uint32_t& b0, int& kb, int& nkl) {
+    if constexpr (BASE == W4_SLAB) {  // range by range: an XCD's items share their panels' columns
+      const int sp = i / n_dp, ns = n_items / n_dp;
+      origin(i % n_dp, m0, n0, m_end, b0);
+      kb = sp * nk / ns;
+      nkl = (sp + 1) * nk / ns - kb;
+      return;
+    }
     const bool tail = i >= n_dp;
     origin(tail ? n_dp + ((i - n_dp) >> 1) : i, m0, n0, m_end, b0);
     kb = tail ? ((i - n_dp) & 1) * (nk >> 1) : 0;
@@ -357,7 +365,7 @@ __device__ __forceinline__ void gemm_w4_tiles(
     // epilogue (MI355X_MICROARCH.md "Valid forms"; the gemm_pp_kernel stream-K hand-off).  A
     // tail item is its workgroup's last, so no prefetch is in flight and the LDS is free for
     // the flag.  own + other is commutative: bit-identical whichever half arrives last.
-    const bool part = it >= n_dp;
+    const bool part = BASE != W4_SLAB && it >= n_dp;
     const int sidx = part ? it - n_dp : 0;
     const auto rs_other = __builtin_amdgcn_make_buffer_rsrc(part ? ws + (size_t)(sidx ^ 1) * 65536 : (float*)C, 0,
                                                            65536 * 4, 0x00020000);
@@ -432,7 +440,20 @@ __device__ __forceinline__ void gemm_w4_tiles(
       // partner's y (cols 0-3), hi = own y (cols 4-7)
       out = u32x4{pack2(lo[0], lo[1]), pack2(lo[2], lo[3]), pack2(hi[0], hi[1]), pack2(hi[2], hi[3])};
     };
-    if constexpr (BASE == W4_ROPE) {
+    if constexpr (BASE == W4_SLAB) {
+      const auto rs_ws = __builtin_amdgcn_make_buffer_rsrc((float*)C + (size_t)(it / n_dp) * M * N, 0, (int)((uint32_t)M * (uint32_t)N * 4u),
+                                                           0x00020000);
+      unroll<NI>([&](auto I_) {
+        constexpr int I = decltype(I_)::value;
+        float v[32];
+        read_block<I>(v);
+        const uint32_t off = ((uint32_t)(m0 + lr + I * 16) * (uint32_t)N + (uint32_t)(n0 + wn * 128 + 4 * qd)) * 4u;
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          __builtin_amdgcn_raw_buffer_store_b128(u32x4{__float_as_uint(v[4 * j]), __float_as_uint(v[4 * j + 1]), __float_as_uint(v[4 * j + 2]),
+                                                       __float_as_uint(v[4 * j + 3])}, rs_ws, off + 64u * j, 0, 0);
+      });
+    } else if constexpr (BASE == W4_ROPE) {
       // RoPE + paged cache from the accumulators: a wave's 128 columns are ONE head, and a
       // lane's rotate-half partners (c, c + 64) sit in acc(i, j) / acc(i, j + 4) element r of the
       // same lane, so nothing is staged in LDS (which stays free for the next tile's prefetch).
@@ -839,6 +860,28 @@ static bool run_w4_t(const uint16_t* A, int lda, const uint16_t* B, int ldb, uin
   }
   kern<<<grid, 256, lds, st>>>(A, lda, B, ldb, C, ldc, M, N, K, gx, gy, gm, re2, n_dp, n_items, ws, cnt);
   return true;
+}
+
+// K in `splits` ranges, one workgroup per (tile, range): fp32 slabs ws[range][M][N].  At most one item per CU, three K-tiles or more each.
+template <int BMT>
+static void run_w4_slab_t(const uint16_t* A, int lda, const uint16_t* B, int ldb, float* ws, int M, int N, int K, int splits, hipStream_t st) {
+  constexpr size_t lds = 2ull * 65536;
+  auto kern = gemm_w4_kernel<W4_SLAB, BMT>;
+  static const bool attr =
+      hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess;
+  (void)attr;
+  const int gx = N / 256, gy = (M + BMT - 1) / BMT, T = gx * gy, gm = std::max(1, std::min(1024 / BMT, gy));
+  RopeEpi re{};
+  re.k_walk = w4_k_walk(N, K, gm * gx, kCus);
+  kern<<<T * splits, 256, lds, st>>>(A, lda, B, ldb, (uint16_t*)ws, N, M, N, K, gx, gy, gm, re, T, T * splits, nullptr, nullptr);
+}
+
+void run_w4_slab(const uint16_t* A, int lda, const uint16_t* B, int ldb, float* ws, int M, int N, int K, int splits, int bm, hipStream_t st) {
+  if (bm == 128) run_w4_slab_t<128>(A, lda, B, ldb, ws, M, N, K, splits, st);
+  else if (bm == 160) run_w4_slab_t<160>(A, lda, B, ldb, ws, M, N, K, splits, st);
+  else if (bm == 192) run_w4_slab_t<192>(A, lda, B, ldb, ws, M, N, K, splits, st);
+  else if (bm == 224) run_w4_slab_t<224>(A, lda, B, ldb, ws, M, N, K, splits, st);
+  else run_w4_slab_t<256>(A, lda, B, ldb, ws, M, N, K, splits, st);
 }
 
 // (a_n: A's rows where a_rows picks them; the kernel's offsets are 32 bits and its tables hold 64 experts)

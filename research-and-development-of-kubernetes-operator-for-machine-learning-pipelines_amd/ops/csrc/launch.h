@@ -158,6 +158,7 @@ bool gemm_sk_available(int* cus);
 bool run_w4(int epi, const uint16_t* A, int lda, const uint16_t* B, int ldb, uint16_t* C, int ldc, int M, int N,
             int K, hipStream_t st, const RopeEpi& re, int bm = 256);
 // the experts' products on it (offsets on the device; a_n: A's rows)
+void run_w4_slab(const uint16_t* A, int lda, const uint16_t* B, int ldb, float* ws, int M, int N, int K, int splits, int bm, hipStream_t st);
 bool gemm_w4_grouped_ok(int M, int N, int K, int n_groups, int a_n);
 void run_w4_grouped(int epi, const uint16_t* A, int lda, const uint16_t* B, int ldb, uint16_t* C, int ldc, int M, int N,
                     int K, hipStream_t st, const RopeEpi& re, const int* offsets, int n_groups);
