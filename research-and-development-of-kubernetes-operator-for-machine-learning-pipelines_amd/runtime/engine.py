@@ -372,7 +372,10 @@ class Engine:
         self.seqs: dict[int, Sequence] = {}
         self._ids = itertools.count()
         self._decode_since_prefill = 0
-        self.graphs: dict[int, tuple] = {}
+        self.graphs: dict[int, tuple] = {}  # rows -> (graph of a step up to the final norm, what its logits are written into)
+        self._graph_hidden: dict[int, torch.Tensor] = {}  # what a graph leaves for the head
+        self._logits_buf: torch.Tensor | None = None
+        self._own_logits = False  # the next graph step's logits go into a tensor of their own
         self.graph_pool = None
         self.stats = collections.Counter()
         # one-step-ahead (async) scheduling state: the in-flight step, its token read-back
@@ -1256,7 +1259,11 @@ class Engine:
         bucket = next((b for b in self.buckets if b >= B), None)
         if not portions and self.graphs.get(bucket) is not None:
             self.meta.fill_decode(rows, ctx, last, pad_to=bucket)
-            logits = self._launch(KIND_GRAPH, bucket, bucket, bucket, 0, 0, bucket)
+            self._own_logits = True
+            try:
+                logits = self._launch(KIND_GRAPH, bucket, bucket, bucket, 0, 0, bucket)
+            finally:
+                self._own_logits = False
         else:
             T, nt, nl = self.meta.fill_mixed(rows, ctx, last, [s.row for s, _, _ in portions],
                                              [len(toks) for _, toks, _ in portions], p_ctx,
@@ -1272,8 +1279,7 @@ class Engine:
             return None
         # the device is not waited for: a caller may feed the next step while this one runs
         if self.model.ps.tp.size == 1 and idx == list(range(len(idx))):
-            rows = logits[:len(idx)]
-            return rows if portions or self.graphs.get(bucket) is None else rows.clone()  # (the graphs' one buffer)
+            return logits[:len(idx)]
         at_d = torch.tensor(idx, pin_memory=logits.is_cuda).to(logits.device, non_blocking=True)
         return logits[at_d]
 
@@ -1334,9 +1340,10 @@ class Engine:
         if self._inject_device_us:  # fault injection: this step is slower on the device only
             torch.ops.mlop.device_delay(self._inject_device_us)
         if kind == KIND_GRAPH:
-            graph, logits_buf = self.graphs[bucket]
-            graph.replay()
-            return self._gather(logits_buf, greedy)
+            self.graphs[bucket][0].replay()
+            # the head is launched behind the graph: it writes into the engine's one buffer or, for a caller that keeps the
+            # logits (feed), into a tensor of their own, where a copy of 700 rows of 128256 took 62 us of a step of 4 ms
+            return self._gather(self._head(bucket, self._own_logits), greedy)
         meta = self.meta.meta(T, nt, nl, part, nparts, npt, pkeys)
         hidden = self.model.forward(self.meta.ids_d[:T], meta, self.kv)
         if nl == 0:
@@ -1415,8 +1422,13 @@ class Engine:
             return bool(safe)
         return all(ops.gemm_is_native(*w.shape[-2:]) for w in m.weight_tensors() if w.dim() > 1)
 
+    def _head(self, bucket: int, own: bool = False) -> torch.Tensor:
+        """This rank's logits of the decode graph's rows, in the engine's buffer unless they are the caller's (``own``)."""
+        hidden, buf = self._graph_hidden[bucket], self._logits_buf
+        return self.model.logits_local(hidden) if own or buf is None else self.model.logits_local(hidden, out=buf[:bucket])
+
     def capture_graphs(self):
-        """Capture one decode graph per batch bucket: the listed ones largest first, each run once before, then the added
+        """Capture one decode graph per batch bucket, up to the head: the listed ones largest first, each run once before, then the added
         ones, which share their kernels and are only captured (2 ms a graph of 32 layers, where a run before it takes
         another 9; shared pool).  Llama-3-8B at 2048 rows: 32 graphs, 20 of them added, 438 -> 130 ms; the 12 listed
         ones, each run first and waited for, took 140."""
@@ -1428,8 +1440,7 @@ class Engine:
         t0 = time.perf_counter()
         verbose = False
         # one graph replays at a time and its logits are read before the next does: all write into one buffer
-        buf = m.logits_buffer(self.buckets[-1]) if hasattr(m, "logits_buffer") else None
-        logits_of = lambda h, b: m.logits_local(h) if buf is None else m.logits_local(h, out=buf[:b])  # noqa: E731
+        self._logits_buf = m.logits_buffer(self.buckets[-1]) if hasattr(m, "logits_buffer") else None
         alone = self._native_products()
         added = [b for b in self.buckets if b not in self.listed_buckets] if alone else []
         order = sorted((b for b in self.buckets if b not in added), reverse=True) + added[::-1]
@@ -1447,7 +1458,8 @@ class Engine:
                 # in order: logits_idx is the identity, so the graph skips the row gather
                 if b not in added:  # warm-up (allocator, autotune, lazy init); the device may run it during the capture
                     self.meta.upload(b, b)
-                    logits_of(m.forward(ids, meta, self.kv), b)
+                    self._graph_hidden[b] = m.forward(ids, meta, self.kv)
+                    self._head(b)
                 if bi == 0 or not alone:  # (a communicator's watchdog may ask for its events, which a capture forbids)
                     torch.cuda.synchronize(self.device)
                 if bi == 0:  # the widest warm-up's memory is the graphs' now
@@ -1458,10 +1470,10 @@ class Engine:
                 g = torch.cuda.CUDAGraph()
                 g.capture_begin(pool=self.graph_pool)
                 try:
-                    logits = logits_of(m.forward(ids, meta, self.kv), b)
+                    self._graph_hidden[b] = m.forward(ids, meta, self.kv)
                 finally:
                     g.capture_end()
-                self.graphs[b] = (g, logits)
+                self.graphs[b] = (g, None if self._logits_buf is None else self._logits_buf[:b])
         torch.cuda.current_stream(self.device).wait_stream(stream)
         torch.cuda.synchronize(self.device)
         torch.cuda.empty_cache()
