@@ -627,6 +627,7 @@ void launch_paged_attention(void* out, float* part_o, float* part_ml, const void
 // 500 61 -> 62 -> 60.5, 64 x 100 36 -> 38.5 -> 37.5.
 using f32x16 = __attribute__((ext_vector_type(16))) float;
 constexpr int kFlashRing = 4;  // pairs in flash_item's rings
+constexpr int kFlashSplits = 16, kFlashPart = 128 * 128 + 2 * 128;  // most key ranges of a tile; floats of one: O, (max, sum) by rows
 constexpr float kRescaleLog2 = 8.f;  // flash prefill's deferred-rescale threshold (exp2 units)
 // two floats -> one dword of two bf16 in ONE v_cvt_pk_bf16_f32 (pack2's two scalar casts
 // become two cvt + shift + or)
@@ -668,14 +669,15 @@ __device__ __forceinline__ void mfma16_settle(f32x4 (&c)[8][2]) {
                  "+v"(c[4][0]), "+v"(c[4][1]), "+v"(c[5][0]), "+v"(c[5][1]), "+v"(c[6][0]), "+v"(c[6][1]), "+v"(c[7][0]), "+v"(c[7][1]));
 }
 
-// one flash tile (128 q-rows of ONE kv head against its whole causal key range)
-template <int G>
+// one flash tile (128 q-rows of ONE kv head against its whole causal key range, or, SPLIT, pairs n split / n_splits .. of its n
+// pairs: O unnormalised [128][128] and (max, sum) [128][2] of the rows to part)
+template <int G, bool SPLIT>
 __device__ __forceinline__ void flash_item(
     uint16_t* smem, int tile, int kvh, uint16_t* __restrict__ out, const uint16_t* __restrict__ q,
     const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc, const int* __restrict__ block_tables,
     int bt_stride, const int* __restrict__ ptile_seq, const int* __restrict__ ptile_q0,
     const int* __restrict__ q_start, const int* __restrict__ q_len, const int* __restrict__ ctx_len, int Hq,
-    int Hkv, float scale_log2, int num_blocks) {
+    int Hkv, float scale_log2, int num_blocks, int split, int n_splits, float* __restrict__ part) {
   constexpr int QB = 128 / G;            // query tokens per workgroup
   constexpr int STAGES = kFlashRing;
   constexpr int STAGE = 4 * kBS * kD;    // bf16 per stage: K page A | K page B | V page A | V page B
@@ -684,10 +686,19 @@ __device__ __forceinline__ void flash_item(
   const int s = ptile_seq[tile], q0 = ptile_q0[tile];
   const int ql = q_len[s], ctx = ctx_len[s], qs = q_start[s];
   const int last_q = min(q0 + QB, ql) - 1;
-  const int kv_end = ctx - ql + last_q + 1;
+  int kv_end = ctx - ql + last_q + 1, first_key = 0;
+  if constexpr (SPLIT) {  // keys and positions from the range's first key on
+    const int n = (kv_end + 31) >> 5, from = n * split / n_splits, to = n * (split + 1) / n_splits;
+    if (from == to) {  // (no pair of a tile of few)
+      if (threadIdx.x < 128) *reinterpret_cast<u32x2*>(part + 128 * 128 + 2 * threadIdx.x) = u32x2{0, 0};
+      return;
+    }
+    first_key = 32 * from;
+    kv_end = min(kv_end, 32 * to) - first_key;
+  }
   const int n_pairs = (kv_end + 31) >> 5;
   const int n_pages = (kv_end + kBS - 1) / kBS;
-  const int wg_min_pos = ctx - ql + q0;
+  const int wg_min_pos = ctx - ql + q0 - first_key;
   const int r16 = lane & 15, g4 = lane >> 4;
 
   // this lane's two q rows (MFMA columns): R = 32 wid + 16 qb + r16
@@ -700,7 +711,7 @@ __device__ __forceinline__ void flash_item(
     const int R = 32 * wid + 16 * b + r16;
     qi[b] = q0 + R / G;
     q_ok[b] = qi[b] < ql;
-    pos_r[b] = q_ok[b] ? ctx - ql + qi[b] : -1;
+    pos_r[b] = q_ok[b] ? ctx - ql + qi[b] - first_key : -1;  // (before the range: all of it masked, sums of 0)
     const uint16_t* qrow = q + ((size_t)(qs + (q_ok[b] ? qi[b] : 0)) * Hq + kvh * G + R % G) * kD + 8 * g4;
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
@@ -715,7 +726,7 @@ __device__ __forceinline__ void flash_item(
 #pragma unroll
     for (int b = 0; b < 2; ++b) o[d][b] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  const int* bt = block_tables + (size_t)s * bt_stride;
+  const int* bt = block_tables + (size_t)s * bt_stride + first_key / kBS;
   const uint32_t page_bytes = (uint32_t)Hkv * (2 * PAGE);
   const int kkey = wid * 4 + (lane >> 4);
   const int ksw = (kkey >> 3) * 4 + (kkey & 3);  // (page B: + 8)
@@ -1016,6 +1027,13 @@ __device__ __forceinline__ void flash_item(
   for (int b = 0; b < 2; ++b) {
     const float sum = sum_x16_x32(l[b]);
     if (!q_ok[b]) continue;
+    if constexpr (SPLIT) {
+      const int R = 32 * wid + 16 * b + r16;
+#pragma unroll
+      for (int d = 0; d < 8; ++d) *reinterpret_cast<f32x4*>(part + R * 128 + 16 * d + 4 * g4) = o[d][b];
+      if (g4 == 0) *reinterpret_cast<u32x2*>(part + 128 * 128 + 2 * R) = u32x2{__float_as_uint(m[b]), __float_as_uint(sum)};
+      continue;
+    }
     const float inv = sum > 0.f ? 1.f / sum : 0.f;
     uint16_t* orow = out + ((size_t)(qs + qi[b]) * Hq + kvh * G + (32 * wid + 16 * b + r16) % G) * kD + 4 * g4;
 #pragma unroll
@@ -1634,17 +1652,70 @@ __global__ void __launch_bounds__(256, WPC) flash_prefill_kernel(
     flash_item_in_turn<G>(smem, blockIdx.x / Hkv, blockIdx.x % Hkv, out, q, kc, vc, block_tables, bt_stride, ptile_seq,
                           ptile_q0, q_start, q_len, ctx_len, Hq, Hkv, scale_log2, num_blocks);
   } else if constexpr (!PERSIST) {
-    flash_item<G>(smem, blockIdx.x / Hkv, blockIdx.x % Hkv, out, q, kc, vc, block_tables, bt_stride, ptile_seq,
-                    ptile_q0, q_start, q_len, ctx_len, Hq, Hkv, scale_log2, num_blocks);
+    flash_item<G, false>(smem, blockIdx.x / Hkv, blockIdx.x % Hkv, out, q, kc, vc, block_tables, bt_stride, ptile_seq,
+                         ptile_q0, q_start, q_len, ctx_len, Hq, Hkv, scale_log2, num_blocks, 0, 1, nullptr);
   } else {
     const int kvh = blockIdx.x % Hkv, j = blockIdx.x / Hkv, S = gridDim.x / Hkv;
     for (int r = 0; r * S < num_ptiles; ++r) {
       const int t = r * S + ((r & 1) ? S - 1 - j : j);
       if (t >= num_ptiles) continue;  // a partial last round: every slot still leaves the loop
       if (r > 0) __syncthreads();      // the previous tile's last ring reads before this tile's DMAs
-      flash_item<G>(smem, t, kvh, out, q, kc, vc, block_tables, bt_stride, ptile_seq, ptile_q0, q_start, q_len,
-                      ctx_len, Hq, Hkv, scale_log2, num_blocks);
+      flash_item<G, false>(smem, t, kvh, out, q, kc, vc, block_tables, bt_stride, ptile_seq, ptile_q0, q_start, q_len,
+                           ctx_len, Hq, Hkv, scale_log2, num_blocks, 0, 1, nullptr);
     }
+  }
+}
+
+// A tile's keys in n_splits ranges, one workgroup each (flash_splits): blockIdx.x = (range * tiles + tile) * Hkv + kv head, parts of
+// kFlashPart floats in that order.
+template <int G>
+__global__ void __launch_bounds__(256, 2) flash_split_kernel(
+    const uint16_t* __restrict__ q, const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc,
+    const int* __restrict__ block_tables, int bt_stride, const int* __restrict__ ptile_seq, const int* __restrict__ ptile_q0,
+    const int* __restrict__ q_start, const int* __restrict__ q_len, const int* __restrict__ ctx_len, int Hq, int Hkv,
+    float scale_log2, int num_blocks, int num_ptiles, int n_splits, float* __restrict__ part) {
+  __shared__ __attribute__((aligned(256))) uint16_t smem[kFlashRing * 4 * kBS * kD];
+  const int i = blockIdx.x / Hkv;
+  flash_item<G, true>(smem, i % num_ptiles, blockIdx.x % Hkv, nullptr, q, kc, vc, block_tables, bt_stride, ptile_seq, ptile_q0,
+                      q_start, q_len, ctx_len, Hq, Hkv, scale_log2, num_blocks, i / num_ptiles, n_splits,
+                      part + (size_t)blockIdx.x * kFlashPart);
+}
+
+// out = sum of the ranges' O, each by 2^(its max - the largest), over their sums so weighted: 32 lanes a row, 32 rows a workgroup
+template <int G>
+__global__ void __launch_bounds__(256) flash_merge_kernel(
+    uint16_t* __restrict__ out, const float* __restrict__ part, const int* __restrict__ ptile_seq, const int* __restrict__ ptile_q0,
+    const int* __restrict__ q_start, const int* __restrict__ q_len, int Hq, int Hkv, float scale_log2, int num_ptiles, int n_splits) {
+  const int tile = blockIdx.x / Hkv, kvh = blockIdx.x % Hkv, s = ptile_seq[tile], q0 = ptile_q0[tile];
+  const int ql = q_len[s], qs = q_start[s], c = (threadIdx.x & 31) * 4;
+  const size_t step = (size_t)num_ptiles * Hkv * kFlashPart;
+  for (int R = blockIdx.y * 32 + (threadIdx.x >> 5); R < (int)blockIdx.y * 32 + 32; R += 8) {
+    const int qi = q0 + R / G;
+    if (qi >= ql) return;
+    const float* p = part + (size_t)blockIdx.x * kFlashPart;
+    float2 ml[kFlashSplits];
+    f32x4 o[kFlashSplits];
+    float M = kNegBig;
+#pragma unroll
+    for (int i = 0; i < kFlashSplits; ++i)
+      if (i < n_splits) {
+        ml[i] = *reinterpret_cast<const float2*>(p + i * step + 128 * 128 + 2 * R);
+        o[i] = *reinterpret_cast<const f32x4*>(p + i * step + R * 128 + c);  // (not written where the range had no pair)
+      }
+#pragma unroll
+    for (int i = 0; i < kFlashSplits; ++i)
+      if (i < n_splits && ml[i].y > 0.f) M = fmaxf(M, ml[i].x);
+    f32x4 y{0.f, 0.f, 0.f, 0.f};
+    float l = 0.f;
+#pragma unroll
+    for (int i = 0; i < kFlashSplits; ++i)
+      if (i < n_splits && ml[i].y > 0.f) {
+        const float f = fast_exp2((ml[i].x - M) * scale_log2);
+        l += f * ml[i].y;
+        y += f * o[i];
+      }
+    y *= l > 0.f ? 1.f / l : 0.f;
+    *reinterpret_cast<u32x2*>(out + ((size_t)(qs + qi) * Hq + kvh * G + R % G) * kD + c) = u32x2{pack2(y[0], y[1]), pack2(y[2], y[3])};
   }
 }
 
@@ -1693,6 +1764,29 @@ static bool flash_in_turn(int num_ptiles, int Hkv, long keys) {
   return mean <= std::min(512L, 200 + (w - 4 * kCus) / 5);
 }
 
+// Key ranges of each tile, for launches of few workgroups over many keys (a chat's next turn behind its cached ones: 150 tokens of 8
+// kv heads are 40 workgroups, each walking all keys, 0.57 us a pair of pages).  By estimated time in us, w workgroups of n pairs
+// each on average: whole 6.8 + .574 n; in s ranges up to 256 of them 10 + .557 n / s + .59 s + .005 w s + .15 w n / 256, up to 512, two on
+// a CU, 12.5 + .58 n / s + .38 s + .0094 w s + .228 w n / 256; the best, where it is 8 % faster.  240 launches of 1 - 32 kv heads
+// (1 and 3 sequences of 17 - 800 tokens behind 0 - 12000 cached ones): 0.80 of the time whole on average, 1.2 % off the best
+// number, at 5 % or more over whole in 2 (1.11).  us, whole -> now, 8 kv heads, groups of 4: 150 tokens behind 1024 / 4096 / 12000 26.1 ->
+// 18.6, 79.3 -> 31.1, 220 -> 54; 512 behind 2048 / 12000 50.8 -> 37.6, 227 -> 106.
+int flash_splits(int num_ptiles, int Hkv, long keys) {
+  if (num_ptiles <= 0 || keys <= 0 || g_flash_form || g_flash_persist) return 1;
+  const float w = (float)num_ptiles * (float)Hkv, n = (float)keys / (float)num_ptiles / 32.f;
+  float best = (6.8f + .574f * n) * .92f;
+  int splits = 1;
+  for (int s = 2; s <= kFlashSplits && w * s <= 2 * kCus && s <= n; ++s) {
+    const float f = (float)s;
+    const float us = w * f <= kCus ? 10.f + .557f * n / f + .59f * f + .005f * w * f + .15f * w * n / kCus
+                                   : 12.5f + .58f * n / f + .38f * f + .0094f * w * f + .228f * w * n / kCus;
+    if (us < best) best = us, splits = s;
+  }
+  return splits;
+}
+
+long flash_part_floats(int num_ptiles, int Hkv, int n_splits) { return (long)num_ptiles * Hkv * n_splits * kFlashPart; }
+
 static int device_cus() {
   static int cus[16] = {};
   int dev = 0;
@@ -1705,8 +1799,25 @@ static int device_cus() {
 void launch_flash_prefill(void* out, const void* q, const void* kc, const void* vc, const int* bt,
                           int bt_stride, const int* ptile_seq, const int* ptile_q0,
                           const int* q_start, const int* q_len, const int* ctx_len, int num_ptiles,
-                          int Hq, int Hkv, float scale_log2, int num_blocks, long keys, hipStream_t st) {
+                          int Hq, int Hkv, float scale_log2, int num_blocks, long keys, int n_splits, float* part, hipStream_t st) {
   if (num_ptiles == 0) return;
+  if (n_splits > 1) {
+    auto run = [&](auto g) {
+      constexpr int G = decltype(g)::value;
+      flash_split_kernel<G><<<num_ptiles * Hkv * n_splits, 256, 0, st>>>(
+          (const uint16_t*)q, (const uint16_t*)kc, (const uint16_t*)vc, bt, bt_stride, ptile_seq, ptile_q0, q_start, q_len, ctx_len, Hq,
+          Hkv, scale_log2, num_blocks, num_ptiles, n_splits, part);
+      flash_merge_kernel<G><<<dim3(num_ptiles * Hkv, 4), 256, 0, st>>>((uint16_t*)out, part, ptile_seq, ptile_q0, q_start, q_len, Hq, Hkv,
+                                                                      scale_log2, num_ptiles, n_splits);
+    };
+    switch (Hq / Hkv) {
+      case 1: return run(std::integral_constant<int, 1>{});
+      case 2: return run(std::integral_constant<int, 2>{});
+      case 4: return run(std::integral_constant<int, 4>{});
+      case 8: return run(std::integral_constant<int, 8>{});
+      default: return;
+    }
+  }
   const bool in_turn = g_flash_form ? g_flash_form == 2 : flash_in_turn(num_ptiles, Hkv, keys);
   const int slots = g_flash_persist >= 64 ? g_flash_persist / 64
                     : g_flash_persist > 0 ? std::max(1, g_flash_persist * device_cus() / Hkv) : 0;

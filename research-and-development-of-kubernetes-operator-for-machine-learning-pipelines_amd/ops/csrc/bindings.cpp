@@ -162,12 +162,15 @@ void flash_prefill(Tensor out, Tensor q, Tensor k_cache, Tensor v_cache, Tensor 
                   block_tables.size(0) >= q_len.numel(),
               "per-sequence arrays");
   c10::DeviceGuard g(q.device());
+  const int n_tiles = (int)ptile_seq.numel(), splits = mlop::flash_splits(n_tiles, Hkv, (long)keys);
+  Tensor part;
+  if (splits > 1) part = at::empty({mlop::flash_part_floats(n_tiles, Hkv, splits)}, q.options().dtype(at::kFloat));
   mlop::launch_flash_prefill(out.data_ptr(), q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
                              block_tables.data_ptr<int>(), (int)block_tables.stride(0),
                              ptile_seq.data_ptr<int>(), ptile_q0.data_ptr<int>(),
                              q_start.data_ptr<int>(), q_len.data_ptr<int>(), ctx_len.data_ptr<int>(),
                              (int)ptile_seq.numel(), Hq, Hkv, (float)(scale * 1.4426950408889634),
-                             (int)k_cache.size(0), (long)keys, cur_stream());
+                             (int)k_cache.size(0), (long)keys, splits, splits > 1 ? part.data_ptr<float>() : nullptr, cur_stream());
 }
 
 // Largest (tile, kv head) pair count that takes the in-launch split-KV combine: no cap (a cap of
@@ -966,6 +969,7 @@ TORCH_LIBRARY(mlop, m) {
   m.def("ep_destroy(int h) -> ()", &ep_destroy);
   m.def("gemm_workspace(int M, int N, int K, int epi) -> int", &gemm_workspace);
   m.def("gemm_plan(int M, int N, int K) -> int[]", &gemm_plan);
+  m.def("flash_splits(int tiles, int kv_heads, int keys) -> int", [](int64_t t, int64_t h, int64_t k) { return (int64_t)mlop::flash_splits((int)t, (int)h, (long)k); });
   m.def("gemm_grouped_height(int[] rows, int N, int K, int cus=256) -> int", &gemm_grouped_height);
   m.def("gemm_grouped_variant(int M, int N, int K, int groups, int rows, int a_n) -> int", &gemm_grouped_variant);
   m.def("gemm_big_variant(int set=-1) -> int", &gemm_big_variant);

@@ -45,7 +45,9 @@ int moe_mid_tok(int set);            // tokens per workgroup of the mid MoE disp
 void launch_flash_prefill(void* out, const void* q, const void* kc, const void* vc, const int* bt,
                           int bt_stride, const int* ptile_seq, const int* ptile_q0,
                           const int* q_start, const int* q_len, const int* ctx_len, int num_ptiles,
-                          int Hq, int Hkv, float scale_log2, int num_blocks, long keys, hipStream_t st);
+                          int Hq, int Hkv, float scale_log2, int num_blocks, long keys, int n_splits, float* part, hipStream_t st);
+int flash_splits(int num_ptiles, int Hkv, long keys);  // key ranges of each tile; with more than one, part has flash_part_floats
+long flash_part_floats(int num_ptiles, int Hkv, int n_splits);
 // QKV projection epilogue (EPI_ROPE): the GEMM's C tile is [q heads | k heads | v heads]
 // of head_dim 128; q/k are rotated (HF rotate-half, cos/sin table [max_pos, 128]) and
 // q goes to q_out [T, Hq, 128], k / v into the paged cache (k [NB, Hkv, BS, 128],

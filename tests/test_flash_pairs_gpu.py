@@ -92,3 +92,35 @@ def test_which_form(gpu, tiles, mean, turn):
         assert not torch.equal(out, again())
     finally:
         torch.ops.mlop.flash_form(0)
+
+
+@pytest.mark.parametrize("grow", [False, True])
+@pytest.mark.parametrize("Hq,Hkv", [(2, 2), (4, 2), (8, 2), (16, 2)])
+@pytest.mark.parametrize("pairs", [30, 60, 120, 1000])
+def test_key_ranges(gpu, Hq, Hkv, grow, pairs):
+    """A tile's keys in ranges, merged: of a pair and of many, tiles with fewer pairs than ranges beside long ones, ranges that
+    end in the tile's diagonal (rows whose keys all lie before the last ones), uneven ones."""
+    q = [37, 1, 50, 33, 5]
+    tiles = sum(-(-n // (128 * Hkv // Hq)) for n in q)
+    splits = torch.ops.mlop.flash_splits(tiles, Hkv, tiles * 32 * pairs)  # (5 - 16; the launch does with what it is told)
+    assert splits > 4
+    ctx = [37, 33, 32 * splits + 1, 1500, 32 * 41 + 5]
+    out, again = launch(gpu, q, ctx, Hq, Hkv, grow, keys=tiles * 32 * pairs)
+    assert torch.equal(out, again())
+    whole, _ = launch(gpu, q, ctx, Hq, Hkv, grow)
+    # both P in bf16 against another max (2^-9 of each addend) and rounded
+    torch.testing.assert_close(out.float(), whole.float(), atol=2.0 ** -7, rtol=2.0 ** -7)
+
+
+@pytest.mark.parametrize("q,cached,splits", [(417, 2000, 4), (417, 1000, 2), (800, 12000, 2), (150, 700, 4)])
+def test_key_ranges_of_chunks(gpu, q, cached, splits):
+    keys = sum(min(q, a + 32) + cached for a in range(0, q, 32))
+    assert torch.ops.mlop.flash_splits(-(-q // 32), 8, keys) == splits
+    launch(gpu, [q], [q + cached], 32, 8, False, keys=keys)
+
+
+def test_key_ranges_rule(gpu):
+    f = torch.ops.mlop.flash_splits
+    assert f(5, 8, 0) == f(5, 8, 5 * 150) == f(29, 8, 29 * 250) == f(128, 8, 128 * 11000) == 1  # unknown, short, many workgroups
+    assert f(5, 8, 5 * 4000) > 1 and f(16, 8, 16 * 12000) > 1
+    assert all(t * h * f(t, h, t * k) <= 512 or f(t, h, t * k) == 1 for t in (1, 3, 17, 40, 65) for h in (1, 2, 8, 32) for k in (100, 3000, 90000))
