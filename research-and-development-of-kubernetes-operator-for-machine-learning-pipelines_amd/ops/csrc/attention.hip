@@ -1766,20 +1766,20 @@ static bool flash_in_turn(int num_ptiles, int Hkv, long keys) {
 
 // Key ranges of each tile, for launches of few workgroups over many keys (a chat's next turn behind its cached ones: 150 tokens of 8
 // kv heads are 40 workgroups, each walking all keys, 0.57 us a pair of pages).  By estimated time in us, w workgroups of n pairs
-// each on average: whole 6.8 + .574 n; in s ranges up to 256 of them 10 + .557 n / s + .59 s + .005 w s + .15 w n / 256, up to 512, two on
-// a CU, 12.5 + .58 n / s + .38 s + .0094 w s + .228 w n / 256; the best, where it is 8 % faster.  240 launches of 1 - 32 kv heads
-// (1 and 3 sequences of 17 - 800 tokens behind 0 - 12000 cached ones): 0.80 of the time whole on average, 1.2 % off the best
-// number, at 5 % or more over whole in 2 (1.11).  us, whole -> now, 8 kv heads, groups of 4: 150 tokens behind 1024 / 4096 / 12000 26.1 ->
-// 18.6, 79.3 -> 31.1, 220 -> 54; 512 behind 2048 / 12000 50.8 -> 37.6, 227 -> 106.
+// each on average: whole 6.9 + .57 n; in s ranges up to 256 of them 10.3 + .5 n / s + .02 s + .0063 w s + .15 w n / 256, up to 512, two on
+// a CU, 11 + .57 n / s + .0103 w s + .215 w n / 256; the best, where it is 10 % faster.  240 launches of 1 - 32 kv heads
+// (1 and 3 sequences of 17 - 800 tokens behind 0 - 12000 cached ones): 0.75 of the time whole on average, 1.2 % off the best
+// number, slower than whole in 1 (1.04).  us, whole -> now, 8 kv heads, groups of 4: 150 tokens behind 1024 / 4096 / 12000 26.1 ->
+// 15.4, 79.3 -> 25.3, 220 -> 46.5; 512 behind 2048 / 12000 50.8 -> 35.6, 227 -> 105.2.
 int flash_splits(int num_ptiles, int Hkv, long keys) {
   if (num_ptiles <= 0 || keys <= 0 || g_flash_form || g_flash_persist) return 1;
   const float w = (float)num_ptiles * (float)Hkv, n = (float)keys / (float)num_ptiles / 32.f;
-  float best = (6.8f + .574f * n) * .92f;
+  float best = (6.9f + .57f * n) / 1.1f;
   int splits = 1;
   for (int s = 2; s <= kFlashSplits && w * s <= 2 * kCus && s <= n; ++s) {
     const float f = (float)s;
-    const float us = w * f <= kCus ? 10.f + .557f * n / f + .59f * f + .005f * w * f + .15f * w * n / kCus
-                                   : 12.5f + .58f * n / f + .38f * f + .0094f * w * f + .228f * w * n / kCus;
+    const float us = w * f <= kCus ? 10.3f + .5f * n / f + .02f * f + .0063f * w * f + .15f * w * n / kCus
+                                   : 11.f + .57f * n / f + .0103f * w * f + .215f * w * n / kCus;
     if (us < best) best = us, splits = s;
   }
   return splits;
