@@ -1964,8 +1964,6 @@ static void few_rows_w4(int M, int N, int K, int epi, Plan& p) {
   p.BM = rows, p.BN = 256, p.splits = 1, p.k_chunk = K, p.variant = rows == 256 ? 5 : 6, p.m_tiles = (M + rows - 1) / rows;
 }
 
-// fp32 slabs of the K ranges: of a plain product, and (add_norm) of one with the residual add + RMSNorm behind it, for which 0
-// also says that there is no such form; the weight-streaming kernel's has none, but A's rows may not suit it
 // GEMM + residual add + RMSNorm above 256 rows: the four-wave kernel over K in 2 - 8 ranges, one workgroup per (tile, range), its
 // fp32 slabs summed by the pass that adds and norms anyway.  A grid of few tiles fills the CUs with whole tiles so: what the
 // K-half hand-over and the stream-K tail send through one workgroup of a tile (a CU takes in 50 GB/s of what is not in its L2) is read by
@@ -2009,6 +2007,8 @@ static bool slab_plan(int M, int N, int K, int& bm, int& splits) {
   return big_plan(M, N, K, true, p, &us) && best * 1.03f + (K < 2600 ? 2.f : 0.f) < us + 3.f + mn * 8.f / 6.f;
 }
 
+// fp32 slabs of the K ranges: of a plain product, and (add_norm) of one with the residual add + RMSNorm behind it, for which 0
+// also says that there is no such form; the weight-streaming kernel's has none, but A's rows may not suit it
 long gemm_workspace_floats(int M, int N, int K, int epi, bool add_norm) {
   if (epi_act(epi)) epi = EPI_NONE;
   if (int bm, s; add_norm && slab_plan(M, N, K, bm, s)) return (long)s * M * N;
