@@ -1683,6 +1683,8 @@ __global__ void __launch_bounds__(256, 2) flash_split_kernel(
 
 // out = sum of the ranges' O, each by 2^(its max - the largest), over their sums so weighted: 32 lanes a row, 8 rows a workgroup
 // (32 one behind the other took four trips to memory: 240 parts of 6 ranges 10.5 us, now 5.0)
+// A range counts unless its sum is 0, and not only where it is above: NaN and infinite scores make the sum NaN, which O and so the
+// output then are, as without ranges.  (By its bits: this file's comparisons need not see a NaN.)
 template <int G>
 __global__ void __launch_bounds__(256) flash_merge_kernel(
     uint16_t* __restrict__ out, const float* __restrict__ part, const int* __restrict__ ptile_seq, const int* __restrict__ ptile_q0,
@@ -1705,12 +1707,12 @@ __global__ void __launch_bounds__(256) flash_merge_kernel(
     }
 #pragma unroll
   for (int i = 0; i < kFlashSplits; ++i)
-    if (i < n_splits && ml[i].y > 0.f) M = fmaxf(M, ml[i].x);
+    if (i < n_splits && __float_as_uint(ml[i].y) != 0) M = fmaxf(M, ml[i].x);
   f32x4 y{0.f, 0.f, 0.f, 0.f};
   float l = 0.f;
 #pragma unroll
   for (int i = 0; i < kFlashSplits; ++i)
-    if (i < n_splits && ml[i].y > 0.f) {
+    if (i < n_splits && __float_as_uint(ml[i].y) != 0) {
       const float f = fast_exp2((ml[i].x - M) * scale_log2);
       l += f * ml[i].y;
       y += f * o[i];

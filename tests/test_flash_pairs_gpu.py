@@ -11,8 +11,9 @@ pytestmark = pytest.mark.gpu
 bf = torch.bfloat16
 
 
-def launch(gpu, q_lens, ctx_lens, Hq, Hkv, grow, keys=0):
-    """Every sequence a prefill of q_lens tokens behind ctx_lens - q_lens cached ones, pages scattered."""
+def launch(gpu, q_lens, ctx_lens, Hq, Hkv, grow, keys=0, spoil=None):
+    """Every sequence a prefill of q_lens tokens behind ctx_lens - q_lens cached ones, pages scattered.  spoil(q, k_cache,
+    v_cache, block tables) puts values there that the reference is not compared with."""
     G, rng, S = Hq // Hkv, np.random.default_rng(len(q_lens) + Hq), len(q_lens)
     pages = [(c + 15) // 16 for c in ctx_lens]
     NB = sum(pages) + 3
@@ -43,6 +44,9 @@ def launch(gpu, q_lens, ctx_lens, Hq, Hkv, grow, keys=0):
             at = torch.arange(n, device=gpu).view(n, 1, 1, 1)
             kc[bt[i, :n]] = (kc[bt[i, :n]].float() * 1.25 ** (at % 24)).to(bf)
     m.pkeys = keys
+    if spoil is not None:
+        spoil(q, kc, vc, bt)
+        return ops.paged_attention(q, kc, vc, m)
     out = ops.paged_attention(q, kc, vc, m)
     exp = ref.paged_attention(q, kc, vc, m)
     # P in bf16 (2^-9 of each addend, which the row's sum does not share) and the result's rounding; |V| < 5
@@ -110,6 +114,39 @@ def test_key_ranges(gpu, Hq, Hkv, grow, pairs):
     whole, _ = launch(gpu, q, ctx, Hq, Hkv, grow)
     # both P in bf16 against another max (2^-9 of each addend) and rounded
     torch.testing.assert_close(out.float(), whole.float(), atol=2.0 ** -7, rtol=2.0 ** -7)
+
+
+def spoil_key(q, kc, vc, bt, at=777):
+    kc[bt[1, at // 16], :, at % 16, 5] = float("nan")
+
+
+def spoil_query(q, kc, vc, bt):
+    q[40, 1, 7] = float("nan")
+
+
+def spoil_score(q, kc, vc, bt, at=777):
+    """One key whose scores are +infinity for some rows and, as good as -infinity or masked by it, nothing for others."""
+    kc[bt[1, at // 16], :, at % 16] = 0
+    kc[bt[1, at // 16], :, at % 16, 5] = 3e38
+    q[..., 5] = torch.where(q[..., 5] >= 0, 2.0, -2.0).to(bf)
+
+
+def spoil_values(q, kc, vc, bt):
+    vc[bt[1, 3], :, 4, 100], vc[bt[1, 80], :, 2, 3] = float("nan"), float("inf")
+
+
+@pytest.mark.parametrize("Hq,Hkv", [(2, 2), (8, 2)])
+@pytest.mark.parametrize("spoil", [spoil_key, spoil_query, spoil_score, spoil_values, lambda *a: [spoil_key(*a, at=i) for i in range(0, 1500, 7)]],
+                         ids=["key", "query", "score", "values", "keys"])
+def test_key_ranges_of_what_is_not_finite(gpu, spoil, Hq, Hkv):
+    """A NaN or an infinity shows in the same outputs as without ranges: of a range that holds it no row is dropped."""
+    q, ctx = [37, 50, 5], [1500, 1500, 900]
+    tiles = sum(-(-n // (128 * Hkv // Hq)) for n in q)
+    keys = tiles * 32 * 60
+    assert torch.ops.mlop.flash_splits(tiles, Hkv, keys) > 4
+    got, whole = (launch(gpu, q, ctx, Hq, Hkv, False, keys=k, spoil=spoil).float() for k in (keys, 0))
+    assert not torch.isfinite(whole).all() and torch.isfinite(whole).any()
+    torch.testing.assert_close(got, whole, atol=2.0 ** -7, rtol=2.0 ** -7, equal_nan=True)
 
 
 @pytest.mark.parametrize("q,cached,splits", [(417, 2000, 4), (417, 1000, 2), (800, 4000, 2), (150, 700, 6), (150, 400, 5)])
