@@ -44,20 +44,27 @@ def test_tiles(gpu, height, tiles, off, N, K, epi):
     assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
 
 
+@pytest.mark.parametrize("variant,bm", [(6, 128), (6, 160), (6, 192), (6, 224), (5, 256)])
 @pytest.mark.parametrize("off", [1, 8, 9, 100])
 @pytest.mark.parametrize("epi", [0, 1])
-def test_rows_past_the_last(gpu, height, off, epi):
+def test_rows_past_the_last(gpu, variant, bm, off, epi):
     """Rows past A's last load nothing: what the LDS holds there (here a product of NaN before) reaches no output, and
-    the waits that count the dropped loads still cover the others (next tile's among them)."""
-    N, K, M = 20736, 448, 2 * height + off
+    the waits that count the dropped loads still cover the others, a workgroup's next tile's among them (513 tiles: two or three
+    each, a third of them partial, behind whole ones and before them)."""
+    N, K, M = 171 * 256, 448, 2 * bm + off
     torch.manual_seed(M)
     w = (0.05 * torch.randn(N, K, device=gpu)).to(bf)
-    nan = torch.full((4 * height, K), float("nan"), device=gpu, dtype=bf)
+    nan = torch.full((4 * bm, K), float("nan"), device=gpu, dtype=bf)
     x = torch.randn(M, K, device=gpu, dtype=bf)
-    whole = ops.gemm(torch.cat([x, x, x])[:3 * height], w, epi=epi)[:M]  # the same rows with no partial tile
-    for _ in range(4):
-        ops.gemm(nan, w)
-        assert torch.equal(ops.gemm(x, w, epi=epi), whole)
+    ops._sk_reserve(torch.device(gpu))
+    torch.ops.mlop.gemm_dense_plan(variant, bm, 256, -1)
+    try:
+        whole = ops.gemm(torch.cat([x, x, x])[:3 * bm], w, epi=epi)[:M]  # the same rows with no partial tile
+        for _ in range(4):
+            ops.gemm(nan, w)
+            assert torch.equal(ops.gemm(x, w, epi=epi), whole)
+    finally:
+        torch.ops.mlop.gemm_dense_plan(-1, -1, -1, -1)
 
 
 # K a multiple of 2048 and not, halves of it, several bands of tiles; weights that the cache behind the L2s holds and not

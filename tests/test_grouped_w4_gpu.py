@@ -96,3 +96,32 @@ def test_grouped(gpu, counts, K, kind):
             sg, su = ops.deinterleave_cols(sums).chunk(2, -1)
             bound = 4 * 2.0 ** -8 * g.abs() * (u.abs() + (lim is not None)) + 1.1 * sg * u.abs() + su * g.abs()
         assert ((got[0][a:b].float() - exp).abs() <= bound + 1e-5).all(), e
+
+
+@pytest.mark.parametrize("height,counts", [(160, [150, 159, 160, 145, 152, 140, 151, 129]), (192, [190, 161, 192, 185, 177, 129, 191, 170]),
+                                           (224, [430, 448, 440, 225, 400, 448, 410, 390]), (256, [257, 10, 300, 255, 250, 256, 240, 256])])
+@pytest.mark.parametrize("gather", [False, True])
+@pytest.mark.parametrize("epi", [0, 1])
+def test_rows_past_an_experts_last(gpu, height, counts, gather, epi):
+    """They load nothing: what the LDS holds there (a product of NaN before) reaches no output, and the waits that count the
+    dropped loads cover the others, the next tile's among them (three tiles a workgroup and more): bit for bit what the same rows give
+    in as many tiles without a partial one."""
+    K, cus = 448, torch.cuda.get_device_properties(gpu).multi_processor_count
+    full = [-(-c // height) * height for c in counts]
+    assert all(torch.ops.mlop.gemm_grouped_height(c, N, K, cus) == height for c in (counts, full))
+    torch.manual_seed(height)
+    w = 0.05 * torch.randn(G, N, K, device=gpu, dtype=bf)
+    ends = lambda c: torch.tensor([0] + c, device=gpu).cumsum(0).int()  # noqa: E731
+    off, off_full = ends(counts), ends(full)
+    toks = torch.randn(int(off[-1]), K, device=gpu, dtype=bf)
+    rows = torch.randperm(toks.shape[0], device=gpu).int() if gather else None
+    x = toks[rows.long()] if gather else toks
+    at = torch.cat([torch.arange(c, device=gpu) + int(off_full[e]) for e, c in enumerate(counts)])
+    padded = torch.randn(sum(full), K, device=gpu, dtype=bf)
+    padded[at] = x
+    ops._sk_reserve(torch.device(gpu))
+    want = ops.grouped_gemm(padded, w, off_full, epi=epi, avg_rows=64)[at]
+    nan, nan_off = torch.full((G * 448, K), float("nan"), device=gpu, dtype=bf), ends([448] * G)
+    for _ in range(4):
+        ops.grouped_gemm(nan, w, nan_off, epi=epi, avg_rows=64)
+        assert torch.equal(ops.grouped_gemm(toks, w, off, epi=epi, avg_rows=64, a_rows=rows), want)
