@@ -300,9 +300,9 @@ int64_t gemm_workspace(int64_t M, int64_t N, int64_t K, int64_t epi) {
   return mlop::gemm_workspace_floats((int)M, (int)N, (int)K, (int)epi);
 }
 
-std::vector<int64_t> gemm_plan(int64_t M, int64_t N, int64_t K) {
+std::vector<int64_t> gemm_plan(int64_t M, int64_t N, int64_t K, int64_t epi) {
   int p[5];
-  mlop::gemm_plan((int)M, (int)N, (int)K, p);
+  mlop::gemm_plan((int)M, (int)N, (int)K, (int)epi, p);
   return {p[0], p[1], p[2], p[3], p[4]};
 }
 
@@ -968,7 +968,7 @@ TORCH_LIBRARY(mlop, m) {
   m.def("ep_mem_mode(int h) -> int", &ep_mem_mode);
   m.def("ep_destroy(int h) -> ()", &ep_destroy);
   m.def("gemm_workspace(int M, int N, int K, int epi) -> int", &gemm_workspace);
-  m.def("gemm_plan(int M, int N, int K) -> int[]", &gemm_plan);
+  m.def("gemm_plan(int M, int N, int K, int epi=0) -> int[]", &gemm_plan);
   m.def("flash_splits(int tiles, int kv_heads, int keys) -> int", [](int64_t t, int64_t h, int64_t k) { return (int64_t)mlop::flash_splits((int)t, (int)h, (long)k); });
   m.def("gemm_grouped_height(int[] rows, int N, int K, int cus=256) -> int", &gemm_grouped_height);
   m.def("gemm_grouped_variant(int M, int N, int K, int groups, int rows, int a_n) -> int", &gemm_grouped_variant);

@@ -1901,17 +1901,18 @@ void launch_mid_self(const void* A, int lda, const void* B, void* out, int ldo, 
 
 static void few_rows_w4(int M, int N, int K, int epi, Plan& p);
 
-void gemm_plan(int M, int N, int K, int out[5]) {
-  if (gemm_on_ws(M, N, K, EPI_NONE)) {
+void gemm_plan(int M, int N, int K, int epi, int out[5]) {
+  if (epi_act(epi)) epi = EPI_NONE;
+  if (gemm_on_ws(M, N, K, epi)) {
     out[0] = -2, out[1] = out[2] = 0, out[3] = 1, out[4] = gemm_weights_nt(1);
     return;
   }
-  if (gemv_takes(M, N, K, EPI_NONE)) {
+  if (gemv_takes(M, N, K, epi)) {
     out[0] = -1, out[1] = out[2] = out[4] = 0, out[3] = 1;
     return;
   }
   Plan p = plan(M, N, K, false, 0, 0);
-  few_rows_w4(M, N, K, EPI_NONE, p);
+  few_rows_w4(M, N, K, epi, p);
   out[0] = p.variant, out[1] = p.BM, out[2] = p.BN, out[3] = p.splits;
   out[4] = (p.variant == 0 || p.variant == 7) && gemm_weights_nt((M + p.BM - 1) / p.BM);
 }
@@ -1919,23 +1920,24 @@ void gemm_plan(int M, int N, int K, int out[5]) {
 // Products of 129 - 256 rows in one K range, gate_up and output heads (the plain ones of more than 32768 columns): the four-wave
 // kernel where it is estimated to be 5 % faster than the weight stream, or than the 256 x 128 tiles that have 130 - 168 tiles of 128
 // columns.  The weight stream's workgroup takes in the whole batch beside its 128 or 256 columns, and a grid of 1.1 rounds takes
-// two; the four-wave kernel has 128-row tiles, two for a column, or one of the batch's height.  us, before -> now: gate_up 28672 x 4096
+// two; the four-wave kernel has 128-row tiles, two for a column, or one of the batch's height.  Not where it would cut the last tiles into K-halves (0.82 - 0.87 of the time
+// at 18432 - 20480 and 65536 - 69888 columns): up to 256 rows no product uses the scratch of the hand-over, so one may run beside another
+// stream's that does (captured decode steps of Dibedra: a layer's experts beside its dense products).  us, before -> now: gate_up 28672 x 4096
 // at 200 / 240 / 256 rows 67 -> 62, 73 -> 65, 75 -> 65, 36864 x 4096 at 200 117 -> 84, 20480 x 4096 at 160 63 -> 48; head 128256 x 4096 at
 // 180 / 210 / 256 217 -> 202, 236 -> 216, 267 -> 236; 57344 x 8192 at 240 244 -> 225.
 // Steps of six Llama-3-8B layers: 240 sequences 1699 -> 1618, a prompt of 250 tokens 1323 -> 1271; three of the 70B, 250 sequences 2225 -> 2137.
 // Estimates in us fitted to 720 points (15 widths of 8192 - 128256, K 2048 - 8192, 135 - 256 rows, cold weights), 5 and 6 % off in the mean.
 // Weight stream of bm rows, g the share of the CUs in a round: 10.1 + a K-step's .117 + .00189 bm + .00121 bm g + .081 g with 128
 // columns, 11.6 + -.261 + .00447 bm + .00168 bm g + .588 g with 256.  Four-wave: rounds of .0227 K (.0262 where K is not whole 2048 and the
-// tiles walk it in step) times the height's share, halves of a tail, and the weights at 5 TB/s (4.5 out of whole 2048; the sixth powers' sum).  The choice: 0.92 of the time before
-// over those points, 1.2 % off the best, 6 - 10 % over before at 5 (57344 x 4096 at 197 - 256 rows).
+// tiles walk it in step) times the height's share, and the weights at 5 TB/s (4.5 out of whole 2048; the sixth powers' sum).  The choice: 0.92 of the time before
+// over those points, 1 % off the best without halves, 6 - 10 % over before at 5 (57344 x 4096 at 197 - 256 rows).
 static void few_rows_w4(int M, int N, int K, int epi, Plan& p) {
-  const SkBuf* b = sk_buf();
-  if (M <= 128 || M > 256 || K < 1024 || !b || g_dp[0] >= 0 || p.splits > 1 || (epi != EPI_SILU_MUL && N <= 32768) || !gemm_w4_ok(M, N, K, K, K)) return;
+  if (M <= 128 || M > 256 || K < 1024 || g_dp[0] >= 0 || p.splits > 1 || (epi != EPI_SILU_MUL && N <= 32768) || !gemm_w4_ok(M, N, K, K, K)) return;
   const int nk = K / kBK;
-  const float C = (float)b->cus, k = (float)K, bm = (float)((M + 31) / 32 * 32);
+  const float C = (float)kCus, k = (float)K, bm = (float)((M + 31) / 32 * 32);
   float now;
   if (p.variant == 7) {
-    const int t = (N + p.BN - 1) / p.BN, rounds = (t + b->cus - 1) / b->cus;
+    const int t = (N + p.BN - 1) / p.BN, rounds = (t + kCus - 1) / kCus;
     const float g = std::min((float)t / C, 1.f);
     const float step = p.BN == 128 ? .117f + .00189f * bm + .00121f * bm * g + .081f * g : -.261f + .00447f * bm + .00168f * bm * g + .588f * g;
     now = (p.BN == 128 ? 10.1f : 11.6f) + (float)(nk * rounds) * step;
@@ -1949,13 +1951,12 @@ static void few_rows_w4(int M, int N, int K, int epi, Plan& p) {
   for (const W4Tile& t : kW4Tiles) {
     if (t.rows < 256 && !g_half_tile) break;
     if (t.rows != 128 && (t.rows < M || t.rows >= M + 32)) continue;
-    const int T = (M + t.rows - 1) / t.rows * (N / 256), q = T / b->cus, r = T % b->cus;
-    const bool halves = gemm_w4_split_ok(T, nk);
+    const int T = (M + t.rows - 1) / t.rows * (N / 256), q = T / kCus, r = T % kCus;
+    if ((r > 0 && 2 * r <= kCus && nk % 2 == 0) || gemm_w4_split_ok(T, nk)) continue;
     const float one = (K % 2048 ? .0262f : .0227f) * k * t.round;
     float us = 2.5f + (float)q * one;
-    if (halves) us += .5f * one + 12.2f - .0018f * k;
-    else if (r > 0) us += one * (1.f - .16f * (1.f - (float)r / C));
-    const float weights = 5.5f + (float)N * k * 2e-6f / ((halves && q == 0 ? 3.8f : 5.f) * (K % 2048 ? .9f : 1.f));
+    if (r > 0) us += one * (1.f - .16f * (1.f - (float)r / C));
+    const float weights = 5.5f + (float)N * k * 2e-6f / (K % 2048 ? 4.5f : 5.f);
     us = std::pow(std::pow(us, 6.f) + std::pow(weights, 6.f), 1.f / 6.f);
     if (us < best) best = us, rows = t.rows;
   }

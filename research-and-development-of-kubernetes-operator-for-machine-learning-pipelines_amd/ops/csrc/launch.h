@@ -135,9 +135,9 @@ constexpr int epi_act(int epi) {
 // split-K reduce fused in: small-M launch_gemm_rope)
 void launch_rope_cache_slabs(const RopeEpi& re, const float* ws, int splits, int T, int N, hipStream_t st);
 long gemm_workspace_floats(int M, int N, int K, int epi, bool add_norm = false);
-// what a plain product of this shape takes: kernel variant (gemm.hip plan; -1 the GEMV, -2 the weight-streaming kernel of
+// what a product of this shape and epilogue takes: kernel variant (gemm.hip plan; -1 the GEMV, -2 the weight-streaming kernel of
 // gemm_ws.hip), tile rows, columns, K ranges, weights loaded non-temporal (weight-streaming tiles)
-void gemm_plan(int M, int N, int K, int out[5]);
+void gemm_plan(int M, int N, int K, int epi, int out[5]);
 bool gemm_weights_nt(int m_tiles);
 // the experts' product of M routed rows, max_rows of them per expert on average, from a_n rows: gemm.hip grouped_plan
 int gemm_grouped_variant(int M, int N, int K, int n_groups, int max_rows, int a_n);

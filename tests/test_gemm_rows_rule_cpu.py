@@ -62,3 +62,22 @@ def test_rows_of_the_weight_stream(N, bm):
     for M in (17, 32):
         assert torch.ops.mlop.gemm_plan(M, N, 4096)[:2] == [7, bm]
     assert torch.ops.mlop.gemm_plan(33, N, 4096)[:2] == [7, 64]
+
+
+def test_few_rows_use_no_scratch():
+    """Up to 256 rows a product may run beside another stream's that uses the four-wave and grouped kernels' scratch for partial tiles
+    (captured decode steps of Dibedra: experts beside the dense products), so none of its tiles is cut into K-halves."""
+    four_wave = 0
+    for M in (129, 150, 160, 161, 192, 193, 224, 225, 256):
+        for N in range(16384, 163841, 256):
+            for K in (1024, 1088, 2048, 4096, 8192):
+                if N * K >= 1 << 30:
+                    continue
+                for epi in (0, 1):
+                    variant, bm = torch.ops.mlop.gemm_plan(M, N, K, epi)[:2]
+                    if variant not in (5, 6):
+                        continue
+                    four_wave += 1
+                    tail = -(-M // bm) * (N // 256) % 256
+                    assert tail == 0 or 2 * tail > 256 or K // 64 % 2, (M, N, K, epi)
+    assert four_wave > 0
