@@ -811,6 +811,11 @@ static int w4_k_walk(int N, int K, int band_tiles, int cus) {
   return K % 2048 == 0 && ((long)N * K * 2 <= (256l << 20) || band_tiles >= cus) ? 5 : 0;
 }
 
+// whether a product's tiles walk K in step: rounds of few_rows_w4's estimate
+bool gemm_w4_in_step(int M, int N, int K, int bm) {
+  return w4_k_walk(N, K, std::max(1, std::min(1024 / bm, (M + bm - 1) / bm)) * ((N + 255) / 256), kCus) == 0;
+}
+
 template <int EPI, int BMT>
 static bool run_w4_t(const uint16_t* A, int lda, const uint16_t* B, int ldb, uint16_t* C, int ldc, int M, int N,
                      int K, hipStream_t st, const RopeEpi& re) {

@@ -155,6 +155,7 @@ void gemm_dense_plan(int variant, int bm, int bn, int splits, int stages = 0);
 bool gemm_w4_ok(int M, int N, int K, int lda, int ldb, int ldc = 0);
 // the four-wave kernel cuts its r = T % CUs tail tiles into K-halves (2r <= CUs, nk even)
 bool gemm_w4_split_ok(int T, int nk);
+bool gemm_w4_in_step(int M, int N, int K, int bm);
 bool gemm_sk_scratch(float** ws, int** cnt, int* cus);
 bool gemm_sk_available(int* cus);
 bool run_w4(int epi, const uint16_t* A, int lda, const uint16_t* B, int ldb, uint16_t* C, int ldc, int M, int N,

@@ -1,5 +1,6 @@
 """gate_up and output heads of 129 - 256 rows on the four-wave kernel (few_rows_w4) against fp32, at the edges of its tiles and of
-its rule: one tile of the batch's height, two of 128 rows, K in halves, K that is not whole 2048, the 256 x 128 tiles' sizes."""
+its rule: one tile of the batch's height, two of 128 rows, K that is not whole 2048, the 256 x 128 tiles' sizes, the rows at which
+products of the weight stream go over."""
 import pytest
 import torch
 
@@ -26,17 +27,31 @@ def run(gpu, M, N, K, epi):
     assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
 
 
-@pytest.mark.parametrize("M", [129, 160, 161, 193, 225, 255, 256])
-@pytest.mark.parametrize("N,K", [(20480, 1024), (36864, 2048), (40960, 1088), (28672, 4096)])
+def height(M):
+    """One tile of the batch's height."""
+    bm = -(-M // 32) * 32
+    return (5 if bm == 256 else 6, bm)
+
+
+# the kernel that each is to run on: variant and rows, of the weight stream (7) or of four-wave tiles
+GATE_UP = {(20480, 1024): lambda M: (6, 128), (36864, 2048): height, (40960, 1088): height,
+           (28672, 4096): lambda M: (6, 128) if M > 224 else (7, -(-M // 32) * 32)}
+HEAD = {(36864, 2048): height, (40960, 1088): height, (128256, 1024): lambda M: height(M) if M > 192 else (7, -(-M // 32) * 32)}
+
+
+@pytest.mark.parametrize("M", [129, 160, 161, 193, 224, 225, 255, 256])
+@pytest.mark.parametrize("N,K", GATE_UP)
 def test_gate_up(gpu, M, N, K):
     ops._sk_reserve(torch.device(gpu))
+    assert tuple(torch.ops.mlop.gemm_plan(M, N, K, 1)[:2]) == GATE_UP[N, K](M)
     run(gpu, M, N, K, 1)
 
 
-@pytest.mark.parametrize("M", [129, 191, 193, 224, 256])
-@pytest.mark.parametrize("N,K", [(36864, 2048), (40960, 1088), (128256, 1024)])
+@pytest.mark.parametrize("M", [129, 191, 192, 193, 224, 256])
+@pytest.mark.parametrize("N,K", HEAD)
 def test_head(gpu, M, N, K):
     ops._sk_reserve(torch.device(gpu))
+    assert tuple(torch.ops.mlop.gemm_plan(M, N, K)[:2]) == HEAD[N, K](M)
     run(gpu, M, N, K, 0)
 
 
