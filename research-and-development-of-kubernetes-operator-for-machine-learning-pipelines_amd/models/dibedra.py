@@ -172,13 +172,15 @@ class DibedraModel:
     # ------------------------------------------------------------ forward --
     def forward(self, ids: torch.Tensor, meta, kv) -> torch.Tensor:
         """ids [T] int64; meta: AttnMeta; kv: KVCache with this model's layout.
-        Returns the final-normed hidden states of every token times the logits' scale, [T, padded width]."""
+        Returns the final-normed hidden states of every token times the logits' scale, [T, padded width], in ``meta.out`` where
+        given."""
         norms = [L["norm"] for L in self.layers] + [self.final_norm]
         alpha, w, b = norms[0]
         res, x = ops.residual_begin(ids, self.embed, 1.0, None, meta.positions, w, 0.0, tanh=(alpha, b))
         for i in range(len(self.layers)):
             alpha, w, b = norms[i + 1]
-            x = ops.residual_step(res, post_w=None, norm_w=w, eps=0.0, store=i + 1 < len(self.layers), tanh=(alpha, b),
+            last = i + 1 == len(self.layers)
+            x = ops.residual_step(res, post_w=None, norm_w=w, eps=0.0, store=not last, tanh=(alpha, b), out=meta.out if last else None,
                                   **self._layer(i, x, meta, kv))
         return x
 

@@ -142,7 +142,7 @@ class KosesunModel:
     # ------------------------------------------------------------ forward --
     def forward(self, ids: torch.Tensor, meta, kv) -> torch.Tensor:
         """ids [T] int64; meta: AttnMeta; kv: KVCache with this model's layout and states.
-        Returns the final-normed hidden states of every token [T, W]."""
+        Returns the final-normed hidden states of every token [T, W], in ``meta.out`` where given."""
         eps, ctx = self.cfg.rms_eps, {}
         _, _, hc, norm = self.subs[0]
         streams, x = ops.hyper_begin(ids, self.embed, self.cfg.embed_scale, self.cfg.streams, hc["in"], norm, eps)
@@ -150,7 +150,7 @@ class KosesunModel:
             last = n + 1 == len(self.subs)
             nxt_in, nxt_norm = (self.ones, self.final_norm) if last else (self.subs[n + 1][2]["in"], self.subs[n + 1][3])
             x = ops.hyper_step(streams, run(i, x, meta, kv, ctx), hc["mix"], hc["out"], nxt_in, nxt_norm, eps,
-                               store=not last)
+                               store=not last, out=meta.out if last else None)
         return x
 
     def logits_local(self, hidden: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:

@@ -127,17 +127,17 @@ class LlamaModel:
         act = ops.gemm(x, L["gate_up"], epi=ops.EPI_SILU_MUL)  # K1/K2 + fused K8
         return linear(act, L["down"])
 
-    def mlp_add_norm(self, i, x, residual, next_norm, eps):
+    def mlp_add_norm(self, i, x, residual, next_norm, eps, out=None):
         """TP=1: MLP whose down projection also does residual += and the next norm."""
         L = self.layers[i]
         act = ops.gemm(x, L["gate_up"], epi=ops.EPI_SILU_MUL)
-        return ops.gemm_add_rmsnorm(act, L["down"], residual, next_norm, eps)
+        return ops.gemm_add_rmsnorm(act, L["down"], residual, next_norm, eps, out)
 
-    def attn_out_mlp(self, i, a, residual, next_norm, eps):
+    def attn_out_mlp(self, i, a, residual, next_norm, eps, out=None):
         """TP=1: O projection with the residual add + post-attention norm in its reduce
         pass, then the MLP block with the next add + norm in the down projection's."""
         x = ops.gemm_add_rmsnorm(a, self.layers[i]["o"], residual, self.layers[i]["post_norm"], eps)
-        return self.mlp_add_norm(i, x, residual, next_norm, eps)
+        return self.mlp_add_norm(i, x, residual, next_norm, eps, out)
 
     # ------------------------------------------------------------ forward --
     def weight_tensors(self):
@@ -153,7 +153,7 @@ class LlamaModel:
 
     def forward(self, ids: torch.Tensor, meta, kv) -> torch.Tensor:
         """ids [T] int64; meta: AttnMeta (positions/slots/tables); kv: KVCache.
-        Returns the final-normed hidden states of every token [T, H]."""
+        Returns the final-normed hidden states of every token [T, H], in ``meta.out`` where given."""
         cfg, tp = self.cfg, self.ps.tp
         eps = cfg.rms_eps
         h = ops.embedding(ids, self.embed, self.vocab_start)
@@ -178,27 +178,29 @@ class LlamaModel:
                 q = ops.qkv_rope_cache_rs(residual, L["qkv"], meta.positions, self.cos_sin, meta.slots, kv.k[i],
                                           kv.v[i], self.n_q, ss, eps, any_tile)
             a = ops.paged_attention(q, kv.k[i], kv.v[i], meta)
-            nxt = self.layers[i + 1]["in_norm"] if i + 1 < len(self.layers) else self.final_norm
+            last = i + 1 == len(self.layers)
+            nxt, out = (self.final_norm, meta.out) if last else (self.layers[i + 1]["in_norm"], None)
             if chain and tp.size > 1:
-                x, ss = self._chain_layer_tp(i, a.view(a.shape[0], -1), residual, i + 1 == len(self.layers), eps, ss)
+                x, ss = self._chain_layer_tp(i, a.view(a.shape[0], -1), residual, last, eps, ss, out)
                 continue
             if chain:
-                x, ss = self._chain_layer(i, a.view(a.shape[0], -1), residual, i + 1 == len(self.layers), eps, any_tile)
+                x, ss = self._chain_layer(i, a.view(a.shape[0], -1), residual, last, eps, any_tile, out)
                 continue
             if tp.size == 1:
-                x = self.attn_out_mlp(i, a.view(a.shape[0], -1), residual, nxt, eps)
+                x = self.attn_out_mlp(i, a.view(a.shape[0], -1), residual, nxt, eps, out)
                 continue
             # row-parallel O / down: the all-reduce + add + RMSNorm of row chunk i run on the
             # communication stream under the GEMM of chunk i+1 (parallel/overlap.py)
             x = row_parallel_add_norm(a.view(a.shape[0], -1), L["o"], tp, residual, L["post_norm"], eps)
-            x = self.mlp_row_parallel(i, x, residual, nxt, eps)
+            x = self.mlp_row_parallel(i, x, residual, nxt, eps, out)
         return x
 
-    def mlp_row_parallel(self, i, x, residual, next_norm, eps):
+    def mlp_row_parallel(self, i, x, residual, next_norm, eps, out=None):
         """TP > 1: gate_up (column-parallel, SiLU-mul fused), then the row-parallel down
         projection with its all-reduce overlapped, + the next residual add / norm."""
         act = ops.gemm(x, self.layers[i]["gate_up"], epi=ops.EPI_SILU_MUL)
-        return row_parallel_add_norm(act, self.layers[i]["down"], self.ps.tp, residual, next_norm, eps)
+        where = {} if out is None else {"out": out}
+        return row_parallel_add_norm(act, self.layers[i]["down"], self.ps.tp, residual, next_norm, eps, **where)
 
     # --------------------------------------------------------- norm chain --
     def _chain_ok(self, M: int, like: int = 0) -> bool:
@@ -212,7 +214,7 @@ class LlamaModel:
                                         (2 * self.inter, H), (H, self.inter)), device=self.device,
                                  epis=(ops.EPI_ROPE, ops.EPI_NONE, ops.EPI_SILU_MUL, ops.EPI_NONE), like=like)
 
-    def _chain_layer(self, i, a, residual, last, eps, any_tile=False):
+    def _chain_layer(self, i, a, residual, last, eps, any_tile=False, out=None):
         """O (+= residual, row partials), gate_up + SiLU on the row-scaled residual, down (+=
         residual, row partials; the last layer's down does the final add + RMSNorm instead).
         Returns (x, ss): x normalised hidden states (last layer) or None with the partials."""
@@ -222,12 +224,12 @@ class LlamaModel:
         ops.gemm_res_ss(a, L["o"], residual, ss_post, any_tile)
         act = ops.gemm_rs(residual, L["gate_up"], ss_post, eps, ops.EPI_SILU_MUL, any_tile)
         if last:
-            return ops.gemm_add_rmsnorm(act, L["down"], residual, self.final_norm, eps), None
+            return ops.gemm_add_rmsnorm(act, L["down"], residual, self.final_norm, eps, out), None
         ss = ops.ss_buffer(M, H, residual.device)
         ops.gemm_res_ss(act, L["down"], residual, ss, any_tile)
         return None, ss
 
-    def _chain_layer_tp(self, i, a, residual, last, eps, ss):
+    def _chain_layer_tp(self, i, a, residual, last, eps, ss, out=None):
         """Tensor-parallel decode chain (M <= GEMV_CHAIN_MAX_M): the row-parallel O / down partial sums are
         all-reduced AND added into the replicated residual in one launch (Group.all_reduce_add,
         K15), gate_up and the next QKV take their rows' RMSNorm factors from the residual chunks
@@ -240,7 +242,7 @@ class LlamaModel:
         d = ops.gemm(act, L["down"])
         tp.all_reduce_add(d, residual)
         if last:
-            return ops.rmsnorm(residual, self.final_norm, eps), None
+            return ops.rmsnorm(residual, self.final_norm, eps, out), None
         return None, ops.ss_init(residual, ss)
 
     def logits_local(self, hidden: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:

@@ -57,14 +57,14 @@ class MixtralModel(LlamaModel):
                            self.expert_start, self.n_local_experts, mode=mode,
                            cap_tokens=max(cap or 0, x.shape[0]))
 
-    def mlp_row_parallel(self, i, x, residual, next_norm, eps):
+    def mlp_row_parallel(self, i, x, residual, next_norm, eps, out=None):
         """TP > 1 (experts sharded over the TP ranks): each rank's partial MoE output, summed by
         the TP all-reduce, then the next residual add / norm."""
         m = self.mlp(i, x)
         self.ps.tp.all_reduce(m)
-        return ops.add_rmsnorm(m, residual, next_norm, eps)
+        return ops.add_rmsnorm(m, residual, next_norm, eps, out)
 
-    def mlp_add_norm(self, i, x, residual, next_norm, eps):
+    def mlp_add_norm(self, i, x, residual, next_norm, eps, out=None):
         """TP = EP = 1: MoE block + the next residual add / norm (decode-size dispatch in one
         launch, combine fused into the norm: parallel.moe.moe_forward_add_norm)."""
         if self.ps.ep.size == 1:
@@ -72,10 +72,10 @@ class MixtralModel(LlamaModel):
 
             L = self.layers[i]
             return moe_forward_add_norm(x, L["router"], L["w13"], L["w2"], self.cfg.top_k, self.expert_start,
-                                        self.n_local_experts, residual, next_norm, eps)
-        return ops.add_rmsnorm(self.mlp(i, x), residual, next_norm, eps)
+                                        self.n_local_experts, residual, next_norm, eps, out=out)
+        return ops.add_rmsnorm(self.mlp(i, x), residual, next_norm, eps, out)
 
-    def attn_out_mlp(self, i, a, residual, next_norm, eps):
+    def attn_out_mlp(self, i, a, residual, next_norm, eps, out=None):
         """TP = EP = 1 decode sizes: O projection GEMV, then ONE launch for residual add +
         post-attention RMSNorm + router + route + sort + gather (moe_dispatch_small's
         prologue), the two grouped GEMMs, and the combine fused into the next add + norm."""
@@ -85,6 +85,7 @@ class MixtralModel(LlamaModel):
             L = self.layers[i]
             o = linear(a, L["o"])
             return moe_forward_add_norm(None, L["router"], L["w13"], L["w2"], self.cfg.top_k, self.expert_start,
-                                        self.n_local_experts, residual, next_norm, eps, pre=(o, L["post_norm"]))
-        return super().attn_out_mlp(i, a, residual, next_norm, eps)
+                                        self.n_local_experts, residual, next_norm, eps, pre=(o, L["post_norm"]),
+                                        out=out)
+        return super().attn_out_mlp(i, a, residual, next_norm, eps, out)
 

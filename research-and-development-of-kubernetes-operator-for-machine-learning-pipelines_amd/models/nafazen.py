@@ -182,13 +182,13 @@ class NafazenModel:
     # ------------------------------------------------------------ forward --
     def forward(self, ids: torch.Tensor, meta, kv) -> torch.Tensor:
         """ids [T] int64; meta: AttnMeta; kv: KVCache with this model's layout.
-        Returns the final-normed hidden states of every token, [T, padded width]."""
+        Returns the final-normed hidden states of every token, [T, padded width], in ``meta.out`` where given."""
         cfg, eps, W = self.cfg, self.cfg.rms_eps, self.cfg.hidden_size
         res, x = ops.residual_begin(ids, self.embed, cfg.embed_scale, None, meta.positions, None, eps, width=W)
         for n, (run, i, norm) in enumerate(self.subs):
             last = n + 1 == len(self.subs)
             x = ops.residual_step(res, post_w=norm, norm_w=self.final_norm if last else None, eps=eps, store=not last, width=W,
-                                  **run(i, x, meta, kv))
+                                  out=meta.out if last else None, **run(i, x, meta, kv))
         return x
 
     def logits_local(self, hidden: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:

@@ -163,13 +163,13 @@ class RegesunModel:
     # ------------------------------------------------------------ forward --
     def forward(self, ids: torch.Tensor, meta, kv) -> torch.Tensor:
         """ids [T] int64; meta: AttnMeta; kv: KVCache with this model's layout and states.
-        Returns the final-normed hidden states of every token [T, W]."""
+        Returns the final-normed hidden states of every token [T, W], in ``meta.out`` where given."""
         eps, subs = self.cfg.rms_eps, self.subs
         res, x = ops.residual_begin(ids, self.embed, 1.0, self.pos, meta.positions, subs[0][2], eps)
         for n, (run, i, _, post) in enumerate(subs):
             last = n + 1 == len(subs)
             x = ops.residual_step(res, run(i, x, meta, kv), post, self.final_norm if last else subs[n + 1][2], eps,
-                                  store=not last)
+                                  store=not last, out=meta.out if last else None)
         return x
 
     def logits_local(self, hidden: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:

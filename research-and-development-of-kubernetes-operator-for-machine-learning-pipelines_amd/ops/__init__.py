@@ -85,9 +85,13 @@ def library_path() -> str:
 
 # ---------------------------------------------------------------- wrappers --
 
+def _into(out: torch.Tensor | None, y: torch.Tensor) -> torch.Tensor:
+    return y if out is None else out.copy_(y)
+
+
 def rmsnorm(x: torch.Tensor, w: torch.Tensor, eps: float, out: torch.Tensor | None = None):
     if not x.is_cuda:
-        return ref.rmsnorm(x, w, eps)
+        return _into(out, ref.rmsnorm(x, w, eps))
     _need_gpu()
     out = torch.empty_like(x) if out is None else out
     torch.ops.mlop.rmsnorm(out, x, w, eps)
@@ -100,10 +104,7 @@ def add_rmsnorm(x: torch.Tensor, residual: torch.Tensor, w: torch.Tensor, eps: f
     if not x.is_cuda:
         y, r = ref.add_rmsnorm(x, residual, w, eps)
         residual.copy_(r)
-        if out is not None:
-            out.copy_(y)
-            return out
-        return y
+        return _into(out, y)
     _need_gpu()
     out = torch.empty_like(x) if out is None else out
     torch.ops.mlop.add_rmsnorm(out, residual, x, w, eps)
@@ -386,13 +387,13 @@ def _nearest_choice(key):
     return best[1] if best else None
 
 
-def gemm_add_rmsnorm(x, w, residual, norm_w, eps: float):
+def gemm_add_rmsnorm(x, w, residual, norm_w, eps: float, out: torch.Tensor | None = None):
     """Decoder projection + residual + norm: residual <- residual + x @ w^T (bf16);
-    returns rmsnorm(residual) * norm_w.  On GPU the split-K MFMA GEMM's reduce
+    returns rmsnorm(residual) * norm_w (in ``out`` where given).  On GPU the split-K MFMA GEMM's reduce
     pass does the add and the norm (one launch fewer, one activation round trip
     fewer) when that beats hipBLASLt + add_rmsnorm for the shape."""
     if not x.is_cuda:
-        return add_rmsnorm(gemm(x, w), residual, norm_w, eps)
+        return add_rmsnorm(gemm(x, w), residual, norm_w, eps, out)
     _need_gpu()
     x2 = x.reshape(-1, x.shape[-1])
     if x2.stride(-1) != 1 or x2.stride(0) % 8:
@@ -406,13 +407,13 @@ def gemm_add_rmsnorm(x, w, residual, norm_w, eps: float):
 
     def fused(res):
         ws = torch.empty(nws, dtype=torch.float32, device=x.device)
-        out = torch.empty(M, N, dtype=x.dtype, device=x.device)
-        if not torch.ops.mlop.gemm_add_rmsnorm(out, res, x2, w, norm_w, ws, eps):
+        y = torch.empty(M, N, dtype=x.dtype, device=x.device) if out is None else out
+        if not torch.ops.mlop.gemm_add_rmsnorm(y, res, x2, w, norm_w, ws, eps):
             return unfused(res)  # (rows of x further apart than a kernel's offsets reach)
-        return out
+        return y
 
     def unfused(res):
-        return add_rmsnorm(gemm(x2, w), res, norm_w, eps)
+        return add_rmsnorm(gemm(x2, w), res, norm_w, eps, out)
 
     key = (_mbucket(M), N, K, EPI_ADD_RMSNORM)
     if nws == 0 or GEMM_BACKEND == "hipblaslt":
@@ -754,13 +755,13 @@ def hyper_begin(ids, table, scale: float, n_streams: int, w_in, norm_w, eps: flo
     return streams, xn
 
 
-def hyper_step(streams, y, mix, w_out, w_in, norm_w, eps: float, store: bool = True):
+def hyper_step(streams, y, mix, w_out, w_in, norm_w, eps: float, store: bool = True, out: torch.Tensor | None = None):
     """streams[:, t] <- sum_s mix[s, t] streams[:, s] + w_out[t] y (in place, unless ``store`` is off:
-    nothing reads them again); returns the next sublayer's input norm(sum_t w_in[t] streams[:, t])."""
+    nothing reads them again); returns the next sublayer's input norm(sum_t w_in[t] streams[:, t]) (in ``out`` where given)."""
     if not y.is_cuda:
-        return ref.hyper_step(streams, y, mix, w_out, w_in, norm_w, eps)
+        return _into(out, ref.hyper_step(streams, y, mix, w_out, w_in, norm_w, eps))
     _need_gpu()
-    xn = torch.empty_like(y)
+    xn = torch.empty_like(y) if out is None else out
     torch.ops.mlop.hyper_step(xn, streams, y, mix, w_out, w_in, norm_w, eps, store)
     return xn
 
@@ -880,17 +881,18 @@ def residual_begin(ids, table, scale: float, pos_table, positions, norm_w, eps: 
 
 
 def residual_step(x, y, post_w, norm_w, eps: float, store: bool = True, width: int | None = None, experts=None, share=None,
-                  tanh=None):
+                  tanh=None, out: torch.Tensor | None = None):
     """x <- x + post_w y / rms(y) (``post_w`` [W] or one number; None: x + y), in place unless ``store`` is off
     (nothing reads it again); returns the next sublayer's input norm_w x / rms(x) (None: x itself).
     ``experts`` = (rows [R, W], inv [T, k], gate [T] or None): gate[t] y[t] + sum_j rows[inv[t, j]] stands in
     y's place (y None: the sum alone; inv < 0: no row).  ``share`` = (w [T, k], h [T, W] or None, u [T] or None): rows
-    times w[t, j], and u[t] h[t] joins the sum.  ``width`` and ``tanh`` as in residual_begin."""
+    times w[t, j], and u[t] h[t] joins the sum.  ``width`` and ``tanh`` as in residual_begin.  ``out``: where the result
+    goes."""
     if not x.is_cuda:
-        return ref.residual_step(x, y, post_w, norm_w, eps, width, experts, share, tanh)
+        return _into(out, ref.residual_step(x, y, post_w, norm_w, eps, width, experts, share, tanh))
     _need_gpu()
     rows, inv, gate = experts or (None, None, None)
-    xn = torch.empty(x.shape, dtype=(rows if y is None else y).dtype, device=x.device)
+    xn = torch.empty(x.shape, dtype=(rows if y is None else y).dtype, device=x.device) if out is None else out
     torch.ops.mlop.residual_step(xn, x, y, post_w, norm_w, eps, store, width or 0, rows, inv, gate, *(share or (None, None, None)),
                                  *(tanh or (None, None)))
     return xn
@@ -1174,30 +1176,31 @@ def moe_dispatch_mid(x, router_w, top_k: int, e0: int, n_local: int, pro=None):
     return topw, topi, xs, offsets, arow, inv
 
 
-def moe_combine_add_rmsnorm(y, inv, topw, residual, norm_w, eps: float):
-    """residual <- residual + combine(y); returns rmsnorm(residual) * norm_w (one launch on GPU)."""
+def moe_combine_add_rmsnorm(y, inv, topw, residual, norm_w, eps: float, out: torch.Tensor | None = None):
+    """residual <- residual + combine(y); returns rmsnorm(residual) * norm_w (one launch on GPU; in ``out`` where given)."""
     if y.is_cuda:
         _need_gpu()
-        out = torch.empty_like(residual)
-        if torch.ops.mlop.moe_combine_add_rmsnorm(out, residual, y, inv, topw, norm_w, eps):
-            return out
-    return add_rmsnorm(moe_combine(y, inv, topw), residual, norm_w, eps)
+        o = torch.empty_like(residual) if out is None else out
+        if torch.ops.mlop.moe_combine_add_rmsnorm(o, residual, y, inv, topw, norm_w, eps):
+            return o
+    return add_rmsnorm(moe_combine(y, inv, topw), residual, norm_w, eps, out)
 
 
-def moe_down_combine_add_rmsnorm(a, w2, offsets, inv, topw, residual, norm_w, eps: float, avg_rows: int):
+def moe_down_combine_add_rmsnorm(a, w2, offsets, inv, topw, residual, norm_w, eps: float, avg_rows: int,
+                                 out: torch.Tensor | None = None):
     """The MoE block's tail: y = grouped down GEMM of the SiLU-mul rows ``a``; residual <-
-    residual + combine(y); returns rmsnorm(residual) * norm_w.  On GPU the combine sums the
+    residual + combine(y); returns rmsnorm(residual) * norm_w (in ``out`` where given).  On GPU the combine sums the
     GEMM's split-K partials itself (one launch fewer than GEMM + reduce + combine)."""
     if a.is_cuda and a.shape[0] > 0:
         _need_gpu()
         _sk_reserve(a.device)
-        out = torch.empty_like(residual)
+        o = torch.empty_like(residual) if out is None else out
         y = torch.empty(a.shape[0], w2.shape[1], dtype=a.dtype, device=a.device)
-        if torch.ops.mlop.moe_down_combine_add_rmsnorm(out, residual, y, a, w2, offsets, avg_rows, inv,
+        if torch.ops.mlop.moe_down_combine_add_rmsnorm(o, residual, y, a, w2, offsets, avg_rows, inv,
                                                        topw.contiguous(), norm_w, eps):
-            return out
+            return o
     y = grouped_gemm(a, w2, offsets, avg_rows=avg_rows)
-    return moe_combine_add_rmsnorm(y, inv, topw, residual, norm_w, eps)
+    return moe_combine_add_rmsnorm(y, inv, topw, residual, norm_w, eps, out)
 
 
 def moe_combine(y, inv, topw):

@@ -36,8 +36,8 @@ def local_experts(x, topw, topi, w13, w2, e0: int, n_local: int, dispatched=None
     gate/up-interleaved) -> grouped down GEMM (K13) -> weighted gather (K14).
     ``dispatched``: (xp, offsets, inv) from ops.moe_dispatch_small; ``combine=False``
     returns (y, inv) so the caller can fuse the weighted gather into its next kernel;
-    ``combine=(residual, norm_w, eps)`` runs the down GEMM, the combine and the residual add +
-    RMSNorm as one op (ops.moe_down_combine_add_rmsnorm) and returns the normed rows."""
+    ``combine=(residual, norm_w, eps, out)`` runs the down GEMM, the combine and the residual add +
+    RMSNorm as one op (ops.moe_down_combine_add_rmsnorm) and returns the normed rows (in ``out`` unless None)."""
     T, k = topi.shape
     arow = None
     if dispatched is None:
@@ -49,20 +49,21 @@ def local_experts(x, topw, topi, w13, w2, e0: int, n_local: int, dispatched=None
     avg = max(1, (T * k) // max(1, n_local))
     a = ops.grouped_gemm(xp, w13, offsets, epi=ops.EPI_SILU_MUL, avg_rows=avg, a_rows=arow)
     if isinstance(combine, tuple):
-        residual, norm_w, eps = combine
-        return ops.moe_down_combine_add_rmsnorm(a, w2, offsets, inv, topw, residual, norm_w, eps, avg)
+        residual, norm_w, eps, out = combine
+        return ops.moe_down_combine_add_rmsnorm(a, w2, offsets, inv, topw, residual, norm_w, eps, avg, out)
     y = ops.grouped_gemm(a, w2, offsets, avg_rows=avg)
     return ops.moe_combine(y, inv, topw) if combine else (y, inv)
 
 
 def moe_forward_add_norm(x, router_w, w13, w2, top_k: int, e0: int, n_local: int, residual, norm_w, eps: float,
-                         pre=None):
+                         pre=None, out=None):
     """Single-rank MoE block followed by the decoder's residual add + RMSNorm.  At decode
     sizes the router GEMV, routing, sort and gather are ONE launch (moe_dispatch_small; at
     16 < T <= 16384 moe_dispatch_mid, whose experts read x in place) and the weighted combine
     rides in the add + RMSNorm launch: 6 MoE glue launches -> 2.
     ``pre=(o, pre_norm_w)``: x is not formed yet; the block's own input add + RMSNorm
-    (residual += o, x = rmsnorm(residual)) becomes the dispatch launch's prologue."""
+    (residual += o, x = rmsnorm(residual)) becomes the dispatch launch's prologue.
+    ``out``: where the result goes (None: a tensor of its own)."""
     mid = None
     if pre is not None:
         o, pre_w = pre
@@ -78,14 +79,14 @@ def moe_forward_add_norm(x, router_w, w13, w2, top_k: int, e0: int, n_local: int
     if mid is not None:  # 16 < T <= 16384: one dispatch launch, the experts read x through arow
         topw, topi, xs, offsets, arow, inv = mid
         return local_experts(xs, topw, topi, w13, w2, e0, n_local, dispatched=(xs, offsets, inv, arow),
-                             combine=(residual, norm_w, eps))
+                             combine=(residual, norm_w, eps, out))
     if d is None:
         topw, topi = route(x, router_w, top_k)
         y, inv = local_experts(x, topw, topi, w13, w2, e0, n_local, combine=False)
     else:
         topw, topi, xp, offsets, _src, inv = d
         y, inv = local_experts(x, topw, topi, w13, w2, e0, n_local, dispatched=(xp, offsets, inv), combine=False)
-    return ops.moe_combine_add_rmsnorm(y, inv, topw, residual, norm_w, eps)
+    return ops.moe_combine_add_rmsnorm(y, inv, topw, residual, norm_w, eps, out)
 
 
 def moe_forward(x, router_w, w13, w2, top_k: int, ep, e0: int, n_local: int, mode: str = "allreduce",

@@ -44,8 +44,9 @@ def chunks_of(M: int, chunk: int = CHUNK_ROWS, align: int = 256):
 
 
 def row_parallel_add_norm(a: torch.Tensor, w: torch.Tensor, tp, residual: torch.Tensor, norm_w: torch.Tensor,
-                          eps: float, chunk: int | None = None, min_rows: int | None = None) -> torch.Tensor:
-    """x = rmsnorm(residual += all_reduce(a @ w^T)) * norm_w, residual updated in place.  On CPU
+                          eps: float, chunk: int | None = None, min_rows: int | None = None,
+                          out: torch.Tensor | None = None) -> torch.Tensor:
+    """x = rmsnorm(residual += all_reduce(a @ w^T)) * norm_w (in ``out`` where given), residual updated in place.  On CPU
     (gloo tests) the chunks run in order on the one stream: same arithmetic, no overlap."""
     M, N = a.shape[0], w.shape[0]
     cuda = a.is_cuda
@@ -65,9 +66,9 @@ def row_parallel_add_norm(a: torch.Tensor, w: torch.Tensor, tp, residual: torch.
     if len(parts) == 1:
         o = ops.gemm(a, w)
         tp.all_reduce(o)
-        return ops.add_rmsnorm(o, residual, norm_w, eps)
+        return ops.add_rmsnorm(o, residual, norm_w, eps, out)
     o = torch.empty(M, N, dtype=a.dtype, device=a.device)
-    x = torch.empty_like(o)
+    x = torch.empty_like(o) if out is None else out
     if cuda:
         cur = torch.cuda.current_stream(a.device)
         comm = comm_stream(a.device)

@@ -66,6 +66,8 @@ class AttnMeta:
     load: torch.Tensor | None = None
     # keys that the flash tiles read, summed over them (0: not known), by which their kernel's form is chosen
     pkeys: int = 0
+    # [T, width]: where the model's forward leaves what it returns (None: in a tensor of its own)
+    out: torch.Tensor | None = None
 
 
 # 128-token partitions: one 32-token page pair per wave at batch 1 (256: 312 tok/s, 128: 322,

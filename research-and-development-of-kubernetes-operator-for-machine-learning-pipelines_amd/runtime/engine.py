@@ -372,9 +372,9 @@ class Engine:
         self.seqs: dict[int, Sequence] = {}
         self._ids = itertools.count()
         self._decode_since_prefill = 0
-        self.graphs: dict[int, tuple] = {}  # rows -> (graph of a step up to the final norm, what its logits are written into)
-        self._graph_hidden: dict[int, torch.Tensor] = {}  # what a graph leaves for the head
-        self._logits_buf: torch.Tensor | None = None
+        self.graphs: dict[int, torch.cuda.CUDAGraph] = {}  # rows -> a step up to the final norm
+        self._graph_hidden: dict[int, torch.Tensor] = {}  # what a graph leaves for the head, all in one buffer
+        self._logits_buf: torch.Tensor | None = None  # of the widest graph's rows: what the head writes behind any of them
         self._own_logits = False  # the next graph step's logits go into a tensor of their own
         self.graph_pool = None
         self.stats = collections.Counter()
@@ -626,7 +626,7 @@ class Engine:
         else:
             self.meta.fill_decode(empty, empty, np.zeros(0, dtype=np.int64), pad_to=bucket)
             self.meta.upload(bucket, bucket, self.rows_hi)
-            self.graphs[bucket][0].replay()
+            self.graphs[bucket].replay()
         if self.device.type == "cuda":
             self._meta_ev = torch.cuda.Event()
             self._meta_ev.record()
@@ -1340,10 +1340,10 @@ class Engine:
         if self._inject_device_us:  # fault injection: this step is slower on the device only
             torch.ops.mlop.device_delay(self._inject_device_us)
         if kind == KIND_GRAPH:
-            self.graphs[bucket][0].replay()
+            self.graphs[bucket].replay()
             # the head is launched behind the graph: it writes into the engine's one buffer or, for a caller that keeps the
             # logits (feed), into a tensor of their own, where a copy of 700 rows of 128256 took 62 us of a step of 4 ms
-            return self._gather(self._head(bucket, self._own_logits), greedy)
+            return self._gather(self._head(self._graph_hidden[bucket], self._own_logits), greedy)
         meta = self.meta.meta(T, nt, nl, part, nparts, npt, pkeys)
         hidden = self.model.forward(self.meta.ids_d[:T], meta, self.kv)
         if nl == 0:
@@ -1422,10 +1422,10 @@ class Engine:
             return bool(safe)
         return all(ops.gemm_is_native(*w.shape[-2:]) for w in m.weight_tensors() if w.dim() > 1)
 
-    def _head(self, bucket: int, own: bool = False) -> torch.Tensor:
-        """This rank's logits of the decode graph's rows, in the engine's buffer unless they are the caller's (``own``)."""
-        hidden, buf = self._graph_hidden[bucket], self._logits_buf
-        return self.model.logits_local(hidden) if own or buf is None else self.model.logits_local(hidden, out=buf[:bucket])
+    def _head(self, hidden: torch.Tensor, own: bool = False) -> torch.Tensor:
+        """This rank's logits of a decode graph's rows, in the engine's buffer unless they are the caller's (``own``)."""
+        buf = self._logits_buf
+        return self.model.logits_local(hidden) if own or buf is None else self.model.logits_local(hidden, out=buf[:hidden.shape[0]])
 
     def capture_graphs(self):
         """Capture one decode graph per batch bucket, up to the head: the listed ones largest first, each run once before, then the added
@@ -1439,7 +1439,9 @@ class Engine:
         empty = np.zeros(0, dtype=np.int32)
         t0 = time.perf_counter()
         verbose = False
-        # one graph replays at a time and its logits are read before the next does: all write into one buffer
+        # one graph replays at a time and its logits are read before the next does: all write into one buffer, and into one
+        # for the head, of the widest one's rows (2048 rows of Llama-3-8B: 16 MiB, where 32 sizes' own would be 126)
+        hidden_buf = None
         self._logits_buf = m.logits_buffer(self.buckets[-1]) if hasattr(m, "logits_buffer") else None
         alone = self._native_products()
         added = [b for b in self.buckets if b not in self.listed_buckets] if alone else []
@@ -1458,8 +1460,12 @@ class Engine:
                 # in order: logits_idx is the identity, so the graph skips the row gather
                 if b not in added:  # warm-up (allocator, autotune, lazy init); the device may run it during the capture
                     self.meta.upload(b, b)
-                    self._graph_hidden[b] = m.forward(ids, meta, self.kv)
-                    self._head(b)
+                    meta.out = None if hidden_buf is None else hidden_buf[:b]
+                    h = m.forward(ids, meta, self.kv)
+                    hidden_buf = torch.empty_like(h) if hidden_buf is None else hidden_buf  # (the widest is the first)
+                    self._head(h)
+                    del h
+                meta.out = hidden_buf[:b]
                 if bi == 0 or not alone:  # (a communicator's watchdog may ask for its events, which a capture forbids)
                     torch.cuda.synchronize(self.device)
                 if bi == 0:  # the widest warm-up's memory is the graphs' now
@@ -1473,7 +1479,7 @@ class Engine:
                     self._graph_hidden[b] = m.forward(ids, meta, self.kv)
                 finally:
                     g.capture_end()
-                self.graphs[b] = (g, None if self._logits_buf is None else self._logits_buf[:b])
+                self.graphs[b] = g
         torch.cuda.current_stream(self.device).wait_stream(stream)
         torch.cuda.synchronize(self.device)
         torch.cuda.empty_cache()

@@ -6,6 +6,7 @@ import torch
 from mlopamd.models import build_model
 from mlopamd.models.config import get_config
 from mlopamd.runtime.engine import Engine, EngineConfig, fill_buckets
+from mlopamd.runtime.sampler import SamplingParams
 
 LISTED = EngineConfig.graph_buckets
 BOUND = 0.032  # two layers in bf16, see test_step_in_an_added_size
@@ -113,15 +114,41 @@ def test_added_sizes_are_not_run_before_their_capture(gpu, model):
 HYBRID = ["kosesun-1b", "nafazen-1b", "dibedra-1b", "regesun-1b"]
 
 
+def _spy_head(eng, m):
+    """The head's calls: rows, whether a buffer was given, and the result of the scheduler's steps beside one in memory of its own."""
+    calls, head, launch = [], m.logits_local, eng._launch
+
+    def logits_local(hidden, out=None):
+        calls.append((hidden.shape[0], out is not None))
+        return head(hidden, out=out)
+
+    def spy(kind, T, nt, nl, part, nparts, bucket, **kw):
+        lg = launch(kind, T, nt, nl, part, nparts, bucket, **kw)
+        if bucket:  # a graph's step
+            steps.append((bucket, lg.data_ptr(), torch.equal(lg, head(eng._graph_hidden[bucket]))))
+        return lg
+
+    steps = []
+    m.logits_local, eng._launch = logits_local, spy
+    return calls, steps
+
+
 @pytest.mark.gpu
-@pytest.mark.parametrize("model", ["llama3-8b", *HYBRID])
+@pytest.mark.parametrize("model", ["llama3-8b", "mixtral-8x7b", *HYBRID])
 def test_graphs_share_one_logits_buffer(gpu, model):
-    """Every graph writes into the buffer of the largest: the added sizes hold no logits of their own."""
+    """The scheduler's steps of all sizes leave their logits in the buffer of the largest, and their graphs what the head reads in
+    one other: the added sizes hold neither of their own."""
     m = build_model(get_config(model, num_layers=2), device=gpu, seed=1)
-    eng = Engine(m, EngineConfig(max_num_seqs=128, max_num_batched_tokens=1024, max_model_len=256, num_kv_blocks=64))
+    eng = Engine(m, EngineConfig(max_num_seqs=128, max_num_batched_tokens=1024, max_model_len=256, num_kv_blocks=256))
     assert set(eng.graphs) == set(fill_buckets([b for b in LISTED if b <= 128]))
-    assert len({logits.data_ptr() for _, logits in eng.graphs.values()}) == 1
-    assert all(logits.shape == (b, m.cfg.vocab_size) for b, (_, logits) in eng.graphs.items())
+    assert len({h.data_ptr() for h in eng._graph_hidden.values()}) == 1
+    assert all(h.shape[0] == b for b, h in eng._graph_hidden.items()) and eng._logits_buf.shape[0] == 128
+    calls, steps = _spy_head(eng, m)
+    long = {100: 3, 60: 6, 40: 9, 12: 12, 3: 15}  # sequences that go on for so many tokens: steps of 112, 64, 48, 16 and 4 rows
+    n = [max(t for k, t in long.items() if i < k) for i in range(100)]
+    eng.generate([[11 + i, 7, 5] for i in range(100)], [SamplingParams(max_tokens=t, ignore_eos=True) for t in n])
+    assert {112, 64, 48, 16, 4} <= {b for b, _, _ in steps} and {a for _, a, _ in steps} == {eng._logits_buf.data_ptr()}
+    assert all(same for _, _, same in steps)
 
 
 def _steps(m, n, graphs, steps, listed=LISTED, rows=512):
@@ -175,7 +202,8 @@ def test_step_in_a_large_added_size(gpu, model, n):
 @pytest.mark.gpu
 @pytest.mark.parametrize("model", ["llama3-8b", "kosesun-1b"])
 def test_logits_outlive_the_next_step(gpu, model):
-    """All graphs write into one buffer: what ``feed`` returned stays as it was while steps of other sizes run."""
+    """What ``feed`` returned stays as it was while steps of other sizes run, whether the head wrote it there or it is a copy of the
+    graphs' one buffer."""
     m = build_model(get_config(model, num_layers=2), device=gpu, seed=1)
     steps = [90, 40, 90, 7]
     got, eng = _steps(m, 90, True, steps)
