@@ -375,6 +375,7 @@ class Engine:
         self.graphs: dict[int, torch.cuda.CUDAGraph] = {}  # rows -> a step up to the final norm
         self._graph_hidden: dict[int, torch.Tensor] = {}  # what a graph leaves for the head, all in one buffer
         self._logits_buf: torch.Tensor | None = None  # of the widest graph's rows: what the head writes behind any of them
+        self._dense_logits = False  # the head's logits have no columns beside the vocabulary's
         self._own_logits = False  # the next graph step's logits go into a tensor of their own
         self.graph_pool = None
         self.stats = collections.Counter()
@@ -1256,10 +1257,16 @@ class Engine:
         for s, _, want in portions:
             at[s.seq_id] = o
             o += len(want)
+        idx = [at[s.seq_id] + (j if len(toks) > 1 else 0) for s, toks, want in live for j in range(len(want))]
+        as_is = self.model.ps.tp.size == 1 and idx == list(range(len(idx)))  # handed out as the head leaves them
         bucket = next((b for b in self.buckets if b >= B), None)
-        if not portions and self.graphs.get(bucket) is not None:
+        graph = not portions and self.graphs.get(bucket) is not None
+        # Written where the caller keeps them, unless that holds more than the wanted rows: columns of padding, or rows of it above
+        # a quarter of the step's (sizes between the listed ones have fewer) and 32.
+        own = graph and as_is and bool(idx) and self._dense_logits and bucket - len(idx) <= max(bucket // 4, 32)
+        if graph:
             self.meta.fill_decode(rows, ctx, last, pad_to=bucket)
-            self._own_logits = True
+            self._own_logits = own
             try:
                 logits = self._launch(KIND_GRAPH, bucket, bucket, bucket, 0, 0, bucket)
             finally:
@@ -1274,12 +1281,12 @@ class Engine:
             s.prompt.extend(toks)
             s.num_cached += len(toks)
         self.stats["fed_tokens"] += total
-        idx = [at[s.seq_id] + (j if len(toks) > 1 else 0) for s, toks, want in live for j in range(len(want))]
         if not idx:
             return None
         # the device is not waited for: a caller may feed the next step while this one runs
-        if self.model.ps.tp.size == 1 and idx == list(range(len(idx))):
-            return logits[:len(idx)]
+        if as_is:
+            rows = logits[:len(idx)]
+            return rows.clone() if graph and not own else rows  # (the graphs' one buffer)
         at_d = torch.tensor(idx, pin_memory=logits.is_cuda).to(logits.device, non_blocking=True)
         return logits[at_d]
 
@@ -1462,9 +1469,10 @@ class Engine:
                     self.meta.upload(b, b)
                     meta.out = None if hidden_buf is None else hidden_buf[:b]
                     h = m.forward(ids, meta, self.kv)
-                    hidden_buf = torch.empty_like(h) if hidden_buf is None else hidden_buf  # (the widest is the first)
-                    self._head(h)
-                    del h
+                    logits = self._head(h)
+                    if hidden_buf is None:  # the widest
+                        hidden_buf, self._dense_logits = torch.empty_like(h), logits.is_contiguous()
+                    del h, logits
                 meta.out = hidden_buf[:b]
                 if bi == 0 or not alone:  # (a communicator's watchdog may ask for its events, which a capture forbids)
                     torch.cuda.synchronize(self.device)

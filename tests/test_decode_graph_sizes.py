@@ -151,6 +151,44 @@ def test_graphs_share_one_logits_buffer(gpu, model):
     assert all(same for _, _, same in steps)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("model,vocab", [("llama3-8b", None), ("dibedra-1b", None), ("kosesun-1b", 5001), ("regesun-1b", 5001)])
+def test_what_feed_hands_out(gpu, model, vocab):
+    """Logits that the caller keeps are written where it keeps them; not where they are not wanted, wanted in another order, or would
+    hold far more than the wanted rows.  The values are those of the eager step, the tensor is dense, and holds little else."""
+    m = build_model(get_config(model, num_layers=2, **({"vocab_size": vocab} if vocab else {})), device=gpu, seed=1)
+    mk = lambda graphs: Engine(m, EngineConfig(max_num_seqs=128, max_num_batched_tokens=1024, max_model_len=256, num_kv_blocks=256,  # noqa: E731
+                                               use_graphs=graphs, graph_buckets=(1, 16, 128), enable_prefix_caching=False))
+    V, dense = m.cfg.vocab_size, not vocab  # (the head's rows are whole tiles)
+    runs = []
+    for graphs in (True, False):
+        eng = mk(graphs)
+        seqs = [eng.open_sequence() for _ in range(100)]
+        eng.feed([(s, [11 + i, 7, 5], []) for i, s in enumerate(seqs)])
+        if graphs:
+            calls, _ = _spy_head(eng, m)
+        out = []
+        for rows, wanted in ((range(100), range(100)), (range(100), ()), (range(100), range(50)), (range(100), range(1, 100, 2)),
+                             (range(12), range(12)), (range(20), range(20)), (range(1), range(1))):
+            out.append(eng.feed([(seqs[i], [13 + i], [0] if i in wanted else []) for i in rows]))
+            if graphs:
+                assert len(calls) == 1
+                calls.clear() if out[-1] is None else out.append(calls.pop())
+        torch.cuda.synchronize()
+        runs.append(out)
+        if graphs:
+            del m.logits_local
+    got, buffered = [x for x in runs[0] if not isinstance(x, tuple)], [x[1] for x in runs[0] if isinstance(x, tuple)]
+    # (all, none, half, every second, 12 in 16 rows, 20 in 128, 1)
+    assert buffered == ([False, True, True, False, True, False] if dense else [True] * 6)
+    for a, b in zip(got, runs[1]):
+        assert (a is None) == (b is None)
+        if a is not None:
+            assert a.is_contiguous() and a.dtype == b.dtype and a.shape == b.shape == (a.shape[0], V)
+            assert a.untyped_storage().nbytes() <= max(4 * a.numel() // 3, a.numel() + 32 * V) * a.element_size()
+            assert float(_row_errors(a.float(), b.float())[-1]) < BOUND
+
+
 def _steps(m, n, graphs, steps, listed=LISTED, rows=512):
     """Logits of the decode steps over ``steps`` sequences each (a prefix of n sequences of three tokens), all kept until the
     last one ran; and the engine."""
