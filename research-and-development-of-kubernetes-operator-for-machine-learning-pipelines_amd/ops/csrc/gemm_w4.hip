@@ -198,9 +198,11 @@ __device__ __forceinline__ void gemm_w4_tiles(
       const int r = (i < NI ? p : p - 4 * NI) * 8 + (lane >> 3);
       const uint32_t ch = (uint32_t)(((lane & 7) ^ ((r >> 1) & 7)) << 4);
       if (i < NI) {
-        // A rows past the last load nothing: past num_records an LDS-DMA is dropped, still counted by vmcnt.  What the LDS then
-        // holds reaches accumulators that are never stored, and multiplying it costs less power than the last row again and again
-        // (three Mixtral layers at 1628 tokens, a tenth of whose tiles is such rows: 3.71 -> 3.66 ms).
+        // A rows past the last load nothing: past num_records an LDS-DMA is dropped, and counted by vmcnt in its turn (of 5e8 words
+        // that a DMA brought from HBM, waited for with a count over eight dropped or half-dropped ones behind it, none was read too early).
+        // What the LDS then holds reaches accumulators that are never stored, and multiplying it costs less power than the last row again and
+        // again (three Mixtral layers at 1628 tokens, a tenth of whose tiles is such rows: 1.2 % of 3.7 ms in two sessions, in which two runs
+        // of one side differ by 1 - 2; no other step beyond what two runs differ).
         const int row = GROUPED && re.a_rows != nullptr ? rows[8 * i + (lane >> 3)] : m0 + r;
         vo[i] = m0 + r < m_end ? (uint32_t)row * (uint32_t)(lda * 2) + ch + kb * 128 : 0x80000000u;
       } else {

@@ -155,13 +155,15 @@ void gemm_dense_plan(int variant, int bm, int bn, int splits, int stages = 0);
 bool gemm_w4_ok(int M, int N, int K, int lda, int ldb, int ldc = 0);
 // the four-wave kernel cuts its r = T % CUs tail tiles into K-halves (2r <= CUs, nk even)
 bool gemm_w4_split_ok(int T, int nk);
+// whether its tiles of bm rows walk K in step (not each XCD from another eighth)
 bool gemm_w4_in_step(int M, int N, int K, int bm);
 bool gemm_sk_scratch(float** ws, int** cnt, int* cus);
 bool gemm_sk_available(int* cus);
 bool run_w4(int epi, const uint16_t* A, int lda, const uint16_t* B, int ldb, uint16_t* C, int ldc, int M, int N,
             int K, hipStream_t st, const RopeEpi& re, int bm = 256);
-// the experts' products on it (offsets on the device; a_n: A's rows)
+// K in ranges on it: fp32 slabs ws[range][M][N]
 void run_w4_slab(const uint16_t* A, int lda, const uint16_t* B, int ldb, float* ws, int M, int N, int K, int splits, int bm, hipStream_t st);
+// the experts' products on it (offsets on the device; a_n: A's rows)
 bool gemm_w4_grouped_ok(int M, int N, int K, int n_groups, int a_n);
 void run_w4_grouped(int epi, const uint16_t* A, int lda, const uint16_t* B, int ldb, uint16_t* C, int ldc, int M, int N,
                     int K, hipStream_t st, const RopeEpi& re, const int* offsets, int n_groups);

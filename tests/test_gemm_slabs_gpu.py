@@ -79,3 +79,24 @@ def test_captured(gpu):
         assert torch.equal(got, out) and torch.equal(res, want)
         other = r0.clone()
         assert torch.equal(ops.gemm_add_rmsnorm(x, w, other, g, 1e-5), out)
+
+
+def test_rows_too_far_apart(gpu, monkeypatch):
+    """Rows of x further apart than the four-wave kernel's offsets reach: the op says no and has written nothing, and the call, with
+    or without a tensor for its result, is the product and the norm one behind the other."""
+    M, N, K = 400, 4096, 4096
+    x, w, g, r0 = operands(gpu, M, N, K)
+    n = torch.ops.mlop.gemm_workspace(M, N, K, 2)
+    assert n >= 2 * M * N
+    far = torch.empty(M, 2_700_000, device=gpu, dtype=bf)[:, :K]
+    out, res = torch.zeros(M, N, device=gpu, dtype=bf), r0.clone()
+    assert not torch.ops.mlop.gemm_add_rmsnorm(out, res, far, w, g, torch.empty(n, device=gpu), 1e-5)
+    assert torch.equal(res, r0) and not out.any()
+    del far
+    want_res = r0.clone()
+    want = ops.add_rmsnorm(ops.gemm(x, w), want_res, g, 1e-5)
+    monkeypatch.setattr(torch.ops.mlop, "gemm_add_rmsnorm", lambda *a: False)
+    for given in (None, out):
+        res = r0.clone()
+        got = ops.gemm_add_rmsnorm(x, w, res, g, 1e-5, given)
+        assert torch.equal(got, want) and torch.equal(res, want_res) and (given is None or got is given)
