@@ -1921,20 +1921,20 @@ void gemm_plan(int M, int N, int K, int epi, int out[5]) {
 // kernel where it is estimated to be 3 % faster than the weight stream, or than the 256 x 128 tiles that have 130 - 168 tiles of 128
 // columns.  The weight stream's workgroup takes in the whole batch beside its 128 or 256 columns, and a grid of 1.1 rounds takes
 // two; the four-wave kernel has 128-row tiles, two for a column, or one of the batch's height.  Not where it would cut the last tiles into
-// K-halves (0.82 - 0.87 of the time at 18432 - 20480 and 65536 - 69888 columns): up to 256 rows no product uses the scratch of the
-// hand-over, so one may run beside another stream's that does (captured decode steps of Dibedra: a layer's experts beside its dense
-// products).  us, cold weights, stream -> four-wave: gate_up 28672 x 4096, which changes over at 225 rows, at 225 / 240 / 256 72 -> 62,
+// K-halves (0.82 - 0.87 of the time at 18432 - 20480 and 65536 - 69888 columns): up to 256 rows no product but those with RoPE uses the
+// scratch of the hand-over, so one may run beside another stream's that does (captured decode steps of Dibedra: a layer's experts beside
+// its dense products).  us, cold weights, stream -> four-wave: gate_up 28672 x 4096, which changes over at 225 rows, at 225 / 240 / 256 72 -> 62,
 // 74 -> 63, 74 -> 64; 57344 x 8192 at the same 235 -> 220, 234 -> 227, 233 -> 227, head 128256 x 4096 252 -> 215, 261 -> 225, 259 -> 229; 36864 x
-// 4096 at 150 / 200 93 -> 76, 115 -> 82, 20480 x 4096 63 -> 54, 64 -> 57.  Steps of six Llama-3-8B layers: 240 sequences 1699 -> 1618, a
-// prompt of 250 tokens 1323 -> 1271; three of the 70B, 250 sequences 2225 -> 2137.
+// 4096 at 150 / 200 93 -> 76, 115 -> 82, 20480 x 4096 63 -> 54, 64 -> 57.  Steps of six Llama-3-8B layers: a prompt of 250
+// tokens 1273 -> 1257, eight of 30 1225 -> 1202.
 // Estimates in us fitted to 720 points (15 widths of 8192 - 128256, K 2048 - 8192, 135 - 256 rows, cold weights), 5 and 6 % off in the
 // mean.  Weight stream of bm rows, g the share of the CUs in a round: 10.1 + a K-step's .117 + .00189 bm + .00121 bm g + .081 g with 128
 // columns, 11.6 + -.261 + .00447 bm + .00168 bm g + .588 g with 256; the 256 x 128 tiles 8 + .0137 K.  Four-wave: 2.5 + rounds of .0227 K, .0262 where
 // its tiles walk K in step, times the height's share, the last one less by .16 of its empty part, or 5.5 + the weights at 5 TB/s: the sixth
 // root of the sum of their sixth powers, a maximum that is 12 % over where the two are level, as it is where a product waits for both.
-// 325 drawn products of 16384 - 160000 columns: the 153 chosen take 0.857 of the stream's time, 4 of them 1.03 - 1.10 (88832 x 1280 at 224 rows
-// 79 -> 87, 97024 x 2560 at 223 135 -> 148, 57344 x 4096 at 256 123 -> 126).  Left on the stream though the other is faster: heads at 193 - 224
-// rows (128256 x 4096 at 197 / 224 241 / 249 and 210 / 218, which the estimates take for 223 and 230), and plain products up to 32768 columns,
+// Of 325 products, these and drawn ones of 16384 - 160000 columns, the 153 chosen take 0.857 of the time, 4 of them 1.03 - 1.10 (88832 x 1280 at
+// 224 rows 79 -> 87, 97024 x 2560 at 223 135 -> 148, 57344 x 4096 at 256 123 -> 126).  Left on the stream though the other is faster: heads at 193 - 224
+// rows (128256 x 4096 at 197 / 224 in another session 241 / 249 and 210 / 218; the estimates say 230 and 223), and plain products up to 32768 columns,
 // which the rule was not drawn for (32768 x 4096 at 256 rows 78 and 65).
 static void few_rows_w4(int M, int N, int K, int epi, Plan& p) {
   if (M <= 128 || M > 256 || K < 1024 || g_dp[0] >= 0 || p.splits > 1 || (epi != EPI_SILU_MUL && N <= 32768) || !gemm_w4_ok(M, N, K, K, K)) return;
